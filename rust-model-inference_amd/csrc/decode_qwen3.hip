@@ -26,6 +26,7 @@
 #include <utility>
 #include <vector>
 
+#include "attn_prompt.h"
 #include "device_math.h"
 #include "device_quant.h"
 #include "device_sample.h"
@@ -513,24 +514,15 @@ struct AttnFromQkv {
     uint16_t *k_row, *v_row;         // the cache rows of this position, [n_head_kv][128] each
     float eps;
 };
-// DENSE: for launches of many workgroups (a prompt pass: positions x heads).  Every phase below is a stretch of
-// dependent instructions, so one workgroup leaves its compute unit idle most of the time; with the registers held
-// to 128 (a short value prefetch) two workgroups share a unit and fill each other's waits.
-constexpr int kDenseWaves = 6, kDenseBatch = 2;
-template <bool FROM_QKV, int PVP = 1, bool DENSE = false>
-__global__ __launch_bounds__(kA128Threads, DENSE ? kDenseWaves : 2) void attention128_quant_kernel(
+template <bool FROM_QKV, int PVP = 1>
+__global__ __launch_bounds__(kA128Threads, 2) void attention128_quant_kernel(
     const uint16_t *__restrict__ q16, const uint16_t *__restrict__ k_cache, const uint16_t *__restrict__ v_cache,
     uint32_t step, uint32_t kv_stride, uint32_t n_head, uint32_t n_head_kv, int8_t *__restrict__ q8,
-    float *__restrict__ scales, int rounding, AttnFromQkv fq, uint32_t tok_q16_stride, uint32_t tok_out_stride) {
+    float *__restrict__ scales, int rounding, AttnFromQkv fq) {
     extern __shared__ double lds_d[];
     __shared__ float red_f[kA128Threads / 64];
     __shared__ uint64_t exp_tab[32];
     __shared__ __attribute__((aligned(16))) uint16_t new16[3][128];  // this step's q, k, v as f16
-    // token blockIdx.z of a launch over several consecutive positions (their cache rows are filled already)
-    step += blockIdx.z;
-    q16 += size_t(blockIdx.z) * tok_q16_stride;
-    q8 += size_t(blockIdx.z) * tok_out_stride;
-    scales += size_t(blockIdx.z) * (tok_out_stride >> 5);
     // grid = (query heads per key/value head, key/value heads), or with PVP parts n_head * PVP workgroups in a row:
     // key/value head fastest, then the query head of its group, then the part
     static_assert(PVP == 1 || PVP == 2 || PVP == 4, "a part is one, two or four blocks of 32 dimensions");
@@ -589,8 +581,8 @@ __global__ __launch_bounds__(kA128Threads, DENSE ? kDenseWaves : 2) void attenti
     // With parts a slice is short (six keys a slice cover 768 keys with four parts; longer slices go on in the batches
     // further down) and its loads are unconditional: a load under
     // a branch makes the wait for this position's q, k, v (issued first) drain most of what was issued behind them.
-    constexpr uint32_t kPre = DENSE ? 1 : (PVP == 1 ? (kA128Threads >= 1024 ? 12 : (kA128Threads >= 512 ? 20 : 40)) : 24 / PVP);
-    constexpr uint32_t kBatch = DENSE ? kDenseBatch : 8;  // keys of a slice in flight beyond the first kPre
+    constexpr uint32_t kPre = PVP == 1 ? (kA128Threads >= 1024 ? 12 : (kA128Threads >= 512 ? 20 : 40)) : 24 / PVP;
+    constexpr uint32_t kBatch = 8;  // keys of a slice in flight beyond the first kPre
     const uint32_t dg = tid % kDgLanes, sl = tid / kDgLanes;
     const uint32_t chunk = (n_cached + kSlices - 1) / kSlices;
     const uint32_t t_begin = sl * chunk, t_end = t_begin + chunk < n_cached ? t_begin + chunk : n_cached;
@@ -690,7 +682,7 @@ __global__ __launch_bounds__(kA128Threads, DENSE ? kDenseWaves : 2) void attenti
     if (tid == 0) {  // the reference adds the weights one after the other in f32; the padding zeros change nothing
         // one lane, one dependent chain of adds; the LDS reads run 32 values ahead of it (two buffers, no copies)
         float acc = 0.0f;
-        constexpr int kAhead = DENSE ? 4 : 8;  // float4 of each buffer
+        constexpr int kAhead = 8;  // float4 of each buffer
         float4 a[kAhead], b[kAhead];
 #pragma unroll
         for (int j = 0; j < kAhead; j++) a[j] = reinterpret_cast<const float4 *>(scores)[j];
@@ -1088,11 +1080,11 @@ static void launch_attention128_from_qkv(const uint16_t *k_cache, const uint16_t
     switch (attn_pv_parts(step + 1)) {
     case 4:
         hipLaunchKernelGGL((attention128_quant_kernel<true, 4>), dim3(n_head * 4), dim3(kA128Threads), lds, st, no_q16, k_cache,
-                           v_cache, step, kv_stride, n_head, n_head_kv, q8, scales, rounding, fq, 0u, 0u);
+                           v_cache, step, kv_stride, n_head, n_head_kv, q8, scales, rounding, fq);
         break;
     default:
         hipLaunchKernelGGL((attention128_quant_kernel<true, 1>), dim3(n_head / n_head_kv, n_head_kv), dim3(kA128Threads), lds, st,
-                           no_q16, k_cache, v_cache, step, kv_stride, n_head, n_head_kv, q8, scales, rounding, fq, 0u, 0u);
+                           no_q16, k_cache, v_cache, step, kv_stride, n_head, n_head_kv, q8, scales, rounding, fq);
     }
 }
 
@@ -1227,21 +1219,28 @@ struct rmi_hip_qwen3 : RmiSession {
     uint16_t *q16b = nullptr;
     int8_t *act_q8b = nullptr;
     void *partialb = nullptr;
+    float *wantb = nullptr;              // the logits that a pass was asked for, kPassWant rows
+    float *attn_scratch = nullptr;       // of the pass's attention
+    size_t attn_scratch_floats = 0;
     void *attn_split = nullptr;          // scratch of the split attention launches (head dimension 128)
 
     ~rmi_hip_qwen3() override;
     int enqueue_step(uint32_t step, hipStream_t st) override;
     const float *step_logits() const override { return logits; }
     bool pass_possible(uint32_t step0, uint32_t n) const override;
-    // every position's logits, whichever are asked for
     int enqueue_pass(uint32_t step0, uint32_t n, const uint32_t *want, uint32_t n_want, bool sample, hipStream_t st) override;
-    const float *pass_logits(uint32_t offset, uint32_t) const override { return logitsb + size_t(offset) * cfg.vocab; }
+    uint32_t max_pass_want() const override;
+    const float *pass_logits(uint32_t, uint32_t i) const override { return wantb + size_t(i) * cfg.vocab; }
 };
 
 namespace {
 
-constexpr uint32_t kPromptBatch = 128;  // most positions a prompt pass takes (the buffers' size); kPromptPassDefault is what it takes
-constexpr uint32_t kPromptPassDefault = 128;
+// Most positions a prompt pass takes, which is also what it takes unless told otherwise.  A pass of 512 gives the
+// attention of sixteen heads two workgroups a compute unit.
+constexpr uint32_t kPromptBatch = 512;
+constexpr uint32_t kHeadBatch = 128;  // positions whose logits are in memory at once
+constexpr uint32_t kPassWant = 64;    // logits of a pass that a caller can ask for
+inline uint32_t prompt_batch(uint32_t capacity) { return capacity < kPromptBatch ? capacity : kPromptBatch; }
 
 template <typename T>
 T *dev_alloc(rmi_hip_qwen3 *s, size_t count, bool zero = false) {
@@ -1335,7 +1334,7 @@ int enqueue_step(rmi_hip_qwen3 *s, uint32_t step, hipStream_t st) {
         } else if (d128)
             hipLaunchKernelGGL(attention128_quant_kernel<false>, dim3(c.n_head / c.n_head_kv, c.n_head_kv), dim3(kA128Threads), attn128_lds_bytes(step + 1),
                                st, s->q16, s->k_cache + layer_base, s->v_cache + layer_base, step, s->kv_stride,
-                               c.n_head, c.n_head_kv, s->act_q8, s->act_scales, rnd, AttnFromQkv{}, 0u, 0u);
+                               c.n_head, c.n_head_kv, s->act_q8, s->act_scales, rnd, AttnFromQkv{});
         else
             hipLaunchKernelGGL(attention_quant_kernel, dim3(c.n_head), dim3(kAttnThreads), attn_lds, st, s->q16,
                                s->k_cache + layer_base, s->v_cache + layer_base, step, s->kv_stride, c.n_head,
@@ -1367,23 +1366,19 @@ int enqueue_step(rmi_hip_qwen3 *s, uint32_t step, hipStream_t st) {
     return RMI_HIP_OK;
 }
 
-// Whether the prompt positions step0 .. step0 + n - 1 can go through one pass: head dimension 128, every launch
-// of the pass within what the single-workgroup attention kernel holds, and short of the split's first position.
+// Whether the prompt positions step0 .. step0 + n - 1 can go through one pass: head dimension 128, buffers for them.
 bool prompt_pass_possible(const rmi_hip_qwen3 *s, uint32_t step0, uint32_t n) {
     const rmi_hip_qwen3_config &c = s->cfg;
-    if (!s->xb || n == 0 || n > kPromptBatch) return false;
-    if (c.n_embd > kNormMaxN) return false;
-    if (s->attn_split && attn128_use_split(step0 + n, c.n_head)) return false;
-    return attn128_lds_bytes(step0 + n) <= 64 * 1024;
+    return s->xb && n > 0 && n <= prompt_batch(c.capacity) && step0 + n <= c.capacity && c.n_embd <= kNormMaxN;
 }
 
 // n consecutive prompt positions from step0 on in one pass: every product reads its weight once for all of them
 // (the x86-64-order GEMV takes up to eight tokens a launch and gives each the bits it gets alone), the other
 // kernels run once per position inside one launch.  Position by position the arithmetic is that of enqueue_step's
 // separate-kernel path; a position's keys and values are in the cache before any attention launch of the pass
-// reads them.  Leaves every position's argmax and top-2 logits, the logits in logitsb, and, behind the last
+// reads them.  Leaves every position's argmax and top-2 logits, the logits asked for in wantb, and, behind the last
 // position, the step counter and the next token's embedding as a single step expects them.
-int enqueue_prompt_pass(rmi_hip_qwen3 *s, uint32_t step0, uint32_t n, hipStream_t st) {
+int enqueue_prompt_pass(rmi_hip_qwen3 *s, uint32_t step0, uint32_t n, const uint32_t *want, uint32_t n_want, hipStream_t st) {
     const rmi_hip_qwen3_config &c = s->cfg;
     const int rnd = c.rounding;
     StepParams *sp = static_cast<StepParams *>(s->params);
@@ -1403,10 +1398,9 @@ int enqueue_prompt_pass(rmi_hip_qwen3 *s, uint32_t step0, uint32_t n, hipStream_
         hipLaunchKernelGGL(qk_norm_rope_store_kernel, dim3(c.n_head + 2 * c.n_head_kv, n), dim3(64), 0, st, s->qkvb, qn, kn,
                            s->cos_t, s->sin_t, step0, s->q16b, s->k_cache + row, s->v_cache + row, c.n_head, c.n_head_kv,
                            c.head_dim_k, c.head_dim_v, c.eps, TokStride3{n_qkv, s->n_q, s->kv_stride});
-        // (a pass ends short of the split's first position, far below the 64 KiB of LDS a launch may take unasked)
-        hipLaunchKernelGGL((attention128_quant_kernel<false, 1, true>), dim3(c.n_head / c.n_head_kv, c.n_head_kv, n), dim3(kA128Threads),
-                           attn128_lds_bytes(step0 + n), st, s->q16b, s->k_cache + layer_base, s->v_cache + layer_base, step0,
-                           s->kv_stride, c.n_head, c.n_head_kv, s->act_q8b, s->act_scalesb, rnd, AttnFromQkv{}, s->n_q, s->n_attn);
+        rc = rmi_launch_attn128_prompt(s->q16b, s->k_cache + layer_base, s->v_cache + layer_base, step0, n, s->kv_stride, c.n_head, c.n_head_kv,
+                                       s->attn_scratch, s->attn_scratch_floats, s->act_q8b, s->act_scalesb, rnd, st);
+        if (rc != RMI_HIP_OK) return rc;
         rc = rmi_gemv_q8_0_tokens(s->w_o[l], s->act_q8b, s->act_scalesb, s->residb, n, c.n_embd, 0, c.n_embd, st);
         if (rc != RMI_HIP_OK) return rc;
         launch_add_rmsnorm_quant(s->xb, s->residb, s->ffn_norm[l], c.n_embd, c.eps, s->act_q8b, s->act_scalesb, rnd, st, n,
@@ -1422,13 +1416,20 @@ int enqueue_prompt_pass(rmi_hip_qwen3 *s, uint32_t step0, uint32_t n, hipStream_
     }
     launch_add_rmsnorm_quant(s->xb, pending, s->output_norm, c.n_embd, c.eps, s->act_q8b, s->act_scalesb, rnd, st, n,
                              TokStride3{c.n_embd, pending_stride, c.n_embd});
-    rc = rmi_gemv_q8_0_tokens(s->head, s->act_q8b, s->act_scalesb, s->logitsb, n, c.vocab, 0, c.vocab, st);
-    if (rc != RMI_HIP_OK) return rc;
-    hipLaunchKernelGGL(argmax_partial_kernel, dim3(kArgmaxGroups, n), dim3(256), 0, st, s->logitsb, c.vocab,
-                       static_cast<Top *>(s->partialb));
-    hipLaunchKernelGGL(argmax_final_batch_kernel<EmbedQ8>, dim3(n), dim3(256), 0, st, static_cast<const Top *>(s->partialb), kArgmaxGroups,
-                       sp, step0, static_cast<const uint32_t *>(nullptr), s->tok, s->step_argmax, s->step_top2, s->nonfinite,
-                       EmbedQ8{s->embd->data, s->embd->n_units, c.vocab, s->x, c.n_embd});
+    for (uint32_t i0 = 0, w = 0; i0 < n; i0 += kHeadBatch) {  // the vocabulary projection and its argmax, kHeadBatch positions at a time
+        const uint32_t nb = n - i0 < kHeadBatch ? n - i0 : kHeadBatch;
+        rc = rmi_gemv_q8_0_tokens(s->head, s->act_q8b + size_t(i0) * c.n_embd, s->act_scalesb + size_t(i0) * (c.n_embd / 32), s->logitsb, nb,
+                                  c.vocab, 0, c.vocab, st);
+        if (rc != RMI_HIP_OK) return rc;
+        hipLaunchKernelGGL(argmax_partial_kernel, dim3(kArgmaxGroups, nb), dim3(256), 0, st, s->logitsb, c.vocab,
+                           static_cast<Top *>(s->partialb));
+        hipLaunchKernelGGL(argmax_final_batch_kernel<EmbedQ8>, dim3(nb), dim3(256), 0, st, static_cast<const Top *>(s->partialb), kArgmaxGroups,
+                           sp, step0 + i0, static_cast<const uint32_t *>(nullptr), s->tok, s->step_argmax, s->step_top2, s->nonfinite,
+                           EmbedQ8{s->embd->data, s->embd->n_units, c.vocab, s->x, c.n_embd});
+        for (; w < n_want && want[w] < i0 + nb; w++)
+            RMI_HIP_CHECK(hipMemcpyAsync(s->wantb + size_t(w) * c.vocab, s->logitsb + size_t(want[w] - i0) * c.vocab, size_t(c.vocab) * 4,
+                                         hipMemcpyDeviceToDevice, st));
+    }
     RMI_HIP_CHECK(hipGetLastError());
     return RMI_HIP_OK;
 }
@@ -1437,9 +1438,10 @@ int enqueue_prompt_pass(rmi_hip_qwen3 *s, uint32_t step0, uint32_t n, hipStream_
 
 int rmi_hip_qwen3::enqueue_step(uint32_t step, hipStream_t st) { return ::enqueue_step(this, step, st); }
 bool rmi_hip_qwen3::pass_possible(uint32_t step0, uint32_t n) const { return prompt_pass_possible(this, step0, n); }
-int rmi_hip_qwen3::enqueue_pass(uint32_t step0, uint32_t n, const uint32_t *, uint32_t, bool, hipStream_t st) {
-    return enqueue_prompt_pass(this, step0, n, st);
+int rmi_hip_qwen3::enqueue_pass(uint32_t step0, uint32_t n, const uint32_t *want, uint32_t n_want, bool, hipStream_t st) {
+    return enqueue_prompt_pass(this, step0, n, want, n_want, st);
 }
+uint32_t rmi_hip_qwen3::max_pass_want() const { return kPassWant; }
 rmi_hip_qwen3::~rmi_hip_qwen3() {
     if (head && head != embd) rmi_hip_free_weight(head);
     if (embd) rmi_hip_free_weight(embd);
@@ -1591,10 +1593,10 @@ int rmi_hip_attention_f16_quantize_q8_0_dev(const uint16_t *q16, const uint16_t 
     if (lds > attn_lds_limit()) return rmi_fail(RMI_HIP_E_INVALID, "%u keys exceed what the kernel holds in LDS", n_keys);
     if (d128 && attn_pv_parts(n_keys) == 4 && lds <= 64 * 1024)  // four workgroups a head, as in the session's own launch
         hipLaunchKernelGGL((attention128_quant_kernel<false, 4>), dim3(n_head * 4), dim3(kA128Threads), lds, static_cast<hipStream_t>(stream),
-                           q16, k_cache, v_cache, n_keys - 1, kv_stride, n_head, n_head_kv, q8, scales, rounding, AttnFromQkv{}, 0u, 0u);
+                           q16, k_cache, v_cache, n_keys - 1, kv_stride, n_head, n_head_kv, q8, scales, rounding, AttnFromQkv{});
     else if (d128)
         hipLaunchKernelGGL(attention128_quant_kernel<false>, dim3(n_head / n_head_kv, n_head_kv), dim3(kA128Threads), lds, static_cast<hipStream_t>(stream),
-                           q16, k_cache, v_cache, n_keys - 1, kv_stride, n_head, n_head_kv, q8, scales, rounding, AttnFromQkv{}, 0u, 0u);
+                           q16, k_cache, v_cache, n_keys - 1, kv_stride, n_head, n_head_kv, q8, scales, rounding, AttnFromQkv{});
     else
         hipLaunchKernelGGL(attention_quant_kernel, dim3(n_head), dim3(kAttnThreads), lds, static_cast<hipStream_t>(stream),
                            q16, k_cache, v_cache, n_keys - 1, kv_stride, n_head, n_head_kv, head_dim_k, head_dim_v, q8,
@@ -1677,7 +1679,7 @@ rmi_hip_qwen3 *rmi_hip_qwen3_create(const rmi_hip_qwen3_config *cfg, const rmi_h
     s->cfg = c;
     s->vocab = c.vocab;
     s->capacity = c.capacity;
-    s->prompt_pass = kPromptPassDefault;
+    s->prompt_pass = prompt_batch(c.capacity);
     s->n_q = c.n_head * c.head_dim_k;
     s->n_k = c.n_head_kv * c.head_dim_k;
     s->n_v = c.n_head_kv * c.head_dim_v;
@@ -1748,16 +1750,17 @@ rmi_hip_qwen3 *rmi_hip_qwen3_create(const rmi_hip_qwen3_config *cfg, const rmi_h
          (s->gu = dev_alloc<float>(s, size_t(2) * c.n_ff)) && (s->logits = dev_alloc<float>(s, c.vocab)) &&
          (s->act_q8 = dev_alloc<int8_t>(s, s->max_n_in)) && (s->act_scales = dev_alloc<float>(s, s->max_n_in / 32)) &&
          s->alloc_sampling();
-    if (ok && c.head_dim_k == 128 && c.head_dim_v == 128)  // prompt passes of kPromptBatch positions (head dimension 128)
-        ok = (s->xb = dev_alloc<float>(s, size_t(kPromptBatch) * c.n_embd)) &&
-             (s->residb = dev_alloc<float>(s, size_t(kPromptBatch) * c.n_embd)) &&
-             (s->qkvb = dev_alloc<float>(s, size_t(kPromptBatch) * (size_t(s->n_q) + s->n_k + s->n_v))) &&
-             (s->q16b = dev_alloc<uint16_t>(s, size_t(kPromptBatch) * s->n_q)) &&
-             (s->gub = dev_alloc<float>(s, size_t(kPromptBatch) * 2 * c.n_ff)) &&
-             (s->logitsb = dev_alloc<float>(s, size_t(kPromptBatch) * c.vocab)) &&
-             (s->act_q8b = dev_alloc<int8_t>(s, size_t(kPromptBatch) * s->max_n_in)) &&
-             (s->act_scalesb = dev_alloc<float>(s, size_t(kPromptBatch) * s->max_n_in / 32)) &&
-             (s->partialb = dev_alloc<Top>(s, size_t(kPromptBatch) * kArgmaxGroups));
+    if (ok && c.head_dim_k == 128 && c.head_dim_v == 128) {  // prompt passes (head dimension 128)
+        const size_t n = prompt_batch(c.capacity), head = n < kHeadBatch ? n : kHeadBatch;
+        s->attn_scratch_floats = rmi_attn_prompt_scratch_floats(c.n_head, uint32_t(n), c.capacity);
+        ok = (s->xb = dev_alloc<float>(s, n * c.n_embd)) && (s->residb = dev_alloc<float>(s, n * c.n_embd)) &&
+             (s->qkvb = dev_alloc<float>(s, n * (size_t(s->n_q) + s->n_k + s->n_v))) &&
+             (s->q16b = dev_alloc<uint16_t>(s, n * s->n_q)) && (s->gub = dev_alloc<float>(s, n * 2 * c.n_ff)) &&
+             (s->logitsb = dev_alloc<float>(s, head * c.vocab)) &&
+             (s->wantb = dev_alloc<float>(s, size_t(n < kPassWant ? n : kPassWant) * c.vocab)) &&
+             (s->act_q8b = dev_alloc<int8_t>(s, n * s->max_n_in)) && (s->act_scalesb = dev_alloc<float>(s, n * s->max_n_in / 32)) &&
+             (s->partialb = dev_alloc<Top>(s, head * kArgmaxGroups)) && (s->attn_scratch = dev_alloc<float>(s, s->attn_scratch_floats));
+    }
     if (ok && c.head_dim_k == 128 && c.head_dim_v == 128 && attn128_use_split(c.capacity, c.n_head))
         ok = (s->attn_split = dev_alloc<uint8_t>(s, attn_split_scratch_bytes(c.n_head, c.capacity), true)) != nullptr;
     if (ok && hipStreamSynchronize(rmi_thread_ctx()->stream) != hipSuccess) {  // the uploads enqueued above
@@ -1780,7 +1783,8 @@ int rmi_hip_qwen3_generate(rmi_hip_qwen3 *s, const uint32_t *prompt, uint32_t n_
 int rmi_hip_qwen3_set_prompt_passes(rmi_hip_qwen3 *s, int enabled) {
     if (!s) return rmi_fail(RMI_HIP_E_INVALID, "null session");
     // 0: off; 1: the default size; more: that many positions a pass, up to the buffers' size
-    s->prompt_pass = enabled <= 0 ? 0u : enabled == 1 ? kPromptPassDefault : uint32_t(enabled) < kPromptBatch ? uint32_t(enabled) : kPromptBatch;
+    const uint32_t most = prompt_batch(s->cfg.capacity);
+    s->prompt_pass = enabled <= 0 ? 0u : enabled == 1 || uint32_t(enabled) > most ? most : uint32_t(enabled);
     return RMI_HIP_OK;
 }
 
