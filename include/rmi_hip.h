@@ -454,12 +454,12 @@ void rmi_hip_qwen3_destroy(rmi_hip_qwen3 *s);
 /* Token ids that end generation (the tokenizer's EOS id and "im_end", src/models/qwen3.rs:1123-1130); none by
  * default.  At most 16. */
 int rmi_hip_qwen3_set_stop_ids(rmi_hip_qwen3 *s, const uint32_t *ids, uint32_t n_ids);
-/* Prompt positions are known in advance, so rmi_hip_qwen3_generate takes them up to 512 to a pass (head dimension 128):
+/* Prompt positions are known in advance, so rmi_hip_qwen3_generate takes them up to 1024 to a pass (head dimension 128):
  * every product is one launch for all of them (the x86-64 order's bits for each), and so is everything else; each
  * position's logits, argmax and cache rows are what the step-by-step run gives, bit for bit.
- * enabled = 1 (the default): 512 positions a pass; 0: every position its own step; n > 1: n positions a pass (at
- * most 512).  Measured on a 1999-token prompt of a Qwen3-0.6B model: 1.1 ms a position step by step beyond 1280 keys,
- * 0.02 ms in passes. */
+ * enabled = 1 (the default): 1024 positions a pass; 0: every position its own step; n > 1: n positions a pass (at
+ * most 1024).  Measured on a 1999-token prompt of a Qwen3-0.6B model: 1.1 ms a position step by step beyond 1280 keys,
+ * 0.0145 ms in passes. */
 int rmi_hip_qwen3_set_prompt_passes(rmi_hip_qwen3 *s, int enabled);
 /* Runs up to n_prompt + max_new - 1 steps, one token per step, positions 0.. (the prompt is fed token by
  * token as generate_inner does), greedy sampling (temperature 0, sample_token's argmax branch).  With stop

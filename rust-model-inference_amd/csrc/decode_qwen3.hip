@@ -1236,8 +1236,9 @@ struct rmi_hip_qwen3 : RmiSession {
 namespace {
 
 // Most positions a prompt pass takes, which is also what it takes unless told otherwise.  A pass of 512 gives the
-// attention of sixteen heads two workgroups a compute unit.
-constexpr uint32_t kPromptBatch = 512;
+// attention of sixteen heads two workgroups a compute unit; one of 1024 the products of 1024 rows a workgroup each (a prompt
+// of 1999 tokens: 36.3 ms in passes of 512, 28.9 in passes of 1024).
+constexpr uint32_t kPromptBatch = 1024;
 constexpr uint32_t kHeadBatch = 128;  // positions whose logits are in memory at once
 constexpr uint32_t kPassWant = 64;    // logits of a pass that a caller can ask for
 inline uint32_t prompt_batch(uint32_t capacity) { return capacity < kPromptBatch ? capacity : kPromptBatch; }

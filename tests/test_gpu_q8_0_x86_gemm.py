@@ -1,0 +1,76 @@
+"""Q8_0 products of more than eight tokens in the x86-64 order on the matrix cores: every token's bits are those of the
+eight-token GEMV (held to the oracle by test_gpu_q8_0.py) and, for some tokens, of the restated AVX2 kernel itself."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _run(H, weight, q, s, n_out, stride, first, last):
+    tokens, n_in = q.shape
+    d_q, d_s = H.DeviceBuffer.from_array(q), H.DeviceBuffer.from_array(s)
+    d_y = H.DeviceBuffer.from_array(np.full((tokens, stride), -7.0, np.float32))
+    out = []
+    for group in (tokens, 8):  # the whole batch in one call, and eight at a time through the GEMV
+        for t in range(0, tokens, group):
+            n = min(group, tokens - t)
+            H.check(H.lib.rmi_hip_gemv_q8_0_dev(weight.w.handle, d_q.ptr + t * n_in, d_s.ptr + t * (n_in // 32) * 4, d_y.ptr + t * stride * 4, n, stride,
+                                                first, last, None))
+        H.check(H.lib.rmi_hip_synchronize())
+        out.append(d_y.to_array(np.float32, (tokens, stride)))
+    for b in (d_q, d_s, d_y):
+        b.free()
+    return out
+
+
+@pytest.mark.parametrize("n_in,n_out,tokens", [
+    (32, 40, 9), (96, 8200, 640), (288, 4111, 512), (1024, 1000, 200), (1440, 333, 13), (992, 130, 33), (256, 70000, 16), (256, 70003, 12),
+    (2048, 1024, 512), (3072, 64, 65), (160, 17, 300)])
+def test_batches_have_the_bits_of_the_gemv(hip, oracle, n_in, n_out, tokens):
+    H = hip.hip
+    rng = np.random.default_rng(n_in + n_out + tokens)
+    w = hip.synth.q8_0_weight(n_out, n_out, n_in)
+    kernel = hip.kernel.Q8Kernel(w, n_in, n_out)
+    q = rng.integers(-128, 128, (tokens, n_in), dtype=np.int8)
+    s = rng.uniform(0, 2, (tokens, n_in // 32)).astype(np.float32)
+    whole, eights = _run(H, kernel, q, s, n_out, n_out, 0, n_out)
+    assert np.array_equal(whole.view(np.uint32), eights.view(np.uint32))
+    for t in (0, tokens // 2, tokens - 1):
+        qt = np.maximum(q[t], -127)  # (the restated kernel is the reference's, which is wrong for quants of -128)
+        ref = oracle.matmul_q8_0_quantized(w, qt.view(np.uint8), s[t], n_in, n_out, oracle.AVX2)
+        y = np.zeros(n_out, np.float32)
+        kernel.forward_prequantized(qt.view(np.uint8), s[t], y, n_in, n_out, 0, 1)
+        assert np.array_equal(y.view(np.uint32), ref.view(np.uint32))
+        if (q[t] >= -127).all():
+            assert np.array_equal(whole[t].view(np.uint32), ref.view(np.uint32))
+
+
+@pytest.mark.parametrize("first,last,stride", [(0, 1000, 1003), (3, 997, 1000), (8, 9, 1000), (61, 130, 131), (992, 1000, 1001)])
+def test_row_ranges_and_strides(hip, first, last, stride):
+    """Rows outside the range keep what was there; token strides that are no multiple of sixteen bytes."""
+    rng = np.random.default_rng(first)
+    kernel = hip.kernel.Q8Kernel(hip.synth.q8_0_weight(5, 1000, 352), 352, 1000)
+    q, s = rng.integers(-127, 128, (150, 352), dtype=np.int8), rng.uniform(0, 2, (150, 11)).astype(np.float32)
+    whole, eights = _run(hip.hip, kernel, q, s, 1000, stride, first, last)
+    assert np.array_equal(whole.view(np.uint32), eights.view(np.uint32))
+    outside = np.ones(stride, bool)
+    outside[first:last] = False
+    assert (whole[:, outside] == -7.0).all()
+
+
+def test_special_scales(hip):
+    """Zero, subnormal, huge, infinite and NaN scales of either operand."""
+    rng = np.random.default_rng(1)
+    n_in, n_out, tokens = 320, 200, 130
+    w = hip.synth.q8_0_weight(3, n_out, n_in).reshape(-1, 34)
+    special = np.array([0x0000, 0x8000, 0x0001, 0x7bff, 0x7c00, 0xfc00, 0x7e00], np.uint16)
+    at = rng.choice(w.shape[0], 60, replace=False)
+    w[at, :2] = special[rng.integers(0, special.size, 60)].view(np.uint8).reshape(60, 2)
+    kernel = hip.kernel.Q8Kernel(w.reshape(-1), n_in, n_out)
+    q, s = rng.integers(-127, 128, (tokens, n_in), dtype=np.int8), rng.uniform(0, 2, (tokens, 10)).astype(np.float32)
+    s[rng.integers(0, tokens, 40), rng.integers(0, 10, 40)] = rng.choice(np.array([0.0, -0.0, 1e-40, 3e38, np.inf, -np.inf, np.nan], np.float32), 40)
+    q[7] = 0
+    whole, eights = _run(hip.hip, kernel, q, s, n_out, n_out, 0, n_out)
+    nan = np.isnan(eights)
+    assert np.array_equal(np.isnan(whole), nan)
+    assert np.array_equal(whole.view(np.uint32)[~nan], eights.view(np.uint32)[~nan])
