@@ -21,20 +21,127 @@ __global__ __launch_bounds__(256) void embed_kernel(RmiEmbed e, const uint32_t *
 }
 
 // ------------------------------------------------------------------ GEMM
-// One workgroup of four waves: BN weight rows x BT tokens, k in steps of 128 bytes a row through two LDS buffers; the
-// pieces of the next PD steps are on their way to registers while one is multiplied.  The largest tile keeps one LDS
-// buffer (NB = 1), so that three workgroups share a compute unit.  A row of a buffer is eight
-// 16-byte pieces, piece p at slot p ^ (row & 7), so that the sixteen rows of a fragment spread over the banks.
-// Weights are the A operand: a lane ends with four consecutive rows of one token.
+// Weights are the A operand: a lane ends with four consecutive rows of one token.  k goes in steps of 128 bytes a row
+// through LDS; a row of a buffer is eight 16-byte pieces, piece p at slot p ^ (row & 7), so that the sixteen rows of a
+// fragment spread over the banks.
 constexpr uint32_t kStepBytes = 128;
 constexpr int kResidual = -1;  // the epilogue that adds to the residual stream; the others are RmiEpilogue's
 
+// A wave's results, NN x NT tiles of sixteen rows x sixteen tokens: a lane has rows 4 g .. 4 g + 3 of one token of each.
+// A finished column segment goes to the residual stream at once (each element is one thread's), so that no second set
+// of accumulators is held.  row, tok: of the lane's first value.
+template <int NN, int NT>
+__device__ __forceinline__ void fold_segment(f32x4 (&acc)[NN][NT], const RmiColSeg &s, float *__restrict__ x, uint32_t width, uint32_t n_tokens,
+                                             uint32_t row0, uint32_t tok0) {
+    const bool quads = (width & 3) == 0;
+#pragma unroll
+    for (int j = 0; j < NT; j++) {
+        const uint32_t tok = tok0 + j * 16;
+#pragma unroll
+        for (int i = 0; i < NN; i++) {
+            const uint32_t row = row0 + i * 16;
+            const size_t at = size_t(tok) * width + row;
+            if (tok < n_tokens && row < width) {
+                if (quads) {
+                    f32x4 v = acc[i][j] * s.scale;
+                    if (s.gate) v *= *reinterpret_cast<const f32x4 *>(s.gate + size_t(tok) * s.gate_ld + row);
+                    *reinterpret_cast<f32x4 *>(x + at) += v;
+                } else {
+#pragma unroll
+                    for (int r = 0; r < 4; r++)
+                        if (row + r < width) x[at + r] += acc[i][j][r] * s.scale * (s.gate ? s.gate[size_t(tok) * s.gate_ld + row + r] : 1.0f);
+                }
+            }
+            acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+        }
+    }
+}
+
+// first_row, tok0: of the wave's first tile and the lane's first token
+template <typename T, int EPI, int NN, int NT>
+__device__ __forceinline__ void store_rows(const f32x4 (&acc)[NN][NT], const RmiRowSegs &rs, uint32_t n_rows, uint32_t n_tokens, uint32_t first_row,
+                                           uint32_t tok0, uint32_t g) {
+#pragma unroll
+    for (int i = 0; i < NN; i++) {
+        const uint32_t tile_row = first_row + i * 16;  // a tile of sixteen rows lies in one segment
+        if (tile_row >= n_rows) continue;
+        const RmiRowSeg &s = rs.s[seg_of(rs, tile_row)];
+        const uint32_t r0 = tile_row - s.row0 + g * 4;
+        float bias[4], lower[4];
+        if constexpr (EPI == kRowsActed || EPI == kRowsTimesTable) {
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                bias[r] = s.bias && r0 + r < s.n ? s.bias[r0 + r] : 0.0f;
+                lower[r] = s.lower && r0 + r < s.n ? s.lower[r0 + r] : 0.0f;
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < NT; j++) {
+            const uint32_t tok = tok0 + j * 16;
+            if constexpr (EPI == kRowsPaired) {  // (gate, up) twice: two results
+                if (tok >= n_tokens) continue;
+                const f32x4 z = acc[i][j];
+                const float v0 = fmaxf(z[0], 0.0f) * z[1], v1 = fmaxf(z[2], 0.0f) * z[3];
+                const size_t at = size_t(tok) * s.ld + r0 / 2;
+                if (sizeof(T) == 2 && s.out_elem && r0 + 2 < s.n && (s.ld & 1) == 0) {  // side by side: one store
+                    reinterpret_cast<uint32_t *>(s.y)[at >> 1] = uint32_t(f32_to_bf16(v0)) | uint32_t(f32_to_bf16(v1)) << 16;
+                    continue;
+                }
+#pragma unroll
+                for (uint32_t r = 0; r < 2; r++) {
+                    const float v = r ? v1 : v0;
+                    if (r0 + 2 * r < s.n) {
+                        if (s.out_elem)
+                            static_cast<T *>(s.y)[at + r] = from_f32<T>(v);
+                        else
+                            static_cast<float *>(s.y)[at + r] = v;
+                    }
+                }
+                continue;
+            }
+            f32x4 o = acc[i][j];
+            if constexpr (EPI == kRowsActed || EPI == kRowsTimesTable) {
+#pragma unroll
+                for (int r = 0; r < 4; r++) o[r] = apply_act<T>(s.act, o[r], bias[r], lower[r]);
+            }
+            if (tok >= n_tokens) continue;
+            if constexpr (EPI == kRowsTimesTable) {
+                if (s.mul) {
+                    const T *m = mul_row<T>(s, tok) + r0;
+#pragma unroll
+                    for (uint32_t r = 0; r < 4; r++)
+                        if (r0 + r < s.n) o[r] *= to_f32(m[r]);
+                }
+            }
+            const size_t at = size_t(tok) * s.ld + r0;
+            if (r0 + 3 < s.n && (s.ld & 3) == 0) {
+                if (s.out_elem)
+                    store4(static_cast<T *>(s.y) + at, o);
+                else
+                    store4(static_cast<float *>(s.y) + at, o);
+            } else {
+#pragma unroll
+                for (int r = 0; r < 4; r++)
+                    if (r0 + r < s.n) {
+                        if (s.out_elem)
+                            static_cast<T *>(s.y)[at + r] = from_f32<T>(o[r]);
+                        else
+                            static_cast<float *>(s.y)[at + r] = o[r];
+                    }
+            }
+        }
+    }
+}
+
+// Small tiles, for products that would leave compute units idle otherwise: four waves, two LDS buffers; the pieces of the
+// next PD steps are on their way to registers while one is multiplied.
 template <typename T, int BN, int BT, int WN, int WT, int PD, int NB, int WPS, int EPI>
 __global__ __launch_bounds__(256, WPS) void dense_gemm_kernel(const T *__restrict__ w, const T *__restrict__ a, uint32_t n_rows,
                                                               uint32_t k_pad, uint32_t ld, uint32_t n_tokens, uint32_t grid_n, uint32_t grid_t, uint32_t xcd_split,
                                                          RmiRowSegs rs, RmiColSegs cs, float *__restrict__ x, uint32_t width) {
     constexpr bool RESIDUAL = EPI == kResidual;
     static_assert((BN / WN) * (BT / WT) == 4, "four waves");
+    static_assert(NB == 2, "two buffers");
     static_assert(kDenseKAlign * sizeof(T) % (kStepBytes * PD) == 0, "whole rounds of the register slots");
     constexpr int NN = WN / 16, NT = WT / 16;
     constexpr int PW = BN * 8 / 256, PA = (BT * 8 + 255) / 256;  // pieces a thread loads per step
@@ -86,34 +193,6 @@ __global__ __launch_bounds__(256, WPS) void dense_gemm_kernel(const T *__restric
         for (int i = 0; i < PA; i++) lds[buf][adst[i]] = ra[slot][i];
     };
     const uint32_t fr = lane & 15, g = lane >> 4;
-    // a finished column segment goes to the residual stream at once (each element is one thread's), so that no second
-    // set of accumulators is held
-    auto fold = [&](const RmiColSeg &s) {
-        if constexpr (RESIDUAL) {
-            const bool quads = (width & 3) == 0;
-#pragma unroll
-            for (int j = 0; j < NT; j++) {
-                const uint32_t tok = tok0 + wt + j * 16 + fr;
-#pragma unroll
-                for (int i = 0; i < NN; i++) {
-                    const uint32_t row = row0 + wn + i * 16 + g * 4;
-                    const size_t at = size_t(tok) * width + row;
-                    if (tok < n_tokens && row < width) {
-                        if (quads) {
-                            f32x4 v = acc[i][j] * s.scale;
-                            if (s.gate) v *= *reinterpret_cast<const f32x4 *>(s.gate + size_t(tok) * s.gate_ld + row);
-                            *reinterpret_cast<f32x4 *>(x + at) += v;
-                        } else {
-#pragma unroll
-                            for (int r = 0; r < 4; r++)
-                                if (row + r < width) x[at + r] += acc[i][j][r] * s.scale * (s.gate ? s.gate[size_t(tok) * s.gate_ld + row + r] : 1.0f);
-                        }
-                    }
-                    acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-                }
-            }
-        }
-    };
 #pragma unroll
     for (int j = 0; j < PD; j++) {
         load(j, j);
@@ -149,103 +228,216 @@ __global__ __launch_bounds__(256, WPS) void dense_gemm_kernel(const T *__restric
 #pragma unroll
                         for (int i2 = 0; i2 < NT; i2++) acc[i][i2] = mma16<T>(fw[i], fa[i2], acc[i][i2]);
                 }
-                if (NB == 1) __syncthreads();
                 park((j + 1) % PD, buf ^ (NB - 1));  // (behind the last step: that step again, read by nobody)
                 load((j + 1) % PD, step + j + 1 + PD);
                 __syncthreads();
             }
         }
-        if (RESIDUAL) fold(cs.s[seg]);
+        if constexpr (RESIDUAL) fold_segment<NN, NT>(acc, cs.s[seg], x, width, n_tokens, row0 + wn + g * 4, tok0 + wt + fr);
     }
 
-    if constexpr (!RESIDUAL) {
+    if constexpr (!RESIDUAL) store_rows<T, EPI, NN, NT>(acc, rs, n_rows, n_tokens, row0 + wn, tok0 + wt + fr, g);
+}
+
+// s_waitcnt's operand: at most vm loads outstanding, and no LDS instruction
+constexpr int rmi_waitcnt(int vm) { return (vm & 15) | (vm >> 4) << 14 | 7 << 4; }
+
+// The same product with wider tiles and eight waves, so that a piece read from LDS feeds more products and the operands
+// cross the L2 less often.  Steps go from memory straight into LDS (the swizzle is on the source side: a lane fetches the
+// piece that belongs at its slot) through NB buffers, one barrier a step: behind it the next step's first half is read while
+// the second half of this one is multiplied, and the buffer that everybody has read takes the step NB on.  The wait in front
+// of the barrier counts the loads in flight, so that those of NB - 2 steps stay under way.
+// What bounds it: LDS, 128 bytes a clock (a step of 128 x 256 reads 128 KB and writes 48: 0.6 us; its products alone would
+// take 0.43), and on a full chip the way from L2 (10 TB/s in 48 KB steps of 1.1 us).
+template <typename T, int BN, int BT, int WN, int WT, int NB, int WPS, int EPI>
+__global__ __launch_bounds__(64 * (BN / WN) * (BT / WT), WPS) void dense_gemm_wide_kernel(const T *__restrict__ w, const T *__restrict__ a, uint32_t n_rows, uint32_t k_pad,
+                                                                 uint32_t ld, uint32_t n_tokens, uint32_t grid_n, uint32_t grid_t, uint32_t xcd_split,
+                                                                 RmiRowSegs rs, RmiColSegs cs, float *__restrict__ x, uint32_t width) {
+    constexpr bool RESIDUAL = EPI == kResidual;
+    constexpr int NN = WN / 16, NT = WT / 16, WAVES = (BN / WN) * (BT / WT);
+    constexpr int FW = BN / (8 * WAVES), FA = BT / (8 * WAVES);  // kilobytes a wave fetches of either operand per step: eight rows each
+    __shared__ u32x4 buf0[(BN + BT) * 8], buf1[(BN + BT) * 8], buf2[NB == 3 ? (BN + BT) * 8 : 1];
+    const uint32_t tid = threadIdx.x, lane = tid & 63, wave = uint32_t(__builtin_amdgcn_readfirstlane(int(tid >> 6)));
+    uint32_t n_tile, t_tile;
+    rmi_gemm_tile_of(blockIdx.x, grid_n, grid_t, 1u, xcd_split, n_tile, t_tile);
+    const uint32_t row0 = n_tile * BN, tok0 = t_tile * BT;
+    const uint32_t wn = (wave % (BN / WN)) * WN, wt = (wave / (BN / WN)) * WT;
+    const uint32_t stride = ld * uint32_t(sizeof(T));
+
+    typedef const uint8_t __attribute__((address_space(1))) *gptr_u8;
+    typedef __attribute__((address_space(3))) void *lptr;
+    const gptr_u8 w_base = as_global<gptr_u8>(reinterpret_cast<const uint8_t *>(w) + size_t(row0) * stride);
+    const gptr_u8 a_base = as_global<gptr_u8>(reinterpret_cast<const uint8_t *>(a) + size_t(tok0) * stride);
+    uint32_t w_off[FW], a_off[FA];
+    const uint32_t piece = ((lane & 7) ^ (lane >> 3)) * 16;  // of row lane >> 3 of eight, at slot lane & 7
 #pragma unroll
-        for (int i = 0; i < NN; i++) {
-            const uint32_t tile_row = row0 + wn + i * 16;  // a tile of sixteen rows lies in one segment
-            if (tile_row >= n_rows) continue;
-            const RmiRowSeg &s = rs.s[seg_of(rs, tile_row)];
-            const uint32_t r0 = tile_row - s.row0 + g * 4;
-            float bias[4], lower[4];
-            if constexpr (EPI == kRowsActed || EPI == kRowsTimesTable) {
+    for (int i = 0; i < FW; i++) {
+        const uint32_t r = (i * WAVES + wave) * 8 + (lane >> 3);
+        w_off[i] = (row0 + r < n_rows ? r : n_rows - 1 - row0) * stride + piece;  // rows past the end are read again and not stored
+    }
 #pragma unroll
-                for (int r = 0; r < 4; r++) {
-                    bias[r] = s.bias && r0 + r < s.n ? s.bias[r0 + r] : 0.0f;
-                    lower[r] = s.lower && r0 + r < s.n ? s.lower[r0 + r] : 0.0f;
-                }
+    for (int i = 0; i < FA; i++) {
+        const uint32_t r = (i * WAVES + wave) * 8 + (lane >> 3);
+        a_off[i] = (tok0 + r < n_tokens ? r : n_tokens - 1 - tok0) * stride + piece;
+    }
+    constexpr uint32_t kStepElems = kStepBytes / sizeof(T);
+    const uint32_t n_steps = k_pad / kStepElems;
+    auto fetch = [&](u32x4 *buf, uint32_t step) {
+        const uint32_t at = (step < n_steps ? step : n_steps - 1) * kStepBytes;  // (behind the last step: that one again, read by nobody)
+#pragma unroll
+        for (int i = 0; i < FW; i++)
+            __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)(w_base + (w_off[i] + at)), (lptr)(buf + (i * WAVES + wave) * 64), 16, 0, 0);
+#pragma unroll
+        for (int i = 0; i < FA; i++)
+            __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)(a_base + (a_off[i] + at)), (lptr)(buf + BN * 8 + (i * WAVES + wave) * 64), 16, 0, 0);
+    };
+    const uint32_t fr = lane & 15, g = lane >> 4;
+    f32x4 acc[NN][NT];
+#pragma unroll
+    for (int i = 0; i < NN; i++)
+#pragma unroll
+        for (int j = 0; j < NT; j++) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    u32x4 fw[2][NN], fa[2][NT];
+    auto read = [&](const u32x4 *buf, int c) {
+        const uint32_t slot = (c * 4 + g) ^ (fr & 7);
+#pragma unroll
+        for (int i = 0; i < NN; i++) fw[c][i] = buf[(wn + i * 16 + fr) * 8 + slot];
+#pragma unroll
+        for (int j = 0; j < NT; j++) fa[c][j] = buf[BN * 8 + (wt + j * 16 + fr) * 8 + slot];
+    };
+    auto multiply = [&](int c) {
+#pragma unroll
+        for (int i = 0; i < NN; i++)
+#pragma unroll
+            for (int j = 0; j < NT; j++) acc[i][j] = mma16<T>(fw[c][i], fa[c][j], acc[i][j]);
+    };
+    // the products stay on their side of what surrounds them
+    auto pin = [&]() {
+#pragma unroll
+        for (int i = 0; i < NN; i++)
+#pragma unroll
+            for (int j = 0; j < NT; j += 2) asm volatile("" : "+v"(acc[i][j]), "+v"(acc[i][j + 1]));
+    };
+    static_assert(NT % 2 == 0, "pinned two at a time");
+    static_assert(NB == 2 || NB == 3, "two or three buffers");
+    auto step_of = [&](u32x4 *cur, u32x4 *next, uint32_t step) {
+        read(cur, 1);
+        multiply(0);
+        pin();
+        // this step is in everybody's registers, the next one in LDS; the loads of the one after it stay in flight
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_waitcnt(rmi_waitcnt((NB - 2) * (FW + FA)));
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        read(next, 0);
+        fetch(cur, step + NB);
+        multiply(1);
+        pin();
+    };
+    fetch(buf0, 0);
+    fetch(buf1, 1);
+    if constexpr (NB == 3) fetch(buf2, 2);
+    __builtin_amdgcn_s_waitcnt(rmi_waitcnt((NB - 1) * (FW + FA)));
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    read(buf0, 0);
+    uint32_t step = 0;
+    if constexpr (NB == 2) {
+        for (uint32_t seg = 0; seg < (RESIDUAL ? cs.n_segs : 1u); seg++) {
+            const uint32_t seg_end = RESIDUAL ? cs.s[seg].k_end / kStepElems : n_steps;  // a multiple of four
+            for (; step < seg_end; step += 2) {
+                step_of(buf0, buf1, step);
+                step_of(buf1, buf0, step + 1);
             }
-#pragma unroll
-            for (int j = 0; j < NT; j++) {
-                const uint32_t tok = tok0 + wt + j * 16 + fr;
-                if constexpr (EPI == kRowsPaired) {  // (gate, up) twice: two results
-                    if (tok >= n_tokens) continue;
-#pragma unroll
-                    for (uint32_t r = 0; r < 2; r++) {
-                        const float v = fmaxf(acc[i][j][2 * r], 0.0f) * acc[i][j][2 * r + 1];
-                        const size_t at = size_t(tok) * s.ld + r0 / 2 + r;
-                        if (r0 + 2 * r < s.n) {
-                            if (s.out_elem)
-                                static_cast<T *>(s.y)[at] = from_f32<T>(v);
-                            else
-                                static_cast<float *>(s.y)[at] = v;
-                        }
-                    }
-                    continue;
-                }
-                f32x4 o = acc[i][j];
-                if constexpr (EPI == kRowsActed || EPI == kRowsTimesTable) {
-#pragma unroll
-                    for (int r = 0; r < 4; r++) o[r] = apply_act<T>(s.act, o[r], bias[r], lower[r]);
-                }
-                if (tok >= n_tokens) continue;
-                if constexpr (EPI == kRowsTimesTable) {
-                    if (s.mul) {
-                        const T *m = mul_row<T>(s, tok) + r0;
-#pragma unroll
-                        for (uint32_t r = 0; r < 4; r++)
-                            if (r0 + r < s.n) o[r] *= to_f32(m[r]);
-                    }
-                }
-                const size_t at = size_t(tok) * s.ld + r0;
-                if (r0 + 3 < s.n && (s.ld & 3) == 0) {
-                    if (s.out_elem)
-                        store4(static_cast<T *>(s.y) + at, o);
-                    else
-                        store4(static_cast<float *>(s.y) + at, o);
-                } else {
-#pragma unroll
-                    for (int r = 0; r < 4; r++)
-                        if (r0 + r < s.n) {
-                            if (s.out_elem)
-                                static_cast<T *>(s.y)[at + r] = from_f32<T>(o[r]);
-                            else
-                                static_cast<float *>(s.y)[at + r] = o[r];
-                        }
-                }
+            if constexpr (RESIDUAL) fold_segment<NN, NT>(acc, cs.s[seg], x, width, n_tokens, row0 + wn + g * 4, tok0 + wt + fr);
+        }
+    } else {
+        uint32_t seg = 0, seg_end = RESIDUAL ? cs.s[0].k_end / kStepElems : n_steps;
+        auto ended = [&]() {  // the step just made was the last one
+            if (++step < seg_end) return false;
+            if constexpr (RESIDUAL) {
+                fold_segment<NN, NT>(acc, cs.s[seg], x, width, n_tokens, row0 + wn + g * 4, tok0 + wt + fr);
+                if (++seg < cs.n_segs) seg_end = cs.s[seg].k_end / kStepElems;
             }
+            return step == n_steps;
+        };
+        for (;;) {
+            step_of(buf0, buf1, step);
+            if (ended()) break;
+            step_of(buf1, buf2, step);
+            if (ended()) break;
+            step_of(buf2, buf0, step);
+            if (ended()) break;
         }
     }
+    if constexpr (!RESIDUAL) store_rows<T, EPI, NN, NT>(acc, rs, n_rows, n_tokens, row0 + wn, tok0 + wt + fr, g);
+}
+
+// Which tile a product takes: the least of estimates, in microseconds, that were fitted to 13 shapes (1024..39040 rows of
+// 1024..20480 columns) with 128..2048 tokens.  A tile costs what a step of k takes a compute unit that holds so many of
+// them (w = tiles over compute units).  bf16 is bound by LDS reads and the traffic between L2 and the compute units, so wider
+// tiles are cheaper an element as long as there are enough of them; f32 is bound by the matrix cores and every tile costs its
+// area, so that only the unevenness of the last round counts.  E.g. in bf16, us by 64 x 64 | 64 x 128 | 128 x 128 | 128 x 256 |
+// 256 x 256: 39040 x 4096, 2048 tokens (four-wave 128 x 128 tiles before: 812) - | 1095 | 813 | 741 | 640; 4096 x 20480, 2048
+// tokens (440 before) - | 479 | 360 | 340 | 521; 2048 x 6144, 1024 tokens 53 | 42 | 65 | 74 | 133; 12288 x 2048, 512 tokens
+// 53 | 39 | 33 | 36 | 55; 1024 x 6144, 512 tokens 21 | 37 | 64 | 74 | 133.
+enum DenseTile { kTile64x16, kTile64x32, kTile64x64, kTile64x128, kTile128x128, kTile128x256, kTile256x256 };
+DenseTile dense_tile_of(bool bf16, uint32_t n_rows, uint32_t n_tokens, uint32_t n_steps) {
+    if (n_tokens <= 16) return kTile64x16;
+    const double cus = rmi_device_cus() > 0 ? rmi_device_cus() : 1;
+    DenseTile best = kTile64x32;
+    double least = 1e30;
+    // us of a step: alone a compute unit, slope beyond; per round of `fit` tiles a compute unit
+    auto consider = [&](DenseTile t, uint32_t bn, uint32_t bt, double fixed, double base, double slope, double fit) {
+        const double w = double((n_rows + bn - 1) / bn) * ((n_tokens + bt - 1) / bt) / cus;
+        const double rounds = double(uint64_t(w / fit)), rest = w - rounds * fit;
+        double step;
+        if (!bf16)
+            step = base * double(uint64_t(w + 0.999));
+        else
+            step = rounds * (base + slope * (fit - 1)) + (rest > 0 ? base + slope * (rest > 1 ? rest - 1 : 0.0) : 0.0);
+        const double us = fixed + n_steps * step;
+        if (us < least) least = us, best = t;
+    };
+    if (bf16) {
+        consider(kTile64x32, 64, 32, 3, 0.17, 0.17, 4);
+        consider(kTile64x64, 64, 64, 4, 0.28, 0.25, 4);
+        consider(kTile64x128, 64, 128, 4, 0.39, 0.27, 2);
+        consider(kTile128x128, 128, 128, 5, 0.68, 0.54, 2);
+        consider(kTile128x256, 128, 256, 7, 1.08, 0, 1);
+        consider(kTile256x256, 256, 256, 8, 1.95, 0, 1);
+    } else {
+        consider(kTile64x32, 64, 32, 3, 0.31, 0, 1);
+        consider(kTile64x64, 64, 64, 4, 0.56, 0, 1);
+        consider(kTile64x128, 64, 128, 4, 0.95, 0, 1);
+        consider(kTile128x128, 128, 128, 5, 1.84, 0, 1);
+    }
+    return best;
 }
 
 template <typename T, int EPI>
 int launch_gemm(const RmiDense &w, const void *a, const RmiRowSegs &rs, const RmiColSegs &cs, float *x, uint32_t width,
                 uint32_t n_tokens, hipStream_t st) {
     const uint32_t n_rows = EPI == kResidual ? width : w.n_rows;
-    auto go = [&](auto kernel, uint32_t bn, uint32_t bt) {
+    auto go = [&](auto kernel, uint32_t bn, uint32_t bt, uint32_t threads = 256) {
         const uint32_t gn = (n_rows + bn - 1) / bn, gt = (n_tokens + bt - 1) / bt;
         const uint32_t split = rmi_gemm_xcd_split(gn, gt, double(n_rows) * w.k_pad, double(n_tokens) * w.k_pad);
-        hipLaunchKernelGGL(kernel, dim3(gn * gt), dim3(256), 0, st, static_cast<const T *>(w.data), static_cast<const T *>(a), n_rows,
+        hipLaunchKernelGGL(kernel, dim3(gn * gt), dim3(threads), 0, st, static_cast<const T *>(w.data), static_cast<const T *>(a), n_rows,
                            w.k_pad, w.ld, n_tokens, gn, gt, split, rs, cs, x, width);
     };
-    const uint64_t cus = uint64_t(rmi_device_cus());
-    auto tiles = [&](uint32_t bn, uint32_t bt) { return uint64_t((n_rows + bn - 1) / bn) * ((n_tokens + bt - 1) / bt); };
-    if (n_tokens <= 16)
-        go(dense_gemm_kernel<T, 64, 16, 16, 16, 4, 2, 4, EPI>, 64, 16);
-    else if (tiles(128, 128) >= 2 * cus)
-        go(dense_gemm_kernel<T, 128, 128, 64, 64, 1, 1, 3, EPI>, 128, 128);
-    else if (tiles(64, 64) >= cus)
-        go(dense_gemm_kernel<T, 64, 64, 32, 32, 4, 2, 4, EPI>, 64, 64);
-    else
-        go(dense_gemm_kernel<T, 64, 32, 32, 16, 4, 2, 4, EPI>, 64, 32);
+    switch (dense_tile_of(sizeof(T) == 2, n_rows, n_tokens, uint32_t(w.k_pad * sizeof(T) / kStepBytes))) {
+    case kTile64x16: go(dense_gemm_kernel<T, 64, 16, 16, 16, 4, 2, 4, EPI>, 64, 16); break;
+    case kTile64x32: go(dense_gemm_kernel<T, 64, 32, 32, 16, 4, 2, 4, EPI>, 64, 32); break;
+    case kTile64x64: go(dense_gemm_kernel<T, 64, 64, 32, 32, 4, 2, 4, EPI>, 64, 64); break;
+    case kTile64x128: go(dense_gemm_wide_kernel<T, 64, 128, 32, 32, 3, 2, EPI>, 64, 128, 512); break;
+    case kTile128x128: go(dense_gemm_wide_kernel<T, 128, 128, 64, 32, 2, 4, EPI>, 128, 128, 512); break;
+    case kTile128x256:
+        if constexpr (sizeof(T) == 2) go(dense_gemm_wide_kernel<T, 128, 256, 64, 64, 3, 2, EPI>, 128, 256, 512);
+        break;
+    case kTile256x256:
+        if constexpr (sizeof(T) == 2) go(dense_gemm_wide_kernel<T, 256, 256, 128, 64, 2, 2, EPI>, 256, 256, 512);
+        break;
+    }
     RMI_HIP_CHECK(hipGetLastError());
     return RMI_HIP_OK;
 }
