@@ -1,5 +1,6 @@
 // Mixers over time (seq_mixers.h): kernels for passes of several tokens and for single tokens.
 #include "seq_mixers.h"
+#include <type_traits>
 
 #include "device_conv.h"
 #include "device_dense.h"
@@ -249,19 +250,21 @@ struct AttnWave {
             for (uint32_t v = 0; v < kVT; v++) o[i][v] = f32x4{0.f, 0.f, 0.f, 0.f};
         }
     }
-    // a block's keys and values fit in registers beside the rest: values of a block and keys of the next are under way
-    // while the block's scores and weights are computed
-    static constexpr bool kAhead = BUCKET * sizeof(T) <= 256;
-    u32x4 kf[2][kAhead ? kKC : 1], vf[kAhead ? kVT * (sizeof(T) / 2) : 1];
+    // A block's keys and values fit in registers beside the rest: values of a block and keys of the next are under way
+    // while the block's scores and weights are computed.  Every load is made, a piece past a narrower head's end as the
+    // last one again: a load behind a branch, even one that all lanes take, is waited for before the next is issued.
+    static constexpr bool kAhead = BUCKET * sizeof(T) <= 256 || (QT == 1 && BUCKET * sizeof(T) <= 512);
+    static constexpr uint32_t kVP = sizeof(T) / 2;  // pieces a lane holds of a value tile
+    u32x4 kf[2][kAhead ? kKC : 1], vf[kAhead ? kVT * kVP : 1];
 
     __device__ __forceinline__ void load_keys(const T *kc, const RmiAttnShape &s, uint32_t k) {
         const uint32_t lane = threadIdx.x & 63, n_kc = s.dk_pad / (4 * kPieceElems<T>);
         const T *row = kc + size_t(k + (lane & 15)) * s.dk_pad + (lane >> 4) * kPieceElems<T>;
 #pragma unroll
         for (uint32_t c = 0; c < (kAhead ? kKC : 0); c++) {
-            if (c >= n_kc) continue;
-            kf[0][c] = *reinterpret_cast<const u32x4 *>(row + c * 4 * kPieceElems<T>);
-            kf[1][c] = *reinterpret_cast<const u32x4 *>(row + c * 4 * kPieceElems<T> + 16 * size_t(s.dk_pad));
+            const T *p = row + (c < n_kc ? c : n_kc - 1) * 4 * kPieceElems<T>;
+            kf[0][c] = *reinterpret_cast<const u32x4 *>(p);
+            kf[1][c] = *reinterpret_cast<const u32x4 *>(p + 16 * size_t(s.dk_pad));
         }
     }
     __device__ __forceinline__ const T *value_at(const T *vc, const RmiAttnShape &s, uint32_t k) {
@@ -274,8 +277,44 @@ struct AttnWave {
 #pragma unroll
         for (uint32_t v = 0; v < (kAhead ? kVT : 0); v++)
 #pragma unroll
-            for (uint32_t t = 0; t < sizeof(T) / 2; t++)
-                if (v < n_vt) vf[v * (sizeof(T) / 2) + t] = *reinterpret_cast<const u32x4 *>(vb + size_t(v) * 16 * kKeyBlock + t * 16);
+            for (uint32_t t = 0; t < kVP; t++)
+                vf[v * kVP + t] = *reinterpret_cast<const u32x4 *>(vb + size_t(v < n_vt ? v : n_vt - 1) * 16 * kKeyBlock + t * 16);
+    }
+    // key o of the loaded block and its value come from LDS: a token's own, which this launch makes
+    __device__ __forceinline__ void put_own(const T *key, const T *value, const RmiAttnShape &s, uint32_t o) {
+        const uint32_t lane = threadIdx.x & 63, fr = lane & 15, g = lane >> 4, n_kc = s.dk_pad / (4 * kPieceElems<T>), n_vt = s.dv_pad / 16;
+        const bool k0 = fr == o, k1 = fr + 16 == o;
+#pragma unroll
+        for (uint32_t c = 0; c < (kAhead ? kKC : 0); c++) {
+            const u32x4 x = *reinterpret_cast<const u32x4 *>(key + ((c < n_kc ? c : 0) * 4 + g) * kPieceElems<T>);
+            kf[0][c] = k0 ? x : kf[0][c];
+            kf[1][c] = k1 ? x : kf[1][c];
+        }
+        const uint32_t slot = value_slot<T>(o), in_piece = slot % kPieceElems<T> * sizeof(T);  // bytes
+        const uint32_t bits = sizeof(T) == 4 ? ~0u : 0xffffu << 8 * (in_piece & 2);
+        uint32_t mask[kVP][4];
+#pragma unroll
+        for (uint32_t t = 0; t < kVP; t++)
+#pragma unroll
+            for (uint32_t e = 0; e < 4; e++) mask[t][e] = slot / kPieceElems<T> == t * 4 + g && in_piece / 4 == e ? bits : 0;
+#pragma unroll
+        for (uint32_t v = 0; v < (kAhead ? kVT : 0); v++) {
+            const T raw = value[(v < n_vt ? v : 0) * 16 + fr];
+            uint32_t x;
+            if constexpr (sizeof(T) == 4)
+                x = __builtin_bit_cast(uint32_t, raw);
+            else
+                x = uint32_t(__builtin_bit_cast(uint16_t, raw)) * 0x10001u;
+#pragma unroll
+            for (uint32_t t = 0; t < kVP; t++)
+#pragma unroll
+                for (uint32_t e = 0; e < 4; e++) vf[v * kVP + t][e] = (vf[v * kVP + t][e] & ~mask[t][e]) | (x & mask[t][e]);
+        }
+    }
+    // the row of the key that lies `back` positions before the one in row `own` (back < 2 capacity)
+    static __device__ __forceinline__ uint32_t row_of(const RmiAttnShape &s, uint32_t own, uint32_t back) {
+        back = back < s.capacity ? back : back - s.capacity;
+        return own >= back ? own - back : own + s.capacity - back;
     }
     // keys [k0, k1), k0 a multiple of 32; column i sees keys up to last[i] (< k1 not required) and, with a window, from
     // last[i] - window + 1 on.  loaded: the first block's keys and values are in kf and vf
@@ -288,6 +327,8 @@ struct AttnWave {
         if (!loaded && k0 < k1) load_keys(kc, s, row);
         for (uint32_t k = k0; k < k1; k += kKeyBlock) {
             const T *vb = value_at(vc, s, row);
+            constexpr uint32_t kGroup = 4;  // pieces of each half under way together where a block does not fit
+            u32x4 kg[2][kAhead ? 1 : kGroup], vg[kAhead ? 1 : kGroup * kVP];
             if (!loaded || k != k0) load_values(vc, s, row);
             const uint32_t next = row + kKeyBlock < s.capacity ? row + kKeyBlock : 0;
             f32x4 sc[QT][2];
@@ -295,16 +336,16 @@ struct AttnWave {
             for (int i = 0; i < QT; i++) sc[i][0] = sc[i][1] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (uint32_t c = 0; c < kKC; c++) {
-                if (c >= n_kc) continue;
-                u32x4 f0, f1;
-                if constexpr (kAhead) {
-                    f0 = kf[0][c];
-                    f1 = kf[1][c];
-                } else {
-                    const T *p = krow + size_t(row) * s.dk_pad + c * 4 * kPieceElems<T>;
-                    f0 = *reinterpret_cast<const u32x4 *>(p);
-                    f1 = *reinterpret_cast<const u32x4 *>(p + 16 * size_t(s.dk_pad));
+                if constexpr (!kAhead) if (c % kGroup == 0) {
+#pragma unroll
+                    for (uint32_t j = 0; j < kGroup; j++) {
+                        const T *p = krow + size_t(row) * s.dk_pad + (c + j < n_kc ? c + j : n_kc - 1) * 4 * kPieceElems<T>;
+                        kg[0][j] = *reinterpret_cast<const u32x4 *>(p);
+                        kg[1][j] = *reinterpret_cast<const u32x4 *>(p + 16 * size_t(s.dk_pad));
+                    }
                 }
+                if (c >= n_kc) continue;
+                const u32x4 f0 = kAhead ? kf[0][kAhead ? c : 0] : kg[0][kAhead ? 0 : c % kGroup], f1 = kAhead ? kf[1][kAhead ? c : 0] : kg[1][kAhead ? 0 : c % kGroup];
 #pragma unroll
                 for (int i = 0; i < QT; i++) {
                     sc[i][0] = mma16<T>(f0, qf[i][c], sc[i][0]);
@@ -353,11 +394,17 @@ struct AttnWave {
             }
 #pragma unroll
             for (uint32_t v = 0; v < kVT; v++) {
+                if constexpr (!kAhead) if (v % kGroup == 0) {
+#pragma unroll
+                    for (uint32_t j = 0; j < kGroup * kVP; j++) {
+                        const uint32_t tile = v + j / kVP;
+                        vg[j] = *reinterpret_cast<const u32x4 *>(vb + size_t(tile < n_vt ? tile : n_vt - 1) * 16 * kKeyBlock + j % kVP * 16);
+                    }
+                }
                 if (v >= n_vt) continue;
 #pragma unroll
-                for (uint32_t t = 0; t < sizeof(T) / 2; t++) {
-                    const u32x4 f = kAhead ? vf[kAhead ? v * (sizeof(T) / 2) + t : 0]
-                                           : *reinterpret_cast<const u32x4 *>(vb + size_t(v) * 16 * kKeyBlock + t * 16);
+                for (uint32_t t = 0; t < kVP; t++) {
+                    const u32x4 f = kAhead ? vf[kAhead ? v * kVP + t : 0] : vg[kAhead ? 0 : v % kGroup * kVP + t];
 #pragma unroll
                     for (int i = 0; i < QT; i++) o[i][v] = mma16<T>(f, pf[i][t], o[i][v]);
                 }
@@ -402,8 +449,7 @@ __global__ __launch_bounds__(256) void attn_pass_kernel(RmiAttnShape s, RmiAttnA
         const T *q = static_cast<const T *>(a.q) + (size_t(kvh) * n_cols + cc) * s.dk_pad + g4 * kPieceElems<T>;
 #pragma unroll
         for (uint32_t c = 0; c < w.kKC; c++) {
-            if (c >= n_kc) continue;
-            w.qf[i][c] = *reinterpret_cast<const u32x4 *>(q + c * 4 * kPieceElems<T>);
+            w.qf[i][c] = *reinterpret_cast<const u32x4 *>(q + (c < n_kc ? c : 0) * 4 * kPieceElems<T>);
         }
     }
     const uint32_t first_col = tile * QT * 16, live = n_cols - first_col < QT * 16 ? n_cols - first_col : QT * 16;
@@ -455,130 +501,162 @@ constexpr uint32_t kStepThreads = 256;  // a workgroup of the single-token launc
 // a part: the columns' maxima, their sums, and [column][channel]
 __host__ __device__ inline uint32_t attn_part_floats(uint32_t dv_pad) { return 16 * (dv_pad + 2); }
 
+// What a workgroup's place follows from, divided out on the host: a division by a number that only the launch knows is
+// some thirty dependent instructions, and ten of them stood before a token's first load.
+struct Div {
+    uint32_t by, m;
+    Div() = default;
+    explicit Div(uint32_t d) : by(d), m(uint32_t((uint64_t(1) << 31) / d + 1)) {}
+    __device__ __forceinline__ uint32_t quot(uint32_t x) const { return __umulhi(2 * x, m); }  // x by < 2^31
+};
+struct SplitPlan {
+    Div parts, tiles, group, half, dv_pad;
+    uint32_t keys_per_part, own;  // own: the row of the first token's key
+};
+
 template <typename T, int BUCKET, bool STEP>
-__device__ __forceinline__ void attn_split(const RmiAttnShape &s, const RmiAttnArgs &a, uint32_t block, uint32_t parts, uint32_t keys_per_part,
-                                           uint8_t *lds, uint32_t *flag) {
-    constexpr uint32_t NW = 4;
+__device__ __forceinline__ void attn_split(const RmiAttnShape &s, const RmiAttnArgs &a, uint32_t block, const SplitPlan &plan, uint8_t *lds,
+                                           uint32_t *flag) {
+    constexpr uint32_t NW = 4, NT = 256;
+    const uint32_t parts = plan.parts.by, tiles = plan.tiles.by, group = plan.group.by, keys_per_part = plan.keys_per_part;
     const uint32_t tid = threadIdx.x, lane = tid & 63, wave = uint32_t(__builtin_amdgcn_readfirstlane(int(tid >> 6))), fr = lane & 15, g4 = lane >> 4;
-    const uint32_t group = s.heads / s.kv_heads, n_cols = a.n_tokens * group, tiles = (n_cols + 15) / 16;
-    const uint32_t part = block % parts, ct = (block / parts) % tiles, kvh = block / parts / tiles;
+    const uint32_t n_cols = STEP ? group : a.n_tokens * group, slot = plan.parts.quot(block), part = block - slot * parts;
+    const uint32_t kvh = plan.tiles.quot(slot), ct = slot - kvh * tiles;
     const uint32_t last_col = ct * 16 + 15 < n_cols ? ct * 16 + 15 : n_cols - 1;
-    const uint32_t begin = first_block(s, a.pos0 + ct * 16 / group), n_keys = a.pos0 + last_col / group + 1;  // what the tile sees
+    auto token_of = [&](uint32_t column) { return STEP ? 0 : plan.group.quot(column); };
+    const uint32_t begin = first_block(s, a.pos0 + token_of(ct * 16)), n_keys = a.pos0 + token_of(last_col) + 1;  // what the tile sees
     const uint32_t n_kc = s.dk_pad / (4 * kPieceElems<T>);
     AttnWave<T, BUCKET, 1> w;
     w.init();
     const uint32_t col = ct * 16 + fr, cc = col < n_cols ? col : n_cols - 1;
-    const int last[1] = {int(a.pos0 + cc / group)};
+    const int last[1] = {int(a.pos0 + token_of(cc))};
     const T *kc = static_cast<const T *>(a.k_cache) + size_t(kvh) * s.capacity * s.dk_pad;
     const T *vc = static_cast<const T *>(a.v_cache) + size_t(kvh) * s.capacity * s.dv_pad;
     const uint32_t p0 = begin + part * keys_per_part, p1 = p0 + keys_per_part < n_keys ? p0 + keys_per_part : n_keys;
-    const uint32_t per_wave = keys_per_part / NW;  // a multiple of the key block
+    const uint32_t per_wave = (keys_per_part + NW * kKeyBlock - 1) / (NW * kKeyBlock) * kKeyBlock;
     const uint32_t k0 = p0 + wave * per_wave, k1 = k0 + per_wave < p1 ? k0 + per_wave : p1;
+    const uint32_t live = n_cols - ct * 16 < 16 ? n_cols - ct * 16 : 16, pairs_out = live * s.dv_pad;
+    auto gate_at = [&](uint32_t e) {
+        const uint32_t mc = ct * 16 + plan.dv_pad.quot(e < pairs_out ? e : 0), t = token_of(mc);
+        return a.gate ? a.gate + size_t(t) * s.heads + kvh * group + mc - t * group : a.u;
+    };
+    float gate0 = *gate_at(tid);  // of the first result that this thread may write: under way from here on
     bool loaded = false;
     if constexpr (STEP) {
-        T *q = reinterpret_cast<T *>(lds);
+        T *q = reinterpret_cast<T *>(lds), *own_k = q + 16 * s.dk_pad, *own_v = own_k + s.dk_pad;
         const uint32_t channels = (s.heads + s.kv_heads) * s.dim + s.kv_heads * s.vdim;
         const ConvCtx x{a.u, a.hist_in, a.conv, channels, s.taps};
         const uint32_t half = s.dk_pad / 2, c_end = n_cols - ct * 16 < 16 ? n_cols - ct * 16 : 16;
-        const uint32_t own = a.pos0 % s.capacity;
+        const uint32_t own = plan.own;
         const bool newest = a.pos0 - p0 < keys_per_part;  // this part holds the token's own key and value
-        // the first block of keys and values: under way behind the convolution's operands, unless it holds the new one
-        auto ahead = [&] {
-            loaded = w.kAhead && k0 < k1 && k0 + kKeyBlock < n_keys;
-            if (loaded) {
-                w.load_keys(kc, s, k0 % s.capacity);
-                w.load_values(vc, s, k0 % s.capacity);
-            }
-        };
         if (conv_pairs_fit(s)) {
             // with the new key and value to make, the last two waves make them and the others the queries
-            const uint32_t q_threads = newest ? 128 : 256, rot = s.rot_dims / 2;
-            const bool is_k = newest && wave == 2, is_v = newest && wave == 3;
+            const uint32_t q_threads = newest ? NT - 128 : NT, rot = s.rot_dims / 2;
+            const bool is_k = newest && wave == NW - 2, is_v = newest && wave == NW - 1;
             const uint32_t n_pairs = is_v ? s.vdim / 2 : is_k ? half : c_end * half, step = is_k || is_v ? 64 : q_threads;
-            bool first = true;
-            for (uint32_t e0 = 0; e0 < n_pairs || first; e0 += step) {
+            const bool keeps = is_k || is_v ? ct == 0 : part == 0;  // the one of all workgroups that carries the history on
+            auto pairs = [&](uint32_t e0, auto first) {
                 const uint32_t e = e0 + (is_k || is_v ? lane : tid), ec = e < n_pairs ? e : 0;
-                const uint32_t c = is_k || is_v ? 0 : ec / half, i = is_k || is_v ? ec : ec % half;
+                const uint32_t c = is_k || is_v ? 0 : plan.half.quot(ec), i = ec - c * half;
                 const bool has = e < n_pairs && (is_v || 2 * i < s.dim);
                 const uint32_t c0 = is_v   ? (s.heads + s.kv_heads) * s.dim + kvh * s.vdim
                                     : is_k ? (s.heads + kvh) * s.dim
                                            : (kvh * group + ct * 16 + c) * s.dim;
                 const uint32_t ch = c0 + (has ? 2 * i : 0);
-                PairTaps t;
+                // the operands, every one by a load of its own that no branch guards (rows and taps that are not there by
+                // loads of others, dropped), and behind them the first block of keys and values
                 float2 r[4];
+                float w0[4], w1[4];
+                const uint32_t off = 4 - s.taps;
 #pragma unroll
-                for (uint32_t j = 0; j < 4; j++) r[j] = pair_row(s, a, channels, 0, 3 - j, ch);
-                t.load(s, a.conv, ch);
+                for (uint32_t j = 0; j < 4; j++) {  // position pos0 - 3 + j: history row j - off
+                    const float *row = j < 3 && j >= off ? a.hist_in + size_t(j - off) * channels : a.u;
+                    r[j] = *reinterpret_cast<const float2 *>(row + ch);
+                    w0[j] = a.conv[ch * s.taps + (j >= off ? j - off : 0)];
+                    w1[j] = a.conv[(ch + 1) * s.taps + (j >= off ? j - off : 0)];
+                }
                 const bool turned = has && !is_v && i < rot;
                 const size_t at = size_t(a.pos0) * rot + (turned ? i : 0);
-                const float cs = turned ? a.cos_t[at] : 1.0f, sn = turned ? a.sin_t[at] : 0.0f;
-                if (first) ahead();
-                first = false;
+                const float cs = *(rot ? a.cos_t + at : a.u), sn = *(rot ? a.sin_t + at : a.u);
+                if constexpr (w.kAhead && first.value) {  // (a wave without keys reads some that are there, and drops them)
+                    const uint32_t row = w.row_of(s, own, a.pos0 - (k0 < k1 ? k0 : begin));
+                    w.load_keys(kc, s, row);
+                    w.load_values(vc, s, row);
+                }
                 float p = 0.0f, o = 0.0f;
 #pragma unroll
                 for (uint32_t j = 0; j < 4; j++) {
-                    p = __builtin_fmaf(t.w0[j], r[j].x, p);
-                    o = __builtin_fmaf(t.w1[j], r[j].y, o);
+                    const bool there = has && j >= off && a.pos0 + j >= 3;
+                    p = __builtin_fmaf(there ? w0[j] : 0.0f, there ? r[j].x : 0.0f, p);
+                    o = __builtin_fmaf(there ? w1[j] : 0.0f, there ? r[j].y : 0.0f, o);
                 }
-                if (!has) p = o = 0.0f;
+                if (keeps && has) {
+#pragma unroll
+                    for (uint32_t j = 1; j < 4; j++)
+                        if (j > off) *reinterpret_cast<float2 *>(a.hist_out + size_t(j - 1 - off) * channels + ch) = r[j];
+                }
                 if (is_v) {  // (at most 64 pairs: one round)
                     const float f = s.v_norm ? 1.0f / sqrtf(wave_sum_f32(__builtin_fmaf(p, p, o * o)) / float(s.vdim) + s.eps) : 1.0f;
                     T *blk = const_cast<T *>(vc) + size_t(own / kKeyBlock) * s.dv_pad * kKeyBlock + value_slot<T>(own % kKeyBlock);
                     if (has) {
-                        blk[size_t(2 * i) * kKeyBlock] = from_f32<T>(p * f);
-                        blk[size_t(2 * i + 1) * kKeyBlock] = from_f32<T>(o * f);
+                        const T v0 = from_f32<T>(p * f), v1 = from_f32<T>(o * f);
+                        blk[size_t(2 * i) * kKeyBlock] = v0;
+                        blk[size_t(2 * i + 1) * kKeyBlock] = v1;
+                        own_v[2 * i] = v0;
+                        own_v[2 * i + 1] = v1;
                     }
+                    for (uint32_t d = s.vdim + lane; d < s.dv_pad; d += 64) own_v[d] = from_f32<T>(0.0f);
                 } else if (e < n_pairs) {
                     const float rp = p;
-                    p = __builtin_fmaf(rp, cs, -(o * sn));
-                    o = __builtin_fmaf(o, cs, rp * sn);
-                    store_pair(is_k ? const_cast<T *>(kc) + size_t(own) * s.dk_pad + 2 * i : q + c * s.dk_pad + 2 * i, p, o);
+                    p = turned ? __builtin_fmaf(rp, cs, -(o * sn)) : p;
+                    o = turned ? __builtin_fmaf(o, cs, rp * sn) : o;
+                    if (is_k) store_pair(const_cast<T *>(kc) + size_t(own) * s.dk_pad + 2 * i, p, o);
+                    store_pair(is_k ? own_k + 2 * i : q + c * s.dk_pad + 2 * i, p, o);
                 }
-            }
+            };
+            pairs(0, std::true_type{});
+            for (uint32_t e0 = step; e0 < n_pairs; e0 += step) pairs(e0, std::false_type{});
+            loaded = w.kAhead;
         } else {
             if (newest) {
                 if (wave == NW - 2) key_row<T>(x, s, a, 0, kvh, lane);
                 if (wave == NW - 1) value_row<T>(x, s, a, 0, kvh, lane);
             }
-            for (uint32_t e = tid; e < c_end * half; e += 256) {
-                const uint32_t c = e / half, i = e % half, head = kvh * group + ct * 16 + c;
+            for (uint32_t e = tid; e < c_end * half; e += NT) {
+                const uint32_t c = plan.half.quot(e), i = e - c * half, head = kvh * group + ct * 16 + c;
                 float p, r;
                 conv_rotate_pair(x, s, a.cos_t, a.sin_t, 0, a.pos0, head * s.dim, i, p, r);
                 store_pair(q + c * s.dk_pad + 2 * i, p, r);
             }
+            if (part == 0) {  // the history of this workgroup's channels
+                const uint32_t h0 = (kvh * group + ct * 16) * s.dim;
+                for (uint32_t d = tid; d < c_end * s.dim; d += NT) conv_carry(x, a.hist_out, 1, h0 + d);
+                if (ct == 0) {
+                    for (uint32_t d = tid; d < s.dim; d += NT) conv_carry(x, a.hist_out, 1, (s.heads + kvh) * s.dim + d);
+                    for (uint32_t d = tid; d < s.vdim; d += NT)
+                        conv_carry(x, a.hist_out, 1, (s.heads + s.kv_heads) * s.dim + kvh * s.vdim + d);
+                }
+            }
         }
         __syncthreads();
+        if (loaded && a.pos0 - k0 < kKeyBlock) w.put_own(own_k, own_v, s, a.pos0 - k0);
         const uint32_t qc = fr < c_end ? fr : c_end - 1;
 #pragma unroll
         for (uint32_t c = 0; c < w.kKC; c++) {
-            if (c >= n_kc) continue;
-            w.qf[0][c] = *reinterpret_cast<const u32x4 *>(q + qc * s.dk_pad + (c * 4 + g4) * kPieceElems<T>);
+            w.qf[0][c] = *reinterpret_cast<const u32x4 *>(q + qc * s.dk_pad + ((c < n_kc ? c : 0) * 4 + g4) * kPieceElems<T>);
         }
         __syncthreads();
     } else {
         const T *q = static_cast<const T *>(a.q) + (size_t(kvh) * n_cols + cc) * s.dk_pad + g4 * kPieceElems<T>;
 #pragma unroll
         for (uint32_t c = 0; c < w.kKC; c++) {
-            if (c >= n_kc) continue;
-            w.qf[0][c] = *reinterpret_cast<const u32x4 *>(q + c * 4 * kPieceElems<T>);
+            w.qf[0][c] = *reinterpret_cast<const u32x4 *>(q + (c < n_kc ? c : 0) * 4 * kPieceElems<T>);
         }
     }
+    asm volatile("" : "+v"(gate0));
     if (k0 < k1) w.keys(kc, vc, s, k0, k1, last, loaded);
-    if constexpr (STEP) {
-        if (part == 0) {  // the history of this workgroup's channels
-            const uint32_t channels = (s.heads + s.kv_heads) * s.dim + s.kv_heads * s.vdim;
-            const ConvCtx x{a.u, a.hist_in, a.conv, channels, s.taps};
-            const uint32_t c_end = n_cols - ct * 16 < 16 ? n_cols - ct * 16 : 16, c0 = (kvh * group + ct * 16) * s.dim;
-            for (uint32_t d = tid; d < c_end * s.dim; d += 256) conv_carry(x, a.hist_out, 1, c0 + d);
-            if (ct == 0) {
-                for (uint32_t d = tid; d < s.dim; d += 256) conv_carry(x, a.hist_out, 1, (s.heads + kvh) * s.dim + d);
-                for (uint32_t d = tid; d < s.vdim; d += 256)
-                    conv_carry(x, a.hist_out, 1, (s.heads + s.kv_heads) * s.dim + kvh * s.vdim + d);
-            }
-        }
-    }
     // the waves' results to LDS, live columns only; then every thread merges (column, channel) pairs
-    const uint32_t live = n_cols - ct * 16 < 16 ? n_cols - ct * 16 : 16, pf = attn_part_floats(s.dv_pad), pl = 32 + live * s.dv_pad;
+    const uint32_t pf = attn_part_floats(s.dv_pad), pl = 32 + live * s.dv_pad;
     float *all = reinterpret_cast<float *>(lds), *mine = all + wave * pl;
     const float l = rows_sum_f32(w.l[0]);
     if (fr < live) {
@@ -591,18 +669,16 @@ __device__ __forceinline__ void attn_split(const RmiAttnShape &s, const RmiAttnA
             if (v * 16 < s.dv_pad) *reinterpret_cast<f32x4 *>(mine + 32 + fr * s.dv_pad + v * 16 + g4 * 4) = w.o[0][v];
     }
     __syncthreads();
-    const uint32_t slot = kvh * tiles + ct;
     float *ws = reinterpret_cast<float *>(static_cast<uint32_t *>(a.scratch) + kAttnCounters) + size_t(slot) * parts * pf;
-    const uint32_t pairs = live * s.dv_pad;
     auto finish = [&](uint32_t e, float o, float sum) {
-        const uint32_t c = e / s.dv_pad, d = e % s.dv_pad;
+        const uint32_t c = plan.dv_pad.quot(e), d = e - c * s.dv_pad;
         if (d >= s.vdim) return;
-        const uint32_t mc = ct * 16 + c, t = mc / group, head = kvh * group + mc % group;
-        static_cast<T *>(a.out)[size_t(t) * a.out_ld + size_t(head) * s.vdim + d] =
-            from_f32<T>(o * ((a.gate ? a.gate[size_t(t) * s.heads + head] : 1.0f) / sum));
+        const uint32_t mc = ct * 16 + c, t = token_of(mc), head = kvh * group + mc - t * group;
+        const float g = e == tid ? gate0 : *gate_at(e);
+        static_cast<T *>(a.out)[size_t(t) * a.out_ld + size_t(head) * s.vdim + d] = from_f32<T>(o * ((a.gate ? g : 1.0f) / sum));
     };
-    for (uint32_t e = tid; e < pairs; e += 256) {
-        const uint32_t c = e / s.dv_pad;
+    for (uint32_t e = tid; e < pairs_out; e += NT) {
+        const uint32_t c = plan.dv_pad.quot(e);
         float m = all[c];
 #pragma unroll
         for (uint32_t i = 1; i < NW; i++) m = fmaxf(m, all[i * pl + c]);
@@ -618,7 +694,7 @@ __device__ __forceinline__ void attn_split(const RmiAttnShape &s, const RmiAttnA
             finish(e, o, sum);
         } else {
             float *dst = ws + size_t(part) * pf;
-            if (e % s.dv_pad == 0) {
+            if (e == c * s.dv_pad) {
                 __hip_atomic_store(dst + c, m, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 __hip_atomic_store(dst + 16 + c, sum, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             }
@@ -639,8 +715,8 @@ __device__ __forceinline__ void attn_split(const RmiAttnShape &s, const RmiAttnA
     }
     __syncthreads();
     if (!*flag) return;
-    for (uint32_t e = tid; e < pairs; e += 256) {
-        const uint32_t c = e / s.dv_pad;
+    for (uint32_t e = tid; e < pairs_out; e += NT) {
+        const uint32_t c = plan.dv_pad.quot(e);
         float m = -INFINITY, sum = 0.0f, o = 0.0f;
         for (uint32_t p0 = 0; p0 < parts; p0 += 8) {  // eight parts' loads at a time
             float mv[8], lv[8], ov[8];
@@ -671,10 +747,10 @@ __device__ __forceinline__ void attn_split(const RmiAttnShape &s, const RmiAttnA
 }
 
 template <typename T, int BUCKET>
-__global__ __launch_bounds__(256) void attn_split_kernel(RmiAttnShape s, RmiAttnArgs a, uint32_t parts, uint32_t keys_per_part) {
+__global__ __launch_bounds__(256) void attn_split_kernel(RmiAttnShape s, RmiAttnArgs a, SplitPlan plan) {
     extern __shared__ __attribute__((aligned(16))) uint8_t lds_raw[];
     __shared__ uint32_t flag;
-    attn_split<T, BUCKET, false>(s, a, blockIdx.x, parts, keys_per_part, lds_raw, &flag);
+    attn_split<T, BUCKET, false>(s, a, blockIdx.x, plan, lds_raw, &flag);
 }
 
 // ---- gated linear recurrence
@@ -683,40 +759,59 @@ template <typename T>
 __device__ __forceinline__ void recur_step(const RmiRecurShape &s, const RmiRecurArgs &a, uint32_t head, float *lds) {
     const uint32_t tid = threadIdx.x, quads = s.v_pad / 4, slices = kStepThreads / quads;
     float *fs = lds, *qs = fs + s.d_pad, *vs = qs + s.d_pad, *part = vs + s.v_pad;  // part [slices][v_pad]
-    for (uint32_t d = tid; d < s.d_pad; d += kStepThreads) {
-        fs[d] = d < s.dim ? a.f[head * s.dim + d] : 1.0f;
-        qs[d] = d < s.dim ? a.q[head * s.dim + d] : 0.0f;
-    }
-    for (uint32_t d = tid; d < s.v_pad; d += kStepThreads) vs[d] = d < s.vdim ? a.v[head * s.vdim + d] : 0.0f;
-    __syncthreads();
     const uint32_t c = tid % quads, sl = tid / quads;
+    const size_t at = size_t(head) * s.d_pad * s.v_pad + c * 4;
+    const float *st = a.state_in + at;
+    float *st_out = a.state_out + at;
+    // eight state rows of a thread in flight, the first ones beside this token's gates and values (unconditional: a row
+    // past the end is the last one again; the first token of a sequence reads what it then drops)
+    constexpr uint32_t kRows = 16;
+    f32x4 r[kRows];
+#define RECUR_LOAD_ROWS(d0)                                                                                                             \
+    _Pragma("unroll") for (uint32_t j = 0; j < kRows; j++) {                                                                            \
+        const uint32_t d = (d0) + j * slices;                                                                                           \
+        r[j] = *reinterpret_cast<const f32x4 *>(st + size_t(d < s.d_pad ? d : s.d_pad - 1) * s.v_pad);                                   \
+    }
+    const uint32_t d1 = tid < s.dim ? tid : 0, e1 = tid < s.vdim ? tid : 0;  // (a head's sizes are at most the number of threads)
+    float f1 = a.f[head * s.dim + d1], q1 = a.q[head * s.dim + d1], v1 = a.v[head * s.vdim + e1], norm = a.norm[e1];
+    RECUR_LOAD_ROWS(sl)
+    asm volatile("" : "+v"(f1), "+v"(q1), "+v"(v1), "+v"(norm));  // (else the loads move into the branches below, behind the rows)
+    if (tid < s.d_pad) {
+        fs[tid] = tid < s.dim ? f1 : 1.0f;
+        qs[tid] = tid < s.dim ? q1 : 0.0f;
+    }
+    if (tid < s.v_pad) vs[tid] = tid < s.vdim ? v1 : 0.0f;
+    __syncthreads();
     f32x4 o = {0.f, 0.f, 0.f, 0.f};
     if (sl < slices) {
-        const size_t at = size_t(head) * s.d_pad * s.v_pad + c * 4;
-        const float *st = a.state_in + at;
-        float *st_out = a.state_out + at;
         const f32x4 v = *reinterpret_cast<const f32x4 *>(vs + c * 4);
-        for (uint32_t d0 = sl; d0 < s.d_pad; d0 += slices * 8) {  // eight rows in flight
-            f32x4 r[8];
+        for (uint32_t d0 = sl; d0 < s.d_pad; d0 += slices * kRows) {
+            if (d0 != sl) {
+                RECUR_LOAD_ROWS(d0)
+            }
+            float fr[kRows], qr[kRows];
 #pragma unroll
-            for (uint32_t j = 0; j < 8; j++) {
-                const uint32_t d = d0 + j * slices;
-                r[j] = f32x4{0.f, 0.f, 0.f, 0.f};
-                if (a.pos0 && d < s.d_pad) r[j] = *reinterpret_cast<const f32x4 *>(st + size_t(d) * s.v_pad);
+            for (uint32_t j = 0; j < kRows; j++) {
+                const uint32_t d = d0 + j * slices < s.d_pad ? d0 + j * slices : s.d_pad - 1;
+                fr[j] = fs[d];
+                qr[j] = qs[d];
             }
 #pragma unroll
-            for (uint32_t j = 0; j < 8; j++) {
+            for (uint32_t j = 0; j < kRows; j++) {
                 const uint32_t d = d0 + j * slices;
-                if (d >= s.d_pad) break;
-                const float f = fs[d], k = 1.0f - f, q = qs[d];
+                if (d < s.d_pad) {
+                    const float f = fr[j], k = 1.0f - f, q = qr[j];
+                    f32x4 n;
 #pragma unroll
-                for (int e = 0; e < 4; e++) {
-                    r[j][e] = __builtin_fmaf(f, r[j][e], k * v[e]);
-                    o[e] = __builtin_fmaf(q, r[j][e], o[e]);
+                    for (int e = 0; e < 4; e++) {
+                        n[e] = __builtin_fmaf(f, a.pos0 ? r[j][e] : 0.0f, k * v[e]);
+                        o[e] = __builtin_fmaf(q, n[e], o[e]);
+                    }
+                    *reinterpret_cast<f32x4 *>(st_out + size_t(d) * s.v_pad) = n;
                 }
-                *reinterpret_cast<f32x4 *>(st_out + size_t(d) * s.v_pad) = r[j];
             }
         }
+#undef RECUR_LOAD_ROWS
         *reinterpret_cast<f32x4 *>(part + sl * s.v_pad + c * 4) = o;
     }
     __syncthreads();
@@ -730,20 +825,26 @@ __device__ __forceinline__ void recur_step(const RmiRecurShape &s, const RmiRecu
     float total = 0.0f;
 #pragma unroll
     for (uint32_t i = 0; i < kStepThreads / 64; i++) total += red[i];
-    const float r = 1.0f / sqrtf(total / float(s.vdim) + s.eps);
-    if (tid < s.vdim) static_cast<T *>(a.out)[size_t(head) * s.vdim + tid] = from_f32<T>(mine * r * a.norm[tid]);
+    const float scale = 1.0f / sqrtf(total / float(s.vdim) + s.eps);
+    if (tid < s.vdim) static_cast<T *>(a.out)[size_t(head) * s.vdim + tid] = from_f32<T>(mine * scale * norm);
 }
 inline size_t recur_step_lds(const RmiRecurShape &s) {
     return (2 * size_t(s.d_pad) + s.v_pad + size_t(kStepThreads / (s.v_pad / 4)) * s.v_pad) * 4;
 }
 
+// A token's mixers of a layer.  It moves little (some 100 KB a head) and is bound by round trips to memory, 1.5 us each as
+// everything here was pushed out by the weights: the arguments, the operands with the first keys, values and state rows, the
+// parts' stores, their count and their loads.  So all that does not depend on another load is under way at once and no
+// division stands before it: 28 layers of 16 heads over 8 of 128 elements, 150 positions, bf16: 12.7 us a launch with loads
+// behind branches, 10.0 as it is; f32, 16 key/value heads and 310 positions: 17.6 and 14.8.  Parts of 64 or of 32 keys, and
+// eight waves a workgroup for 256 keys without a second workgroup, all took as long or longer.
 template <typename T, int BUCKET>
-__global__ __launch_bounds__(kStepThreads) void mixers_step_kernel(RmiAttnShape s, RmiAttnArgs a, uint32_t attn_blocks, uint32_t parts,
-                                                          uint32_t keys_per_part, RmiRecurShape rs, RmiRecurArgs ra) {
+__global__ __launch_bounds__(kStepThreads) void mixers_step_kernel(RmiAttnShape s, RmiAttnArgs a, uint32_t attn_blocks, SplitPlan plan,
+                                                                   RmiRecurShape rs, RmiRecurArgs ra) {
     extern __shared__ __attribute__((aligned(16))) uint8_t lds_raw[];
     __shared__ uint32_t flag;
     if (blockIdx.x < attn_blocks)
-        attn_split<T, BUCKET, true>(s, a, blockIdx.x, parts, keys_per_part, lds_raw, &flag);
+        attn_split<T, BUCKET, true>(s, a, blockIdx.x, plan, lds_raw, &flag);
     else
         recur_step<T>(rs, ra, blockIdx.x - attn_blocks, reinterpret_cast<float *>(lds_raw));
 }
@@ -954,22 +1055,29 @@ __global__ __launch_bounds__(256) void recur_norm_kernel(RmiRecurShape s, RmiRec
 }
 
 // ------------------------------------------------------------------ launches
-// Keys over workgroups where the columns alone would not fill the chip; at most kMaxParts parts of 128 keys or more.
+// Keys over workgroups where the columns alone would not fill the chip; at most kMaxParts parts of about 128 keys or more.
 constexpr uint32_t kSplitMaxCols = 256;  // per key/value head
-void attn_parts(const RmiAttnShape &s, uint32_t n_tokens, uint32_t n_keys, uint32_t *parts, uint32_t *keys_per_part) {
+SplitPlan attn_parts(const RmiAttnShape &s, uint32_t n_tokens, uint32_t pos0) {
+    uint32_t n_keys = pos0 + n_tokens;
     const uint32_t group = s.heads / s.kv_heads, tiles = (n_tokens * group + 15) / 16;
     // the most that a tile of sixteen columns sees, from a block's edge on
     const uint64_t seen = s.window ? uint64_t(s.window) + 15 / group + 1 + kKeyBlock : n_keys;
     if (seen < n_keys) n_keys = uint32_t(seen);
     const uint32_t slots = s.kv_heads * tiles, cus = uint32_t(rmi_device_cus());
-    uint32_t p = (n_keys + 127) / 128;
+    uint32_t p = (n_keys + 4 * kKeyBlock - 1) / (4 * kKeyBlock);
     const uint32_t fill = (cus + slots - 1) / slots;
     if (p > fill) p = fill;
     if (p > kMaxParts) p = kMaxParts;
     if (slots > kAttnCounters || p < 1) p = 1;
-    const uint32_t align = 4 * kKeyBlock;  // each wave whole value blocks
-    *keys_per_part = ((n_keys + p - 1) / p + align - 1) / align * align;
-    *parts = (n_keys + *keys_per_part - 1) / *keys_per_part;
+    SplitPlan plan;
+    plan.keys_per_part = ((n_keys + p - 1) / p + kKeyBlock - 1) / kKeyBlock * kKeyBlock;
+    plan.parts = Div((n_keys + plan.keys_per_part - 1) / plan.keys_per_part);
+    plan.tiles = Div(tiles);
+    plan.group = Div(group);
+    plan.half = Div(s.dk_pad / 2);
+    plan.dv_pad = Div(s.dv_pad);
+    plan.own = pos0 % s.capacity;
+    return plan;
 }
 
 int check_attn(const RmiAttnShape &s, const RmiAttnArgs &a) {
@@ -986,7 +1094,7 @@ uint32_t bucket_of(const RmiAttnShape &s) {
 }
 size_t split_lds(uint32_t elem_bytes, const RmiAttnShape &s, uint32_t n_tokens) {
     const uint32_t cols = n_tokens * (s.heads / s.kv_heads), live = cols < 16 ? cols : 16;
-    const size_t q = size_t(16) * s.dk_pad * elem_bytes, merge = size_t(4) * (32 + live * s.dv_pad) * 4;
+    const size_t q = (size_t(17) * s.dk_pad + s.dv_pad) * elem_bytes, merge = size_t(4) * (32 + live * s.dv_pad) * 4;
     return q > merge ? q : merge;
 }
 
@@ -1000,13 +1108,12 @@ int attn_pass(const RmiAttnShape &s, const RmiAttnArgs &a, hipStream_t st) {
         hipLaunchKernelGGL(conv_rotate_kernel<T>, conv_grid, dim3(256), 0, st, s, a);
     const uint32_t bucket = bucket_of(s);
     if (n_cols <= kSplitMaxCols) {
-        uint32_t parts, kpp;
-        attn_parts(s, a.n_tokens, a.pos0 + a.n_tokens, &parts, &kpp);
-        const dim3 grid(s.kv_heads * ((n_cols + 15) / 16) * parts);
+        const SplitPlan plan = attn_parts(s, a.n_tokens, a.pos0);
+        const dim3 grid(s.kv_heads * plan.tiles.by * plan.parts.by);
         const size_t lds = split_lds(sizeof(T), s, a.n_tokens);
         auto go = [&](auto kernel) {
             const int rc = rmi_allow_lds(kernel, lds);
-            if (rc == RMI_HIP_OK) hipLaunchKernelGGL(kernel, grid, dim3(256), lds, st, s, a, parts, kpp);
+            if (rc == RMI_HIP_OK) hipLaunchKernelGGL(kernel, grid, dim3(256), lds, st, s, a, plan);
             return rc;
         };
         const int rc = bucket == 64 ? go(attn_split_kernel<T, 64>) : bucket == 128 ? go(attn_split_kernel<T, 128>) : go(attn_split_kernel<T, 256>);
@@ -1041,11 +1148,12 @@ int mixers_step(const RmiAttnShape *as, const RmiAttnArgs *aa, const RmiRecurSha
     const RmiAttnArgs a = aa ? *aa : RmiAttnArgs{};
     const RmiRecurShape r = rs ? *rs : RmiRecurShape{};
     const RmiRecurArgs b = ra ? *ra : RmiRecurArgs{};
-    uint32_t parts = 1, kpp = 0, blocks = 0;
+    SplitPlan plan{};
+    uint32_t blocks = 0;
     size_t lds = 0;
     if (as) {
-        attn_parts(s, 1, a.pos0 + 1, &parts, &kpp);
-        blocks = s.kv_heads * ((s.heads / s.kv_heads + 15) / 16) * parts;
+        plan = attn_parts(s, 1, a.pos0);
+        blocks = s.kv_heads * plan.tiles.by * plan.parts.by;
         lds = split_lds(sizeof(T), s, 1);
     }
     if (rs && recur_step_lds(r) > lds) lds = recur_step_lds(r);
@@ -1053,7 +1161,7 @@ int mixers_step(const RmiAttnShape *as, const RmiAttnArgs *aa, const RmiRecurSha
     const uint32_t bucket = as ? bucket_of(s) : 64;
     auto go = [&](auto kernel) {
         const int rc = rmi_allow_lds(kernel, lds);
-        if (rc == RMI_HIP_OK) hipLaunchKernelGGL(kernel, grid, dim3(kStepThreads), lds, st, s, a, blocks, parts, kpp, r, b);
+        if (rc == RMI_HIP_OK) hipLaunchKernelGGL(kernel, grid, dim3(kStepThreads), lds, st, s, a, blocks, plan, r, b);
         return rc;
     };
     const int rc = bucket == 64 ? go(mixers_step_kernel<T, 64>) : bucket == 128 ? go(mixers_step_kernel<T, 128>) : go(mixers_step_kernel<T, 256>);
