@@ -2,6 +2,10 @@
 // elementwise work in their epilogue.
 #include "dense_launch.h"
 
+#include "device_args.h"
+
+#include <type_traits>
+
 namespace {
 
 // The activation sits in LDS, zero past its end, so that a piece past the end of a row (the last one is read again)
@@ -25,9 +29,12 @@ struct GemvPair {
     GemvProblem p[2];
 };
 
-// A wave takes ROWS weight rows, its lanes the pieces of a row, two rounds of 64 in flight; R: quads of the input a
+template <typename T>
+using UintOf = std::conditional_t<sizeof(T) == 4, uint32_t, uint16_t>;
+
+// A wave takes ROWS weight rows, its lanes the pieces of a row, U rounds of 64 in flight; R: quads of the input a
 // thread keeps (n <= 1024 R).
-template <typename T, int NORM, bool ADD, int ROWS, int R>
+template <typename T, int NORM, bool ADD, int ROWS, int R, int U>
 __device__ __forceinline__ void gemv_block(const GemvProblem &p, uint32_t block, u32x4 *act, float *red) {
     const uint32_t tid = threadIdx.x, lane = tid & 63, k_pad = p.k_pad;
     const uint32_t row0 = (block * 4 + uint32_t(__builtin_amdgcn_readfirstlane(int(tid >> 6)))) * ROWS;
@@ -42,32 +49,44 @@ __device__ __forceinline__ void gemv_block(const GemvProblem &p, uint32_t block,
         const uint32_t row = row0 + r < rs.n_rows ? row0 + r : rs.n_rows - 1;
         src[r] = reinterpret_cast<const u32x4 *>(w + size_t(row) * p.ld);
     }
-    u32x4 cur[2][ROWS];
+    u32x4 cur[U][ROWS];
     auto load = [&](uint32_t p0) {
 #pragma unroll
-        for (int u = 0; u < 2; u++) {
+        for (int u = 0; u < U; u++) {
             const uint32_t at = p0 + u * 64 + lane;
 #pragma unroll
             for (int r = 0; r < ROWS; r++) cur[u][r] = src[r][at < pieces ? at : pieces - 1];
         }
     };
-    load(0);
     const RmiRowSeg seg = rs.s[seg_of(rs, row0)];
+    // what the epilogue reads goes out here, too: at the end it would be one more wait for memory, or two.  No branch guards
+    // a load (there is always an input to read); lanes without a row read the segment's first.
+    const float *no_vector = p.in.x;
+    uint32_t tok = *(seg.mul ? seg.mul_tok : reinterpret_cast<const uint32_t *>(no_vector));
+    load(0);
+    uint32_t at = row0 + lane - seg.row0;
+    const uint32_t at_e = uint32_t(lane) < ROWS && at < seg.n ? at : 0;
+    float bias = *(seg.bias ? seg.bias + at_e : no_vector), lower = *(seg.lower ? seg.lower + at_e : no_vector);
+    tok = seg.mul && tok >= seg.mul_rows ? seg.mul_rows - 1 : tok;  // ids past the end read the last row
+    T mul = *(seg.mul ? static_cast<const T *>(seg.mul) + size_t(tok) * seg.mul_ld + at_e : reinterpret_cast<const T *>(no_vector));
     in.finish(p.in, 0, p.in.x_out && block == 0, red);
     in.store(p.in, 0, reinterpret_cast<T *>(act), padded * kPieceElems<T>);
     __syncthreads();
+    uint32_t mul_bits = __builtin_bit_cast(UintOf<T>, mul);
+    asm volatile("" : "+v"(bias), "+v"(lower), "+v"(mul_bits));  // (else these loads move to the end again)
     float acc[ROWS];
 #pragma unroll
     for (int r = 0; r < ROWS; r++) acc[r] = 0.0f;
-    for (uint32_t p0 = 0; p0 < pieces; p0 += 128) {
-        u32x4 now[2][ROWS];
+    for (uint32_t p0 = 0; p0 < pieces; p0 += 64 * U) {
+        u32x4 now[U][ROWS];
 #pragma unroll
-        for (int u = 0; u < 2; u++)
+        for (int u = 0; u < U; u++)
 #pragma unroll
             for (int r = 0; r < ROWS; r++) now[u][r] = cur[u][r];
-        if (p0 + 128 < pieces) load(p0 + 128);
+        if (p0 + 64 * U < pieces) load(p0 + 64 * U);
 #pragma unroll
-        for (int u = 0; u < 2; u++) {
+        for (int u = 0; u < U; u++) {
+            if (64 * U > kGemvRound && p0 + u * 64 >= padded) break;
             const u32x4 hv = act[p0 + u * 64 + lane];
 #pragma unroll
             for (int r = 0; r < ROWS; r++) acc[r] = dot_piece<T>(now[u][r], hv, acc[r]);
@@ -79,7 +98,6 @@ __device__ __forceinline__ void gemv_block(const GemvProblem &p, uint32_t block,
         const float s = wave_sum_f32(acc[r]);
         if (lane == uint32_t(r)) mine = s;
     }
-    uint32_t at = row0 + lane - seg.row0;
     float o;
     bool mine_to_store = lane < ROWS && row0 + lane < rs.n_rows && at < seg.n;
     if (ROWS % 2 == 0 && seg.act == kActReluGlu) {  // (gate, up) pairs in neighbouring lanes
@@ -88,8 +106,8 @@ __device__ __forceinline__ void gemv_block(const GemvProblem &p, uint32_t block,
         at >>= 1;
     } else {
         if (!mine_to_store) return;
-        o = apply_act<T>(seg.act, mine, seg.bias ? seg.bias[at] : 0.0f, seg.lower ? seg.lower[at] : 0.0f);
-        if (seg.mul) o *= to_f32(mul_row<T>(seg, 0)[at]);
+        o = apply_act<T>(seg.act, mine, seg.bias ? bias : 0.0f, seg.lower ? lower : 0.0f);
+        if (seg.mul) o *= to_f32(__builtin_bit_cast(T, UintOf<T>(mul_bits)));
     }
     if (!mine_to_store) return;
     if (seg.out_elem)
@@ -98,40 +116,39 @@ __device__ __forceinline__ void gemv_block(const GemvProblem &p, uint32_t block,
         static_cast<float *>(seg.y)[at] = o;
 }
 
-template <typename T, int NORM, bool ADD, int ROWS, int R>
+template <typename T, int NORM, bool ADD, int ROWS, int R, int U>
 __global__ __launch_bounds__(256) void input_gemv_kernel(GemvProblem p) {
     extern __shared__ u32x4 act[];
     __shared__ float red[12];
-    gemv_block<T, NORM, ADD, ROWS, R>(p, blockIdx.x, act, red);
+    fetch_args<sizeof(GemvProblem)>();
+    gemv_block<T, NORM, ADD, ROWS, R, U>(p, blockIdx.x, act, red);
 }
 template <typename T, int NORM, int ROWS, int R>
 __global__ __launch_bounds__(256) void input_gemv_pair_kernel(GemvPair p) {
     extern __shared__ u32x4 act[];
     __shared__ float red[12];
+    fetch_args<sizeof(GemvPair)>();
     const uint32_t second = blockIdx.x >= p.p[0].blocks ? 1u : 0u;
-    gemv_block<T, NORM, false, ROWS, R>(p.p[second], second ? blockIdx.x - p.p[0].blocks : blockIdx.x, act, red);
+    gemv_block<T, NORM, false, ROWS, R, 2>(p.p[second], second ? blockIdx.x - p.p[0].blocks : blockIdx.x, act, red);
 }
 
 // A workgroup takes ROWS rows, each wave a quarter of their columns, so that a long row is in flight at once; the
 // waves' sums meet in LDS.  A lane's products count with the gate and scale of the column segment its piece lies in.
+// Bound by the round trips in front of the weights: 1024 rows of 6144 bf16 take 4.4 us, 5.5 while sixteen scalar loads of
+// gates, one after the other, stood there and the old x was read at the end.
 template <typename T, int ROWS>
 __global__ __launch_bounds__(256) void gemv_residual_kernel(const T *__restrict__ w, uint32_t k_pad, uint32_t ld, const T *__restrict__ a,
                                                             RmiColSegs cs, float *__restrict__ x, uint32_t width) {
     constexpr int U = 4;
     __shared__ float part[4][ROWS];
+    fetch_args<40 + sizeof(RmiColSegs) + 12>();
     const uint32_t tid = threadIdx.x, lane = tid & 63, wave = uint32_t(__builtin_amdgcn_readfirstlane(int(tid >> 6)));
     const uint32_t row0 = blockIdx.x * ROWS;
     const uint32_t pieces = k_pad / kPieceElems<T>, per_wave = ((pieces + 3) / 4 + 63) / 64 * 64;
     const uint32_t p_begin = wave * per_wave, p_end = p_begin + per_wave < pieces ? p_begin + per_wave : pieces;
     const u32x4 *src[ROWS], *hsrc = reinterpret_cast<const u32x4 *>(a);
-    float gate[ROWS][kMaxColSegs];
 #pragma unroll
-    for (int r = 0; r < ROWS; r++) {
-        const uint32_t row = row0 + r < width ? row0 + r : width - 1;
-        src[r] = reinterpret_cast<const u32x4 *>(w + size_t(row) * ld);
-#pragma unroll
-        for (uint32_t i = 0; i < kMaxColSegs; i++) gate[r][i] = i < cs.n_segs ? (cs.s[i].gate ? cs.s[i].gate[row] : 1.0f) * cs.s[i].scale : 0.0f;
-    }
+    for (int r = 0; r < ROWS; r++) src[r] = reinterpret_cast<const u32x4 *>(w + size_t(row0 + r < width ? row0 + r : width - 1) * ld);
     float acc[ROWS];
 #pragma unroll
     for (int r = 0; r < ROWS; r++) acc[r] = 0.0f;
@@ -146,6 +163,21 @@ __global__ __launch_bounds__(256) void gemv_residual_kernel(const T *__restrict_
         }
     };
     if (p_begin < p_end) load(p_begin);
+    const uint32_t out_row = row0 + (tid < ROWS ? tid : 0);
+    float x_old = x[out_row < width ? out_row : width - 1];
+    // the gates behind the first weights, each by a load that no branch guards (there is always an x to read)
+    float gate[ROWS][kMaxColSegs];
+#pragma unroll
+    for (uint32_t i = 0; i < kMaxColSegs; i++) {
+        const bool has = i < cs.n_segs, gated = has && cs.s[i].gate;
+        const float *g = gated ? cs.s[i].gate : x, scale = has ? cs.s[i].scale : 0.0f;
+#pragma unroll
+        for (int r = 0; r < ROWS; r++) {
+            const float v = g[row0 + r < width ? row0 + r : width - 1];
+            gate[r][i] = (gated ? v : 1.0f) * scale;
+        }
+    }
+    asm volatile("" : "+v"(x_old));
     for (uint32_t p0 = p_begin; p0 < p_end; p0 += 64 * U) {
         u32x4 now[U][ROWS], hv[U];
 #pragma unroll
@@ -175,7 +207,7 @@ __global__ __launch_bounds__(256) void gemv_residual_kernel(const T *__restrict_
         if (lane == 0) part[wave][r] = t;
     }
     __syncthreads();
-    if (tid < ROWS && row0 + tid < width) x[row0 + tid] += (part[0][tid] + part[1][tid]) + (part[2][tid] + part[3][tid]);
+    if (tid < ROWS && row0 + tid < width) x[row0 + tid] = x_old + ((part[0][tid] + part[1][tid]) + (part[2][tid] + part[3][tid]));
 }
 
 GemvProblem problem_of(const RmiDense &w, const RmiInput &in, const RmiRowSegs &segs, uint32_t rows) {
@@ -186,9 +218,10 @@ template <typename T>
 int gemv(const RmiDense &w, const RmiInput &in, const RmiRowSegs &segs, hipStream_t st) {
     const size_t lds = size_t(gemv_lds_pieces<T>(w.k_pad)) * 16;
     // A wave takes four rows; fewer where that would leave compute units with little to do (the prologue, which every
-    // workgroup repeats, then weighs less than the wait for memory).  Pairs of rows stay together.
+    // workgroup repeats, then weighs less than the wait for memory).  Pairs of rows stay together.  (12 288 rows of 2048
+    // f32: 19.1 us with four, 20.8 with two, of which one and a fifth of a chip's fill are resident; 6176 rows: two.)
     const uint32_t cus = uint32_t(rmi_device_cus()), pairs = rmi_epilogue_of(segs) == kRowsPaired ? 2 : 1;
-    const uint32_t rows = in.norm == kNormRms || w.n_rows > 64 * cus ? 4 : w.n_rows > 4 * cus ? 2 : pairs;
+    const uint32_t rows = in.norm == kNormRms || w.n_rows >= 32 * cus ? 4 : w.n_rows > 4 * cus ? 2 : pairs;
     const GemvProblem p = problem_of(w, in, segs, rows);
     auto go = [&](auto kernel) {
         const int rc = rmi_allow_lds(kernel, lds);
@@ -197,11 +230,17 @@ int gemv(const RmiDense &w, const RmiInput &in, const RmiRowSegs &segs, hipStrea
     };
     const int rc = rmi_input_dispatch(in, [&](auto norm, auto add, auto r) {
         if constexpr (norm.value != kNormRms && (!add.value || r.value <= 4)) {
-            if (rows == 1) return go(input_gemv_kernel<T, norm.value, add.value, 1, r.value>);
-            if (rows == 2) return go(input_gemv_kernel<T, norm.value, add.value, 2, r.value>);
+            // Up to two workgroups a compute unit leave memory idle with two rounds of a wave in flight (32 of them: 5.7 us,
+            // with eight rounds 4.7; 256 of 2 x 4096 f32: 12.2 and 11.0); with three, eight rounds' registers keep
+            // workgroups out (772: 13.2 and 14.6).  Rows of up to two rounds gain nothing.
+            const bool deep = p.blocks <= 2 * cus && w.k_pad / kPieceElems<T> > 128;
+            if (rows == 1 && deep) return go(input_gemv_kernel<T, norm.value, add.value, 1, r.value, 8>);
+            if (rows == 1) return go(input_gemv_kernel<T, norm.value, add.value, 1, r.value, 2>);
+            if (rows == 2 && deep) return go(input_gemv_kernel<T, norm.value, add.value, 2, r.value, 8>);
+            if (rows == 2) return go(input_gemv_kernel<T, norm.value, add.value, 2, r.value, 2>);
         }
         if constexpr (!add.value || r.value <= 4)
-            return go(input_gemv_kernel<T, norm.value, add.value, 4, r.value>);
+            return go(input_gemv_kernel<T, norm.value, add.value, 4, r.value, 2>);
         else
             return rmi_fail(RMI_HIP_E_INVALID, "too many values to add in front of a product");
     });

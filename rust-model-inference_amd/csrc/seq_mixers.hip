@@ -2,6 +2,7 @@
 #include "seq_mixers.h"
 #include <type_traits>
 
+#include "device_args.h"
 #include "device_conv.h"
 #include "device_dense.h"
 
@@ -843,6 +844,7 @@ __global__ __launch_bounds__(kStepThreads) void mixers_step_kernel(RmiAttnShape 
                                                                    RmiRecurShape rs, RmiRecurArgs ra) {
     extern __shared__ __attribute__((aligned(16))) uint8_t lds_raw[];
     __shared__ uint32_t flag;
+    fetch_args<sizeof(RmiAttnShape) + sizeof(RmiAttnArgs) + sizeof(SplitPlan) + sizeof(RmiRecurShape) + sizeof(RmiRecurArgs)>();
     if (blockIdx.x < attn_blocks)
         attn_split<T, BUCKET, true>(s, a, blockIdx.x, plan, lds_raw, &flag);
     else
