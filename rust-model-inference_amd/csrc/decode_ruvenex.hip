@@ -90,7 +90,10 @@ int RuvenexSession::enqueue_layers(uint32_t step0, uint32_t n, hipStream_t st, f
         r.scratch = recur_scratch;
         if (n == 1 && rmi_dense_gemv_fits(elem, k_in)) {
             rc = rmi_dense_gemv(elem, y.w_in, normed(y.norm), y.in, st);
-            if (rc == RMI_HIP_OK) rc = rmi_mixers_step(elem, &y.attn, &a, &y.recur, &r, st);
+            RmiAhead ahead{};
+            rmi_dense_ahead_residual(elem, y.w_out, width, &ahead);
+            if (l + 1 < n_runs) rmi_dense_ahead_gemv(elem, layers[l + 1].w_in, normed(y.norm), layers[l + 1].in, &ahead);
+            if (rc == RMI_HIP_OK) rc = rmi_mixers_step(elem, &y.attn, &a, &y.recur, &r, ahead, st);
             if (rc == RMI_HIP_OK) rc = rmi_dense_gemv_residual(elem, y.w_out, act, y.out, x, width, st);
         } else {
             rc = rmi_dense_input(elem, normed(y.norm), nullptr, h, n, k_in, st);

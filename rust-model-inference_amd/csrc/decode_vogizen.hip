@@ -207,7 +207,7 @@ int VogizenSession::mixer(const VogizenLayer &l, const VogizenRun &r, uint32_t s
     a.pos0 = step0;
     a.n_tokens = n;
     a.scratch = attn_scratch;
-    return n == 1 ? rmi_mixers_step(elem, &l.attn, &a, nullptr, nullptr, st) : rmi_attn_pass(elem, l.attn, a, st);
+    return n == 1 ? rmi_mixers_step(elem, &l.attn, &a, nullptr, nullptr, RmiAhead{}, st) : rmi_attn_pass(elem, l.attn, a, st);
 }
 
 int VogizenSession::enqueue_layers(uint32_t step0, uint32_t n, hipStream_t st, float *host_layers) {

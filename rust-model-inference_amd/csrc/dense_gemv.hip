@@ -214,14 +214,19 @@ GemvProblem problem_of(const RmiDense &w, const RmiInput &in, const RmiRowSegs &
     return GemvProblem{w.data, w.k_pad, w.ld, (w.n_rows + 4 * rows - 1) / (4 * rows), in, segs};
 }
 
+constexpr uint32_t kResidualRows = 2;
+// A wave takes four rows; fewer where that would leave compute units with little to do (the prologue, which every
+// workgroup repeats, then weighs less than the wait for memory).  Pairs of rows stay together.  (12 288 rows of 2048
+// f32: 19.1 us with four, 20.8 with two, of which one and a fifth of a chip's fill are resident; 6176 rows: two.)
+uint32_t rows_of_wave(const RmiDense &w, const RmiInput &in, const RmiRowSegs &segs) {
+    const uint32_t cus = uint32_t(rmi_device_cus()), pairs = rmi_epilogue_of(segs) == kRowsPaired ? 2 : 1;
+    return in.norm == kNormRms || w.n_rows >= 32 * cus ? 4 : w.n_rows > 4 * cus ? 2 : pairs;
+}
+
 template <typename T>
 int gemv(const RmiDense &w, const RmiInput &in, const RmiRowSegs &segs, hipStream_t st) {
     const size_t lds = size_t(gemv_lds_pieces<T>(w.k_pad)) * 16;
-    // A wave takes four rows; fewer where that would leave compute units with little to do (the prologue, which every
-    // workgroup repeats, then weighs less than the wait for memory).  Pairs of rows stay together.  (12 288 rows of 2048
-    // f32: 19.1 us with four, 20.8 with two, of which one and a fifth of a chip's fill are resident; 6176 rows: two.)
-    const uint32_t cus = uint32_t(rmi_device_cus()), pairs = rmi_epilogue_of(segs) == kRowsPaired ? 2 : 1;
-    const uint32_t rows = in.norm == kNormRms || w.n_rows >= 32 * cus ? 4 : w.n_rows > 4 * cus ? 2 : pairs;
+    const uint32_t cus = uint32_t(rmi_device_cus()), rows = rows_of_wave(w, in, segs);
     const GemvProblem p = problem_of(w, in, segs, rows);
     auto go = [&](auto kernel) {
         const int rc = rmi_allow_lds(kernel, lds);
@@ -266,7 +271,7 @@ int gemv_pair(const GemvPair &p, hipStream_t st) {
 
 template <typename T>
 int gemv_residual(const RmiDense &w, const void *a, const RmiColSegs &segs, float *x, uint32_t width, hipStream_t st) {
-    constexpr int kRows = 2;
+    constexpr int kRows = kResidualRows;
     hipLaunchKernelGGL((gemv_residual_kernel<T, kRows>), dim3((width + kRows - 1) / kRows), dim3(256), 0, st,
                        static_cast<const T *>(w.data), w.k_pad, w.ld, static_cast<const T *>(a), segs, x, width);
     RMI_HIP_CHECK(hipGetLastError());
@@ -318,4 +323,13 @@ int rmi_dense_gemv_residual(uint32_t elem_bytes, const RmiDense &w, const void *
     const int rc = rmi_check_col_segs(elem_bytes, w, segs, width);
     if (rc != RMI_HIP_OK) return rc;
     return elem_bytes == 2 ? gemv_residual<rmi_bf16>(w, a, segs, x, width, st) : gemv_residual<float>(w, a, segs, x, width, st);
+}
+
+void rmi_dense_ahead_gemv(uint32_t elem_bytes, const RmiDense &w, const RmiInput &in, const RmiRowSegs &segs, RmiAhead *ahead) {
+    const uint32_t rows = 4 * rows_of_wave(w, in, segs);
+    ahead->add(w.data, size_t(rows) * w.ld * elem_bytes, w.n_rows / rows);
+}
+
+void rmi_dense_ahead_residual(uint32_t elem_bytes, const RmiDense &w, uint32_t width, RmiAhead *ahead) {
+    ahead->add(w.data, size_t(kResidualRows) * w.ld * elem_bytes, width / kResidualRows);
 }

@@ -30,8 +30,8 @@ inline uint32_t rmi_attn_rows(uint32_t window, uint32_t pass_rows, uint32_t capa
     return rmi_dense_pad(ring < capacity ? uint32_t(ring) : capacity, kKeyBlock);
 }
 // One pass's pointers.  u: f32 [n_tokens][channels], channels = q heads | k heads | v heads, before the convolution;
-// hist_in: the taps - 1 rows before it (row j = position pos0 - (taps - 1) + j; rows of positions below zero are
-// never read); hist_out, another buffer, gets the taps - 1 rows before the next pass's first.
+// hist_in: the taps - 1 rows before it (row j = position pos0 - (taps - 1) + j; rows of positions below zero
+// may be read and count for nothing); hist_out, another buffer, gets the taps - 1 rows before the next pass's first.
 struct RmiAttnArgs {
     const float *u, *hist_in;
     float *hist_out;
@@ -54,7 +54,7 @@ struct RmiRecurShape {
 };
 struct RmiRecurArgs {
     const float *q, *f, *v;  // [n_tokens][heads * dim], f = the forget gate; [n_tokens][heads * vdim]
-    const float *state_in;   // [head][d_pad][v_pad]; not read at pos0 == 0
+    const float *state_in;   // [head][d_pad][v_pad]; counts for nothing at pos0 == 0
     float *state_out;        // another buffer
     const float *norm;       // [vdim]
     void *out;               // [token * out_ld + head * vdim + channel], the model's element type
@@ -94,6 +94,6 @@ int rmi_attn_pass(uint32_t elem_bytes, const RmiAttnShape &s, const RmiAttnArgs 
 int rmi_recur_pass(uint32_t elem_bytes, const RmiRecurShape &s, const RmiRecurArgs &a, hipStream_t st);
 // one token: either mixer may be left out (nullptr); both go into one launch
 int rmi_mixers_step(uint32_t elem_bytes, const RmiAttnShape *as, const RmiAttnArgs *aa, const RmiRecurShape *rs, const RmiRecurArgs *ra,
-                    hipStream_t st);
+                    const RmiAhead &ahead, hipStream_t st);
 int rmi_delta_pass(uint32_t elem_bytes, const RmiDeltaShape &s, const RmiDeltaArgs &a, hipStream_t st);
 int rmi_delta_step(uint32_t elem_bytes, const RmiDeltaShape &s, const RmiDeltaArgs &a, hipStream_t st);

@@ -841,14 +841,16 @@ inline size_t recur_step_lds(const RmiRecurShape &s) {
 // eight waves a workgroup for 256 keys without a second workgroup, all took as long or longer.
 template <typename T, int BUCKET>
 __global__ __launch_bounds__(kStepThreads) void mixers_step_kernel(RmiAttnShape s, RmiAttnArgs a, uint32_t attn_blocks, SplitPlan plan,
-                                                                   RmiRecurShape rs, RmiRecurArgs ra) {
+                                                                   RmiRecurShape rs, RmiRecurArgs ra, RmiAhead ahead) {
     extern __shared__ __attribute__((aligned(16))) uint8_t lds_raw[];
     __shared__ uint32_t flag;
     fetch_args<sizeof(RmiAttnShape) + sizeof(RmiAttnArgs) + sizeof(SplitPlan) + sizeof(RmiRecurShape) + sizeof(RmiRecurArgs)>();
     if (blockIdx.x < attn_blocks)
         attn_split<T, BUCKET, true>(s, a, blockIdx.x, plan, lds_raw, &flag);
-    else
+    else if (blockIdx.x < attn_blocks + rs.heads)
         recur_step<T>(rs, ra, blockIdx.x - attn_blocks, reinterpret_cast<float *>(lds_raw));
+    else
+        fetch_ahead<kStepThreads>(ahead, attn_blocks + rs.heads);
 }
 
 // Several tokens, in chunks of sixteen.  With P_t the product of f over the chunk's tokens up to t:
@@ -1145,7 +1147,8 @@ int check_recur(const RmiRecurShape &s) {
 }
 
 template <typename T>
-int mixers_step(const RmiAttnShape *as, const RmiAttnArgs *aa, const RmiRecurShape *rs, const RmiRecurArgs *ra, hipStream_t st) {
+int mixers_step(const RmiAttnShape *as, const RmiAttnArgs *aa, const RmiRecurShape *rs, const RmiRecurArgs *ra, const RmiAhead &ahead,
+                hipStream_t st) {
     const RmiAttnShape s = as ? *as : RmiAttnShape{};
     const RmiAttnArgs a = aa ? *aa : RmiAttnArgs{};
     const RmiRecurShape r = rs ? *rs : RmiRecurShape{};
@@ -1159,11 +1162,11 @@ int mixers_step(const RmiAttnShape *as, const RmiAttnArgs *aa, const RmiRecurSha
         lds = split_lds(sizeof(T), s, 1);
     }
     if (rs && recur_step_lds(r) > lds) lds = recur_step_lds(r);
-    const dim3 grid(blocks + (rs ? r.heads : 0));
+    const dim3 grid(blocks + (rs ? r.heads : 0) + rmi_ahead_blocks(ahead));
     const uint32_t bucket = as ? bucket_of(s) : 64;
     auto go = [&](auto kernel) {
         const int rc = rmi_allow_lds(kernel, lds);
-        if (rc == RMI_HIP_OK) hipLaunchKernelGGL(kernel, grid, dim3(kStepThreads), lds, st, s, a, blocks, plan, r, b);
+        if (rc == RMI_HIP_OK) hipLaunchKernelGGL(kernel, grid, dim3(kStepThreads), lds, st, s, a, blocks, plan, r, b, ahead);
         return rc;
     };
     const int rc = bucket == 64 ? go(mixers_step_kernel<T, 64>) : bucket == 128 ? go(mixers_step_kernel<T, 128>) : go(mixers_step_kernel<T, 256>);
@@ -1228,10 +1231,10 @@ int rmi_recur_pass(uint32_t elem_bytes, const RmiRecurShape &s, const RmiRecurAr
 }
 
 int rmi_mixers_step(uint32_t elem_bytes, const RmiAttnShape *as, const RmiAttnArgs *aa, const RmiRecurShape *rs, const RmiRecurArgs *ra,
-                    hipStream_t st) {
+                    const RmiAhead &ahead, hipStream_t st) {
     if (!as && !rs) return RMI_HIP_OK;
     int rc = as ? check_attn(*as, *aa) : RMI_HIP_OK;
     if (rc == RMI_HIP_OK && rs) rc = check_recur(*rs);
     if (rc != RMI_HIP_OK) return rc;
-    return elem_bytes == 2 ? mixers_step<rmi_bf16>(as, aa, rs, ra, st) : mixers_step<float>(as, aa, rs, ra, st);
+    return elem_bytes == 2 ? mixers_step<rmi_bf16>(as, aa, rs, ra, ahead, st) : mixers_step<float>(as, aa, rs, ra, ahead, st);
 }

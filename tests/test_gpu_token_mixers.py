@@ -28,3 +28,14 @@ def test_every_place_of_a_block(open_model, dtype, dim, vdim, taps):
         got = feed(s, t, sizes)
         # bf16 keeps 8 bits of 24: the tolerance of the sessions' other tests; a key or value in a wrong place errs by its whole weight
         assert rel(got, ref) < TOL[dtype], (sizes, int(np.argmax(np.abs(got - ref).max(-1))))
+
+
+@pytest.mark.parametrize("dtype", [F32, BF16])
+@pytest.mark.parametrize("width,ffs", [(33, [None]), (40, [7, None]), (130, [None, 300, 5]), (1030, [5000, 9, 2100])])
+def test_weights_fetched_ahead(open_model, dtype, width, ffs):
+    """The launch also reads weights of its layer's output and of the next layer's input: less and more than its budget,
+    layers of different sizes, none behind the last."""
+    cfg = G.config([G.layer_config(ff=ff) for ff in ffs], width=width)
+    s, w = open_model(cfg, None, dtype, 40)
+    t = G.tokens(cfg, 9)
+    assert rel(feed(s, t, [1]), P.forward(cfg, w, t)) < TOL[dtype]  # nothing depends on what is read
