@@ -1046,12 +1046,12 @@ def run_decode(args, pkg, ev):
     result = base_result(args, "decode token-steps/s, Qwen3-0.6B Q8_0, 512 prompt + 128 greedy tokens, 1 GPU", "tok/s",
                          round(token_steps / wall, 1), wall, "int8 dot4 -> f32 (F16 KV cache)", {
         "workload": "device-resident greedy decode of a synthetic Q8_0 GGUF (Qwen3-0.6B architecture, 28 layers, "
-                    "vocab 151936), 512 prompt positions (128 to a pass) + 127 generated tokens = 639 token-steps per "
+                    "vocab 151936), 512 prompt positions (one pass) + 127 generated tokens = 639 token-steps per "
                     "generation, logits computed at every position; one bench step = one generation",
         "token_steps_per_generation": token_steps, "launches_per_token_step": 1 + 5 * 28 + 4,
         "device": dev_name.strip(), "compute_units": cus})
     result["ms_per_token_step"] = round(per_token * 1e3, 4)
-    # the two phases apart: the prompt (positions known in advance: the session takes them 128 to a pass, each
+    # the two phases apart: the prompt (positions known in advance: the session takes them up to 1024 to a pass, each
     # position's logits still computed and bit-identical to its own step) and the generated tokens (one step each)
     if args.no_phases:
         t_prompt = None
@@ -1067,13 +1067,13 @@ def run_decode(args, pkg, ev):
         sess.set_prompt_passes(True)
         result["phases"]["every_position_its_own_step_tok_s"] = round(token_steps / t_steps, 1)
     # HBM bytes against time for the generated tokens, each of which reads every weight once; the prompt passes
-    # read a weight once for 128 positions, so the whole generation's time per token-step would flatter the figure
+    # read a weight once for up to 1024 positions, so the whole generation's time per token-step would flatter the figure
     if t_prompt is not None:
         per_generated = (t_all - t_prompt) / (n_new - 1)
         basis = "generated tokens (one step each, 512-638 cached positions)"
     else:
         per_generated = per_token
-        basis = "whole generation, prompt passes included (they read a weight once for 128 positions: an upper bound)"
+        basis = "whole generation, prompt passes included (they read a weight once for up to 1024 positions: an upper bound)"
     achieved = alg / per_generated / 1e9
     result["roofline"] = {"bound": "hbm", "kernel": "Q8_0 GEMV kernels (4 per layer + lm_head = 113 launches per token-step)",
                           "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
