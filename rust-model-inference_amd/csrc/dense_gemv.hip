@@ -28,6 +28,13 @@ struct GemvProblem {
 struct GemvPair {
     GemvProblem p[2];
 };
+struct ResidualProblem {
+    const void *w, *a;
+    uint32_t k_pad, ld;
+    RmiColSegs segs;
+    float *x;
+    uint32_t width;
+};
 
 template <typename T>
 using UintOf = std::conditional_t<sizeof(T) == 4, uint32_t, uint16_t>;
@@ -120,14 +127,14 @@ template <typename T, int NORM, bool ADD, int ROWS, int R, int U>
 __global__ __launch_bounds__(256) void input_gemv_kernel(GemvProblem p) {
     extern __shared__ u32x4 act[];
     __shared__ float red[12];
-    fetch_args<sizeof(GemvProblem)>();
+    fetch_args<GemvProblem>();
     gemv_block<T, NORM, ADD, ROWS, R, U>(p, blockIdx.x, act, red);
 }
 template <typename T, int NORM, int ROWS, int R>
 __global__ __launch_bounds__(256) void input_gemv_pair_kernel(GemvPair p) {
     extern __shared__ u32x4 act[];
     __shared__ float red[12];
-    fetch_args<sizeof(GemvPair)>();
+    fetch_args<GemvPair>();
     const uint32_t second = blockIdx.x >= p.p[0].blocks ? 1u : 0u;
     gemv_block<T, NORM, false, ROWS, R, 2>(p.p[second], second ? blockIdx.x - p.p[0].blocks : blockIdx.x, act, red);
 }
@@ -137,18 +144,22 @@ __global__ __launch_bounds__(256) void input_gemv_pair_kernel(GemvPair p) {
 // Bound by the round trips in front of the weights: 1024 rows of 6144 bf16 take 4.4 us, 5.5 while sixteen scalar loads of
 // gates, one after the other, stood there and the old x was read at the end.
 template <typename T, int ROWS>
-__global__ __launch_bounds__(256) void gemv_residual_kernel(const T *__restrict__ w, uint32_t k_pad, uint32_t ld, const T *__restrict__ a,
-                                                            RmiColSegs cs, float *__restrict__ x, uint32_t width) {
+__global__ __launch_bounds__(256) void gemv_residual_kernel(ResidualProblem p) {
     constexpr int U = 4;
     __shared__ float part[4][ROWS];
-    fetch_args<40 + sizeof(RmiColSegs) + 12>();
+    fetch_args<ResidualProblem>();
+    const T *__restrict__ w = static_cast<const T *>(p.w), *__restrict__ a = static_cast<const T *>(p.a);
+    float *__restrict__ x = p.x;
+    const uint32_t k_pad = p.k_pad, width = p.width;
+    const size_t ld = p.ld;
+    const RmiColSegs &cs = p.segs;
     const uint32_t tid = threadIdx.x, lane = tid & 63, wave = uint32_t(__builtin_amdgcn_readfirstlane(int(tid >> 6)));
     const uint32_t row0 = blockIdx.x * ROWS;
     const uint32_t pieces = k_pad / kPieceElems<T>, per_wave = ((pieces + 3) / 4 + 63) / 64 * 64;
     const uint32_t p_begin = wave * per_wave, p_end = p_begin + per_wave < pieces ? p_begin + per_wave : pieces;
     const u32x4 *src[ROWS], *hsrc = reinterpret_cast<const u32x4 *>(a);
 #pragma unroll
-    for (int r = 0; r < ROWS; r++) src[r] = reinterpret_cast<const u32x4 *>(w + size_t(row0 + r < width ? row0 + r : width - 1) * ld);
+    for (int r = 0; r < ROWS; r++) src[r] = reinterpret_cast<const u32x4 *>(w + (row0 + r < width ? row0 + r : width - 1) * ld);
     float acc[ROWS];
 #pragma unroll
     for (int r = 0; r < ROWS; r++) acc[r] = 0.0f;
@@ -273,7 +284,7 @@ template <typename T>
 int gemv_residual(const RmiDense &w, const void *a, const RmiColSegs &segs, float *x, uint32_t width, hipStream_t st) {
     constexpr int kRows = kResidualRows;
     hipLaunchKernelGGL((gemv_residual_kernel<T, kRows>), dim3((width + kRows - 1) / kRows), dim3(256), 0, st,
-                       static_cast<const T *>(w.data), w.k_pad, w.ld, static_cast<const T *>(a), segs, x, width);
+                       ResidualProblem{w.data, a, w.k_pad, w.ld, segs, x, width});
     RMI_HIP_CHECK(hipGetLastError());
     return RMI_HIP_OK;
 }

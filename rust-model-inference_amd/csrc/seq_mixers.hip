@@ -839,18 +839,26 @@ inline size_t recur_step_lds(const RmiRecurShape &s) {
 // division stands before it: 28 layers of 16 heads over 8 of 128 elements, 150 positions, bf16: 12.7 us a launch with loads
 // behind branches, 10.0 as it is; f32, 16 key/value heads and 310 positions: 17.6 and 14.8.  Parts of 64 or of 32 keys, and
 // eight waves a workgroup for 256 keys without a second workgroup, all took as long or longer.
+struct MixersStep {
+    RmiAttnShape s;
+    RmiAttnArgs a;
+    SplitPlan plan;
+    RmiRecurShape rs;
+    RmiRecurArgs ra;
+    RmiAhead ahead;
+    uint32_t attn_blocks;
+};
 template <typename T, int BUCKET>
-__global__ __launch_bounds__(kStepThreads) void mixers_step_kernel(RmiAttnShape s, RmiAttnArgs a, uint32_t attn_blocks, SplitPlan plan,
-                                                                   RmiRecurShape rs, RmiRecurArgs ra, RmiAhead ahead) {
+__global__ __launch_bounds__(kStepThreads) void mixers_step_kernel(MixersStep p) {
     extern __shared__ __attribute__((aligned(16))) uint8_t lds_raw[];
     __shared__ uint32_t flag;
-    fetch_args<sizeof(RmiAttnShape) + sizeof(RmiAttnArgs) + sizeof(SplitPlan) + sizeof(RmiRecurShape) + sizeof(RmiRecurArgs)>();
-    if (blockIdx.x < attn_blocks)
-        attn_split<T, BUCKET, true>(s, a, blockIdx.x, plan, lds_raw, &flag);
-    else if (blockIdx.x < attn_blocks + rs.heads)
-        recur_step<T>(rs, ra, blockIdx.x - attn_blocks, reinterpret_cast<float *>(lds_raw));
+    fetch_args<MixersStep>();
+    if (blockIdx.x < p.attn_blocks)
+        attn_split<T, BUCKET, true>(p.s, p.a, blockIdx.x, p.plan, lds_raw, &flag);
+    else if (blockIdx.x < p.attn_blocks + p.rs.heads)
+        recur_step<T>(p.rs, p.ra, blockIdx.x - p.attn_blocks, reinterpret_cast<float *>(lds_raw));
     else
-        fetch_ahead<kStepThreads>(ahead, attn_blocks + rs.heads);
+        fetch_ahead<kStepThreads>(p.ahead, p.attn_blocks + p.rs.heads);
 }
 
 // Several tokens, in chunks of sixteen.  With P_t the product of f over the chunk's tokens up to t:
@@ -1149,24 +1157,26 @@ int check_recur(const RmiRecurShape &s) {
 template <typename T>
 int mixers_step(const RmiAttnShape *as, const RmiAttnArgs *aa, const RmiRecurShape *rs, const RmiRecurArgs *ra, const RmiAhead &ahead,
                 hipStream_t st) {
-    const RmiAttnShape s = as ? *as : RmiAttnShape{};
-    const RmiAttnArgs a = aa ? *aa : RmiAttnArgs{};
-    const RmiRecurShape r = rs ? *rs : RmiRecurShape{};
-    const RmiRecurArgs b = ra ? *ra : RmiRecurArgs{};
-    SplitPlan plan{};
-    uint32_t blocks = 0;
+    MixersStep p{};
+    p.ahead = ahead;
+    if (rs) {
+        p.rs = *rs;
+        p.ra = *ra;
+    }
     size_t lds = 0;
     if (as) {
-        plan = attn_parts(s, 1, a.pos0);
-        blocks = s.kv_heads * plan.tiles.by * plan.parts.by;
-        lds = split_lds(sizeof(T), s, 1);
+        p.s = *as;
+        p.a = *aa;
+        p.plan = attn_parts(p.s, 1, p.a.pos0);
+        p.attn_blocks = p.s.kv_heads * p.plan.tiles.by * p.plan.parts.by;
+        lds = split_lds(sizeof(T), p.s, 1);
     }
-    if (rs && recur_step_lds(r) > lds) lds = recur_step_lds(r);
-    const dim3 grid(blocks + (rs ? r.heads : 0) + rmi_ahead_blocks(ahead));
-    const uint32_t bucket = as ? bucket_of(s) : 64;
+    if (rs && recur_step_lds(p.rs) > lds) lds = recur_step_lds(p.rs);
+    const dim3 grid(p.attn_blocks + p.rs.heads + rmi_ahead_blocks(ahead));
+    const uint32_t bucket = as ? bucket_of(p.s) : 64;
     auto go = [&](auto kernel) {
         const int rc = rmi_allow_lds(kernel, lds);
-        if (rc == RMI_HIP_OK) hipLaunchKernelGGL(kernel, grid, dim3(kStepThreads), lds, st, s, a, blocks, plan, r, b, ahead);
+        if (rc == RMI_HIP_OK) hipLaunchKernelGGL(kernel, grid, dim3(kStepThreads), lds, st, p);
         return rc;
     };
     const int rc = bucket == 64 ? go(mixers_step_kernel<T, 64>) : bucket == 128 ? go(mixers_step_kernel<T, 128>) : go(mixers_step_kernel<T, 256>);
