@@ -31,6 +31,22 @@ constexpr uint32_t kThreads = 256, kRows = kAttnPromptRows, kTurn = 64;  // kTur
 constexpr uint32_t kTurnStride = kTurn + 4;                             // floats; four lanes' 16-byte reads on different banks
 
 __device__ __forceinline__ double half_f64(f16x8 v, int i) { return double(float(v[i])); }
+// Zeros in the place of infinities and NaN; whether there was one.
+__device__ __forceinline__ bool take_out_nonfinite(f16x8 (&v)[4]) {
+    uint32_t odd = 0;
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        u32x4 u = __builtin_bit_cast(u32x4, v[i]);
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const uint32_t lo = (u[j] & 0x7c00u) == 0x7c00u ? 0xffffu : 0u, hi = (u[j] & 0x7c000000u) == 0x7c000000u ? 0xffff0000u : 0u;
+            odd |= lo | hi;
+            u[j] &= ~(lo | hi);
+        }
+        v[i] = __builtin_bit_cast(f16x8, u);
+    }
+    return odd != 0;
+}
 
 __global__ __launch_bounds__(kThreads, 2) void attn128_prompt_kernel(const uint16_t *__restrict__ q16, const uint16_t *__restrict__ k_cache,
                                                                      const uint16_t *__restrict__ v_cache, uint32_t step0, uint32_t n_tok,
@@ -146,9 +162,10 @@ __global__ __launch_bounds__(kThreads, 2) void attn128_prompt_kernel(const uint1
     __syncthreads();
 
     // ---- 3: weights and values.  Lane (c16, g): weights of position c16 and keys 4 g .. 4 g + 3 of the sixteen (as A);
-    // dimensions 8 c16 .. + 7 of the same keys (as B), so that product j's columns are the dimensions 8 c16 + j.  Weights
-    // of later positions are zero: a value that is not finite would still count (0 x inf), but a prompt with such a value
-    // in its cache ends in non-finite logits and an error.
+    // dimensions 8 c16 .. + 7 of the same keys (as B), so that product j's columns are the dimensions 8 c16 + j.  A key
+    // behind a position has weight zero there, which hides its value as long as that is finite (0 x inf is NaN, which the
+    // quantizer drops): of the few keys that some positions of the tile see and others do not, other values are taken out
+    // and counted afterwards.
     f64x4 acc[8];
 #pragma unroll
     for (int j = 0; j < 8; j++) acc[j] = f64x4{0.0, 0.0, 0.0, 0.0};
@@ -165,16 +182,21 @@ __global__ __launch_bounds__(kThreads, 2) void attn128_prompt_kernel(const uint1
                 vv[i] = *reinterpret_cast<const f16x8 *>(vbase + size_t(key) * kv_stride);
             }
         };
+        auto weight = [&](float ev, uint32_t key) {
+            const float w32 = total > 0.0f ? ev / total : ev;
+            return key <= last ? double(h2f(rmi_f2h(w32))) : 0.0;
+        };
         f16x8 vv[4], vn[4];
         float4 e, en;
+        bool odd = false;
         load_values(vv, e, wave);
         for (uint32_t kt = wave; kt < key_tiles; kt += 4) {
             load_values(vn, en, kt + 4);
             const float ev[4] = {e.x, e.y, e.z, e.w};
+            if (kt * 16 + 15 > step0 + t0) odd |= take_out_nonfinite(vv);
 #pragma unroll
             for (uint32_t i = 0; i < 4; i++) {
-                const float w32 = total > 0.0f ? ev[i] / total : ev[i];
-                const double w = kt * 16 + 4 * g + i <= last ? double(h2f(rmi_f2h(w32))) : 0.0;
+                const double w = weight(ev[i], kt * 16 + 4 * g + i);
 #pragma unroll
                 for (int j = 0; j < 8; j++) acc[j] = __builtin_amdgcn_mfma_f64_16x16x4f64(w, half_f64(vv[i], j), acc[j], 0, 0, 0);
             }
@@ -182,6 +204,25 @@ __global__ __launch_bounds__(kThreads, 2) void attn128_prompt_kernel(const uint1
             for (int i = 0; i < 4; i++) vv[i] = vn[i];
             e = en;
         }
+        if (__any(odd))  // what was taken out, one position after the other, without the values behind it
+            for (uint32_t kt = wave; kt < key_tiles; kt += 4) {
+                if (kt * 16 + 15 <= step0 + t0) continue;
+#pragma unroll 1
+                for (uint32_t r = 0; r < rows; r++)
+#pragma unroll 1
+                    for (uint32_t i = 0; i < 4; i++) {
+                        const uint32_t key = kt * 16 + 4 * g + i, there = key < n_keys ? key : n_keys - 1;
+                        const double w = weight(s_row0[size_t(c16) * score_stride + key], key);
+                        const f16x8 v = *reinterpret_cast<const f16x8 *>(vbase + size_t(there) * kv_stride);
+#pragma unroll
+                        for (int j = 0; j < 8; j++) {
+                            const bool finite = fabsf(float(v[j])) <= 65504.0f;
+                            const f64x4 o = __builtin_amdgcn_mfma_f64_16x16x4f64(w, finite || key > step0 + t0 + r ? 0.0 : half_f64(v, j), f64x4{0.0, 0.0, 0.0, 0.0}, 0, 0, 0);
+#pragma unroll
+                            for (uint32_t q = 0; q < 4; q++) acc[j][q] += 4 * q + g == r ? o[q] : 0.0;
+                        }
+                    }
+            }
     }
     // lane (c16, g), register i: position 4 i + g, dimensions 8 c16 + j
     if (wave > 0) {

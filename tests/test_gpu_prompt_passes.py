@@ -42,3 +42,56 @@ def test_a_pass_that_is_asked_for_more_logits_than_it_holds(hip, tmp_path):
     slow = session.generate(prompt, 2, dump_steps=range(201))
     session.close()
     assert np.array_equal(fast["dump"].view(np.uint32), slow["dump"].view(np.uint32))
+
+
+def _put(raw, n_in, row, block, scale, quants):
+    """One block of 32 of a row of Q8_0 bytes."""
+    b = raw.reshape(-1, n_in // 32, 34)[row, block]
+    b[:2] = np.frombuffer(np.float16(scale).tobytes(), np.uint8)
+    b[2:] = np.asarray(quants, np.int8).view(np.uint8)
+
+
+@pytest.mark.parametrize("seen", [True, False])
+@pytest.mark.parametrize("n_prompt,at", [(5, 4), (7, 2), (33, 32), (40, 20), (40, 35), (100, 80), (130, 129)])
+def test_a_value_that_is_not_finite_counts_from_its_position_on(hip, tmp_path, n_prompt, at, seen):
+    """One prompt token's values overflow f16.  seen: its weight is not zero, so that its position and those behind it have
+    logits that are not finite, and their number is in the error.  Otherwise every weight of it rounds to zero: 0 x inf is
+    NaN, which the quantizer drops, from that position on and not before."""
+    width, heads, special = 256, 2, 999
+    path = os.path.join(str(tmp_path), "m.gguf")
+    hip.gguf.write_synthetic_qwen3(path, seed=5, n_layer=1, n_embd=width, n_head=heads, n_head_kv=heads, head_dim=128, n_ff=256, vocab=1000, n_ctx=4096)
+    f = hip.gguf.GGUFFile(path)
+    t = {name: np.array(v[2]) for name, v in f.tensors.items()}
+    # elements 0 and 1 of the stream: the special token's mark, and one that all tokens have
+    for row in range(1000):
+        q = t["token_embd.weight"].reshape(-1, width // 32, 34)[row, 0, 2:].view(np.int8)
+        q[0], q[1] = 0, 127
+    _put(t["token_embd.weight"], width, special, 0, 1.0, [127, 127] + [0] * 30)
+    for row in range(0, heads * 128, 5):  # some values of every block (of nothing but NaN the largest is NaN): 500 x 127 times the mark
+        _put(t["blk.0.attn_v.weight"], width, row, 0, 500.0, [127] + [0] * 31)
+    if not seen:  # one element a head, of one sign in every query, of the other sign in the special token's key: scores of +-100
+        for name in ("attn_q", "attn_k"):
+            w = t[f"blk.0.{name}.weight"].reshape(-1, width // 32, 34)
+            w[:, :, 2:] = 0
+            for head in range(heads):
+                _put(t[f"blk.0.{name}.weight"], width, head * 128 + 63, 0, 0.1, [-127 if name == "attn_k" else 0, 64] + [0] * 30)
+            t[f"blk.0.{name}_norm.weight"] = np.full(128, 3.0, np.float32)
+    session = hip.decode.Qwen3Session(f.metadata, t, capacity=n_prompt + 4)
+    prompt = np.random.default_rng(n_prompt).integers(0, 999, n_prompt, dtype=np.uint32)
+    prompt[at] = special
+
+    def outcome(passes):
+        session.set_prompt_passes(passes)
+        try:
+            r = session.generate(prompt, 1, dump_steps=range(n_prompt))
+        except hip.hip.RmiHipError as e:
+            return str(e)
+        return r["dump"].view(np.uint32), r["argmax"], r["tokens"]
+
+    fast, slow = outcome(True), outcome(False)
+    session.close()
+    if seen:
+        assert f"{n_prompt - at} steps" in slow and fast == slow
+    else:
+        assert not isinstance(slow, str), slow
+        assert all(np.array_equal(a, b) for a, b in zip(fast, slow))
