@@ -1219,7 +1219,6 @@ struct rmi_hip_qwen3 : RmiSession {
     uint16_t *q16b = nullptr;
     int8_t *act_q8b = nullptr;
     void *partialb = nullptr;
-    float *wantb = nullptr;              // the logits that a pass was asked for, kPassWant rows
     float *attn_scratch = nullptr;       // of the pass's attention
     size_t attn_scratch_floats = 0;
     void *attn_split = nullptr;          // scratch of the split attention launches (head dimension 128)
@@ -1228,9 +1227,7 @@ struct rmi_hip_qwen3 : RmiSession {
     int enqueue_step(uint32_t step, hipStream_t st) override;
     const float *step_logits() const override { return logits; }
     bool pass_possible(uint32_t step0, uint32_t n) const override;
-    int enqueue_pass(uint32_t step0, uint32_t n, const uint32_t *want, uint32_t n_want, bool sample, hipStream_t st) override;
-    uint32_t max_pass_want() const override;
-    const float *pass_logits(uint32_t, uint32_t i) const override { return wantb + size_t(i) * cfg.vocab; }
+    int enqueue_pass(uint32_t step0, uint32_t n, const uint32_t *want, uint32_t n_want, bool sample, hipStream_t st, const RmiLogitsOf &of) override;
 };
 
 namespace {
@@ -1240,7 +1237,6 @@ namespace {
 // of 1999 tokens: 36.3 ms in passes of 512, 28.9 in passes of 1024).
 constexpr uint32_t kPromptBatch = 1024;
 constexpr uint32_t kHeadBatch = 128;  // positions whose logits are in memory at once
-constexpr uint32_t kPassWant = 64;    // logits of a pass that a caller can ask for
 inline uint32_t prompt_batch(uint32_t capacity) { return capacity < kPromptBatch ? capacity : kPromptBatch; }
 
 template <typename T>
@@ -1377,9 +1373,10 @@ bool prompt_pass_possible(const rmi_hip_qwen3 *s, uint32_t step0, uint32_t n) {
 // (the x86-64-order GEMV takes up to eight tokens a launch and gives each the bits it gets alone), the other
 // kernels run once per position inside one launch.  Position by position the arithmetic is that of enqueue_step's
 // separate-kernel path; a position's keys and values are in the cache before any attention launch of the pass
-// reads them.  Leaves every position's argmax and top-2 logits, the logits asked for in wantb, and, behind the last
-// position, the step counter and the next token's embedding as a single step expects them.
-int enqueue_prompt_pass(rmi_hip_qwen3 *s, uint32_t step0, uint32_t n, const uint32_t *want, uint32_t n_want, hipStream_t st) {
+// reads them.  Leaves every position's argmax and top-2 logits and, behind the last position, the step counter and the
+// next token's embedding as a single step expects them.
+int enqueue_prompt_pass(rmi_hip_qwen3 *s, uint32_t step0, uint32_t n, const uint32_t *want, uint32_t n_want, hipStream_t st,
+                        const RmiLogitsOf &of) {
     const rmi_hip_qwen3_config &c = s->cfg;
     const int rnd = c.rounding;
     StepParams *sp = static_cast<StepParams *>(s->params);
@@ -1427,9 +1424,7 @@ int enqueue_prompt_pass(rmi_hip_qwen3 *s, uint32_t step0, uint32_t n, const uint
         hipLaunchKernelGGL(argmax_final_batch_kernel<EmbedQ8>, dim3(nb), dim3(256), 0, st, static_cast<const Top *>(s->partialb), kArgmaxGroups,
                            sp, step0 + i0, static_cast<const uint32_t *>(nullptr), s->tok, s->step_argmax, s->step_top2, s->nonfinite,
                            EmbedQ8{s->embd->data, s->embd->n_units, c.vocab, s->x, c.n_embd});
-        for (; w < n_want && want[w] < i0 + nb; w++)
-            RMI_HIP_CHECK(hipMemcpyAsync(s->wantb + size_t(w) * c.vocab, s->logitsb + size_t(want[w] - i0) * c.vocab, size_t(c.vocab) * 4,
-                                         hipMemcpyDeviceToDevice, st));
+        for (; w < n_want && want[w] < i0 + nb; w++) of(step0 + want[w], s->logitsb + size_t(want[w] - i0) * c.vocab);
     }
     RMI_HIP_CHECK(hipGetLastError());
     return RMI_HIP_OK;
@@ -1439,10 +1434,9 @@ int enqueue_prompt_pass(rmi_hip_qwen3 *s, uint32_t step0, uint32_t n, const uint
 
 int rmi_hip_qwen3::enqueue_step(uint32_t step, hipStream_t st) { return ::enqueue_step(this, step, st); }
 bool rmi_hip_qwen3::pass_possible(uint32_t step0, uint32_t n) const { return prompt_pass_possible(this, step0, n); }
-int rmi_hip_qwen3::enqueue_pass(uint32_t step0, uint32_t n, const uint32_t *want, uint32_t n_want, bool, hipStream_t st) {
-    return enqueue_prompt_pass(this, step0, n, want, n_want, st);
+int rmi_hip_qwen3::enqueue_pass(uint32_t step0, uint32_t n, const uint32_t *want, uint32_t n_want, bool, hipStream_t st, const RmiLogitsOf &of) {
+    return enqueue_prompt_pass(this, step0, n, want, n_want, st, of);
 }
-uint32_t rmi_hip_qwen3::max_pass_want() const { return kPassWant; }
 rmi_hip_qwen3::~rmi_hip_qwen3() {
     if (head && head != embd) rmi_hip_free_weight(head);
     if (embd) rmi_hip_free_weight(embd);
@@ -1758,7 +1752,6 @@ rmi_hip_qwen3 *rmi_hip_qwen3_create(const rmi_hip_qwen3_config *cfg, const rmi_h
              (s->qkvb = dev_alloc<float>(s, n * (size_t(s->n_q) + s->n_k + s->n_v))) &&
              (s->q16b = dev_alloc<uint16_t>(s, n * s->n_q)) && (s->gub = dev_alloc<float>(s, n * 2 * c.n_ff)) &&
              (s->logitsb = dev_alloc<float>(s, head * c.vocab)) &&
-             (s->wantb = dev_alloc<float>(s, size_t(n < kPassWant ? n : kPassWant) * c.vocab)) &&
              (s->act_q8b = dev_alloc<int8_t>(s, n * s->max_n_in)) && (s->act_scalesb = dev_alloc<float>(s, n * s->max_n_in / 32)) &&
              (s->partialb = dev_alloc<Top>(s, head * kArgmaxGroups)) && (s->attn_scratch = dev_alloc<float>(s, s->attn_scratch_floats));
     }

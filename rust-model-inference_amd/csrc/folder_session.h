@@ -42,9 +42,8 @@ struct rmi_hip_folder_session : RmiSession {
     int enqueue_step(uint32_t step, hipStream_t st) override;
     const float *step_logits() const override { return logits; }
     bool pass_possible(uint32_t step0, uint32_t n) const override { return n <= pass_rows && step0 + n <= capacity; }
-    int enqueue_pass(uint32_t step0, uint32_t n, const uint32_t *want, uint32_t n_want, bool sample, hipStream_t st) override;
+    int enqueue_pass(uint32_t step0, uint32_t n, const uint32_t *want, uint32_t n_want, bool sample, hipStream_t st, const RmiLogitsOf &of) override;
     uint32_t max_pass_want() const override { return logit_rows; }
-    const float *pass_logits(uint32_t, uint32_t i) const override { return logits + size_t(i) * vocab; }
     int feed(const uint32_t *tokens, uint32_t n, const uint32_t *want, uint32_t n_want, float *out, float *host_layers);
 
   protected:

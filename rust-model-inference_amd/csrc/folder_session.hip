@@ -83,7 +83,8 @@ int rmi_hip_folder_session::enqueue_step(uint32_t step, hipStream_t st) {
     return rc;
 }
 
-int rmi_hip_folder_session::enqueue_pass(uint32_t step0, uint32_t n, const uint32_t *want, uint32_t n_want, bool sample, hipStream_t st) {
+int rmi_hip_folder_session::enqueue_pass(uint32_t step0, uint32_t n, const uint32_t *want, uint32_t n_want, bool sample, hipStream_t st,
+                                         const RmiLogitsOf &of) {
     int rc = embed_tokens(step0, n, st);
     if (rc == RMI_HIP_OK) rc = enqueue_layers(step0, n, st, nullptr);
     std::vector<uint32_t> rows(want, want + n_want);
@@ -94,6 +95,7 @@ int rmi_hip_folder_session::enqueue_pass(uint32_t step0, uint32_t n, const uint3
     rc = set_rows(rows.data(), uint32_t(rows.size()), st);
     if (rc == RMI_HIP_OK) rc = enqueue_logits(want_rows, uint32_t(rows.size()), st);
     if (rc == RMI_HIP_OK) rc = enqueue_sample(step0, want_rows, uint32_t(rows.size()), rows.back(), st);
+    for (uint32_t i = 0; rc == RMI_HIP_OK && i < n_want; i++) of(step0 + want[i], logits + size_t(i) * vocab);
     if (rows.back() == n - 1) embedded = step0 + n;
     return rc;
 }

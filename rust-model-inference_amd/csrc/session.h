@@ -3,12 +3,16 @@
 // src/models/qwen3.rs:581-1158, is the loop's model).
 #pragma once
 
+#include <functional>
 #include <vector>
 
 #include "rmi_internal.h"
 
 constexpr uint32_t kArgmaxGroups = 256;
 constexpr size_t kTopBytes = 16;  // one Top of device_sample.h
+
+// Called while a pass is enqueued, with a position and where its logits lie at that point of the stream.
+using RmiLogitsOf = std::function<void(uint32_t step, const float *logits)>;
 
 struct RmiSession {
     uint32_t vocab = 0, capacity = 0;
@@ -42,11 +46,10 @@ struct RmiSession {
     // Whether the prompt positions step0 .. step0 + n - 1 can go through one pass.
     virtual bool pass_possible(uint32_t step0, uint32_t n) const = 0;
     // Such a pass, after which the session stands where a single step would have left it.  want (ascending, below n):
-    // the positions whose logits the caller reads; a session may compute more.  sample: the pass ends the prompt.
-    virtual int enqueue_pass(uint32_t step0, uint32_t n, const uint32_t *want, uint32_t n_want, bool sample, hipStream_t st) = 0;
+    // the positions whose logits the caller reads, through `of`; a session may compute more.  sample: the pass ends the
+    // prompt.
+    virtual int enqueue_pass(uint32_t step0, uint32_t n, const uint32_t *want, uint32_t n_want, bool sample, hipStream_t st, const RmiLogitsOf &of) = 0;
     virtual uint32_t max_pass_want() const { return 0xffffffffu; }
-    // the logits of want[i] = offset
-    virtual const float *pass_logits(uint32_t offset, uint32_t i) const = 0;
 };
 
 // rmi_hip_<model>_generate: see rmi_hip_qwen3_generate in the header

@@ -83,7 +83,7 @@ int rmi_session_generate(RmiSession *s, const uint32_t *prompt, uint32_t n_promp
     const bool stops = !s->stop_ids.empty() && max_new > 0;
     uint32_t n_valid = max_new, steps_done = 0, checked = 0;
     std::vector<uint32_t> seen(stops ? max_new : 0), want;
-    auto dump = [&](uint32_t step, const float *logits) {
+    const RmiLogitsOf dump = [&](uint32_t step, const float *logits) {
         for (uint32_t d = 0; d < n_dump && e == hipSuccess; d++)
             if (dump_steps[d] == step)
                 e = hipMemcpyAsync(d_dump + size_t(d) * vocab, logits, size_t(vocab) * 4, hipMemcpyDeviceToDevice, st);
@@ -108,8 +108,7 @@ int rmi_session_generate(RmiSession *s, const uint32_t *prompt, uint32_t n_promp
                     n = want.back() + 1 - step;
                 }
                 for (uint32_t &w : want) w -= step;
-                rc = s->enqueue_pass(step, n, want.data(), uint32_t(want.size()), step + n == n_prompt, st);
-                for (uint32_t i = 0; rc == RMI_HIP_OK && i < want.size(); i++) dump(step + want[i], s->pass_logits(want[i], i));
+                rc = s->enqueue_pass(step, n, want.data(), uint32_t(want.size()), step + n == n_prompt, st, dump);
                 step += n;
                 continue;
             }

@@ -30,16 +30,17 @@ def test_passes_have_the_bits_of_single_steps(hip, tmp_path, heads, kv_heads, n_
     assert np.array_equal(fast["dump"].view(np.uint32), slow["dump"].view(np.uint32))
 
 
-def test_a_pass_that_is_asked_for_more_logits_than_it_holds(hip, tmp_path):
-    """64 positions' logits of a pass can be asked for; with more the pass ends early and the next one goes on."""
+@pytest.mark.parametrize("n_prompt", [200, 300])
+def test_logits_of_every_position_of_a_pass(hip, tmp_path, n_prompt):
+    """A pass makes logits 128 positions at a time and hands on those asked for, here all of them."""
     path = os.path.join(str(tmp_path), "m.gguf")
     hip.gguf.write_synthetic_qwen3(path, seed=9, n_layer=2, n_embd=256, n_head=4, n_head_kv=2, head_dim=128, n_ff=512, vocab=1000, n_ctx=4096)
     f = hip.gguf.GGUFFile(path)
-    session = hip.decode.Qwen3Session(f.metadata, {name: t[2] for name, t in f.tensors.items()}, capacity=202)
-    prompt = np.random.default_rng(4).integers(0, 1000, 200, dtype=np.uint32)
-    fast = session.generate(prompt, 2, dump_steps=range(201))
+    session = hip.decode.Qwen3Session(f.metadata, {name: t[2] for name, t in f.tensors.items()}, capacity=n_prompt + 2)
+    prompt = np.random.default_rng(4).integers(0, 1000, n_prompt, dtype=np.uint32)
+    fast = session.generate(prompt, 2, dump_steps=range(n_prompt + 1))
     session.set_prompt_passes(False)
-    slow = session.generate(prompt, 2, dump_steps=range(201))
+    slow = session.generate(prompt, 2, dump_steps=range(n_prompt + 1))
     session.close()
     assert np.array_equal(fast["dump"].view(np.uint32), slow["dump"].view(np.uint32))
 
