@@ -8,7 +8,8 @@
 // lets both be matrix products: v_mfma_f64_16x16x4 with sixteen positions as its rows.
 //
 // A workgroup of four waves takes sixteen consecutive positions of one query head:
-//   1  scores of sixteen keys a wave and turn into a row of scratch a position (L2), and each position's maximum;
+//   1  scores of sixteen keys a wave and turn into a row of scratch a position (at 2000 keys the rows of an XCD's workgroups,
+//      8 MB, are twice its L2), and each position's maximum;
 //   2  numerators, 64 keys of all sixteen positions a turn; lane r of the first wave adds position r's in order;
 //   3  weights and p . v, sixteen keys a wave and turn; the waves' sums meet in LDS, then the quantizer.
 // What bounds it: the matrix cores at f64 (64 clocks an instruction: 75 TFLOP/s), two of the four products of a
@@ -16,7 +17,8 @@
 // sixteen chains side by side on one wave, hidden behind the other workgroup of the compute unit.  Measured (16 heads, 512
 // positions): 46 us over the first 512 keys, 178 us at 2000 keys, half of the f64 rate; the kernel before it, a workgroup
 // a position and head on the vector ALU, took 31 us for 128 positions of the first 512 and went position by position from
-// 1280 keys on (a prompt of 1999 tokens, 28 layers: 885 -> 47.5 ms, one of 512 and 32 answers: 37.4 -> 33.0 ms).
+// 1280 keys on (a prompt of 1999 tokens, 28 layers: 885 -> 47.5 ms, one of 512 and 32 answers: 37.4 -> 33.0 ms);
+// it still does passes of up to 1024 positions times heads (pass_by_positions in decode_qwen3.hip).
 #include "attn_prompt.h"
 
 #include "device_math.h"

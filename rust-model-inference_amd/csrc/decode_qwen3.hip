@@ -514,8 +514,13 @@ struct AttnFromQkv {
     uint16_t *k_row, *v_row;         // the cache rows of this position, [n_head_kv][128] each
     float eps;
 };
-template <bool FROM_QKV, int PVP = 1>
-__global__ __launch_bounds__(kA128Threads, 2) void attention128_quant_kernel(
+// PASS: several consecutive positions, blockIdx.z, whose cache rows are filled already; q16, q8 and scales are theirs one
+// after the other.  Every phase is a stretch of dependent instructions, so one workgroup leaves its compute unit idle most
+// of the time; with the registers held to 80 (a short value prefetch) three workgroups share a unit and fill each other's
+// waits.
+constexpr int kPassWaves = 6;
+template <bool FROM_QKV, int PVP = 1, bool PASS = false>
+__global__ __launch_bounds__(kA128Threads, PASS ? kPassWaves : 2) void attention128_quant_kernel(
     const uint16_t *__restrict__ q16, const uint16_t *__restrict__ k_cache, const uint16_t *__restrict__ v_cache,
     uint32_t step, uint32_t kv_stride, uint32_t n_head, uint32_t n_head_kv, int8_t *__restrict__ q8,
     float *__restrict__ scales, int rounding, AttnFromQkv fq) {
@@ -523,6 +528,13 @@ __global__ __launch_bounds__(kA128Threads, 2) void attention128_quant_kernel(
     __shared__ float red_f[kA128Threads / 64];
     __shared__ uint64_t exp_tab[32];
     __shared__ __attribute__((aligned(16))) uint16_t new16[3][128];  // this step's q, k, v as f16
+    if constexpr (PASS) {
+        const uint32_t first = blockIdx.z * n_head * 128;
+        step += blockIdx.z;
+        q16 += first;
+        q8 += first;
+        scales += first / 32;
+    }
     // grid = (query heads per key/value head, key/value heads), or with PVP parts n_head * PVP workgroups in a row:
     // key/value head fastest, then the query head of its group, then the part
     static_assert(PVP == 1 || PVP == 2 || PVP == 4, "a part is one, two or four blocks of 32 dimensions");
@@ -581,8 +593,8 @@ __global__ __launch_bounds__(kA128Threads, 2) void attention128_quant_kernel(
     // With parts a slice is short (six keys a slice cover 768 keys with four parts; longer slices go on in the batches
     // further down) and its loads are unconditional: a load under
     // a branch makes the wait for this position's q, k, v (issued first) drain most of what was issued behind them.
-    constexpr uint32_t kPre = PVP == 1 ? (kA128Threads >= 1024 ? 12 : (kA128Threads >= 512 ? 20 : 40)) : 24 / PVP;
-    constexpr uint32_t kBatch = 8;  // keys of a slice in flight beyond the first kPre
+    constexpr uint32_t kPre = PASS ? 1 : PVP == 1 ? (kA128Threads >= 1024 ? 12 : (kA128Threads >= 512 ? 20 : 40)) : 24 / PVP;
+    constexpr uint32_t kBatch = PASS ? 2 : 8;  // keys of a slice in flight beyond the first kPre
     const uint32_t dg = tid % kDgLanes, sl = tid / kDgLanes;
     const uint32_t chunk = (n_cached + kSlices - 1) / kSlices;
     const uint32_t t_begin = sl * chunk, t_end = t_begin + chunk < n_cached ? t_begin + chunk : n_cached;
@@ -682,7 +694,7 @@ __global__ __launch_bounds__(kA128Threads, 2) void attention128_quant_kernel(
     if (tid == 0) {  // the reference adds the weights one after the other in f32; the padding zeros change nothing
         // one lane, one dependent chain of adds; the LDS reads run 32 values ahead of it (two buffers, no copies)
         float acc = 0.0f;
-        constexpr int kAhead = 8;  // float4 of each buffer
+        constexpr int kAhead = PASS ? 4 : 8;  // float4 of each buffer
         float4 a[kAhead], b[kAhead];
 #pragma unroll
         for (int j = 0; j < kAhead; j++) a[j] = reinterpret_cast<const float4 *>(scores)[j];
@@ -1369,6 +1381,16 @@ bool prompt_pass_possible(const rmi_hip_qwen3 *s, uint32_t step0, uint32_t n) {
     return s->xb && n > 0 && n <= prompt_batch(c.capacity) && step0 + n <= c.capacity && c.n_embd <= kNormMaxN;
 }
 
+// Whether a pass's attention takes a workgroup a position and head, as a single step's does, instead of one for sixteen
+// positions.  Sixteen positions' ordered sums and scratch are a longer chain that only pays where the chip has enough to do
+// in its shadow: up to four workgroups a compute unit the first way is never slower, whatever the context (16 heads, 12
+// layers, us a layer and pass, a workgroup a position | sixteen: 2 positions 33.2 | 37.4, 16: 39.9 | 43.6, 64: 57.1 | 57.4,
+// 96: 67.3 | 65.1; behind 900 keys 2: 44 | 87, 64: 84 | 105, 128: 121 | 112; 32 heads: 32: 53.2 | 53.8, 48: 62.7 | 57.3).
+// Its keys lie in LDS, as much as a launch may take unasked (64 KiB, the kernel's own arrays among them).
+bool pass_by_positions(const rmi_hip_qwen3_config &c, uint32_t step0, uint32_t n) {
+    return uint64_t(n) * c.n_head <= 4u * uint32_t(rmi_device_cus()) && attn128_lds_bytes(step0 + n) <= 62 * 1024;
+}
+
 // n consecutive prompt positions from step0 on in one pass: every product reads its weight once for all of them
 // (the x86-64-order GEMV takes up to eight tokens a launch and gives each the bits it gets alone), the other
 // kernels run once per position inside one launch.  Position by position the arithmetic is that of enqueue_step's
@@ -1396,9 +1418,13 @@ int enqueue_prompt_pass(rmi_hip_qwen3 *s, uint32_t step0, uint32_t n, const uint
         hipLaunchKernelGGL(qk_norm_rope_store_kernel, dim3(c.n_head + 2 * c.n_head_kv, n), dim3(64), 0, st, s->qkvb, qn, kn,
                            s->cos_t, s->sin_t, step0, s->q16b, s->k_cache + row, s->v_cache + row, c.n_head, c.n_head_kv,
                            c.head_dim_k, c.head_dim_v, c.eps, TokStride3{n_qkv, s->n_q, s->kv_stride});
-        rc = rmi_launch_attn128_prompt(s->q16b, s->k_cache + layer_base, s->v_cache + layer_base, step0, n, s->kv_stride, c.n_head, c.n_head_kv,
-                                       s->attn_scratch, s->attn_scratch_floats, s->act_q8b, s->act_scalesb, rnd, st);
-        if (rc != RMI_HIP_OK) return rc;
+        if (pass_by_positions(c, step0, n))
+            hipLaunchKernelGGL((attention128_quant_kernel<false, 1, true>), dim3(c.n_head / c.n_head_kv, c.n_head_kv, n), dim3(kA128Threads),
+                               attn128_lds_bytes(step0 + n), st, s->q16b, s->k_cache + layer_base, s->v_cache + layer_base, step0, s->kv_stride,
+                               c.n_head, c.n_head_kv, s->act_q8b, s->act_scalesb, rnd, AttnFromQkv{});
+        else if ((rc = rmi_launch_attn128_prompt(s->q16b, s->k_cache + layer_base, s->v_cache + layer_base, step0, n, s->kv_stride, c.n_head,
+                                                 c.n_head_kv, s->attn_scratch, s->attn_scratch_floats, s->act_q8b, s->act_scalesb, rnd, st)) != RMI_HIP_OK)
+            return rc;
         rc = rmi_gemv_q8_0_tokens(s->w_o[l], s->act_q8b, s->act_scalesb, s->residb, n, c.n_embd, 0, c.n_embd, st);
         if (rc != RMI_HIP_OK) return rc;
         launch_add_rmsnorm_quant(s->xb, s->residb, s->ffn_norm[l], c.n_embd, c.eps, s->act_q8b, s->act_scalesb, rnd, st, n,

@@ -1,5 +1,5 @@
-"""Prompt passes of the Qwen3 session over the range of contexts: sixteen positions of a head share a workgroup of the
-pass's attention, so lengths on both sides of a tile, of a 64-key turn and of a pass, with the keys of earlier passes in
+"""Prompt passes of the Qwen3 session over the range of contexts: in larger passes sixteen positions of a head share a
+workgroup of the attention, so lengths on both sides of a tile, of a 64-key turn and of a pass, with the keys of earlier passes in
 front.  Every position its own step is the reference (held to the CPU loop by test_gpu_decode_device.py): all bits equal."""
 import os
 
@@ -11,7 +11,9 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("heads,kv_heads,n_prompt,per_pass", [
     (8, 4, 2, True), (8, 4, 16, True), (8, 4, 17, True), (3, 3, 65, True), (8, 2, 127, 33), (4, 1, 512, True), (4, 4, 513, True),
-    (2, 1, 700, 129), (4, 2, 1300, True), (2, 2, 2100, True)])
+    (2, 1, 700, 129), (4, 2, 1300, True), (2, 2, 2100, True),
+    # up to 1024 positions times heads (256 compute units) a workgroup takes one position, beyond that sixteen
+    (8, 4, 128, True), (8, 4, 129, True), (64, 8, 16, True), (64, 8, 17, True), (64, 16, 33, True), (32, 8, 700, 40), (64, 8, 300, 63), (32, 4, 700, 30)])
 def test_passes_have_the_bits_of_single_steps(hip, tmp_path, heads, kv_heads, n_prompt, per_pass):
     path = os.path.join(str(tmp_path), "m.gguf")
     hip.gguf.write_synthetic_qwen3(path, seed=heads, n_layer=2, n_embd=256, n_head=heads, n_head_kv=kv_heads, head_dim=128, n_ff=512, vocab=1000,
@@ -53,12 +55,12 @@ def _put(raw, n_in, row, block, scale, quants):
 
 
 @pytest.mark.parametrize("seen", [True, False])
-@pytest.mark.parametrize("n_prompt,at", [(5, 4), (7, 2), (33, 32), (40, 20), (40, 35), (100, 80), (130, 129)])
-def test_a_value_that_is_not_finite_counts_from_its_position_on(hip, tmp_path, n_prompt, at, seen):
+@pytest.mark.parametrize("heads,n_prompt,at", [(2, 5, 4), (2, 40, 20), (64, 17, 16), (64, 18, 2), (64, 33, 32), (64, 40, 20), (64, 40, 35), (64, 100, 80), (64, 130, 129)])
+def test_a_value_that_is_not_finite_counts_from_its_position_on(hip, tmp_path, heads, n_prompt, at, seen):
     """One prompt token's values overflow f16.  seen: its weight is not zero, so that its position and those behind it have
     logits that are not finite, and their number is in the error.  Otherwise every weight of it rounds to zero: 0 x inf is
     NaN, which the quantizer drops, from that position on and not before."""
-    width, heads, special = 256, 2, 999
+    width, special = 256, 999
     path = os.path.join(str(tmp_path), "m.gguf")
     hip.gguf.write_synthetic_qwen3(path, seed=5, n_layer=1, n_embd=width, n_head=heads, n_head_kv=heads, head_dim=128, n_ff=256, vocab=1000, n_ctx=4096)
     f = hip.gguf.GGUFFile(path)
