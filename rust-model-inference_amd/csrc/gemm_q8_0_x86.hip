@@ -163,9 +163,9 @@ __global__ __launch_bounds__(64 * WR * WT, WPS) void gemm_q8_0_x86_kernel(RmiGem
         for (int j = 0; j < NT; j++) f.xd[j] = *reinterpret_cast<const float *>(base + kScaleB + (b * BT + wt + j * 16 + fr) * 4);
     };
     // A block's products, one ahead of the sums.  The empty statements hold that order: left to itself the compiler issues
-    // every product of a quad first and spills the results, or each right in front of its sums and waits for it.  A result
-    // that passed through one is opaque to the compiler's own wait states; sixteen fmas lie between it and its first reader
-    // (an instruction of eight passes asks for eleven wait states).
+    // every product of a quad first and spills the results, or each right in front of its sums and waits for it.  They hold
+    // no instruction, so the wait states between a product and its first reader stay the compiler's own (it counts them on
+    // the finished code, past such a statement; tests/test_build_checks.py pins that).
 #define X86_SUMS(c) "+v"(c[0][h]), "+v"(c[0][2 + h]), "+v"(c[0][4 + h]), "+v"(c[0][6 + h]), "+v"(c[1][h]), "+v"(c[1][2 + h]), \
                     "+v"(c[1][4 + h]), "+v"(c[1][6 + h]), "+v"(c[2][h]), "+v"(c[2][2 + h]), "+v"(c[2][4 + h]), "+v"(c[2][6 + h]), \
                     "+v"(c[3][h]), "+v"(c[3][2 + h]), "+v"(c[3][4 + h]), "+v"(c[3][6 + h])

@@ -6,6 +6,8 @@ import os
 import subprocess
 import sys
 
+import pytest
+
 HERE = os.path.dirname(os.path.abspath(__file__))
 CHECK = os.path.join(HERE, "..", "rust-model-inference_amd", "csrc", "check_dpp_hazards.py")
 
@@ -99,3 +101,44 @@ def test_reading_a_matrix_core_result_too_early_fails(tmp_path):
     assert _run(tmp_path, [mfma, "s_nop 3", use]).returncode == 1
     assert _run(tmp_path, [mfma, "v_mov_b32_e32 v9, v1", use]).returncode == 0  # v9 is another value by then
     assert _run(tmp_path, ["v_mfma_i32_32x32x32_i8 v[0:15], v[16:19], v[20:23], 0"]).returncode == 1
+
+
+HIPCC = "/opt/rocm/bin/hipcc"
+
+
+@pytest.mark.skipif(not os.path.exists(HIPCC), reason="no device compiler")
+def test_an_empty_asm_statement_hides_no_matrix_core_result(tmp_path):
+    """Kernels hold the order of their products with asm statements that contain nothing.  The compiler looks past such a
+    statement when it puts the wait states between a product and its first reader: as many with it as without."""
+    body = """
+    typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
+    typedef float f32x16 __attribute__((ext_vector_type(16)));
+    typedef float f32x4 __attribute__((ext_vector_type(4)));
+    typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+    #define K(name, R, T, mfma, between) extern "C" __global__ void name(T *a, float *p, float s) { \\
+        R d = mfma(a[threadIdx.x], a[threadIdx.x + 64], R{}, 0, 0, 0); between; p[threadIdx.x] = d[3] * s; }
+    #define BOTH(name, R, T, mfma) K(name##_plain, R, T, mfma, ) K(name##_held, R, T, mfma, asm volatile("" : "+v"(d)))
+    BOTH(four, f32x4, f16x4, __builtin_amdgcn_mfma_f32_4x4x4f16)
+    BOTH(x86, f32x16, f16x4, __builtin_amdgcn_mfma_f32_16x16x4f16)
+    BOTH(bf16, f32x4, bf16x8, __builtin_amdgcn_mfma_f32_16x16x32_bf16)
+    BOTH(f32, f32x4, float, __builtin_amdgcn_mfma_f32_16x16x4f32)
+    """
+    src, out = tmp_path / "k.hip", tmp_path / "k.s"
+    src.write_text("#include <hip/hip_runtime.h>\n" + body)
+    subprocess.run([HIPCC, "--offload-arch=gfx950", "-O3", "-mllvm", "-amdgpu-mfma-vgpr-form=1", "-S", "--cuda-device-only", str(src), "-o", str(out)],
+                   check=True, capture_output=True)
+    waits, name, after = {}, None, None
+    for line in out.read_text().splitlines():
+        word = line.split(";")[0].split()
+        if not word:
+            continue
+        if word[0].endswith(("_plain:", "_held:")):
+            name, after = word[0][:-1], None
+        elif word[0].startswith("v_mfma"):
+            after = 0
+        elif word[0] == "v_mul_f32_e32" and after is not None:
+            waits[name], after = after, None
+        elif after is not None:
+            after += int(word[1]) + 1 if word[0] == "s_nop" else 1
+    assert len(waits) == 8 and all(waits[k + "_held"] == waits[k + "_plain"] > 4 for k in ("four", "x86", "bf16", "f32")), waits
+    assert waits["x86_held"] >= 11
