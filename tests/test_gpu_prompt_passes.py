@@ -98,3 +98,21 @@ def test_a_value_that_is_not_finite_counts_from_its_position_on(hip, tmp_path, h
     else:
         assert not isinstance(slow, str), slow
         assert all(np.array_equal(a, b) for a, b in zip(fast, slow))
+
+
+def test_a_pass_whose_scores_exceed_the_scratch(hip, tmp_path):
+    """64 heads' scores of 1024 positions at a capacity of 2000 are more than the 256 MB of scratch: several launches a pass."""
+    heads, n_prompt = 64, 1990
+    path = os.path.join(str(tmp_path), "m.gguf")
+    hip.gguf.write_synthetic_qwen3(path, seed=2, n_layer=1, n_embd=64, n_head=heads, n_head_kv=8, head_dim=128, n_ff=64, vocab=500, n_ctx=4096)
+    f = hip.gguf.GGUFFile(path)
+    session = hip.decode.Qwen3Session(f.metadata, {name: t[2] for name, t in f.tensors.items()}, capacity=2000)
+    prompt = np.random.default_rng(3).integers(0, 500, n_prompt, dtype=np.uint32)
+    dumps = [0, 255, 500, 511, 512, 800, 1023, 1024, 1500, 1700, 1989, 1992]
+    fast = session.generate(prompt, 4, dump_steps=dumps)
+    session.set_prompt_passes(False)
+    slow = session.generate(prompt, 4, dump_steps=dumps)
+    session.close()
+    assert np.array_equal(fast["tokens"], slow["tokens"]) and np.array_equal(fast["argmax"], slow["argmax"])
+    assert np.array_equal(fast["top2"].view(np.uint32), slow["top2"].view(np.uint32))
+    assert np.array_equal(fast["dump"].view(np.uint32), slow["dump"].view(np.uint32))
