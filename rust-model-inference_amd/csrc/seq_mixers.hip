@@ -234,7 +234,9 @@ __global__ __launch_bounds__(256) void conv_rotate_pairs_kernel(RmiAttnShape s, 
 // token; a wave takes QT tiles of sixteen.  Scores come as K q (rows: keys, columns: queries), so a lane holds the
 // weights of one column and the running maximum and sum are a lane's own; the weights then are the operand of
 // V^T p as they lie, because the value blocks hold their keys in that order.
-template <typename T, int BUCKET, int QT>
+// EVERY: every load of a block is made, a piece past a narrower head's end as the last one again, for a load behind a branch,
+// even one that all lanes take, is waited for before the next is issued.  Otherwise only what is there: attn_pass says where.
+template <typename T, int BUCKET, int QT, bool EVERY = true>
 struct AttnWave {
     static constexpr uint32_t kKC = BUCKET / (4 * kPieceElems<T>);  // 16-byte pieces a lane holds of a head's keys
     static constexpr uint32_t kVT = BUCKET / 16;
@@ -252,18 +254,21 @@ struct AttnWave {
         }
     }
     // A block's keys and values fit in registers beside the rest: values of a block and keys of the next are under way
-    // while the block's scores and weights are computed.  Every load is made, a piece past a narrower head's end as the
-    // last one again: a load behind a branch, even one that all lanes take, is waited for before the next is issued.
-    static constexpr bool kAhead = BUCKET * sizeof(T) <= 256 || (QT == 1 && BUCKET * sizeof(T) <= 512);
+    // while the block's scores and weights are computed.
+    static constexpr bool kAhead = BUCKET * sizeof(T) <= 256 || (EVERY && QT == 1 && BUCKET * sizeof(T) <= 512);
     static constexpr uint32_t kVP = sizeof(T) / 2;  // pieces a lane holds of a value tile
     u32x4 kf[2][kAhead ? kKC : 1], vf[kAhead ? kVT * kVP : 1];
+
+    static __device__ __forceinline__ uint32_t piece(uint32_t c, uint32_t n) { return !EVERY || c < n ? c : n - 1; }
+    static __device__ __forceinline__ bool skipped(uint32_t c, uint32_t n) { return !EVERY && c >= n; }
 
     __device__ __forceinline__ void load_keys(const T *kc, const RmiAttnShape &s, uint32_t k) {
         const uint32_t lane = threadIdx.x & 63, n_kc = s.dk_pad / (4 * kPieceElems<T>);
         const T *row = kc + size_t(k + (lane & 15)) * s.dk_pad + (lane >> 4) * kPieceElems<T>;
 #pragma unroll
         for (uint32_t c = 0; c < (kAhead ? kKC : 0); c++) {
-            const T *p = row + (c < n_kc ? c : n_kc - 1) * 4 * kPieceElems<T>;
+            if (skipped(c, n_kc)) continue;
+            const T *p = row + piece(c, n_kc) * 4 * kPieceElems<T>;
             kf[0][c] = *reinterpret_cast<const u32x4 *>(p);
             kf[1][c] = *reinterpret_cast<const u32x4 *>(p + 16 * size_t(s.dk_pad));
         }
@@ -279,7 +284,7 @@ struct AttnWave {
         for (uint32_t v = 0; v < (kAhead ? kVT : 0); v++)
 #pragma unroll
             for (uint32_t t = 0; t < kVP; t++)
-                vf[v * kVP + t] = *reinterpret_cast<const u32x4 *>(vb + size_t(v < n_vt ? v : n_vt - 1) * 16 * kKeyBlock + t * 16);
+                if (!skipped(v, n_vt)) vf[v * kVP + t] = *reinterpret_cast<const u32x4 *>(vb + size_t(piece(v, n_vt)) * 16 * kKeyBlock + t * 16);
     }
     // key o of the loaded block and its value come from LDS: a token's own, which this launch makes
     __device__ __forceinline__ void put_own(const T *key, const T *value, const RmiAttnShape &s, uint32_t o) {
@@ -328,7 +333,7 @@ struct AttnWave {
         if (!loaded && k0 < k1) load_keys(kc, s, row);
         for (uint32_t k = k0; k < k1; k += kKeyBlock) {
             const T *vb = value_at(vc, s, row);
-            constexpr uint32_t kGroup = 4;  // pieces of each half under way together where a block does not fit
+            constexpr uint32_t kGroup = EVERY ? 4 : 1;  // pieces of each half under way together where a block does not fit
             u32x4 kg[2][kAhead ? 1 : kGroup], vg[kAhead ? 1 : kGroup * kVP];
             if (!loaded || k != k0) load_values(vc, s, row);
             const uint32_t next = row + kKeyBlock < s.capacity ? row + kKeyBlock : 0;
@@ -337,10 +342,11 @@ struct AttnWave {
             for (int i = 0; i < QT; i++) sc[i][0] = sc[i][1] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (uint32_t c = 0; c < kKC; c++) {
+                if (skipped(c, n_kc)) continue;
                 if constexpr (!kAhead) if (c % kGroup == 0) {
 #pragma unroll
                     for (uint32_t j = 0; j < kGroup; j++) {
-                        const T *p = krow + size_t(row) * s.dk_pad + (c + j < n_kc ? c + j : n_kc - 1) * 4 * kPieceElems<T>;
+                        const T *p = krow + size_t(row) * s.dk_pad + piece(c + j, n_kc) * 4 * kPieceElems<T>;
                         kg[0][j] = *reinterpret_cast<const u32x4 *>(p);
                         kg[1][j] = *reinterpret_cast<const u32x4 *>(p + 16 * size_t(s.dk_pad));
                     }
@@ -395,11 +401,12 @@ struct AttnWave {
             }
 #pragma unroll
             for (uint32_t v = 0; v < kVT; v++) {
+                if (skipped(v, n_vt)) continue;
                 if constexpr (!kAhead) if (v % kGroup == 0) {
 #pragma unroll
                     for (uint32_t j = 0; j < kGroup * kVP; j++) {
                         const uint32_t tile = v + j / kVP;
-                        vg[j] = *reinterpret_cast<const u32x4 *>(vb + size_t(tile < n_vt ? tile : n_vt - 1) * 16 * kKeyBlock + j % kVP * 16);
+                        vg[j] = *reinterpret_cast<const u32x4 *>(vb + size_t(piece(tile, n_vt)) * 16 * kKeyBlock + j % kVP * 16);
                     }
                 }
                 if (v >= n_vt) continue;
@@ -433,13 +440,13 @@ __device__ __forceinline__ void attn_store(const RmiAttnShape &s, const RmiAttnA
 }
 
 // several tokens: a workgroup takes QT tiles, each of its four waves a quarter of the keys they see; merged in LDS
-template <typename T, int BUCKET, int QT>
+template <typename T, int BUCKET, int QT, bool EVERY>
 __global__ __launch_bounds__(256) void attn_pass_kernel(RmiAttnShape s, RmiAttnArgs a) {
     extern __shared__ __attribute__((aligned(16))) uint8_t lds_raw[];
     const uint32_t tid = threadIdx.x, lane = tid & 63, wave = uint32_t(__builtin_amdgcn_readfirstlane(int(tid >> 6))), fr = lane & 15, g4 = lane >> 4;
     const uint32_t group = s.heads / s.kv_heads, kvh = blockIdx.x % s.kv_heads, n_cols = a.n_tokens * group;
     const uint32_t tile = gridDim.x / s.kv_heads - 1 - blockIdx.x / s.kv_heads;  // the longest columns first
-    AttnWave<T, BUCKET, QT> w;
+    AttnWave<T, BUCKET, QT, EVERY> w;
     w.init();
     int last[QT];
     const uint32_t n_kc = s.dk_pad / (4 * kPieceElems<T>);
@@ -450,7 +457,8 @@ __global__ __launch_bounds__(256) void attn_pass_kernel(RmiAttnShape s, RmiAttnA
         const T *q = static_cast<const T *>(a.q) + (size_t(kvh) * n_cols + cc) * s.dk_pad + g4 * kPieceElems<T>;
 #pragma unroll
         for (uint32_t c = 0; c < w.kKC; c++) {
-            w.qf[i][c] = *reinterpret_cast<const u32x4 *>(q + (c < n_kc ? c : 0) * 4 * kPieceElems<T>);
+            if (w.skipped(c, n_kc)) continue;
+            w.qf[i][c] = *reinterpret_cast<const u32x4 *>(q + w.piece(c, n_kc) * 4 * kPieceElems<T>);
         }
     }
     const uint32_t first_col = tile * QT * 16, live = n_cols - first_col < QT * 16 ? n_cols - first_col : QT * 16;
@@ -1131,16 +1139,27 @@ int attn_pass(const RmiAttnShape &s, const RmiAttnArgs &a, hipStream_t st) {
         const int rc = bucket == 64 ? go(attn_split_kernel<T, 64>) : bucket == 128 ? go(attn_split_kernel<T, 128>) : go(attn_split_kernel<T, 256>);
         if (rc != RMI_HIP_OK) return rc;
     } else {
-        auto go = [&](auto kernel, uint32_t qt) {
+        const uint32_t qt = bucket == 256 ? 1 : 2, blocks = (n_cols + 16 * qt - 1) / (16 * qt) * s.kv_heads;
+        auto go = [&](auto kernel) {
             const size_t lds = size_t(4) * qt * 16 * (s.dv_pad + 6) * 4;
             const int rc = rmi_allow_lds(kernel, lds);
-            if (rc == RMI_HIP_OK)
-                hipLaunchKernelGGL(kernel, dim3((n_cols + 16 * qt - 1) / (16 * qt) * s.kv_heads), dim3(256), lds, st, s, a);
+            if (rc == RMI_HIP_OK) hipLaunchKernelGGL(kernel, dim3(blocks), dim3(256), lds, st, s, a);
             return rc;
         };
-        const int rc = bucket == 64    ? go(attn_pass_kernel<T, 64, 2>, 2)
-                       : bucket == 128 ? go(attn_pass_kernel<T, 128, 2>, 2)
-                                       : go(attn_pass_kernel<T, 256, 1>, 1);
+        auto with = [&](auto every) {
+            return bucket == 64    ? go(attn_pass_kernel<T, 64, 2, every.value>)
+                   : bucket == 128 ? go(attn_pass_kernel<T, 128, 2, every.value>)
+                                   : go(attn_pass_kernel<T, 256, 1, every.value>);
+        };
+        // With few workgroups a compute unit the waits for loads behind branches count (256 elements a head of bf16, 300
+        // tokens: 25.8 us, 15.3 with every load); with many the other waves cover them, and every load costs its issue and,
+        // in a narrower head, those past its end (2048 tokens of bf16: 128 elements 60.7 and 62.6, 160 of 256 111 and 148;
+        // f32 160 of 256 331 and 457, 300 tokens 29.0 and 30.2).  Heads that fill the bucket gain by it however many there
+        // are where a block's loads are most: 256 elements, bf16 234 and 211, f32 513 and 506; 128 of f32 215 and 207.
+        const bool filled = s.dk_pad == bucket && s.dv_pad == bucket;
+        const uint64_t cus = uint64_t(rmi_device_cus());
+        const bool branches = sizeof(T) == 2 ? !(filled && bucket == 256) && 2 * uint64_t(blocks) > (bucket == 64 ? 6 : 5) * cus : !filled && blocks > cus;
+        const int rc = branches ? with(std::false_type()) : with(std::true_type());
         if (rc != RMI_HIP_OK) return rc;
     }
     RMI_HIP_CHECK(hipGetLastError());
