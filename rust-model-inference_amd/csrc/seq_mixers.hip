@@ -542,7 +542,7 @@ __device__ __forceinline__ void attn_split(const RmiAttnShape &s, const RmiAttnA
     const T *kc = static_cast<const T *>(a.k_cache) + size_t(kvh) * s.capacity * s.dk_pad;
     const T *vc = static_cast<const T *>(a.v_cache) + size_t(kvh) * s.capacity * s.dv_pad;
     const uint32_t p0 = begin + part * keys_per_part, p1 = p0 + keys_per_part < n_keys ? p0 + keys_per_part : n_keys;
-    const uint32_t per_wave = (keys_per_part + NW * kKeyBlock - 1) / (NW * kKeyBlock) * kKeyBlock;
+    const uint32_t per_wave = keys_per_part / NW;  // a multiple of the key block
     const uint32_t k0 = p0 + wave * per_wave, k1 = k0 + per_wave < p1 ? k0 + per_wave : p1;
     const uint32_t live = n_cols - ct * 16 < 16 ? n_cols - ct * 16 : 16, pairs_out = live * s.dv_pad;
     auto gate_at = [&](uint32_t e) {
@@ -1075,7 +1075,7 @@ __global__ __launch_bounds__(256) void recur_norm_kernel(RmiRecurShape s, RmiRec
 }
 
 // ------------------------------------------------------------------ launches
-// Keys over workgroups where the columns alone would not fill the chip; at most kMaxParts parts of about 128 keys or more.
+// Keys over workgroups where the columns alone would not fill the chip; at most kMaxParts parts of 128 keys or more.
 constexpr uint32_t kSplitMaxCols = 256;  // per key/value head
 SplitPlan attn_parts(const RmiAttnShape &s, uint32_t n_tokens, uint32_t pos0) {
     uint32_t n_keys = pos0 + n_tokens;
@@ -1084,13 +1084,14 @@ SplitPlan attn_parts(const RmiAttnShape &s, uint32_t n_tokens, uint32_t pos0) {
     const uint64_t seen = s.window ? uint64_t(s.window) + 15 / group + 1 + kKeyBlock : n_keys;
     if (seen < n_keys) n_keys = uint32_t(seen);
     const uint32_t slots = s.kv_heads * tiles, cus = uint32_t(rmi_device_cus());
-    uint32_t p = (n_keys + 4 * kKeyBlock - 1) / (4 * kKeyBlock);
+    uint32_t p = (n_keys + 127) / 128;
     const uint32_t fill = (cus + slots - 1) / slots;
     if (p > fill) p = fill;
     if (p > kMaxParts) p = kMaxParts;
     if (slots > kAttnCounters || p < 1) p = 1;
     SplitPlan plan;
-    plan.keys_per_part = ((n_keys + p - 1) / p + kKeyBlock - 1) / kKeyBlock * kKeyBlock;
+    constexpr uint32_t kAlign = 4 * kKeyBlock;  // each wave whole blocks: a finer cut makes more parts, and no wave's keys fewer
+    plan.keys_per_part = ((n_keys + p - 1) / p + kAlign - 1) / kAlign * kAlign;
     plan.parts = Div((n_keys + plan.keys_per_part - 1) / plan.keys_per_part);
     plan.tiles = Div(tiles);
     plan.group = Div(group);
