@@ -523,7 +523,7 @@ struct SplitPlan {
     uint32_t keys_per_part, own;  // own: the row of the first token's key
 };
 
-template <typename T, int BUCKET, bool STEP>
+template <typename T, int BUCKET, bool STEP, bool EVERY = true>
 __device__ __forceinline__ void attn_split(const RmiAttnShape &s, const RmiAttnArgs &a, uint32_t block, const SplitPlan &plan, uint8_t *lds,
                                            uint32_t *flag) {
     constexpr uint32_t NW = 4, NT = 256;
@@ -535,7 +535,7 @@ __device__ __forceinline__ void attn_split(const RmiAttnShape &s, const RmiAttnA
     auto token_of = [&](uint32_t column) { return STEP ? 0 : plan.group.quot(column); };
     const uint32_t begin = first_block(s, a.pos0 + token_of(ct * 16)), n_keys = a.pos0 + token_of(last_col) + 1;  // what the tile sees
     const uint32_t n_kc = s.dk_pad / (4 * kPieceElems<T>);
-    AttnWave<T, BUCKET, 1> w;
+    AttnWave<T, BUCKET, 1, EVERY> w;
     w.init();
     const uint32_t col = ct * 16 + fr, cc = col < n_cols ? col : n_cols - 1;
     const int last[1] = {int(a.pos0 + token_of(cc))};
@@ -549,7 +549,9 @@ __device__ __forceinline__ void attn_split(const RmiAttnShape &s, const RmiAttnA
         const uint32_t mc = ct * 16 + plan.dv_pad.quot(e < pairs_out ? e : 0), t = token_of(mc);
         return a.gate ? a.gate + size_t(t) * s.heads + kvh * group + mc - t * group : a.u;
     };
-    float gate0 = *gate_at(tid);  // of the first result that this thread may write: under way from here on
+    // the gate of the first result that this thread may write: a token's is under way from here on; with several tokens the
+    // wait for it would stand before the first keys' loads
+    float gate0 = STEP ? *gate_at(tid) : 0.0f;
     bool loaded = false;
     if constexpr (STEP) {
         T *q = reinterpret_cast<T *>(lds), *own_k = q + 16 * s.dk_pad, *own_v = own_k + s.dk_pad;
@@ -659,10 +661,11 @@ __device__ __forceinline__ void attn_split(const RmiAttnShape &s, const RmiAttnA
         const T *q = static_cast<const T *>(a.q) + (size_t(kvh) * n_cols + cc) * s.dk_pad + g4 * kPieceElems<T>;
 #pragma unroll
         for (uint32_t c = 0; c < w.kKC; c++) {
-            w.qf[0][c] = *reinterpret_cast<const u32x4 *>(q + (c < n_kc ? c : 0) * 4 * kPieceElems<T>);
+            if (w.skipped(c, n_kc)) continue;
+            w.qf[0][c] = *reinterpret_cast<const u32x4 *>(q + w.piece(c, n_kc) * 4 * kPieceElems<T>);
         }
     }
-    asm volatile("" : "+v"(gate0));
+    if constexpr (STEP) asm volatile("" : "+v"(gate0));
     if (k0 < k1) w.keys(kc, vc, s, k0, k1, last, loaded);
     // the waves' results to LDS, live columns only; then every thread merges (column, channel) pairs
     const uint32_t pf = attn_part_floats(s.dv_pad), pl = 32 + live * s.dv_pad;
@@ -683,7 +686,7 @@ __device__ __forceinline__ void attn_split(const RmiAttnShape &s, const RmiAttnA
         const uint32_t c = plan.dv_pad.quot(e), d = e - c * s.dv_pad;
         if (d >= s.vdim) return;
         const uint32_t mc = ct * 16 + c, t = token_of(mc), head = kvh * group + mc - t * group;
-        const float g = e == tid ? gate0 : *gate_at(e);
+        const float g = STEP && e == tid ? gate0 : *gate_at(e);
         static_cast<T *>(a.out)[size_t(t) * a.out_ld + size_t(head) * s.vdim + d] = from_f32<T>(o * ((a.gate ? g : 1.0f) / sum));
     };
     for (uint32_t e = tid; e < pairs_out; e += NT) {
@@ -755,11 +758,11 @@ __device__ __forceinline__ void attn_split(const RmiAttnShape &s, const RmiAttnA
     }
 }
 
-template <typename T, int BUCKET>
+template <typename T, int BUCKET, bool EVERY>
 __global__ __launch_bounds__(256) void attn_split_kernel(RmiAttnShape s, RmiAttnArgs a, SplitPlan plan) {
     extern __shared__ __attribute__((aligned(16))) uint8_t lds_raw[];
     __shared__ uint32_t flag;
-    attn_split<T, BUCKET, false>(s, a, blockIdx.x, plan, lds_raw, &flag);
+    attn_split<T, BUCKET, false, EVERY>(s, a, blockIdx.x, plan, lds_raw, &flag);
 }
 
 // ---- gated linear recurrence
@@ -1128,6 +1131,8 @@ int attn_pass(const RmiAttnShape &s, const RmiAttnArgs &a, hipStream_t st) {
     else
         hipLaunchKernelGGL(conv_rotate_kernel<T>, conv_grid, dim3(256), 0, st, s, a);
     const uint32_t bucket = bucket_of(s);
+    const bool filled = s.dk_pad == bucket && s.dv_pad == bucket;
+    const uint64_t cus = uint64_t(rmi_device_cus());
     if (n_cols <= kSplitMaxCols) {
         const SplitPlan plan = attn_parts(s, a.n_tokens, a.pos0);
         const dim3 grid(s.kv_heads * plan.tiles.by * plan.parts.by);
@@ -1137,7 +1142,12 @@ int attn_pass(const RmiAttnShape &s, const RmiAttnArgs &a, hipStream_t st) {
             if (rc == RMI_HIP_OK) hipLaunchKernelGGL(kernel, grid, dim3(256), lds, st, s, a, plan);
             return rc;
         };
-        const int rc = bucket == 64 ? go(attn_split_kernel<T, 64>) : bucket == 128 ? go(attn_split_kernel<T, 128>) : go(attn_split_kernel<T, 256>);
+        auto with = [&](auto every) {
+            return bucket == 64    ? go(attn_split_kernel<T, 64, every.value>)
+                   : bucket == 128 ? go(attn_split_kernel<T, 128, every.value>)
+                                   : go(attn_split_kernel<T, 256, every.value>);
+        };
+        const int rc = grid.x > cus && !filled ? with(std::false_type()) : with(std::true_type());  // (as below)
         if (rc != RMI_HIP_OK) return rc;
     } else {
         const uint32_t qt = bucket == 256 ? 1 : 2, blocks = (n_cols + 16 * qt - 1) / (16 * qt) * s.kv_heads;
@@ -1157,8 +1167,6 @@ int attn_pass(const RmiAttnShape &s, const RmiAttnArgs &a, hipStream_t st) {
         // in a narrower head, those past its end (2048 tokens of bf16: 128 elements 60.7 and 62.6, 160 of 256 111 and 148;
         // f32 160 of 256 331 and 457, 300 tokens 29.0 and 30.2).  Heads that fill the bucket gain by it however many there
         // are where a block's loads are most: 256 elements, bf16 234 and 211, f32 513 and 506; 128 of f32 215 and 207.
-        const bool filled = s.dk_pad == bucket && s.dv_pad == bucket;
-        const uint64_t cus = uint64_t(rmi_device_cus());
         const bool branches = sizeof(T) == 2 ? !(filled && bucket == 256) && 2 * uint64_t(blocks) > (bucket == 64 ? 6 : 5) * cus : !filled && blocks > cus;
         const int rc = branches ? with(std::false_type()) : with(std::true_type());
         if (rc != RMI_HIP_OK) return rc;
