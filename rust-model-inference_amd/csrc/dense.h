@@ -120,6 +120,9 @@ int rmi_dense_embed(uint32_t elem_bytes, const RmiEmbed &e, const uint32_t *tok,
 int rmi_dense_gemm(uint32_t elem_bytes, const RmiDense &w, const void *a, const RmiRowSegs &segs, uint32_t n_tokens, hipStream_t st);
 int rmi_dense_gemm_residual(uint32_t elem_bytes, const RmiDense &w, const void *a, const RmiColSegs &segs, float *x, uint32_t width,
                             uint32_t n_tokens, hipStream_t st);
+// the tile that such a product takes, weight rows << 16 | tokens << 4 | waves (n_rows: of the weight, or a residual one's width;
+// epilogue: -1 residual, else RmiEpilogue's)
+uint32_t rmi_dense_tile(uint32_t elem_bytes, int epilogue, uint32_t n_rows, uint32_t k_pad, uint32_t n_tokens);
 // one token: the input in front of the product is part of the launch, for as many columns as a workgroup holds; the
 // second form computes two products with inputs of their own side by side
 bool rmi_dense_gemv_fits(uint32_t elem_bytes, uint32_t k_pad);

@@ -133,15 +133,15 @@ __device__ __forceinline__ void store_rows(const f32x4 (&acc)[NN][NT], const Rmi
     }
 }
 
-// Small tiles, for products that would leave compute units idle otherwise: four waves, two LDS buffers; the pieces of the
-// next PD steps are on their way to registers while one is multiplied.
+// Four waves; the pieces of the next PD steps are on their way to registers while one is multiplied.  Small tiles, for
+// products that would leave compute units idle otherwise, have two LDS buffers; 128 x 128 keeps one (NB = 1), so that three
+// workgroups share a compute unit: one round where wider tiles would start a second one for a few workgroups.
 template <typename T, int BN, int BT, int WN, int WT, int PD, int NB, int WPS, int EPI>
 __global__ __launch_bounds__(256, WPS) void dense_gemm_kernel(const T *__restrict__ w, const T *__restrict__ a, uint32_t n_rows,
                                                               uint32_t k_pad, uint32_t ld, uint32_t n_tokens, uint32_t grid_n, uint32_t grid_t, uint32_t xcd_split,
                                                          RmiRowSegs rs, RmiColSegs cs, float *__restrict__ x, uint32_t width) {
     constexpr bool RESIDUAL = EPI == kResidual;
     static_assert((BN / WN) * (BT / WT) == 4, "four waves");
-    static_assert(NB == 2, "two buffers");
     static_assert(kDenseKAlign * sizeof(T) % (kStepBytes * PD) == 0, "whole rounds of the register slots");
     constexpr int NN = WN / 16, NT = WT / 16;
     constexpr int PW = BN * 8 / 256, PA = (BT * 8 + 255) / 256;  // pieces a thread loads per step
@@ -228,6 +228,7 @@ __global__ __launch_bounds__(256, WPS) void dense_gemm_kernel(const T *__restric
 #pragma unroll
                         for (int i2 = 0; i2 < NT; i2++) acc[i][i2] = mma16<T>(fw[i], fa[i2], acc[i][i2]);
                 }
+                if (NB == 1) __syncthreads();
                 park((j + 1) % PD, buf ^ (NB - 1));  // (behind the last step: that step again, read by nobody)
                 load((j + 1) % PD, step + j + 1 + PD);
                 __syncthreads();
@@ -373,76 +374,97 @@ __global__ __launch_bounds__(64 * (BN / WN) * (BT / WT), WPS) void dense_gemm_wi
     if constexpr (!RESIDUAL) store_rows<T, EPI, NN, NT>(acc, rs, n_rows, n_tokens, row0 + wn, tok0 + wt + fr, g);
 }
 
-// Which tile a product takes: the least of estimates, in microseconds, that were fitted to 13 shapes (1024..39040 rows of
-// 1024..20480 columns) with 128..2048 tokens.  A tile costs what a step of k takes a compute unit that holds so many of
-// them (w = tiles over compute units).  bf16 is bound by LDS reads and the traffic between L2 and the compute units, so wider
-// tiles are cheaper an element as long as there are enough of them; f32 is bound by the matrix cores and every tile costs its
-// area, so that only the unevenness of the last round counts.  E.g. in bf16, us by 64 x 64 | 64 x 128 | 128 x 128 | 128 x 256 |
-// 256 x 256: 39040 x 4096, 2048 tokens (four-wave 128 x 128 tiles before: 812) - | 1095 | 813 | 741 | 640; 4096 x 20480, 2048
-// tokens (440 before) - | 479 | 360 | 340 | 521; 2048 x 6144, 1024 tokens 53 | 42 | 65 | 74 | 133; 12288 x 2048, 512 tokens
-// 53 | 39 | 33 | 36 | 55; 1024 x 6144, 512 tokens 21 | 37 | 64 | 74 | 133.
-enum DenseTile { kTile64x16, kTile64x32, kTile64x64, kTile64x128, kTile128x128, kTile128x256, kTile256x256 };
-DenseTile dense_tile_of(bool bf16, uint32_t n_rows, uint32_t n_tokens, uint32_t n_steps) {
-    if (n_tokens <= 16) return kTile64x16;
-    const double cus = rmi_device_cus() > 0 ? rmi_device_cus() : 1;
-    DenseTile best = kTile64x32;
-    double least = 1e30;
-    // us of a step: alone a compute unit, slope beyond; per round of `fit` tiles a compute unit
-    auto consider = [&](DenseTile t, uint32_t bn, uint32_t bt, double fixed, double base, double slope, double fit) {
-        const double w = double((n_rows + bn - 1) / bn) * ((n_tokens + bt - 1) / bt) / cus;
-        const double rounds = double(uint64_t(w / fit)), rest = w - rounds * fit;
-        double step;
-        if (!bf16)
-            step = base * double(uint64_t(w + 0.999));
-        else
-            step = rounds * (base + slope * (fit - 1)) + (rest > 0 ? base + slope * (rest > 1 ? rest - 1 : 0.0) : 0.0);
-        const double us = fixed + n_steps * step;
-        if (us < least) least = us, best = t;
+// Which tile a product takes: the least of estimates, in microseconds, that were fitted to every tile's time on 51 weights
+// (320..39968 rows of 256..20480 columns, plain, activated, paired and residual ones) with 17..2048 tokens, each launch with a
+// weight from HBM as in a model.  w: tiles a compute unit; `fit` of them run side by side and make a round.  A step of k
+// takes `round` in a whole round; the tiles left over take `first`, and `more` and `whole` for what is beyond one a compute
+// unit, by its share and by the whole tile.  An epilogue is not overlapped where a compute unit holds one workgroup, and adds
+// to or activates a whole tile: so much a tile, which decides between wide tiles at 1024 columns.
+// bf16 is bound by LDS reads and the traffic between L2 and the compute units, so wider tiles are cheaper an element as long
+// as there are enough of them; f32 is bound by the matrix cores and every tile costs its area.  Over 597 products of bf16 and
+// as many of f32 the choice costs 0.7 % and 0.03 % over the best tile of each (four waves alone: 6 and 5 %).  E.g. in bf16, us by 64 x 64 |
+// 64 x 128 | 128 x 128 with four waves | with eight | 128 x 256 | 256 x 256:
+//   activated 12304 x 1024, 2048 tokens    138 |  129 | 103 | 104 | 121 | 120     768 tokens    54 |  53 |  47 |  50 |  67 |  61
+//   activated 39968 x 4096, 2048 tokens   1504 | 1169 | 797 | 846 | 760 | 687     512 tokens   320 | 280 | 210 | 231 | 233 | 264
+//   residual 4096 x 12288, 2048 tokens     375 |  303 | 246 | 239 | 193 | 341     512 tokens   102 | 104 | 150 | 170 | 195 | 357
+enum DenseTile { kTile64x16, kTile64x32, kTile64x64, kTile64x128, kTile128x128w4, kTile128x128, kTile128x256, kTile256x256 };
+struct TileCost {
+    DenseTile tile;
+    uint32_t rows, tokens, waves, fit;
+    float fixed, round, first, more, whole, out, activated, residual;
+};
+constexpr TileCost kTile16 = {kTile64x16, 64, 16, 4, 4, 0, 0, 0, 0, 0, 0, 0, 0};
+constexpr TileCost kCostsBf16[] = {
+    {kTile64x32, 64, 32, 4, 4, 4.04f, 0.728f, 0.174f, 0.078f, 0.113f, 0.347f, 0, 0},
+    {kTile64x64, 64, 64, 4, 4, 3.86f, 0.845f, 0.302f, 0.0412f, 0.154f, 1.08f, 1.81f, 0.973f},
+    {kTile64x128, 64, 128, 8, 2, 3.78f, 0.809f, 0.525f, 0.123f, 0.184f, 0.789f, 1.14f, 0},
+    {kTile128x128w4, 128, 128, 4, 3, 4.09f, 1.6f, 0.884f, 0, 0.308f, 2.44f, 4.23f, 0},
+    {kTile128x128, 128, 128, 8, 2, 7.06f, 1.1f, 0.844f, 0.268f, 0, 0, 6.78f, 0},
+    {kTile128x256, 128, 256, 8, 1, 7.53f, 0.947f, 0.882f, 0, 0, 4.05f, 12.6f, 0},
+    {kTile256x256, 256, 256, 8, 1, 23.8f, 1.83f, 1.27f, 0, 0, 0, 24.5f, 0}};
+constexpr TileCost kCostsF32[] = {
+    {kTile64x32, 64, 32, 4, 4, 4.23f, 1.12f, 0.322f, 0.0836f, 0.187f, 0.438f, 0.803f, 0.103f},
+    {kTile64x64, 64, 64, 4, 4, 4.36f, 1.96f, 0.588f, 0.0653f, 0.408f, 0.986f, 1.14f, 2.62f},
+    {kTile64x128, 64, 128, 8, 2, 3.56f, 1.78f, 0.959f, 0, 0.845f, 2.04f, 2.0f, 6.56f},
+    {kTile128x128, 128, 128, 8, 2, 6.12f, 3.54f, 1.81f, 0.04f, 1.67f, 2.36f, 5.63f, 16.2f}};
+
+const TileCost &dense_tile_of(bool bf16, int epilogue, uint32_t n_rows, uint32_t n_tokens, uint32_t n_steps) {
+    if (n_tokens <= kTile16.tokens) return kTile16;
+    const uint32_t cus = rmi_device_cus() > 0 ? uint32_t(rmi_device_cus()) : 1;
+    const TileCost *best = nullptr;
+    double least = 0;
+    auto consider = [&](const TileCost &c) {
+        if (epilogue == kResidual && c.tile == kTile256x256) return;  // (2 % the better at the widest at most, and registers spill)
+        const uint64_t tiles = uint64_t((n_rows + c.rows - 1) / c.rows) * ((n_tokens + c.tokens - 1) / c.tokens);
+        const uint64_t rounds = tiles / (c.fit * cus), left = tiles % (c.fit * cus);
+        double step = double(rounds) * c.round;
+        if (left) step += c.first + c.whole * double((left - 1) / cus) + (left > cus ? c.more * (double(left) / cus - 1.0) : 0.0);
+        const double end = c.out + (epilogue == kResidual ? c.residual : epilogue == kRowsActed || epilogue == kRowsTimesTable ? c.activated : 0.0f);
+        const double us = c.fixed + n_steps * step + double(tiles) / cus * end;
+        if (!best || us < least) least = us, best = &c;
     };
-    if (bf16) {
-        consider(kTile64x32, 64, 32, 3, 0.17, 0.17, 4);
-        consider(kTile64x64, 64, 64, 4, 0.28, 0.25, 4);
-        consider(kTile64x128, 64, 128, 4, 0.39, 0.27, 2);
-        consider(kTile128x128, 128, 128, 5, 0.68, 0.54, 2);
-        consider(kTile128x256, 128, 256, 7, 1.08, 0, 1);
-        consider(kTile256x256, 256, 256, 8, 1.95, 0, 1);
-    } else {
-        consider(kTile64x32, 64, 32, 3, 0.31, 0, 1);
-        consider(kTile64x64, 64, 64, 4, 0.56, 0, 1);
-        consider(kTile64x128, 64, 128, 4, 0.95, 0, 1);
-        consider(kTile128x128, 128, 128, 5, 1.84, 0, 1);
-    }
-    return best;
+    if (bf16)
+        for (const TileCost &c : kCostsBf16) consider(c);
+    else
+        for (const TileCost &c : kCostsF32) consider(c);
+    return *best;
 }
 
 template <typename T, int EPI>
 int launch_gemm(const RmiDense &w, const void *a, const RmiRowSegs &rs, const RmiColSegs &cs, float *x, uint32_t width,
                 uint32_t n_tokens, hipStream_t st) {
     const uint32_t n_rows = EPI == kResidual ? width : w.n_rows;
-    auto go = [&](auto kernel, uint32_t bn, uint32_t bt, uint32_t threads = 256) {
-        const uint32_t gn = (n_rows + bn - 1) / bn, gt = (n_tokens + bt - 1) / bt;
+    const TileCost &tile = dense_tile_of(sizeof(T) == 2, EPI, n_rows, n_tokens, uint32_t(w.k_pad * sizeof(T) / kStepBytes));
+    auto go = [&](auto kernel) {
+        const uint32_t gn = (n_rows + tile.rows - 1) / tile.rows, gt = (n_tokens + tile.tokens - 1) / tile.tokens;
         const uint32_t split = rmi_gemm_xcd_split(gn, gt, double(n_rows) * w.k_pad, double(n_tokens) * w.k_pad);
-        hipLaunchKernelGGL(kernel, dim3(gn * gt), dim3(threads), 0, st, static_cast<const T *>(w.data), static_cast<const T *>(a), n_rows,
+        hipLaunchKernelGGL(kernel, dim3(gn * gt), dim3(64 * tile.waves), 0, st, static_cast<const T *>(w.data), static_cast<const T *>(a), n_rows,
                            w.k_pad, w.ld, n_tokens, gn, gt, split, rs, cs, x, width);
     };
-    switch (dense_tile_of(sizeof(T) == 2, n_rows, n_tokens, uint32_t(w.k_pad * sizeof(T) / kStepBytes))) {
-    case kTile64x16: go(dense_gemm_kernel<T, 64, 16, 16, 16, 4, 2, 4, EPI>, 64, 16); break;
-    case kTile64x32: go(dense_gemm_kernel<T, 64, 32, 32, 16, 4, 2, 4, EPI>, 64, 32); break;
-    case kTile64x64: go(dense_gemm_kernel<T, 64, 64, 32, 32, 4, 2, 4, EPI>, 64, 64); break;
-    case kTile64x128: go(dense_gemm_wide_kernel<T, 64, 128, 32, 32, 3, 2, EPI>, 64, 128, 512); break;
-    case kTile128x128: go(dense_gemm_wide_kernel<T, 128, 128, 64, 32, 2, 4, EPI>, 128, 128, 512); break;
-    case kTile128x256:
-        if constexpr (sizeof(T) == 2) go(dense_gemm_wide_kernel<T, 128, 256, 64, 64, 3, 2, EPI>, 128, 256, 512);
-        break;
-    case kTile256x256:
-        if constexpr (sizeof(T) == 2) go(dense_gemm_wide_kernel<T, 256, 256, 128, 64, 2, 2, EPI>, 256, 256, 512);
-        break;
+    switch (tile.tile) {
+    case kTile64x16: go(dense_gemm_kernel<T, 64, 16, 16, 16, 4, 2, 4, EPI>); break;
+    case kTile64x32: go(dense_gemm_kernel<T, 64, 32, 32, 16, 4, 2, 4, EPI>); break;
+    case kTile64x64: go(dense_gemm_kernel<T, 64, 64, 32, 32, 4, 2, 4, EPI>); break;
+    case kTile64x128: go(dense_gemm_wide_kernel<T, 64, 128, 32, 32, 3, 2, EPI>); break;
+    case kTile128x128: go(dense_gemm_wide_kernel<T, 128, 128, 64, 32, 2, 4, EPI>); break;
+    default:
+        if constexpr (sizeof(T) == 2) {
+            if (tile.tile == kTile128x128w4) go(dense_gemm_kernel<T, 128, 128, 64, 64, 1, 1, 3, EPI>);
+            if (tile.tile == kTile128x256) go(dense_gemm_wide_kernel<T, 128, 256, 64, 64, 3, 2, EPI>);
+            if constexpr (EPI != kResidual)
+                if (tile.tile == kTile256x256) go(dense_gemm_wide_kernel<T, 256, 256, 128, 64, 2, 2, EPI>);
+        }
     }
     RMI_HIP_CHECK(hipGetLastError());
     return RMI_HIP_OK;
 }
 
 }  // namespace
+
+uint32_t rmi_dense_tile(uint32_t elem_bytes, int epilogue, uint32_t n_rows, uint32_t k_pad, uint32_t n_tokens) {
+    const TileCost &t = dense_tile_of(elem_bytes == 2, epilogue, n_rows, n_tokens, k_pad * elem_bytes / kStepBytes);
+    return t.rows << 16 | t.tokens << 4 | t.waves;
+}
 
 int rmi_dense_input(uint32_t elem_bytes, const RmiInput &in, const uint32_t *rows, void *h, uint32_t n_tokens, uint32_t k_pad,
                     hipStream_t st) {

@@ -1,5 +1,6 @@
-"""Dense products of several tokens, one size for every tile that the launcher picks, ragged rows and tokens among them,
-through the library's own launch functions (they are C++ symbols; the structures are those of csrc/dense.h).
+"""Dense products of several tokens, ragged rows and tokens among them, through the library's own launch functions (they
+are C++ symbols; the structures are those of csrc/dense.h).  test_every_tile takes each tile with each epilogue and asserts
+that the launcher picks it; the other sizes are what the launcher makes of them.
 
 Reference: the f32 product of the same operands.  Bound: both sides add k f32 products, each sum within
 k 2^-24 sum|a b| of the exact one."""
@@ -126,3 +127,134 @@ def test_relu_pairs(hip, elem, rows, k, tokens):
     err = 2 * k * 2.0**-24 * size
     bound = err[:, 0::2] * np.abs(up) + err[:, 1::2] * gate + err[:, 0::2] * err[:, 1::2] + 2.0**(-8 if elem == 2 else -22) * np.abs(gate * up)
     assert (np.abs(got - gate * up) <= bound).all()
+
+
+# A size for every tile that a product takes, rows and tokens past whole tiles, by the launcher's choice on 256 compute units:
+# (element size, rows, tokens, waves of the tile), then rows, columns and tokens of a plain, an activated and a residual product.
+TILES = [
+    ((2, 64, 16, 4), (80, 512, 5), (80, 512, 5), (80, 512, 5)),
+    ((2, 64, 32, 4), (80, 512, 45), (80, 512, 45), (80, 512, 45)),
+    ((2, 64, 64, 4), (12048, 512, 45), (25168, 2048, 45), (25168, 1024, 45)),
+    ((2, 64, 128, 8), (4832, 512, 205), (12704, 512, 109), (4832, 512, 205)),
+    ((2, 128, 128, 4), (22544, 512, 299), (17952, 1024, 299), (22544, 512, 299)),
+    ((2, 128, 128, 8), (17296, 512, 205), (17296, 1024, 205), (17296, 512, 205)),
+    ((2, 128, 256, 8), (6800, 2048, 909), (8768, 2048, 701), (6800, 2048, 909)),
+    ((2, 256, 256, 8), (12704, 2048, 909), (12704, 2048, 909), None),
+    ((4, 64, 16, 4), (80, 512, 5), (80, 512, 5), (80, 512, 5)),
+    ((4, 64, 32, 4), (80, 512, 45), (80, 512, 45), (80, 512, 45)),
+    ((4, 64, 64, 4), (26576, 512, 45), (15776, 512, 45), (20576, 2048, 109)),
+    ((4, 64, 128, 8), (12576, 512, 109), (12576, 512, 109), (12576, 2048, 109)),
+    ((4, 128, 128, 8), (28576, 512, 205), (28976, 4096, 205), (7888, 4096, 909))]
+CASES = [(tile, kind, size) for tile, plain, acted, res in TILES
+         for kind, size in (("plain", plain), ("acted", acted), ("table", acted), ("residual", res)) if size]
+EPILOGUES = {"plain": 0, "acted": 1, "table": 3, "residual": -1}  # csrc/dense_launch.h
+K_SIGMOID, K_SILU, K_GELU, K_FORGET = 1, 2, 3, 4
+
+
+def _sigmoid(z):
+    with np.errstate(over="ignore"):
+        return 1.0 / (1.0 + np.exp(-z))
+
+
+def _act(act, z, bias, lower):
+    """in 64 bits, and the largest slope"""
+    if act == K_SIGMOID:
+        return _sigmoid(z + bias), 0.25
+    if act == K_SILU:
+        return z * _sigmoid(z), 1.1
+    if act == K_GELU:
+        return z * _sigmoid(1.59576912160573071176 * (z + 0.044715 * z**3)), 1.13
+    if act == K_FORGET:
+        return lower + (1.0 - lower) * _sigmoid(z + bias), 0.25
+    return z, 1.0
+
+
+def _chosen(hip, elem, kind, rows, k, tokens):
+    fn = hip.hip.lib._Z14rmi_dense_tilejijjj
+    fn.restype = C.c_uint32
+    t = fn(C.c_uint32(elem), C.c_int(EPILOGUES[kind]), C.c_uint32(rows), C.c_uint32(k), C.c_uint32(tokens))
+    return t >> 16, t >> 4 & 0xfff, t & 15
+
+
+# us of bf16 products, each launch with a weight from HBM, by the tiles of 64 x 64, 64 x 128, 128 x 128 with four and with eight
+# waves, 128 x 256 and 256 x 256
+MEASURED_TILES = [(64, 64, 4), (64, 128, 8), (128, 128, 4), (128, 128, 8), (128, 256, 8), (256, 256, 8)]
+MEASURED = [("acted", 12304, 1024, 2048, (138, 129, 103.5, 104.5, 121, 120)), ("acted", 12304, 1024, 768, (54.4, 53.0, 47.3, 49.9, 67.4, 61.3)),
+            ("acted", 39968, 4096, 2048, (1504, 1169, 797, 846, 760, 687)), ("acted", 39968, 4096, 512, (320, 280, 210, 231, 233, 264)),
+            ("residual", 4096, 12288, 2048, (375, 303, 246, 239, 193, 341)), ("residual", 4096, 12288, 512, (102.1, 104.4, 150, 170, 195, 357))]
+
+
+@pytest.mark.parametrize("kind,rows,k,tokens,us", MEASURED)
+def test_the_choice_follows_the_measurements(hip, kind, rows, k, tokens, us):
+    """The fitted estimates pick a tile within 3 % of the fastest."""
+    if hip.hip.device_info()[1] != 256:
+        pytest.skip("measured on 256 compute units")
+    assert us[MEASURED_TILES.index(_chosen(hip, 2, kind, rows, k, tokens))] <= 1.03 * min(us)
+
+
+@pytest.mark.parametrize("tile,kind,size", CASES, ids=["%d-%dx%dx%d-%s" % (*t, k) for t, k, _ in CASES])
+def test_every_tile(hip, tile, kind, size):
+    """Bounds: the product's as above, times the activation's largest slope; an exponential's argument is off by a few 2^-24 of
+    itself, and arguments beyond 100 only make zeros and ones: 2^-14 of the value; the rounding of the output."""
+    H = hip.hip
+    elem, (rows, k, tokens) = tile[0], size
+    if H.device_info()[1] == 256:
+        assert _chosen(hip, elem, kind, rows, k, tokens) == tile[1:]
+    rng = np.random.default_rng(rows + k)
+    w, wv, ld = _operand(rng, rows, k, elem)
+    x, xv, _ = _operand(rng, tokens, k, elem)
+    if kind != "residual":  # results of a size at which the activations bend
+        xv = xv / 8  # (exact)
+        padded = np.zeros((tokens, ld), np.float32)
+        padded[:, :k] = xv
+        x = padded if elem == 4 else (padded.view(np.uint32) >> 16).astype(np.uint16)
+    bufs = [H.DeviceBuffer.from_array(v) for v in (w, x)]
+    z, size = (xv @ wv.T).astype(np.float64), np.abs(xv) @ np.abs(wv).T
+    err = 2 * k * 2.0**-24 * size
+    d_w = Dense(bufs[0].ptr, rows, k, ld)
+
+    if kind == "residual":
+        half = k // 2 // 256 * 256
+        acc = rng.standard_normal((tokens, rows), dtype=np.float32)
+        gate = rng.uniform(0, 1, (tokens, rows)).astype(np.float32)
+        bufs += [H.DeviceBuffer.from_array(v) for v in (acc, gate)]
+        segs = ColSegs()
+        segs.s[0], segs.s[1], segs.n_segs = ColSeg(bufs[3].ptr, rows, 0.5, half), ColSeg(None, 0, 2.0, k), 2
+        assert getattr(H.lib, RESIDUAL)(C.c_uint32(elem), C.byref(d_w), C.c_void_p(bufs[1].ptr), C.byref(segs), C.c_void_p(bufs[2].ptr),
+                                        C.c_uint32(rows), C.c_uint32(tokens), None) == 0
+        H.check(H.lib.rmi_hip_synchronize())
+        got = bufs[2].to_array(np.float32, (tokens, rows))
+        want = acc + 0.5 * gate * (xv[:, :half] @ wv[:, :half].T) + 2.0 * (xv[:, half:] @ wv[:, half:].T)
+        assert (np.abs(got - want) <= 2 * err + 2.0**-22 * (np.abs(acc) + np.abs(want))).all()
+        return
+
+    cuts = [0, *(rows * i // 4 // 16 * 16 for i in (1, 2, 3)), rows]
+    acts = {"plain": (0, 0, 0, 0), "acted": (K_SIGMOID, K_GELU, K_FORGET, 0), "table": (K_GELU, 0, K_SILU, K_GELU)}[kind]
+    bias, lower = rng.standard_normal(rows, dtype=np.float32), rng.uniform(0, 1, rows).astype(np.float32)
+    ids = rng.integers(0, 9, tokens, dtype=np.uint32)  # past the table's end: its last row
+    table, table_v, _ = _operand(rng, 7, rows, elem)
+    bufs += [H.DeviceBuffer.from_array(v) for v in (bias, lower, ids, table)]
+    segs, outs = RowSegs(), []
+    for i in range(4):
+        a, n = cuts[i], cuts[i + 1] - cuts[i]
+        out_elem = int(i == 1 and kind != "plain")
+        outs.append(H.DeviceBuffer(n * tokens * (elem if out_elem else 4)))
+        mul = kind == "table" and i != 1
+        segs.s[i] = RowSeg(outs[i].ptr, bufs[2].ptr + 4 * a, bufs[3].ptr + 4 * a, bufs[5].ptr + elem * a if mul else None, bufs[4].ptr if mul else None,
+                           table.shape[1], 7, a, n, n, acts[i], out_elem)
+        segs.start[i] = a
+    segs.start[4:] = [rows] * 8
+    segs.n_segs, segs.n_rows = 4, rows
+    assert getattr(H.lib, ROWS)(C.c_uint32(elem), C.byref(d_w), C.c_void_p(bufs[1].ptr), C.byref(segs), C.c_uint32(tokens), None) == 0
+    H.check(H.lib.rmi_hip_synchronize())
+    for i in range(4):
+        at = slice(cuts[i], cuts[i + 1])
+        n, short = cuts[i + 1] - cuts[i], segs.s[i].out_elem and elem == 2
+        got = (outs[i].to_array(np.uint16, (tokens, n)).astype(np.uint32) << 16).view(np.float32) if short else outs[i].to_array(np.float32, (tokens, n))
+        want, slope = _act(acts[i], z[:, at], bias[at].astype(np.float64), lower[at].astype(np.float64))
+        bound = slope * err[:, at]
+        if segs.s[i].mul:
+            rows_of = table_v[np.minimum(ids, 6)][:, at]
+            want, bound = want * rows_of, bound * np.abs(rows_of)
+        bound = bound + (2.0**-14 if acts[i] else 2.0**-22) * np.abs(want) + (2.0**-8 * np.abs(want) if short else 0) + 2.0**-20
+        assert (np.abs(got - want) <= bound).all(), (i, np.abs(got - want).max())
