@@ -775,7 +775,7 @@ __device__ __forceinline__ void recur_step(const RmiRecurShape &s, const RmiRecu
     const size_t at = size_t(head) * s.d_pad * s.v_pad + c * 4;
     const float *st = a.state_in + at;
     float *st_out = a.state_out + at;
-    // eight state rows of a thread in flight, the first ones beside this token's gates and values (unconditional: a row
+    // sixteen state rows of a thread in flight, the first ones beside this token's gates and values (unconditional: a row
     // past the end is the last one again; the first token of a sequence reads what it then drops)
     constexpr uint32_t kRows = 16;
     f32x4 r[kRows];
@@ -1147,7 +1147,11 @@ int attn_pass(const RmiAttnShape &s, const RmiAttnArgs &a, hipStream_t st) {
                    : bucket == 128 ? go(attn_split_kernel<T, 128, every.value>)
                                    : go(attn_split_kernel<T, 256, every.value>);
         };
-        const int rc = grid.x > cus && !filled ? with(std::false_type()) : with(std::true_type());  // (as below)
+        // As below, and with 256 elements of bf16 a block's keys and values fit beside the rest only where every load is made,
+        // which pays from two blocks a wave on (200 tokens, 160 of 256, every load | branches: 32 heads, 3000 keys in front
+        // 150 | 192 us; 16 heads, none in front 81 | 67).
+        const bool branches = grid.x > cus && (sizeof(T) == 2 && bucket == 256 ? plan.keys_per_part <= 4 * kKeyBlock : !filled);
+        const int rc = branches ? with(std::false_type()) : with(std::true_type());
         if (rc != RMI_HIP_OK) return rc;
     } else {
         const uint32_t qt = bucket == 256 ? 1 : 2, blocks = (n_cols + 16 * qt - 1) / (16 * qt) * s.kv_heads;
@@ -1158,16 +1162,22 @@ int attn_pass(const RmiAttnShape &s, const RmiAttnArgs &a, hipStream_t st) {
             return rc;
         };
         auto with = [&](auto every) {
-            return bucket == 64    ? go(attn_pass_kernel<T, 64, 2, every.value>)
+            return bucket == 64    ? go(attn_pass_kernel<T, 64, 2, every.value || sizeof(T) == 2>)
                    : bucket == 128 ? go(attn_pass_kernel<T, 128, 2, every.value>)
                                    : go(attn_pass_kernel<T, 256, 1, every.value>);
         };
-        // With few workgroups a compute unit the waits for loads behind branches count (256 elements a head of bf16, 300
-        // tokens: 25.8 us, 15.3 with every load); with many the other waves cover them, and every load costs its issue and,
-        // in a narrower head, those past its end (2048 tokens of bf16: 128 elements 60.7 and 62.6, 160 of 256 111 and 148;
-        // f32 160 of 256 331 and 457, 300 tokens 29.0 and 30.2).  Heads that fill the bucket gain by it however many there
-        // are where a block's loads are most: 256 elements, bf16 234 and 211, f32 513 and 506; 128 of f32 215 and 207.
-        const bool branches = sizeof(T) == 2 ? !(filled && bucket == 256) && 2 * uint64_t(blocks) > (bucket == 64 ? 6 : 5) * cus : !filled && blocks > cus;
+        // Every load: the waits for loads behind branches count wherever workgroups do not cover them.  Branches: a head that
+        // leaves more than an eighth of the bucket's pieces loads those past its end for nothing, which tells once every compute
+        // unit has its workgroups.  Five numbers of heads, 140 to 2048 tokens, us with the convolution in front, every load |
+        // branches:
+        //   bf16  128 elements, 32 heads over 8, 2048 tokens 129 | 141, 1024 tokens 52 | 52, 16 heads 1500 tokens 56 | 52: with
+        //         three or four workgroups a compute unit, in the second round of two, branches are up to 6 % the better;
+        //         16 heads over 8, 2048 tokens: 160 of 256 281 | 247, 256 elements 375 | 399; up to 64 elements branches never gain
+        //   f32   16 heads over 8, 2048 tokens: 160 of 256 598 | 469, 128 elements 227 | 235; 32 over 8: 48 of 64 198 | 216
+        const bool narrow = 4 * (s.dk_pad + s.dv_pad) < 7 * bucket;
+        const bool branches = sizeof(T) == 4 ? narrow && blocks > cus
+                              : narrow       ? bucket > 64 && blocks > 2 * cus
+                                             : bucket == 128 && blocks > 2 * cus && blocks <= 4 * cus;
         const int rc = branches ? with(std::false_type()) : with(std::true_type());
         if (rc != RMI_HIP_OK) return rc;
     }
