@@ -47,7 +47,8 @@ def test_attention(hip, elem, heads, kv_heads, dim, pos0, tokens):
     size.restype = C.c_size_t
     d_u, ones = H.DeviceBuffer.from_array(u), H.DeviceBuffer.from_array(np.ones(channels, np.float32))
     hist, q = H.DeviceBuffer(channels * 4), H.DeviceBuffer(heads * total * s.dk_pad * elem)
-    keys, values = H.DeviceBuffer(kv_heads * s.capacity * s.dk_pad * elem), H.DeviceBuffer(kv_heads * s.capacity * s.dv_pad * elem)
+    # (caches start as zeros: a row that is not filled yet has weight zero, whatever finite value it holds)
+    keys, values = (H.DeviceBuffer.from_array(np.zeros(kv_heads * s.capacity * pad * elem, np.uint8)) for pad in (s.dk_pad, s.dv_pad))
     out = H.DeviceBuffer(total * heads * dim * elem)
     scratch = H.DeviceBuffer.from_array(np.zeros(size(C.byref(s)) // 4 + 1, np.uint32))
     for first, n in ((0, pos0), (pos0, tokens)):
