@@ -5,18 +5,22 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
-// A token's mixers are a few workgroups that wait for memory; meanwhile HBM and nine in ten of the compute units idle,
-// and the product behind them is bound by HBM.  So such a launch gets kAheadBlocks more workgroups, which read what comes
-// next and drop it.  28 layers of width 1024 in bf16, 12.6 MB of output weights and 25 MB of the next layer's input
-// weights a layer, a token: 689 us without; 641 with the output weights and 96 workgroups, 650 with 16 MB and 128, 659 with
-// 24 MB and 128 (the fetch outlasts the mixers), 630 with 24 MB and 192, a workgroup on most compute units.  Qwen3's attention
-// launch, with 64 workgroups that all read keys, lost by it (11 -> 21 us) and has none.
+// A token's mixers are a few workgroups that wait for memory; meanwhile HBM and most of the compute units idle, and the product
+// behind them is bound by HBM.  So such a launch gets a workgroup more for every compute unit that the mixers leave, which read
+// what comes next and drop it.  28 layers of width 1024 in bf16, 12.6 MB of output weights and 25 MB of the next layer's input
+// weights a layer, us a token behind 16 | 512 | 2048 | 4096 keys (where the mixers are 16 to 144 workgroups):
+//   nothing fetched                        578 | 643 | 749 | 804
+//   16 MB, 128 workgroups at any context   530 | 597 | 711 | 774
+//   24 MB, 192 workgroups                  519 | 580 | 707 | 781
+//   24 MB, a workgroup a unit left         522 | 583 | 693 | 761
+//   32 MB, a workgroup a unit left         545 | 574 | 710 | 765     (all of the L2s: what the mixers read goes, too)
+// In f32 and at widths of 2048 and 4096 the kept setting is within 3 % of the best of the five, and no token is slower for it.
+// Qwen3's attention launch, with 64 workgroups that all read keys, lost by it (11 -> 21 us) and has none.
 // Workgroup b of the launch that reads a region reads its bytes [b chunk, (b + 1) chunk).  Workgroups go round the eight
 // XCDs in turn, each with an L2 of its own: what workgroup b will read is read on the XCD b % 8.  Only a hint: if the
 // workgroups go elsewhere, the bytes are still nearer than HBM.
 constexpr uint32_t kAheadRegions = 2;
-constexpr uint32_t kAheadBlocks = 128;          // a multiple of the XCDs
-constexpr uint64_t kAheadBytes = 16u << 20;     // half of all L2s
+constexpr uint64_t kAheadBytes = 24u << 20;  // three quarters of all L2s
 struct RmiAhead {
     struct Region {
         const void *p;
@@ -33,7 +37,8 @@ struct RmiAhead {
         n_regions++;
     }
 };
-inline uint32_t rmi_ahead_blocks(const RmiAhead &a) { return a.bytes ? kAheadBlocks : 0; }
+// workgroups for it beside `used` others: a multiple of the XCDs
+inline uint32_t rmi_ahead_blocks(const RmiAhead &a, uint32_t used, uint32_t cus) { return a.bytes && used < cus ? (cus - used) / 8 * 8 : 0; }
 
 // One of the launch's last workgroups, those from `first` on (all of them with THREADS threads): a workgroup a chunk.
 template <uint32_t THREADS>

@@ -1210,7 +1210,8 @@ int mixers_step(const RmiAttnShape *as, const RmiAttnArgs *aa, const RmiRecurSha
         lds = split_lds(sizeof(T), p.s, 1);
     }
     if (rs && recur_step_lds(p.rs) > lds) lds = recur_step_lds(p.rs);
-    const dim3 grid(p.attn_blocks + p.rs.heads + rmi_ahead_blocks(ahead));
+    const uint32_t used = p.attn_blocks + p.rs.heads;
+    const dim3 grid(used + rmi_ahead_blocks(ahead, used, uint32_t(rmi_device_cus())));
     const uint32_t bucket = as ? bucket_of(p.s) : 64;
     auto go = [&](auto kernel) {
         const int rc = rmi_allow_lds(kernel, lds);
