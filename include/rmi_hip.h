@@ -123,10 +123,11 @@ int rmi_hip_matmul_q8_0_quantized_batch(const rmi_hip_weight *w, const uint8_t *
 int rmi_hip_set_forward_batched_mode(int mode);
 int rmi_hip_get_forward_batched_mode(void);
 /* Kernel::forward / forward_batched with f32 input (trait_.rs:59-109):
- * quantize each token row on the device (rounding as given), then the GEMV in
- * the x86-64 kernel's order for every token, eight tokens a launch.  As in the
- * reference, a token's result does not depend on the batch it arrives in:
- * forward_batched(x)[t] == forward(x[t]) bit for bit. */
+ * quantize each token row on the device (rounding as given), then products in
+ * the x86-64 kernel's order for every token: launches of the GEMV, or from nine
+ * tokens on one launch on the matrix cores where that is faster (the same
+ * bits).  As in the reference, a token's result does not depend on the batch it
+ * arrives in: forward_batched(x)[t] == forward(x[t]) bit for bit. */
 int rmi_hip_q8_0_forward_batched(const rmi_hip_weight *w, const float *input, float *output, uint32_t n_in,
                                  uint32_t n_out, uint32_t n_tokens, int rounding);
 /* The same call on the matrix cores, in the aarch64 kernel's accumulation order (neon.rs:49-73) for every

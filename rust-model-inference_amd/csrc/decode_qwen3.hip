@@ -1391,11 +1391,10 @@ bool pass_by_positions(const rmi_hip_qwen3_config &c, uint32_t step0, uint32_t n
     return uint64_t(n) * c.n_head <= 4u * uint32_t(rmi_device_cus()) && attn128_lds_bytes(step0 + n) <= 62 * 1024;
 }
 
-// n consecutive prompt positions from step0 on in one pass: every product reads its weight once for all of them
-// (the x86-64-order GEMV takes up to eight tokens a launch and gives each the bits it gets alone), the other
-// kernels run once per position inside one launch.  Position by position the arithmetic is that of enqueue_step's
-// separate-kernel path; a position's keys and values are in the cache before any attention launch of the pass
-// reads them.  Leaves every position's argmax and top-2 logits and, behind the last position, the step counter and the
+// n consecutive prompt positions from step0 on in one pass: a product of all of them gives each position the bits it gets
+// alone (rmi_gemv_q8_0_tokens), attention goes by positions or by sixteen of them, and the other kernels run once per
+// position inside one launch.  Position by position the arithmetic is that of enqueue_step's separate-kernel path; a
+// position's keys and values are in the cache before any attention launch of the pass reads them.  Leaves every position's argmax and top-2 logits and, behind the last position, the step counter and the
 // next token's embedding as a single step expects them.
 int enqueue_prompt_pass(rmi_hip_qwen3 *s, uint32_t step0, uint32_t n, const uint32_t *want, uint32_t n_want, hipStream_t st,
                         const RmiLogitsOf &of) {
