@@ -375,15 +375,15 @@ __global__ __launch_bounds__(64 * (BN / WN) * (BT / WT), WPS) void dense_gemm_wi
 }
 
 // Which tile a product takes: the least of estimates, in microseconds, that were fitted to every tile's time on 51 weights
-// (320..39968 rows of 256..20480 columns, plain, activated, paired and residual ones) with 17..2048 tokens, each launch with a
-// weight from HBM as in a model.  w: tiles a compute unit; `fit` of them run side by side and make a round.  A step of k
-// takes `round` in a whole round; the tiles left over take `first`, and `more` and `whole` for what is beyond one a compute
-// unit, by its share and by the whole tile.  An epilogue is not overlapped where a compute unit holds one workgroup, and adds
-// to or activates a whole tile: so much a tile, which decides between wide tiles at 1024 columns.
+// (64..39968 rows of 256..20480 columns; plain, activated, paired, table and residual ones) with 17..2048 tokens, each launch
+// with a weight from HBM as in a model.  `fit` tiles run side by side on a compute unit and make a round.  A step of k takes
+// `round` in a whole round; the tiles left over take `first`, and `more` and `whole` for what is beyond one a compute unit, by
+// its share and by the whole tile.  An epilogue is not overlapped where a compute unit holds one workgroup, and adds to or
+// activates a whole tile: so much a tile, which decides between wide tiles at 1024 columns.
 // bf16 is bound by LDS reads and the traffic between L2 and the compute units, so wider tiles are cheaper an element as long
 // as there are enough of them; f32 is bound by the matrix cores and every tile costs its area.  Over 597 products of bf16 and
-// as many of f32 the choice costs 0.7 % and 0.03 % over the best tile of each (four waves alone: 6 and 5 %).  E.g. in bf16, us by 64 x 64 |
-// 64 x 128 | 128 x 128 with four waves | with eight | 128 x 256 | 256 x 256:
+// as many of f32 the choice costs 0.7 % and 0.03 % over the best tile of each (four waves alone: 6 and 5 %).  E.g. in bf16, us
+// by 64 x 64 | 64 x 128 | 128 x 128 with four waves | with eight | 128 x 256 | 256 x 256:
 //   activated 12304 x 1024, 2048 tokens    138 |  129 | 103 | 104 | 121 | 120     768 tokens    54 |  53 |  47 |  50 |  67 |  61
 //   activated 39968 x 4096, 2048 tokens   1504 | 1169 | 797 | 846 | 760 | 687     512 tokens   320 | 280 | 210 | 231 | 233 | 264
 //   residual 4096 x 12288, 2048 tokens     375 |  303 | 246 | 239 | 193 | 341     512 tokens   102 | 104 | 150 | 170 | 195 | 357
