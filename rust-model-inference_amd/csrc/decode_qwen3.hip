@@ -1233,6 +1233,8 @@ struct rmi_hip_qwen3 : RmiSession {
     void *partialb = nullptr;
     float *attn_scratch = nullptr;       // of the pass's attention
     size_t attn_scratch_floats = 0;
+    RmiAttnLimbs attn_limbs;
+    std::vector<bool> limbs_hold;        // by layer: its norms keep queries and keys below what limbs hold
     void *attn_split = nullptr;          // scratch of the split attention launches (head dimension 128)
 
     ~rmi_hip_qwen3() override;
@@ -1381,18 +1383,18 @@ bool prompt_pass_possible(const rmi_hip_qwen3 *s, uint32_t step0, uint32_t n) {
     return s->xb && n > 0 && n <= prompt_batch(c.capacity) && step0 + n <= c.capacity && c.n_embd <= kNormMaxN;
 }
 
-// Whether a pass's attention takes a workgroup a position and head, as a single step's does, instead of one for sixteen
-// positions.  Sixteen positions' ordered sums and scratch are a longer chain that only pays where the chip has enough to do
-// in its shadow: up to four workgroups a compute unit the first way is never slower, whatever the context (16 heads, 12
-// layers, us a layer and pass, a workgroup a position | sixteen: 2 positions 33.2 | 37.4, 16: 39.9 | 43.6, 64: 57.1 | 57.4,
-// 96: 67.3 | 65.1; behind 900 keys 2: 44 | 87, 64: 84 | 105, 128: 121 | 112; 32 heads: 32: 53.2 | 53.8, 48: 62.7 | 57.3).
+// Whether a pass's attention takes a workgroup a position and head, as a single step's does, instead of one for sixteen or
+// 32 positions.  Many positions' ordered sums and scratch are a longer chain that only pays where the chip has enough to do
+// in its shadow: up to four workgroups a compute unit the first way is never slower, whatever the context (16 heads, us a layer
+// and pass, a workgroup a position | many: 2 positions 47.3 | 54.7, 16: 55.6 | 63.6, 64: 81.3 | 84.5; 1024 tokens in passes
+// of 2 44 | 67, of 64 88 | 98; 32 heads: 32: 234 | 242, 1024 tokens in passes of 32 226 | 234).
 // Its keys lie in LDS, as much as a launch may take unasked (64 KiB, the kernel's own arrays among them).
 bool pass_by_positions(const rmi_hip_qwen3_config &c, uint32_t step0, uint32_t n) {
     return uint64_t(n) * c.n_head <= 4u * uint32_t(rmi_device_cus()) && attn128_lds_bytes(step0 + n) <= 62 * 1024;
 }
 
 // n consecutive prompt positions from step0 on in one pass: a product of all of them gives each position the bits it gets
-// alone (rmi_gemv_q8_0_tokens), attention goes by positions or by sixteen of them, and the other kernels run once per
+// alone (rmi_gemv_q8_0_tokens), attention goes by positions or by tiles of them, and the other kernels run once per
 // position inside one launch.  Position by position the arithmetic is that of enqueue_step's separate-kernel path; a
 // position's keys and values are in the cache before any attention launch of the pass reads them.  Leaves every position's argmax and top-2 logits and, behind the last position, the step counter and the
 // next token's embedding as a single step expects them.
@@ -1422,7 +1424,8 @@ int enqueue_prompt_pass(rmi_hip_qwen3 *s, uint32_t step0, uint32_t n, const uint
                                attn128_lds_bytes(step0 + n), st, s->q16b, s->k_cache + layer_base, s->v_cache + layer_base, step0, s->kv_stride,
                                c.n_head, c.n_head_kv, s->act_q8b, s->act_scalesb, rnd, AttnFromQkv{});
         else if ((rc = rmi_launch_attn128_prompt(s->q16b, s->k_cache + layer_base, s->v_cache + layer_base, step0, n, s->kv_stride, c.n_head,
-                                                 c.n_head_kv, s->attn_scratch, s->attn_scratch_floats, s->act_q8b, s->act_scalesb, rnd, st)) != RMI_HIP_OK)
+                                                 c.n_head_kv, s->attn_scratch, s->attn_scratch_floats, s->attn_limbs, s->limbs_hold[l],
+                                                 s->act_q8b, s->act_scalesb, rnd, st)) != RMI_HIP_OK)
             return rc;
         rc = rmi_gemv_q8_0_tokens(s->w_o[l], s->act_q8b, s->act_scalesb, s->residb, n, c.n_embd, 0, c.n_embd, st);
         if (rc != RMI_HIP_OK) return rc;
@@ -1742,6 +1745,11 @@ rmi_hip_qwen3 *rmi_hip_qwen3_create(const rmi_hip_qwen3_config *cfg, const rmi_h
         if (ok) s->attn_norm.push_back(f);
         ok = ok && (f = upload_f32(s, wt->ffn_norm[l], c.n_embd));
         if (ok) s->ffn_norm.push_back(f);
+        // a vector of 128 whose mean square is one has no pair of elements longer than sqrt(128), and the rotation keeps lengths
+        float largest = c.has_qk_norm ? 0.0f : INFINITY;
+        for (uint32_t i = 0; c.has_qk_norm && i < c.head_dim_k; i++)
+            largest = fmaxf(largest, fmaxf(fabsf(wt->q_norm[l][i]), fabsf(wt->k_norm[l][i])));
+        s->limbs_hold.push_back(largest < 11.2f);
         if (ok && c.has_qk_norm) {
             ok = ok && (f = upload_f32(s, wt->q_norm[l], c.head_dim_k));
             if (ok) s->q_norm.push_back(f);
@@ -1779,6 +1787,11 @@ rmi_hip_qwen3 *rmi_hip_qwen3_create(const rmi_hip_qwen3_config *cfg, const rmi_h
              (s->logitsb = dev_alloc<float>(s, head * c.vocab)) &&
              (s->act_q8b = dev_alloc<int8_t>(s, n * s->max_n_in)) && (s->act_scalesb = dev_alloc<float>(s, n * s->max_n_in / 32)) &&
              (s->partialb = dev_alloc<Top>(s, head * kArgmaxGroups)) && (s->attn_scratch = dev_alloc<float>(s, s->attn_scratch_floats));
+        if (const size_t bytes = rmi_attn_limbs_bytes(c.n_head_kv, c.capacity)) {
+            void *p = ok ? dev_alloc<uint8_t>(s, bytes) : nullptr;
+            ok = p != nullptr;
+            s->attn_limbs = rmi_attn_limbs_at(p, c.n_head_kv, c.capacity);
+        }
     }
     if (ok && c.head_dim_k == 128 && c.head_dim_v == 128 && attn128_use_split(c.capacity, c.n_head))
         ok = (s->attn_split = dev_alloc<uint8_t>(s, attn_split_scratch_bytes(c.n_head, c.capacity), true)) != nullptr;

@@ -1,5 +1,5 @@
-"""Prompt passes of the Qwen3 session over the range of contexts: in larger passes sixteen positions of a head share a
-workgroup of the attention, so lengths on both sides of a tile, of a 64-key turn and of a pass, with the keys of earlier passes in
+"""Prompt passes of the Qwen3 session over the range of contexts: in larger passes 32 positions of a head share a
+workgroup of the attention, so lengths on both sides of a tile, of a 128-key turn and of a pass, with the keys of earlier passes in
 front.  Every position its own step is the reference (held to the CPU loop by test_gpu_decode_device.py): all bits equal."""
 import os
 
@@ -12,7 +12,7 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("heads,kv_heads,n_prompt,per_pass", [
     (8, 4, 2, True), (8, 4, 16, True), (8, 4, 17, True), (3, 3, 65, True), (8, 2, 127, 33), (4, 1, 512, True), (4, 4, 513, True),
     (2, 1, 700, 129), (4, 2, 1300, True), (2, 2, 2100, True),
-    # up to 1024 positions times heads (256 compute units) a workgroup takes one position, beyond that sixteen
+    # up to 1024 positions times heads (256 compute units) a workgroup takes one position, beyond that 32
     (8, 4, 128, True), (8, 4, 129, True), (64, 8, 16, True), (64, 8, 17, True), (64, 16, 33, True), (32, 8, 700, 40), (64, 8, 300, 63), (32, 4, 700, 30)])
 def test_passes_have_the_bits_of_single_steps(hip, tmp_path, heads, kv_heads, n_prompt, per_pass):
     path = os.path.join(str(tmp_path), "m.gguf")
@@ -47,6 +47,32 @@ def test_logits_of_every_position_of_a_pass(hip, tmp_path, n_prompt):
     assert np.array_equal(fast["dump"].view(np.uint32), slow["dump"].view(np.uint32))
 
 
+@pytest.mark.parametrize("heads,kv_heads,n_prompt,per_pass", [
+    # below and from a million products of a query and a key on (there in limbs)
+    (64, 8, 95, True), (32, 8, 130, True), (64, 8, 181, True), (64, 8, 224, True), (64, 8, 225, True), (32, 8, 257, True), (8, 2, 600, True), (64, 8, 330, 161)])
+@pytest.mark.parametrize("q,k,v", [(10.0, 10.0, 1.0), (40.0, 1.0, 1.0), (1.0, 1.0, 150.0), (10.0, 5.0, 400.0), (1e-5, 0.3, 1e-6)])
+def test_values_at_the_edge_of_what_limbs_hold(hip, tmp_path, heads, kv_heads, n_prompt, per_pass, q, k, v):
+    """Queries, keys and values times q, k, v: below 127 they go as four int8 limbs, a head that holds others in f64; large
+    scores make weights of one and a half (a fourth limb), small factors subnormal f16 values."""
+    path = os.path.join(str(tmp_path), "m.gguf")
+    hip.gguf.write_synthetic_qwen3(path, seed=heads, n_layer=2, n_embd=256, n_head=heads, n_head_kv=kv_heads, head_dim=128, n_ff=256, vocab=500, n_ctx=4096)
+    f = hip.gguf.GGUFFile(path)
+    t = {name: np.array(x[2]) for name, x in f.tensors.items()}
+    for layer in range(2):
+        t[f"blk.{layer}.attn_q_norm.weight"] = t[f"blk.{layer}.attn_q_norm.weight"] * np.float32(q)
+        t[f"blk.{layer}.attn_k_norm.weight"] = t[f"blk.{layer}.attn_k_norm.weight"] * np.float32(k)
+        blocks = t[f"blk.{layer}.attn_v.weight"].reshape(-1, 34)
+        blocks[:, :2] = (blocks[:, :2].copy().view(np.float16) * np.float16(v)).view(np.uint8)
+    session = hip.decode.Qwen3Session(f.metadata, t, capacity=n_prompt + 4)
+    prompt = np.random.default_rng(n_prompt).integers(0, 500, n_prompt, dtype=np.uint32)
+    session.set_prompt_passes(per_pass)
+    fast = session.generate(prompt, 2, dump_steps=range(n_prompt + 1))
+    session.set_prompt_passes(False)
+    slow = session.generate(prompt, 2, dump_steps=range(n_prompt + 1))
+    session.close()
+    assert np.array_equal(fast["dump"].view(np.uint32), slow["dump"].view(np.uint32))
+
+
 def _put(raw, n_in, row, block, scale, quants):
     """One block of 32 of a row of Q8_0 bytes."""
     b = raw.reshape(-1, n_in // 32, 34)[row, block]
@@ -55,7 +81,7 @@ def _put(raw, n_in, row, block, scale, quants):
 
 
 @pytest.mark.parametrize("seen", [True, False])
-@pytest.mark.parametrize("heads,n_prompt,at", [(2, 5, 4), (2, 40, 20), (64, 17, 16), (64, 18, 2), (64, 33, 32), (64, 40, 20), (64, 40, 35), (64, 100, 80), (64, 130, 129)])
+@pytest.mark.parametrize("heads,n_prompt,at", [(2, 5, 4), (2, 40, 20), (64, 17, 16), (64, 18, 2), (64, 33, 32), (64, 40, 20), (64, 40, 35), (64, 100, 80), (64, 130, 129), (64, 230, 20), (64, 230, 200), (64, 230, 229)])
 def test_a_value_that_is_not_finite_counts_from_its_position_on(hip, tmp_path, heads, n_prompt, at, seen):
     """One prompt token's values overflow f16.  seen: its weight is not zero, so that its position and those behind it have
     logits that are not finite, and their number is in the error.  Otherwise every weight of it rounds to zero: 0 x inf is
