@@ -1,5 +1,7 @@
 // Products of several tokens on dense bf16 / f32 weights: the inputs (norms) in front of them, a tiled matrix-core
 // GEMM with the layer's elementwise work in its epilogue (activations, gates, gated residual), and the embedding.
+#include <type_traits>
+
 #include "dense_launch.h"
 
 namespace {
@@ -54,6 +56,20 @@ __device__ __forceinline__ void fold_segment(f32x4 (&acc)[NN][NT], const RmiColS
             }
             acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
         }
+    }
+}
+
+// A segment's end: its results join x, or go on as part of the next one's.
+template <int NN, int NT>
+__device__ __forceinline__ void end_segment(f32x4 (&acc)[NN][NT], const RmiColSeg &s, float *__restrict__ x, uint32_t width, uint32_t n_tokens,
+                                            uint32_t row0, uint32_t tok0) {
+    if (s.carry == 0.0f) {
+        fold_segment<NN, NT>(acc, s, x, width, n_tokens, row0, tok0);
+    } else {
+#pragma unroll
+        for (int i = 0; i < NN; i++)
+#pragma unroll
+            for (int j = 0; j < NT; j++) acc[i][j] = acc[i][j] * s.carry;
     }
 }
 
@@ -132,6 +148,144 @@ __device__ __forceinline__ void store_rows(const f32x4 (&acc)[NN][NT], const Rmi
         }
     }
 }
+
+// The same results by whole lines: sixteen tokens at a time through LDS of the wave's own, from where a lane takes four
+// consecutive rows of one token and its neighbours the rows beside them.  From the registers a token's stores are 64 bytes (32
+// in bf16) of a line here and the rest of it in later instructions, and the code is written out for every tile of sixteen by
+// sixteen: with the activations more than the instruction cache holds, a miss a line in every wave.  Of 256 x 256 tiles in bf16
+// (activated, 39168 x 4096, 2048 tokens) 213 of 690 us were this epilogue; 146 of them are left (268 MB of f32 and bf16 results, and the
+// activations).  Segments are whole groups
+// of sixteen rows, so a lane's rows are one's; where the wave's rows are of several it goes through them one by one.
+// tile: 16 (WN + 4) floats.
+template <typename T, int EPI, int WN, int NN, int NT>
+__device__ __forceinline__ void store_lines(const f32x4 (&acc)[NN][NT], const RmiRowSegs &rs, uint32_t n_tokens, uint32_t first_row, uint32_t tok_first,
+                                            float *tile) {
+    constexpr uint32_t kLanes = WN / 4, kAtOnce = 64 / kLanes, kLd = WN + 4;  // lanes of a token, tokens of an instruction
+    constexpr bool kActs = EPI == kRowsActed || EPI == kRowsTimesTable;
+    const uint32_t lane = threadIdx.x & 63, fr = lane & 15, g = lane >> 4, r = lane % kLanes * 4;
+    for (uint32_t si = uint32_t(__builtin_amdgcn_readfirstlane(int(seg_of(rs, first_row)))); si < rs.n_segs; si++) {
+        const RmiRowSeg &s = rs.s[si];
+        if (s.row0 >= first_row + WN) break;
+        const uint32_t r0 = first_row + r - s.row0;  // (rows in front of the segment are far behind its end)
+        const bool whole = r0 < s.n && s.n - r0 >= 4 && (s.ld & 3) == 0;
+        f32x4 bias = {0.f, 0.f, 0.f, 0.f}, lower = bias;
+        if constexpr (kActs) {
+#pragma unroll
+            for (uint32_t e = 0; e < 4; e++) {
+                if (s.bias && r0 < s.n) bias[e] = s.bias[r0 + e < s.n ? r0 + e : s.n - 1];
+                if (s.lower && r0 < s.n) lower[e] = s.lower[r0 + e < s.n ? r0 + e : s.n - 1];
+            }
+        }
+        auto sixteen = [&](int j, auto act_c) {
+#pragma unroll 2
+            for (uint32_t t = lane / kLanes; t < 16; t += kAtOnce) {
+                f32x4 o = *reinterpret_cast<const f32x4 *>(tile + t * kLd + r);
+                const uint32_t tok = tok_first + j * 16 + t;
+                if (tok >= n_tokens || r0 >= s.n) break;
+                if constexpr (EPI == kRowsPaired) {  // (gate, up) twice: two results
+                    const float v0 = fmaxf(o[0], 0.0f) * o[1], v1 = fmaxf(o[2], 0.0f) * o[3];
+                    const size_t at = size_t(tok) * s.ld + r0 / 2;
+                    if (sizeof(T) == 2 && s.out_elem && r0 + 2 < s.n && (s.ld & 1) == 0) {  // side by side: one store
+                        reinterpret_cast<uint32_t *>(s.y)[at >> 1] = uint32_t(f32_to_bf16(v0)) | uint32_t(f32_to_bf16(v1)) << 16;
+                    } else {
+#pragma unroll
+                        for (uint32_t e = 0; e < 2; e++)
+                            if (r0 + 2 * e < s.n) {
+                                if (s.out_elem)
+                                    static_cast<T *>(s.y)[at + e] = from_f32<T>(e ? v1 : v0);
+                                else
+                                    static_cast<float *>(s.y)[at + e] = e ? v1 : v0;
+                            }
+                    }
+                } else {
+                    if constexpr (kActs) {
+#pragma unroll
+                        for (int e = 0; e < 4; e++) o[e] = apply_act<T>(decltype(act_c)::value, o[e], bias[e], lower[e]);
+                    }
+                    if constexpr (EPI == kRowsTimesTable) {
+                        if (s.mul) {
+                            const T *m = mul_row<T>(s, tok) + r0;
+#pragma unroll
+                            for (uint32_t e = 0; e < 4; e++)
+                                if (r0 + e < s.n) o[e] *= to_f32(m[e]);
+                        }
+                    }
+                    const size_t at = size_t(tok) * s.ld + r0;
+                    if (whole) {
+                        if (s.out_elem)
+                            store4(static_cast<T *>(s.y) + at, o);
+                        else
+                            store4(static_cast<float *>(s.y) + at, o);
+                    } else {
+#pragma unroll
+                        for (uint32_t e = 0; e < 4; e++)
+                            if (r0 + e < s.n) {
+                                if (s.out_elem)
+                                    static_cast<T *>(s.y)[at + e] = from_f32<T>(o[e]);
+                                else
+                                    static_cast<float *>(s.y)[at + e] = o[e];
+                            }
+                    }
+                }
+            }
+        };
+#pragma unroll
+        for (int j = 0; j < NT; j++) {
+#pragma unroll
+            for (int i = 0; i < NN; i++) *reinterpret_cast<f32x4 *>(tile + fr * kLd + i * 16 + g * 4) = acc[i][j];
+            rmi_wave_lds_fence();
+            switch (kActs ? s.act : uint16_t(kActNone)) {
+            case kActSigmoid: sixteen(j, std::integral_constant<uint32_t, kActSigmoid>{}); break;
+            case kActSilu: sixteen(j, std::integral_constant<uint32_t, kActSilu>{}); break;
+            case kActGeluTanh: sixteen(j, std::integral_constant<uint32_t, kActGeluTanh>{}); break;
+            case kActForgetGate: sixteen(j, std::integral_constant<uint32_t, kActForgetGate>{}); break;
+            default: sixteen(j, std::integral_constant<uint32_t, kActNone>{});
+            }
+            rmi_wave_lds_fence();
+        }
+    }
+}
+
+// The same for a product that joins x: what is there and the gates are asked for together, in front of the tiles' way through
+// LDS.
+template <int WN, int NT>
+struct ResidualLines {
+    static constexpr uint32_t kLanes = WN / 4, kAtOnce = 64 / kLanes, kLd = WN + 4, kTimes = 16 / kAtOnce;
+    f32x4 v[NT][kTimes], gate[NT][kTimes];
+
+    static __device__ __forceinline__ uint32_t row_of(uint32_t first_row) { return first_row + (threadIdx.x & 63) % kLanes * 4; }
+    static __device__ __forceinline__ uint32_t tok_of(uint32_t tok_first, int j, uint32_t k) { return tok_first + j * 16 + k * kAtOnce + (threadIdx.x & 63) / kLanes; }
+    __device__ __forceinline__ void load(const RmiColSeg &s, const float *x, uint32_t width, uint32_t n_tokens, uint32_t first_row, uint32_t tok_first) {
+        const uint32_t row = row_of(first_row) < width ? row_of(first_row) : width - 4;
+#pragma unroll
+        for (int j = 0; j < NT; j++)
+#pragma unroll
+            for (uint32_t k = 0; k < kTimes; k++) {
+                const uint32_t t = tok_of(tok_first, j, k), tok = t < n_tokens ? t : n_tokens - 1;
+                v[j][k] = *reinterpret_cast<const f32x4 *>(x + size_t(tok) * width + row);
+                gate[j][k] = f32x4{1.f, 1.f, 1.f, 1.f};
+                if (s.gate) gate[j][k] = *reinterpret_cast<const f32x4 *>(s.gate + size_t(tok) * s.gate_ld + row);
+            }
+    }
+    template <int NN>
+    __device__ __forceinline__ void add(const f32x4 (&acc)[NN][NT], const RmiColSeg &s, float *x, uint32_t width, uint32_t n_tokens, uint32_t first_row,
+                                        uint32_t tok_first, float *tile) {
+        const uint32_t lane = threadIdx.x & 63, fr = lane & 15, g = lane >> 4, row = row_of(first_row);
+#pragma unroll
+        for (int j = 0; j < NT; j++) {
+#pragma unroll
+            for (int i = 0; i < NN; i++) *reinterpret_cast<f32x4 *>(tile + fr * kLd + i * 16 + g * 4) = acc[i][j];
+            rmi_wave_lds_fence();
+#pragma unroll
+            for (uint32_t k = 0; k < kTimes; k++) {
+                const f32x4 o = *reinterpret_cast<const f32x4 *>(tile + (k * kAtOnce + lane / kLanes) * kLd + lane % kLanes * 4);
+                const uint32_t tok = tok_of(tok_first, j, k);
+                if (tok < n_tokens && row < width) *reinterpret_cast<f32x4 *>(x + size_t(tok) * width + row) = v[j][k] + o * s.scale * gate[j][k];
+            }
+            rmi_wave_lds_fence();
+        }
+    }
+};
 
 // Four waves; the pieces of the next PD steps are on their way to registers while one is multiplied.  Small tiles, for
 // products that would leave compute units idle otherwise, have two LDS buffers; 128 x 128 keeps one (NB = 1), so that three
@@ -234,7 +388,7 @@ __global__ __launch_bounds__(256, WPS) void dense_gemm_kernel(const T *__restric
                 __syncthreads();
             }
         }
-        if constexpr (RESIDUAL) fold_segment<NN, NT>(acc, cs.s[seg], x, width, n_tokens, row0 + wn + g * 4, tok0 + wt + fr);
+        if constexpr (RESIDUAL) end_segment<NN, NT>(acc, cs.s[seg], x, width, n_tokens, row0 + wn + g * 4, tok0 + wt + fr);
     }
 
     if constexpr (!RESIDUAL) store_rows<T, EPI, NN, NT>(acc, rs, n_rows, n_tokens, row0 + wn, tok0 + wt + fr, g);
@@ -248,8 +402,10 @@ constexpr int rmi_waitcnt(int vm) { return (vm & 15) | (vm >> 4) << 14 | 7 << 4;
 // piece that belongs at its slot) through NB buffers, one barrier a step: behind it the next step's first half is read while
 // the second half of this one is multiplied, and the buffer that everybody has read takes the step NB on.  The wait in front
 // of the barrier counts the loads in flight, so that those of NB - 2 steps stay under way.
-// What bounds it: LDS, 128 bytes a clock (a step of 128 x 256 reads 128 KB and writes 48: 0.6 us; its products alone would
-// take 0.43), and on a full chip the way from L2 (10 TB/s in 48 KB steps of 1.1 us).
+// What bounds it: the matrix cores at the clock that they have under full load, and the way from L2.  Of the 312 us of 128 x 256
+// tiles (4096 x 20480, 2048 tokens) the products and barriers alone are 263 (1300 TFLOP/s, what a large library product
+// reaches); 256 x 256 tiles (39168 x 4096) run their loop in 474 us, 1386 TFLOP/s, in front of 146 us of results; 64 x 128
+// tiles ask 96 bytes a clock and compute unit of L2, and take as long as that does.
 template <typename T, int BN, int BT, int WN, int WT, int NB, int WPS, int EPI>
 __global__ __launch_bounds__(64 * (BN / WN) * (BT / WT), WPS) void dense_gemm_wide_kernel(const T *__restrict__ w, const T *__restrict__ a, uint32_t n_rows, uint32_t k_pad,
                                                                  uint32_t ld, uint32_t n_tokens, uint32_t grid_n, uint32_t grid_t, uint32_t xcd_split,
@@ -282,7 +438,7 @@ __global__ __launch_bounds__(64 * (BN / WN) * (BT / WT), WPS) void dense_gemm_wi
         a_off[i] = (tok0 + r < n_tokens ? r : n_tokens - 1 - tok0) * stride + piece;
     }
     constexpr uint32_t kStepElems = kStepBytes / sizeof(T);
-    const uint32_t n_steps = k_pad / kStepElems;
+    const uint32_t first = RESIDUAL ? cs.k_begin / kStepElems : 0, n_steps = (RESIDUAL ? cs.s[cs.n_segs - 1].k_end : k_pad) / kStepElems;
     auto fetch = [&](u32x4 *buf, uint32_t step) {
         const uint32_t at = (step < n_steps ? step : n_steps - 1) * kStepBytes;  // (behind the last step: that one again, read by nobody)
 #pragma unroll
@@ -312,66 +468,84 @@ __global__ __launch_bounds__(64 * (BN / WN) * (BT / WT), WPS) void dense_gemm_wi
 #pragma unroll
             for (int j = 0; j < NT; j++) acc[i][j] = mma16<T>(fw[c][i], fa[c][j], acc[i][j]);
     };
-    // the products stay on their side of what surrounds them
-    auto pin = [&]() {
-#pragma unroll
-        for (int i = 0; i < NN; i++)
-#pragma unroll
-            for (int j = 0; j < NT; j += 2) asm volatile("" : "+v"(acc[i][j]), "+v"(acc[i][j + 1]));
-    };
-    static_assert(NT % 2 == 0, "pinned two at a time");
     static_assert(NB == 2 || NB == 3, "two or three buffers");
+    // The order of what stands between two of these: one of the LDS reads (and of the loads) behind every product or two.  Left
+    // to itself the compiler puts the reads behind the products, right in front of the wait for them (256 x 256, activated 39168 x
+    // 4096, 2048 tokens: 720 -> 690 us).
+    auto spread = [&](int loads) {
+        constexpr int kReads = NN + NT, kProducts = NN * NT * int(sizeof(T) == 2 ? 1 : 4);
+        constexpr int kEach = kProducts / (2 * kReads) > 0 ? kProducts / (2 * kReads) : 1;
+#pragma unroll
+        for (int i = 0; i < kReads; i++) {
+#pragma unroll
+            for (int n = 0; n < kEach; n++) __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+            if (i < loads) {
+                __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
+                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+            }
+            __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+        }
+        __builtin_amdgcn_sched_group_barrier(0x008, kProducts, 0);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    uint32_t seg = 0, seg_end = RESIDUAL ? cs.s[0].k_end / kStepElems : n_steps;
     auto step_of = [&](u32x4 *cur, u32x4 *next, uint32_t step) {
+        if (RESIDUAL && step == seg_end) {  // on into the next segment, in its scale
+#pragma unroll
+            for (int i = 0; i < NN; i++)
+#pragma unroll
+                for (int j = 0; j < NT; j++) acc[i][j] = acc[i][j] * cs.s[seg].carry;
+            seg_end = cs.s[++seg].k_end / kStepElems;
+        }
         read(cur, 1);
         multiply(0);
-        pin();
+        spread(0);
         // this step is in everybody's registers, the next one in LDS; the loads of the one after it stay in flight
         asm volatile("" ::: "memory");
         __builtin_amdgcn_s_waitcnt(rmi_waitcnt((NB - 2) * (FW + FA)));
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
         read(next, 0);
         fetch(cur, step + NB);
         multiply(1);
-        pin();
+        spread(FW + FA);
     };
-    fetch(buf0, 0);
-    fetch(buf1, 1);
-    if constexpr (NB == 3) fetch(buf2, 2);
+    fetch(buf0, first);
+    fetch(buf1, first + 1);
+    if constexpr (NB == 3) fetch(buf2, first + 2);
     __builtin_amdgcn_s_waitcnt(rmi_waitcnt((NB - 1) * (FW + FA)));
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
     read(buf0, 0);
-    uint32_t step = 0;
-    if constexpr (NB == 2) {
-        for (uint32_t seg = 0; seg < (RESIDUAL ? cs.n_segs : 1u); seg++) {
-            const uint32_t seg_end = RESIDUAL ? cs.s[seg].k_end / kStepElems : n_steps;  // a multiple of four
-            for (; step < seg_end; step += 2) {
-                step_of(buf0, buf1, step);
-                step_of(buf1, buf0, step + 1);
-            }
-            if constexpr (RESIDUAL) fold_segment<NN, NT>(acc, cs.s[seg], x, width, n_tokens, row0 + wn + g * 4, tok0 + wt + fr);
-        }
-    } else {
-        uint32_t seg = 0, seg_end = RESIDUAL ? cs.s[0].k_end / kStepElems : n_steps;
-        auto ended = [&]() {  // the step just made was the last one
-            if (++step < seg_end) return false;
-            if constexpr (RESIDUAL) {
-                fold_segment<NN, NT>(acc, cs.s[seg], x, width, n_tokens, row0 + wn + g * 4, tok0 + wt + fr);
-                if (++seg < cs.n_segs) seg_end = cs.s[seg].k_end / kStepElems;
-            }
-            return step == n_steps;
-        };
-        for (;;) {
-            step_of(buf0, buf1, step);
-            if (ended()) break;
-            step_of(buf1, buf2, step);
-            if (ended()) break;
-            step_of(buf2, buf0, step);
-            if (ended()) break;
-        }
+    // Whole turns of the buffers in a loop that has no other way out: with one, the compiler takes it that a buffer may be read
+    // right behind its fetch, and waits for every load in flight once a turn (128 x 256, residual 4096 x 20480, 2048 tokens: 367 us with that and the
+    // results joining x from the registers, segments in the loop; 312 without, a launch for each gate).
+    uint32_t step = first;
+    auto buffer = [&](int i) { return i % NB == 0 ? buf0 : i % NB == 1 ? buf1 : buf2; };
+    for (; step + NB <= n_steps; step += NB) {
+#pragma unroll
+        for (int i = 0; i < NB; i++) step_of(buffer(i), buffer(i + 1), step + i);
     }
-    if constexpr (!RESIDUAL) store_rows<T, EPI, NN, NT>(acc, rs, n_rows, n_tokens, row0 + wn, tok0 + wt + fr, g);
+    if (step < n_steps) step_of(buffer(0), buffer(1), step);
+    if (NB == 3 && step + 1 < n_steps) step_of(buffer(1), buffer(2), step + 1);
+
+    if (RESIDUAL && (width & 3)) {
+        fold_segment<NN, NT>(acc, cs.s[cs.n_segs - 1], x, width, n_tokens, row0 + wn + g * 4, tok0 + wt + fr);
+        return;
+    }
+    __builtin_amdgcn_s_waitcnt(rmi_waitcnt(0));  // the steps behind the end are in LDS, and everybody has read the last one
+    ResidualLines<WN, NT> there;
+    if constexpr (RESIDUAL) there.load(cs.s[cs.n_segs - 1], x, width, n_tokens, row0 + wn, tok0 + wt);
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    constexpr uint32_t kTile = 16 * (WN + 4) / 4;  // in pieces; half of the waves' in either buffer
+    static_assert(WAVES / 2 * kTile <= (BN + BT) * 8, "the waves' tiles fit the buffers");
+    float *tile = reinterpret_cast<float *>((wave < WAVES / 2 ? buf0 : buf1) + wave % (WAVES / 2) * kTile);
+    if constexpr (RESIDUAL)
+        there.template add<NN>(acc, cs.s[cs.n_segs - 1], x, width, n_tokens, row0 + wn, tok0 + wt, tile);
+    else
+        store_lines<T, EPI, WN, NN, NT>(acc, rs, n_tokens, row0 + wn, tok0 + wt, tile);
 }
 
 // Which tile a product takes: the least of estimates, in microseconds, that were fitted to every tile's time on 51 weights
@@ -387,6 +561,8 @@ __global__ __launch_bounds__(64 * (BN / WN) * (BT / WT), WPS) void dense_gemm_wi
 //   activated 12304 x 1024, 2048 tokens    138 |  129 | 103 | 104 | 121 | 120     768 tokens    54 |  53 |  47 |  50 |  67 |  61
 //   activated 39968 x 4096, 2048 tokens   1504 | 1169 | 797 | 846 | 760 | 687     512 tokens   320 | 280 | 210 | 231 | 233 | 264
 //   residual 4096 x 12288, 2048 tokens     375 |  303 | 246 | 239 | 193 | 341     512 tokens   102 | 104 | 150 | 170 | 195 | 357
+// (Fitted and measured with results that left the wide tiles from the registers; by lines they are 5 to 15 % faster, which the
+// estimates don't know: the choice errs to the narrower side.)
 enum DenseTile { kTile64x16, kTile64x32, kTile64x64, kTile64x128, kTile128x128w4, kTile128x128, kTile128x256, kTile256x256 };
 struct TileCost {
     DenseTile tile;
@@ -435,24 +611,38 @@ int launch_gemm(const RmiDense &w, const void *a, const RmiRowSegs &rs, const Rm
                 uint32_t n_tokens, hipStream_t st) {
     const uint32_t n_rows = EPI == kResidual ? width : w.n_rows;
     const TileCost &tile = dense_tile_of(sizeof(T) == 2, EPI, n_rows, n_tokens, uint32_t(w.k_pad * sizeof(T) / kStepBytes));
-    auto go = [&](auto kernel) {
+    auto launch = [&](auto kernel, const RmiColSegs &c) {
         const uint32_t gn = (n_rows + tile.rows - 1) / tile.rows, gt = (n_tokens + tile.tokens - 1) / tile.tokens;
         const uint32_t split = rmi_gemm_xcd_split(gn, gt, double(n_rows) * w.k_pad, double(n_tokens) * w.k_pad);
         hipLaunchKernelGGL(kernel, dim3(gn * gt), dim3(64 * tile.waves), 0, st, static_cast<const T *>(w.data), static_cast<const T *>(a), n_rows,
-                           w.k_pad, w.ld, n_tokens, gn, gt, split, rs, cs, x, width);
+                           w.k_pad, w.ld, n_tokens, gn, gt, split, rs, c, x, width);
+    };
+    auto go = [&](auto kernel) { launch(kernel, cs); };
+    auto go_wide = [&](auto kernel) {  // a launch for every run of segments whose sums go on into the next
+        if constexpr (EPI != kResidual) {
+            launch(kernel, cs);
+        } else {
+            for (uint32_t i = 0; i < cs.n_segs;) {
+                RmiColSegs run{};
+                run.k_begin = i ? cs.s[i - 1].k_end : 0;
+                do run.s[run.n_segs++] = cs.s[i];
+                while (cs.s[i++].carry != 0.0f);
+                launch(kernel, run);
+            }
+        }
     };
     switch (tile.tile) {
     case kTile64x16: go(dense_gemm_kernel<T, 64, 16, 16, 16, 4, 2, 4, EPI>); break;
     case kTile64x32: go(dense_gemm_kernel<T, 64, 32, 32, 16, 4, 2, 4, EPI>); break;
     case kTile64x64: go(dense_gemm_kernel<T, 64, 64, 32, 32, 4, 2, 4, EPI>); break;
-    case kTile64x128: go(dense_gemm_wide_kernel<T, 64, 128, 32, 32, 3, 2, EPI>); break;
-    case kTile128x128: go(dense_gemm_wide_kernel<T, 128, 128, 64, 32, 2, 4, EPI>); break;
+    case kTile64x128: go_wide(dense_gemm_wide_kernel<T, 64, 128, 32, 32, 3, 2, EPI>); break;
+    case kTile128x128: go_wide(dense_gemm_wide_kernel<T, 128, 128, 64, 32, 2, 4, EPI>); break;
     default:
         if constexpr (sizeof(T) == 2) {
             if (tile.tile == kTile128x128w4) go(dense_gemm_kernel<T, 128, 128, 64, 64, 1, 1, 3, EPI>);
-            if (tile.tile == kTile128x256) go(dense_gemm_wide_kernel<T, 128, 256, 64, 64, 3, 2, EPI>);
+            if (tile.tile == kTile128x256) go_wide(dense_gemm_wide_kernel<T, 128, 256, 64, 64, 3, 2, EPI>);
             if constexpr (EPI != kResidual)
-                if (tile.tile == kTile256x256) go(dense_gemm_wide_kernel<T, 256, 256, 128, 64, 2, 2, EPI>);
+                if (tile.tile == kTile256x256) go_wide(dense_gemm_wide_kernel<T, 256, 256, 128, 64, 2, 2, EPI>);
         }
     }
     RMI_HIP_CHECK(hipGetLastError());
@@ -515,6 +705,16 @@ int rmi_dense_gemm_residual(uint32_t elem_bytes, const RmiDense &w, const void *
     if (n_tokens == 0) return RMI_HIP_OK;
     const int rc = rmi_check_col_segs(elem_bytes, w, segs, width);
     if (rc != RMI_HIP_OK) return rc;
-    return elem_bytes == 2 ? launch_gemm<rmi_bf16, kResidual>(w, a, RmiRowSegs{}, segs, x, width, n_tokens, st)
-                           : launch_gemm<float, kResidual>(w, a, RmiRowSegs{}, segs, x, width, n_tokens, st);
+    // A segment that ends reads and writes all of x and reads its gate; where the next one has the same gate, its sums go on
+    // from these instead, in the next one's scale (4096 x 20480, 2048 tokens, three segments of two gates: 384 -> 367 us).
+    RmiColSegs carried = segs;
+    carried.s[segs.n_segs - 1].carry = 0.0f;
+    for (uint32_t i = 0; i + 1 < segs.n_segs; i++) {
+        const RmiColSeg &s0 = segs.s[i], &s1 = segs.s[i + 1];
+        const float ratio = s1.scale != 0.0f ? s0.scale / s1.scale : 0.0f;
+        const bool same = s0.gate == s1.gate && (!s0.gate || s0.gate_ld == s1.gate_ld);
+        carried.s[i].carry = same && fabsf(ratio) >= 0x1p-10f && fabsf(ratio) <= 0x1p10f ? ratio : 0.0f;
+    }
+    return elem_bytes == 2 ? launch_gemm<rmi_bf16, kResidual>(w, a, RmiRowSegs{}, carried, x, width, n_tokens, st)
+                           : launch_gemm<float, kResidual>(w, a, RmiRowSegs{}, carried, x, width, n_tokens, st);
 }

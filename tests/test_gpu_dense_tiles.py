@@ -258,3 +258,67 @@ def test_every_tile(hip, tile, kind, size):
             want, bound = want * rows_of, bound * np.abs(rows_of)
         bound = bound + (2.0**-14 if acts[i] else 2.0**-22) * np.abs(want) + (2.0**-8 * np.abs(want) if short else 0) + 2.0**-20
         assert (np.abs(got - want) <= bound).all(), (i, np.abs(got - want).max())
+
+
+@pytest.mark.parametrize("elem,rows,tokens", [(2, 6800, 909), (2, 4832, 205), (2, 17296, 205), (2, 4100, 1025), (2, 1002, 130), (2, 80, 45), (4, 12576, 109), (4, 28576, 205)])
+def test_residual_segments_of_one_gate(hip, elem, rows, tokens):
+    """Segments that share a gate in scales of their own go on from each other's sums; one with another gate, or a scale of zero
+    behind it, ends them.  Four segments of 4, 8, 4 and 8 steps of bf16: ends at every place of the buffers' turn."""
+    H = hip.hip
+    ends, gates = (256, 768, 1024, 1536), (0, 0, 1, 1)
+    for scales in ((1.0, 0.75, 0.5, 1.5), (1.0, 0.75, 0.5, 0.0)):
+        rng = np.random.default_rng(rows)
+        padded = (rows + 15) // 16 * 16
+        w, wv, ld = _operand(rng, padded, ends[-1], elem)
+        a, av, _ = _operand(rng, tokens, ends[-1], elem)
+        x = rng.standard_normal((tokens, rows), dtype=np.float32)
+        gate = rng.uniform(0, 1, (2, tokens, rows)).astype(np.float32)
+        bufs = [H.DeviceBuffer.from_array(v) for v in (w, a, x, gate[0], gate[1])]
+        segs, want, size, first = ColSegs(), x.astype(np.float64), 0.0, 0
+        for i in range(4):
+            segs.s[i] = ColSeg(bufs[3 + gates[i]].ptr, rows, scales[i], ends[i])
+            part = np.s_[:, first:ends[i]]
+            want = want + scales[i] * gate[gates[i]] * (av[part] @ wv[:rows][part].T)
+            size = size + 2.0 * np.abs(av[part]) @ np.abs(wv[:rows][part]).T
+            first = ends[i]
+        segs.n_segs = 4
+        assert getattr(H.lib, RESIDUAL)(C.c_uint32(elem), C.byref(Dense(bufs[0].ptr, padded, ends[-1], ld)), C.c_void_p(bufs[1].ptr), C.byref(segs),
+                                        C.c_void_p(bufs[2].ptr), C.c_uint32(rows), C.c_uint32(tokens), None) == 0
+        H.check(H.lib.rmi_hip_synchronize())
+        got = bufs[2].to_array(np.float32, (tokens, rows))
+        # sums of k products as above, and a few roundings of what they are part of
+        assert (np.abs(got - want) <= 2 * ends[-1] * 2.0**-24 * size + 2.0**-21 * (np.abs(x) + np.abs(want))).all()
+
+
+@pytest.mark.parametrize("elem,last,k,tokens", [(2, 12704, 2048, 909), (2, 6800, 2048, 909), (2, 4832, 512, 205), (2, 17296, 512, 205), (4, 12576, 512, 109)])
+@pytest.mark.parametrize("narrow", [(16, 13, 32, 7), (48, 2, 100, 30)])
+def test_narrow_segments_of_a_wide_tile(hip, elem, last, k, tokens, narrow):
+    """Several segments within a wave's rows, of lengths and distances that are not whole quads, in either type; nothing is
+    written between a segment's rows."""
+    H = hip.hip
+    rng = np.random.default_rng(last + k)
+    lengths, segs, row = [*narrow, last], RowSegs(), 0
+    rows = sum((n + 15) // 16 * 16 for n in lengths)
+    w, wv, ld = _operand(rng, rows, k, elem)
+    x, xv, _ = _operand(rng, tokens, k, elem)
+    bufs, outs = [H.DeviceBuffer.from_array(v) for v in (w, x)], []
+    for i, n in enumerate(lengths):
+        out_elem, stride = i % 2, n + (i % 3)
+        old = np.full((tokens, stride), 7, np.uint16 if out_elem and elem == 2 else np.float32)
+        bufs.append(H.DeviceBuffer.from_array(old))
+        outs.append((row, n, stride, old.dtype))
+        segs.s[i] = RowSeg(bufs[-1].ptr, None, None, None, None, 0, 0, row, n, stride, 0, out_elem)
+        segs.start[i] = row
+        row += (n + 15) // 16 * 16
+    segs.start[len(lengths):] = [rows] * (12 - len(lengths))
+    segs.n_segs, segs.n_rows = len(lengths), rows
+    assert getattr(H.lib, ROWS)(C.c_uint32(elem), C.byref(Dense(bufs[0].ptr, rows, k, ld)), C.c_void_p(bufs[1].ptr), C.byref(segs), C.c_uint32(tokens), None) == 0
+    H.check(H.lib.rmi_hip_synchronize())
+    for buf, (row0, n, stride, dtype) in zip(bufs[2:], outs):
+        got = buf.to_array(dtype, (tokens, stride))
+        assert (got[:, n:] == 7).all()
+        bits = dtype == np.uint16
+        got = ((got.astype(np.uint32) << 16).view(np.float32) if bits else got)[:, :n]
+        want = xv @ wv[row0:row0 + n].T
+        bound = 2 * k * 2.0**-24 * (np.abs(xv) @ np.abs(wv[row0:row0 + n]).T) + (2.0**-8 * np.abs(want) if bits else 0)
+        assert (np.abs(got - want) <= bound).all()
