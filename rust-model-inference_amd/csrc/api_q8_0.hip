@@ -146,16 +146,16 @@ int host_gemv_range(const rmi_hip_weight *w, const uint8_t *input_q8, const floa
     int rc = stage_x(c, input_q8, input_scales, size_t(n_tokens) * w->n_in, size_t(n_tokens) * (w->n_in / 32), &x);
     if (rc != RMI_HIP_OK) return rc;
     const uint32_t n_rows = row_end - row_start;
-    float *d_y = static_cast<float *>(rmi_dev_buf(c, 1, size_t(n_tokens) * n_rows * 4));
-    if (!d_y) return RMI_HIP_E_RUNTIME;
-    // device y holds only the row slice: y[t][row - row_start]
-    rc = rmi_gemv_q8_0_tokens(w, x.d_q8, x.d_scales, d_y - row_start, n_tokens, n_rows, row_start, row_end, c->stream);
-    if (rc != RMI_HIP_OK) return rc;
-    if (out_stride == n_rows) return fetch(c, out_row_start, d_y, size_t(n_tokens) * n_rows * 4, 1);
+    // only the row slice, y[t][row - row_start], straight into pinned memory (see forward_batched)
     float *pin = static_cast<float *>(rmi_pin_buf(c, 1, size_t(n_tokens) * n_rows * 4));
     if (!pin) return RMI_HIP_E_RUNTIME;
-    RMI_HIP_CHECK(hipMemcpyAsync(pin, d_y, size_t(n_tokens) * n_rows * 4, hipMemcpyDeviceToHost, c->stream));
+    rc = rmi_gemv_q8_0_tokens(w, x.d_q8, x.d_scales, pin - row_start, n_tokens, n_rows, row_start, row_end, c->stream);
+    if (rc != RMI_HIP_OK) return rc;
     RMI_HIP_CHECK(hipStreamSynchronize(c->stream));
+    if (out_stride == n_rows) {
+        memcpy(out_row_start, pin, size_t(n_tokens) * n_rows * 4);
+        return RMI_HIP_OK;
+    }
     for (uint32_t t = 0; t < n_tokens; t++)
         memcpy(out_row_start + size_t(t) * out_stride, pin + size_t(t) * n_rows, size_t(n_rows) * 4);
     return RMI_HIP_OK;
@@ -218,14 +218,21 @@ static int forward_batched(const rmi_hip_weight *w, const float *input, float *o
     RmiThreadCtx *c = rmi_thread_ctx();
     if (!c) return RMI_HIP_E_RUNTIME;
     const size_t n_x = size_t(n_tokens) * n_in;
-    float *pin = static_cast<float *>(rmi_pin_buf(c, 0, n_x * 4));
-    float *d_x = static_cast<float *>(rmi_dev_buf(c, 0, n_x * 4));
+    const size_t x_bytes = n_x * 4, y_bytes = size_t(n_tokens) * n_out * 4;
+    // The quantizer reads every input once and the x86-64-order products write every result once, so both may use the pinned
+    // buffers themselves: a copy command less on either side, each of which is 5 to 8 us between dependent kernels.  From some
+    // 700 KB on the copy is the faster reader; writing was never slower (512 x 500 to 4096 x 12000, 1 to 300 tokens).  us with
+    // copies | x in place | y in place | both: 2048 x 6144, 1 token 31.5 | 28.5 | 22.4 | 20.4, 13 tokens 60.9 | 54.9 | 53.0 |
+    // 45.5, 100 tokens (800 KB) 209.0 | 211.1 | 200.3 | 202.6; 8192 x 3000, 300 tokens (9.6 MB) 616 | 661 | 571 | 612.
+    const bool x_in_place = x_bytes <= 512 * 1024, y_in_place = x86_order;
+    float *pin = static_cast<float *>(rmi_pin_buf(c, 0, x_bytes));
+    float *d_x = x_in_place ? pin : static_cast<float *>(rmi_dev_buf(c, 0, x_bytes));
     int8_t *d_q8 = static_cast<int8_t *>(rmi_dev_buf(c, 2, n_x));
     float *d_sc = static_cast<float *>(rmi_dev_buf(c, 3, n_x / 32 * 4));
-    float *d_y = static_cast<float *>(rmi_dev_buf(c, 1, size_t(n_tokens) * n_out * 4));
+    float *d_y = static_cast<float *>(y_in_place ? rmi_pin_buf(c, 1, y_bytes) : rmi_dev_buf(c, 1, y_bytes));
     if (!pin || !d_x || !d_q8 || !d_sc || !d_y) return RMI_HIP_E_RUNTIME;
-    memcpy(pin, input, n_x * 4);
-    RMI_HIP_CHECK(hipMemcpyAsync(d_x, pin, n_x * 4, hipMemcpyHostToDevice, c->stream));
+    memcpy(pin, input, x_bytes);
+    if (!x_in_place) RMI_HIP_CHECK(hipMemcpyAsync(d_x, pin, x_bytes, hipMemcpyHostToDevice, c->stream));
     rc = rmi_launch_quantize_q8_0(d_x, d_q8, d_sc, n_tokens, n_in, rounding, c->stream);
     if (rc != RMI_HIP_OK) return rc;
     // (measured per launch: the small-batch kernel is level with the GEMM or ahead up to 16 tokens for any matrix
@@ -248,7 +255,10 @@ static int forward_batched(const rmi_hip_weight *w, const float *input, float *o
                              n_tokens - t0 < chunk ? n_tokens - t0 : chunk, n_out, 0, n_out, c->stream);
     }
     if (rc != RMI_HIP_OK) return rc;
-    return fetch(c, output, d_y, size_t(n_tokens) * n_out * 4, 1);
+    if (!y_in_place) return fetch(c, output, d_y, y_bytes, 1);
+    RMI_HIP_CHECK(hipStreamSynchronize(c->stream));
+    memcpy(output, d_y, y_bytes);
+    return RMI_HIP_OK;
 }
 
 int rmi_hip_q8_0_forward_batched(const rmi_hip_weight *w, const float *input, float *output, uint32_t n_in,

@@ -717,3 +717,19 @@ def test_misaligned_device_pointers_are_refused(hip):
     rc = H.lib.rmi_hip_gemv_q4_k_q8k_dev(q4k.w.handle, buf.ptr, buf.ptr + 1024, buf.ptr + 2048 + 2, y.ptr, 1, 16, 0, 16, None)
     assert rc == -1 and "aligned" in H.last_error()
     H.check(H.lib.rmi_hip_synchronize())
+
+
+@pytest.mark.parametrize("n_tokens", [1, 32, 33, 5])
+def test_host_batches_on_both_sides_of_the_input_copy(hip, oracle, n_tokens):
+    """Inputs of up to 512 KB are read where the host left them, larger ones are copied first: 32 and 33 tokens of 4096."""
+    n_in, n_out = 4096, 200
+    w = hip.synth.q8_0_weight(5, n_out, n_in)
+    kernel = hip.kernel.Q8Kernel(w, n_in, n_out)
+    for seed in (1, 2):  # the buffers of the call before, with other inputs
+        x = hip.synth.activations(seed, n_tokens, n_in)
+        y = np.zeros((n_tokens, n_out), np.float32)
+        kernel.forward_batched(x, y, n_in, n_out)
+        for t in {0, n_tokens // 2, n_tokens - 1}:
+            q8, sc = oracle.quantize_q8_0(x[t], oracle.AVX2)
+            want = oracle.matmul_q8_0_quantized(w, q8, sc, n_in, n_out, oracle.AVX2)
+            assert np.array_equal(y[t].view(np.uint32), want.view(np.uint32))
