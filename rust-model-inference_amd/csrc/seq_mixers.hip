@@ -961,12 +961,19 @@ __global__ __launch_bounds__(256) void recur_factors_kernel(RmiRecurShape s, Rmi
 // state's row tiles w, w + 4, ..  A tile of the state in accumulator form (row 4g + r in register r) is the right
 // operand of (q P) S as it lies.  The segments of a long pass run side by side: a first launch (STATE_ONLY) takes every
 // segment but the last from a zero state and leaves what it adds and how much it keeps; the second puts its starting
-// state together from those before it.
-template <int TPW, bool STATE_ONLY>
+// state together from those before it.  Heads go round the XCDs: the workgroups of a head read the same factors.
+// What bounds it: the chain from one chunk's state to the next, 1.3 us a chunk (two segments of 64, 32 heads of 128).  So the
+// state waits for nothing else: the waves' parts of o meet once in four chunks, when each wave finishes one of the four; FULL,
+// where every wave has all its row tiles, makes a chunk straight-line code in which the tiles' chains of products run side by
+// side; a value past the end is taken out where it is used, not behind its load, and whole groups of chunks have no way out
+// (either made the compiler wait for every load in flight once a turn of the ring).  2048 tokens, the two launches: 47 and 118
+// us with a barrier and a branch a chunk and the value blocks of a head on eight XCDs, 45 and 104 with the head on one, 36 and 88.
+template <int TPW, bool STATE_ONLY, bool FULL>
 __global__ __launch_bounds__(256) void recur_scan_kernel(RmiRecurShape s, RmiRecurArgs a, uint32_t n_chunks, uint32_t seg_chunks) {
-    __shared__ f32x4 part[2][4][64];
+    constexpr uint32_t kGroup = 4;  // chunks whose parts of o meet at one barrier
+    __shared__ f32x4 part[STATE_ONLY ? 1 : 2][kGroup][4][64];
     const uint32_t tid = threadIdx.x, lane = tid & 63, wave = uint32_t(__builtin_amdgcn_readfirstlane(int(tid >> 6))), fr = lane & 15, g = lane >> 4;
-    const uint32_t head = blockIdx.y, v0 = blockIdx.x * 16, seg = blockIdx.z, n_tiles = s.d_pad / 16;
+    const uint32_t head = blockIdx.x, v0 = blockIdx.y * 16, seg = blockIdx.z, n_tiles = s.d_pad / 16;
     const uint32_t c_begin = seg * seg_chunks, c_end = c_begin + seg_chunks < n_chunks ? c_begin + seg_chunks : n_chunks;
     const RecurScratch ws = recur_scratch_at(a.scratch, s, n_chunks);
     f32x4 st[TPW], kept[TPW];
@@ -1007,8 +1014,7 @@ __global__ __launch_bounds__(256) void recur_scan_kernel(RmiRecurShape s, RmiRec
         for (int r = 0; r < 4; r++) {
             const uint32_t t = chunk * kChunk + g * 4 + r;
             const bool live = t < a.n_tokens && v0 + fr < s.vdim;
-            const float v = a.v[live ? size_t(t) * s.heads * s.vdim + size_t(head) * s.vdim + v0 + fr : 0];
-            x.v[r] = live ? v : 0.0f;
+            x.v[r] = a.v[live ? size_t(t) * s.heads * s.vdim + size_t(head) * s.vdim + v0 + fr : 0];
         }
         return x;
     };
@@ -1016,33 +1022,48 @@ __global__ __launch_bounds__(256) void recur_scan_kernel(RmiRecurShape s, RmiRec
     Operands ring[kAhead];
 #pragma unroll
     for (uint32_t j = 0; j < kAhead; j++) ring[j] = load(c_begin + j < c_end ? c_begin + j : c_end - 1);
-    for (uint32_t chunk0 = c_begin; chunk0 < c_end; chunk0 += kAhead) {
+    auto step = [&](uint32_t j, uint32_t chunk) __attribute__((always_inline)) {
+        const Operands &x = ring[j % kAhead];
+        f32x4 v;
 #pragma unroll
-        for (uint32_t j = 0; j < kAhead; j++) {
-            const uint32_t chunk = chunk0 + j;
-            if (chunk >= c_end) break;
-            const Operands &x = ring[j];
-            f32x4 o[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};  // two chains
-            if (!STATE_ONLY && wave == 3) o[0] = mma16_f32(x.am, x.v, o[0]);
+        for (uint32_t r = 0; r < 4; r++) v[r] = chunk * kChunk + g * 4 + r < a.n_tokens && v0 + fr < s.vdim ? x.v[r] : 0.0f;
+        f32x4 o[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};  // two chains
+        if (!STATE_ONLY && wave == 3) o[0] = mma16_f32(x.am, v, o[0]);
 #pragma unroll
-            for (int i = 0; i < TPW; i++) {
-                if (wave + 4 * i >= n_tiles) continue;
-                if (!STATE_ONLY) o[(i + 1) & 1] = mma16_f32(x.q[STATE_ONLY ? 0 : i], st[i], o[(i + 1) & 1]);
-                st[i] *= x.p[i];
-                if (STATE_ONLY) kept[i] *= x.p[i];
-                st[i] = mma16_f32(x.k[i], x.v, st[i]);
-            }
-            ring[j] = load(chunk + kAhead < c_end ? chunk + kAhead : c_end - 1);
-            if (STATE_ONLY) continue;
-            part[chunk & 1][wave][lane] = o[0] + o[1];
-            __syncthreads();  // (two buffers: the next chunk's writes cannot meet this one's reads)
-            if (wave == (chunk & 3)) {
-                const f32x4 sum = (part[chunk & 1][0][lane] + part[chunk & 1][1][lane]) + (part[chunk & 1][2][lane] + part[chunk & 1][3][lane]);
-                float *dst = ws.o + ((size_t(head) * n_chunks + chunk) * kChunk + g * 4) * s.v_pad + v0 + fr;
-#pragma unroll
-                for (int r = 0; r < 4; r++) dst[size_t(r) * s.v_pad] = sum[r];
-            }
+        for (int i = 0; i < TPW; i++) {
+            if (!FULL && wave + 4 * i >= n_tiles) continue;
+            if (!STATE_ONLY) o[(i + 1) & 1] = mma16_f32(x.q[STATE_ONLY ? 0 : i], st[i], o[(i + 1) & 1]);
+            st[i] *= x.p[i];
+            if (STATE_ONLY) kept[i] *= x.p[i];
+            st[i] = mma16_f32(x.k[i], v, st[i]);
         }
+        ring[j % kAhead] = load(chunk + kAhead < c_end ? chunk + kAhead : c_end - 1);
+        if (!STATE_ONLY) part[(chunk - c_begin) / kGroup & 1][j][wave][lane] = o[0] + o[1];
+    };
+    // o of a group's chunks, one a wave
+    auto finish = [&](uint32_t chunk0, uint32_t n) __attribute__((always_inline)) {
+        if (STATE_ONLY) return;
+        __syncthreads();  // (two buffers: the next group's writes cannot meet this one's reads)
+        if (wave >= n) return;
+        const f32x4 (&p)[4][64] = part[(chunk0 - c_begin) / kGroup & 1][wave];
+        const f32x4 sum = (p[0][lane] + p[1][lane]) + (p[2][lane] + p[3][lane]);
+        float *dst = ws.o + ((size_t(head) * n_chunks + chunk0 + wave) * kChunk + g * 4) * s.v_pad + v0 + fr;
+#pragma unroll
+        for (int r = 0; r < 4; r++) dst[size_t(r) * s.v_pad] = sum[r];
+    };
+    uint32_t chunk0 = c_begin;
+    for (; chunk0 + kGroup <= c_end; chunk0 += kGroup) {
+#pragma unroll
+        for (uint32_t j = 0; j < kGroup; j++) step(j, chunk0 + j);
+        finish(chunk0, kGroup);
+    }
+    if (chunk0 < c_end) {
+#pragma unroll
+        for (uint32_t j = 0; j + 1 < kGroup; j++) {
+            if (chunk0 + j >= c_end) break;
+            step(j, chunk0 + j);
+        }
+        finish(chunk0, c_end - chunk0);
     }
     if (!STATE_ONLY && c_end != n_chunks) return;  // the last segment ends with the pass's state
     float *out = STATE_ONLY ? ws.seg_state + size_t(seg) * s.heads * head_state + at : a.state_out + at;
@@ -1052,7 +1073,7 @@ __global__ __launch_bounds__(256) void recur_scan_kernel(RmiRecurShape s, RmiRec
         if (tile >= n_tiles) continue;
 #pragma unroll
         for (int r = 0; r < 4; r++) out[size_t(tile * 16 + g * 4 + r) * s.v_pad] = st[i][r];
-        if (STATE_ONLY && blockIdx.x == 0 && fr == 0)
+        if (STATE_ONLY && v0 == 0 && fr == 0)
             *reinterpret_cast<f32x4 *>(ws.seg_decay + (size_t(seg) * s.heads + head) * s.d_pad + tile * 16 + g * 4) = kept[i];
     }
 }
@@ -1261,15 +1282,21 @@ int rmi_recur_pass(uint32_t elem_bytes, const RmiRecurShape &s, const RmiRecurAr
     const uint32_t seg_chunks = (n_chunks + segs - 1) / segs;
     segs = (n_chunks + seg_chunks - 1) / seg_chunks;
     auto scan = [&](auto state_only, auto whole) {
-        if (segs > 1) hipLaunchKernelGGL(state_only, dim3(s.v_pad / 16, s.heads, segs - 1), dim3(256), 0, st, s, a, n_chunks, seg_chunks);
-        hipLaunchKernelGGL(whole, dim3(s.v_pad / 16, s.heads, segs), dim3(256), 0, st, s, a, n_chunks, seg_chunks);
+        if (segs > 1) hipLaunchKernelGGL(state_only, dim3(s.heads, s.v_pad / 16, segs - 1), dim3(256), 0, st, s, a, n_chunks, seg_chunks);
+        hipLaunchKernelGGL(whole, dim3(s.heads, s.v_pad / 16, segs), dim3(256), 0, st, s, a, n_chunks, seg_chunks);
     };
-    if (s.d_pad <= 64)
-        scan(recur_scan_kernel<1, true>, recur_scan_kernel<1, false>);
-    else if (s.d_pad <= 128)
-        scan(recur_scan_kernel<2, true>, recur_scan_kernel<2, false>);
+    if (s.d_pad == 64)
+        scan(recur_scan_kernel<1, true, true>, recur_scan_kernel<1, false, true>);
+    else if (s.d_pad < 64)
+        scan(recur_scan_kernel<1, true, false>, recur_scan_kernel<1, false, false>);
+    else if (s.d_pad == 128)
+        scan(recur_scan_kernel<2, true, true>, recur_scan_kernel<2, false, true>);
+    else if (s.d_pad < 128)
+        scan(recur_scan_kernel<2, true, false>, recur_scan_kernel<2, false, false>);
+    else if (s.d_pad == 256)
+        scan(recur_scan_kernel<4, true, true>, recur_scan_kernel<4, false, true>);
     else
-        scan(recur_scan_kernel<4, true>, recur_scan_kernel<4, false>);
+        scan(recur_scan_kernel<4, true, false>, recur_scan_kernel<4, false, false>);
     const dim3 ngrid((a.n_tokens + 3) / 4, s.heads);
     if (elem_bytes == 2)
         hipLaunchKernelGGL(recur_norm_kernel<rmi_bf16>, ngrid, dim3(256), 0, st, s, a, n_chunks);

@@ -353,3 +353,16 @@ def test_command_line_generates(hip, tmp_path, capsys):
         s.close()
         assert cli.main(["--model", path, "--tokens", "5,17,3", "--max-new", "9", *args]) == 0
         assert [int(t) for t in capsys.readouterr().out.strip().split(",")] == want
+
+
+@pytest.mark.parametrize("rdim", [16, 48, 64, 80, 128, 144, 256])
+def test_recurrence_of_every_group_and_segment(open_model, rdim):
+    """Prompts of 1, 3, 4, 5, 8 chunks of sixteen tokens and of segments that end within a group of four chunks, at row tiles that
+    fill the four waves (64, 128, 256) and that don't; the last chunk whole, of one token, and with an odd rest."""
+    cfg = G.config([G.layer_config(rheads=9, rdim=rdim, rvdim=40)], width=40)
+    s, w = open_model(cfg, None, F32, 620)
+    t = G.tokens(cfg, 610)
+    ref = P.forward(cfg, w, t)
+    for sizes in ([16, 33], [48, 64], [65, 80], [127, 128, 129], [289, 300], [610]):
+        s.reset()
+        assert rel(feed(s, t, sizes), ref) < TOL[F32], sizes
