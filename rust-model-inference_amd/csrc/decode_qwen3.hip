@@ -1447,9 +1447,9 @@ int enqueue_prompt_pass(rmi_hip_qwen3 *s, uint32_t step0, uint32_t n, const uint
         rc = rmi_gemv_q8_0_tokens(s->head, s->act_q8b + size_t(i0) * c.n_embd, s->act_scalesb + size_t(i0) * (c.n_embd / 32), s->logitsb, nb,
                                   c.vocab, 0, c.vocab, st);
         if (rc != RMI_HIP_OK) return rc;
-        hipLaunchKernelGGL(argmax_partial_kernel, dim3(kArgmaxGroups, nb), dim3(256), 0, st, s->logitsb, c.vocab,
+        hipLaunchKernelGGL(argmax_partial_kernel, dim3(rmi_argmax_groups(nb), nb), dim3(256), 0, st, s->logitsb, c.vocab,
                            static_cast<Top *>(s->partialb));
-        hipLaunchKernelGGL(argmax_final_batch_kernel<EmbedQ8>, dim3(nb), dim3(256), 0, st, static_cast<const Top *>(s->partialb), kArgmaxGroups,
+        hipLaunchKernelGGL(argmax_final_batch_kernel<EmbedQ8>, dim3(nb), dim3(256), 0, st, static_cast<const Top *>(s->partialb), rmi_argmax_groups(nb),
                            sp, step0 + i0, static_cast<const uint32_t *>(nullptr), s->tok, s->step_argmax, s->step_top2, s->nonfinite,
                            EmbedQ8{s->embd->data, s->embd->n_units, c.vocab, s->x, c.n_embd});
         for (; w < n_want && want[w] < i0 + nb; w++) of(step0 + want[w], s->logitsb + size_t(want[w] - i0) * c.vocab);

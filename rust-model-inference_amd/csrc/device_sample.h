@@ -49,15 +49,24 @@ __global__ __launch_bounds__(256) void argmax_partial_kernel(const float *__rest
     logits += size_t(blockIdx.y) * n;  // token blockIdx.y of a launch over several: its logits, its partial results
     partial += size_t(blockIdx.y) * gridDim.x;
     Top t{-INFINITY, -INFINITY, 0xffffffffu, 1u};
-    for (uint32_t i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256) {
-        const float l = logits[i];
-        if (!(fabsf(l) <= 3.4028234663852886e38f)) t.finite = 0;  // NaN or inf
-        if (l > t.best) {
-            t.second = t.best;
-            t.best = l;
-            t.id = i;
-        } else if (l > t.second) {
-            t.second = l;
+    constexpr uint32_t kAtOnce = 4;  // loads under way
+    const uint32_t stride = gridDim.x * 256;
+    for (uint32_t i0 = blockIdx.x * 256 + threadIdx.x; i0 < n; i0 += kAtOnce * stride) {
+        float l[kAtOnce];
+#pragma unroll
+        for (uint32_t j = 0; j < kAtOnce; j++) l[j] = logits[i0 + j * stride < n ? i0 + j * stride : i0];
+#pragma unroll
+        for (uint32_t j = 0; j < kAtOnce; j++) {
+            const uint32_t i = i0 + j * stride;
+            if (i >= n) break;
+            if (!(fabsf(l[j]) <= 3.4028234663852886e38f)) t.finite = 0;  // NaN or inf
+            if (l[j] > t.best) {
+                t.second = t.best;
+                t.best = l[j];
+                t.id = i;
+            } else if (l[j] > t.second) {
+                t.second = l[j];
+            }
         }
     }
     const Top r = top_block_reduce(t, sm);

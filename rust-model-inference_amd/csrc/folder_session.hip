@@ -54,10 +54,10 @@ int rmi_hip_folder_session::enqueue_logits(const uint32_t *rows, uint32_t n_rows
 
 // last: the place of the pass's last sampled position, whose token's embedding is left for the next step
 int rmi_hip_folder_session::enqueue_sample(uint32_t step0, const uint32_t *rows, uint32_t n_rows, uint32_t last, hipStream_t st) {
-    hipLaunchKernelGGL(argmax_partial_kernel, dim3(kArgmaxGroups, n_rows), dim3(256), 0, st, logits, vocab, static_cast<Top *>(partial));
+    hipLaunchKernelGGL(argmax_partial_kernel, dim3(rmi_argmax_groups(n_rows), n_rows), dim3(256), 0, st, logits, vocab, static_cast<Top *>(partial));
     auto finish = [&](auto embed_next) {
         hipLaunchKernelGGL((argmax_final_batch_kernel<decltype(embed_next)>), dim3(n_rows), dim3(256), 0, st,
-                           static_cast<const Top *>(partial), kArgmaxGroups, static_cast<StepParams *>(params), step0, rows, tok, step_argmax,
+                           static_cast<const Top *>(partial), rmi_argmax_groups(n_rows), static_cast<StepParams *>(params), step0, rows, tok, step_argmax,
                            step_top2, nonfinite, embed_next);
     };
     if (elem == 2)

@@ -9,6 +9,13 @@
 #include "rmi_internal.h"
 
 constexpr uint32_t kArgmaxGroups = 256;
+// Workgroups that share a position's logits: all of them for a few positions; for many, sixteen a compute unit in all, so that
+// a thread has more to read than its workgroup's reduction takes (128 positions of 151936: 45.8 us with 256 a position, 16.5
+// with 32 and four loads a thread under way).
+inline uint32_t rmi_argmax_groups(uint32_t positions) {
+    const uint32_t n = 4096 / (positions ? positions : 1);
+    return n >= kArgmaxGroups ? kArgmaxGroups : n < 1 ? 1 : n;
+}
 constexpr size_t kTopBytes = 16;  // one Top of device_sample.h
 
 // Called while a pass is enqueued, with a position and where its logits lie at that point of the stream.
