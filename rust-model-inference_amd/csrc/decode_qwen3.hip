@@ -146,8 +146,10 @@ void launch_add_rmsnorm_quant(float *x, const float *r, const float *weight, uin
         hipLaunchKernelGGL(add_rmsnorm_quant_kernel<16>, dim3(n_tok), dim3(256), 0, st, x, r, weight, n, eps, q8, scales, rounding, ts);
 }
 
-// Per head of the stacked q|k|v vector: q/k RMS norm, NeoX rotation, f16 rounding; k and v go to the cache row.
-__global__ __launch_bounds__(64) void qk_norm_rope_store_kernel(const float *__restrict__ qkv,
+// Per head of the stacked q|k|v vector: q/k RMS norm, NeoX rotation, f16 rounding; k and v go to the cache row.  A wave a head
+// and token; up to four tokens a workgroup (1024 tokens of 32 heads: 9.0 us with a workgroup a wave, 7.6 with four).
+constexpr uint32_t kRopeTokens = 4;
+__global__ __launch_bounds__(64 * kRopeTokens) void qk_norm_rope_store_kernel(const float *__restrict__ qkv,
                                                                 const float *__restrict__ q_norm,
                                                                 const float *__restrict__ k_norm,
                                                                 const float *__restrict__ cos_t,
@@ -155,14 +157,16 @@ __global__ __launch_bounds__(64) void qk_norm_rope_store_kernel(const float *__r
                                                                 uint16_t *__restrict__ q16, uint16_t *__restrict__ k_row,
                                                                 uint16_t *__restrict__ v_row, uint32_t n_head,
                                                                 uint32_t n_head_kv, uint32_t hk, uint32_t hv, float eps,
-                                                                TokStride3 tok_stride) {
+                                                                TokStride3 tok_stride, uint32_t n_tok) {
     const uint32_t head = blockIdx.x, tid = threadIdx.x;
-    // token blockIdx.y of a launch over several: the next position, its qkv, q16 and cache rows tok_stride apart
-    qkv += size_t(blockIdx.y) * tok_stride.x;
-    q16 += size_t(blockIdx.y) * tok_stride.y;
-    k_row += size_t(blockIdx.y) * tok_stride.z;
-    v_row += size_t(blockIdx.y) * tok_stride.z;
-    pos += blockIdx.y;
+    // a token of a launch over several: the next position, its qkv, q16 and cache rows tok_stride apart
+    const uint32_t t = blockIdx.y * blockDim.y + uint32_t(__builtin_amdgcn_readfirstlane(int(threadIdx.y)));
+    if (t >= n_tok) return;  // (a wave's own token: nothing meets behind this)
+    qkv += size_t(t) * tok_stride.x;
+    q16 += size_t(t) * tok_stride.y;
+    k_row += size_t(t) * tok_stride.z;
+    v_row += size_t(t) * tok_stride.z;
+    pos += t;
     if (head >= n_head + n_head_kv) {  // v: rounding only
         const uint32_t kvh = head - n_head - n_head_kv;
         const float *src = qkv + size_t(n_head) * hk + size_t(n_head_kv) * hk + size_t(kvh) * hv;
@@ -1333,7 +1337,7 @@ int enqueue_step(rmi_hip_qwen3 *s, uint32_t step, hipStream_t st) {
             if (rc != RMI_HIP_OK) return rc;
             hipLaunchKernelGGL(qk_norm_rope_store_kernel, dim3(c.n_head + 2 * c.n_head_kv), dim3(64), 0, st, s->qkv, qn, kn,
                                s->cos_t, s->sin_t, step, s->q16, s->k_cache + row, s->v_cache + row, c.n_head,
-                               c.n_head_kv, c.head_dim_k, c.head_dim_v, c.eps, TokStride3{0, 0, 0});
+                               c.n_head_kv, c.head_dim_k, c.head_dim_v, c.eps, TokStride3{0, 0, 0}, 1u);
         }
         if (qkv_in_attention) {
             // done above
@@ -1416,9 +1420,9 @@ int enqueue_prompt_pass(rmi_hip_qwen3 *s, uint32_t step0, uint32_t n, const uint
                                  TokStride3{c.n_embd, pending_stride, c.n_embd});
         rc = rmi_gemv_q8_0_tokens(s->w_qkv[l], s->act_q8b, s->act_scalesb, s->qkvb, n, n_qkv, 0, n_qkv, st);
         if (rc != RMI_HIP_OK) return rc;
-        hipLaunchKernelGGL(qk_norm_rope_store_kernel, dim3(c.n_head + 2 * c.n_head_kv, n), dim3(64), 0, st, s->qkvb, qn, kn,
+        hipLaunchKernelGGL(qk_norm_rope_store_kernel, dim3(c.n_head + 2 * c.n_head_kv, (n + kRopeTokens - 1) / kRopeTokens), dim3(64, kRopeTokens), 0, st, s->qkvb, qn, kn,
                            s->cos_t, s->sin_t, step0, s->q16b, s->k_cache + row, s->v_cache + row, c.n_head, c.n_head_kv,
-                           c.head_dim_k, c.head_dim_v, c.eps, TokStride3{n_qkv, s->n_q, s->kv_stride});
+                           c.head_dim_k, c.head_dim_v, c.eps, TokStride3{n_qkv, s->n_q, s->kv_stride}, n);
         if (pass_by_positions(c, step0, n))
             hipLaunchKernelGGL((attention128_quant_kernel<false, 1, true>), dim3(c.n_head / c.n_head_kv, c.n_head_kv, n), dim3(kA128Threads),
                                attn128_lds_bytes(step0 + n), st, s->q16b, s->k_cache + layer_base, s->v_cache + layer_base, step0, s->kv_stride,
@@ -1555,7 +1559,7 @@ int rmi_hip_qk_norm_rope_f16_dev(const float *qkv, const float *q_norm, const fl
     if (n_head == 0 || n_head_kv == 0 || head_dim_k % 2) return rmi_fail(RMI_HIP_E_INVALID, "bad head shape");
     hipLaunchKernelGGL(qk_norm_rope_store_kernel, dim3(n_head + 2 * n_head_kv), dim3(64), 0,
                        static_cast<hipStream_t>(stream), qkv, q_norm, k_norm, cos_row, sin_row, 0u, q16, k_row, v_row,
-                       n_head, n_head_kv, head_dim_k, head_dim_v, eps, TokStride3{0, 0, 0});
+                       n_head, n_head_kv, head_dim_k, head_dim_v, eps, TokStride3{0, 0, 0}, 1u);
     RMI_HIP_CHECK(hipGetLastError());
     return RMI_HIP_OK;
 }
