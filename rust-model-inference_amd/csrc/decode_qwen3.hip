@@ -22,6 +22,7 @@
 // and that flips the f32 rounding of the mean (about 2^-29 per norm).  A rounded
 // int8 quant that flips would move logits by 1e-2, so the step is held to
 // bit-identical logits against the CPU path, not to a tolerance.
+#include <algorithm>
 #include <cmath>
 #include <utility>
 #include <vector>
@@ -1791,7 +1792,8 @@ rmi_hip_qwen3 *rmi_hip_qwen3_create(const rmi_hip_qwen3_config *cfg, const rmi_h
              (s->logitsb = dev_alloc<float>(s, head * c.vocab)) &&
              (s->act_q8b = dev_alloc<int8_t>(s, n * s->max_n_in)) && (s->act_scalesb = dev_alloc<float>(s, n * s->max_n_in / 32)) &&
              (s->partialb = dev_alloc<Top>(s, head * kArgmaxGroups)) && (s->attn_scratch = dev_alloc<float>(s, s->attn_scratch_floats));
-        if (const size_t bytes = rmi_attn_limbs_bytes(c.n_head_kv, c.capacity)) {
+        const bool any = std::find(s->limbs_hold.begin(), s->limbs_hold.end(), true) != s->limbs_hold.end();
+        if (const size_t bytes = any ? rmi_attn_limbs_bytes(c.n_head_kv, c.capacity) : 0) {
             void *p = ok ? dev_alloc<uint8_t>(s, bytes) : nullptr;
             ok = p != nullptr;
             s->attn_limbs = rmi_attn_limbs_at(p, c.n_head_kv, c.capacity);
