@@ -57,13 +57,12 @@ struct RmiColSeg {
     uint32_t gate_ld;
     float scale;
     uint32_t k_end;
-    float carry;  // products of several tokens, set by their launch: 0 = none, else what the sums are times in the next one's scale
 };
 constexpr uint32_t kMaxColSegs = 4;
 struct RmiColSegs {
     RmiColSeg s[kMaxColSegs];
     uint32_t n_segs;
-    uint32_t k_begin;  // of the first segment, set by the launches that take some of a product's
+    uint32_t k_begin;  // of the first segment, set by the launches that take one of a product's
 };
 
 struct RmiDense {

@@ -59,20 +59,6 @@ __device__ __forceinline__ void fold_segment(f32x4 (&acc)[NN][NT], const RmiColS
     }
 }
 
-// A segment's end: its results join x, or go on as part of the next one's.
-template <int NN, int NT>
-__device__ __forceinline__ void end_segment(f32x4 (&acc)[NN][NT], const RmiColSeg &s, float *__restrict__ x, uint32_t width, uint32_t n_tokens,
-                                            uint32_t row0, uint32_t tok0) {
-    if (s.carry == 0.0f) {
-        fold_segment<NN, NT>(acc, s, x, width, n_tokens, row0, tok0);
-    } else {
-#pragma unroll
-        for (int i = 0; i < NN; i++)
-#pragma unroll
-            for (int j = 0; j < NT; j++) acc[i][j] = acc[i][j] * s.carry;
-    }
-}
-
 // first_row, tok0: of the wave's first tile and the lane's first token
 template <typename T, int EPI, int NN, int NT>
 __device__ __forceinline__ void store_rows(const f32x4 (&acc)[NN][NT], const RmiRowSegs &rs, uint32_t n_rows, uint32_t n_tokens, uint32_t first_row,
@@ -388,7 +374,7 @@ __global__ __launch_bounds__(256, WPS) void dense_gemm_kernel(const T *__restric
                 __syncthreads();
             }
         }
-        if constexpr (RESIDUAL) end_segment<NN, NT>(acc, cs.s[seg], x, width, n_tokens, row0 + wn + g * 4, tok0 + wt + fr);
+        if constexpr (RESIDUAL) fold_segment<NN, NT>(acc, cs.s[seg], x, width, n_tokens, row0 + wn + g * 4, tok0 + wt + fr);
     }
 
     if constexpr (!RESIDUAL) store_rows<T, EPI, NN, NT>(acc, rs, n_rows, n_tokens, row0 + wn, tok0 + wt + fr, g);
@@ -438,7 +424,7 @@ __global__ __launch_bounds__(64 * (BN / WN) * (BT / WT), WPS) void dense_gemm_wi
         a_off[i] = (tok0 + r < n_tokens ? r : n_tokens - 1 - tok0) * stride + piece;
     }
     constexpr uint32_t kStepElems = kStepBytes / sizeof(T);
-    const uint32_t first = RESIDUAL ? cs.k_begin / kStepElems : 0, n_steps = (RESIDUAL ? cs.s[cs.n_segs - 1].k_end : k_pad) / kStepElems;
+    const uint32_t first = RESIDUAL ? cs.k_begin / kStepElems : 0, n_steps = (RESIDUAL ? cs.s[0].k_end : k_pad) / kStepElems;
     auto fetch = [&](u32x4 *buf, uint32_t step) {
         const uint32_t at = (step < n_steps ? step : n_steps - 1) * kStepBytes;  // (behind the last step: that one again, read by nobody)
 #pragma unroll
@@ -488,15 +474,7 @@ __global__ __launch_bounds__(64 * (BN / WN) * (BT / WT), WPS) void dense_gemm_wi
         __builtin_amdgcn_sched_group_barrier(0x008, kProducts, 0);
         __builtin_amdgcn_sched_barrier(0);
     };
-    uint32_t seg = 0, seg_end = RESIDUAL ? cs.s[0].k_end / kStepElems : n_steps;
     auto step_of = [&](u32x4 *cur, u32x4 *next, uint32_t step) {
-        if (RESIDUAL && step == seg_end) {  // on into the next segment, in its scale
-#pragma unroll
-            for (int i = 0; i < NN; i++)
-#pragma unroll
-                for (int j = 0; j < NT; j++) acc[i][j] = acc[i][j] * cs.s[seg].carry;
-            seg_end = cs.s[++seg].k_end / kStepElems;
-        }
         read(cur, 1);
         multiply(0);
         spread(0);
@@ -520,7 +498,7 @@ __global__ __launch_bounds__(64 * (BN / WN) * (BT / WT), WPS) void dense_gemm_wi
     read(buf0, 0);
     // Whole turns of the buffers in a loop that has no other way out: with one, the compiler takes it that a buffer may be read
     // right behind its fetch, and waits for every load in flight once a turn (128 x 256, residual 4096 x 20480, 2048 tokens: 367 us with that and the
-    // results joining x from the registers, segments in the loop; 312 without, a launch for each gate).
+    // results joining x from the registers, segments in the loop; 312 without, in two launches).
     uint32_t step = first;
     auto buffer = [&](int i) { return i % NB == 0 ? buf0 : i % NB == 1 ? buf1 : buf2; };
     for (; step + NB <= n_steps; step += NB) {
@@ -531,19 +509,19 @@ __global__ __launch_bounds__(64 * (BN / WN) * (BT / WT), WPS) void dense_gemm_wi
     if (NB == 3 && step + 1 < n_steps) step_of(buffer(1), buffer(2), step + 1);
 
     if (RESIDUAL && (width & 3)) {
-        fold_segment<NN, NT>(acc, cs.s[cs.n_segs - 1], x, width, n_tokens, row0 + wn + g * 4, tok0 + wt + fr);
+        fold_segment<NN, NT>(acc, cs.s[0], x, width, n_tokens, row0 + wn + g * 4, tok0 + wt + fr);
         return;
     }
     __builtin_amdgcn_s_waitcnt(rmi_waitcnt(0));  // the steps behind the end are in LDS, and everybody has read the last one
     ResidualLines<WN, NT> there;
-    if constexpr (RESIDUAL) there.load(cs.s[cs.n_segs - 1], x, width, n_tokens, row0 + wn, tok0 + wt);
+    if constexpr (RESIDUAL) there.load(cs.s[0], x, width, n_tokens, row0 + wn, tok0 + wt);
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
     constexpr uint32_t kTile = 16 * (WN + 4) / 4;  // in pieces; half of the waves' in either buffer
     static_assert(WAVES / 2 * kTile <= (BN + BT) * 8, "the waves' tiles fit the buffers");
     float *tile = reinterpret_cast<float *>((wave < WAVES / 2 ? buf0 : buf1) + wave % (WAVES / 2) * kTile);
     if constexpr (RESIDUAL)
-        there.template add<NN>(acc, cs.s[cs.n_segs - 1], x, width, n_tokens, row0 + wn, tok0 + wt, tile);
+        there.template add<NN>(acc, cs.s[0], x, width, n_tokens, row0 + wn, tok0 + wt, tile);
     else
         store_lines<T, EPI, WN, NN, NT>(acc, rs, n_tokens, row0 + wn, tok0 + wt, tile);
 }
@@ -618,16 +596,16 @@ int launch_gemm(const RmiDense &w, const void *a, const RmiRowSegs &rs, const Rm
                            w.k_pad, w.ld, n_tokens, gn, gt, split, rs, c, x, width);
     };
     auto go = [&](auto kernel) { launch(kernel, cs); };
-    auto go_wide = [&](auto kernel) {  // a launch for every run of segments whose sums go on into the next
+    auto go_wide = [&](auto kernel) {  // a launch for every column segment
         if constexpr (EPI != kResidual) {
             launch(kernel, cs);
         } else {
-            for (uint32_t i = 0; i < cs.n_segs;) {
-                RmiColSegs run{};
-                run.k_begin = i ? cs.s[i - 1].k_end : 0;
-                do run.s[run.n_segs++] = cs.s[i];
-                while (cs.s[i++].carry != 0.0f);
-                launch(kernel, run);
+            for (uint32_t i = 0; i < cs.n_segs; i++) {
+                RmiColSegs one{};
+                one.s[0] = cs.s[i];
+                one.n_segs = 1;
+                one.k_begin = i ? cs.s[i - 1].k_end : 0;
+                launch(kernel, one);
             }
         }
     };
@@ -705,16 +683,6 @@ int rmi_dense_gemm_residual(uint32_t elem_bytes, const RmiDense &w, const void *
     if (n_tokens == 0) return RMI_HIP_OK;
     const int rc = rmi_check_col_segs(elem_bytes, w, segs, width);
     if (rc != RMI_HIP_OK) return rc;
-    // A segment that ends reads and writes all of x and reads its gate; where the next one has the same gate, its sums go on
-    // from these instead, in the next one's scale (4096 x 20480, 2048 tokens, three segments of two gates: 384 -> 367 us).
-    RmiColSegs carried = segs;
-    carried.s[segs.n_segs - 1].carry = 0.0f;
-    for (uint32_t i = 0; i + 1 < segs.n_segs; i++) {
-        const RmiColSeg &s0 = segs.s[i], &s1 = segs.s[i + 1];
-        const float ratio = s1.scale != 0.0f ? s0.scale / s1.scale : 0.0f;
-        const bool same = s0.gate == s1.gate && (!s0.gate || s0.gate_ld == s1.gate_ld);
-        carried.s[i].carry = same && fabsf(ratio) >= 0x1p-10f && fabsf(ratio) <= 0x1p10f ? ratio : 0.0f;
-    }
-    return elem_bytes == 2 ? launch_gemm<rmi_bf16, kResidual>(w, a, RmiRowSegs{}, carried, x, width, n_tokens, st)
-                           : launch_gemm<float, kResidual>(w, a, RmiRowSegs{}, carried, x, width, n_tokens, st);
+    return elem_bytes == 2 ? launch_gemm<rmi_bf16, kResidual>(w, a, RmiRowSegs{}, segs, x, width, n_tokens, st)
+                           : launch_gemm<float, kResidual>(w, a, RmiRowSegs{}, segs, x, width, n_tokens, st);
 }

@@ -262,8 +262,8 @@ def test_every_tile(hip, tile, kind, size):
 
 @pytest.mark.parametrize("elem,rows,tokens", [(2, 6800, 909), (2, 4832, 205), (2, 17296, 205), (2, 4100, 1025), (2, 1002, 130), (2, 80, 45), (4, 12576, 109), (4, 28576, 205)])
 def test_residual_segments_of_one_gate(hip, elem, rows, tokens):
-    """Segments that share a gate in scales of their own go on from each other's sums; one with another gate, or a scale of zero
-    behind it, ends them.  Four segments of 4, 8, 4 and 8 steps of bf16: ends at every place of the buffers' turn."""
+    """Segments that share a gate in scales of their own, one of them zero.  Four segments of 4, 8, 4 and 8 steps of bf16: ends at
+    every place of the buffers' turn."""
     H = hip.hip
     ends, gates = (256, 768, 1024, 1536), (0, 0, 1, 1)
     for scales in ((1.0, 0.75, 0.5, 1.5), (1.0, 0.75, 0.5, 0.0)):
@@ -288,6 +288,47 @@ def test_residual_segments_of_one_gate(hip, elem, rows, tokens):
         got = bufs[2].to_array(np.float32, (tokens, rows))
         # sums of k products as above, and a few roundings of what they are part of
         assert (np.abs(got - want) <= 2 * ends[-1] * 2.0**-24 * size + 2.0**-21 * (np.abs(x) + np.abs(want))).all()
+
+
+@pytest.mark.parametrize("elem,rows,tokens", [(2, 6800, 909), (2, 4832, 205), (2, 17296, 205), (2, 22544, 299), (2, 1002, 130), (2, 80, 45), (4, 12576, 109), (4, 28576, 205)])
+@pytest.mark.parametrize("size,scales", [(0, (0.7, 1.3, 0.6)), (115, (1.0, 2.0**-10, 1.0))])
+def test_segments_join_one_after_the_other(hip, elem, rows, tokens, size, scales):
+    """Each segment's sums are scaled, gated and rounded by themselves, whatever the next one's gate: the bits of a product for
+    each.  Sums near 2^119 stay finite in front of a segment of a smaller scale."""
+    H = hip.hip
+    ends, gate_of = (256, 768, 1024), (0, 0, 1)
+    rng = np.random.default_rng(rows + size)
+    padded = (rows + 15) // 16 * 16
+    _, wv, _ = _operand(rng, padded, ends[-1], elem)
+    _, av, _ = _operand(rng, tokens, ends[-1], elem)
+    av = av * np.float32(2.0**size)  # (exact)
+    x = rng.standard_normal((tokens, rows), dtype=np.float32)
+    gates = [H.DeviceBuffer.from_array(rng.uniform(0, 1, (tokens, rows)).astype(np.float32)) for _ in range(2)]
+
+    def operand(v):
+        k = v.shape[1]
+        a = np.zeros((v.shape[0], k + (128 // elem if k * elem % 256 == 0 else 0)), np.float32)
+        a[:, :k] = v
+        return H.DeviceBuffer.from_array(a if elem == 4 else (a.view(np.uint32) >> 16).astype(np.uint16)), a.shape[1]
+
+    def add(d_x, first, segments):
+        k = ends[segments[-1]] - first
+        (d_w, ld), (d_a, _) = operand(wv[:, first:first + k]), operand(av[:, first:first + k])
+        segs = ColSegs()
+        for i, j in enumerate(segments):
+            segs.s[i] = ColSeg(gates[gate_of[j]].ptr, rows, scales[j], ends[j] - first)
+        segs.n_segs = len(segments)
+        assert getattr(H.lib, RESIDUAL)(C.c_uint32(elem), C.byref(Dense(d_w.ptr, padded, k, ld)), C.c_void_p(d_a.ptr), C.byref(segs),
+                                        C.c_void_p(d_x.ptr), C.c_uint32(rows), C.c_uint32(tokens), None) == 0
+        H.check(H.lib.rmi_hip_synchronize())
+
+    together, apart = H.DeviceBuffer.from_array(x), H.DeviceBuffer.from_array(x)
+    add(together, 0, [0, 1, 2])
+    for j, first in enumerate((0, *ends[:-1])):
+        add(apart, first, [j])
+    got = together.to_array(np.float32, (tokens, rows))
+    assert np.isfinite(got).all()
+    assert np.array_equal(got.view(np.uint32), apart.to_array(np.uint32, (tokens, rows)))
 
 
 @pytest.mark.parametrize("elem,last,k,tokens", [(2, 12704, 2048, 909), (2, 6800, 2048, 909), (2, 4832, 512, 205), (2, 17296, 512, 205), (4, 12576, 512, 109)])
