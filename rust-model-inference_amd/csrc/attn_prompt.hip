@@ -679,16 +679,11 @@ __global__ __launch_bounds__(kThreads, 2) void attn128_prompt_kernel(PromptArgs 
 // limbs, 16 heads: prompt of 128 99 | 103, 256 139 | 140, 384 184 | 182, 700 299 | 277, 1024 394 | 349; 2048 tokens in passes
 // of 65 141 | 132, of 512 265 | 228, of 1024 476 | 380; 32 heads: prompt of 192 581 | 584, 256 691 | 690, 512 1215 | 1193, 1024
 // 2428 | 2336.  Values that don't fit, 16 heads: prompt of 512 212 | 243, 1024 399 | 417, 2048 tokens in passes of 1024 488 | 489.
-bool limbs_pay(uint32_t n_head, uint32_t step0, uint32_t n_tok, bool limbs_hold) {
-    return limbs_hold && uint64_t(n_head) * n_tok * (step0 + n_tok / 2) >= 1u << 20;
-}
+bool limbs_pay(uint32_t n_head, uint32_t step0, uint32_t n_tok) { return uint64_t(n_head) * n_tok * (step0 + n_tok / 2) >= 1u << 20; }
 
 }  // namespace
 
-size_t rmi_attn_limbs_bytes(uint32_t n_head_kv, uint32_t capacity) {
-    const size_t blocks = (capacity + 63) / 64;
-    return capacity > kAttnLimbKeys ? 0 : blocks * n_head_kv * 2 * (kLimbBlock + 4);
-}
+size_t rmi_attn_limbs_bytes(uint32_t n_head_kv, uint32_t capacity) { return size_t((capacity + 63) / 64) * n_head_kv * 2 * (kLimbBlock + 4); }
 RmiAttnLimbs rmi_attn_limbs_at(void *base, uint32_t n_head_kv, uint32_t capacity) {
     if (!base) return RmiAttnLimbs{};
     const uint32_t blocks = (capacity + 63) / 64;
@@ -697,11 +692,14 @@ RmiAttnLimbs rmi_attn_limbs_at(void *base, uint32_t n_head_kv, uint32_t capacity
     return RmiAttnLimbs{p, p + plane, reinterpret_cast<uint32_t *>(p + 2 * plane), blocks};
 }
 
+bool rmi_attn_prompt_in_limbs(uint32_t n_head, uint32_t step0, uint32_t n_tok, const RmiAttnLimbs &limbs, bool limbs_hold) {
+    return limbs.blocks && limbs_hold && step0 + n_tok <= kAttnLimbKeys && limbs_pay(n_head, step0, n_tok);
+}
 int rmi_launch_attn128_prompt(const uint16_t *q16, const uint16_t *k_cache, const uint16_t *v_cache, uint32_t step0, uint32_t n_tok,
                               uint32_t kv_stride, uint32_t n_head, uint32_t n_head_kv, float *scratch, size_t scratch_floats,
                               const RmiAttnLimbs &limbs, bool limbs_hold, int8_t *q8, float *scales, int rounding, hipStream_t st) {
     const uint32_t cus = uint32_t(rmi_device_cus()), stride = rmi_attn_prompt_score_stride(step0 + n_tok);
-    const bool use_limbs = limbs.blocks && limbs_pay(n_head, step0, n_tok, limbs_hold);
+    const bool use_limbs = rmi_attn_prompt_in_limbs(n_head, step0, n_tok, limbs, limbs_hold);
     const uint32_t rows = use_limbs ? kRows : 16, tiles = (n_tok + rows - 1) / rows;
     const size_t tile_floats = size_t(n_head) * rows * stride;
     const uint32_t most = uint32_t(scratch_floats / tile_floats);  // tiles a launch has scratch for

@@ -1793,8 +1793,8 @@ rmi_hip_qwen3 *rmi_hip_qwen3_create(const rmi_hip_qwen3_config *cfg, const rmi_h
              (s->act_q8b = dev_alloc<int8_t>(s, n * s->max_n_in)) && (s->act_scalesb = dev_alloc<float>(s, n * s->max_n_in / 32)) &&
              (s->partialb = dev_alloc<Top>(s, head * kArgmaxGroups)) && (s->attn_scratch = dev_alloc<float>(s, s->attn_scratch_floats));
         const bool any = std::find(s->limbs_hold.begin(), s->limbs_hold.end(), true) != s->limbs_hold.end();
-        if (const size_t bytes = any ? rmi_attn_limbs_bytes(c.n_head_kv, c.capacity) : 0) {
-            void *p = ok ? dev_alloc<uint8_t>(s, bytes) : nullptr;
+        if (any) {
+            void *p = ok ? dev_alloc<uint8_t>(s, rmi_attn_limbs_bytes(c.n_head_kv, c.capacity)) : nullptr;
             ok = p != nullptr;
             s->attn_limbs = rmi_attn_limbs_at(p, c.n_head_kv, c.capacity);
         }

@@ -52,8 +52,9 @@ def test_logits_of_every_position_of_a_pass(hip, tmp_path, n_prompt):
     (64, 8, 95, True), (32, 8, 130, True), (64, 8, 181, True), (64, 8, 224, True), (64, 8, 225, True), (32, 8, 257, True), (8, 2, 600, True), (64, 8, 330, 161)])
 @pytest.mark.parametrize("q,k,v", [(10.0, 10.0, 1.0), (40.0, 1.0, 1.0), (1.0, 1.0, 150.0), (10.0, 5.0, 400.0), (1e-5, 0.3, 1e-6)])
 def test_values_at_the_edge_of_what_limbs_hold(hip, tmp_path, heads, kv_heads, n_prompt, per_pass, q, k, v):
-    """Queries, keys and values times q, k, v: below 127 they go as four int8 limbs, a head that holds others in f64; large
-    scores make weights of one and a half (a fourth limb), small factors subnormal f16 values."""
+    """Queries, keys and values times q, k, v: large scores make weights of one and of a half (a fourth limb), small factors
+    subnormal f16 values; values from 127 on put their head in f64, norms from 11.2 on (40) the whole layer.  The bits are the
+    same in every form; test_gpu_attn_prompt.py says which pass takes which, and has queries and keys at the edge."""
     path = os.path.join(str(tmp_path), "m.gguf")
     hip.gguf.write_synthetic_qwen3(path, seed=heads, n_layer=2, n_embd=256, n_head=heads, n_head_kv=kv_heads, head_dim=128, n_ff=256, vocab=500, n_ctx=4096)
     f = hip.gguf.GGUFFile(path)
