@@ -16,8 +16,8 @@
 // once where it leaves them for f64.  Sixteen int8 products take a quarter of the matrix cores' time of one in f64, and the
 // weights of a block are twelve unless one of them is above 0.498.  Keys and values are split once a pass and layer, by
 // attn128_limbs_kernel, which lays them out as the matrix cores take them; queries and weights by the workgroup that uses
-// them.  A workgroup whose head has other keys or values (from 127 on, infinite, NaN), or which has such queries, does its
-// positions in f64.
+// them.  Where a head has other keys or values (from 127 on, infinite, NaN), or a tile such queries, the tile's positions are
+// done in f64.
 //
 // Phases of a workgroup:
 //   1  scores of sixteen keys a wave and turn into a row of scratch a position, and each position's maximum;
@@ -546,49 +546,18 @@ __device__ __forceinline__ void limb_values(const PromptArgs &a, PromptLds<kRows
                 l.out[rt * 16 + 4 * g + i][wave * 32 + dt * 16 + c16] = float(__builtin_fma(hi, 0x1p24, lo) * 0x1p-48);
             }
 }
-template <uint32_t ROWS>
-__global__ __launch_bounds__(kThreads, 2) void attn128_prompt_kernel(PromptArgs a) {
-    __shared__ PromptLds<ROWS> l;
+// A tile of a head's positions from t0 on, in limbs (the queries' are in LDS) or in f64
+template <uint32_t ROWS, bool LIMBS>
+__device__ __forceinline__ void prompt_tile(const PromptArgs &a, PromptLds<ROWS> &l, uint32_t head, uint32_t kvh, uint32_t rank, uint32_t t0, float *s_row0) {
     const uint32_t tid = threadIdx.x, lane = tid & 63, wave = uint32_t(__builtin_amdgcn_readfirstlane(int(tid >> 6)));
-    const uint32_t c16 = lane & 15, g = lane >> 4;
-    // key/value head fastest: with eight of them every workgroup that reads a head's limbs is on one XCD
-    const uint32_t kvh = blockIdx.x % a.n_head_kv, hpk = a.n_head / a.n_head_kv;
-    const uint32_t head = kvh * hpk + (blockIdx.x / a.n_head_kv) % hpk;
-    const uint32_t rank = blockIdx.x / a.n_head, tile = a.first_tile + prompt_tile_of(rank, a.n_tiles, a.half_tiles);
-    const uint32_t t0 = tile * ROWS;                                    // first position of the tile, within the pass
     const uint32_t rows = a.n_tok - t0 < ROWS ? a.n_tok - t0 : ROWS;
-    const uint32_t n_keys = a.step0 + t0 + rows;                         // of the tile's last position
-    const uint32_t n_blocks = (n_keys + 63) / 64;
-    float *s_row0 = a.scratch + size_t(blockIdx.x) * ROWS * a.score_stride;  // [position][key], rows of whole turns
-    const uint64_t tab_entry = kRmiExp2fTab[tid & 31];
-
-    // ---- the queries' limbs.  Wave w: positions 16 (w / 2) .. + 15, half w % 2 of the dimensions, lane (c16, g) sixteen of
-    // them of position c16
-    bool wide = ROWS != kRows;
-    if constexpr (ROWS == kRows) {
-        const uint32_t r = (wave >> 1) * 16 + c16, t = t0 + (r < rows ? r : rows - 1);
-        const u32x4 *src = reinterpret_cast<const u32x4 *>(a.q16 + (size_t(t) * a.n_head + head) * 128 + (wave & 1) * 64 + g * 16);
-        const u32x4 u[2] = {src[0], src[1]};
-        for (uint32_t b = tid; b < n_blocks; b += kThreads)
-            wide |= (a.limbs.wide[kvh * a.limbs.blocks + b] | a.limbs.wide[(a.n_head_kv + kvh) * a.limbs.blocks + b]) != 0;
-        _Float16 h[16];
-#pragma unroll
-        for (int j = 0; j < 16; j++) h[j] = __builtin_bit_cast(f16x8, u[j >> 3])[j & 7];
-#pragma unroll
-        for (int j = 0; j < 2; j++)
-#pragma unroll
-            for (int k = 0; k < 4; k++) wide |= !limbs_hold(u[j][k]);
-        u32x4 ql[4];
-        limbs_of16(h, ql);
-#pragma unroll
-        for (int j = 0; j < 4; j++) l.q[wave][j][lane] = ql[j];
-        wide = __syncthreads_or(wide);
-    }
+    const uint32_t n_keys = a.step0 + t0 + rows;  // of the tile's last position
     // ---- 1
-    if (wide)
-        wide_scores<ROWS>(a, l, head, kvh, t0, rows, s_row0);
-    else if constexpr (ROWS == kRows)
+    const uint64_t tab_entry = kRmiExp2fTab[tid & 31];
+    if constexpr (LIMBS)
         limb_scores(a, l, kvh, t0, rows, s_row0);
+    else
+        wide_scores<ROWS>(a, l, head, kvh, t0, rows, s_row0);
     if (tid < 32) l.exp_tab[tid] = tab_entry;
     __syncthreads();
 
@@ -617,7 +586,7 @@ __global__ __launch_bounds__(kThreads, 2) void attn128_prompt_kernel(PromptArgs 
                     next[j] = at(ahead, j);
                     const float x[4] = {sc.x - max_val, sc.y - max_val, sc.z - max_val, sc.w - max_val};
                     float4 e;
-                    if (wide)
+                    if constexpr (!LIMBS)
                         e = {rmi_expf_tab(x[0], l.exp_tab), rmi_expf_tab(x[1], l.exp_tab), rmi_expf_tab(x[2], l.exp_tab), rmi_expf_tab(x[3], l.exp_tab)};
                     else
                         e = {expf_nonpositive(x[0], l.exp_tab), expf_nonpositive(x[1], l.exp_tab), expf_nonpositive(x[2], l.exp_tab), expf_nonpositive(x[3], l.exp_tab)};
@@ -655,10 +624,10 @@ __global__ __launch_bounds__(kThreads, 2) void attn128_prompt_kernel(PromptArgs 
     __syncthreads();
 
     // ---- 3
-    if (wide)
-        wide_values<ROWS>(a, l, kvh, t0, rows, s_row0);
-    else if constexpr (ROWS == kRows)
+    if constexpr (LIMBS)
         limb_values(a, l, kvh, t0, rows, s_row0);
+    else
+        wide_values<ROWS>(a, l, kvh, t0, rows, s_row0);
     __syncthreads();
 #pragma unroll
     for (uint32_t k = 0; k < ROWS / 8; k++) {  // four dimensions a thread: whole groups of eight lanes for the quantizer
@@ -673,12 +642,73 @@ __global__ __launch_bounds__(kThreads, 2) void attn128_prompt_kernel(PromptArgs 
     }
 }
 
+// Which head and tile a launch's workgroup takes: key/value head fastest, so that with eight of them every workgroup that
+// reads a head's keys is on one XCD
+struct PromptPlace {
+    uint32_t kvh, head, rank, tile;
+};
+__device__ __forceinline__ PromptPlace prompt_place(const PromptArgs &a, uint32_t i) {
+    const uint32_t kvh = i % a.n_head_kv, hpk = a.n_head / a.n_head_kv, rank = i / a.n_head;
+    return {kvh, kvh * hpk + (i / a.n_head_kv) % hpk, rank, a.first_tile + prompt_tile_of(rank, a.n_tiles, a.half_tiles)};
+}
+__global__ __launch_bounds__(kThreads, 2) void attn128_prompt_kernel(PromptArgs a) {
+    __shared__ PromptLds<16> l;
+    const PromptPlace p = prompt_place(a, blockIdx.x);
+    prompt_tile<16, false>(a, l, p.head, p.kvh, p.rank, p.tile * 16, a.scratch + size_t(blockIdx.x) * 16 * a.score_stride);
+}
+// 32 positions a workgroup, in limbs where they hold.  In f64 those are a longer chain than sixteen, which tells where a
+// compute unit has no other workgroup: there (gridDim.y = 2) such a tile is two workgroups' of sixteen, and the workgroups
+// y = 1, whose tiles are in the other order, end at once otherwise.
+__global__ __launch_bounds__(kThreads, 2) void attn128_prompt_limbs_kernel(PromptArgs a) {
+    __shared__ union {
+        PromptLds<kRows> whole;
+        PromptLds<16> half;
+    } l;
+    const uint32_t tid = threadIdx.x, lane = tid & 63, wave = uint32_t(__builtin_amdgcn_readfirstlane(int(tid >> 6)));
+    const uint32_t c16 = lane & 15, g = lane >> 4, second = blockIdx.y;
+    const uint32_t i = second ? (a.n_tiles - 1 - blockIdx.x / a.n_head) * a.n_head + blockIdx.x % a.n_head : blockIdx.x;
+    const PromptPlace p = prompt_place(a, i);
+    const uint32_t t0 = p.tile * kRows, rows = a.n_tok - t0 < kRows ? a.n_tok - t0 : kRows;
+    const uint32_t n_blocks = (a.step0 + t0 + rows + 63) / 64;
+    float *s_row0 = a.scratch + size_t(i) * kRows * a.score_stride;  // [position][key], rows of whole turns
+
+    // Wave w: positions 16 (w / 2) .. + 15, half w % 2 of the dimensions, lane (c16, g) sixteen of them of position c16
+    const uint32_t r = (wave >> 1) * 16 + c16, t = t0 + (r < rows ? r : rows - 1);
+    const u32x4 *src = reinterpret_cast<const u32x4 *>(a.q16 + (size_t(t) * a.n_head + p.head) * 128 + (wave & 1) * 64 + g * 16);
+    const u32x4 u[2] = {src[0], src[1]};
+    bool wide = false;
+    for (uint32_t b = tid; b < n_blocks; b += kThreads)
+        wide |= (a.limbs.wide[p.kvh * a.limbs.blocks + b] | a.limbs.wide[(a.n_head_kv + p.kvh) * a.limbs.blocks + b]) != 0;
+#pragma unroll
+    for (int j = 0; j < 2; j++)
+#pragma unroll
+        for (int k = 0; k < 4; k++) wide |= !limbs_hold(u[j][k]);
+    {
+        _Float16 h[16];
+#pragma unroll
+        for (int j = 0; j < 16; j++) h[j] = __builtin_bit_cast(f16x8, u[j >> 3])[j & 7];
+        u32x4 ql[4];
+        limbs_of16(h, ql);
+#pragma unroll
+        for (int j = 0; j < 4; j++) l.whole.q[wave][j][lane] = ql[j];
+    }
+    wide = __syncthreads_or(wide);  // the same in both workgroups of a tile
+    if (!wide) {
+        if (second == 0) prompt_tile<kRows, true>(a, l.whole, p.head, p.kvh, p.rank, t0, s_row0);
+    } else if (gridDim.y == 1) {
+        prompt_tile<kRows, false>(a, l.whole, p.head, p.kvh, p.rank, t0, s_row0);
+    } else if (second * 16 < rows) {
+        prompt_tile<16, false>(a, l.half, p.head, p.kvh, p.rank, t0 + second * 16, s_row0 + size_t(second) * 16 * a.score_stride);
+    }
+}
+
 // Whether a pass's keys and values are split into limbs: the splitting is a launch of 5 to 7 us that the products have to
-// win back, and a workgroup that finds values that limbs don't hold does 32 positions in f64 where two would have shared them.
-// So only where norms keep queries and keys small, and from a million products of a query and a key on.  us a layer, f64 |
-// limbs, 16 heads: prompt of 128 99 | 103, 256 139 | 140, 384 184 | 182, 700 299 | 277, 1024 394 | 349; 2048 tokens in passes
-// of 65 141 | 132, of 512 265 | 228, of 1024 476 | 380; 32 heads: prompt of 192 581 | 584, 256 691 | 690, 512 1215 | 1193, 1024
-// 2428 | 2336.  Values that don't fit, 16 heads: prompt of 512 212 | 243, 1024 399 | 417, 2048 tokens in passes of 1024 488 | 489.
+// win back, and a head of values that limbs don't hold has it for nothing and its positions in f64.  So only where norms keep
+// queries and keys small, and from a million products of a query and a key on.  us a layer, f64 | limbs, 16 heads: prompt of
+// 128 99 | 103, 256 139 | 140, 384 184 | 182, 700 299 | 277, 1024 394 | 349; 2048 tokens in passes of 65 141 | 132, of 512 265 |
+// 228, of 1024 476 | 380; 32 heads: prompt of 192 581 | 584, 256 691 | 690, 512 1215 | 1193, 1024 2428 | 2336.  Values that
+// don't fit, 16 heads, in f64 from the start | found here: prompt of 384 196 | 204, 512 223 | 225 (216 and 245 with 32 positions a
+// workgroup), 700 310 | 330, 1024 409 | 419, 2048 977 | 974.
 bool limbs_pay(uint32_t n_head, uint32_t step0, uint32_t n_tok) { return uint64_t(n_head) * n_tok * (step0 + n_tok / 2) >= 1u << 20; }
 
 }  // namespace
@@ -713,9 +743,9 @@ int rmi_launch_attn128_prompt(const uint16_t *q16, const uint16_t *k_cache, cons
         const uint32_t half = n * n_head <= 2 * cus && n * n_head > cus ? (cus + n_head - 1) / n_head : n;
         const PromptArgs args{q16, k_cache, v_cache, step0, n_tok, kv_stride, n_head, n_head_kv, t, n, half, stride, scratch, q8, scales, rounding, limbs};
         if (use_limbs)
-            hipLaunchKernelGGL(attn128_prompt_kernel<kRows>, dim3(n * n_head), dim3(kThreads), 0, st, args);
+            hipLaunchKernelGGL(attn128_prompt_limbs_kernel, dim3(n * n_head, n * n_head <= cus ? 2 : 1), dim3(kThreads), 0, st, args);
         else
-            hipLaunchKernelGGL(attn128_prompt_kernel<16>, dim3(n * n_head), dim3(kThreads), 0, st, args);
+            hipLaunchKernelGGL(attn128_prompt_kernel, dim3(n * n_head), dim3(kThreads), 0, st, args);
     }
     RMI_HIP_CHECK(hipGetLastError());
     return RMI_HIP_OK;

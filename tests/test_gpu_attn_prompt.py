@@ -43,10 +43,12 @@ PLANTED = {
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("heads,kv_heads,step0,n_tok,one_launch", [
-    (8, 4, 300, 320, True), (8, 4, 293, 321, False), (8, 4, 0, 528, True), (16, 4, 333, 160, True), (8, 4, 1000, 143, False), (8, 4, 129, 433, True)])
+    (8, 4, 300, 320, True), (8, 4, 293, 321, False), (8, 4, 0, 528, True), (16, 4, 333, 160, True), (8, 4, 1000, 143, False), (8, 4, 129, 433, True), (64, 8, 200, 161, True)])
 @pytest.mark.parametrize("planted", PLANTED)
 def test_limbs_have_the_bits_of_f64(hip, heads, kv_heads, step0, n_tok, one_launch, planted):
-    """Passes of whole tiles and of a rest of 1, 15, 16 and 17 positions; in one launch, and with scratch for a tile at a time."""
+    """Passes of whole tiles and of a rest of 1, 15, 16 and 17 positions; in one launch, and with scratch for a tile at a time;
+    more tiles than compute units (64 heads), where one workgroup does all 32 positions that limbs don't hold, and fewer, where
+    two do."""
     H = hip.hip
     rng = np.random.default_rng(n_tok)
     n_keys, n_blocks = step0 + n_tok, (step0 + n_tok + 63) // 64
