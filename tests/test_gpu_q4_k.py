@@ -61,6 +61,30 @@ def test_q8_k_quantizer_bit_exact(hip, oracle):
         assert np.array_equal(bits(d), bits(rd)) and np.array_equal(qs, rq) and np.array_equal(bs, rb)
 
 
+@pytest.mark.parametrize("rest", [-13, -1, 0, 1, 2, 5, 8, 11, 15])
+@pytest.mark.parametrize("blocks_of_a_wave", [1, 2, 4])
+def test_quantize_q8_k_of_many_blocks(hip, oracle, blocks_of_a_wave, rest):
+    """A wave takes two blocks from 32 and four from 64 blocks a compute unit on: on both sides of either line, with every rest of
+    a wave and a workgroup.  Blocks of zeros and blocks whose largest magnitude is there with both signs, at every place of a
+    wave; nothing is written behind the ends."""
+    H, n = hip.hip, {1: 700, 2: 32, 4: 64}[blocks_of_a_wave]
+    n = n + 13 + rest if blocks_of_a_wave == 1 else n * H.device_info()[1] + rest
+    x = np.random.default_rng(n).standard_normal((n, 256), dtype=np.float32)
+    x[::7] = 0  # (7 and 5: every place of a wave of two or four)
+    sign = np.float32(1) if rest % 2 else np.float32(-1)
+    x[3::5, 200], x[3::5, 17], x[3::5, 19] = 9 * sign, -9 * sign, 9 * sign
+    x[-1, [0, 255]] = 11 * sign, -11 * sign
+    guard = 64
+    bufs = [H.DeviceBuffer.from_array(np.full(size + guard, 77, t)) for t, size in ((np.float32, n), (np.int8, n * 256), (np.int16, n * 16))]
+    d_x = H.DeviceBuffer.from_array(x)
+    H.check(H.lib.rmi_hip_quantize_row_q8_k_dev(d_x.ptr, *(b.ptr for b in bufs), n, 256, None))
+    H.check(H.lib.rmi_hip_synchronize())
+    for b, want in zip(bufs, oracle.quantize_row_q8_k(x.reshape(-1), A)):
+        got = b.to_array(want.dtype, want.size + guard)
+        assert got[:want.size].tobytes() == want.tobytes()
+        assert (got[want.size:] == 77).all()
+
+
 # ------------------------------------------------------------------ integer path
 
 @pytest.mark.parametrize("n_out,n_in", [(6144, 2048), (2048, 6144), (1, 256), (13, 512), (100, 1024)])
