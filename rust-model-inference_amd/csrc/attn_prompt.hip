@@ -166,18 +166,6 @@ __global__ __launch_bounds__(kThreads) void attn128_limbs_kernel(const uint16_t 
 }
 
 // ---- the pass
-// rmi_expf_tab of a finite value that is not above zero: nothing overflows, and what underflows is zero
-__device__ __forceinline__ float expf_nonpositive(float x, const uint64_t *tab) {
-    const double inv_ln2_n = 0x1.71547652b82fep+0 * 32, shift = 0x1.8p+52;
-    const double c0 = 0x1.c6af84b912394p-5 / 32 / 32 / 32, c1 = 0x1.ebfce50fac4f3p-3 / 32 / 32, c2 = 0x1.62e42ff0c52d6p-1 / 32;
-    const double xd = double(x), z = inv_ln2_n * xd, kd = z + shift, r = __builtin_fma(inv_ln2_n, xd, -(kd - shift));
-    const uint32_t k = uint32_t(__double_as_longlong(kd));
-    const u32x2 t = *reinterpret_cast<const u32x2 *>(tab + (k & 31));
-    const double s = __hiloint2double(int(t[1] + (k << 15)), int(t[0]));  // table + (k << 47)
-    const double p = __builtin_fma(c0, r, c1), r2 = r * r;
-    const double y = __builtin_fma(p, r2, __builtin_fma(c2, r, 1.0)) * s;
-    return x < -0x1.9fe368p6f ? 0.0f : float(y);
-}
 constexpr uint32_t kSuper = 4;  // blocks of 64 keys whose weights are in LDS at once
 template <uint32_t ROWS>
 struct PromptLds {
@@ -589,7 +577,7 @@ __device__ __forceinline__ void prompt_tile(const PromptArgs &a, PromptLds<ROWS>
                     if constexpr (!LIMBS)
                         e = {rmi_expf_tab(x[0], l.exp_tab), rmi_expf_tab(x[1], l.exp_tab), rmi_expf_tab(x[2], l.exp_tab), rmi_expf_tab(x[3], l.exp_tab)};
                     else
-                        e = {expf_nonpositive(x[0], l.exp_tab), expf_nonpositive(x[1], l.exp_tab), expf_nonpositive(x[2], l.exp_tab), expf_nonpositive(x[3], l.exp_tab)};
+                        e = {rmi_expf_nonpositive(x[0], l.exp_tab), rmi_expf_nonpositive(x[1], l.exp_tab), rmi_expf_nonpositive(x[2], l.exp_tab), rmi_expf_nonpositive(x[3], l.exp_tab)};
                     if (behind) {
                         const uint32_t key = turn_i * kTurn + k4 + j * kAcross;
                         e.x = key <= last ? e.x : 0.0f;

@@ -24,7 +24,18 @@ __device__ static constexpr uint64_t kRmiExp2fTab[32] = {
     0x3fef5818dcfba487ull, 0x3fef7c97337b9b5full, 0x3fefa4afa2a490daull, 0x3fefd0765b6e4540ull,
 };
 
-// `tab` is kRmiExp2fTab or a copy of it in LDS (a kernel that calls this in a latency-bound phase copies it first)
+// The reduction and the polynomial, of an x that neither overflows nor underflows to zero.  `tab` is kRmiExp2fTab or a copy of
+// it in LDS (a kernel that calls this in a latency-bound phase copies it first).
+__device__ __forceinline__ float rmi_expf_inside(float x, const uint64_t *tab) {
+    const double inv_ln2_n = 0x1.71547652b82fep+0 * 32, shift = 0x1.8p+52;
+    const double c0 = 0x1.c6af84b912394p-5 / 32 / 32 / 32, c1 = 0x1.ebfce50fac4f3p-3 / 32 / 32, c2 = 0x1.62e42ff0c52d6p-1 / 32;
+    const double xd = double(x), z = inv_ln2_n * xd, kd = z + shift, r = __builtin_fma(inv_ln2_n, xd, -(kd - shift));
+    const uint32_t k = uint32_t(__double_as_longlong(kd));
+    const uint64_t t = tab[k & 31];
+    const double s = __hiloint2double(int(uint32_t(t >> 32) + (k << 15)), int(uint32_t(t)));  // table + (k << 47)
+    const double p = __builtin_fma(c0, r, c1), r2 = r * r;
+    return float(__builtin_fma(p, r2, __builtin_fma(c2, r, 1.0)) * s);
+}
 __device__ __forceinline__ float rmi_expf_tab(float x, const uint64_t *tab) {
     const uint32_t ux = __float_as_uint(x);
     const uint32_t abstop = (ux >> 20) & 0x7ff;
@@ -34,23 +45,12 @@ __device__ __forceinline__ float rmi_expf_tab(float x, const uint64_t *tab) {
         if (x > 0x1.62e42ep6f) return __uint_as_float(0x7f800000u);  // overflow
         if (x < -0x1.9fe368p6f) return 0.0f;                         // underflow
     }
-    const double inv_ln2_n = 0x1.71547652b82fep+0 * 32, shift = 0x1.8p+52;
-    const double c0 = 0x1.c6af84b912394p-5 / 32 / 32 / 32, c1 = 0x1.ebfce50fac4f3p-3 / 32 / 32,
-                 c2 = 0x1.62e42ff0c52d6p-1 / 32;
-    const double xd = double(x);
-    const double z = inv_ln2_n * xd;
-    double kd = z + shift;
-    const uint64_t ki = uint64_t(__double_as_longlong(kd));
-    kd -= shift;
-    const double r = __builtin_fma(inv_ln2_n, xd, -kd);
-    const uint64_t t = tab[ki & 31] + (ki << 47);
-    const double s = __longlong_as_double((long long)t);
-    const double p = __builtin_fma(c0, r, c1);
-    const double r2 = r * r;
-    double y = __builtin_fma(c2, r, 1.0);
-    y = __builtin_fma(p, r2, y);
-    y = y * s;
-    return float(y);
+    return rmi_expf_inside(x, tab);
+}
+// of a finite x that is not above zero: nothing overflows, and what underflows is zero
+__device__ __forceinline__ float rmi_expf_nonpositive(float x, const uint64_t *tab) {
+    const float y = rmi_expf_inside(x, tab);
+    return x < -0x1.9fe368p6f ? 0.0f : y;
 }
 
 __device__ __forceinline__ float rmi_expf(float x) { return rmi_expf_tab(x, kRmiExp2fTab); }
