@@ -146,7 +146,8 @@ int host_gemv_range(const rmi_hip_weight *w, const uint8_t *input_q8, const floa
     int rc = stage_x(c, input_q8, input_scales, size_t(n_tokens) * w->n_in, size_t(n_tokens) * (w->n_in / 32), &x);
     if (rc != RMI_HIP_OK) return rc;
     const uint32_t n_rows = row_end - row_start;
-    // only the row slice, y[t][row - row_start], straight into pinned memory (see forward_batched)
+    // only the row slice, y[t][row - row_start], straight into pinned memory (see forward_batched).  us with a copy | without, 1
+    // token: Q8_0 1024 x 3072 23.4 | 21.1, sixteen rows of it 22.9 | 20.7, 1024 x 151936 74.8 | 64.7; Q4_0 4096 x 12288 34.1 | 26.7
     float *pin = static_cast<float *>(rmi_pin_buf(c, 1, size_t(n_tokens) * n_rows * 4));
     if (!pin) return RMI_HIP_E_RUNTIME;
     rc = rmi_gemv_q8_0_tokens(w, x.d_q8, x.d_scales, pin - row_start, n_tokens, n_rows, row_start, row_end, c->stream);
@@ -219,11 +220,13 @@ static int forward_batched(const rmi_hip_weight *w, const float *input, float *o
     if (!c) return RMI_HIP_E_RUNTIME;
     const size_t n_x = size_t(n_tokens) * n_in;
     const size_t x_bytes = n_x * 4, y_bytes = size_t(n_tokens) * n_out * 4;
-    // The quantizer reads every input once and the x86-64-order products write every result once, so both may use the pinned
+    // The quantizer reads every input once, and the x86-64-order products only write results and never read them back (of the
+    // tokens behind whole groups of eight, up to five are written twice, with the same bits), so both may use the pinned
     // buffers themselves: a copy command less on either side, each of which is 5 to 8 us between dependent kernels.  From some
-    // 700 KB on the copy is the faster reader; writing was never slower (512 x 500 to 4096 x 12000, 1 to 300 tokens).  us with
-    // copies | x in place | y in place | both: 2048 x 6144, 1 token 31.5 | 28.5 | 22.4 | 20.4, 13 tokens 60.9 | 54.9 | 53.0 |
-    // 45.5, 100 tokens (800 KB) 209.0 | 211.1 | 200.3 | 202.6; 8192 x 3000, 300 tokens (9.6 MB) 616 | 661 | 571 | 612.
+    // 700 KB on the copy is the faster reader.  us with copies | x in place | y in place | both: 2048 x 6144, 1 token 31.5 | 28.5 |
+    // 22.4 | 20.4, 13 tokens 60.9 | 54.9 | 53.0 | 45.5, 100 tokens (800 KB) 209.0 | 211.1 | 200.3 | 202.6; 8192 x 3000, 300 tokens
+    // (9.6 MB) 616 | 661 | 571 | 612.  Results in place, of 24 to 1000 tokens (50 KB to 48 MB) through 512..8192 x 500..12000: 0.98 to
+    // 1.18 times as fast as with a copy, 5 % in the mean; 1024 x 3072, 300 tokens 281 | 276, 8192 x 12000, 1000 tokens 5498 | 4776.
     const bool x_in_place = x_bytes <= 512 * 1024, y_in_place = x86_order;
     float *pin = static_cast<float *>(rmi_pin_buf(c, 0, x_bytes));
     float *d_x = x_in_place ? pin : static_cast<float *>(rmi_dev_buf(c, 0, x_bytes));

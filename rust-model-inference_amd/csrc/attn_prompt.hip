@@ -28,8 +28,7 @@
 // the first 1024 keys 50 us, 127): the int8 products at 2.9 POP/s in phase 1 (a third of the time; the same with the results'
 // conversion or the scores' stores taken out, so the matrix cores at the clock they have under it), the f64 of the libm's
 // expf and the ordered sums in phase 2 (a quarter), and the weights' division and limbs in turn with the products in phase 3.
-// Four waves a SIMD in the place of two (eight waves a workgroup, 128 registers) took as long.
-// A prompt of 1999 tokens, 28 layers: 29.0 -> 22.2 ms; passes of up to 1024 positions times heads take a workgroup a position
+// A prompt of 1999 tokens, 28 layers: 29.0 ms in f64, 21.5 in limbs; passes of up to 1024 positions times heads take a workgroup a position
 // and head (pass_by_positions in decode_qwen3.hip).
 #include "attn_prompt.h"
 

@@ -388,9 +388,9 @@ constexpr int rmi_waitcnt(int vm) { return (vm & 15) | (vm >> 4) << 14 | 7 << 4;
 // piece that belongs at its slot) through NB buffers, one barrier a step: behind it the next step's first half is read while
 // the second half of this one is multiplied, and the buffer that everybody has read takes the step NB on.  The wait in front
 // of the barrier counts the loads in flight, so that those of NB - 2 steps stay under way.
-// What bounds it: the matrix cores at the clock that they have under full load, and the way from L2.  Of the 312 us of 128 x 256
-// tiles (4096 x 20480, 2048 tokens) the products and barriers alone are 263 (1300 TFLOP/s, what a large library product
-// reaches); 256 x 256 tiles (39168 x 4096) run their loop in 474 us, 1386 TFLOP/s, in front of 146 us of results; 64 x 128
+// What bounds it: the matrix cores at the clock that they have under full load, and the way from L2.  Of the 327 us of 128 x 256
+// tiles (4096 x 20480, 2048 tokens, three column segments and so three launches) the products and barriers alone are 263 (1300
+// TFLOP/s, what a large library product reaches); 256 x 256 tiles (39168 x 4096) run their loop in 474 us, 1386 TFLOP/s, in front of 146 us of results; 64 x 128
 // tiles ask 96 bytes a clock and compute unit of L2, and take as long as that does.
 template <typename T, int BN, int BT, int WN, int WT, int NB, int WPS, int EPI>
 __global__ __launch_bounds__(64 * (BN / WN) * (BT / WT), WPS) void dense_gemm_wide_kernel(const T *__restrict__ w, const T *__restrict__ a, uint32_t n_rows, uint32_t k_pad,
@@ -497,8 +497,8 @@ __global__ __launch_bounds__(64 * (BN / WN) * (BT / WT), WPS) void dense_gemm_wi
     asm volatile("" ::: "memory");
     read(buf0, 0);
     // Whole turns of the buffers in a loop that has no other way out: with one, the compiler takes it that a buffer may be read
-    // right behind its fetch, and waits for every load in flight once a turn (128 x 256, residual 4096 x 20480, 2048 tokens: 367 us with that and the
-    // results joining x from the registers, segments in the loop; 312 without, in two launches).
+    // right behind its fetch, and waits for every load in flight once a turn (128 x 256, residual 4096 x 20480, 2048 tokens: 355 us with that, the
+    // three segments in the loop and the results joining x from the registers; 327 without, in three launches).
     uint32_t step = first;
     auto buffer = [&](int i) { return i % NB == 0 ? buf0 : i % NB == 1 ? buf1 : buf2; };
     for (; step + NB <= n_steps; step += NB) {
@@ -539,8 +539,10 @@ __global__ __launch_bounds__(64 * (BN / WN) * (BT / WT), WPS) void dense_gemm_wi
 //   activated 12304 x 1024, 2048 tokens    138 |  129 | 103 | 104 | 121 | 120     768 tokens    54 |  53 |  47 |  50 |  67 |  61
 //   activated 39968 x 4096, 2048 tokens   1504 | 1169 | 797 | 846 | 760 | 687     512 tokens   320 | 280 | 210 | 231 | 233 | 264
 //   residual 4096 x 12288, 2048 tokens     375 |  303 | 246 | 239 | 193 | 341     512 tokens   102 | 104 | 150 | 170 | 195 | 357
-// (Fitted and measured with results that left the wide tiles from the registers; by lines they are 5 to 15 % faster, which the
-// estimates don't know: the choice errs to the narrower side.)
+// All of that with results that left the wide tiles from the registers.  By lines they are faster (the first four rows with SiLU and
+// results in bf16 now: 128 | 96 | 97 | 79 | 78 | 71 and 45 | 37 | 42 | 38 | 41 | 35, 1481 | 1080 | 770 | 741 | 599 | 528 and
+// 315 | 252 | 202 | 227 | 181 | 207), which the estimates don't know: over 264 products of eleven weights the choice costs 5 % over
+// the best tile, at most 40 %, nearly always by being narrower than that.
 enum DenseTile { kTile64x16, kTile64x32, kTile64x64, kTile64x128, kTile128x128w4, kTile128x128, kTile128x256, kTile256x256 };
 struct TileCost {
     DenseTile tile;
@@ -568,7 +570,7 @@ const TileCost &dense_tile_of(bool bf16, int epilogue, uint32_t n_rows, uint32_t
     const TileCost *best = nullptr;
     double least = 0;
     auto consider = [&](const TileCost &c) {
-        if (epilogue == kResidual && c.tile == kTile256x256) return;  // (2 % the better at the widest at most, and registers spill)
+        if (epilogue == kResidual && c.tile == kTile256x256) return;  // (2 % the better at the widest at most, and registers spilled, by the older way out)
         const uint64_t tiles = uint64_t((n_rows + c.rows - 1) / c.rows) * ((n_tokens + c.tokens - 1) / c.tokens);
         const uint64_t rounds = tiles / (c.fit * cus), left = tiles % (c.fit * cus);
         double step = double(rounds) * c.round;

@@ -177,19 +177,33 @@ def _chosen(hip, elem, kind, rows, k, tokens):
 
 
 # us of bf16 products, each launch with a weight from HBM, by the tiles of 64 x 64, 64 x 128, 128 x 128 with four and with eight
-# waves, 128 x 256 and 256 x 256
+# waves, 128 x 256 and 256 x 256: as the estimates were fitted, when the wide tiles' results left from the registers, and as the
+# tiles are (SiLU, results in bf16; residual products have no 256 x 256)
 MEASURED_TILES = [(64, 64, 4), (64, 128, 8), (128, 128, 4), (128, 128, 8), (128, 256, 8), (256, 256, 8)]
 MEASURED = [("acted", 12304, 1024, 2048, (138, 129, 103.5, 104.5, 121, 120)), ("acted", 12304, 1024, 768, (54.4, 53.0, 47.3, 49.9, 67.4, 61.3)),
             ("acted", 39968, 4096, 2048, (1504, 1169, 797, 846, 760, 687)), ("acted", 39968, 4096, 512, (320, 280, 210, 231, 233, 264)),
             ("residual", 4096, 12288, 2048, (375, 303, 246, 239, 193, 341)), ("residual", 4096, 12288, 512, (102.1, 104.4, 150, 170, 195, 357))]
+MEASURED_SINCE = [("acted", 12304, 1024, 2048, (128.0, 96.2, 97.1, 78.8, 78.4, 70.9)), ("acted", 12304, 1024, 768, (45.4, 36.7, 41.8, 37.9, 40.7, 34.8)),
+                  ("acted", 39968, 4096, 2048, (1481, 1080, 770, 741, 599, 528)), ("acted", 39968, 4096, 512, (315, 252, 202, 227, 181, 207)),
+                  ("residual", 4096, 12288, 2048, (345, 270, 241, 210, 164, np.inf)), ("residual", 4096, 12288, 512, (100.1, 82.0, 142, 158, 152, np.inf))]
 
 
 @pytest.mark.parametrize("kind,rows,k,tokens,us", MEASURED)
 def test_the_choice_follows_the_measurements(hip, kind, rows, k, tokens, us):
-    """The fitted estimates pick a tile within 3 % of the fastest."""
+    """The fitted estimates pick a tile within 3 % of the fastest of those they were fitted to.  (A new fit replaces these times by
+    those below.)"""
     if hip.hip.device_info()[1] != 256:
         pytest.skip("measured on 256 compute units")
     assert us[MEASURED_TILES.index(_chosen(hip, 2, kind, rows, k, tokens))] <= 1.03 * min(us)
+
+
+@pytest.mark.parametrize("kind,rows,k,tokens,us", MEASURED_SINCE)
+def test_how_far_the_choice_is_from_todays_tiles(hip, kind, rows, k, tokens, us):
+    """Within 40 % of the fastest, the worst over 264 products (5 % in the mean): the wide tiles became faster than the estimates
+    know."""
+    if hip.hip.device_info()[1] != 256:
+        pytest.skip("measured on 256 compute units")
+    assert us[MEASURED_TILES.index(_chosen(hip, 2, kind, rows, k, tokens))] <= 1.4 * min(us)
 
 
 @pytest.mark.parametrize("tile,kind,size", CASES, ids=["%d-%dx%dx%d-%s" % (*t, k) for t, k, _ in CASES])
