@@ -6,15 +6,23 @@
 // acc[L]), block after block.  The dots come from v_mfma_f32_16x16x4_4b_f16: four independent 16 x 16 products of
 // depth four, so one instruction is sixteen rows x sixteen tokens x four slices.  An int8 is exact in f16, the products
 // and the sum of four of them are exact in f32, so the dot arrives as the f32 the fma takes: no conversion, and what is
-// left on the vector ALU is the order's own fma and one scale product for eight of them.  Slices 2 beta and 2 beta + 1
+// left on the vector ALU is the order's own fma.  Slices 2 beta and 2 beta + 1
 // are the two instructions' block beta, so that a lane reads both operands of a block with one 16-byte LDS load, and
 // holds all eight sums of its four rows and one token: the horizontal sum at the end crosses no lanes.
 //
-// What bounds it: the vector ALU, 36 instructions per 16 x 16 x 32 (32 fma, 4 scale products) = 61 ns a SIMD with four
-// waves on it, 66 with two (277 / 254 TOP/s for the chip if nothing else cost anything); the matrix cores are busy half
-// of that.  Converting the operands to f16 as they are staged is 5 vector instructions per 4 values, shared by the waves
-// that read them.  Measured: 4096 x 1024, 512 tokens 53 -> 28 us, 151936 x 1024, 128 tokens 529 -> 220 (182 TOP/s), against
-// eight tokens to a workgroup with int8 dots (4 x 4 x 4) and a conversion each, on the GEMV's kernel.
+// The scale products wd * xd come from the same instruction, four outer products of sixteen rows and sixteen tokens: the weight
+// scale is an f16, the token scale the reference's quantizers write is an f16 value held in an f32 (src/ops/quant/q8_0.rs:63,
+// 121, 207), and the product of two f16 values is exact in f32.  (v_mfma_f32_16x16x1_4b_f32 would take any f32 scale, but f32
+// products of the matrix cores and f32 sums of the vector ALU keep each other from running: 64 sums and two products 119 ns a
+// wave with f16 operands, 148 with f32 ones.)  A tile with a token scale that is no f16 value, a caller's own, is made again
+// on the vector ALU behind the loop.
+//
+// What bounds it: the vector ALU, 32 fma per 16 x 16 x 32 = 54 ns a SIMD with four waves on it, beside which the conversion of
+// the operands to f16 as they are staged costs 5 instructions per 4 values, shared by the waves that read them: 642 vector
+// instructions a quad of a wave's four tiles, issued 80 % of the time with the two waves whose sums fit the registers.  us, with
+// the scale products on the vector ALU | as it is: 64 x 64 tiles, 6144 x 1024, 1024 tokens 70.8 | 68.5, 151936 x 1024, 128
+// tokens 213 | 207; 32 x 32 tiles, 1024 x 3072, 512 tokens 26.3 | 25.0, 1024 x 2048, 512 tokens 19.5 | 18.4.
+// Eight tokens to a workgroup of the GEMV with int8 dots (4 x 4 x 4) and a conversion each: 151936 x 1024, 128 tokens 529.
 #include "rmi_internal.h"
 
 #include "device_common.h"
@@ -35,23 +43,25 @@ __device__ __forceinline__ u32x2 i8x4_to_f16x4(uint32_t q) {
                  __builtin_bit_cast(uint32_t, __builtin_bit_cast(f16x2, hi) + off)};
 }
 
-// A workgroup of WR x WT waves, each NR x NT tiles of sixteen rows x sixteen tokens; k in quads of four blocks through
-// two LDS buffers, the next quad's bytes on their way to registers meanwhile.  One block of a buffer is [row][32 f16].
+// A workgroup of WR x WT waves, each NR x NT tiles of sixteen rows x sixteen tokens; k in quads of four blocks through two LDS
+// buffers, the next quad's bytes on their way to registers meanwhile.  One block of a buffer is [row][32 f16]; behind the blocks
+// stand the quad's scales, [row][4 f16].
 template <int NR, int NT, int WR, int WT>
 struct X86Tile {
     static constexpr int BN = 16 * NR * WR, BT = 16 * NT * WT, THREADS = 64 * WR * WT;
     static constexpr int ABLK = BN * 64 + 64, BBLK = BT * 64 + 64;  // bytes of a block, off a multiple of 256
-    static constexpr int LDS_BUF = 4 * (ABLK + BBLK) + 16 * (BN + BT);
+    static constexpr int LDS_BUF = 4 * (ABLK + BBLK) + 8 * (BN + BT);
 };
 
 template <int NR, int NT, int WR, int WT, int WPS>
 __global__ __launch_bounds__(64 * WR * WT, WPS) void gemm_q8_0_x86_kernel(RmiGemvProblem p, uint32_t n_tokens, uint32_t grid_n,
-                                                                          uint32_t grid_t, uint32_t t_fastest, uint32_t xcd_split) {
+                                                                               uint32_t grid_t, uint32_t t_fastest, uint32_t xcd_split) {
     using TL = X86Tile<NR, NT, WR, WT>;
     constexpr int BN = TL::BN, BT = TL::BT, TH = TL::THREADS;
     constexpr int PA = (BN * 8 + TH - 1) / TH, PB = (BT * 8 + TH - 1) / TH;  // 16-byte pieces a thread stages per quad
     constexpr int PS = (BT * 4 + TH - 1) / TH;
     static_assert(BN <= TH, "one thread a row for the weight scales");
+    static_assert(NR * NT == 1 || (NR == 2 && NT == 2), "four scale products an instruction: of four blocks or of four tiles");
     extern __shared__ uint4 lds_raw[];
     uint8_t *lds = reinterpret_cast<uint8_t *>(lds_raw);
     const uint32_t tid = threadIdx.x, lane = tid & 63, wave = uint32_t(__builtin_amdgcn_readfirstlane(int(tid >> 6)));
@@ -69,28 +79,35 @@ __global__ __launch_bounds__(64 * WR * WT, WPS) void gemm_q8_0_x86_kernel(RmiGem
     const gptr_u8 x_base = as_global<gptr_u8>(p.x_q8 + size_t(tok0) * p.n_in);
     const gptr_u8 xs_base = as_global<gptr_u8>(p.x_scales + size_t(tok0) * nb);
     const uint32_t last_tile = p.n_tiles - 1 - tile0, last_tok = n_tokens - 1 - tok0;  // past them these are read again and not stored
-    uint32_t a_off[PA], b_off[PB], bs_off[PS];
+    // weights: lane 8 r + L of a tile's pieces, each the slice L of four blocks; a wave's pieces lie in one tile
+    const uint32_t a_lane = p.n_oct * 128 + (tid & 63) * 16;
+    gptr_u8 a_base[PA];
 #pragma unroll
-    for (int i = 0; i < PA; i++) {  // lane 8 r + L of a tile's pieces
-        const uint32_t e = (tid + i * TH) % (BN * 8), t = (e >> 6) < last_tile ? e >> 6 : last_tile;
-        a_off[i] = t * uint32_t(tile_bytes) + p.n_oct * 128 + (e & 63) * 16;
+    for (int i = 0; i < PA; i++) {
+        const uint32_t t = wave + i * (TH / 64);
+        a_base[i] = w_base + size_t(t < last_tile ? t : last_tile) * tile_bytes;
     }
-    const uint32_t a_dst = ((tid % (BN * 8)) >> 3) * 64 + (tid & 7) * 8;  // piece i: TH / 8 rows on
+    // (what follows from the thread's number in an instruction or two is made where it is used: a register less each)
+    auto me = [&] {
+        uint32_t t = tid;
+        if (NR * NT > 1 || WT == 1) asm volatile("" : "+v"(t));
+        return t;
+    };
+    uint32_t b_off[PB], bs_off[PS];
 #pragma unroll
     for (int i = 0; i < PB; i++) {  // token, half block tid & 7
-        const uint32_t e = (tid + i * TH) % (BT * 8), t = (e >> 3) < last_tok ? e >> 3 : last_tok;
+        const uint32_t e = (tid + i * TH) % (BT * 8) / 8, t = e < last_tok ? e : last_tok;
         b_off[i] = t * p.n_in + (tid & 1) * 16;
     }
-    const uint32_t b_blk = (tid >> 1) & 3, b_dst = 4 * TL::ABLK + b_blk * TL::BBLK + ((tid % (BT * 8)) >> 3) * 64 + (tid & 1) * 32;
-    const uint32_t s_row = tid < BN ? tid : BN - 1, s_tile = (s_row >> 3) < last_tile ? s_row >> 3 : last_tile;
+    const uint32_t b_dst = 4 * TL::ABLK + (tid >> 1 & 3) * TL::BBLK + ((tid % (BT * 8)) / 8) * 64 + (tid & 1) * 32;
+    const uint32_t s_row = tid % BN, s_tile = (s_row >> 3) < last_tile ? s_row >> 3 : last_tile;
     const uint32_t as_off = s_tile * uint32_t(tile_bytes) + (s_row & 7) * 16;
-    constexpr uint32_t kScaleA = 4 * (TL::ABLK + TL::BBLK), kScaleB = kScaleA + 16 * BN;
+    constexpr uint32_t kScaleA = 4 * (TL::ABLK + TL::BBLK), kScaleB = kScaleA + 8 * BN;
 #pragma unroll
     for (int i = 0; i < PS; i++) {
         const uint32_t e = (tid + i * TH) % (BT * 4), t = (e >> 2) < last_tok ? e >> 2 : last_tok;
         bs_off[i] = t * nb * 4;
     }
-    const uint32_t bs_blk = tid & 3, bs_dst = kScaleB + (bs_blk * BT + ((tid % (BT * 4)) >> 2)) * 4;
     u32x4 ra[PA], rb[PB];
     u32x2 rsa;
     float rsb[PS];
@@ -98,21 +115,27 @@ __global__ __launch_bounds__(64 * WR * WT, WPS) void gemm_q8_0_x86_kernel(RmiGem
         // always issued (past the end the last quad again): a skipped load would make the waits wait for all of them
         q = q < n_quads ? q : n_quads - 1;
 #pragma unroll
-        for (int i = 0; i < PA; i++) ra[i] = *(gptr_u4)(w_base + (a_off[i] + q * 1024));
-        const uint32_t bb = 4 * q + b_blk < nb ? 4 * q + b_blk : nb - 1;  // (a block past the end is not multiplied)
+        for (int i = 0; i < PA; i++) {
+            uint32_t lane_off = a_lane;
+            asm volatile("" : "+v"(lane_off));  // (else its sum with the base is kept, two registers a piece)
+            ra[i] = *(gptr_u4)(a_base[i] + q * 1024 + lane_off);
+        }
+        const uint32_t t = me(), b_at = 4 * q + (t >> 1 & 3), bb = b_at < nb ? b_at : nb - 1;  // (a block past the end is not multiplied)
 #pragma unroll
         for (int i = 0; i < PB; i++) rb[i] = *(gptr_u4)(x_base + (b_off[i] + bb * 32));
         rsa = *(gptr_u2)(w_base + (as_off + (q >> 1) * 128 + (q & 1) * 8));
-        const uint32_t bs = 4 * q + bs_blk < nb ? 4 * q + bs_blk : nb - 1;
+        const uint32_t bs_at = 4 * q + (t & 3), bs = bs_at < nb ? bs_at : nb - 1;
 #pragma unroll
         for (int i = 0; i < PS; i++) rsb[i] = *(gptr_f32)(xs_base + (bs_off[i] + bs * 4));
     };
+    uint64_t not_f16 = 0;  // lanes that staged a token scale which is not a finite f16 value
     auto park = [&](uint32_t buf) {
         uint8_t *base = lds + buf * TL::LDS_BUF;
+        const uint32_t t = me();
 #pragma unroll
         for (int i = 0; i < PA; i++)
 #pragma unroll
-            for (int b = 0; b < 4; b++) *reinterpret_cast<u32x2 *>(base + b * TL::ABLK + a_dst + i * (TH * 8)) = i8x4_to_f16x4(ra[i][b]);
+            for (int b = 0; b < 4; b++) *reinterpret_cast<u32x2 *>(base + t * 8 + (b * TL::ABLK + i * (TH * 8))) = i8x4_to_f16x4(ra[i][b]);
 #pragma unroll
         for (int i = 0; i < PB; i++)
 #pragma unroll
@@ -120,15 +143,16 @@ __global__ __launch_bounds__(64 * WR * WT, WPS) void gemm_q8_0_x86_kernel(RmiGem
                 const u32x2 u = i8x4_to_f16x4(rb[i][2 * k]), v = i8x4_to_f16x4(rb[i][2 * k + 1]);
                 *reinterpret_cast<u32x4 *>(base + b_dst + i * (TH * 8) + 16 * k) = u32x4{u[0], u[1], v[0], v[1]};
             }
-        if (tid < BN) {
+        if (t < BN) *reinterpret_cast<u32x2 *>(base + kScaleA + t * 8) = rsa;
 #pragma unroll
-            for (int b = 0; b < 4; b++)
-                *reinterpret_cast<float *>(base + kScaleA + (b * BN + tid) * 4) = h2f(b & 1 ? rsa[b >> 1] >> 16 : rsa[b >> 1] & 0xffffu);
+        for (int i = 0; i < PS; i++) {
+            const _Float16 x = _Float16(rsb[i]);
+            *reinterpret_cast<_Float16 *>(base + kScaleB + (t % (BT * 4)) * 2 + i * TH * 2) = x;
+            // x - f32(f16(x)) is +-0 exactly when x is a finite f16 value (inf - inf and NaN are not)
+            not_f16 |= __builtin_amdgcn_ballot_w64(!(rsb[i] - float(x) == 0.0f));
         }
-#pragma unroll
-        for (int i = 0; i < PS; i++) *reinterpret_cast<float *>(base + bs_dst + i * TH) = rsb[i];
     };
-    static_assert((BN * 8) % TH == 0 || BN * 8 < TH, "whole rounds of weight pieces");
+    static_assert((BN * 8) % TH == 0, "whole rounds of weight pieces");
     static_assert((BT * 8) % TH == 0 || BT * 8 < TH, "whole rounds of token pieces");
     static_assert((BT * 4) % TH == 0 || BT * 4 < TH, "whole rounds of token scales");
 
@@ -147,39 +171,43 @@ __global__ __launch_bounds__(64 * WR * WT, WPS) void gemm_q8_0_x86_kernel(RmiGem
     for (int i = 0; i < 16; i++) zero[i] = 0.0f;
     struct Frags {
         u32x4 a[NR], b[NT];
-        f32x4v wd[NR];
-        float xd[NT];
     };
-    auto read = [&](Frags &f, const uint8_t *base, int b) {
+    const uint8_t *const read_a = lds + (wr + fr) * 64 + g * 16, *const read_b = lds + 4 * TL::ABLK + (wt + fr) * 64 + g * 16;
+    auto read = [&](Frags &f, uint32_t buf, int b) {
 #pragma unroll
-        for (int i = 0; i < NR; i++) f.a[i] = *reinterpret_cast<const u32x4 *>(base + b * TL::ABLK + (wr + i * 16 + fr) * 64 + g * 16);
+        for (int i = 0; i < NR; i++) f.a[i] = *reinterpret_cast<const u32x4 *>(read_a + buf + (b * TL::ABLK + i * 1024));
 #pragma unroll
-        for (int j = 0; j < NT; j++) f.b[j] = *reinterpret_cast<const u32x4 *>(base + 4 * TL::ABLK + b * TL::BBLK + (wt + j * 16 + fr) * 64 + g * 16);
+        for (int j = 0; j < NT; j++) f.b[j] = *reinterpret_cast<const u32x4 *>(read_b + buf + (b * TL::BBLK + j * 1024));
     };
-    auto read_scales = [&](Frags &f, const uint8_t *base, int b) {
-#pragma unroll
-        for (int i = 0; i < NR; i++) f.wd[i] = *reinterpret_cast<const f32x4v *>(base + kScaleA + (b * BN + wr + i * 16 + g * 4) * 4);
-#pragma unroll
-        for (int j = 0; j < NT; j++) f.xd[j] = *reinterpret_cast<const float *>(base + kScaleB + (b * BT + wt + j * 16 + fr) * 4);
+    // The scale products: outer products of sixteen rows and sixteen tokens, four of them an instruction (four tiles of a block,
+    // or a tile's four blocks), in the layout of the dots.
+    constexpr bool BY_TILE = NR * NT == 4;
+    auto sc_a = [&](uint32_t t) { return lds + (kScaleA + wr * 8) + ((t & 15) * 8 + (BY_TILE ? (t >> 5 & 1) * 128 : (t >> 4 & 3) * 2)); };
+    auto sc_b = [&](uint32_t t) { return lds + (kScaleB + wt * 8) + ((t & 15) * 8 + (BY_TILE ? (t >> 4 & 1) * 128 : (t >> 4 & 3) * 2)); };
+    auto outer = [&](u32x2 a, u32x2 b) { return __builtin_amdgcn_mfma_f32_16x16x4f16(__builtin_bit_cast(f16x4, a), __builtin_bit_cast(f16x4, b), zero, 0, 0, 0); };
+    // the weights' scale alone in its k slot, zero against all others (the tokens' are finite)
+    auto scales_by_tile = [&](u32x2 wd, u32x2 xd, int blk) {
+        return outer(u32x2{blk < 2 ? wd[0] & (blk & 1 ? 0xffff0000u : 0xffffu) : 0u, blk < 2 ? 0u : wd[1] & (blk & 1 ? 0xffff0000u : 0xffffu)}, xd);
     };
     // A block's products, one ahead of the sums.  The empty statements hold that order: left to itself the compiler issues
     // every product of a quad first and spills the results, or each right in front of its sums and waits for it.  They hold
     // no instruction, so the wait states between a product and its first reader stay the compiler's own (it counts them on
     // the finished code, past such a statement; tests/test_build_checks.py pins that).
-#define X86_SUMS(c) "+v"(c[0][h]), "+v"(c[0][2 + h]), "+v"(c[0][4 + h]), "+v"(c[0][6 + h]), "+v"(c[1][h]), "+v"(c[1][2 + h]), \
-                    "+v"(c[1][4 + h]), "+v"(c[1][6 + h]), "+v"(c[2][h]), "+v"(c[2][2 + h]), "+v"(c[2][4 + h]), "+v"(c[2][6 + h]), \
-                    "+v"(c[3][h]), "+v"(c[3][2 + h]), "+v"(c[3][4 + h]), "+v"(c[3][6 + h])
+#define X86_SUM(v, beta) "+v"(c[v][2 * (beta) + h])
+#define X86_SUMS(c) X86_SUM(0, 0), X86_SUM(0, 1), X86_SUM(0, 2), X86_SUM(0, 3), X86_SUM(1, 0), X86_SUM(1, 1), X86_SUM(1, 2), X86_SUM(1, 3), \
+                    X86_SUM(2, 0), X86_SUM(2, 1), X86_SUM(2, 2), X86_SUM(2, 3), X86_SUM(3, 0), X86_SUM(3, 1), X86_SUM(3, 2), X86_SUM(3, 3)
+    constexpr int kSteps = 2 * NR * NT;
     auto product = [&](const Frags &f, int s) {
         const u32x4 a = f.a[(s >> 1) / NT], b = f.b[(s >> 1) % NT];
         const u32x2 pa = s & 1 ? u32x2{a[2], a[3]} : u32x2{a[0], a[1]}, pb = s & 1 ? u32x2{b[2], b[3]} : u32x2{b[0], b[1]};
         return __builtin_amdgcn_mfma_f32_16x16x4f16(__builtin_bit_cast(f16x4, pa), __builtin_bit_cast(f16x4, pb), zero, 0, 0, 0);
     };
-    constexpr int kSteps = 2 * NR * NT;
-    // d: the first product of f; returns the first one of `after`, the block behind it (nullptr: none)
-    auto block = [&](const Frags &f, const Frags *after, f32x16 d) {
+    // d: the first product of f; returns the first one of `after`, the block behind it (nullptr: none).  sc: the scale products,
+    // this block's from sc[4 blk] on or its tiles'
+    auto block = [&](const Frags &f, const Frags *after, f32x16 d, const f32x16 &sc, int blk) {
 #pragma unroll
         for (int s = 0; s < kSteps; s++) {
-            const int h = s & 1, i = (s >> 1) / NT, j = (s >> 1) % NT;
+            const int h = s & 1, i = (s >> 1) / NT, j = (s >> 1) % NT, at = 4 * (BY_TILE ? i * NT + j : blk);
             auto &c = acc[i][j];
             f32x16 next = d;
             if (s + 1 < kSteps || after) {
@@ -187,15 +215,33 @@ __global__ __launch_bounds__(64 * WR * WT, WPS) void gemm_q8_0_x86_kernel(RmiGem
                 asm volatile("" : "+v"(next), X86_SUMS(c));
             }
 #pragma unroll
-            for (int v = 0; v < 4; v++) {
-                const float sc = f.wd[i][v] * f.xd[j];
+            for (int v = 0; v < 4; v++)
 #pragma unroll
-                for (int beta = 0; beta < 4; beta++) c[v][2 * beta + h] = __builtin_fmaf(sc, d[4 * beta + v], c[v][2 * beta + h]);
-            }
+                for (int beta = 0; beta < 4; beta++) c[v][2 * beta + h] = __builtin_fmaf(sc[at + v], d[4 * beta + v], c[v][2 * beta + h]);
             asm volatile("" : X86_SUMS(c));
             d = next;
         }
         return d;
+    };
+    auto quad = [&](uint32_t buf) {
+        Frags f[4];
+        read(f[0], buf, 0);
+        const uint32_t t = me();
+        f32x16 sc;
+        u32x2 wd, xd;
+        if constexpr (BY_TILE) {
+            wd = *reinterpret_cast<const u32x2 *>(sc_a(t) + buf);
+            xd = *reinterpret_cast<const u32x2 *>(sc_b(t) + buf);
+        } else {
+            sc = outer(u32x2{*reinterpret_cast<const uint16_t *>(sc_a(t) + buf), 0u}, u32x2{*reinterpret_cast<const uint16_t *>(sc_b(t) + buf), 0u});
+        }
+        f32x16 d = product(f[0], 0);
+#pragma unroll
+        for (int b = 0; b < 4; b++) {
+            if (b < 3) read(f[b + 1], buf, b + 1);
+            if constexpr (BY_TILE) sc = scales_by_tile(wd, xd, b);
+            d = block(f[b], b < 3 ? &f[b + 1] : nullptr, d, sc, b);
+        }
     };
 
     load(0);
@@ -204,31 +250,59 @@ __global__ __launch_bounds__(64 * WR * WT, WPS) void gemm_q8_0_x86_kernel(RmiGem
     __syncthreads();
     const uint32_t n_full = nb >> 2;
     for (uint32_t q = 0; q < n_full; q++) {
-        const uint8_t *base = lds + (q & 1) * TL::LDS_BUF;
-        Frags f[4];
-        read(f[0], base, 0);
-        f32x16 d = product(f[0], 0);
-#pragma unroll
-        for (int b = 0; b < 4; b++) {
-            if (b < 3) read(f[b + 1], base, b + 1);
-            if (NR * NT == 4 || b == 0) read_scales(f[b], base, b);  // (the largest tile has no registers for them a block ahead)
-            if (NR * NT < 4 && b < 3) read_scales(f[b + 1], base, b + 1);
-            d = block(f[b], b < 3 ? &f[b + 1] : nullptr, d);
-        }
+        quad((q & 1) * TL::LDS_BUF);
         park((q + 1) & 1);  // (behind the last quad: that quad again, read by nobody)
         load(q + 2);
         __syncthreads();
     }
-    for (uint32_t b = 0; b < (nb & 3); b++) {  // the reference multiplies no others
+    // the rest of a quad (the reference multiplies no others), block by block: where an instruction takes four blocks' scales they
+    // are four times this one's
+    const uint32_t rest = (n_full & 1) * TL::LDS_BUF;
+    for (uint32_t b = 0; b < (nb & 3); b++) {
         Frags f;
-        read(f, lds + (n_full & 1) * TL::LDS_BUF, int(b));
-        read_scales(f, lds + (n_full & 1) * TL::LDS_BUF, int(b));
-        block(f, nullptr, product(f, 0));
+        read(f, rest, int(b));
+        const uint32_t at = rest + b * 2 - (BY_TILE ? 0 : g * 2), t = me();
+        block(f, nullptr, product(f, 0),
+              outer(u32x2{*reinterpret_cast<const uint16_t *>(sc_a(t) + at), 0u}, u32x2{*reinterpret_cast<const uint16_t *>(sc_b(t) + at), 0u}), 0);
     }
 
+    uint32_t again = tid;
+    asm volatile("" : "+v"(again));  // (what follows is not kept through the loop)
+    const uint32_t lane1 = again & 63, fr1 = lane1 & 15, g1 = lane1 >> 4;
+    if (__syncthreads_or(not_f16 != 0)) {
+        // Token scales that are not f16 values: the tile again, block by block straight from memory, with scale products and dots
+        // of the vector ALU.  Slow, and only a caller's own scales get here.
+#pragma unroll
+        for (int i = 0; i < NR; i++)
+#pragma unroll
+            for (int j = 0; j < NT; j++) {
+                const uint32_t row0 = wr + i * 16 + g1 * 4, tok = wt + j * 16 + fr1, tk = tok < last_tok ? tok : last_tok;
+                const uint32_t t = (row0 >> 3) < last_tile ? row0 >> 3 : last_tile;
+                const gptr_u8 wp = w_base + size_t(t) * tile_bytes;
+#pragma unroll
+                for (int v = 0; v < 4; v++)
+#pragma unroll
+                    for (int l = 0; l < 8; l++) acc[i][j][v][l] = 0.0f;
+#pragma unroll 1
+                for (uint32_t b = 0; b < nb; b++) {
+                    const float xd = *(gptr_f32)(xs_base + (size_t(tk) * nb + b) * 4);
+#pragma unroll
+                    for (int v = 0; v < 4; v++) {
+                        const uint32_t r = (row0 & 7) + v;
+                        const float sc = h2f(*(gptr_u16)(wp + (b >> 3) * 128 + r * 16 + (b & 7) * 2)) * xd;
+#pragma unroll
+                        for (int l = 0; l < 8; l++) {
+                            const int wq = int(*(gptr_u32)(wp + p.n_oct * 128 + (b >> 2) * 1024 + r * 128 + l * 16 + (b & 3) * 4));
+                            const int xq = int(*(gptr_u32)(x_base + (size_t(tk) * p.n_in + b * 32 + l * 4)));
+                            acc[i][j][v][l] = __builtin_fmaf(sc, float(__builtin_amdgcn_sdot4(wq, xq, 0, false)), acc[i][j][v][l]);
+                        }
+                    }
+                }
+            }
+    }
 #pragma unroll
     for (int j = 0; j < NT; j++) {
-        const uint32_t tok = tok0 + wt + j * 16 + fr;
+        const uint32_t tok = tok0 + wt + j * 16 + fr1;
         if (tok >= n_tokens) continue;
 #pragma unroll
         for (int i = 0; i < NR; i++) {
@@ -238,7 +312,7 @@ __global__ __launch_bounds__(64 * WR * WT, WPS) void gemm_q8_0_x86_kernel(RmiGem
                 const float *l = acc[i][j][v];
                 y[v] = ((l[0] + l[4]) + (l[1] + l[5])) + ((l[2] + l[6]) + (l[3] + l[7]));
             }
-            const uint32_t row = (p.tile0 + tile0) * 8 + wr + i * 16 + g * 4;
+            const uint32_t row = (p.tile0 + tile0) * 8 + wr + i * 16 + g1 * 4;
             float *dst = p.y + size_t(tok) * p.y_stride + row;
             if (row >= p.row_start && row + 3 < p.row_end && (reinterpret_cast<uintptr_t>(dst) & 15) == 0)
                 *reinterpret_cast<f32x4v *>(dst) = f32x4v{y[0], y[1], y[2], y[3]};
