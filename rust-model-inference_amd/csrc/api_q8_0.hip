@@ -30,13 +30,12 @@ RmiGemvProblem make_problem(const rmi_hip_weight *w, const int8_t *x_q8, const f
     p.row_end = row_end;
     p.tile0 = row_start / kTileRows;
     p.n_tiles = row_end > row_start ? (row_end + kTileRows - 1) / kTileRows - p.tile0 : 0;
-    p.reserved = 0;
     return p;
 }
 
-// tokens per GEMV launch so that the LDS staging fits
-uint32_t gemv_chunk(const rmi_hip_weight *w) {
-    const size_t per_token = size_t(w->n_units) * (w->dtype == RMI_HIP_DTYPE_Q4_0 ? 320 : 288);
+// tokens per Q4_0 GEMV launch so that the LDS staging fits
+uint32_t q4_0_chunk(const rmi_hip_weight *w) {
+    const size_t per_token = size_t(w->n_units) * 320;
     uint32_t c = per_token ? uint32_t((64 * 1024) / per_token) : 8;
     return c > 8 ? 8 : c;
 }
@@ -45,38 +44,34 @@ uint32_t gemv_chunk(const rmi_hip_weight *w) {
 
 // whether rmi_gemv_q8_0_tokens can stage a row of this weight at all (callers that must not enqueue anything
 // before every check has passed ask first)
-bool rmi_gemv_q8_0_tokens_fits(const rmi_hip_weight *w) { return gemv_chunk(w) != 0; }
+bool rmi_gemv_q8_0_tokens_fits(const rmi_hip_weight *w) {
+    return w->dtype == RMI_HIP_DTYPE_Q4_0 ? q4_0_chunk(w) != 0 : rmi_gemv_q8_0_groups(w->n_units, 0, 1).tokens != 0;
+}
 
 // device pointers in, rows [row_start,row_end) of n_tokens tokens
 int rmi_gemv_q8_0_tokens(const rmi_hip_weight *w, const int8_t *x_q8, const float *x_scales, float *y, uint32_t n_tokens,
                          uint32_t y_stride, uint32_t row_start, uint32_t row_end, hipStream_t s) {
-    const uint32_t chunk = gemv_chunk(w);
-    if (chunk == 0) return rmi_fail(RMI_HIP_E_INVALID, "n_in=%u is too long for the GEMV staging", w->n_in);
-    const uint32_t nb = w->n_in / 32;
-    if (w->dtype == RMI_HIP_DTYPE_Q8_0 && row_end > row_start && rmi_gemm_q8_0_x86_wins(row_end - row_start, n_tokens, w->n_in))
-        return rmi_launch_gemm_q8_0_x86(make_problem(w, x_q8, x_scales, y, y_stride, row_start, row_end), n_tokens, s);
-    uint32_t t0 = 0;
-    if (w->dtype != RMI_HIP_DTYPE_Q4_0 && n_tokens >= 2 * chunk) {
-        // every full group of `chunk` tokens in one launch (the groups re-read the weight from L2), up to what a
-        // grid's second dimension holds
-        const uint32_t groups = n_tokens / chunk < 65535 ? n_tokens / chunk : 65535;
-        RmiGemvProblem p = make_problem(w, x_q8, x_scales, y, y_stride, row_start, row_end);
-        int rc = rmi_launch_gemv_q8_0_single(p, chunk, s, groups);
-        if (rc != RMI_HIP_OK) return rc;
-        t0 = groups * chunk;
-    }
-    for (; t0 < n_tokens; t0 += chunk) {
-        uint32_t nt = n_tokens - t0 < chunk ? n_tokens - t0 : chunk;
-        const bool small = uint64_t(row_end - row_start) * w->n_in <= (4u << 20);
-        if (w->dtype != RMI_HIP_DTYPE_Q4_0 && chunk == 8 && t0 >= 8 && (nt == 5 || nt == 7 || ((nt == 3 || nt == 6) && small))) {
-            // behind whole groups: a whole group again, which is spread over workgroups as these numbers are not (some tokens
-            // are computed twice, to the same bits; 1024 x 3072, 13 tokens: 18.1 -> 14.4 us, 6112 x 6174: 44 -> 39)
-            t0 = n_tokens - 8;
-            nt = 8;
+    if (!rmi_gemv_q8_0_tokens_fits(w)) return rmi_fail(RMI_HIP_E_INVALID, "n_in=%u is too long for the GEMV staging", w->n_in);
+    if (n_tokens == 0) return RMI_HIP_OK;
+    const uint32_t nb = w->n_in / 32, n_rows = row_end > row_start ? row_end - row_start : 0;
+    auto problem_at = [&](uint32_t t0) {
+        return make_problem(w, x_q8 + size_t(t0) * w->n_in, x_scales + size_t(t0) * nb, y + size_t(t0) * y_stride, y_stride, row_start, row_end);
+    };
+    if (w->dtype == RMI_HIP_DTYPE_Q4_0) {
+        const uint32_t chunk = q4_0_chunk(w);
+        for (uint32_t t0 = 0; t0 < n_tokens; t0 += chunk) {
+            const int rc = rmi_launch_gemv_q4_0(problem_at(t0), n_tokens - t0 < chunk ? n_tokens - t0 : chunk, s);
+            if (rc != RMI_HIP_OK) return rc;
         }
-        RmiGemvProblem p = make_problem(w, x_q8 + size_t(t0) * w->n_in, x_scales + size_t(t0) * nb,
-                                        y + size_t(t0) * y_stride, y_stride, row_start, row_end);
-        int rc = w->dtype == RMI_HIP_DTYPE_Q4_0 ? rmi_launch_gemv_q4_0(p, nt, s) : rmi_launch_gemv_q8_0_single(p, nt, s);
+        return RMI_HIP_OK;
+    }
+    if (n_rows && rmi_gemm_q8_0_x86_wins(n_rows, n_tokens, w->n_in)) return rmi_launch_gemm_q8_0_x86(problem_at(0), n_tokens, s);
+    const RmiTokenGroups g = rmi_gemv_q8_0_groups(w->n_units, uint64_t(n_rows) * w->n_in, n_tokens);
+    const uint32_t together = n_tokens - g.apart, most = 65535 * g.tokens;  // a grid's second dimension
+    for (uint32_t t0 = 0, n; t0 < n_tokens; t0 += n) {
+        n = (t0 < together ? together : n_tokens) - t0;
+        n = n < most ? n : most;
+        const int rc = rmi_launch_gemv_q8_0_single(problem_at(t0), n < g.tokens ? n : g.tokens, s, n);
         if (rc != RMI_HIP_OK) return rc;
     }
     return RMI_HIP_OK;
@@ -220,8 +215,8 @@ static int forward_batched(const rmi_hip_weight *w, const float *input, float *o
     if (!c) return RMI_HIP_E_RUNTIME;
     const size_t n_x = size_t(n_tokens) * n_in;
     const size_t x_bytes = n_x * 4, y_bytes = size_t(n_tokens) * n_out * 4;
-    // The quantizer reads every input once, and the x86-64-order products only write results and never read them back (of the
-    // tokens behind whole groups of eight, up to five are written twice, with the same bits), so both may use the pinned
+    // The quantizer reads every input once, and the x86-64-order products only write results and never read them back (those of
+    // up to seven tokens are written twice, with the same bits), so both may use the pinned
     // buffers themselves: a copy command less on either side, each of which is 5 to 8 us between dependent kernels.  From some
     // 700 KB on the copy is the faster reader.  us with copies | x in place | y in place | both: 2048 x 6144, 1 token 31.5 | 28.5 |
     // 22.4 | 20.4, 13 tokens 60.9 | 54.9 | 53.0 | 45.5, 100 tokens (800 KB) 209.0 | 211.1 | 200.3 | 202.6; 8192 x 3000, 300 tokens

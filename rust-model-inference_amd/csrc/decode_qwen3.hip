@@ -1282,7 +1282,7 @@ int gemv(const rmi_hip_weight *w, const int8_t *q8, const float *scales, float *
     p.row_end = w->n_out;
     p.tile0 = 0;
     p.n_tiles = w->n_tiles;
-    return rmi_launch_gemv_q8_0_single(p, 1, st);
+    return rmi_launch_gemv_q8_0_single(p, 1, st, 1);
 }
 
 // One decoder step at position `step` (the host's copy of the counter in HBM, which the last kernel advances).

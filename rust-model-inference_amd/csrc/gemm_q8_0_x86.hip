@@ -23,6 +23,8 @@
 // the scale products on the vector ALU | as it is: 64 x 64 tiles, 6144 x 1024, 1024 tokens 70.8 | 68.5, 151936 x 1024, 128
 // tokens 213 | 207; 32 x 32 tiles, 1024 x 3072, 512 tokens 26.3 | 25.0, 1024 x 2048, 512 tokens 19.5 | 18.4.
 // Eight tokens to a workgroup of the GEMV with int8 dots (4 x 4 x 4) and a conversion each: 151936 x 1024, 128 tokens 529.
+#include <cmath>
+
 #include "rmi_internal.h"
 
 #include "device_common.h"
@@ -340,31 +342,34 @@ int launch(const RmiGemvProblem &p, uint32_t n_tokens, hipStream_t s) {
     return RMI_HIP_OK;
 }
 
-// Which tile a product takes, or none (the GEMV's launches of up to eight tokens are faster): microseconds estimated from
-// what one block of k costs a compute unit that holds w workgroups of a tile, measured on 37..151936 rows of 32..6400
-// columns with 9..1000 tokens.  64 x 64: 0.43 alone, 0.71 for two (two fit); 32 x 32: 0.17, 0.25, 0.33, 0.41 for one to four
-// (four fit); 64 x 16: 0.19, 0.25, 0.38 (three fit).  The GEMV: 85 TOP/s on short rows, 45 at 6400 columns, behind 4.5 us a
-// launch; tokens beyond whole groups of eight are a launch of their own, which reads the weight again.
-// (E.g. 4096 x 1024: 16 tokens 6.6 us there, 8.3 here; 128: 16.7 and 11.4; 512: 53 and 28.  1024 x 3072: 64 tokens 15 and
-// 20 us, 512: 38 and 27.  151936 x 1024, 128 tokens: 529 and 231.)
+// Which tile a product takes, or none (the GEMV's token groups are faster): microseconds estimated from what was measured on
+// 500..151936 rows of 256..12288 columns with 9..1000 tokens (812 products; the choice is 0.4 % over the best in the mean).
+// Tiles: what one block of k costs a compute unit that holds w workgroups: 64 x 64 0.43 alone, 0.73 for two (two fit), 32 x 32
+// 0.16, 0.22, 0.32, 0.42 for one to four (four fit), 64 x 16 0.19, 0.26, 0.38 (three).  The GEMV: a wave's walk along a row
+// beside the vector ALU's work for all groups' tokens, their workgroups and the weights, which only groups of long rows read from
+// beyond L2 each.
+// (E.g. 4096 x 1024: 16 tokens 5.1 us there, 8.0 here; 64: 8.4 and 8.1; 512: 53 and 28.  1024 x 3072: 64 tokens 14.4 and 18.3,
+// 512: 38 and 25.  151936 x 1024, 128 tokens: 529 and 208.)
 enum X86Plan { kPlanGemv, kPlan64x64, kPlan32x32, kPlan64x16 };
 X86Plan plan(uint32_t n_rows, uint32_t n_tokens, uint32_t n_in) {
-    const double cus = rmi_device_cus() > 0 ? rmi_device_cus() : 1, nb = n_in / 32;
-    auto estimate = [&](uint32_t bn, uint32_t bt, const double *us, int fit) {
+    if (n_tokens <= 8) return kPlanGemv;
+    const double cus = rmi_device_cus() > 0 ? rmi_device_cus() : 1, nb = n_in / 32, weights = double(n_rows) * n_in;
+    auto estimate = [&](double fixed, uint32_t bn, uint32_t bt, const double *us, int fit) {
         const double groups = double((n_rows + bn - 1) / bn) * ((n_tokens + bt - 1) / bt);
         const uint64_t w = uint64_t((groups + cus - 1) / cus);
-        return 3.2 + nb * (double(w / fit) * us[fit - 1] + (w % fit ? us[w % fit - 1] : 0.0));
+        return fixed + nb * (double(w / fit) * us[fit - 1] + (w % fit ? us[w % fit - 1] : 0.0));
     };
-    const uint32_t rest = n_tokens % 8;
-    const double rate = 85e6 / (1.0 + (n_in > 2048 ? n_in - 2048 : 0) / 8000.0), macs = double(n_rows) * n_in;
-    // (five and seven beyond whole groups cost what eight do)
-    const bool whole = rest == 5 || rest == 7;
-    const double gemv = 4.5 + 2.0 * macs * (n_tokens - rest) / rate +
-                        (rest == 0 ? 0.0 : rest == 1 ? 2.5 + macs / 6e6 : 4.5 + (whole ? 0.04 : 0.02) * nb + macs / 12e6 + 2.0 * macs * (whole ? 8 : rest) / rate);
-    const double k64[] = {0.43, 0.71}, k32[] = {0.17, 0.25, 0.33, 0.41}, k16[] = {0.19, 0.25, 0.38};
-    const double t64 = estimate(64, 64, k64, 2), t32 = estimate(32, 32, k32, 4), t16 = n_tokens <= 16 ? estimate(64, 16, k16, 3) : 1e30;
+    const uint32_t n_oct = (n_in + 255) / 256;
+    const RmiTokenGroups g = rmi_gemv_q8_0_groups(n_oct, uint64_t(n_rows) * n_in, n_tokens);
+    if (g.tokens == 0) return kPlan32x32;  // rows too long for the GEMV's staging
+    const bool x4 = g.tokens == 8 || g.tokens == 4;
+    const double work = (x4 ? 0.0222 : 0.0322) * 1e-6 * weights * (g.groups * g.tokens + g.apart) + 0.0275e-3 * n_rows * g.groups,
+                 memory = 0.0232e-6 * weights * (g.tokens == 8 ? 1 : g.groups);
+    const double gemv = 2.7 + std::pow(std::pow(0.363 * n_oct, 1.5) + std::pow(work + memory, 1.5), 2.0 / 3) + (g.apart ? 19.7 + 0.0232e-6 * weights : 0.0);
+    const double k64[] = {0.43, 0.73}, k32[] = {0.163, 0.224, 0.317, 0.42}, k16[] = {0.186, 0.264, 0.377};
+    const double t64 = estimate(3.6, 64, 64, k64, 2), t32 = estimate(3.0, 32, 32, k32, 4), t16 = n_tokens <= 16 ? estimate(3.1, 64, 16, k16, 3) : 1e30;
     const double best = t64 < t32 ? (t64 < t16 ? t64 : t16) : (t32 < t16 ? t32 : t16);
-    if (n_tokens <= 8 || gemv < best) return kPlanGemv;
+    if (gemv < best) return kPlanGemv;
     return best == t64 ? kPlan64x64 : best == t32 ? kPlan32x32 : kPlan64x16;
 }
 

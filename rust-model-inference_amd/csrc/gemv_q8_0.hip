@@ -306,6 +306,16 @@ __device__ __forceinline__ void factors_sum(float &acc, const float4 *src) {
     }
 }
 
+// A launch may spread its tokens over workgroups, gridDim.y groups of B tokens: the problem of the group blockIdx.y, the last one
+// of which begins early enough to have B.
+template <int B>
+__device__ __forceinline__ void to_token_group(RmiGemvProblem &p) {
+    const uint32_t at = blockIdx.y * B, last = p.n_tokens - B, t0 = blockIdx.y == 0 || at < last ? at : last;
+    p.x_q8 += size_t(t0) * p.n_in;
+    p.x_scales += size_t(t0) * (p.n_in >> 5);
+    p.y += size_t(t0) * p.y_stride;
+}
+
 // A wave owns a short run of consecutive 8-row tiles of ONE matrix (about 34 KiB of
 // weights) and walks it four octets deep (device_run_ring.h).  A launch has far more
 // waves than fit on the chip at once: the dispatcher hands out runs as waves retire,
@@ -334,10 +344,7 @@ __global__ __launch_bounds__(MAXT) void gemv_q8_0_kernel(RmiGemvProblem single,
         k_end = run.y + run.z;
     } else {
         p = single;
-        // a launch may spread its tokens over workgroups (gridDim.y groups of B tokens each): the group's B tokens
-        p.x_q8 += size_t(blockIdx.y) * B * p.n_in;
-        p.x_scales += size_t(blockIdx.y) * B * (p.n_in >> 5);
-        p.y += size_t(blockIdx.y) * B * p.y_stride;
+        to_token_group<B>(p);
         k = w_idx * tiles_per_wave < p.n_tiles ? w_idx * tiles_per_wave : p.n_tiles;
         k_end = k + tiles_per_wave < p.n_tiles ? k + tiles_per_wave : p.n_tiles;
     }
@@ -528,9 +535,7 @@ __global__ __launch_bounds__(MAXT, kX4WavesPerSimd) void gemv_q8_0_x4_kernel(Rmi
         k_end = run.y + run.z;
     } else {
         p = single;
-        p.x_q8 += size_t(blockIdx.y) * B * p.n_in;  // token group blockIdx.y of the launch
-        p.x_scales += size_t(blockIdx.y) * B * (p.n_in >> 5);
-        p.y += size_t(blockIdx.y) * B * p.y_stride;
+        to_token_group<B>(p);
         k = w_idx * tiles_per_wave < p.n_tiles ? w_idx * tiles_per_wave : p.n_tiles;
         k_end = k + tiles_per_wave < p.n_tiles ? k + tiles_per_wave : p.n_tiles;
     }
@@ -1214,6 +1219,11 @@ int dispatch_gemv_deep(const RmiGemvProblem &p, hipStream_t s) {
     }
 }
 
+// what the kernel with its dots on the matrix cores takes of LDS: the staged tokens, and behind them what its waves park
+size_t gemv_x4_bytes(uint32_t n_tokens, uint32_t n_oct, uint32_t wpg) {
+    return size_t(n_tokens) * rmi_gemv_x4_token_u4(n_oct) * 16 + size_t(wpg) * kX4WaveFloats(n_tokens) * 4;
+}
+
 template <int B>
 int launch_gemv(const RmiGemvProblem *single, const RmiGemvProblem *d_list, const uint4 *d_runs, uint32_t n_waves,
                 uint32_t wpg,
@@ -1226,7 +1236,7 @@ int launch_gemv(const RmiGemvProblem *single, const RmiGemvProblem *d_list, cons
     if constexpr (B >= 4) {
         // the kernel with the dots on the matrix cores, where its staging fits (its tokens lie further apart, and its
         // waves park finished tiles behind them)
-        const size_t x4_bytes = size_t(B) * rmi_gemv_x4_token_u4(max_n_oct) * 16 + size_t(wpg) * kX4WaveFloats(B) * 4;
+        const size_t x4_bytes = gemv_x4_bytes(B, max_n_oct, wpg);
         if (x4_bytes <= 64 * 1024) {
             lds_bytes = x4_bytes;
             if (single && wpg == 1)
@@ -1415,21 +1425,51 @@ int rmi_launch_copy(const void *src, void *dst, size_t nbytes, hipStream_t s) {
     return RMI_HIP_OK;
 }
 
-// token_groups groups of n_tokens tokens each (n_tokens <= 8), consecutive in x_q8, x_scales and y, in one launch
-int rmi_launch_gemv_q8_0_single(const RmiGemvProblem &p, uint32_t n_tokens, hipStream_t s, uint32_t token_groups) {
-    if (p.n_tiles == 0 || p.n_oct == 0 || token_groups == 0) return RMI_HIP_OK;
-    if (n_tokens == 1 && token_groups == 1 && p.n_oct <= kDeepMaxOct && p.n_tiles <= kDeepMaxTiles) return dispatch_gemv_deep(p, s);
-    const uint32_t tpw = rmi_gemv_tiles_per_wave(p.n_oct, p.n_tiles, n_tokens);
+// All groups go out in one launch (they re-read the weight from L2): a launch behind it for what is beyond whole groups takes as
+// long as the groups together (1024 x 3072: 13 tokens 13.4 us as 8 and 8, 7.4 as one launch; 9 tokens 9.2 as 8 and 1, 7.3).
+// A group is eight tokens where the kernel with its dots on the matrix cores can stage them; four where that leaves out a group's
+// half (up to 28 tokens: 4096 x 4096, 9 tokens 11.8 us by fours, 18.4 by eights, 18 tokens 13.7 | 19.0; from 32 on level), and
+// on longer rows, for the kernel that can stage more there is twice to three times as slow (8192 columns, 8 tokens, by fours |
+// by what fits: 1024 rows 14.4 | 40.7, 4096 rows 20.8 | 38.2; 5 tokens 14.6 | 25.5 and 20.8 | 23.5).  Of a large matrix, where a
+// group more costs as much as the matrix again, neither, but for eight tokens of a long row (12288 x 8192: 8 tokens 33.6 | 55.0,
+// 5 tokens 40.1 | 31.5, 13 tokens 68 | 52), and there up to half a group is a launch of its own (151936 x 1024, 9 tokens 67 us
+// and 76 as two groups, 20 tokens 104 and 110; one token more on long rows: 4096 x 12288, 9 tokens 42 and 49).
+RmiTokenGroups rmi_gemv_q8_0_groups(uint32_t n_oct, uint64_t weights, uint32_t n_tokens) {
+    constexpr size_t kLds = 64 * 1024;
+    constexpr uint64_t kLarge = 64u << 20, kLong = 36u << 20;
+    const bool rows_fit = gemv_x4_bytes(8, n_oct, 4) <= kLds, large = weights >= kLarge;
+    RmiTokenGroups g{8, 0, 0};
+    if (rows_fit) {
+        if (!large && n_tokens > 8 && n_tokens <= 28 && (n_tokens - 1) % 8 < 4) g.tokens = 4;
+    } else {
+        const uint32_t fit = uint32_t(kLds / (size_t(n_oct) * 288));
+        const bool fours = !large || n_tokens == 8 || (n_tokens > fit && n_tokens < 8);
+        g.tokens = fours && gemv_x4_bytes(4, n_oct, 4) <= kLds ? 4 : fit < 8 ? fit : 8;
+        if (g.tokens == 0) return g;
+    }
+    if (n_tokens < g.tokens) g.tokens = n_tokens;
+    const uint32_t rest = n_tokens % g.tokens;
+    if (n_tokens > g.tokens && (large ? rest <= g.tokens / 2 : !rows_fit && rest == 1 && weights >= kLong)) g.apart = rest;
+    g.groups = (n_tokens - g.apart + g.tokens - 1) / g.tokens;
+    return g;
+}
+
+int rmi_launch_gemv_q8_0_single(const RmiGemvProblem &problem, uint32_t group, hipStream_t s, uint32_t n_tokens) {
+    if (problem.n_tiles == 0 || problem.n_oct == 0 || n_tokens == 0) return RMI_HIP_OK;
+    RmiGemvProblem p = problem;
+    p.n_tokens = n_tokens;
+    if (n_tokens == 1 && p.n_oct <= kDeepMaxOct && p.n_tiles <= kDeepMaxTiles) return dispatch_gemv_deep(p, s);
+    const uint32_t tpw = rmi_gemv_tiles_per_wave(p.n_oct, p.n_tiles, group);
     const uint32_t n_waves = (p.n_tiles + tpw - 1) / tpw, cus = uint32_t(rmi_device_cus() > 0 ? rmi_device_cus() : 1);
     {
         // A matrix of a few MB at several tokens is a launch of a few hundred waves with a long instruction stream
         // each (the x86-64 order costs about 30 vector instructions a token and octet): its tokens are spread over
         // workgroups, two or four to each, which re-read the weight from L2 and finish in a half or a quarter of
         // the time (every token's result is that of any other grouping: a token has its own accumulators).
-        uint32_t per_group = n_tokens, groups = token_groups;
-        while (per_group > 2 && per_group % 2 == 0 && n_waves * groups < 4 * cus) {
+        uint32_t per_group = group, groups = (n_tokens + group - 1) / group;
+        while (per_group > 2 && per_group % 2 == 0 && n_waves * groups < (per_group == 8 ? 8 : 4) * cus) {
             per_group >>= 1;
-            groups <<= 1;
+            groups = (n_tokens + per_group - 1) / per_group;
         }
         if (groups > 1) {
             // the waves of a workgroup share the staged tokens of their group: as many as leave every compute unit
@@ -1440,12 +1480,12 @@ int rmi_launch_gemv_q8_0_single(const RmiGemvProblem &p, uint32_t n_tokens, hipS
             return dispatch_gemv(per_group, &p, nullptr, nullptr, n_waves, wpg, tpw, p.n_oct, s, groups);
         }
     }
-    uint32_t wpg = rmi_gemv_waves_per_group(size_t(n_tokens) * p.n_oct * 288, size_t(tpw) * p.n_oct * kOctetBytes);
-    if (n_tokens >= 4 && wpg > 4) wpg = 4;
+    uint32_t wpg = rmi_gemv_waves_per_group(size_t(group) * p.n_oct * 288, size_t(tpw) * p.n_oct * kOctetBytes);
+    if (group >= 4 && wpg > 4) wpg = 4;
     // a launch with fewer waves than would give every compute unit a workgroup of that size is bound by latency,
     // not by the staging it shares: smaller workgroups on more compute units
     while (wpg > 1 && n_waves / wpg < cus) wpg >>= 1;
-    return dispatch_gemv(n_tokens, &p, nullptr, nullptr, n_waves, wpg, tpw, p.n_oct, s);
+    return dispatch_gemv(group, &p, nullptr, nullptr, n_waves, wpg, tpw, p.n_oct, s);
 }
 
 bool rmi_gemv_q8_0_norm_fusable(const rmi_hip_weight *w) {

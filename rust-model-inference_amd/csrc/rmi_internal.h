@@ -174,10 +174,17 @@ struct RmiGemvProblem {
     uint32_t row_end;
     uint32_t tile0;        // first tile touched
     uint32_t n_tiles;      // tiles touched
-    uint32_t reserved;
+    uint32_t n_tokens;     // of a launch over token groups of B: group g begins at token min(g B, n_tokens - B)
 };
-// token_groups groups of n_tokens (<= 8) tokens each, consecutive in the problem's arrays, in one launch
-int rmi_launch_gemv_q8_0_single(const RmiGemvProblem &p, uint32_t n_tokens, hipStream_t s, uint32_t token_groups = 1);
+// n_tokens tokens in one launch, in groups of `group` (<= 8, <= n_tokens) or fewer; where they don't come out even the last group
+// begins earlier, and what two groups share is written twice, with the same bits
+int rmi_launch_gemv_q8_0_single(const RmiGemvProblem &p, uint32_t group, hipStream_t s, uint32_t n_tokens);
+// how n_tokens (> 0) tokens of a matrix of that many weights are grouped; tokens = 0: not even one's activation fits the staging
+struct RmiTokenGroups {
+    uint32_t tokens, groups;  // of a group; of one launch
+    uint32_t apart;           // the last ones, in a launch of their own
+};
+RmiTokenGroups rmi_gemv_q8_0_groups(uint32_t n_oct, uint64_t weights, uint32_t n_tokens);
 // any number of tokens in one launch, the same bits (gemm_q8_0_x86.hip), and whether that is the faster way
 bool rmi_gemm_q8_0_x86_wins(uint32_t n_rows, uint32_t n_tokens, uint32_t n_in);
 int rmi_launch_gemm_q8_0_x86(const RmiGemvProblem &p, uint32_t n_tokens, hipStream_t s);

@@ -1,5 +1,6 @@
-"""Products of several tokens in the x86-64 order (matmul_q8_0_vs_q8_0_avx2, src/ops/kernel/q8_0/avx2.rs:71-173): the tiles of
-the matrix cores with token scales that are not f16 values.  Every output has the bits of the checker's AVX2 order."""
+"""Products of several tokens in the x86-64 order (matmul_q8_0_vs_q8_0_avx2, src/ops/kernel/q8_0/avx2.rs:71-173): the GEMV's
+token groups, of eight and of four, whole, ragged (the last group begins earlier) and with a launch behind them, and the tiles
+of the matrix cores with token scales that are not f16 values.  Every output has the bits of the checker's AVX2 order."""
 import numpy as np
 import pytest
 
@@ -27,6 +28,33 @@ def _run(hip, w, q8, sc, n_out, n_in, r0, r1, stride):
     got = d_y.to_array(np.float32, (n_tokens, stride))
     assert np.all(got[:, :r0] == -3.75) and np.all(got[:, r1:] == -3.75), "outside the row range"
     return got[:, r0:r1]
+
+
+# rows of 1024 and 1056 columns are staged by eights, 7424 and 12288 by fours; 9..12 and 17..20 tokens go by fours on any row
+@pytest.mark.parametrize("n_in", [256, 1056, 7424, 12288])
+@pytest.mark.parametrize("n_tokens", [4, 5, 7, 8, 9, 12, 13, 16, 17, 23, 28, 29])
+def test_token_groups(hip, oracle, n_tokens, n_in):
+    n_out = 8 * 5 + 3
+    w = hip.synth.q8_0_weight(n_in + n_tokens, n_out, n_in)
+    q8, sc = _activation(hip, oracle, 60 + n_tokens, n_tokens, n_in)
+    for r0, r1, stride in ((0, n_out, n_out), (3, 30, n_out + 5)):
+        got = _run(hip, w, q8, sc, n_out, n_in, r0, r1, stride)
+        for t in range(n_tokens):
+            ref = oracle.matmul_q8_0_quantized(w, q8[t], sc[t], n_in, n_out, A)[r0:r1]
+            assert np.array_equal(bits(got[t]), bits(ref)), (t, r0)
+
+
+@pytest.mark.parametrize("n_in,n_tokens", [(1024, 9), (1024, 20), (8192, 5), (8192, 8), (8192, 9)])
+def test_large_matrix(hip, oracle, n_tokens, n_in):
+    """From 64 M weights on the tokens beyond whole groups are a launch of their own, and long rows take larger groups."""
+    n_out = (64 << 20) // n_in + 8
+    w = hip.synth.q8_0_weight(3, n_out, n_in)
+    q8, sc = _activation(hip, oracle, 90 + n_tokens, n_tokens, n_in)
+    got = _run(hip, w, q8, sc, n_out, n_in, 0, n_out, n_out)
+    rows = np.unique(np.concatenate([np.arange(16), np.arange(n_out - 16, n_out), np.random.default_rng(1).integers(0, n_out, 200)]))
+    wr = np.ascontiguousarray(w.reshape(n_out, -1)[rows]).reshape(-1)
+    for t in range(n_tokens):
+        assert np.array_equal(bits(got[t, rows]), bits(oracle.matmul_q8_0_quantized(wr, q8[t], sc[t], n_in, rows.size, A))), t
 
 
 # tiles of 64 x 16, of 32 x 32 and of 64 x 64, each with ragged edges, one of them with blocks beyond whole quads
