@@ -117,6 +117,8 @@ struct RmiEmbed {
     float *x, *x_also;
 };
 int rmi_dense_embed(uint32_t elem_bytes, const RmiEmbed &e, const uint32_t *tok, uint32_t pos0, uint32_t n_tokens, hipStream_t st);
+// one token that the host knows: it travels with the launch, which leaves it in *tok for those behind it
+int rmi_dense_embed_token(uint32_t elem_bytes, const RmiEmbed &e, uint32_t token, uint32_t *tok, uint32_t pos, hipStream_t st);
 // several tokens: matrix cores; a = [n_tokens] rows of k_pad elements, rmi_dense_ld apart
 int rmi_dense_gemm(uint32_t elem_bytes, const RmiDense &w, const void *a, const RmiRowSegs &segs, uint32_t n_tokens, hipStream_t st);
 int rmi_dense_gemm_residual(uint32_t elem_bytes, const RmiDense &w, const void *a, const RmiColSegs &segs, float *x, uint32_t width,

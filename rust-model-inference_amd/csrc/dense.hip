@@ -22,6 +22,12 @@ __global__ __launch_bounds__(256) void embed_kernel(RmiEmbed e, const uint32_t *
     embed_row<T>(e, tok[blockIdx.x], pos0 + blockIdx.x, blockIdx.x);
 }
 
+template <typename T>
+__global__ __launch_bounds__(256) void embed_token_kernel(RmiEmbed e, uint32_t token, uint32_t *tok, uint32_t pos) {
+    if (threadIdx.x == 0) *tok = token;
+    embed_row<T>(e, token, pos, 0);
+}
+
 // ------------------------------------------------------------------ GEMM
 // Weights are the A operand: a lane ends with four consecutive rows of one token.  k goes in steps of 128 bytes a row
 // through LDS; a row of a buffer is eight 16-byte pieces, piece p at slot p ^ (row & 7), so that the sixteen rows of a
@@ -660,6 +666,15 @@ int rmi_dense_embed(uint32_t elem_bytes, const RmiEmbed &e, const uint32_t *tok,
         hipLaunchKernelGGL(embed_kernel<rmi_bf16>, dim3(n_tokens), dim3(256), 0, st, e, tok, pos0);
     else
         hipLaunchKernelGGL(embed_kernel<float>, dim3(n_tokens), dim3(256), 0, st, e, tok, pos0);
+    RMI_HIP_CHECK(hipGetLastError());
+    return RMI_HIP_OK;
+}
+
+int rmi_dense_embed_token(uint32_t elem_bytes, const RmiEmbed &e, uint32_t token, uint32_t *tok, uint32_t pos, hipStream_t st) {
+    if (elem_bytes == 2)
+        hipLaunchKernelGGL(embed_token_kernel<rmi_bf16>, dim3(1), dim3(256), 0, st, e, token, tok, pos);
+    else
+        hipLaunchKernelGGL(embed_token_kernel<float>, dim3(1), dim3(256), 0, st, e, token, tok, pos);
     RMI_HIP_CHECK(hipGetLastError());
     return RMI_HIP_OK;
 }
