@@ -230,6 +230,12 @@ __global__ __launch_bounds__(256) void conv_rotate_pairs_kernel(RmiAttnShape s, 
     }
 }
 
+// p + bytes: a uniform pointer and 32 bits of a lane's own, which an access takes as they are
+template <typename P>
+__device__ __forceinline__ const P *at_bytes(const P *p, uint32_t bytes) {
+    return reinterpret_cast<const P *>(reinterpret_cast<const uint8_t *>(p) + bytes);
+}
+
 // ---- attention.  The columns of a key/value head are its pass's (token, query head of the group) pairs, token by
 // token; a wave takes QT tiles of sixteen.  Scores come as K q (rows: keys, columns: queries), so a lane holds the
 // weights of one column and the running maximum and sum are a lane's own; the weights then are the operand of
@@ -264,7 +270,7 @@ struct AttnWave {
 
     __device__ __forceinline__ void load_keys(const T *kc, const RmiAttnShape &s, uint32_t k) {
         const uint32_t lane = threadIdx.x & 63, n_kc = s.dk_pad / (4 * kPieceElems<T>);
-        const T *row = kc + size_t(k + (lane & 15)) * s.dk_pad + (lane >> 4) * kPieceElems<T>;
+        const T *row = at_bytes(kc + size_t(k) * s.dk_pad, ((lane & 15) * s.dk_pad + (lane >> 4) * kPieceElems<T>) * uint32_t(sizeof(T)));
 #pragma unroll
         for (uint32_t c = 0; c < (kAhead ? kKC : 0); c++) {
             if (skipped(c, n_kc)) continue;
@@ -275,7 +281,7 @@ struct AttnWave {
     }
     __device__ __forceinline__ const T *value_at(const T *vc, const RmiAttnShape &s, uint32_t k) {
         const uint32_t lane = threadIdx.x & 63;
-        return vc + size_t(k / kKeyBlock) * s.dv_pad * kKeyBlock + size_t(lane & 15) * kKeyBlock + (lane >> 4) * kPieceElems<T>;
+        return at_bytes(vc + size_t(k / kKeyBlock) * s.dv_pad * kKeyBlock, ((lane & 15) * kKeyBlock + (lane >> 4) * kPieceElems<T>) * uint32_t(sizeof(T)));
     }
     __device__ __forceinline__ void load_values(const T *vc, const RmiAttnShape &s, uint32_t k) {
         const T *vb = value_at(vc, s, k);
@@ -523,10 +529,21 @@ struct SplitPlan {
     uint32_t keys_per_part, own;  // own: the row of the first token's key
 };
 
-template <typename T, int BUCKET, bool STEP, bool EVERY = true>
-__device__ __forceinline__ void attn_split(const RmiAttnShape &s, const RmiAttnArgs &a, uint32_t block, const SplitPlan &plan, uint8_t *lds,
+// TAPS > 0: heads fill the kernel (keys and values of BUCKET elements) behind a convolution of that many taps, so that every size
+// below but the number of heads is the compiler's to know: a token runs every instruction once, so their number is its time.
+// A launch of 28 layers in bf16, 16 heads over 8 of 128, four taps, at 150 | 320 | 2060 positions, with the sizes as arguments,
+// 64-bit offsets and eight parts' loads in the last merge: 10.1 | 11.2 | 14.3 us; as it is: 7.9 | 8.4 | 12.0.
+template <typename T, int BUCKET, bool STEP, bool EVERY = true, int TAPS = 0>
+__device__ __forceinline__ void attn_split(const RmiAttnShape &shape, const RmiAttnArgs &a, uint32_t block, const SplitPlan &plan, uint8_t *lds,
                                            uint32_t *flag) {
     constexpr uint32_t NW = 4, NT = 256;
+    RmiAttnShape s = shape;
+    if constexpr (TAPS > 0) {
+        s.dim = s.vdim = s.dk_pad = s.dv_pad = BUCKET;
+        s.taps = TAPS;
+    }
+    auto by_half = [&](uint32_t x) { return TAPS > 0 ? x / (BUCKET / 2) : plan.half.quot(x); };
+    auto by_dv = [&](uint32_t x) { return TAPS > 0 ? x / BUCKET : plan.dv_pad.quot(x); };
     const uint32_t parts = plan.parts.by, tiles = plan.tiles.by, group = plan.group.by, keys_per_part = plan.keys_per_part;
     const uint32_t tid = threadIdx.x, lane = tid & 63, wave = uint32_t(__builtin_amdgcn_readfirstlane(int(tid >> 6))), fr = lane & 15, g4 = lane >> 4;
     const uint32_t n_cols = STEP ? group : a.n_tokens * group, slot = plan.parts.quot(block), part = block - slot * parts;
@@ -546,7 +563,7 @@ __device__ __forceinline__ void attn_split(const RmiAttnShape &s, const RmiAttnA
     const uint32_t k0 = p0 + wave * per_wave, k1 = k0 + per_wave < p1 ? k0 + per_wave : p1;
     const uint32_t live = n_cols - ct * 16 < 16 ? n_cols - ct * 16 : 16, pairs_out = live * s.dv_pad;
     auto gate_at = [&](uint32_t e) {
-        const uint32_t mc = ct * 16 + plan.dv_pad.quot(e < pairs_out ? e : 0), t = token_of(mc);
+        const uint32_t mc = ct * 16 + by_dv(e < pairs_out ? e : 0), t = token_of(mc);
         return a.gate ? a.gate + size_t(t) * s.heads + kvh * group + mc - t * group : a.u;
     };
     // the gate of the first result that this thread may write: a token's is under way from here on; with several tokens the
@@ -560,7 +577,7 @@ __device__ __forceinline__ void attn_split(const RmiAttnShape &s, const RmiAttnA
         const uint32_t half = s.dk_pad / 2, c_end = n_cols - ct * 16 < 16 ? n_cols - ct * 16 : 16;
         const uint32_t own = plan.own;
         const bool newest = a.pos0 - p0 < keys_per_part;  // this part holds the token's own key and value
-        if (conv_pairs_fit(s)) {
+        if (TAPS > 0 || conv_pairs_fit(s)) {
             // with the new key and value to make, the last two waves make them and the others the queries
             const uint32_t q_threads = newest ? NT - 128 : NT, rot = s.rot_dims / 2;
             const bool is_k = newest && wave == NW - 2, is_v = newest && wave == NW - 1;
@@ -568,7 +585,7 @@ __device__ __forceinline__ void attn_split(const RmiAttnShape &s, const RmiAttnA
             const bool keeps = is_k || is_v ? ct == 0 : part == 0;  // the one of all workgroups that carries the history on
             auto pairs = [&](uint32_t e0, auto first) {
                 const uint32_t e = e0 + (is_k || is_v ? lane : tid), ec = e < n_pairs ? e : 0;
-                const uint32_t c = is_k || is_v ? 0 : plan.half.quot(ec), i = ec - c * half;
+                const uint32_t c = is_k || is_v ? 0 : by_half(ec), i = ec - c * half;
                 const bool has = e < n_pairs && (is_v || 2 * i < s.dim);
                 const uint32_t c0 = is_v   ? (s.heads + s.kv_heads) * s.dim + kvh * s.vdim
                                     : is_k ? (s.heads + kvh) * s.dim
@@ -581,10 +598,21 @@ __device__ __forceinline__ void attn_split(const RmiAttnShape &s, const RmiAttnA
                 const uint32_t off = 4 - s.taps;
 #pragma unroll
                 for (uint32_t j = 0; j < 4; j++) {  // position pos0 - 3 + j: history row j - off
+                    if (TAPS > 0 && j < off) continue;
                     const float *row = j < 3 && j >= off ? a.hist_in + size_t(j - off) * channels : a.u;
-                    r[j] = *reinterpret_cast<const float2 *>(row + ch);
+                    r[j] = *reinterpret_cast<const float2 *>(at_bytes(row, ch * 4));
+                    if (TAPS == 4) continue;
                     w0[j] = a.conv[ch * s.taps + (j >= off ? j - off : 0)];
                     w1[j] = a.conv[(ch + 1) * s.taps + (j >= off ? j - off : 0)];
+                }
+                if constexpr (TAPS == 4) {  // a pair's taps by two loads
+                    const f32x4 *taps = reinterpret_cast<const f32x4 *>(at_bytes(a.conv, ch * 16));
+                    const f32x4 v0 = taps[0], v1 = taps[1];
+#pragma unroll
+                    for (int j = 0; j < 4; j++) {
+                        w0[j] = v0[j];
+                        w1[j] = v1[j];
+                    }
                 }
                 const bool turned = has && !is_v && i < rot;
                 const size_t at = size_t(a.pos0) * rot + (turned ? i : 0);
@@ -597,9 +625,19 @@ __device__ __forceinline__ void attn_split(const RmiAttnShape &s, const RmiAttnA
                 float p = 0.0f, o = 0.0f;
 #pragma unroll
                 for (uint32_t j = 0; j < 4; j++) {
+                    if (TAPS > 0) {
+                        if (j < off || a.pos0 + j < 3) continue;
+                        p = __builtin_fmaf(w0[j], r[j].x, p);
+                        o = __builtin_fmaf(w1[j], r[j].y, o);
+                        continue;
+                    }
                     const bool there = has && j >= off && a.pos0 + j >= 3;
                     p = __builtin_fmaf(there ? w0[j] : 0.0f, there ? r[j].x : 0.0f, p);
                     o = __builtin_fmaf(there ? w1[j] : 0.0f, there ? r[j].y : 0.0f, o);
+                }
+                if (TAPS > 0 && BUCKET < 128) {  // (of the others every lane of a wave has a pair, or all it makes is dropped)
+                    p = has ? p : 0.0f;
+                    o = has ? o : 0.0f;
                 }
                 if (keeps && has) {
 #pragma unroll
@@ -634,7 +672,7 @@ __device__ __forceinline__ void attn_split(const RmiAttnShape &s, const RmiAttnA
                 if (wave == NW - 1) value_row<T>(x, s, a, 0, kvh, lane);
             }
             for (uint32_t e = tid; e < c_end * half; e += NT) {
-                const uint32_t c = plan.half.quot(e), i = e - c * half, head = kvh * group + ct * 16 + c;
+                const uint32_t c = by_half(e), i = e - c * half, head = kvh * group + ct * 16 + c;
                 float p, r;
                 conv_rotate_pair(x, s, a.cos_t, a.sin_t, 0, a.pos0, head * s.dim, i, p, r);
                 store_pair(q + c * s.dk_pad + 2 * i, p, r);
@@ -683,14 +721,14 @@ __device__ __forceinline__ void attn_split(const RmiAttnShape &s, const RmiAttnA
     __syncthreads();
     float *ws = reinterpret_cast<float *>(static_cast<uint32_t *>(a.scratch) + kAttnCounters) + size_t(slot) * parts * pf;
     auto finish = [&](uint32_t e, float o, float sum) {
-        const uint32_t c = plan.dv_pad.quot(e), d = e - c * s.dv_pad;
+        const uint32_t c = by_dv(e), d = e - c * s.dv_pad;
         if (d >= s.vdim) return;
         const uint32_t mc = ct * 16 + c, t = token_of(mc), head = kvh * group + mc - t * group;
         const float g = STEP && e == tid ? gate0 : *gate_at(e);
         static_cast<T *>(a.out)[size_t(t) * a.out_ld + size_t(head) * s.vdim + d] = from_f32<T>(o * ((a.gate ? g : 1.0f) / sum));
     };
     for (uint32_t e = tid; e < pairs_out; e += NT) {
-        const uint32_t c = plan.dv_pad.quot(e);
+        const uint32_t c = by_dv(e);
         float m = all[c];
 #pragma unroll
         for (uint32_t i = 1; i < NW; i++) m = fmaxf(m, all[i * pl + c]);
@@ -727,34 +765,77 @@ __device__ __forceinline__ void attn_split(const RmiAttnShape &s, const RmiAttnA
     }
     __syncthreads();
     if (!*flag) return;
-    for (uint32_t e = tid; e < pairs_out; e += NT) {
-        const uint32_t c = plan.dv_pad.quot(e);
-        float m = -INFINITY, sum = 0.0f, o = 0.0f;
-        for (uint32_t p0 = 0; p0 < parts; p0 += 8) {  // eight parts' loads at a time
-            float mv[8], lv[8], ov[8];
+    auto merge = [&](auto at_a_time) {
+        constexpr uint32_t N = at_a_time.value;  // parts whose loads are under way together
+        for (uint32_t e = tid; e < pairs_out; e += NT) {
+            const uint32_t c = by_dv(e);
+            float m = -INFINITY, sum = 0.0f, o = 0.0f;
+            for (uint32_t p0 = 0; p0 < parts; p0 += N) {
+                float mv[N], lv[N], ov[N];
 #pragma unroll
-            for (uint32_t j = 0; j < 8; j++) {
-                const float *src = ws + size_t(p0 + j < parts ? p0 + j : parts - 1) * pf;
-                mv[j] = __hip_atomic_load(src + c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                lv[j] = __hip_atomic_load(src + 16 + c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                ov[j] = __hip_atomic_load(src + 32 + e, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                for (uint32_t j = 0; j < N; j++) {
+                    const float *src = ws + size_t(p0 + j < parts ? p0 + j : parts - 1) * pf;
+                    mv[j] = __hip_atomic_load(src + c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    lv[j] = __hip_atomic_load(src + 16 + c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    ov[j] = __hip_atomic_load(src + 32 + e, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                }
+                float top = m;
+#pragma unroll
+                for (uint32_t j = 0; j < N; j++)
+                    if (p0 + j < parts) top = fmaxf(top, mv[j]);
+                const float ref = top == -INFINITY ? 0.0f : top, keep = exp_t<T>(m - ref);
+                sum *= keep;
+                o *= keep;
+#pragma unroll
+                for (uint32_t j = 0; j < N; j++) {
+                    const float f = p0 + j < parts ? exp_t<T>(mv[j] - ref) : 0.0f;
+                    sum = __builtin_fmaf(lv[j], f, sum);
+                    o = __builtin_fmaf(ov[j], f, o);
+                }
+                m = top;
             }
-            float top = m;
-#pragma unroll
-            for (uint32_t j = 0; j < 8; j++)
-                if (p0 + j < parts) top = fmaxf(top, mv[j]);
-            const float ref = top == -INFINITY ? 0.0f : top, keep = exp_t<T>(m - ref);
-            sum *= keep;
-            o *= keep;
-#pragma unroll
-            for (uint32_t j = 0; j < 8; j++) {
-                const float f = p0 + j < parts ? exp_t<T>(mv[j] - ref) : 0.0f;
-                sum = __builtin_fmaf(lv[j], f, sum);
-                o = __builtin_fmaf(ov[j], f, o);
-            }
-            m = top;
+            finish(e, o, sum);
         }
-        finish(e, o, sum);
+    };
+    // Few parts: every thread reads all, and of no more parts than there are, as a load past the caches is 40 ns of a wave (a
+    // token of 28 layers at 150 positions, two parts: 560 us with eight parts' loads, 537 with two parts', by lanes 551).  More:
+    // by lanes (2048 positions, f32: 980 us where every thread reads all, 914 by lanes; 700 positions, bf16: 569 and 551).
+    if (parts == 2) return merge(std::integral_constant<uint32_t, 2>());
+    if (parts <= 4) return merge(std::integral_constant<uint32_t, 4>());
+    if constexpr (TAPS > 0) {
+        // A wave's results are of one column: a lane reads one part's maximum or sum of it, and weighs that part for all.
+        static_assert(2 * kMaxParts <= 64 && BUCKET % 64 == 0);
+        auto merge_lanes = [&](auto at_a_time) {
+            constexpr uint32_t N = at_a_time.value;
+            for (uint32_t e = tid; e < pairs_out; e += NT) {
+                const uint32_t c = uint32_t(__builtin_amdgcn_readfirstlane(int(by_dv(e)))), mine = lane % kMaxParts;
+                const bool there = mine < parts;
+                auto part_at = [&](uint32_t i) { return (i < parts ? i : parts - 1) * pf; };
+                float ml = __hip_atomic_load(ws + part_at(mine) + c + lane / kMaxParts * 16, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                float ov[N], o = 0.0f, f = 0.0f, sum = 0.0f;
+                for (uint32_t p0 = 0; p0 < parts; p0 += N) {
+#pragma unroll
+                    for (uint32_t j = 0; j < N; j++)
+                        ov[j] = __hip_atomic_load(ws + part_at(p0 + j) + 32 + e, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    if (p0 == 0) {
+                        const float top = wave_max_f32(lane < kMaxParts && there ? ml : -INFINITY), ref = top == -INFINITY ? 0.0f : top;
+                        f = there ? exp_t<T>(__shfl(ml, int(mine)) - ref) : 0.0f;  // in both halves
+                        sum = wave_sum_f32(lane >= kMaxParts && there ? ml * f : 0.0f);
+                    }
+#pragma unroll
+                    for (uint32_t j = 0; j < N; j++)
+                        if (p0 + j < parts)
+                            o = __builtin_fmaf(ov[j], __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, f), int(p0 + j))), o);
+                }
+                finish(e, o, sum);
+            }
+        };
+        if (parts <= 8)
+            merge_lanes(std::integral_constant<uint32_t, 8>());
+        else
+            merge_lanes(std::integral_constant<uint32_t, 16>());
+    } else {
+        merge(std::integral_constant<uint32_t, 8>());
     }
 }
 
@@ -848,8 +929,8 @@ inline size_t recur_step_lds(const RmiRecurShape &s) {
 // everything here was pushed out by the weights: the arguments, the operands with the first keys, values and state rows, the
 // parts' stores, their count and their loads.  So all that does not depend on another load is under way at once and no
 // division stands before it: 28 layers of 16 heads over 8 of 128 elements, 150 positions, bf16: 12.7 us a launch with loads
-// behind branches, 10.0 as it is; f32, 16 key/value heads and 310 positions: 17.6 and 14.8.  Parts of 64 or of 32 keys, and
-// eight waves a workgroup for 256 keys without a second workgroup, all took as long or longer.
+// behind branches, 10.0 without; f32, 16 key/value heads and 310 positions: 17.6 and 14.8.  Parts of 64 or of 32 keys, and
+// eight waves a workgroup for 256 keys without a second workgroup (3 to 15 % of a whole token), all took as long or longer.
 struct MixersStep {
     RmiAttnShape s;
     RmiAttnArgs a;
@@ -859,13 +940,13 @@ struct MixersStep {
     RmiAhead ahead;
     uint32_t attn_blocks;
 };
-template <typename T, int BUCKET>
+template <typename T, int BUCKET, int TAPS>
 __global__ __launch_bounds__(kStepThreads) void mixers_step_kernel(MixersStep p) {
     extern __shared__ __attribute__((aligned(16))) uint8_t lds_raw[];
     __shared__ uint32_t flag;
     fetch_args<MixersStep>();
     if (blockIdx.x < p.attn_blocks)
-        attn_split<T, BUCKET, true>(p.s, p.a, blockIdx.x, p.plan, lds_raw, &flag);
+        attn_split<T, BUCKET, true, true, TAPS>(p.s, p.a, blockIdx.x, p.plan, lds_raw, &flag);
     else if (blockIdx.x < p.attn_blocks + p.rs.heads)
         recur_step<T>(p.rs, p.ra, blockIdx.x - p.attn_blocks, reinterpret_cast<float *>(lds_raw));
     else
@@ -1239,7 +1320,15 @@ int mixers_step(const RmiAttnShape *as, const RmiAttnArgs *aa, const RmiRecurSha
         if (rc == RMI_HIP_OK) hipLaunchKernelGGL(kernel, grid, dim3(kStepThreads), lds, st, p);
         return rc;
     };
-    const int rc = bucket == 64 ? go(mixers_step_kernel<T, 64>) : bucket == 128 ? go(mixers_step_kernel<T, 128>) : go(mixers_step_kernel<T, 256>);
+    // Heads that fill a kernel, behind four taps or without a convolution, and no wider than a wave's pairs of channels; a
+    // token of 28 layers at 16 | 150 | 2048 positions: 560 | 606 | 730 us with the sizes as arguments, 545 | 569 | 670 known.
+    const bool filled = as && bucket <= 128 && p.s.dim == bucket && p.s.vdim == bucket && p.s.dk_pad == bucket && p.s.dv_pad == bucket &&
+                        reinterpret_cast<uintptr_t>(p.a.conv) % 16 == 0;
+    auto with = [&](auto taps) { return bucket == 64 ? go(mixers_step_kernel<T, 64, taps.value>) : go(mixers_step_kernel<T, 128, taps.value>); };
+    const int rc = filled && p.s.taps == 4   ? with(std::integral_constant<int, 4>())
+                   : filled && p.s.taps == 1 ? with(std::integral_constant<int, 1>())
+                   : bucket == 256           ? go(mixers_step_kernel<T, 256, 0>)
+                                             : with(std::integral_constant<int, 0>());
     if (rc != RMI_HIP_OK) return rc;
     RMI_HIP_CHECK(hipGetLastError());
     return RMI_HIP_OK;
