@@ -28,6 +28,7 @@
 #include <vector>
 
 #include "attn_prompt.h"
+#include "device_ahead.h"
 #include "device_math.h"
 #include "device_quant.h"
 #include "device_sample.h"
@@ -518,6 +519,7 @@ struct AttnFromQkv {
     const float *cos_row, *sin_row;  // [64] each: the angles of this position
     uint16_t *k_row, *v_row;         // the cache rows of this position, [n_head_kv][128] each
     float eps;
+    RmiAhead ahead;                  // what workgroups behind the heads' fetch
 };
 // PASS: several consecutive positions, blockIdx.z, whose cache rows are filled already; q16, q8 and scales are theirs one
 // after the other.  Every phase is a stretch of dependent instructions, so one workgroup leaves its compute unit idle most
@@ -529,6 +531,13 @@ __global__ __launch_bounds__(kA128Threads, PASS ? kPassWaves : 2) void attention
     const uint16_t *__restrict__ q16, const uint16_t *__restrict__ k_cache, const uint16_t *__restrict__ v_cache,
     uint32_t step, uint32_t kv_stride, uint32_t n_head, uint32_t n_head_kv, int8_t *__restrict__ q8,
     float *__restrict__ scales, int rounding, AttnFromQkv fq) {
+    if constexpr (FROM_QKV && PVP > 1) {
+        if (blockIdx.x >= n_head * PVP) {
+            __builtin_amdgcn_s_sleep(64);  // 1.7 us: the keys and values first
+            fetch_ahead<kA128Threads>(fq.ahead, n_head * PVP);
+            return;
+        }
+    }
     extern __shared__ double lds_d[];
     __shared__ float red_f[kA128Threads / 64];
     __shared__ uint64_t exp_tab[32];
@@ -1085,6 +1094,11 @@ __global__ __launch_bounds__(kAttnSplitThreads) void attn128_weights_pv_kernel(
     }
 }
 
+// With parts, compute units that have no head fetch the output product's weights meanwhile, if they are no more than this.  28
+// layers of width 1024 (2.2 MB a layer), a prompt of 70 | 512 | 1000 tokens and 32 more: 20.1 | 28.58 | 36.1 ms without,
+// 19.9 | 28.26 | 35.6 with; eight layers of 2048 (4.5 MB) 11.32 and 11.25; four of 4096 with the 18 MB of each 13.58 and 13.59.
+// The gate, up, down or the next q/k/v weights too, 9 to 17 MB: 28.7 to 29.4 ms at 512, more in the attention than saved behind it.
+constexpr size_t kAttnAheadBytes = 8u << 20;
 // One position's attention straight from its f32 q | k | v: the launch with the p.v sums of a head split over parts.
 // Four parts from 64 keys on (measured over 512..638 keys, 28 layers: 0.840 ms a generated token with one part, 0.789
 // with two, 0.779 with four); below, the p.v sums are a few terms and one workgroup a head is enough.
@@ -1095,10 +1109,12 @@ static void launch_attention128_from_qkv(const uint16_t *k_cache, const uint16_t
     const size_t lds = attn128_lds_bytes(step + 1);
     const uint16_t *no_q16 = nullptr;
     switch (attn_pv_parts(step + 1)) {
-    case 4:
-        hipLaunchKernelGGL((attention128_quant_kernel<true, 4>), dim3(n_head * 4), dim3(kA128Threads), lds, st, no_q16, k_cache,
+    case 4: {
+        const uint32_t used = n_head * 4, ahead = rmi_ahead_blocks(fq.ahead, used, uint32_t(rmi_device_cus()));
+        hipLaunchKernelGGL((attention128_quant_kernel<true, 4>), dim3(used + ahead), dim3(kA128Threads), lds, st, no_q16, k_cache,
                            v_cache, step, kv_stride, n_head, n_head_kv, q8, scales, rounding, fq);
         break;
+    }
     default:
         hipLaunchKernelGGL((attention128_quant_kernel<true, 1>), dim3(n_head / n_head_kv, n_head_kv), dim3(kA128Threads), lds, st,
                            no_q16, k_cache, v_cache, step, kv_stride, n_head, n_head_kv, q8, scales, rounding, fq);
@@ -1321,8 +1337,9 @@ int enqueue_step(rmi_hip_qwen3 *s, uint32_t step, hipStream_t st) {
             rc = norm_gemv(s->w_qkv[l], pending, s->attn_norm[l], s->qkv);
             if (rc != RMI_HIP_OK) return rc;
             const size_t half = 64;
-            const AttnFromQkv fq{s->qkv, qn, kn, s->cos_t + size_t(step) * half, s->sin_t + size_t(step) * half,
-                                 s->k_cache + row, s->v_cache + row, c.eps};
+            AttnFromQkv fq{s->qkv, qn, kn, s->cos_t + size_t(step) * half, s->sin_t + size_t(step) * half,
+                           s->k_cache + row, s->v_cache + row, c.eps, RmiAhead{}};
+            rmi_gemv_q8_0_ahead(s->w_o[l], kAttnAheadBytes, &fq.ahead);
             launch_attention128_from_qkv(s->k_cache + layer_base, s->v_cache + layer_base, step, s->kv_stride, c.n_head, c.n_head_kv,
                                          s->act_q8, s->act_scales, rnd, fq, st);
         } else if (rmi_gemv_q8_0_norm_rope_fusable(s->w_qkv[l], c.n_head, c.n_head_kv, c.head_dim_k, c.head_dim_v)) {
@@ -1648,7 +1665,7 @@ int rmi_hip_qkv_attention_f16_quantize_q8_0_dev(const float *qkv, const float *q
                         "(rmi_hip_qk_norm_rope_f16_dev, then rmi_hip_attention_f16_quantize_q8_0_dev)", n_keys,
                         uint32_t((48 * 1024 - (kA128Threads / 64) * 128 * 8 - 128) / 12 / kAttnPad * kAttnPad));
     const size_t row = size_t(n_keys - 1) * kv_stride;
-    const AttnFromQkv fq{qkv, q_norm, k_norm, cos_row, sin_row, k_cache + row, v_cache + row, eps};
+    const AttnFromQkv fq{qkv, q_norm, k_norm, cos_row, sin_row, k_cache + row, v_cache + row, eps, RmiAhead{}};
     launch_attention128_from_qkv(k_cache, v_cache, n_keys - 1, kv_stride, n_head, n_head_kv, q8, scales, rounding, fq,
                                  static_cast<hipStream_t>(stream));
     RMI_HIP_CHECK(hipGetLastError());

@@ -15,7 +15,7 @@
 //   24 MB, a workgroup a unit left         522 | 583 | 693 | 761
 //   32 MB, a workgroup a unit left         545 | 574 | 710 | 765     (all of the L2s: what the mixers read goes, too)
 // In f32 and at widths of 2048 and 4096 the kept setting is within 3 % of the best of the five, and no token is slower for it.
-// Qwen3's attention launch, with 64 workgroups that all read keys, lost by it (11 -> 21 us) and has none.
+// Qwen3's attention launch, with 64 workgroups that all read keys, lost by as much (11 -> 21 us) and fetches a few MB only.
 // Workgroup b of the launch that reads a region reads its bytes [b chunk, (b + 1) chunk).  Workgroups go round the eight
 // XCDs in turn, each with an L2 of its own: what workgroup b will read is read on the XCD b % 8.  Only a hint: if the
 // workgroups go elsewhere, the bytes are still nearer than HBM.

@@ -6,6 +6,7 @@
 // taking fma(f32(wd)*xs[b], float(sum_{k=4L..4L+3} w*x), acc_L) block after
 // block, then hsum_ps (src/ops/dot.rs:447-456).  Eight GPU lanes hold the eight
 // accumulators of one row, so results match that kernel bit for bit.
+#include "device_ahead.h"
 #include "device_math.h"
 #include "device_quant.h"
 #include "rmi_internal.h"
@@ -1486,6 +1487,11 @@ int rmi_launch_gemv_q8_0_single(const RmiGemvProblem &problem, uint32_t group, h
     // not by the staging it shares: smaller workgroups on more compute units
     while (wpg > 1 && n_waves / wpg < cus) wpg >>= 1;
     return dispatch_gemv(group, &p, nullptr, nullptr, n_waves, wpg, tpw, p.n_oct, s);
+}
+
+void rmi_gemv_q8_0_ahead(const rmi_hip_weight *w, size_t most, RmiAhead *ahead) {
+    const size_t tile = size_t(w->n_units) * kOctetBytes;
+    if (w->n_units <= kDeepMaxOct && w->n_tiles <= kDeepMaxTiles && tile * w->n_tiles <= most) ahead->add(w->data, tile, w->n_tiles);
 }
 
 bool rmi_gemv_q8_0_norm_fusable(const rmi_hip_weight *w) {
