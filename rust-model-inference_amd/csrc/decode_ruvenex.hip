@@ -92,7 +92,7 @@ int RuvenexSession::enqueue_layers(uint32_t step0, uint32_t n, hipStream_t st, f
             rc = rmi_dense_gemv(elem, y.w_in, normed(y.norm), y.in, st);
             RmiAhead ahead{};
             rmi_dense_ahead_residual(elem, y.w_out, width, &ahead);
-            if (l + 1 < n_runs) rmi_dense_ahead_gemv(elem, layers[l + 1].w_in, normed(y.norm), layers[l + 1].in, &ahead);
+            if (l + 1 < n_runs) rmi_dense_ahead_gemv(elem, layers[l + 1].w_in, kNormRms, layers[l + 1].in, &ahead);
             if (rc == RMI_HIP_OK) rc = rmi_mixers_step(elem, &y.attn, &a, &y.recur, &r, ahead, st);
             if (rc == RMI_HIP_OK) rc = rmi_dense_gemv_residual(elem, y.w_out, act, y.out, x, width, st);
         } else {

@@ -133,7 +133,7 @@ int rmi_dense_gemv(uint32_t elem_bytes, const RmiDense &w, const RmiInput &in, c
 int rmi_dense_gemv_pair(uint32_t elem_bytes, const RmiDense &w0, const RmiInput &in0, const RmiRowSegs &segs0, const RmiDense &w1,
                         const RmiInput &in1, const RmiRowSegs &segs1, hipStream_t st);
 // what the products of one token read, for a launch in front of them to fetch (device_ahead.h)
-void rmi_dense_ahead_gemv(uint32_t elem_bytes, const RmiDense &w, const RmiInput &in, const RmiRowSegs &segs, RmiAhead *ahead);
+void rmi_dense_ahead_gemv(uint32_t elem_bytes, const RmiDense &w, RmiNorm norm, const RmiRowSegs &segs, RmiAhead *ahead);
 void rmi_dense_ahead_residual(uint32_t elem_bytes, const RmiDense &w, uint32_t width, RmiAhead *ahead);
 int rmi_dense_gemv_residual(uint32_t elem_bytes, const RmiDense &w, const void *a, const RmiColSegs &segs, float *x, uint32_t width,
                             hipStream_t st);

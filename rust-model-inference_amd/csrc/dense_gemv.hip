@@ -229,15 +229,15 @@ constexpr uint32_t kResidualRows = 2;
 // A wave takes four rows; fewer where that would leave compute units with little to do (the prologue, which every
 // workgroup repeats, then weighs less than the wait for memory).  Pairs of rows stay together.  (12 288 rows of 2048
 // f32: 19.1 us with four, 20.8 with two, of which one and a fifth of a chip's fill are resident; 6176 rows: two.)
-uint32_t rows_of_wave(const RmiDense &w, const RmiInput &in, const RmiRowSegs &segs) {
+uint32_t rows_of_wave(const RmiDense &w, RmiNorm norm, const RmiRowSegs &segs) {
     const uint32_t cus = uint32_t(rmi_device_cus()), pairs = rmi_epilogue_of(segs) == kRowsPaired ? 2 : 1;
-    return in.norm == kNormRms || w.n_rows >= 32 * cus ? 4 : w.n_rows > 4 * cus ? 2 : pairs;
+    return norm == kNormRms || w.n_rows >= 32 * cus ? 4 : w.n_rows > 4 * cus ? 2 : pairs;
 }
 
 template <typename T>
 int gemv(const RmiDense &w, const RmiInput &in, const RmiRowSegs &segs, hipStream_t st) {
     const size_t lds = size_t(gemv_lds_pieces<T>(w.k_pad)) * 16;
-    const uint32_t cus = uint32_t(rmi_device_cus()), rows = rows_of_wave(w, in, segs);
+    const uint32_t cus = uint32_t(rmi_device_cus()), rows = rows_of_wave(w, in.norm, segs);
     const GemvProblem p = problem_of(w, in, segs, rows);
     auto go = [&](auto kernel) {
         const int rc = rmi_allow_lds(kernel, lds);
@@ -336,8 +336,8 @@ int rmi_dense_gemv_residual(uint32_t elem_bytes, const RmiDense &w, const void *
     return elem_bytes == 2 ? gemv_residual<rmi_bf16>(w, a, segs, x, width, st) : gemv_residual<float>(w, a, segs, x, width, st);
 }
 
-void rmi_dense_ahead_gemv(uint32_t elem_bytes, const RmiDense &w, const RmiInput &in, const RmiRowSegs &segs, RmiAhead *ahead) {
-    const uint32_t rows = 4 * rows_of_wave(w, in, segs);
+void rmi_dense_ahead_gemv(uint32_t elem_bytes, const RmiDense &w, RmiNorm norm, const RmiRowSegs &segs, RmiAhead *ahead) {
+    const uint32_t rows = 4 * rows_of_wave(w, norm, segs);
     ahead->add(w.data, size_t(rows) * w.ld * elem_bytes, w.n_rows / rows);
 }
 

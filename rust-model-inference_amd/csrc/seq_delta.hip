@@ -36,9 +36,13 @@ __device__ __forceinline__ void delta_carry(const RmiDeltaShape &s, const RmiDel
 //   u = beta (v - g S^T k),   o = g S^T q + (k . q) u,   S' = g S + k u^T
 constexpr uint32_t kStepThreads = 512;
 template <typename T, int NR>
-__global__ __launch_bounds__(kStepThreads) void delta_step_kernel(RmiDeltaShape s, RmiDeltaArgs a) {
+__global__ __launch_bounds__(kStepThreads) void delta_step_kernel(RmiDeltaShape s, RmiDeltaArgs a, RmiAhead ahead) {
     __shared__ __attribute__((aligned(16))) float ks[kMaxHeadDim], qs[kMaxHeadDim], vs[kMaxHeadDim], us[kMaxHeadDim], red[8];
     __shared__ __attribute__((aligned(16))) float part[2][4 * kStepThreads];  // [S^T k, S^T q][slice][column]
+    if (blockIdx.x >= s.heads) {
+        fetch_ahead<kStepThreads>(ahead, s.heads);
+        return;
+    }
     const uint32_t tid = threadIdx.x, lane = tid & 63, h = blockIdx.x, group = s.heads / s.kv_heads, g = h / group;
     const ConvCtx x{a.u, a.hist_in, a.conv, delta_channels(s), s.taps};
     const uint32_t n_ch = 2 * s.dim + s.vdim;  // this head's channels: queries, keys, values
@@ -526,9 +530,10 @@ int delta_pass(const RmiDeltaShape &s, const RmiDeltaArgs &a, hipStream_t st) {
 }
 
 template <typename T>
-int delta_step(const RmiDeltaShape &s, const RmiDeltaArgs &a, hipStream_t st) {
+int delta_step(const RmiDeltaShape &s, const RmiDeltaArgs &a, const RmiAhead &ahead, hipStream_t st) {
     const uint32_t slices = kStepThreads / (s.v_pad / 4), rows = (s.d_pad + slices - 1) / slices;  // at most 32
-    auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3(s.heads), dim3(kStepThreads), 0, st, s, a); };
+    const dim3 grid(s.heads + rmi_ahead_blocks(ahead, s.heads, uint32_t(rmi_device_cus())));
+    auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(kStepThreads), 0, st, s, a, ahead); };
     if (rows <= 8)
         go(delta_step_kernel<T, 8>);
     else
@@ -550,9 +555,9 @@ int rmi_delta_pass(uint32_t elem_bytes, const RmiDeltaShape &s, const RmiDeltaAr
     return elem_bytes == 2 ? delta_pass<rmi_bf16>(s, a, st) : delta_pass<float>(s, a, st);
 }
 
-int rmi_delta_step(uint32_t elem_bytes, const RmiDeltaShape &s, const RmiDeltaArgs &a, hipStream_t st) {
+int rmi_delta_step(uint32_t elem_bytes, const RmiDeltaShape &s, const RmiDeltaArgs &a, const RmiAhead &ahead, hipStream_t st) {
     if (a.n_tokens != 1) return rmi_fail(RMI_HIP_E_INVALID, "a step takes one token");
     const int rc = check_delta(s);
     if (rc != RMI_HIP_OK) return rc;
-    return elem_bytes == 2 ? delta_step<rmi_bf16>(s, a, st) : delta_step<float>(s, a, st);
+    return elem_bytes == 2 ? delta_step<rmi_bf16>(s, a, ahead, st) : delta_step<float>(s, a, ahead, st);
 }

@@ -96,4 +96,4 @@ int rmi_recur_pass(uint32_t elem_bytes, const RmiRecurShape &s, const RmiRecurAr
 int rmi_mixers_step(uint32_t elem_bytes, const RmiAttnShape *as, const RmiAttnArgs *aa, const RmiRecurShape *rs, const RmiRecurArgs *ra,
                     const RmiAhead &ahead, hipStream_t st);
 int rmi_delta_pass(uint32_t elem_bytes, const RmiDeltaShape &s, const RmiDeltaArgs &a, hipStream_t st);
-int rmi_delta_step(uint32_t elem_bytes, const RmiDeltaShape &s, const RmiDeltaArgs &a, hipStream_t st);
+int rmi_delta_step(uint32_t elem_bytes, const RmiDeltaShape &s, const RmiDeltaArgs &a, const RmiAhead &ahead, hipStream_t st);
