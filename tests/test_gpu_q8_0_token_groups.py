@@ -1,6 +1,6 @@
 """Products of several tokens in the x86-64 order (matmul_q8_0_vs_q8_0_avx2, src/ops/kernel/q8_0/avx2.rs:71-173): the GEMV's
 token groups, of eight and of four, whole, ragged (the last group begins earlier) and with a launch behind them, and the tiles
-of the matrix cores with token scales that are not f16 values.  Every output has the bits of the checker's AVX2 order."""
+of the matrix cores with token scales that are not f16 values.  Every output has the bits of the oracle's AVX2 order."""
 import numpy as np
 import pytest
 
@@ -8,7 +8,7 @@ from conftest import bits
 
 pytestmark = pytest.mark.gpu
 
-A = 1  # the checker's AVX2 order
+A = 1  # the oracle's AVX2 order
 
 
 def _activation(hip, oracle, seed, n_tokens, n_in):
