@@ -803,29 +803,38 @@ __device__ __forceinline__ void attn_split(const RmiAttnShape &shape, const RmiA
     if (parts == 2) return merge(std::integral_constant<uint32_t, 2>());
     if (parts <= 4) return merge(std::integral_constant<uint32_t, 4>());
     if constexpr (TAPS > 0) {
-        // A wave's results are of one column: a lane reads one part's maximum or sum of it, and weighs that part for all.
+        // A wave's results are of one column: a lane reads one part's maximum or sum of it, and weighs that part for all.  The order
+        // is that of the eight parts above, step by step, so that the bits are, too.
         static_assert(2 * kMaxParts <= 64 && BUCKET % 64 == 0);
+        auto of_lane = [](float x, uint32_t i) { return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, x), int(i))); };
         auto merge_lanes = [&](auto at_a_time) {
             constexpr uint32_t N = at_a_time.value;
             for (uint32_t e = tid; e < pairs_out; e += NT) {
-                const uint32_t c = uint32_t(__builtin_amdgcn_readfirstlane(int(by_dv(e)))), mine = lane % kMaxParts;
-                const bool there = mine < parts;
+                const uint32_t c = uint32_t(__builtin_amdgcn_readfirstlane(int(by_dv(e))));
                 auto part_at = [&](uint32_t i) { return (i < parts ? i : parts - 1) * pf; };
-                float ml = __hip_atomic_load(ws + part_at(mine) + c + lane / kMaxParts * 16, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                float ov[N], o = 0.0f, f = 0.0f, sum = 0.0f;
+                // lane i the maximum of part i, lane kMaxParts + i its sum
+                const float ml = __hip_atomic_load(ws + part_at(lane % kMaxParts) + c + lane / kMaxParts * 16, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                float ov[N], m = -INFINITY, o = 0.0f, sum = 0.0f;
                 for (uint32_t p0 = 0; p0 < parts; p0 += N) {
 #pragma unroll
                     for (uint32_t j = 0; j < N; j++)
                         ov[j] = __hip_atomic_load(ws + part_at(p0 + j) + 32 + e, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                    if (p0 == 0) {
-                        const float top = wave_max_f32(lane < kMaxParts && there ? ml : -INFINITY), ref = top == -INFINITY ? 0.0f : top;
-                        f = there ? exp_t<T>(__shfl(ml, int(mine)) - ref) : 0.0f;  // in both halves
-                        sum = wave_sum_f32(lane >= kMaxParts && there ? ml * f : 0.0f);
-                    }
 #pragma unroll
-                    for (uint32_t j = 0; j < N; j++)
-                        if (p0 + j < parts)
-                            o = __builtin_fmaf(ov[j], __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, f), int(p0 + j))), o);
+                    for (uint32_t g = 0; g < N; g += 8) {
+                        if (p0 + g >= parts) break;
+                        const float top = fmaxf(m, wave_max_f32(lane < parts && lane / 8 == (p0 + g) / 8 ? ml : -INFINITY));
+                        const float ref = top == -INFINITY ? 0.0f : top, keep = exp_t<T>(m - ref), f = exp_t<T>(ml - ref);
+                        sum *= keep;
+                        o *= keep;
+#pragma unroll
+                        for (uint32_t j = g; j < g + 8; j++)
+                            if (p0 + j < parts) {
+                                const float fj = of_lane(f, p0 + j);
+                                sum = __builtin_fmaf(of_lane(ml, kMaxParts + p0 + j), fj, sum);
+                                o = __builtin_fmaf(ov[j], fj, o);
+                            }
+                        m = top;
+                    }
                 }
                 finish(e, o, sum);
             }

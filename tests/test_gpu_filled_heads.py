@@ -25,3 +25,26 @@ def test_every_number_of_parts(hip, tmp_path, dtype, heads, kv_heads, dim, taps)
     o.close()
     # the sessions' own tolerance: a part left out or weighed wrongly errs by its share of the weights, 1/17 and more
     assert rel(got, ref) < TOL[dtype], int(np.argmax(np.abs(got - ref).max(-1)))
+
+
+@pytest.mark.parametrize("dtype", [F32, BF16])
+@pytest.mark.parametrize("heads,kv_heads,dim,taps", [(4, 2, 128, 4), (3, 1, 64, 4), (5, 1, 128, 1), (20, 1, 64, 1)])
+def test_bits_are_those_of_heads_of_any_size(hip, tmp_path, dtype, heads, kv_heads, dim, taps):
+    """The same model with a tap of zeros more or less: 4 taps and 1 are the kernel that knows its sizes, 3 and 2 the one for any
+    head.  A tap of zeros changes no sum, so all that can differ is how parts are put together."""
+    def cfg(n):
+        return G.config([G.layer_config(heads=heads, kv_heads=kv_heads, dim=dim, vdim=dim, taps=n, rot_dims=dim // 2, rdim=8, rvdim=8)], width=40)
+
+    few, many = (3, 4) if taps == 4 else (1, 2)
+    w = G.weights(cfg(few), 3)
+    padded = {n: np.pad(a, ((0, 0), (1, 0))) if n.endswith(".conv") else a for n, a in w.items()}
+    o = Opener(hip, tmp_path, G)
+    s, s2 = o(cfg(few), w, dtype, 5000)[0], o(cfg(many), padded, dtype, 5000)[0]
+    sizes, at = [1] * 6, 6
+    for keys in (128, 256, 512, 640, 1024, 1152, 1700, 2048, 2176, 3072, 4096, 4900):  # from 512 on more parts than four
+        sizes += [keys - 2 - at] + [1] * 4
+        at = keys + 2
+    t = G.tokens(cfg(few), at)
+    a, b = feed(s, t, sizes), feed(s2, t, sizes)
+    o.close()
+    assert np.array_equal(a.view(np.uint32), b.view(np.uint32)), np.flatnonzero((a != b).any(-1))[:8]
