@@ -14,16 +14,19 @@
 // scale is an f16, the token scale the reference's quantizers write is an f16 value held in an f32 (src/ops/quant/q8_0.rs:63,
 // 121, 207), and the product of two f16 values is exact in f32.  (v_mfma_f32_16x16x1_4b_f32 would take any f32 scale, but f32
 // products of the matrix cores and f32 sums of the vector ALU keep each other from running: 64 sums and two products 119 ns a
-// wave with f16 operands, 148 with f32 ones.)  A tile with a token scale that is no f16 value, a caller's own, is made again
-// on the vector ALU behind the loop.
+// wave with f16 operands, 148 with f32 ones.)  From the first quad on in which some token scale is no finite f16 value (a caller's
+// own, or the quantizer's infinity for values from 8.3e6 on) a tile has scale products of the vector ALU.
 //
 // What bounds it: the vector ALU, 32 fma per 16 x 16 x 32 = 54 ns a SIMD with four waves on it, beside which the conversion of
-// the operands to f16 as they are staged costs 5 instructions per 4 values, shared by the waves that read them: 642 vector
-// instructions a quad of a wave's four tiles, issued 80 % of the time with the two waves whose sums fit the registers.  us, with
-// the scale products on the vector ALU | as it is: 64 x 64 tiles, 6144 x 1024, 1024 tokens 70.8 | 68.5, 151936 x 1024, 128
-// tokens 213 | 207; 32 x 32 tiles, 1024 x 3072, 512 tokens 26.3 | 25.0, 1024 x 2048, 512 tokens 19.5 | 18.4.
+// the operands to f16 as they are staged costs 5 instructions per 4 values, shared by the waves that read them: 648 vector
+// instructions a quad of a wave's four tiles, with the two waves whose sums fit the registers.  us, with all scale products on the
+// vector ALU | as it is | as it is, no token scale an f16 value: 64 x 64 tiles, 6144 x 1024, 1024 tokens 70.8 | 69.3 | 73.5, 151936 x
+// 1024, 128 tokens 214 | 209 | 222; 32 x 32 tiles, 1024 x 3072, 512 tokens 26.1 | 25.4 | 26.6, 1024 x 2048, 512 tokens 18.5 | 18.2 |
+// 19.1; 64 x 16 tiles, 20003 x 1056, 12 tokens 12.1 | 12.4 | 12.9.  (A second pass over such a tile, from memory and without
+// staging, took 1085 us in the place of 73.5.)
 // Eight tokens to a workgroup of the GEMV with int8 dots (4 x 4 x 4) and a conversion each: 151936 x 1024, 128 tokens 529.
 #include <cmath>
+#include <type_traits>
 
 #include "rmi_internal.h"
 
@@ -47,12 +50,13 @@ __device__ __forceinline__ u32x2 i8x4_to_f16x4(uint32_t q) {
 
 // A workgroup of WR x WT waves, each NR x NT tiles of sixteen rows x sixteen tokens; k in quads of four blocks through two LDS
 // buffers, the next quad's bytes on their way to registers meanwhile.  One block of a buffer is [row][32 f16]; behind the blocks
-// stand the quad's scales, [row][4 f16].
+// stand the quad's scales, [row][4 f16] and [token][4 f16], or, for any token scale, [block][row f32] and [block][token f32].
 template <int NR, int NT, int WR, int WT>
 struct X86Tile {
     static constexpr int BN = 16 * NR * WR, BT = 16 * NT * WT, THREADS = 64 * WR * WT;
     static constexpr int ABLK = BN * 64 + 64, BBLK = BT * 64 + 64;  // bytes of a block, off a multiple of 256
-    static constexpr int LDS_BUF = 4 * (ABLK + BBLK) + 8 * (BN + BT);
+    static constexpr int LDS_BUF = 4 * (ABLK + BBLK) + 16 * (BN + BT);
+    static constexpr int LDS = 2 * LDS_BUF + 16;  // and three flags
 };
 
 template <int NR, int NT, int WR, int WT, int WPS>
@@ -104,7 +108,7 @@ __global__ __launch_bounds__(64 * WR * WT, WPS) void gemm_q8_0_x86_kernel(RmiGem
     const uint32_t b_dst = 4 * TL::ABLK + (tid >> 1 & 3) * TL::BBLK + ((tid % (BT * 8)) / 8) * 64 + (tid & 1) * 32;
     const uint32_t s_row = tid % BN, s_tile = (s_row >> 3) < last_tile ? s_row >> 3 : last_tile;
     const uint32_t as_off = s_tile * uint32_t(tile_bytes) + (s_row & 7) * 16;
-    constexpr uint32_t kScaleA = 4 * (TL::ABLK + TL::BBLK), kScaleB = kScaleA + 8 * BN;
+    constexpr uint32_t kScaleA = 4 * (TL::ABLK + TL::BBLK), kScaleB = kScaleA + 8 * BN, kScaleBAny = kScaleA + 16 * BN;
 #pragma unroll
     for (int i = 0; i < PS; i++) {
         const uint32_t e = (tid + i * TH) % (BT * 4), t = (e >> 2) < last_tok ? e >> 2 : last_tok;
@@ -112,7 +116,14 @@ __global__ __launch_bounds__(64 * WR * WT, WPS) void gemm_q8_0_x86_kernel(RmiGem
     }
     u32x4 ra[PA], rb[PB];
     u32x2 rsa;
-    float rsb[PS];
+    float rsb[PS];  // token scales, of the quad behind those in ra .. rsa
+    _Float16 rsb16[PS];
+    auto load_scales = [&](uint32_t q, float (&r)[PS]) {
+        q = q < n_quads ? q : n_quads - 1;
+        const uint32_t bs_at = 4 * q + (me() & 3), bs = bs_at < nb ? bs_at : nb - 1;
+#pragma unroll
+        for (int i = 0; i < PS; i++) r[i] = *(gptr_f32)(xs_base + (bs_off[i] + bs * 4));
+    };
     auto load = [&](uint32_t q) {
         // always issued (past the end the last quad again): a skipped load would make the waits wait for all of them
         q = q < n_quads ? q : n_quads - 1;
@@ -126,12 +137,35 @@ __global__ __launch_bounds__(64 * WR * WT, WPS) void gemm_q8_0_x86_kernel(RmiGem
 #pragma unroll
         for (int i = 0; i < PB; i++) rb[i] = *(gptr_u4)(x_base + (b_off[i] + bb * 32));
         rsa = *(gptr_u2)(w_base + (as_off + (q >> 1) * 128 + (q & 1) * 8));
-        const uint32_t bs_at = 4 * q + (t & 3), bs = bs_at < nb ? bs_at : nb - 1;
-#pragma unroll
-        for (int i = 0; i < PS; i++) rsb[i] = *(gptr_f32)(xs_base + (bs_off[i] + bs * 4));
     };
-    uint64_t not_f16 = 0;  // lanes that staged a token scale which is not a finite f16 value
-    auto park = [&](uint32_t buf) {
+    // Whether a quad holds a token scale that is no finite f16 value is known to all waves an iteration before the quad's turn, so
+    // that nobody waits for it: flag q & 1 is that of quad q, set in iteration q - 2 and read in iteration q - 1; flag 2 is quad 0's.
+    uint32_t *const not_f16 = reinterpret_cast<uint32_t *>(lds + 2 * TL::LDS_BUF);
+    auto take_scales = [&](const float (&r)[PS], uint32_t flag) {
+#pragma unroll
+        for (int i = 0; i < PS; i++) {
+            rsb16[i] = _Float16(r[i]);
+            // x - f32(f16(x)) is +-0 exactly when x is a finite f16 value (inf - inf and NaN are not)
+            if (!(r[i] - float(rsb16[i]) == 0.0f)) not_f16[flag] = 1;
+        }
+    };
+    auto park_scales = [&](uint8_t *base, auto any) {
+        const uint32_t t = me();
+        if constexpr (any.value) {
+            if (t < BN) {
+#pragma unroll
+                for (int b = 0; b < 4; b++)
+                    *reinterpret_cast<float *>(base + kScaleA + (b * BN + t) * 4) = h2f(b & 1 ? rsa[b >> 1] >> 16 : rsa[b >> 1] & 0xffffu);
+            }
+#pragma unroll
+            for (int i = 0; i < PS; i++) *reinterpret_cast<float *>(base + kScaleBAny + ((t & 3) * BT + ((t % (BT * 4)) >> 2)) * 4 + i * TH) = rsb[i];
+        } else {
+            if (t < BN) *reinterpret_cast<u32x2 *>(base + kScaleA + t * 8) = rsa;
+#pragma unroll
+            for (int i = 0; i < PS; i++) *reinterpret_cast<_Float16 *>(base + kScaleB + (t % (BT * 4)) * 2 + i * TH * 2) = rsb16[i];
+        }
+    };
+    auto park = [&](uint32_t buf, auto any) {
         uint8_t *base = lds + buf * TL::LDS_BUF;
         const uint32_t t = me();
 #pragma unroll
@@ -145,14 +179,7 @@ __global__ __launch_bounds__(64 * WR * WT, WPS) void gemm_q8_0_x86_kernel(RmiGem
                 const u32x2 u = i8x4_to_f16x4(rb[i][2 * k]), v = i8x4_to_f16x4(rb[i][2 * k + 1]);
                 *reinterpret_cast<u32x4 *>(base + b_dst + i * (TH * 8) + 16 * k) = u32x4{u[0], u[1], v[0], v[1]};
             }
-        if (t < BN) *reinterpret_cast<u32x2 *>(base + kScaleA + t * 8) = rsa;
-#pragma unroll
-        for (int i = 0; i < PS; i++) {
-            const _Float16 x = _Float16(rsb[i]);
-            *reinterpret_cast<_Float16 *>(base + kScaleB + (t % (BT * 4)) * 2 + i * TH * 2) = x;
-            // x - f32(f16(x)) is +-0 exactly when x is a finite f16 value (inf - inf and NaN are not)
-            not_f16 |= __builtin_amdgcn_ballot_w64(!(rsb[i] - float(x) == 0.0f));
-        }
+        park_scales(base, any);
     };
     static_assert((BN * 8) % TH == 0, "whole rounds of weight pieces");
     static_assert((BT * 8) % TH == 0 || BT * 8 < TH, "whole rounds of token pieces");
@@ -204,12 +231,12 @@ __global__ __launch_bounds__(64 * WR * WT, WPS) void gemm_q8_0_x86_kernel(RmiGem
         const u32x2 pa = s & 1 ? u32x2{a[2], a[3]} : u32x2{a[0], a[1]}, pb = s & 1 ? u32x2{b[2], b[3]} : u32x2{b[0], b[1]};
         return __builtin_amdgcn_mfma_f32_16x16x4f16(__builtin_bit_cast(f16x4, pa), __builtin_bit_cast(f16x4, pb), zero, 0, 0, 0);
     };
-    // d: the first product of f; returns the first one of `after`, the block behind it (nullptr: none).  sc: the scale products,
-    // this block's from sc[4 blk] on or its tiles'
-    auto block = [&](const Frags &f, const Frags *after, f32x16 d, const f32x16 &sc, int blk) {
+    // d: the first product of f; returns the first one of `after`, the block behind it (nullptr: none).  scale(i, j, v): the scale
+    // product of row 4 g + v and this lane's token of tile i, j
+    auto block = [&](const Frags &f, const Frags *after, f32x16 d, auto scale) {
 #pragma unroll
         for (int s = 0; s < kSteps; s++) {
-            const int h = s & 1, i = (s >> 1) / NT, j = (s >> 1) % NT, at = 4 * (BY_TILE ? i * NT + j : blk);
+            const int h = s & 1, i = (s >> 1) / NT, j = (s >> 1) % NT;
             auto &c = acc[i][j];
             f32x16 next = d;
             if (s + 1 < kSteps || after) {
@@ -217,9 +244,11 @@ __global__ __launch_bounds__(64 * WR * WT, WPS) void gemm_q8_0_x86_kernel(RmiGem
                 asm volatile("" : "+v"(next), X86_SUMS(c));
             }
 #pragma unroll
-            for (int v = 0; v < 4; v++)
+            for (int v = 0; v < 4; v++) {
+                const float sc = scale(i, j, v);
 #pragma unroll
-                for (int beta = 0; beta < 4; beta++) c[v][2 * beta + h] = __builtin_fmaf(sc[at + v], d[4 * beta + v], c[v][2 * beta + h]);
+                for (int beta = 0; beta < 4; beta++) c[v][2 * beta + h] = __builtin_fmaf(sc, d[4 * beta + v], c[v][2 * beta + h]);
+            }
             asm volatile("" : X86_SUMS(c));
             d = next;
         }
@@ -242,19 +271,75 @@ __global__ __launch_bounds__(64 * WR * WT, WPS) void gemm_q8_0_x86_kernel(RmiGem
         for (int b = 0; b < 4; b++) {
             if (b < 3) read(f[b + 1], buf, b + 1);
             if constexpr (BY_TILE) sc = scales_by_tile(wd, xd, b);
-            d = block(f[b], b < 3 ? &f[b + 1] : nullptr, d, sc, b);
+            d = block(f[b], b < 3 ? &f[b + 1] : nullptr, d, [&](int i, int j, int v) { return sc[4 * (BY_TILE ? i * NT + j : b) + v]; });
         }
     };
 
-    load(0);
-    park(0);
-    load(1);
-    __syncthreads();
+    struct Scales {
+        f32x4v wd[NR];
+        float xd[NT];
+    };
+    auto read_scales = [&](Scales &s, uint32_t buf, int b) {
+        const uint32_t t = me();
+#pragma unroll
+        for (int i = 0; i < NR; i++) s.wd[i] = *reinterpret_cast<const f32x4v *>(lds + buf + kScaleA + (b * BN + wr + i * 16) * 4 + (t >> 4 & 3) * 16);
+#pragma unroll
+        for (int j = 0; j < NT; j++) s.xd[j] = *reinterpret_cast<const float *>(lds + buf + kScaleBAny + (b * BT + wt + j * 16) * 4 + (t & 15) * 4);
+    };
+    auto quad_any = [&](uint32_t buf) {
+        Frags f[4];
+        Scales s[4];
+        read(f[0], buf, 0);
+        f32x16 d = product(f[0], 0);
+#pragma unroll
+        for (int b = 0; b < 4; b++) {
+            if (b < 3) read(f[b + 1], buf, b + 1);
+            if (b == 0) read_scales(s[b], buf, b);
+            if (b < 3) read_scales(s[b + 1], buf, b + 1);
+            d = block(f[b], b < 3 ? &f[b + 1] : nullptr, d, [&](int i, int j, int v) { return s[b].wd[i][v] * s[b].xd[j]; });
+        }
+    };
+
     const uint32_t n_full = nb >> 2;
-    for (uint32_t q = 0; q < n_full; q++) {
+    float first[PS];
+    load_scales(0, first);
+    load_scales(1, rsb);
+    load(0);
+    if (tid < 4) not_f16[tid] = 0;
+    __syncthreads();
+    take_scales(first, 2);
+    park(0, std::false_type());
+    take_scales(rsb, 1);
+    load(1);
+    load_scales(2, rsb);
+    __syncthreads();
+    uint32_t q = 0, any = __builtin_amdgcn_readfirstlane(int(not_f16[2]));
+    for (; q < n_full && !any; q++) {
+        const uint32_t next = not_f16[(q + 1) & 1];
         quad((q & 1) * TL::LDS_BUF);
-        park((q + 1) & 1);  // (behind the last quad: that quad again, read by nobody)
+        park((q + 1) & 1, std::false_type());  // (behind the last quad: that quad again, read by nobody)
+        take_scales(rsb, q & 1);
         load(q + 2);
+        load_scales(q + 3, rsb);
+        any = __builtin_amdgcn_readfirstlane(int(next));
+        __syncthreads();
+    }
+    // A quad with a scale that is no f16 value: what is left has scale products of the vector ALU.  The quad is in its buffer, but for
+    // such scales, and the next one in registers.
+    if (any && q < n_quads) {
+        const u32x2 wd = rsa;
+        rsa = *(gptr_u2)(w_base + (as_off + (q >> 1) * 128 + (q & 1) * 8));
+        load_scales(q, rsb);
+        park_scales(lds + (q & 1) * TL::LDS_BUF, std::true_type());
+        rsa = wd;
+        load_scales(q + 1, rsb);
+        __syncthreads();
+    }
+    for (; q < n_full; q++) {
+        quad_any((q & 1) * TL::LDS_BUF);
+        park((q + 1) & 1, std::true_type());
+        load(q + 2);
+        load_scales(q + 2, rsb);
         __syncthreads();
     }
     // the rest of a quad (the reference multiplies no others), block by block: where an instruction takes four blocks' scales they
@@ -263,45 +348,22 @@ __global__ __launch_bounds__(64 * WR * WT, WPS) void gemm_q8_0_x86_kernel(RmiGem
     for (uint32_t b = 0; b < (nb & 3); b++) {
         Frags f;
         read(f, rest, int(b));
-        const uint32_t at = rest + b * 2 - (BY_TILE ? 0 : g * 2), t = me();
-        block(f, nullptr, product(f, 0),
-              outer(u32x2{*reinterpret_cast<const uint16_t *>(sc_a(t) + at), 0u}, u32x2{*reinterpret_cast<const uint16_t *>(sc_b(t) + at), 0u}), 0);
+        f32x16 sc;
+        if (any) {
+            Scales s;
+            read_scales(s, rest, int(b));
+#pragma unroll
+            for (int k = 0; k < 4 * NR * NT; k++) sc[k] = s.wd[k / (4 * NT)][k & 3] * s.xd[(k >> 2) % NT];
+        } else {
+            const uint32_t at = rest + b * 2 - (BY_TILE ? 0 : g * 2), t = me();
+            sc = outer(u32x2{*reinterpret_cast<const uint16_t *>(sc_a(t) + at), 0u}, u32x2{*reinterpret_cast<const uint16_t *>(sc_b(t) + at), 0u});
+        }
+        block(f, nullptr, product(f, 0), [&](int i, int j, int v) { return sc[4 * (i * NT + j) + v]; });
     }
 
     uint32_t again = tid;
     asm volatile("" : "+v"(again));  // (what follows is not kept through the loop)
     const uint32_t lane1 = again & 63, fr1 = lane1 & 15, g1 = lane1 >> 4;
-    if (__syncthreads_or(not_f16 != 0)) {
-        // Token scales that are not f16 values: the tile again, block by block straight from memory, with scale products and dots
-        // of the vector ALU.  Slow, and only a caller's own scales get here.
-#pragma unroll
-        for (int i = 0; i < NR; i++)
-#pragma unroll
-            for (int j = 0; j < NT; j++) {
-                const uint32_t row0 = wr + i * 16 + g1 * 4, tok = wt + j * 16 + fr1, tk = tok < last_tok ? tok : last_tok;
-                const uint32_t t = (row0 >> 3) < last_tile ? row0 >> 3 : last_tile;
-                const gptr_u8 wp = w_base + size_t(t) * tile_bytes;
-#pragma unroll
-                for (int v = 0; v < 4; v++)
-#pragma unroll
-                    for (int l = 0; l < 8; l++) acc[i][j][v][l] = 0.0f;
-#pragma unroll 1
-                for (uint32_t b = 0; b < nb; b++) {
-                    const float xd = *(gptr_f32)(xs_base + (size_t(tk) * nb + b) * 4);
-#pragma unroll
-                    for (int v = 0; v < 4; v++) {
-                        const uint32_t r = (row0 & 7) + v;
-                        const float sc = h2f(*(gptr_u16)(wp + (b >> 3) * 128 + r * 16 + (b & 7) * 2)) * xd;
-#pragma unroll
-                        for (int l = 0; l < 8; l++) {
-                            const int wq = int(*(gptr_u32)(wp + p.n_oct * 128 + (b >> 2) * 1024 + r * 128 + l * 16 + (b & 3) * 4));
-                            const int xq = int(*(gptr_u32)(x_base + (size_t(tk) * p.n_in + b * 32 + l * 4)));
-                            acc[i][j][v][l] = __builtin_fmaf(sc, float(__builtin_amdgcn_sdot4(wq, xq, 0, false)), acc[i][j][v][l]);
-                        }
-                    }
-                }
-            }
-    }
 #pragma unroll
     for (int j = 0; j < NT; j++) {
         const uint32_t tok = tok0 + wt + j * 16 + fr1;
@@ -329,7 +391,7 @@ __global__ __launch_bounds__(64 * WR * WT, WPS) void gemm_q8_0_x86_kernel(RmiGem
 template <int NR, int NT, int WR, int WT, int WPS>
 int launch(const RmiGemvProblem &p, uint32_t n_tokens, hipStream_t s) {
     using TL = X86Tile<NR, NT, WR, WT>;
-    constexpr size_t lds = 2 * TL::LDS_BUF;
+    constexpr size_t lds = TL::LDS;
     auto kernel = gemm_q8_0_x86_kernel<NR, NT, WR, WT, WPS>;
     if constexpr (lds > 64 * 1024) {
         static const hipError_t asked = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, int(lds));

@@ -1,5 +1,7 @@
 """Q8_0 products of more than eight tokens in the x86-64 order on the matrix cores: every token's bits are those of the
 eight-token GEMV (held to the oracle by test_gpu_q8_0.py) and, for some tokens, of the restated AVX2 kernel itself."""
+import time
+
 import numpy as np
 import pytest
 
@@ -74,3 +76,43 @@ def test_special_scales(hip):
     nan = np.isnan(eights)
     assert np.array_equal(np.isnan(whole), nan)
     assert np.array_equal(whole.view(np.uint32)[~nan], eights.view(np.uint32)[~nan])
+
+
+# tiles of 32 x 32, of 64 x 64 and of 64 x 16, eight whole quads of blocks and one block
+@pytest.mark.parametrize("n_out,n_in,tokens", [(3005, 1056, 300), (4083, 1056, 450), (20003, 1056, 12)])
+def test_a_scale_that_is_no_f16_value_at_any_block(hip, n_out, n_in, tokens):
+    """Scales are f16 values, as the quantizer leaves them, but for one: in the first quad, at both ends of inner ones, in the last
+    and in the block behind them.  The quads in front of it take the other way."""
+    rng = np.random.default_rng(n_out)
+    kernel = hip.kernel.Q8Kernel(hip.synth.q8_0_weight(9, n_out, n_in), n_in, n_out)
+    q = rng.integers(-127, 128, (tokens, n_in), dtype=np.int8)
+    f16 = rng.uniform(0, 2, (tokens, n_in // 32)).astype(np.float16).astype(np.float32)
+    for block in (None, 0, 3, 4, 11, 20, 31, 32):
+        s = f16.copy()
+        if block is not None:
+            s[tokens * 2 // 3, block] = 0.1
+        whole, eights = _run(hip.hip, kernel, q, s, n_out, n_out, 0, n_out)
+        assert np.array_equal(whole.view(np.uint32), eights.view(np.uint32)), block
+
+
+def test_any_token_scale_takes_about_as_long(hip):
+    """Scales that are f16 values and others: the same work but for one vector instruction in ten (measured 1.03; 2 is far from
+    both that and a second, slower pass over the tile, which took 14 times as long)."""
+    H, (n_out, n_in, tokens) = hip.hip, (4096, 1024, 512)
+    rng = np.random.default_rng(4)
+    kernel = hip.kernel.Q8Kernel(hip.synth.q8_0_weight(2, n_out, n_in), n_in, n_out)
+    d_q = H.DeviceBuffer.from_array(rng.integers(-127, 128, (tokens, n_in), dtype=np.int8))
+    d_y = H.DeviceBuffer(tokens * n_out * 4)
+    scales = rng.uniform(0.5, 1, (tokens, n_in // 32)).astype(np.float16).astype(np.float32)
+    best = []
+    for s in (scales, scales * np.float32(1.0001)):
+        d_s, times = H.DeviceBuffer.from_array(s), []
+        for _ in range(5):
+            H.check(H.lib.rmi_hip_synchronize())
+            t0 = time.perf_counter()
+            for _ in range(50):
+                H.check(H.lib.rmi_hip_gemv_q8_0_dev(kernel.w.handle, d_q.ptr, d_s.ptr, d_y.ptr, tokens, n_out, 0, n_out, None))
+            H.check(H.lib.rmi_hip_synchronize())
+            times.append(time.perf_counter() - t0)
+        best.append(min(times))
+    assert best[1] < 2 * best[0], best
