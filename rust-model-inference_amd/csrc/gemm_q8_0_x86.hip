@@ -20,9 +20,9 @@
 // What bounds it: the vector ALU, 32 fma per 16 x 16 x 32 = 54 ns a SIMD with four waves on it, beside which the conversion of
 // the operands to f16 as they are staged costs 5 instructions per 4 values, shared by the waves that read them: 648 vector
 // instructions a quad of a wave's four tiles, with the two waves whose sums fit the registers.  us, with all scale products on the
-// vector ALU | as it is | as it is, no token scale an f16 value: 64 x 64 tiles, 6144 x 1024, 1024 tokens 70.8 | 69.3 | 73.5, 151936 x
+// vector ALU | as it is | as it is, no token scale an f16 value: 64 x 64 tiles, 6144 x 1024, 1024 tokens 70.8 | 69.0 | 72.5, 151936 x
 // 1024, 128 tokens 214 | 209 | 222; 32 x 32 tiles, 1024 x 3072, 512 tokens 26.1 | 25.4 | 26.6, 1024 x 2048, 512 tokens 18.5 | 18.2 |
-// 19.1; 64 x 16 tiles, 20003 x 1056, 12 tokens 12.1 | 12.4 | 12.9.  (A second pass over such a tile, from memory and without
+// 19.0; 64 x 16 tiles, 20003 x 1056, 12 tokens 12.1 | 12.1 | 12.8.  (A second pass over such a tile, from memory and without
 // staging, took 1085 us in the place of 73.5.)
 // Eight tokens to a workgroup of the GEMV with int8 dots (4 x 4 x 4) and a conversion each: 151936 x 1024, 128 tokens 529.
 #include <cmath>
@@ -165,13 +165,13 @@ __global__ __launch_bounds__(64 * WR * WT, WPS) void gemm_q8_0_x86_kernel(RmiGem
             for (int i = 0; i < PS; i++) *reinterpret_cast<_Float16 *>(base + kScaleB + (t % (BT * 4)) * 2 + i * TH * 2) = rsb16[i];
         }
     };
+    const uint32_t a_dst = tid * 8;  // (kept: as it is made anew, the registers it takes keep the conversions behind the last block's sums)
     auto park = [&](uint32_t buf, auto any) {
         uint8_t *base = lds + buf * TL::LDS_BUF;
-        const uint32_t t = me();
 #pragma unroll
         for (int i = 0; i < PA; i++)
 #pragma unroll
-            for (int b = 0; b < 4; b++) *reinterpret_cast<u32x2 *>(base + t * 8 + (b * TL::ABLK + i * (TH * 8))) = i8x4_to_f16x4(ra[i][b]);
+            for (int b = 0; b < 4; b++) *reinterpret_cast<u32x2 *>(base + a_dst + (b * TL::ABLK + i * (TH * 8))) = i8x4_to_f16x4(ra[i][b]);
 #pragma unroll
         for (int i = 0; i < PB; i++)
 #pragma unroll
@@ -315,8 +315,8 @@ __global__ __launch_bounds__(64 * WR * WT, WPS) void gemm_q8_0_x86_kernel(RmiGem
     __syncthreads();
     uint32_t q = 0, any = __builtin_amdgcn_readfirstlane(int(not_f16[2]));
     for (; q < n_full && !any; q++) {
-        const uint32_t next = not_f16[(q + 1) & 1];
         quad((q & 1) * TL::LDS_BUF);
+        const uint32_t next = not_f16[(q + 1) & 1];
         park((q + 1) & 1, std::false_type());  // (behind the last quad: that quad again, read by nobody)
         take_scales(rsb, q & 1);
         load(q + 2);
