@@ -65,7 +65,9 @@ int rmi_gemv_q8_0_tokens(const rmi_hip_weight *w, const int8_t *x_q8, const floa
         }
         return RMI_HIP_OK;
     }
-    if (n_rows && rmi_gemm_q8_0_x86_wins(n_rows, n_tokens, w->n_in)) return rmi_launch_gemm_q8_0_x86(problem_at(0), n_tokens, s);
+    const RmiGemvProblem all = problem_at(0);
+    const RmiX86Plan plan = rmi_gemm_q8_0_x86_plan(all.n_tiles * kTileRows, n_tokens, w->n_in);
+    if (plan != kX86Gemv) return rmi_launch_gemm_q8_0_x86(plan, all, n_tokens, s);
     const RmiTokenGroups g = rmi_gemv_q8_0_groups(w->n_units, uint64_t(n_rows) * w->n_in, n_tokens);
     const uint32_t together = n_tokens - g.apart, most = 65535 * g.tokens;  // a grid's second dimension
     for (uint32_t t0 = 0, n; t0 < n_tokens; t0 += n) {

@@ -404,6 +404,8 @@ int launch(const RmiGemvProblem &p, uint32_t n_tokens, hipStream_t s) {
     return RMI_HIP_OK;
 }
 
+}  // namespace
+
 // Which tile a product takes, or none (the GEMV's token groups are faster): microseconds estimated from what was measured on
 // 500..151936 rows of 256..12288 columns with 9..1000 tokens (812 products; the choice is 0.4 % over the best in the mean).
 // Tiles: what one block of k costs a compute unit that holds w workgroups: 64 x 64 0.43 alone, 0.73 for two (two fit), 32 x 32
@@ -412,9 +414,8 @@ int launch(const RmiGemvProblem &p, uint32_t n_tokens, hipStream_t s) {
 // beyond L2 each.
 // (E.g. 4096 x 1024: 16 tokens 5.1 us there, 8.0 here; 64: 8.4 and 8.1; 512: 53 and 28.  1024 x 3072: 64 tokens 14.4 and 18.3,
 // 512: 38 and 25.  151936 x 1024, 128 tokens: 529 and 208.)
-enum X86Plan { kPlanGemv, kPlan64x64, kPlan32x32, kPlan64x16 };
-X86Plan plan(uint32_t n_rows, uint32_t n_tokens, uint32_t n_in) {
-    if (n_tokens <= 8) return kPlanGemv;
+RmiX86Plan rmi_gemm_q8_0_x86_plan(uint32_t n_rows, uint32_t n_tokens, uint32_t n_in) {
+    if (n_tokens <= 8 || n_rows == 0) return kX86Gemv;
     const double cus = rmi_device_cus() > 0 ? rmi_device_cus() : 1, nb = n_in / 32, weights = double(n_rows) * n_in;
     auto estimate = [&](double fixed, uint32_t bn, uint32_t bt, const double *us, int fit) {
         const double groups = double((n_rows + bn - 1) / bn) * ((n_tokens + bt - 1) / bt);
@@ -423,7 +424,6 @@ X86Plan plan(uint32_t n_rows, uint32_t n_tokens, uint32_t n_in) {
     };
     const uint32_t n_oct = (n_in + 255) / 256;
     const RmiTokenGroups g = rmi_gemv_q8_0_groups(n_oct, uint64_t(n_rows) * n_in, n_tokens);
-    if (g.tokens == 0) return kPlan32x32;  // rows too long for the GEMV's staging
     const bool x4 = g.tokens == 8 || g.tokens == 4;
     const double work = (x4 ? 0.0222 : 0.0322) * 1e-6 * weights * (g.groups * g.tokens + g.apart) + 0.0275e-3 * n_rows * g.groups,
                  memory = 0.0232e-6 * weights * (g.tokens == 8 ? 1 : g.groups);
@@ -431,19 +431,16 @@ X86Plan plan(uint32_t n_rows, uint32_t n_tokens, uint32_t n_in) {
     const double k64[] = {0.43, 0.73}, k32[] = {0.163, 0.224, 0.317, 0.42}, k16[] = {0.186, 0.264, 0.377};
     const double t64 = estimate(3.6, 64, 64, k64, 2), t32 = estimate(3.0, 32, 32, k32, 4), t16 = n_tokens <= 16 ? estimate(3.1, 64, 16, k16, 3) : 1e30;
     const double best = t64 < t32 ? (t64 < t16 ? t64 : t16) : (t32 < t16 ? t32 : t16);
-    if (gemv < best) return kPlanGemv;
-    return best == t64 ? kPlan64x64 : best == t32 ? kPlan32x32 : kPlan64x16;
+    if (gemv < best) return kX86Gemv;
+    return best == t64 ? kX86Tile64x64 : best == t32 ? kX86Tile32x32 : kX86Tile64x16;
 }
 
-}  // namespace
-
-bool rmi_gemm_q8_0_x86_wins(uint32_t n_rows, uint32_t n_tokens, uint32_t n_in) { return plan(n_rows, n_tokens, n_in) != kPlanGemv; }
-
-int rmi_launch_gemm_q8_0_x86(const RmiGemvProblem &p, uint32_t n_tokens, hipStream_t s) {
+int rmi_launch_gemm_q8_0_x86(RmiX86Plan plan, const RmiGemvProblem &p, uint32_t n_tokens, hipStream_t s) {
     if (p.n_tiles == 0 || p.n_oct == 0 || n_tokens == 0) return RMI_HIP_OK;
-    switch (plan(p.n_tiles * 8, n_tokens, p.n_in)) {
-        case kPlan64x64: return launch<2, 2, 2, 2, 2>(p, n_tokens, s);
-        case kPlan64x16: return launch<1, 1, 4, 1, 4>(p, n_tokens, s);
-        default: return launch<1, 1, 2, 2, 4>(p, n_tokens, s);
+    switch (plan) {
+        case kX86Tile64x64: return launch<2, 2, 2, 2, 2>(p, n_tokens, s);
+        case kX86Tile32x32: return launch<1, 1, 2, 2, 4>(p, n_tokens, s);
+        case kX86Tile64x16: return launch<1, 1, 4, 1, 4>(p, n_tokens, s);
+        default: return rmi_fail(RMI_HIP_E_INVALID, "no tile size %d", int(plan));
     }
 }

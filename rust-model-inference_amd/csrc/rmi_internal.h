@@ -187,9 +187,11 @@ struct RmiTokenGroups {
     uint32_t apart;           // the last ones, in a launch of their own
 };
 RmiTokenGroups rmi_gemv_q8_0_groups(uint32_t n_oct, uint64_t weights, uint32_t n_tokens);
-// any number of tokens in one launch, the same bits (gemm_q8_0_x86.hip), and whether that is the faster way
-bool rmi_gemm_q8_0_x86_wins(uint32_t n_rows, uint32_t n_tokens, uint32_t n_in);
-int rmi_launch_gemm_q8_0_x86(const RmiGemvProblem &p, uint32_t n_tokens, hipStream_t s);
+// any number of tokens in one launch, the same bits (gemm_q8_0_x86.hip): by tiles of that size, and which size, if any, is the
+// faster way for rows that the GEMV can stage (n_rows: whole tiles of the weight)
+enum RmiX86Plan { kX86Gemv, kX86Tile64x64, kX86Tile32x32, kX86Tile64x16 };
+RmiX86Plan rmi_gemm_q8_0_x86_plan(uint32_t n_rows, uint32_t n_tokens, uint32_t n_in);
+int rmi_launch_gemm_q8_0_x86(RmiX86Plan plan, const RmiGemvProblem &p, uint32_t n_tokens, hipStream_t s);
 // rows [row_start,row_end) of n_tokens tokens of a Q8_0 or Q4_0 weight, as many GEMV launches (x86-64 order) as
 // the LDS staging of the tokens asks for; device pointers, nothing allocated
 bool rmi_gemv_q8_0_tokens_fits(const rmi_hip_weight *w);
