@@ -53,7 +53,7 @@ int rmi_gemv_q8_0_tokens(const rmi_hip_weight *w, const int8_t *x_q8, const floa
                          uint32_t y_stride, uint32_t row_start, uint32_t row_end, hipStream_t s) {
     if (!rmi_gemv_q8_0_tokens_fits(w)) return rmi_fail(RMI_HIP_E_INVALID, "n_in=%u is too long for the GEMV staging", w->n_in);
     if (n_tokens == 0) return RMI_HIP_OK;
-    const uint32_t nb = w->n_in / 32, n_rows = row_end > row_start ? row_end - row_start : 0;
+    const uint32_t nb = w->n_in / 32;
     auto problem_at = [&](uint32_t t0) {
         return make_problem(w, x_q8 + size_t(t0) * w->n_in, x_scales + size_t(t0) * nb, y + size_t(t0) * y_stride, y_stride, row_start, row_end);
     };
@@ -68,7 +68,7 @@ int rmi_gemv_q8_0_tokens(const rmi_hip_weight *w, const int8_t *x_q8, const floa
     const RmiGemvProblem all = problem_at(0);
     const RmiX86Plan plan = rmi_gemm_q8_0_x86_plan(all.n_tiles * kTileRows, n_tokens, w->n_in);
     if (plan != kX86Gemv) return rmi_launch_gemm_q8_0_x86(plan, all, n_tokens, s);
-    const RmiTokenGroups g = rmi_gemv_q8_0_groups(w->n_units, uint64_t(n_rows) * w->n_in, n_tokens);
+    const RmiTokenGroups g = rmi_gemv_q8_0_groups(w->n_units, all.n_tiles * kTileRows, n_tokens);
     const uint32_t together = n_tokens - g.apart, most = 65535 * g.tokens;  // a grid's second dimension
     for (uint32_t t0 = 0, n; t0 < n_tokens; t0 += n) {
         n = (t0 < together ? together : n_tokens) - t0;

@@ -25,7 +25,6 @@
 // 19.0; 64 x 16 tiles, 20003 x 1056, 12 tokens 12.1 | 12.1 | 12.8.  (A second pass over such a tile, from memory and without
 // staging, took 1085 us in the place of 73.5.)
 // Eight tokens to a workgroup of the GEMV with int8 dots (4 x 4 x 4) and a conversion each: 151936 x 1024, 128 tokens 529.
-#include <cmath>
 #include <type_traits>
 
 #include "rmi_internal.h"
@@ -407,31 +406,28 @@ int launch(const RmiGemvProblem &p, uint32_t n_tokens, hipStream_t s) {
 }  // namespace
 
 // Which tile a product takes, or none (the GEMV's token groups are faster): microseconds estimated from what was measured on
-// 500..151936 rows of 256..12288 columns with 9..1000 tokens (812 products; the choice is 0.4 % over the best in the mean).
-// Tiles: what one block of k costs a compute unit that holds w workgroups: 64 x 64 0.43 alone, 0.73 for two (two fit), 32 x 32
-// 0.16, 0.22, 0.32, 0.42 for one to four (four fit), 64 x 16 0.19, 0.26, 0.38 (three).  The GEMV: a wave's walk along a row
-// beside the vector ALU's work for all groups' tokens, their workgroups and the weights, which only groups of long rows read from
-// beyond L2 each.
-// (E.g. 4096 x 1024: 16 tokens 5.1 us there, 8.0 here; 64: 8.4 and 8.1; 512: 53 and 28.  1024 x 3072: 64 tokens 14.4 and 18.3,
-// 512: 38 and 25.  151936 x 1024, 128 tokens: 529 and 208.)
+// 300..160000 rows of 256..30720 columns with 9..1000 tokens (2600 products; the choice is 0.5 % over the best in the mean, 5 % or
+// more in one of thirty-five).  A tile's launch with w workgroups a compute unit costs `block` for every block of k, by the most that a unit
+// has up to four, from there on in proportion, and `group` a workgroup of a unit for what stands around its loop; within 3 % of what was
+// measured.
+// (E.g. 4096 x 1024: 16 tokens 5.1 us by groups, 8.0 by tiles; 64: 8.4 and 8.1; 512: 53 and 26.  1024 x 3072: 64 tokens 14.4 and
+// 18.3, 512: 38 and 25.  151936 x 1024, 128 tokens: 529 and 209.  33166 x 6144, 17 tokens: 146 and 95.)
 RmiX86Plan rmi_gemm_q8_0_x86_plan(uint32_t n_rows, uint32_t n_tokens, uint32_t n_in) {
     if (n_tokens <= 8 || n_rows == 0) return kX86Gemv;
-    const double cus = rmi_device_cus() > 0 ? rmi_device_cus() : 1, nb = n_in / 32, weights = double(n_rows) * n_in;
-    auto estimate = [&](double fixed, uint32_t bn, uint32_t bt, const double *us, int fit) {
-        const double groups = double((n_rows + bn - 1) / bn) * ((n_tokens + bt - 1) / bt);
-        const uint64_t w = uint64_t((groups + cus - 1) / cus);
-        return fixed + nb * (double(w / fit) * us[fit - 1] + (w % fit ? us[w % fit - 1] : 0.0));
+    const double cus = rmi_device_cus() > 0 ? rmi_device_cus() : 1, nb = n_in / 32;
+    struct Tile {
+        uint32_t rows, tokens;
+        double fixed, group, block[4], more, from;
     };
-    const uint32_t n_oct = (n_in + 255) / 256;
-    const RmiTokenGroups g = rmi_gemv_q8_0_groups(n_oct, uint64_t(n_rows) * n_in, n_tokens);
-    const bool x4 = g.tokens == 8 || g.tokens == 4;
-    const double work = (x4 ? 0.0222 : 0.0322) * 1e-6 * weights * (g.groups * g.tokens + g.apart) + 0.0275e-3 * n_rows * g.groups,
-                 memory = 0.0232e-6 * weights * (g.tokens == 8 ? 1 : g.groups);
-    const double gemv = 2.7 + std::pow(std::pow(0.363 * n_oct, 1.5) + std::pow(work + memory, 1.5), 2.0 / 3) + (g.apart ? 19.7 + 0.0232e-6 * weights : 0.0);
-    const double k64[] = {0.43, 0.73}, k32[] = {0.163, 0.224, 0.317, 0.42}, k16[] = {0.186, 0.264, 0.377};
-    const double t64 = estimate(3.6, 64, 64, k64, 2), t32 = estimate(3.0, 32, 32, k32, 4), t16 = n_tokens <= 16 ? estimate(3.1, 64, 16, k16, 3) : 1e30;
+    auto us = [&](const Tile &t) {
+        const double w = double((n_rows + t.rows - 1) / t.rows) * ((n_tokens + t.tokens - 1) / t.tokens) / cus;
+        return t.fixed + t.group * w + nb * (w <= 4 ? t.block[w <= 1 ? 0 : w <= 2 ? 1 : w <= 3 ? 2 : 3] : t.more * (w + t.from));
+    };
+    const double t64 = us({64, 64, 3.2, 1.20, {0.428, 0.647, 1.003, 1.285}, 0.319, 0.54}),
+                 t32 = us({32, 32, 2.6, 0.44, {0.173, 0.229, 0.304, 0.383}, 0.0895, 0.83}),
+                 t16 = n_tokens <= 16 ? us({64, 16, 2.8, 0.57, {0.199, 0.268, 0.356, 0.487}, 0.1058, 1.06}) : 1e30;
     const double best = t64 < t32 ? (t64 < t16 ? t64 : t16) : (t32 < t16 ? t32 : t16);
-    if (gemv < best) return kX86Gemv;
+    if (rmi_gemv_q8_0_groups((n_in + 255) / 256, n_rows, n_tokens).us < best) return kX86Gemv;
     return best == t64 ? kX86Tile64x64 : best == t32 ? kX86Tile32x32 : kX86Tile64x16;
 }
 

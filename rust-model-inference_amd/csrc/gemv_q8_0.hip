@@ -6,6 +6,8 @@
 // taking fma(f32(wd)*xs[b], float(sum_{k=4L..4L+3} w*x), acc_L) block after
 // block, then hsum_ps (src/ops/dot.rs:447-456).  Eight GPU lanes hold the eight
 // accumulators of one row, so results match that kernel bit for bit.
+#include <cmath>
+
 #include "device_ahead.h"
 #include "device_math.h"
 #include "device_quant.h"
@@ -1426,33 +1428,66 @@ int rmi_launch_copy(const void *src, void *dst, size_t nbytes, hipStream_t s) {
     return RMI_HIP_OK;
 }
 
+// Microseconds of more than eight tokens in groups of g: a wave's walk along a row, beside the vector ALU's work for all groups'
+// tokens (ragged ones twice), the groups' workgroups and the weights, which all groups read.  Fitted to those of 2600 products of
+// 300..160000 rows of 256..14336 columns, 9..1000 tokens, where groups are not far from the fastest way; 8 % off in the mean (rows too
+// long for eight staged tokens 13 %, and for four, of up to 30720 columns, 25 %).
+static double groups_us(uint32_t n_oct, uint32_t n_rows, uint32_t g, uint32_t groups, bool eights_fit, bool dots_on_mfma) {
+    const double k_rows = 1e-3 * n_rows, m = 0.256 * k_rows * n_oct;
+    // (from seventeen octets on eight staged tokens leave room for three workgroups a compute unit instead of four)
+    const double crowded = n_oct > 16 && k_rows * groups >= 16 ? 1.15 : 1.0;
+    if (eights_fit && g == 8) return crowded * (2.7 + 0.32 * n_oct + m * (0.0237 * 8 * groups + 0.032 + 0.0082 * (groups - 1)) + 0.030 * k_rows * groups);
+    if (eights_fit) return 2.5 + 0.32 * n_oct + m * (0.0245 * g * groups + 0.1) + 0.029 * k_rows * groups;
+    const double slower[] = {0, 3.1, 1.6, 1.3, 1.3}, work = m * (0.0312 * g * groups + 0.08 + 0.016 * (groups - 1));
+    return (1.0 + std::pow(std::pow(0.394 * n_oct, 1.3) + std::pow(work, 1.3), 1 / 1.3)) * (dots_on_mfma ? 1.0 : slower[g < 4 ? g : 4]);
+}
+
 // All groups go out in one launch (they re-read the weight from L2): a launch behind it for what is beyond whole groups takes as
 // long as the groups together (1024 x 3072: 13 tokens 13.4 us as 8 and 8, 7.4 as one launch; 9 tokens 9.2 as 8 and 1, 7.3).
-// A group is eight tokens where the kernel with its dots on the matrix cores can stage them; four where that leaves out a group's
-// half (up to 28 tokens: 4096 x 4096, 9 tokens 11.8 us by fours, 18.4 by eights, 18 tokens 13.7 | 19.0; from 32 on level), and
-// on longer rows, for the kernel that can stage more there is twice to three times as slow (8192 columns, 8 tokens, by fours |
-// by what fits: 1024 rows 14.4 | 40.7, 4096 rows 20.8 | 38.2; 5 tokens 14.6 | 25.5 and 20.8 | 23.5).  Of a large matrix, where a
-// group more costs as much as the matrix again, neither, but for eight tokens of a long row (12288 x 8192: 8 tokens 33.6 | 55.0,
-// 5 tokens 40.1 | 31.5, 13 tokens 68 | 52), and there up to half a group is a launch of its own (151936 x 1024, 9 tokens 67 us
-// and 76 as two groups, 20 tokens 104 and 110; one token more on long rows: 4096 x 12288, 9 tokens 42 and 49).
-RmiTokenGroups rmi_gemv_q8_0_groups(uint32_t n_oct, uint64_t weights, uint32_t n_tokens) {
+// More than eight tokens go by eights or by fours, whichever leaves less to do by the estimates (4096 x 4096, 9 tokens 11.8 us by
+// fours, 18.4 by eights), and by fours on rows too long for the kernel with its dots on the matrix cores to stage eight, as the
+// kernel that can stage more there is twice to three times as slow (8192 columns, 8 tokens, by fours | by what fits: 1024 rows 14.4 |
+// 40.7, 4096 rows 20.8 | 38.2; 9984 columns, 5 tokens: 3965 rows 20.8 | 33.2).  Up to seven tokens of a large matrix with such
+// rows, where a group more costs as much as the matrix again, are one group if they fit (5 tokens: 14979 x 11200 42.4 us, by fours
+// 63.6; 7 tokens: 22598 x 7424 57.7 and 59.0).  Five or six of which only four fit are four and the rest where two groups' waves, two
+// workgroups a compute unit, would take a second round (5 tokens: 5077 x 11776 39.5, by fours 46.8; 6528 x 14080 48.9 and 78.3; 13206 x
+// 12704 67.3 and 73.6; but 1380 x 12800 34.6 and 22.8; 6 of 13617 x 12320 64.1 and 72.5).
+RmiTokenGroups rmi_gemv_q8_0_groups(uint32_t n_oct, uint32_t n_rows, uint32_t n_tokens) {
     constexpr size_t kLds = 64 * 1024;
-    constexpr uint64_t kLarge = 64u << 20, kLong = 36u << 20;
-    const bool rows_fit = gemv_x4_bytes(8, n_oct, 4) <= kLds, large = weights >= kLarge;
-    RmiTokenGroups g{8, 0, 0};
-    if (rows_fit) {
-        if (!large && n_tokens > 8 && n_tokens <= 28 && (n_tokens - 1) % 8 < 4) g.tokens = 4;
-    } else {
-        const uint32_t fit = uint32_t(kLds / (size_t(n_oct) * 288));
-        const bool fours = !large || n_tokens == 8 || (n_tokens > fit && n_tokens < 8);
-        g.tokens = fours && gemv_x4_bytes(4, n_oct, 4) <= kLds ? 4 : fit < 8 ? fit : 8;
-        if (g.tokens == 0) return g;
+    const uint32_t most = n_oct ? uint32_t(kLds / (size_t(n_oct) * 288)) : 8, fit = most < 8 ? most : 8;
+    const bool eights = gemv_x4_bytes(8, n_oct, 4) <= kLds, fours = gemv_x4_bytes(4, n_oct, 4) <= kLds, large = uint64_t(n_rows) * n_oct * 256 >= (64u << 20);
+    auto by = [&](uint32_t g) {
+        const uint32_t groups = (n_tokens + g - 1) / g;
+        return RmiTokenGroups{g, groups, 0, groups_us(n_oct, n_rows, g, groups, eights, eights || (fours && g == 4))};
+    };
+    if (fit == 0) return RmiTokenGroups{};
+    if (n_tokens <= (eights ? 8 : large && n_tokens < 8 ? fit : 4) && n_tokens <= fit) return by(n_tokens);
+    if (eights) {
+        const RmiTokenGroups by8 = by(8), by4 = by(4);
+        return by8.us <= by4.us ? by8 : by4;
     }
-    if (n_tokens < g.tokens) g.tokens = n_tokens;
-    const uint32_t rest = n_tokens % g.tokens;
-    if (n_tokens > g.tokens && (large ? rest <= g.tokens / 2 : !rows_fit && rest == 1 && weights >= kLong)) g.apart = rest;
-    g.groups = (n_tokens - g.apart + g.tokens - 1) / g.tokens;
+    RmiTokenGroups g = by(fours ? 4 : fit);
+    const uint32_t cus = uint32_t(rmi_device_cus() > 0 ? rmi_device_cus() : 1);
+    if (fit == 4 && n_rows > 16 * cus && (n_tokens == 5 || n_tokens == 6)) g.groups = 1, g.apart = n_tokens - 4;
     return g;
+}
+
+// A matrix of a few MB at several tokens is a launch of a few hundred waves with a long instruction stream each (the x86-64 order
+// costs about 30 vector instructions a token and octet): its tokens are spread over workgroups, two or four to each, which re-read
+// the weight from L2 and finish in a half or a quarter of the time (every token's result is that of any other grouping: a token has
+// its own accumulators).  Eight tokens to a wave use the matrix cores better than four: they are halved until a launch has four
+// waves a compute unit, on rows of three octets and more six, and in several groups seven from five and eight from nine on.  us, halved up to eight
+// waves | up to four: 13468 x 512, 8 tokens 6.3 | 5.5, 15790 x 3840, 8 tokens 25.7 | 19.9; 8684 x 2560, 8 tokens 11.4 | 13.4,
+// 4949 x 6656, 16 tokens 26.8 | 44.9.
+uint32_t rmi_gemv_q8_0_per_workgroup(uint32_t n_waves, uint32_t n_oct, uint32_t group, uint32_t n_tokens) {
+    const uint32_t cus = uint32_t(rmi_device_cus() > 0 ? rmi_device_cus() : 1);
+    uint32_t groups = (n_tokens + group - 1) / group;
+    const uint32_t waves_of_eights = n_oct < 3 ? 4 : n_oct < 5 || groups == 1 ? 6 : n_oct < 9 ? 7 : 8;
+    while (group > 2 && group % 2 == 0 && n_waves * groups < (group == 8 ? waves_of_eights : 4) * cus) {
+        group >>= 1;
+        groups = (n_tokens + group - 1) / group;
+    }
+    return group;
 }
 
 int rmi_launch_gemv_q8_0_single(const RmiGemvProblem &problem, uint32_t group, hipStream_t s, uint32_t n_tokens) {
@@ -1463,15 +1498,7 @@ int rmi_launch_gemv_q8_0_single(const RmiGemvProblem &problem, uint32_t group, h
     const uint32_t tpw = rmi_gemv_tiles_per_wave(p.n_oct, p.n_tiles, group);
     const uint32_t n_waves = (p.n_tiles + tpw - 1) / tpw, cus = uint32_t(rmi_device_cus() > 0 ? rmi_device_cus() : 1);
     {
-        // A matrix of a few MB at several tokens is a launch of a few hundred waves with a long instruction stream
-        // each (the x86-64 order costs about 30 vector instructions a token and octet): its tokens are spread over
-        // workgroups, two or four to each, which re-read the weight from L2 and finish in a half or a quarter of
-        // the time (every token's result is that of any other grouping: a token has its own accumulators).
-        uint32_t per_group = group, groups = (n_tokens + group - 1) / group;
-        while (per_group > 2 && per_group % 2 == 0 && n_waves * groups < (per_group == 8 ? 8 : 4) * cus) {
-            per_group >>= 1;
-            groups = (n_tokens + per_group - 1) / per_group;
-        }
+        const uint32_t per_group = rmi_gemv_q8_0_per_workgroup(n_waves, p.n_oct, group, n_tokens), groups = (n_tokens + per_group - 1) / per_group;
         if (groups > 1) {
             // the waves of a workgroup share the staged tokens of their group: as many as leave every compute unit
             // two workgroups or more

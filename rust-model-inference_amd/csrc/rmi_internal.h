@@ -181,12 +181,15 @@ struct RmiGemvProblem {
 // n_tokens tokens in one launch, in groups of `group` (<= 8, <= n_tokens) or fewer; where they don't come out even the last group
 // begins earlier, and what two groups share is written twice, with the same bits
 int rmi_launch_gemv_q8_0_single(const RmiGemvProblem &p, uint32_t group, hipStream_t s, uint32_t n_tokens);
-// how n_tokens (> 0) tokens of a matrix of that many weights are grouped; tokens = 0: not even one's activation fits the staging
+// how n_tokens (> 0) tokens of a matrix of that many octets and rows are grouped; tokens = 0: not even one's activation fits the staging
 struct RmiTokenGroups {
     uint32_t tokens, groups;  // of a group; of one launch
     uint32_t apart;           // the last ones, in a launch of their own
+    double us;                // of the launch, estimated for more than eight tokens
 };
-RmiTokenGroups rmi_gemv_q8_0_groups(uint32_t n_oct, uint64_t weights, uint32_t n_tokens);
+RmiTokenGroups rmi_gemv_q8_0_groups(uint32_t n_oct, uint32_t n_rows, uint32_t n_tokens);
+// how many tokens of a launch in groups a workgroup takes: fewer where that many waves (a token group's) leave compute units idle
+uint32_t rmi_gemv_q8_0_per_workgroup(uint32_t n_waves, uint32_t n_oct, uint32_t group, uint32_t n_tokens);
 // any number of tokens in one launch, the same bits (gemm_q8_0_x86.hip): by tiles of that size, and which size, if any, is the
 // faster way for rows that the GEMV can stage (n_rows: whole tiles of the weight)
 enum RmiX86Plan { kX86Gemv, kX86Tile64x64, kX86Tile32x32, kX86Tile64x16 };
