@@ -4,7 +4,9 @@ import numpy as np
 import pytest
 import ruvenex_gen as G
 import ruvenex_plain as P
-from folder_helpers import BF16, F32, TOL, Opener, feed, rel
+import vogizen_gen
+import vogizen_plain
+from folder_helpers import BF16, F32, TOL, Opener, feed, feed_layers, rel
 
 pytestmark = pytest.mark.gpu
 
@@ -48,3 +50,25 @@ def test_bits_are_those_of_heads_of_any_size(hip, tmp_path, dtype, heads, kv_hea
     a, b = feed(s, t, sizes), feed(s2, t, sizes)
     o.close()
     assert np.array_equal(a.view(np.uint32), b.view(np.uint32)), np.flatnonzero((a != b).any(-1))[:8]
+
+
+@pytest.mark.parametrize("dtype", [F32, BF16])
+@pytest.mark.parametrize("dim,window", [(128, 600), (64, 1000), (128, 1100), (64, 2000), (128, 2100)])
+def test_parts_behind_a_window(hip, tmp_path, dtype, dim, window):
+    """Five parts of 128 keys and more whose first key is not the sequence's: single tokens from the window's end on and where the
+    cache's rows come round.  The attention alone, all else silenced: what the layer adds against the plain statement."""
+    cfg = vogizen_gen.config([vogizen_gen.latent(heads=3, dim=dim, vdim=dim, window=window, scale=2 / dim**0.5, ff=None)], loop=None)
+    w = vogizen_gen.weights(cfg, 5)
+    w["l0.side.norm"] = np.zeros_like(w["l0.side.norm"])
+    n = 2 * window + 40
+    o = Opener(hip, tmp_path, vogizen_gen)
+    s, _ = o(cfg, w, dtype, n)
+    t = vogizen_gen.tokens(cfg, n)
+    ref = []
+    vogizen_plain.forward(cfg, w, t, layers_out=ref)
+    half = window // 2
+    got = feed_layers(s, t, [half, window - 2 - half] + [1] * 8 + [half, window - 50 - half] + [1] * 84)[0]
+    o.close()
+    x0 = vogizen_plain.embedding(cfg, w, np.asarray(t))
+    at = np.r_[window - 2:window + 6, 2 * window - 44:n]
+    assert rel((got - x0)[at], (ref[0] - x0)[at]) < TOL[dtype]
