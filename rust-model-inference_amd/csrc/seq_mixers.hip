@@ -814,26 +814,45 @@ __device__ __forceinline__ void attn_split(const RmiAttnShape &shape, const RmiA
                 auto part_at = [&](uint32_t i) { return (i < parts ? i : parts - 1) * pf; };
                 // lane i the maximum of part i, lane kMaxParts + i its sum
                 const float ml = __hip_atomic_load(ws + part_at(lane % kMaxParts) + c + lane / kMaxParts * 16, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                float ov[N], m = -INFINITY, o = 0.0f, sum = 0.0f;
-                for (uint32_t p0 = 0; p0 < parts; p0 += N) {
+                float ov[N], o = 0.0f, sum = 0.0f;
+                auto load = [&](uint32_t p0) {
 #pragma unroll
                     for (uint32_t j = 0; j < N; j++)
                         ov[j] = __hip_atomic_load(ws + part_at(p0 + j) + 32 + e, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                };
+                load(0);
+                // the largest of eight parts' maxima in all their lanes, then of all parts up to these eight
+                constexpr uint32_t G = N == 8 ? 1 : kMaxParts / 8;
+                const float top8 = max8_lanes(lane < parts ? ml : -INFINITY);
+                float top[G], mine = 0.0f;
 #pragma unroll
-                    for (uint32_t g = 0; g < N; g += 8) {
-                        if (p0 + g >= parts) break;
-                        const float top = fmaxf(m, wave_max_f32(lane < parts && lane / 8 == (p0 + g) / 8 ? ml : -INFINITY));
-                        const float ref = top == -INFINITY ? 0.0f : top, keep = exp_t<T>(m - ref), f = exp_t<T>(ml - ref);
-                        sum *= keep;
-                        o *= keep;
+                for (uint32_t g = 0; g < G; g++) {
+                    top[g] = fmaxf(g ? top[g - 1] : -INFINITY, of_lane(top8, 8 * g));
+                    mine = G == 1 || lane / 8 == g ? top[g] : mine;
+                }
+                const float f = exp_t<T>(ml - (mine == -INFINITY ? 0.0f : mine));
+                for (uint32_t p0 = 0; p0 < parts; p0 += N) {
+                    if (p0 > 0) load(p0);
 #pragma unroll
-                        for (uint32_t j = g; j < g + 8; j++)
-                            if (p0 + j < parts) {
-                                const float fj = of_lane(f, p0 + j);
-                                sum = __builtin_fmaf(of_lane(ml, kMaxParts + p0 + j), fj, sum);
-                                o = __builtin_fmaf(ov[j], fj, o);
+                    for (uint32_t g = 0; g < N / 8; g++) {
+                        const uint32_t first = p0 + 8 * g;
+                        if (first >= parts) break;
+                        if (first > 0) {  // (what eight parts came to, against the larger maximum)
+                            float before = top[0], now = top[0];
+#pragma unroll
+                            for (uint32_t i = 1; i < G; i++)
+                                if (first == 8 * i) before = top[i - 1], now = top[i];
+                            const float keep = exp_t<T>(before - (now == -INFINITY ? 0.0f : now));
+                            sum *= keep;
+                            o *= keep;
+                        }
+#pragma unroll
+                        for (uint32_t j = 0; j < 8; j++)
+                            if (first + j < parts) {
+                                const float fj = of_lane(f, first + j);
+                                sum = __builtin_fmaf(of_lane(ml, kMaxParts + first + j), fj, sum);
+                                o = __builtin_fmaf(ov[8 * g + j], fj, o);
                             }
-                        m = top;
                     }
                 }
                 finish(e, o, sum);
