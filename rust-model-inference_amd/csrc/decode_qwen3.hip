@@ -1094,11 +1094,14 @@ __global__ __launch_bounds__(kAttnSplitThreads) void attn128_weights_pv_kernel(
     }
 }
 
-// With parts, compute units that have no head fetch the output product's weights meanwhile, if they are no more than this.  28
-// layers of width 1024 (2.2 MB a layer), a prompt of 70 | 512 | 1000 tokens and 32 more: 20.1 | 28.58 | 36.1 ms without,
-// 19.9 | 28.26 | 35.6 with; eight layers of 2048 (4.5 MB) 11.32 and 11.25; four of 4096 with the 18 MB of each 13.58 and 13.59.
-// The gate, up, down or the next q/k/v weights too, 9 to 17 MB: 28.7 to 29.4 ms at 512, more in the attention than saved behind it.
-constexpr size_t kAttnAheadBytes = 8u << 20;
+// With parts, compute units that have no head fetch the output product's weights meanwhile, if they are no more than this, and no
+// less than so much a key: what the product saves goes with the bytes, what the attention loses with the keys it reads meanwhile.
+// us a token without | with, 28 layers of width 1024 (2.2 MB a layer) at 70 | 150 | 300 | 512 | 900 | 980 | 1100 | 1240 keys: 573 | 569,
+// 601 | 594, 643 | 637, 714 | 708, 855 | 870, 930 | 901, 892 | 905, 932 | 948, so up to 825 keys; eight layers of 2048 (4.5 MB) at
+// 300 | 700 | 900 | 1200: 282 | 278, 320 | 319, 362 | 350, 394 | 383; four of 4096 with the 18 MB of each the same.
+// The gate, up, down or the next q/k/v weights too, 9 to 17 MB: 28.7 to 29.4 ms for a prompt of 512 and 32 tokens, 28.3 as it is,
+// more in the attention than saved behind it.
+constexpr size_t kAttnAheadBytes = 8u << 20, kAttnAheadKeyBytes = 2700;
 // One position's attention straight from its f32 q | k | v: the launch with the p.v sums of a head split over parts.
 // Four parts from 64 keys on (measured over 512..638 keys, 28 layers: 0.840 ms a generated token with one part, 0.789
 // with two, 0.779 with four); below, the p.v sums are a few terms and one workgroup a head is enough.
@@ -1339,7 +1342,7 @@ int enqueue_step(rmi_hip_qwen3 *s, uint32_t step, hipStream_t st) {
             const size_t half = 64;
             AttnFromQkv fq{s->qkv, qn, kn, s->cos_t + size_t(step) * half, s->sin_t + size_t(step) * half,
                            s->k_cache + row, s->v_cache + row, c.eps, RmiAhead{}};
-            rmi_gemv_q8_0_ahead(s->w_o[l], kAttnAheadBytes, &fq.ahead);
+            rmi_gemv_q8_0_ahead(s->w_o[l], kAttnAheadKeyBytes * (step + 1), kAttnAheadBytes, &fq.ahead);
             launch_attention128_from_qkv(s->k_cache + layer_base, s->v_cache + layer_base, step, s->kv_stride, c.n_head, c.n_head_kv,
                                          s->act_q8, s->act_scales, rnd, fq, st);
         } else if (rmi_gemv_q8_0_norm_rope_fusable(s->w_qkv[l], c.n_head, c.n_head_kv, c.head_dim_k, c.head_dim_v)) {

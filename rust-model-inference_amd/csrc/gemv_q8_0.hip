@@ -1516,9 +1516,9 @@ int rmi_launch_gemv_q8_0_single(const RmiGemvProblem &problem, uint32_t group, h
     return dispatch_gemv(group, &p, nullptr, nullptr, n_waves, wpg, tpw, p.n_oct, s);
 }
 
-void rmi_gemv_q8_0_ahead(const rmi_hip_weight *w, size_t most, RmiAhead *ahead) {
-    const size_t tile = size_t(w->n_units) * kOctetBytes;
-    if (w->n_units <= kDeepMaxOct && w->n_tiles <= kDeepMaxTiles && tile * w->n_tiles <= most) ahead->add(w->data, tile, w->n_tiles);
+void rmi_gemv_q8_0_ahead(const rmi_hip_weight *w, size_t least, size_t most, RmiAhead *ahead) {
+    const size_t tile = size_t(w->n_units) * kOctetBytes, all = tile * w->n_tiles;
+    if (w->n_units <= kDeepMaxOct && w->n_tiles <= kDeepMaxTiles && all >= least && all <= most) ahead->add(w->data, tile, w->n_tiles);
 }
 
 bool rmi_gemv_q8_0_norm_fusable(const rmi_hip_weight *w) {
