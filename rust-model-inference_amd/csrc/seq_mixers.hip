@@ -532,7 +532,7 @@ struct SplitPlan {
 // TAPS > 0: heads fill the kernel (keys and values of BUCKET elements) behind a convolution of that many taps, so that every size
 // below but the number of heads is the compiler's to know: a token runs every instruction once, so their number is its time.
 // A launch of 28 layers in bf16, 16 heads over 8 of 128, four taps, at 150 | 320 | 2060 positions, with the sizes as arguments,
-// 64-bit offsets and eight parts' loads in the last merge: 10.1 | 11.2 | 14.3 us; as it is: 7.9 | 8.4 | 12.0.
+// 64-bit offsets and eight parts' loads in the last merge: 10.1 | 11.2 | 14.3 us; as it is: 7.8 | 8.4 | 11.0.
 template <typename T, int BUCKET, bool STEP, bool EVERY = true, int TAPS = 0>
 __device__ __forceinline__ void attn_split(const RmiAttnShape &shape, const RmiAttnArgs &a, uint32_t block, const SplitPlan &plan, uint8_t *lds,
                                            uint32_t *flag) {
@@ -799,7 +799,7 @@ __device__ __forceinline__ void attn_split(const RmiAttnShape &shape, const RmiA
     };
     // Few parts: every thread reads all, and of no more parts than there are, as a load past the caches is 40 ns of a wave (a
     // token of 28 layers at 150 positions, two parts: 560 us with eight parts' loads, 537 with two parts', by lanes 551).  More:
-    // by lanes (2048 positions, f32: 980 us where every thread reads all, 914 by lanes; 700 positions, bf16: 569 and 551).
+    // by lanes (2048 positions, f32: 980 us where every thread reads all, 914 by lanes; 700 positions, bf16: 572 and 553).
     if (parts == 2) return merge(std::integral_constant<uint32_t, 2>());
     if (parts <= 4) return merge(std::integral_constant<uint32_t, 4>());
     if constexpr (TAPS > 0) {
@@ -1349,7 +1349,7 @@ int mixers_step(const RmiAttnShape *as, const RmiAttnArgs *aa, const RmiRecurSha
         return rc;
     };
     // Heads that fill a kernel, behind four taps or without a convolution, and no wider than a wave's pairs of channels; a
-    // token of 28 layers at 16 | 150 | 2048 positions: 560 | 606 | 730 us with the sizes as arguments, 545 | 569 | 670 known.
+    // token of 28 layers at 16 | 150 | 2048 positions: 555 | 585 | 734 us with the sizes as arguments, 538 | 549 | 623 known.
     const bool filled = as && bucket <= 128 && p.s.dim == bucket && p.s.vdim == bucket && p.s.dk_pad == bucket && p.s.dv_pad == bucket &&
                         reinterpret_cast<uintptr_t>(p.a.conv) % 16 == 0;
     auto with = [&](auto taps) { return bucket == 64 ? go(mixers_step_kernel<T, 64, taps.value>) : go(mixers_step_kernel<T, 128, taps.value>); };
