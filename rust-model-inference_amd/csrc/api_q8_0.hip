@@ -217,9 +217,8 @@ static int forward_batched(const rmi_hip_weight *w, const float *input, float *o
     if (!c) return RMI_HIP_E_RUNTIME;
     const size_t n_x = size_t(n_tokens) * n_in;
     const size_t x_bytes = n_x * 4, y_bytes = size_t(n_tokens) * n_out * 4;
-    // The quantizer reads every input once, and the x86-64-order products only write results and never read them back (those of
-    // up to seven tokens are written twice, with the same bits), so both may use the pinned
-    // buffers themselves: a copy command less on either side, each of which is 5 to 8 us between dependent kernels.  From some
+    // The quantizer reads every input once, and the x86-64-order products write every result once and never read it back, so both
+    // may use the pinned buffers themselves: a copy command less on either side, each of which is 5 to 8 us between dependent kernels.  From some
     // 700 KB on the copy is the faster reader.  us with copies | x in place | y in place | both: 2048 x 6144, 1 token 31.5 | 28.5 |
     // 22.4 | 20.4, 13 tokens 60.9 | 54.9 | 53.0 | 45.5, 100 tokens (800 KB) 209.0 | 211.1 | 200.3 | 202.6; 8192 x 3000, 300 tokens
     // (9.6 MB) 616 | 661 | 571 | 612.  Results in place, of 24 to 1000 tokens (50 KB to 48 MB) through 512..8192 x 500..12000: 0.98 to

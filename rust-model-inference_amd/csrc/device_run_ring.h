@@ -91,14 +91,14 @@ struct RmiRunResults {
     }
     __device__ __forceinline__ bool group_full() const { return (tiles_done & 7) == 0; }
     __device__ __forceinline__ bool pending() const { return flushed < tiles_done; }
-    // first_tile: index of the run's first tile in the matrix; rows outside [row_start, row_end) are not stored
+    // first_tile: index of the run's first tile in the matrix; rows outside [row_start, row_end) and tokens before `first` are not stored
     template <typename YPtr>
     __device__ __forceinline__ void flush(YPtr y, uint32_t y_stride, uint32_t first_tile, uint32_t r, uint32_t t8,
-                                          uint32_t row_start, uint32_t row_end) {
+                                          uint32_t row_start, uint32_t row_end, uint32_t first = 0) {
         const uint32_t row = (first_tile + flushed + t8) * 8 + r;
 #pragma unroll
         for (int t = 0; t < B; t++)
-            if (flushed + t8 < tiles_done && row >= row_start && row < row_end) y[size_t(t) * y_stride + row] = res[t];
+            if (uint32_t(t) >= first && flushed + t8 < tiles_done && row >= row_start && row < row_end) y[size_t(t) * y_stride + row] = res[t];
         flushed = tiles_done;
     }
 };

@@ -310,13 +310,15 @@ __device__ __forceinline__ void factors_sum(float &acc, const float4 *src) {
 }
 
 // A launch may spread its tokens over workgroups, gridDim.y groups of B tokens: the problem of the group blockIdx.y, the last one
-// of which begins early enough to have B.
+// of which begins early enough to have B.  Returns how many of its tokens are the group's before it, which stores them (where
+// results go to the host's memory every store is bytes across PCIe).
 template <int B>
-__device__ __forceinline__ void to_token_group(RmiGemvProblem &p) {
+__device__ __forceinline__ uint32_t to_token_group(RmiGemvProblem &p) {
     const uint32_t at = blockIdx.y * B, last = p.n_tokens - B, t0 = blockIdx.y == 0 || at < last ? at : last;
     p.x_q8 += size_t(t0) * p.n_in;
     p.x_scales += size_t(t0) * (p.n_in >> 5);
     p.y += size_t(t0) * p.y_stride;
+    return at - t0;
 }
 
 // A wave owns a short run of consecutive 8-row tiles of ONE matrix (about 34 KiB of
@@ -339,7 +341,7 @@ __global__ __launch_bounds__(MAXT) void gemv_q8_0_kernel(RmiGemvProblem single,
     const uint32_t w_idx = __builtin_amdgcn_readfirstlane(blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6));
 
     RmiGemvProblem p;
-    uint32_t k, k_end;
+    uint32_t k, k_end, first = 0;  // first: the first token whose results are stored
     if (GROUPED) {
         const uint4 run = runs[w_idx];
         p = list[run.x];
@@ -347,7 +349,7 @@ __global__ __launch_bounds__(MAXT) void gemv_q8_0_kernel(RmiGemvProblem single,
         k_end = run.y + run.z;
     } else {
         p = single;
-        to_token_group<B>(p);
+        first = to_token_group<B>(p);
         k = w_idx * tiles_per_wave < p.n_tiles ? w_idx * tiles_per_wave : p.n_tiles;
         k_end = k + tiles_per_wave < p.n_tiles ? k + tiles_per_wave : p.n_tiles;
     }
@@ -410,11 +412,11 @@ __global__ __launch_bounds__(MAXT) void gemv_q8_0_kernel(RmiGemvProblem single,
             }
             o = 0;
             out.keep(y, L);
-            if (out.group_full()) out.flush(yp, p.y_stride, p.tile0 + k, r, L, p.row_start, p.row_end);
+            if (out.group_full()) out.flush(yp, p.y_stride, p.tile0 + k, r, L, p.row_start, p.row_end, first);
         }
     };
     rmi_ring_walk(ring, n_units, cur, consume);
-    if (out.pending()) out.flush(yp, p.y_stride, p.tile0 + k, r, L, p.row_start, p.row_end);
+    if (out.pending()) out.flush(yp, p.y_stride, p.tile0 + k, r, L, p.row_start, p.row_end, first);
 }
 
 // ---- The same GEMV for four to eight tokens with the 4-byte dots on the matrix cores.
@@ -530,7 +532,7 @@ __global__ __launch_bounds__(MAXT, kX4WavesPerSimd) void gemv_q8_0_x4_kernel(Rmi
     const uint32_t w_idx = __builtin_amdgcn_readfirstlane(blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6));
 
     RmiGemvProblem p;
-    uint32_t k, k_end;
+    uint32_t k, k_end, first = 0;  // first: the first token whose results are stored
     if (GROUPED) {
         const uint4 run = runs[w_idx];
         p = list[run.x];
@@ -538,7 +540,7 @@ __global__ __launch_bounds__(MAXT, kX4WavesPerSimd) void gemv_q8_0_x4_kernel(Rmi
         k_end = run.y + run.z;
     } else {
         p = single;
-        to_token_group<B>(p);
+        first = to_token_group<B>(p);
         k = w_idx * tiles_per_wave < p.n_tiles ? w_idx * tiles_per_wave : p.n_tiles;
         k_end = k + tiles_per_wave < p.n_tiles ? k + tiles_per_wave : p.n_tiles;
     }
@@ -597,7 +599,7 @@ __global__ __launch_bounds__(MAXT, kX4WavesPerSimd) void gemv_q8_0_x4_kernel(Rmi
 #pragma unroll
         for (int t = 0; t < B; t++) {
             const float v = park[(t4 * B + t) * 8 + (lane & 7)];
-            if (live) yp[size_t(t) * p.y_stride + row] = v;
+            if (live && uint32_t(t) >= first) yp[size_t(t) * p.y_stride + row] = v;
         }
         flushed = tiles_done;
     };

@@ -179,7 +179,7 @@ struct RmiGemvProblem {
     uint32_t n_tokens;     // of a launch over token groups of B: group g begins at token min(g B, n_tokens - B)
 };
 // n_tokens tokens in one launch, in groups of `group` (<= 8, <= n_tokens) or fewer; where they don't come out even the last group
-// begins earlier, and what two groups share is written twice, with the same bits
+// begins earlier, and what two groups share is written by the first of them
 int rmi_launch_gemv_q8_0_single(const RmiGemvProblem &p, uint32_t group, hipStream_t s, uint32_t n_tokens);
 // how n_tokens (> 0) tokens of a matrix of that many octets and rows are grouped; tokens = 0: not even one's activation fits the staging
 struct RmiTokenGroups {
