@@ -29,11 +29,13 @@
 
 #include "attn_prompt.h"
 #include "device_ahead.h"
+#include "device_attn128.h"
 #include "device_math.h"
 #include "device_quant.h"
 #include "device_sample.h"
 #include "rmi_internal.h"
 #include "session.h"
+#include "walk_qwen3.h"
 
 #include "device_common.h"
 
@@ -442,61 +444,6 @@ __global__ __launch_bounds__(kAttnThreads) void attention_quant_kernel(
 // waves, two per SIMD: with sixteen the kernel took a third longer (the waves of a SIMD run one after another
 // through such dependent code, so more of them only repeat the per-thread set-up), with four it lost on long contexts.
 constexpr uint32_t kA128Threads = 512;
-typedef _Float16 half8 __attribute__((ext_vector_type(8)));
-__device__ __forceinline__ half8 as_half8(const uint4 &v) { return __builtin_bit_cast(half8, v); }
-__device__ __forceinline__ double quad_sum(double v) {  // (l0 + l1) + (l2 + l3) in every lane of the quad
-    int lo = __double2loint(v), hi = __double2hiint(v);
-    v += __hiloint2double(__builtin_amdgcn_mov_dpp(hi, 0xB1, 0xf, 0xf, true), __builtin_amdgcn_mov_dpp(lo, 0xB1, 0xf, 0xf, true));
-    lo = __double2loint(v), hi = __double2hiint(v);
-    v += __hiloint2double(__builtin_amdgcn_mov_dpp(hi, 0x4E, 0xf, 0xf, true), __builtin_amdgcn_mov_dpp(lo, 0x4E, 0xf, 0xf, true));
-    return v;
-}
-template <int XOR>
-__device__ __forceinline__ double swizzle_xor_f64(double v) {  // the value of lane ^ XOR (XOR < 32)
-    constexpr int kPattern = 0x1f | (XOR << 10);
-    return __hiloint2double(__builtin_amdgcn_ds_swizzle(__double2hiint(v), kPattern),
-                            __builtin_amdgcn_ds_swizzle(__double2loint(v), kPattern));
-}
-__device__ __forceinline__ double swizzle_xor16_f64(double v) { return swizzle_xor_f64<16>(v); }
-// Two registers exchange lanes in one vector instruction (v_permlane32_swap: lanes 32..63 of the first with lanes
-// 0..31 of the second; v_permlane16_swap: the odd rows of sixteen of the first with the even rows of the second).
-// a + b afterwards is, in the lower half (the even rows), a summed over both halves (both rows of a pair), and in the
-// upper half (the odd rows) b summed likewise: two values to reduce become one, without the LDS crossbar.
-template <bool ROWS>
-__device__ __forceinline__ double swap_add_f64(double a, double b) {
-    const uint64_t ab = __builtin_bit_cast(uint64_t, a), bb = __builtin_bit_cast(uint64_t, b);
-    uint64_t x, y;
-    if constexpr (ROWS) {
-        const auto lo = __builtin_amdgcn_permlane16_swap(uint32_t(ab), uint32_t(bb), false, false);
-        const auto hi = __builtin_amdgcn_permlane16_swap(uint32_t(ab >> 32), uint32_t(bb >> 32), false, false);
-        x = uint64_t(lo[0]) | (uint64_t(hi[0]) << 32);
-        y = uint64_t(lo[1]) | (uint64_t(hi[1]) << 32);
-    } else {
-        const auto lo = __builtin_amdgcn_permlane32_swap(uint32_t(ab), uint32_t(bb), false, false);
-        const auto hi = __builtin_amdgcn_permlane32_swap(uint32_t(ab >> 32), uint32_t(bb >> 32), false, false);
-        x = uint64_t(lo[0]) | (uint64_t(hi[0]) << 32);
-        y = uint64_t(lo[1]) | (uint64_t(hi[1]) << 32);
-    }
-    return __builtin_bit_cast(double, x) + __builtin_bit_cast(double, y);
-}
-// The eight f64 sums of a lane (dimensions 8 dg .. 8 dg + 7, dg = lane % DG_LANES) added over the wave's 64 / DG_LANES
-// key slices (lanes DG_LANES apart; DG_LANES = 4, 8 or 16).  Halves, then rows, halve the values as they halve the
-// lanes; what is left inside a row of sixteen goes round it by DPP.  Lane l ends with two sums, those of dimensions
-// 8 dg + pv_dim_base(l) and the next one.  (f64 sums of exact terms: the order of the additions is free.)
-__device__ __forceinline__ uint32_t pv_dim_base(uint32_t lane) { return 2 * ((lane >> 4) & 1) + 4 * (lane >> 5); }
-template <int DG_LANES>
-__device__ __forceinline__ void pv_slices_sum(const double (&acc)[8], double (&u)[2]) {
-    static_assert(DG_LANES == 4 || DG_LANES == 8 || DG_LANES == 16, "slices are whole parts of a row of sixteen lanes");
-    double r[4];
-#pragma unroll
-    for (int k = 0; k < 4; k++) r[k] = swap_add_f64<false>(acc[k], acc[k + 4]);
-#pragma unroll
-    for (int k = 0; k < 2; k++) {
-        u[k] = swap_add_f64<true>(r[k], r[k + 2]);
-        if constexpr (DG_LANES <= 8) u[k] += dpp_f64<0x128>(u[k]);  // row_ror:8
-        if constexpr (DG_LANES <= 4) u[k] += dpp_f64<0x124>(u[k]);  // row_ror:4
-    }
-}
 __host__ __device__ inline size_t attn128_lds_bytes(uint32_t n_keys) {
     const size_t n_pad = (size_t(n_keys) + kAttnPad - 1) / kAttnPad * kAttnPad;
     return n_pad * 12 + (kA128Threads / 64) * 128 * 8 + 128;  // 32 floats of room behind the scores
@@ -1260,12 +1207,19 @@ struct rmi_hip_qwen3 : RmiSession {
     RmiAttnLimbs attn_limbs;
     std::vector<bool> limbs_hold;        // by layer: its norms keep queries and keys below what limbs hold
     void *attn_split = nullptr;          // scratch of the split attention launches (head dimension 128)
+    RmiWalkArgs walk{};                  // what its launches have in common, where the shape can be walked (walk.words is set)
+    RmiWalkShape walk_shape{};
+    size_t walk_words = 0;
+    bool walk_off = false;               // a wait of a walk was given up once
 
     ~rmi_hip_qwen3() override;
     int enqueue_step(uint32_t step, hipStream_t st) override;
     const float *step_logits() const override { return logits; }
     bool pass_possible(uint32_t step0, uint32_t n) const override;
     int enqueue_pass(uint32_t step0, uint32_t n, const uint32_t *want, uint32_t n_want, bool sample, hipStream_t st, const RmiLogitsOf &of) override;
+    uint32_t walk_steps(uint32_t step, uint32_t most) const override;
+    int enqueue_walk(uint32_t step, uint32_t n, uint32_t n_prompt, bool keep_logits, hipStream_t st) override;
+    bool walk_gave_up() override;
 };
 
 namespace {
@@ -1489,6 +1443,31 @@ int rmi_hip_qwen3::enqueue_step(uint32_t step, hipStream_t st) { return ::enqueu
 bool rmi_hip_qwen3::pass_possible(uint32_t step0, uint32_t n) const { return prompt_pass_possible(this, step0, n); }
 int rmi_hip_qwen3::enqueue_pass(uint32_t step0, uint32_t n, const uint32_t *want, uint32_t n_want, bool, hipStream_t st, const RmiLogitsOf &of) {
     return enqueue_prompt_pass(this, step0, n, want, n_want, st, of);
+}
+uint32_t rmi_hip_qwen3::walk_steps(uint32_t step, uint32_t most) const {
+    if (!walk.words || walk_off || step == 0 || step + 1 >= kWalkMaxKeys) return 0;
+    const uint32_t fit = kWalkMaxKeys - 1 - step, n = most < fit ? most : fit;
+    return n < kWalkMaxSteps ? n : kWalkMaxSteps;
+}
+int rmi_hip_qwen3::enqueue_walk(uint32_t step, uint32_t n, uint32_t n_prompt, bool keep_logits, hipStream_t st) {
+    const uint32_t tags = rmi_walk_qwen3_tags(n, cfg.n_layer);
+    if (walk.tag0 > 0xffffffffu - tags) {  // the words' tags start anew
+        RMI_HIP_CHECK(hipMemsetAsync(walk.words, 0, walk_words * 8, st));
+        walk.tag0 = 0;
+    }
+    RmiWalkArgs a = walk;
+    a.step0 = step;
+    a.n_steps = n;
+    a.n_prompt = n_prompt;
+    a.keep_logits = keep_logits;
+    walk.tag0 += tags;
+    return rmi_launch_walk_qwen3(walk_shape, a, st);
+}
+bool rmi_hip_qwen3::walk_gave_up() {
+    uint32_t failed = 0;
+    if (!walk.words || walk_off || hipMemcpy(&failed, walk.failed, 4, hipMemcpyDeviceToHost) != hipSuccess) return false;
+    walk_off = failed != 0;
+    return walk_off;
 }
 rmi_hip_qwen3::~rmi_hip_qwen3() {
     if (head && head != embd) rmi_hip_free_weight(head);
@@ -1821,6 +1800,22 @@ rmi_hip_qwen3 *rmi_hip_qwen3_create(const rmi_hip_qwen3_config *cfg, const rmi_h
     }
     if (ok && c.head_dim_k == 128 && c.head_dim_v == 128 && attn128_use_split(c.capacity, c.n_head))
         ok = (s->attn_split = dev_alloc<uint8_t>(s, attn_split_scratch_bytes(c.n_head, c.capacity), true)) != nullptr;
+    s->walk_shape = RmiWalkShape{c.n_embd, c.n_head, c.n_head_kv, c.head_dim_k, c.head_dim_v, c.n_ff, c.vocab, c.n_layer, s->kv_stride};
+    if (ok && rmi_walk_qwen3_fits(s->walk_shape)) {
+        std::vector<RmiWalkLayer> layers;
+        for (uint32_t l = 0; l < c.n_layer; l++)
+            layers.push_back(RmiWalkLayer{s->w_qkv[l]->data, s->w_o[l]->data, s->w_gu[l]->data, s->w_down[l]->data, s->attn_norm[l], s->ffn_norm[l],
+                                          c.has_qk_norm ? s->q_norm[l] : nullptr, c.has_qk_norm ? s->k_norm[l] : nullptr});
+        s->walk_words = rmi_walk_qwen3_words(s->walk_shape);
+        RmiWalkLayer *d_layers = dev_alloc<RmiWalkLayer>(s, c.n_layer);
+        uint64_t *words = dev_alloc<uint64_t>(s, s->walk_words, true);
+        uint32_t *failed = dev_alloc<uint32_t>(s, 1, true);
+        ok = d_layers && words && failed &&
+             hipMemcpy(d_layers, layers.data(), layers.size() * sizeof(RmiWalkLayer), hipMemcpyHostToDevice) == hipSuccess;
+        s->walk = RmiWalkArgs{d_layers, s->embd->data, s->head->data, s->output_norm, s->cos_t, s->sin_t, s->k_cache, s->v_cache, s->x, s->logits,
+                              words, failed, s->tok, s->step_argmax, s->nonfinite, s->step_top2, s->params, c.n_layer, c.n_head, c.n_head_kv,
+                              c.n_ff, c.vocab, c.capacity, s->kv_stride, 0, 0, 0, 0, 0, 0, 0, 0, kWalkSpins, c.eps, c.rounding};
+    }
     if (ok && hipStreamSynchronize(rmi_thread_ctx()->stream) != hipSuccess) {  // the uploads enqueued above
         rmi_set_error("weight upload failed");
         ok = false;
@@ -1843,6 +1838,14 @@ int rmi_hip_qwen3_set_prompt_passes(rmi_hip_qwen3 *s, int enabled) {
     // 0: off; 1: the default size; more: that many positions a pass, up to the buffers' size
     const uint32_t most = prompt_batch(s->cfg.capacity);
     s->prompt_pass = enabled <= 0 ? 0u : enabled == 1 || uint32_t(enabled) > most ? most : uint32_t(enabled);
+    return RMI_HIP_OK;
+}
+
+int rmi_hip_qwen3_set_walks(rmi_hip_qwen3 *s, int enabled) {
+    if (!s) return rmi_fail(RMI_HIP_E_INVALID, "null session");
+    s->walk_off = enabled <= 0;
+    s->walk.spins = enabled > 1 ? uint32_t(enabled) : kWalkSpins;
+    if (enabled > 0 && s->walk.words) RMI_HIP_CHECK(hipMemset(s->walk.failed, 0, 4));
     return RMI_HIP_OK;
 }
 

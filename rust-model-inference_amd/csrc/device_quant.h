@@ -57,3 +57,40 @@ __device__ __forceinline__ uint32_t rmi_quantize_block8(float4 v, int rounding, 
     *scale = float(_Float16(d));
     return uint32_t(i0 & 0xff) | (uint32_t(i1 & 0xff) << 8) | (uint32_t(i2 & 0xff) << 16) | (uint32_t(i3 & 0xff) << 24);
 }
+
+// The same for 32 lanes that hold a block's elements one each (lanes 0..31 and 32..63 of a wave, two blocks): the four quants of
+// a quad of lanes, packed, in each of its lanes; *scale in all 32.  All 64 lanes must be active.
+__device__ __forceinline__ uint32_t rmi_quantize_block32(float v, int rounding, float *scale) {
+    auto max32 = [](float a) {
+        a = max8_lanes(a);
+        a = fmaxf(a, dpp_f32<kDppRowMirror>(a));
+        const auto w = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(a), false, false);
+        return fmaxf(__uint_as_float(w[0]), __uint_as_float(w[1]));
+    };
+    float amax = max32(fabsf(v));
+    int q;
+    float d;
+    if (rounding == RMI_HIP_ROUND_NEON) {
+        if (max32(v != v ? 1.0f : 0.0f) != 0.0f) amax = __builtin_nanf("");
+        d = amax / 127.0f;
+        const float inv = d > 0.0f ? 1.0f / d : 0.0f, t = v * inv;
+        q = t != t ? 0 : int(rintf(fminf(fmaxf(t, -127.0f), 127.0f)));
+    } else {
+        const bool even = rounding == RMI_HIP_ROUND_TIES_EVEN;
+        d = amax == 0.0f ? 0.0f : amax / 127.0f;
+        float r;
+        if (even) {
+            const float id = amax == 0.0f ? 0.0f : 127.0f / amax;
+            r = rintf(v * id);
+        } else {
+            const float inv = d == 0.0f ? 0.0f : 1.0f / d;
+            r = roundf(v * inv);
+        }
+        q = (r != r && !even) ? 0 : int(fminf(fmaxf(r, -128.0f), 127.0f));
+    }
+    *scale = float(_Float16(d));
+    uint32_t p = uint32_t(q & 0xff) << (8 * (threadIdx.x & 3));
+    p |= dpp_u32<kDppQuadXor1>(p);
+    p |= dpp_u32<kDppQuadXor2>(p);
+    return p;
+}

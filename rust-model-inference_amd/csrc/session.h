@@ -57,6 +57,16 @@ struct RmiSession {
     // prompt.
     virtual int enqueue_pass(uint32_t step0, uint32_t n, const uint32_t *want, uint32_t n_want, bool sample, hipStream_t st, const RmiLogitsOf &of) = 0;
     virtual uint32_t max_pass_want() const { return 0xffffffffu; }
+    // How many positions from `step` on, up to `most`, one launch can take one after the other; 0: none.
+    virtual uint32_t walk_steps(uint32_t step, uint32_t most) const { (void)step, (void)most; return 0; }
+    // Such a launch; afterwards the session stands where the last of n single steps would have left it, with the last one's
+    // logits in step_logits() if keep_logits.
+    virtual int enqueue_walk(uint32_t step, uint32_t n, uint32_t n_prompt, bool keep_logits, hipStream_t st) {
+        (void)step, (void)n, (void)n_prompt, (void)keep_logits, (void)st;
+        return RMI_HIP_E_INVALID;
+    }
+    // Whether a walk enqueued before could not finish (asked behind a synchronisation); walk_steps gives 0 from then on.
+    virtual bool walk_gave_up() { return false; }
 };
 
 // rmi_hip_<model>_generate: see rmi_hip_qwen3_generate in the header

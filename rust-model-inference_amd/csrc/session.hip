@@ -45,9 +45,10 @@ int rmi_session_set_stop_ids(RmiSession *s, const uint32_t *ids, uint32_t n_ids)
     return RMI_HIP_OK;
 }
 
-int rmi_session_generate(RmiSession *s, const uint32_t *prompt, uint32_t n_prompt, uint32_t max_new, uint32_t *generated,
-                         uint32_t *step_argmax, float *step_top2, const uint32_t *dump_steps, uint32_t n_dump,
-                         float *dump_logits, double *seconds) {
+static int session_generate_once(RmiSession *s, const uint32_t *prompt, uint32_t n_prompt, uint32_t max_new, uint32_t *generated,
+                                 uint32_t *step_argmax, float *step_top2, const uint32_t *dump_steps, uint32_t n_dump,
+                                 float *dump_logits, double *seconds, bool *again) {
+    *again = false;
     RMI_REQUIRE_INIT();
     if (!s || !prompt || n_prompt == 0 || (max_new && !generated))
         return rmi_fail(RMI_HIP_E_INVALID, "null session, prompt or output");
@@ -112,6 +113,15 @@ int rmi_session_generate(RmiSession *s, const uint32_t *prompt, uint32_t n_promp
                 step += n;
                 continue;
             }
+            if (uint32_t n_walk = s->walk_steps(step, until - step); n_walk > 0) {  // up to the next position whose logits are asked for
+                const auto next = std::lower_bound(dumps.begin(), dumps.end(), step);
+                const bool keep = next != dumps.end() && *next < step + n_walk;
+                if (keep) n_walk = *next + 1 - step;
+                rc = s->enqueue_walk(step, n_walk, n_prompt, keep, st);
+                step += n_walk;
+                if (rc == RMI_HIP_OK && keep) dump(step - 1, s->step_logits());
+                continue;
+            }
             rc = s->enqueue_step(step, st);
             if (rc == RMI_HIP_OK) dump(step, s->step_logits());
             step++;
@@ -135,7 +145,8 @@ int rmi_session_generate(RmiSession *s, const uint32_t *prompt, uint32_t n_promp
     if (e == hipSuccess) e = hipStreamSynchronize(st);
     if (seconds) *seconds = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
     uint32_t nonfinite = 0;
-    if (e == hipSuccess && rc == RMI_HIP_OK) {
+    *again = e == hipSuccess && rc == RMI_HIP_OK && s->walk_gave_up();
+    if (e == hipSuccess && rc == RMI_HIP_OK && !*again) {
         if (n_valid) e = hipMemcpy(generated, s->tok + n_prompt, size_t(n_valid) * 4, hipMemcpyDeviceToHost);
         if (e == hipSuccess && step_argmax) e = hipMemcpy(step_argmax, s->step_argmax, size_t(steps_done) * 4, hipMemcpyDeviceToHost);
         if (e == hipSuccess && step_top2) e = hipMemcpy(step_top2, s->step_top2, size_t(steps_done) * 8, hipMemcpyDeviceToHost);
@@ -147,4 +158,14 @@ int rmi_session_generate(RmiSession *s, const uint32_t *prompt, uint32_t n_promp
     if (e != hipSuccess) return rmi_fail(RMI_HIP_E_RUNTIME, "decode failed: %s", hipGetErrorString(e));
     if (nonfinite) return rmi_fail(RMI_HIP_E_RUNTIME, "non-finite logits in %u steps", nonfinite);
     return int(n_valid);
+}
+
+int rmi_session_generate(RmiSession *s, const uint32_t *prompt, uint32_t n_prompt, uint32_t max_new, uint32_t *generated,
+                         uint32_t *step_argmax, float *step_top2, const uint32_t *dump_steps, uint32_t n_dump,
+                         float *dump_logits, double *seconds) {
+    bool again = false;
+    int rc = session_generate_once(s, prompt, n_prompt, max_new, generated, step_argmax, step_top2, dump_steps, n_dump, dump_logits, seconds, &again);
+    if (again)  // a walk could not finish: the whole sequence once more, by single launches
+        rc = session_generate_once(s, prompt, n_prompt, max_new, generated, step_argmax, step_top2, dump_steps, n_dump, dump_logits, seconds, &again);
+    return rc;
 }

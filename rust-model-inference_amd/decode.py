@@ -109,6 +109,10 @@ class Qwen3Session(_Session):
         if not self._h:
             raise hip.RmiHipError(-1, hip.last_error())
 
+    def set_walks(self, enabled):
+        """Tokens by the launch that walks all layers (rmi_hip_qwen3_set_walks): 1 (default) on, 0 off."""
+        hip.check(hip.lib.rmi_hip_qwen3_set_walks(self._h, int(enabled)))
+
     @classmethod
     def from_gguf(cls, loader, capacity, rounding=hip.ROUND_TIES_EVEN):
         """Qwen3Model::from_source + Qwen3Session::new over an open ``loader.GGUFLoader``: tensor bytes go from

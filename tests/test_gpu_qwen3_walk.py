@@ -1,0 +1,99 @@
+"""Generated tokens of a Qwen3 session by the launch that walks all layers (csrc/walk_qwen3.hip), against the same session by
+single launches and against the CPU loop: tokens, every step's argmax and two largest logits and the asked logits bit for bit,
+where its branches change: heads that share their keys' scores (from 352 keys on), slices of values longer than what is loaded
+ahead (from 769 keys on), the last position it takes (1279 keys), launches of up to 16 tokens."""
+import threading
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+_SAME = ("tokens", "argmax", "top2", "dump")
+
+
+def _model(rmi, tmp_path, name="m", **kw):
+    path = str(tmp_path / (name + ".gguf"))
+    rmi.gguf.write_synthetic_qwen3(path, seed=5, **{"n_layer": 2, "vocab": 3000, **kw})
+    f = rmi.gguf.GGUFFile(path)
+    return f.metadata, {k: t[2] for k, t in f.tensors.items()}
+
+
+def _equal(a, b, what):
+    for k in _SAME:
+        assert np.array_equal(np.asarray(a[k]).view(np.uint32), np.asarray(b[k]).view(np.uint32)), (what, k)
+
+
+@pytest.mark.parametrize("kw,drop,rounding", [
+    ({}, (), "TIES_EVEN"), ({"n_head_kv": 16, "vocab": 2999}, (), "HALF_AWAY"), ({"n_head_kv": 2, "n_layer": 1, "vocab": 70}, (), "NEON"),
+    ({"n_layer": 3}, ("attn_q_norm", "attn_k_norm"), "TIES_EVEN")])
+def test_walk_is_the_single_launches_bit_for_bit(hip, tmp_path, kw, drop, rounding):
+    meta, tensors = _model(hip, tmp_path, **kw)
+    tensors = {n: t for n, t in tensors.items() if not any(d in n for d in drop)}
+    s = hip.decode.Qwen3Session(meta, tensors, 1300, getattr(hip.hip, "ROUND_" + rounding))
+    rng = np.random.default_rng(3)
+    for n, new, passes in ((1, 20, 1), (2, 1, 1), (40, 17, 0), (62, 4, 1), (345, 16, 1), (762, 12, 1), (1262, 30, 1)):
+        prompt = rng.integers(0, s.vocab, n, dtype=np.uint32)
+        dumps = sorted({n - 1, n + new // 2 - 1, n + new - 2})
+        s.set_prompt_passes(passes)
+        s.set_walks(1)
+        walked = s.generate(prompt, new, dumps)
+        again = s.generate(prompt, new, dumps)
+        s.set_walks(0)
+        single = s.generate(prompt, new, dumps)
+        _equal(walked, single, (kw, n, new))
+        _equal(again, single, (kw, n, new, "again"))
+    s.close()
+
+
+@pytest.mark.parametrize("n,new", [(1, 12), (348, 8), (766, 6)])
+def test_walk_is_the_cpu_loop(hip, oracle, tmp_path, n, new):
+    meta, tensors = _model(hip, tmp_path)
+    pool = oracle.Pool(8)
+    prompt = np.random.default_rng(n).integers(0, 3000, n, dtype=np.uint32)
+    dumps = sorted({n - 1, n, n + new - 2})
+    cpu = oracle.Qwen3Decoder(meta, tensors, pool).generate(prompt, new, dump_steps=dumps)
+    s = hip.decode.Qwen3Session(meta, tensors, n + new)
+    _equal(s.generate(prompt, new, dumps), cpu, n)
+    s.close()
+    pool.close()
+
+
+def test_a_wait_that_is_given_up_leaves_the_single_launches(hip, tmp_path):
+    meta, tensors = _model(hip, tmp_path)
+    s = hip.decode.Qwen3Session(meta, tensors, 200)
+    prompt = np.random.default_rng(8).integers(0, 3000, 100, dtype=np.uint32)
+    good = s.generate(prompt, 40, [99, 120, 138])
+    s.set_walks(2)  # no vector crosses the chip that fast
+    _equal(s.generate(prompt, 40, [99, 120, 138]), good, "given up")
+    _equal(s.generate(prompt, 40, [99, 120, 138]), good, "single launches from then on")
+    s.set_walks(1)
+    _equal(s.generate(prompt, 40, [99, 120, 138]), good, "on again")
+    stop = int(good["tokens"][21])
+    first = int(np.flatnonzero(good["tokens"] == stop)[0])
+    s.set_stop_ids([stop])
+    assert np.array_equal(s.generate(prompt, 40)["tokens"], good["tokens"][:first])
+    s.close()
+
+
+def test_two_sessions_walk_on_two_threads(hip, tmp_path):
+    meta, tensors = _model(hip, tmp_path)
+    prompts = [np.random.default_rng(k).integers(0, 3000, 30 + 200 * k, dtype=np.uint32) for k in range(2)]
+    sessions = [hip.decode.Qwen3Session(meta, tensors, 300) for _ in range(2)]
+    alone = [s.generate(p, 40, [len(p) + 38]) for s, p in zip(sessions, prompts)]
+    got = [[], []]
+
+    def run(k):
+        for _ in range(6):
+            got[k].append(sessions[k].generate(prompts[k], 40, [len(prompts[k]) + 38]))
+
+    threads = [threading.Thread(target=run, args=(k,)) for k in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    for k in range(2):
+        assert len(got[k]) == 6
+        for g in got[k]:
+            _equal(g, alone[k], k)
+        sessions[k].close()
