@@ -109,30 +109,31 @@ __device__ __forceinline__ uint32_t bytes_to_f16_pair(uint32_t w) {
 // DUMP (parity only): instead of folding them, the kernel writes the integers of every super-block as they leave
 // the matrix cores, sumi = 8 * D_hi + D_lo and prod (the min term's f16 MFMA result, an integer below 2^24), to
 // reinterpret_cast<int32_t *>(y)[((t * n_out + n) * n_sb + sb) * 2 + {0, 1}].
-// KS > 1: KS groups of four waves share the tile; group ks takes the super-blocks ks, ks + KS, ... (n_in / 256 must
+// KS > 1: KS groups of NW waves (32 NW rows) share the tile; group ks takes the super-blocks ks, ks + KS, ... (n_in / 256 must
 // be a multiple of KS), stages them in LDS of its own and keeps its own f32 chains; at the end the groups' results
-// are added in group order.  For launches with no more tiles than the chip has compute units (a long row, a few
-// hundred tokens): eight waves a compute unit instead of four, and half as many super-blocks in sequence.
-template <int TTW, int WAVES_PER_SIMD, bool DUMP, int KS = 1>
-__global__ __launch_bounds__(256 * KS, WAVES_PER_SIMD) void gemm_q4_k_kernel(const uint8_t *__restrict__ w, const float *__restrict__ q8d,
+// are added in group order.  For launches with no more tiles than the chip has compute units, where a wave's chain of
+// super-blocks, 1.0 us each with one token tile and 1.4 with two, is what a launch takes: fewer of them in sequence.
+template <int TTW, int WAVES_PER_SIMD, bool DUMP, int KS = 1, int NW = 4>
+__global__ __launch_bounds__(64 * NW * KS, WAVES_PER_SIMD) void gemm_q4_k_kernel(const uint8_t *__restrict__ w, const float *__restrict__ q8d,
                                                                          const int8_t *__restrict__ q8qs,
                                                                          const int16_t *__restrict__ q8bs, float *__restrict__ y,
                                                                          uint32_t n_out, uint32_t n_sb, uint32_t n_tiles,
                                                                          uint32_t n_tokens, uint32_t y_stride, uint32_t grid_n,
                                                                          uint32_t grid_t, uint32_t t_fastest, uint32_t xcd_split) {
-    constexpr int kTileN = 128, kTileT = 32 * TTW;
-    constexpr int kXPieces = kTileT * 16 / 256;  // 16-byte pieces of the token tile per thread and super-block
+    constexpr int kTileN = 32 * NW, kTileT = 32 * TTW, kThreads = 64 * NW;  // threads of a group
+    constexpr int kXPieces = kTileT * 16 / kThreads;  // 16-byte pieces of the token tile per thread and super-block
+    constexpr int kBs = 256 / kThreads;               // pairs of bsums of 32 tokens per thread
     constexpr int kXBuf = kTileT * kXRow, kBBuf = kTileT * kBRow, kWBuf = kTileN * kWRow;
     static_assert(kXPieces <= 4, "the token pieces move to LDS in the first four calls of a super-block");
     __shared__ __attribute__((aligned(16))) uint8_t sm_w_all[KS * 2 * kWBuf];
     __shared__ __attribute__((aligned(16))) uint8_t sm_x_all[KS * 2 * kXBuf];
     __shared__ __attribute__((aligned(16))) uint8_t sm_b_all[KS * 2 * kBBuf];
-    static_assert(KS == 1 || (KS - 1) * kTileT * 4 <= KS * 2 * kWRow, "the groups' results meet in the weight buffers");
+    static_assert(KS == 1 || (KS - 1) * kTileN * kTileT * 4 <= KS * 2 * kWBuf, "the groups' results meet in the weight buffers");
 
     // ks: this wave's group; tid, wave: position inside the group (the whole workgroup for KS = 1)
-    const uint32_t ks = KS == 1 ? 0u : uint32_t(__builtin_amdgcn_readfirstlane(int(threadIdx.x >> 8)));
+    const uint32_t ks = KS == 1 ? 0u : uint32_t(__builtin_amdgcn_readfirstlane(int(threadIdx.x / kThreads)));
     uint8_t *const sm_w = sm_w_all + ks * 2 * kWBuf, *const sm_x = sm_x_all + ks * 2 * kXBuf, *const sm_b = sm_b_all + ks * 2 * kBBuf;
-    const uint32_t tid = threadIdx.x & 255, lane = tid & 63, wave = uint32_t(__builtin_amdgcn_readfirstlane(int(tid >> 6)));
+    const uint32_t tid = threadIdx.x & (kThreads - 1), lane = tid & 63, wave = uint32_t(__builtin_amdgcn_readfirstlane(int(tid >> 6)));
     const uint32_t c = lane & 31, h = lane >> 5;
     const uint32_t n_off = wave * 32;
     uint32_t n_tile, t_tile;  // one XCD's workgroups take neighbouring tiles
@@ -155,12 +156,12 @@ __global__ __launch_bounds__(256 * KS, WAVES_PER_SIMD) void gemm_q4_k_kernel(con
         if (tile >= n_tiles) tile = n_tiles - 1;
         hd_off = (tile - tile_first) * n_sb * kQ4KSuperBytes + (row & 7) * 16;
     }
-    // Weight nibbles: wave w copies the tiles w, w + 4, w + 8, w + 12 of the workgroup's 16, one 16-byte piece a
+    // Weight nibbles: wave w copies the tiles w, w + NW, w + 2 NW, w + 3 NW of the workgroup's 4 NW, one 16-byte piece a
     // lane (1 KB per instruction, as it lies in the stream); piece lane % 8 of row lane / 8 of the tile.
     uint32_t w_tile_off[4];  // wave-uniform
 #pragma unroll
     for (int i = 0; i < 4; i++) {
-        uint32_t tile = (n0 >> 3) + wave + 4 * i;
+        uint32_t tile = (n0 >> 3) + wave + NW * i;
         if (tile >= n_tiles) tile = n_tiles - 1;
         w_tile_off[i] = (tile - tile_first) * n_sb * kQ4KSuperBytes + 128;
     }
@@ -168,24 +169,28 @@ __global__ __launch_bounds__(256 * KS, WAVES_PER_SIMD) void gemm_q4_k_kernel(con
     const uint32_t w_dst = (8 * wave + (lane >> 3)) * kWRow + (lane & 7) * 16;
     const uint32_t last_tok = n_tokens - 1 - t0;
     const int8_t *x_base = q8qs + size_t(t0) * n_in;
-    // Token quants: load i of a thread is piece tid % 16 of token tid / 16 + 16 i (16 lanes cover a token's 256
+    // Token quants: load i of a thread is piece tid % 16 of token tid / 16 + 4 NW i (16 lanes cover a token's 256
     // bytes).  Piece 2j + hq is half hq of sub-block j = 2g + e; its dword T belongs to call 2T + e, lane half hq,
     // dword g.
     uint32_t x_off, x_lim, x_dst;
     {
         const uint32_t piece = tid & 15, j = piece >> 1, hq = piece & 1, g = j >> 1, e = j & 1;
-        x_off = (tid >> 4) * n_in + piece * 16;  // + 16 i tokens, clamped to the last token's piece
+        x_off = (tid >> 4) * n_in + piece * 16;  // + 4 NW i tokens, clamped to the last token's piece
         x_lim = last_tok * n_in + piece * 16;
         x_dst = (tid >> 4) * kXRow + e * 32 + hq * 16 + g * 4;
     }
-    // bsums: thread (token tid / 8, pair tid % 8) of each 32-token group
+    // bsums: thread (token tid / 8, pair tid % 8) of each 8 NW tokens
     const uint8_t *bs_base = reinterpret_cast<const uint8_t *>(q8bs + size_t(t0) * n_sb * 16);
     const uint8_t *d_base = reinterpret_cast<const uint8_t *>(q8d + size_t(t0) * n_sb);
-    uint32_t bs_off[TTW], d_off[TTW];
+    uint32_t bs_off[TTW * kBs], d_off[TTW];
+#pragma unroll
+    for (int i = 0; i < TTW * kBs; i++) {
+        const uint32_t tokb = i * (kThreads / 8) + (tid >> 3);
+        bs_off[i] = (tokb < last_tok ? tokb : last_tok) * n_sb * 32 + (tid & 7) * 4;
+    }
 #pragma unroll
     for (int tt = 0; tt < TTW; tt++) {
-        const uint32_t tokb = tt * 32 + (tid >> 3), tokd = tt * 32 + c;
-        bs_off[tt] = (tokb < last_tok ? tokb : last_tok) * n_sb * 32 + (tid & 7) * 4;
+        const uint32_t tokd = tt * 32 + c;
         d_off[tt] = (tokd < last_tok ? tokd : last_tok) * n_sb * 4;
     }
     const uint32_t b_dst = (tid >> 3) * kBRow + (tid & 7) * 2;
@@ -195,7 +200,7 @@ __global__ __launch_bounds__(256 * KS, WAVES_PER_SIMD) void gemm_q4_k_kernel(con
     u32x4 raw[2];         // piece T of this lane's row half, out of LDS: dword g = nibbles of sub-blocks 2g, 2g+1
     u32x4 hdr_n;          // the next super-block's header of this lane's row: d, dmin, 12 bytes of scales and mins
     u32x4 xst[kXPieces];  // token pieces on their way to LDS
-    uint32_t bst[TTW];    // two bsums on their way to LDS
+    uint32_t bst[TTW * kBs];  // two bsums each on their way to LDS
     float xd[TTW], xd_n[TTW];
     // current super-block: s_hi (low half) and s_lo (high half) of its eight sub-blocks; the eight mins as f16;
     // d of this lane's row in lanes 0..31 and -dmin in lanes 32..63 (the scale MFMA's operand)
@@ -207,7 +212,7 @@ __global__ __launch_bounds__(256 * KS, WAVES_PER_SIMD) void gemm_q4_k_kernel(con
         wst[i] = *(gptr_u4)(sbase(w_base + size_t(realsb(sb)) * kQ4KSuperBytes + w_tile_off[i]) + voff(w_ld));
     };
     auto store_w = [&](int i, int buf) __attribute__((always_inline)) {
-        *reinterpret_cast<u32x4 *>(sm_w + buf * kWBuf + w_dst + i * 32 * kWRow) = wst[i];
+        *reinterpret_cast<u32x4 *>(sm_w + buf * kWBuf + w_dst + i * 8 * NW * kWRow) = wst[i];
     };
     auto load_hdr = [&](uint32_t sb) __attribute__((always_inline)) {
         hdr_n = *(gptr_u4)(sbase(w_base + size_t(realsb(sb)) * kQ4KSuperBytes) + voff(hd_off));
@@ -228,12 +233,12 @@ __global__ __launch_bounds__(256 * KS, WAVES_PER_SIMD) void gemm_q4_k_kernel(con
         for (int tt = 0; tt < TTW; tt++) xd[tt] = xd_n[tt];
     };
     auto load_x = [&](int i, uint32_t sb) __attribute__((always_inline)) {
-        uint32_t off = x_off + uint32_t(i) * 16 * n_in;
+        uint32_t off = x_off + uint32_t(i) * (kThreads / 16) * n_in;
         off = off < x_lim ? off : x_lim;
         xst[i] = *(gptr_u4)(sbase(x_base + size_t(realsb(sb)) * 256) + voff(off));
     };
     auto store_x = [&](int i, int buf) __attribute__((always_inline)) {
-        uint8_t *dst = sm_x + buf * kXBuf + x_dst + i * 16 * kXRow;
+        uint8_t *dst = sm_x + buf * kXBuf + x_dst + i * (kThreads / 16) * kXRow;
         *reinterpret_cast<uint32_t *>(dst) = xst[i].x;
         *reinterpret_cast<uint32_t *>(dst + 64) = xst[i].y;
         *reinterpret_cast<uint32_t *>(dst + 128) = xst[i].z;
@@ -241,13 +246,13 @@ __global__ __launch_bounds__(256 * KS, WAVES_PER_SIMD) void gemm_q4_k_kernel(con
     };
     auto load_bs = [&](uint32_t sb) __attribute__((always_inline)) {
 #pragma unroll
-        for (int tt = 0; tt < TTW; tt++) bst[tt] = *(gptr_u32)(sbase(bs_base + size_t(realsb(sb)) * 32) + voff(bs_off[tt]));
+        for (int i = 0; i < TTW * kBs; i++) bst[i] = *(gptr_u32)(sbase(bs_base + size_t(realsb(sb)) * 32) + voff(bs_off[i]));
     };
     auto store_bs = [&](int buf) __attribute__((always_inline)) {
 #pragma unroll
-        for (int tt = 0; tt < TTW; tt++) {  // pair sum of bsums: even part and lowest bit, both exact as f16
-            const int s = int(int16_t(bst[tt] & 0xffffu)) + int(int16_t(bst[tt] >> 16));
-            uint8_t *dst = sm_b + buf * kBBuf + tt * 32 * kBRow + b_dst;
+        for (int i = 0; i < TTW * kBs; i++) {  // pair sum of bsums: even part and lowest bit, both exact as f16
+            const int s = int(int16_t(bst[i] & 0xffffu)) + int(int16_t(bst[i] >> 16));
+            uint8_t *dst = sm_b + buf * kBBuf + i * (kThreads / 8) * kBRow + b_dst;
             *reinterpret_cast<_Float16 *>(dst) = _Float16(float(s & ~1));
             *reinterpret_cast<_Float16 *>(dst + 16) = _Float16(float(s & 1));
         }
@@ -414,7 +419,7 @@ __global__ __launch_bounds__(256 * KS, WAVES_PER_SIMD) void gemm_q4_k_kernel(con
 #pragma unroll
             for (int tt = 0; tt < TTW; tt++)
 #pragma unroll
-                for (int i = 0; i < 16; i++) comb[((((ks - 1) * 4 + wave) * TTW + tt) * 16 + i) * 64 + lane] = acc[tt][i];
+                for (int i = 0; i < 16; i++) comb[((((ks - 1) * NW + wave) * TTW + tt) * 16 + i) * 64 + lane] = acc[tt][i];
         }
         __syncthreads();
         if (ks != 0) return;
@@ -424,7 +429,7 @@ __global__ __launch_bounds__(256 * KS, WAVES_PER_SIMD) void gemm_q4_k_kernel(con
             for (int tt = 0; tt < TTW; tt++)
 #pragma unroll
                 for (int i = 0; i < 16; i++) {
-                    acc[tt][i] += comb[((((g - 1) * 4 + wave) * TTW + tt) * 16 + i) * 64 + lane];
+                    acc[tt][i] += comb[((((g - 1) * NW + wave) * TTW + tt) * 16 + i) * 64 + lane];
                     acc_m[tt][i] = 0.0f;
                 }
     }
@@ -441,67 +446,74 @@ __global__ __launch_bounds__(256 * KS, WAVES_PER_SIMD) void gemm_q4_k_kernel(con
     }
 }
 
-template <int TTW, int WAVES_PER_SIMD, bool DUMP = false, int KS = 1>
+template <bool DUMP, int TTW, int KS, int NW>
 void launch(const rmi_hip_weight *w, const float *d, const int8_t *qs, const int16_t *bs, float *y, uint32_t n_tokens,
             uint32_t y_stride, hipStream_t s) {
-    const uint32_t grid_n = (w->n_out + 127) / 128, grid_t = (n_tokens + 32 * TTW - 1) / (32 * TTW);
+    const uint32_t grid_n = (w->n_out + 32 * NW - 1) / (32 * NW), grid_t = (n_tokens + 32 * TTW - 1) / (32 * TTW);
     const uint32_t xcd_split = rmi_gemm_xcd_split(grid_n, grid_t, double(w->n_out) * w->n_units * 144.0, double(n_tokens) * w->n_units * 292.0);
-    hipLaunchKernelGGL((gemm_q4_k_kernel<TTW, WAVES_PER_SIMD, DUMP, KS>), dim3(grid_n * grid_t), dim3(256 * KS), 0, s, w->data, d, qs, bs, y,
+    hipLaunchKernelGGL((gemm_q4_k_kernel<TTW, 2, DUMP, KS, NW>), dim3(grid_n * grid_t), dim3(64 * NW * KS), 0, s, w->data, d, qs, bs, y,
                        w->n_out, w->n_units, w->n_tiles, n_tokens, y_stride, grid_n, grid_t, n_tokens < w->n_out ? 1u : 0u, xcd_split);
+}
+
+// Token tile width (in units of 32), groups of waves and waves of a group.  RMI_Q4K_GEMM_TTW and RMI_Q4K_GEMM_GROUPS force the first
+// two where the row allows it (the parity tests run them all).  As long as a plan's tiles are no more than compute units, a launch
+// takes a wave's chain, so the row goes over as many groups as the LDS holds; beyond, rounds of workgroups, and then wide tiles
+// without groups.  us a launch, {32 tokens, 1 group} | {32, 2} | {64, 1} | {64, 2} | {32, 4 of two waves}:
+//   6144 x 2048, 64 tokens 24.4 | 19.3 | 32.1 | 27.0 | 13.6; 512: 25.4 | 22.3 | 32.8 | 28.4 | 27.9; 700: 36.1 | 40.1 | 33.2 | 30.0 | -;
+//   1000: 41.4 | 41.9 | 36.3 | 34.6 | 55.2; 1600: 76.6 | 83.7 | 59.1 | 66.4 | -; 12288 x 4096, 64 tokens 46.0 | 34.3 | 60.5 | 50.5 | 23.2;
+//   2048 x 6144, 256 tokens 15.2 | 17.9 | 14.4 | 13.6 | 22.1; 2048 x 2048, 1000 tokens 16.7 | 18.8 | 15.8 | 15.9 | 29.3;
+//   1024 x 6144, 64 tokens 6.9 | 6.8 | 8.6 | 8.9 | 6.2; 256: 9.7 | 12.5 | 9.3 | 9.7 | 16.4.
+// (Two groups of 64 tokens want eight super-blocks a group: with four they win at three quarters of the compute units and lose at all.)
+struct Q4kPlan {
+    int ttw, groups, waves;
+};
+Q4kPlan gemm_q4_k_plan(const rmi_hip_weight *w, uint32_t n_tokens) {
+    const uint64_t cus = uint64_t(rmi_device_cus());
+    auto tiles = [&](uint32_t rows, uint32_t tokens) { return uint64_t((w->n_out + rows - 1) / rows) * ((n_tokens + tokens - 1) / tokens); };
+    const char *et = getenv("RMI_Q4K_GEMM_TTW"), *eg = getenv("RMI_Q4K_GEMM_GROUPS");
+    const int ttw = et ? atoi(et) : 0, groups = eg ? atoi(eg) : 0;
+    const bool even = w->n_units % 2 == 0, quads = w->n_units % 4 == 0;
+    if (ttw != 1 && ttw != 2 && groups == 0) {
+        if (quads && tiles(64, 32) <= cus) return {1, 4, 2};
+        if (even && tiles(128, 32) <= cus) return {1, 2, 4};
+        if (even && w->n_units >= 16 && tiles(128, 32) > cus && tiles(128, 64) <= cus) return {2, 2, 4};
+        return {tiles(128, 32) <= cus ? 1 : 2, 1, 4};
+    }
+    if (groups == 4 && quads) return {1, 4, 2};
+    if (groups == 2 && even) return {ttw == 2 ? 2 : 1, 2, 4};
+    return {ttw == 1 || (ttw != 2 && tiles(128, 32) <= cus) ? 1 : 2, 1, 4};
+}
+
+template <bool DUMP>
+int run(const rmi_hip_weight *w, const float *d, const int8_t *qs, const int16_t *bsums, float *y, uint32_t n_tokens, uint32_t y_stride, hipStream_t s) {
+    if (n_tokens == 0 || w->n_out == 0 || w->n_units == 0) return RMI_HIP_OK;
+    const Q4kPlan p = gemm_q4_k_plan(w, n_tokens);
+    if (uint64_t((w->n_out + 63) / 64) * ((n_tokens + 31) / 32) > 0x7fffffffull)
+        return rmi_fail(RMI_HIP_E_INVALID, "GEMM too large for one launch");
+    if (p.groups == 4)
+        launch<DUMP, 1, 4, 2>(w, d, qs, bsums, y, n_tokens, y_stride, s);
+    else if (p.groups == 2 && p.ttw == 2)
+        launch<DUMP, 2, 2, 4>(w, d, qs, bsums, y, n_tokens, y_stride, s);
+    else if (p.groups == 2)
+        launch<DUMP, 1, 2, 4>(w, d, qs, bsums, y, n_tokens, y_stride, s);
+    else if (p.ttw == 2)
+        launch<DUMP, 2, 1, 4>(w, d, qs, bsums, y, n_tokens, y_stride, s);
+    else
+        launch<DUMP, 1, 1, 4>(w, d, qs, bsums, y, n_tokens, y_stride, s);
+    RMI_HIP_CHECK(hipGetLastError());
+    return RMI_HIP_OK;
 }
 
 }  // namespace
 
-// Two groups of waves per tile, on the even and the odd super-blocks: where the 32-token tiles are no more than the
-// chip has compute units and each group still has eight super-blocks or more (measured at 2048 x 6144, 512 tokens:
-// 29.5 -> 24.3 us).  RMI_Q4K_GEMM_GROUPS = 1 or 2 forces a count where the row allows it.
-static int gemm_q4_k_groups(const rmi_hip_weight *w, uint32_t n_tokens) {
-    const uint64_t groups32 = uint64_t((w->n_out + 127) / 128) * ((n_tokens + 31) / 32);
-    const char *e = getenv("RMI_Q4K_GEMM_GROUPS");
-    const int force = e ? atoi(e) : 0;
-    if (w->n_units % 2 != 0 || force == 1) return 1;
-    if (force == 2) return 2;
-    return groups32 <= uint64_t(rmi_device_cus()) && w->n_units >= 16 ? 2 : 1;
-}
-
-// token tile width (in units of 32) the launcher takes for this problem; RMI_Q4K_GEMM_TTW = 1 or 2 forces one
-static int gemm_q4_k_ttw(const rmi_hip_weight *w, uint32_t n_tokens) {
-    const uint64_t groups64 = uint64_t((w->n_out + 127) / 128) * ((n_tokens + 63) / 64);
-    const char *e = getenv("RMI_Q4K_GEMM_TTW");
-    const int force = e ? atoi(e) : 0;
-    return force == 2 || (force != 1 && groups64 >= 2 * uint64_t(rmi_device_cus())) ? 2 : 1;
-}
-
-// The same kernel, same tile width as the product would take, writing its per-super-block integers instead of y:
+// The same kernel, same plan as the product would take, writing its per-super-block integers instead of y:
 // ints[n_tokens][n_out][n_sb][2] = {sumi, prod} (parity entry point).
 int rmi_launch_gemm_q4_k_block_ints(const rmi_hip_weight *w, const float *d, const int8_t *qs, const int16_t *bsums,
                                     int32_t *ints, uint32_t n_tokens, hipStream_t s) {
-    if (n_tokens == 0 || w->n_out == 0 || w->n_units == 0) return RMI_HIP_OK;
-    if (uint64_t((w->n_out + 127) / 128) * ((n_tokens + 31) / 32) > 0x7fffffffull)
-        return rmi_fail(RMI_HIP_E_INVALID, "GEMM too large for one launch");
-    if (gemm_q4_k_groups(w, n_tokens) == 2)
-        launch<1, 2, true, 2>(w, d, qs, bsums, reinterpret_cast<float *>(ints), n_tokens, w->n_out, s);
-    else if (gemm_q4_k_ttw(w, n_tokens) == 2)
-        launch<2, 2, true>(w, d, qs, bsums, reinterpret_cast<float *>(ints), n_tokens, w->n_out, s);
-    else
-        launch<1, 2, true>(w, d, qs, bsums, reinterpret_cast<float *>(ints), n_tokens, w->n_out, s);
-    RMI_HIP_CHECK(hipGetLastError());
-    return RMI_HIP_OK;
+    return run<true>(w, d, qs, bsums, reinterpret_cast<float *>(ints), n_tokens, w->n_out, s);
 }
 
 int rmi_launch_gemm_q4_k(const rmi_hip_weight *w, const float *d, const int8_t *qs, const int16_t *bsums, float *y,
                          uint32_t n_tokens, uint32_t y_stride, hipStream_t s) {
-    if (n_tokens == 0 || w->n_out == 0 || w->n_units == 0) return RMI_HIP_OK;
-    const uint64_t groups32 = uint64_t((w->n_out + 127) / 128) * ((n_tokens + 31) / 32);
-    if (groups32 > 0x7fffffffull) return rmi_fail(RMI_HIP_E_INVALID, "GEMM too large for one launch");
-    // 64-token tiles halve the vector work per output but want two workgroups on every compute unit;
-    // RMI_Q4K_GEMM_TTW = 1 or 2 forces a width (the parity tests run both)
-    if (gemm_q4_k_groups(w, n_tokens) == 2)
-        launch<1, 2, false, 2>(w, d, qs, bsums, y, n_tokens, y_stride, s);
-    else if (gemm_q4_k_ttw(w, n_tokens) == 2)
-        launch<2, 2>(w, d, qs, bsums, y, n_tokens, y_stride, s);
-    else
-        launch<1, 2>(w, d, qs, bsums, y, n_tokens, y_stride, s);
-    RMI_HIP_CHECK(hipGetLastError());
-    return RMI_HIP_OK;
+    return run<false>(w, d, qs, bsums, y, n_tokens, y_stride, s);
 }
