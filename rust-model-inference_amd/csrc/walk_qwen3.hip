@@ -18,10 +18,14 @@
 // Every wait is bounded: a wave that has asked `spins` times marks the launch as failed, which ends the others' waits too, and the
 // session generates again by single launches.  All workgroups run at once, since the launch is a cooperative one.
 //
-// us a token, 28 layers and a vocabulary of 151936, by launches | walked: behind 100 keys 590 | 460, 700: 761 | 540, 1250: 932 | 714.
-// A layer at 544 keys is 18 us: six exchanges of 0.9 to 1.4 (a word alone takes 0.4 to one's own XCD, 0.6 to another, and the
-// last of 64 to 128 workgroups counts), the norms in front of two products 0.75 each, the products 0.5, 0.8, 1.1 and 1.1,
-// attention 4.7 of which the f32 sum in key order is 1.8.
+// us a token, 28 layers and a vocabulary of 151936, by launches | walked: behind 100 keys 590 | 425, 700: 761 | 520, 1250: 932 | 685.
+// What a layer takes: six exchanges of 0.9 to 1.4 us (a word alone takes 0.4 to one's own XCD, 0.6 to another, and the last of
+// 64 to 128 workgroups counts), the norms in front of two products 0.75 each, the products, and attention, of which the f32 sum
+// in key order is 1.8 at 544 keys.
+//
+// A workgroup's words go out before any of its waves asks for the next weights (the barriers in front of those loads): stores
+// of a late wave queue behind the other waves' loads, and everybody waits for that wave's words.  Without the barriers, and with
+// arrays in LDS that 16-byte reads found unaligned, the three were 460, 540 and 714.
 //
 // Roles.  attention: four workgroups a head, as in attention128_quant_kernel<true, 4>.  residual: the o and down products, two
 // tiles of eight rows a workgroup and four waves a tile, the rows' residual stream in registers.  norm: rms_norm, quantizer and
@@ -37,11 +41,11 @@
 #include "device_quant.h"
 #include "device_run_ring.h"
 #include "device_sample.h"
+#include "device_walk.h"
 
 namespace {
 
 constexpr uint32_t kWalkThreads = 512;
-typedef uint64_t __attribute__((address_space(1))) *gptr_word;
 
 // where the vectors of the exchange lie, in words.  Quantized ones by blocks of 32 values: eight words of four quants, the scale.
 struct WalkWords {
@@ -67,49 +71,17 @@ __host__ __device__ inline WalkWords walk_words(uint32_t n_embd, uint32_t n_head
     return w;
 }
 
-__device__ __forceinline__ void word_store(gptr_word at, uint32_t v, uint32_t tag) {
-    __hip_atomic_store(at, uint64_t(v) | (uint64_t(tag) << 32), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
 // A quantized block of 32, held as rmi_quantize_block32 leaves it in a wave's two halves: a copy from each.
 __device__ __forceinline__ void block_store(gptr_word at, uint32_t copy, uint32_t q, float scale, uint32_t tag) {
     const uint32_t lane = threadIdx.x & 63, e = lane & 31;
     if ((e & 3) == 0 || e == 1) word_store(at + (lane >> 5) * copy + (e == 1 ? 8 : e >> 2), e == 1 ? __float_as_uint(scale) : q, tag);
 }
-// Which half of the chip this is (XCDs 0..3 and 4..7 sit on one base die each).  Every word is stored twice, and a workgroup
-// reads the copy of its half: lines that are asked for on one die only.  (64 workgroups to 128 and back, 1024 words each way,
-// us an exchange with 1 | 2 | 4 | 8 copies: 1.27 | 0.93 | 1.28 | 1.17; two copies by odd and even XCDs 1.26.)
-__device__ __forceinline__ uint32_t die_half() {
-    constexpr int kXccId = 20;  // HW_REG_XCC_ID
-    return (uint32_t(__builtin_amdgcn_s_getreg((3 << 11) | kXccId)) >> 2) & 1;
-}
-// The N words at[i] of every lane, once all lanes' have the tag.  false: the wait was given up.
-template <int N>
-__device__ __forceinline__ bool words_wait(const gptr_word (&at)[N], uint32_t tag, uint32_t (&v)[N], const RmiWalkArgs &a) {
-    for (uint32_t spin = 0;; spin++) {
-        uint64_t w[N];
-#pragma unroll
-        for (int i = 0; i < N; i++) w[i] = __hip_atomic_load(at[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        bool here = true;
-#pragma unroll
-        for (int i = 0; i < N; i++) {
-            v[i] = uint32_t(w[i]);
-            here = here && uint32_t(w[i] >> 32) == tag;
-        }
-        if (__all(here)) return true;
-        if (spin >= a.spins) {
-            __hip_atomic_store(a.failed, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            return false;
-        }
-        if ((spin & 255) == 255 && __hip_atomic_load(a.failed, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0) return false;
-    }
-}
-
 struct WalkLds {  // of every role
     double red[8];
     float gu[64];
     Top top[64];
     uint32_t bad, token;
-    uint16_t new16[3][128];
+    alignas(16) uint16_t new16[3][128];  // (read by pieces of 16 bytes)
     uint64_t exp_tab[32];
     float max8[8];
 };
@@ -135,7 +107,7 @@ __device__ __forceinline__ bool stage_norm(gptr_word words, uint32_t tag, const 
     uint32_t v[W];
 #pragma unroll
     for (int j = 0; j < W; j++) at[j] = words + j * kWalkThreads + tid;
-    if (!words_wait<W>(at, tag, v, a)) sm.bad = 1;
+    if (!words_wait<W>(at, tag, v, WalkBound{a.failed, a.spins})) sm.bad = 1;
     double part = 0.0;
 #pragma unroll
     for (int j = 0; j < W; j++) {
@@ -179,7 +151,7 @@ __device__ __forceinline__ bool stage_quants(gptr_word words, uint32_t tag, uint
         const uint32_t w = j * kWalkThreads + tid;
         at[j] = words + (w < n ? w : n - 1);
     }
-    if (!words_wait<MAXW>(at, tag, v, a)) sm.bad = 1;
+    if (!words_wait<MAXW>(at, tag, v, WalkBound{a.failed, a.spins})) sm.bad = 1;
     uint32_t *dq = reinterpret_cast<uint32_t *>(lds);
 #pragma unroll
     for (int j = 0; j < MAXW; j++) {
@@ -307,7 +279,7 @@ __device__ bool walk_attention(const RmiWalkArgs &a, const WalkWords &at, gptr_w
     float *scores = reinterpret_cast<float *>(part + (T / 64) * 32);    // [kWalkMaxKeys + 32]
     const uint32_t row_u4 = a.kv_stride >> 3;
     const size_t layer_base = size_t(l) * a.capacity * a.kv_stride;
-    const RmiWalkLayer &w = a.layers[l];
+    const RmiWalkLayer w = table_entry(a.layers + l);
     // the cached keys whose scores this workgroup makes: [k_first, k_end)
     const bool share = n_keys >= kWalkShareKeys;
     const uint32_t quarter = (n_keys + 3) / 4, k_first = share ? pv_part * quarter : 0;
@@ -353,12 +325,16 @@ __device__ bool walk_attention(const RmiWalkArgs &a, const WalkWords &at, gptr_w
     uint4 kraw[2];  // the round behind the converted ones
     kraw[0] = key_at(key0 + kPreK * kRound)[0];
     kraw[1] = key_at(key0 + kPreK * kRound)[8];
+    // keys and values have arrived before anything is stored: a later wait for them would be one for the stores, too
+    for (const uint4 &r : kraw) asm volatile("" ::"v"(r.x));
+#pragma unroll
+    for (uint32_t j = 0; j < kPre; j++) asm volatile("" ::"v"(vp[j].x));
     if (tid < 192) {  // wave 0: q of this head, wave 1: the new k, wave 2: the new v; lane i owns (i, i + 64)
         const uint32_t which = tid >> 6;
         const uint32_t src = which == 0 ? head * 128 : a.n_head * 128 + (which == 1 ? kvh : a.n_head_kv + kvh) * 128;
         const gptr_word from[2] = {mine + at.qkv + src + lane, mine + at.qkv + src + lane + 64};
         uint32_t v[2];
-        if (!words_wait<2>(from, tag, v, a)) sm.bad = 1;
+        if (!words_wait<2>(from, tag, v, WalkBound{a.failed, a.spins})) sm.bad = 1;
         const float raw0 = __uint_as_float(v[0]), raw1 = __uint_as_float(v[1]);
         uint16_t h0, h1;
         if (which == 2) {
@@ -447,7 +423,7 @@ __device__ bool walk_attention(const RmiWalkArgs &a, const WalkWords &at, gptr_w
         uint32_t v[kMine];
 #pragma unroll
         for (int j = 0; j < kMine; j++) from[j] = score_words + (j * T + tid < n_keys ? j * T + tid : n_keys - 1);
-        if (!words_wait<kMine>(from, tag, v, a)) sm.bad = 1;
+        if (!words_wait<kMine>(from, tag, v, WalkBound{a.failed, a.spins})) sm.bad = 1;
         my_max = -INFINITY;
 #pragma unroll
         for (int j = 0; j < kMine; j++) {
@@ -605,9 +581,10 @@ __global__ __launch_bounds__(kWalkThreads) void qwen3_walk_kernel(RmiWalkArgs a)
     if (b < a.n_attn) {
         for (uint32_t i = 0; i < a.n_steps; i++) {
             const uint32_t tag = a.tag0 + 1 + i * (a.n_layer + 1);
-            for (uint32_t l = 0; l < a.n_layer; l++)
+            for (uint32_t l = 0; l < a.n_layer; l++) {
                 if (!walk_attention(a, at, words, mine, b, a.step0 + i, l, tag + l, lds, sm)) return;
-            __syncthreads();
+                __syncthreads();  // the words first: behind the other waves' keys and values they would wait for those
+            }
             if (!walk_head<NE>(a, at, words, mine, tag + a.n_layer, a.keep_logits && i + 1 == a.n_steps, lds, sm)) return;
         }
         return;
@@ -624,17 +601,19 @@ __global__ __launch_bounds__(kWalkThreads) void qwen3_walk_kernel(RmiWalkArgs a)
             octets_load<ND>(gd, a.layers[0].down, tile, ND * 4, sub * ND, lane);
             const uint32_t told = a.tok[step + 1];  // (the next token where the prompt still says it)
             for (uint32_t l = 0; l < a.n_layer; l++) {
-                const uint32_t next = l + 1 < a.n_layer ? l + 1 : l;
+                const RmiWalkLayer next = table_entry(a.layers + (l + 1 < a.n_layer ? l + 1 : l));
                 if (!stage_quants<(NO * 4 * 72 + kWalkThreads - 1) / kWalkThreads>(mine + at.att, tag + l, NO * 4, a, lds, sm)) return;
                 float y = tile_product<NO>(go, lds, sub, lane, hand);
                 x = x + y;
                 if (sub == 0 && L < 2) word_store(words + L * at.n + at.xm + row, __float_as_uint(x), tag + l);
-                octets_load<NO>(go, a.layers[next].o, tile, NO * 4, sub * NO, lane);
+                __syncthreads();  // the words first: behind other waves' weights they would wait for those
+                octets_load<NO>(go, next.o, tile, NO * 4, sub * NO, lane);
                 if (!stage_quants<(ND * 4 * 72 + kWalkThreads - 1) / kWalkThreads>(mine + at.h, tag + l, ND * 4, a, lds, sm)) return;
                 y = tile_product<ND>(gd, lds, sub, lane, hand);
                 x = x + y;
                 if (sub == 0 && L < 2) word_store(words + L * at.n + at.x + row, __float_as_uint(x), tag + l + 1);
-                octets_load<ND>(gd, a.layers[next].down, tile, ND * 4, sub * ND, lane);
+                __syncthreads();  // (x first, too)
+                octets_load<ND>(gd, next.down, tile, ND * 4, sub * ND, lane);
             }
             __syncthreads();
             if (!walk_head<NE>(a, at, words, mine, tag + a.n_layer, a.keep_logits && i + 1 == a.n_steps, lds, sm)) return;
@@ -642,7 +621,7 @@ __global__ __launch_bounds__(kWalkThreads) void qwen3_walk_kernel(RmiWalkArgs a)
             const uint32_t n_wg = gridDim.x, g = tid < n_wg ? tid : n_wg - 1;
             const gptr_word top[4] = {mine + at.top + g * 4, mine + at.top + g * 4 + 1, mine + at.top + g * 4 + 2, mine + at.top + g * 4 + 3};
             uint32_t v[4];
-            if (!words_wait<4>(top, tag + a.n_layer, v, a)) sm.bad = 1;
+            if (!words_wait<4>(top, tag + a.n_layer, v, WalkBound{a.failed, a.spins})) sm.bad = 1;
             Top m{__uint_as_float(v[0]), __uint_as_float(v[1]), v[2], v[3]};
             if (tid >= n_wg) m = Top{-INFINITY, -INFINITY, 0xffffffffu, 1u};
 #pragma unroll
@@ -693,7 +672,7 @@ __global__ __launch_bounds__(kWalkThreads) void qwen3_walk_kernel(RmiWalkArgs a)
         wa.load(a.layers[0].attn_norm);
         wf.load(a.layers[0].ffn_norm);
         for (uint32_t l = 0; l < a.n_layer; l++) {
-            const RmiWalkLayer &next = a.layers[l + 1 < a.n_layer ? l + 1 : l];
+            const RmiWalkLayer next = table_entry(a.layers + (l + 1 < a.n_layer ? l + 1 : l));
             if (!stage_norm<NE>(mine + at.x, tag + l, wa, a, lds, sm)) return;
             {
                 float acc = 0.0f;
@@ -701,6 +680,7 @@ __global__ __launch_bounds__(kWalkThreads) void qwen3_walk_kernel(RmiWalkArgs a)
                 const float y = hsum8_lanes(acc);
                 if (q_live && L < 2) word_store(words + L * at.n + at.qkv + q_tile * 8 + r, __float_as_uint(y), tag + l);
             }
+            __syncthreads();  // every wave's words first: behind others' weights they would wait for those
             octets_load<NE>(gq, next.qkv, q_live ? q_tile : 0, NE, 0, lane);
             wa.load(next.attn_norm);
             if (!g_live) continue;
@@ -722,6 +702,7 @@ __global__ __launch_bounds__(kWalkThreads) void qwen3_walk_kernel(RmiWalkArgs a)
                 }
                 if (blk + a.n_norm < n_blk) __syncthreads();  // gu is written again
             }
+            __syncthreads();
             octets_load<NE>(gg, next.gu, g_off + idx * 4, NE, 0, lane);
             wf.load(next.ffn_norm);
         }
