@@ -7,6 +7,7 @@
 // stand the mixers: three launches a layer and token, the norm included.  Several tokens (prompt passes, portions)
 // take the matrix-core products and the mixers' several-token kernels.
 #include <cmath>
+#include <cstring>
 #include <map>
 #include <string>
 #include <utility>
@@ -14,6 +15,7 @@
 
 #include "folder_session.h"
 #include "seq_mixers.h"
+#include "walk_ruvenex.h"
 
 namespace {
 
@@ -41,7 +43,18 @@ struct RuvenexSession : rmi_hip_folder_session {
     void *attn_scratch = nullptr;
     float *recur_scratch = nullptr;
     int now = 0;  // which of a layer's two history and state buffers the last pass left
+    RmiWalkRvArgs walk{};  // what the launches that walk all layers have in common, where the layers can be walked (walk.words is set)
+    size_t walk_words = 0;
 
+    ~RuvenexSession() override {
+        if (walk.failed) (void)hipHostFree(walk.failed);
+    }
+    bool prepare_walk();
+    bool walk_gave_up() override;
+    void back_one() override {
+        position--;
+        now ^= 1;
+    }
     bool load(const RmiModelFolder &f) override;
     int enqueue_layers(uint32_t step0, uint32_t n, hipStream_t st, float *host_layers) override;
     RmiInput normed(const float *weight) const {
@@ -58,6 +71,22 @@ struct RuvenexSession : rmi_hip_folder_session {
 
 int RuvenexSession::enqueue_layers(uint32_t step0, uint32_t n, hipStream_t st, float *host_layers) {
     int rc = RMI_HIP_OK;
+    if (n == 1 && walks && walk.words && !host_layers && step0 > 0 && step0 < kWalkRvMaxKeys) {
+        if (walk.tag0 > 0xffffffffu - n_runs - 1) {  // the words' tags start anew
+            RMI_HIP_CHECK(hipMemsetAsync(walk.words, 0, walk_words * 8, st));
+            walk.tag0 = 0;
+        }
+        RmiWalkRvArgs a = walk;
+        a.x = x;
+        a.pos = step0;
+        a.now = uint32_t(now);
+        if (walk_spins) a.spins = walk_spins;
+        walk.tag0 += n_runs + 1;
+        rc = rmi_launch_walk_ruvenex(a, st);
+        now ^= 1;
+        position = step0 + 1;
+        return rc;
+    }
     for (uint32_t l = 0; l < n_runs && rc == RMI_HIP_OK; l++) {
         const RuvenexLayer &y = layers[l];
         RmiAttnArgs a{};
@@ -107,6 +136,77 @@ int RuvenexSession::enqueue_layers(uint32_t step0, uint32_t n, hipStream_t st, f
     now ^= 1;
     position = step0 + n;
     return rc;
+}
+
+bool RuvenexSession::walk_gave_up() {
+    if (!walk.failed || !*static_cast<volatile uint32_t *>(walk.failed)) return false;
+    *walk.failed = 0;
+    walks = false;
+    return true;
+}
+
+// The walk's tables, where every layer is of one shape that it takes; false + error text only if memory is missing.
+bool RuvenexSession::prepare_walk() {
+    if (elem != 2) return true;
+    const RuvenexLayer &y0 = layers[0];
+    const RmiAttnShape &a = y0.attn;
+    const RmiRecurShape &r = y0.recur;
+    RmiWalkRvShape s{};
+    constexpr uint32_t kSegs = sizeof s.seg / sizeof *s.seg - 1;
+    if (a.dim != 128 || a.vdim != 128 || r.dim != 128 || r.vdim != 128 || !a.v_norm || a.window || y0.in.n_segs != kSegs) return true;
+    for (const RuvenexLayer &y : layers) {
+        if (memcmp(&y.attn, &a, sizeof a) || memcmp(&y.recur, &r, sizeof r) || memcmp(y.in.start, y0.in.start, sizeof y.in.start) ||
+            y.in.n_segs != kSegs || y.in.n_rows != y0.in.n_rows || y.k_attn != y0.k_attn || y.k_recur != y0.k_recur || y.w_out.k_pad != y0.w_out.k_pad ||
+            y.out.s[0].scale != y0.out.s[0].scale || y.out.s[1].scale != y0.out.s[1].scale)
+            return true;
+    }
+    s.width = width;
+    s.k_in = k_in;
+    s.n_rows = y0.in.n_rows;
+    s.in_ld = y0.w_in.ld;
+    s.out_ld = y0.w_out.ld;
+    s.k_attn = y0.k_attn;
+    s.k_recur = y0.k_recur;
+    s.k_pad = y0.w_out.k_pad;
+    for (uint32_t i = 0; i < kSegs; i++) s.seg[i] = y0.in.start[i];
+    s.seg[kSegs] = s.n_rows;
+    s.heads = a.heads;
+    s.kv_heads = a.kv_heads;
+    s.recur_heads = r.heads;
+    s.taps = a.taps;
+    s.rot_dims = a.rot_dims;
+    s.capacity = cap_pad;
+    s.n_layer = n_runs;
+    s.attn_scale = a.scale;
+    s.left_scale = y0.out.s[0].scale;
+    s.right_scale = y0.out.s[1].scale;
+    s.eps = eps;
+    if (!rmi_walk_ruvenex_fits(s)) return true;
+    std::vector<RmiWalkRvLayer> table;
+    for (const RuvenexLayer &y : layers) {
+        RmiWalkRvLayer t{};
+        t.attn = {y.conv, y.cos_t, y.sin_t, y.k_cache, y.v_cache, {y.hist[0], y.hist[1]}};
+        t.recur = {{y.state[0], y.state[1]}, y.recur_norm};
+        t.in = {y.w_in.data, y.norm, y.in.s[5].bias, y.in.s[5].lower, y.in.s[7].bias, y.in.s[8].bias};
+        t.out = {y.w_out.data};
+        table.push_back(t);
+    }
+    walk_words = rmi_walk_ruvenex_words(s);
+    RmiWalkRvLayer *d = alloc<RmiWalkRvLayer>(table.size());
+    uint64_t *words = alloc<uint64_t>(walk_words, true);
+    if (!d || !words) return false;
+    if (hipMemcpy(d, table.data(), table.size() * sizeof table[0], hipMemcpyHostToDevice) != hipSuccess ||
+        hipHostMalloc(reinterpret_cast<void **>(&walk.failed), 64, hipHostMallocMapped) != hipSuccess) {
+        walk.failed = nullptr;
+        rmi_set_error("the walk's tables could not be uploaded");
+        return false;
+    }
+    *walk.failed = 0;
+    walk.s = s;
+    walk.layers = d;
+    walk.words = words;
+    walk.spins = kWalkRvSpins;
+    return true;
 }
 
 bool RuvenexSession::load(const RmiModelFolder &folder) {
@@ -306,7 +406,7 @@ bool RuvenexSession::load(const RmiModelFolder &folder) {
             !(y.state[1] = alloc<float>(size_t(r.heads) * r.d_pad * r.v_pad, true)))
             return false;
     }
-    return rd.ok;
+    return rd.ok && prepare_walk();
 }
 
 }  // namespace

@@ -26,12 +26,16 @@ struct rmi_hip_folder_session : RmiSession {
     uint32_t *want_rows = nullptr;
     uint32_t position = 0;    // tokens of the current sequence so far
     uint32_t embedded = ~0u;  // the position whose embedding the last sampling launch left in x
+    bool walks = true;        // a token's layers may go through one launch, where the design has it
+    uint32_t walk_spins = 0;  // how often a wait inside such a launch asks; 0: as often as the design has it
 
     // Sizes, weights and buffers; false + error text.
     virtual bool load(const RmiModelFolder &f) = 0;
     // The layers over positions step0 .. step0 + n - 1, whose embeddings are in x.  host_layers: the residual stream
     // behind every layer run, [run][n][width] (synchronises; for comparisons).
     virtual int enqueue_layers(uint32_t step0, uint32_t n, hipStream_t st, float *host_layers) = 0;
+    // The sequence as it was before its last token, which was the last call's only one.
+    virtual void back_one() { position--; }
     // What the head reads of the stream behind the last layer (x_out is not used).
     virtual RmiInput head_input() const = 0;
 
@@ -54,6 +58,7 @@ struct rmi_hip_folder_session : RmiSession {
     int copy_layer(float *host_layers, uint32_t run, uint32_t n, hipStream_t st);
 
   private:
+    int feed_passes(const uint32_t *tokens, uint32_t n, const uint32_t *want, uint32_t n_want, float *out, float *host_layers, hipStream_t st);
     RmiEmbed embed_to() const;
     int embed_tokens(uint32_t step0, uint32_t n, hipStream_t st);
     int enqueue_logits(const uint32_t *rows, uint32_t n_rows, hipStream_t st);

@@ -121,6 +121,19 @@ int rmi_hip_folder_session::feed(const uint32_t *tokens, uint32_t n, const uint3
         RMI_HIP_CHECK(hipStreamSynchronize(st));
     }
     embedded = ~0u;
+    const bool walks_before = walks;
+    if (n > 1) walks = false;  // one that gives up would take the tokens before with it
+    const int rc = feed_passes(tokens, n, want, n_want, out, host_layers, st);
+    if (n > 1) walks = walks_before;
+    if (rc != RMI_HIP_OK || n != 1 || !walk_gave_up()) return rc;
+    // the token once more, by single launches: what the walk wrote lies where they write it, what they read is as it was
+    back_one();
+    return feed_passes(tokens, n, want, n_want, out, host_layers, st);
+}
+
+int rmi_hip_folder_session::feed_passes(const uint32_t *tokens, uint32_t n, const uint32_t *want, uint32_t n_want, float *out, float *host_layers,
+                                        hipStream_t st) {
+    const uint32_t step0 = position;
     const uint32_t most = prompt_pass ? (prompt_pass < pass_rows ? prompt_pass : pass_rows) : 1;
     for (uint32_t at = 0; at < n;) {
         const uint32_t m = n - at < most ? n - at : most;
@@ -264,6 +277,14 @@ int rmi_hip_folder_generate(rmi_hip_folder_session *s, const uint32_t *prompt, u
 int rmi_hip_folder_set_prompt_passes(rmi_hip_folder_session *s, int enabled) {
     if (!s) return rmi_fail(RMI_HIP_E_INVALID, "null session");
     s->prompt_pass = enabled <= 0 ? 0u : enabled == 1 || uint32_t(enabled) > s->pass_rows ? s->pass_rows : uint32_t(enabled);
+    return RMI_HIP_OK;
+}
+
+int rmi_hip_folder_set_walks(rmi_hip_folder_session *s, int enabled) {
+    if (!s) return rmi_fail(RMI_HIP_E_INVALID, "null session");
+    (void)s->walk_gave_up();
+    s->walks = enabled > 0;
+    s->walk_spins = enabled > 1 ? uint32_t(enabled) : 0;
     return RMI_HIP_OK;
 }
 

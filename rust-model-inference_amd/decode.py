@@ -33,6 +33,11 @@ class _Session:
         rounding for model folders)."""
         hip.check(self._fn("set_prompt_passes")(self._h, int(enabled)))
 
+    def set_walks(self, enabled):
+        """Tokens by the launch that walks all layers, where the model's sizes have one (rmi_hip_qwen3_set_walks,
+        rmi_hip_folder_set_walks): 1 (default) on, 0 off."""
+        hip.check(self._fn("set_walks")(self._h, int(enabled)))
+
     def generate(self, prompt, max_new, dump_steps=()):
         prompt = np.ascontiguousarray(prompt, np.uint32)
         steps = prompt.size + max_new - 1
@@ -108,10 +113,6 @@ class Qwen3Session(_Session):
         self._h = hip.lib.rmi_hip_qwen3_create(C.byref(c), C.byref(w))
         if not self._h:
             raise hip.RmiHipError(-1, hip.last_error())
-
-    def set_walks(self, enabled):
-        """Tokens by the launch that walks all layers (rmi_hip_qwen3_set_walks): 1 (default) on, 0 off."""
-        hip.check(hip.lib.rmi_hip_qwen3_set_walks(self._h, int(enabled)))
 
     @classmethod
     def from_gguf(cls, loader, capacity, rounding=hip.ROUND_TIES_EVEN):

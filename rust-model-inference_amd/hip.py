@@ -178,6 +178,7 @@ SIGNATURES = {
     "rmi_hip_folder_reset": (C.c_int, [_vp]),
     "rmi_hip_folder_set_stop_ids": (C.c_int, [_vp, _u32p, _u32]),
     "rmi_hip_folder_set_prompt_passes": (C.c_int, [_vp, C.c_int]),
+    "rmi_hip_folder_set_walks": (C.c_int, [_vp, C.c_int]),
     "rmi_hip_folder_generate": (C.c_int, [_vp, _u32p, _u32, _u32, _u32p, _u32p, _f32p, _u32p, _u32, _f32p,
                                            C.POINTER(C.c_double)]),
     "rmi_hip_ruvenex_open": (_vp, [C.c_char_p, C.c_int, _u32]),
