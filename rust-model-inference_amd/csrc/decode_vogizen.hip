@@ -12,11 +12,13 @@
 // Launches of a layer and token: norm + all that reads it; the mixer (the delta rule one launch, latent attention two:
 // norms + up-projections, attention); output + scale + residual; G; P; a feed-forward adds two.
 #include <cmath>
+#include <cstring>
 #include <string>
 #include <vector>
 
 #include "folder_session.h"
 #include "seq_mixers.h"
+#include "walk_vogizen.h"
 
 namespace {
 
@@ -65,7 +67,18 @@ struct VogizenSession : rmi_hip_folder_session {
     float *delta_scratch = nullptr;
     const float *pending = nullptr;  // the weight of the result in y that x still lacks
     int now = 0;                     // which of a run's two history and state buffers the last pass left
+    RmiWalkVgArgs walk{};  // what the launches that walk all runs have in common, where the runs can be walked (walk.words is set)
+    size_t walk_words = 0;
 
+    ~VogizenSession() override {
+        if (walk.failed) (void)hipHostFree(walk.failed);
+    }
+    bool prepare_walk();
+    bool walk_gave_up() override;
+    void back_one() override {
+        position--;
+        now ^= 1;
+    }
     void begin_sequence() override {
         rmi_hip_folder_session::begin_sequence();
         pending = nullptr;
@@ -222,6 +235,26 @@ int VogizenSession::enqueue_layers(uint32_t step0, uint32_t n, hipStream_t st, f
     const bool one = n == 1 && one_token_gemv, in_prologue = !one || width <= kGemvAddMax;
     int rc = RMI_HIP_OK;
     pending = nullptr;
+    if (n == 1 && walks && walk.words && !host_layers && step0 > 0 && (step0 < walk.s.window ? step0 + 1 : walk.s.window) <= kWalkVgKeys) {
+        if (walk.tag0 > 0xffffffffu - n_runs - 1) {  // the words' tags start anew
+            RMI_HIP_CHECK(hipMemsetAsync(walk.words, 0, walk_words * 8, st));
+            walk.tag0 = 0;
+        }
+        RmiWalkVgArgs a = walk;
+        a.x = x;
+        a.y = y;
+        a.embedded = x_embedded;
+        a.tok = tok;
+        a.pos = step0;
+        a.now = uint32_t(now);
+        if (walk_spins) a.spins = walk_spins;
+        walk.tag0 += n_runs + 1;
+        rc = rmi_launch_walk_vogizen(a, st);
+        pending = layers[runs.back().layer].side_norm;
+        now ^= 1;
+        position = step0 + 1;
+        return rc;
+    }
     for (uint32_t i = 0; i < runs.size() && rc == RMI_HIP_OK; i++) {
         const VogizenRun &r = runs[i];
         const VogizenLayer &l = layers[r.layer];
@@ -254,6 +287,102 @@ int VogizenSession::enqueue_layers(uint32_t step0, uint32_t n, hipStream_t st, f
     now ^= 1;
     position = step0 + n;
     return rc;
+}
+
+bool VogizenSession::walk_gave_up() {
+    if (!walk.failed || !*static_cast<volatile uint32_t *>(walk.failed)) return false;
+    *walk.failed = 0;
+    walks = false;
+    return true;
+}
+
+// The walk's tables, where all layers of a kind are of one shape that it takes; false + error text only if memory is missing.
+bool VogizenSession::prepare_walk() {
+    if (!one_token_gemv || k_in != width) return true;
+    const VogizenLayer *d0 = nullptr, *a0 = nullptr;
+    constexpr uint32_t kDeltaSegs = 6, kDim = 128, kHeads = 16;
+    for (const VogizenLayer &l : layers) {
+        const VogizenLayer *&first = l.delta ? d0 : a0;
+        if (!first) first = &l;
+        if (!l.ffn || l.ff.s[0].n != 6 * width || l.down.s[0].k_end != 3 * width || l.in.n_rows != first->in.n_rows || l.gate.s[0].n != layers[0].gate.s[0].n) return true;
+        if (l.delta) {
+            const RmiDeltaShape &r = l.rule;
+            if (memcmp(&r, &first->rule, sizeof r) || r.heads != kHeads || r.dim != kDim || r.vdim != kDim || l.in.n_segs != kDeltaSegs) return true;
+        } else {
+            const RmiAttnShape &r = l.attn;
+            if (r.heads != kHeads || r.dim != kDim || r.vdim != kDim || r.capacity != first->attn.capacity || r.window != first->attn.window ||
+                r.scale != first->attn.scale || l.q_rank != first->q_rank || l.kv_rank != first->kv_rank || l.w_uq.k_pad != l.q_rank ||
+                l.w_ukv.k_pad != l.kv_rank)
+                return true;
+        }
+    }
+    RmiWalkVgShape s{};
+    s.elem_bytes = elem;
+    s.width = width;
+    s.n_run = n_runs;
+    s.ld_w = layers[0].w_in.ld;
+    s.ld_v = layers[0].w_out.ld;
+    s.ld_ff = layers[0].w_down.ld;
+    s.ld_side = layers[0].w_proj.ld;
+    s.ld_loop = w_loop.ld;
+    s.side = layers[0].gate.s[0].n;
+    s.mul_ld = side_table.ld;
+    s.vocab = vocab;
+    s.kv_heads = kHeads;
+    s.taps = 2;
+    s.window = kWalkVgKeys;
+    s.capacity = kWalkVgKeys;
+    s.eps = eps;
+    if (d0) {
+        s.delta_rows = d0->in.n_rows;
+        s.seg_b = d0->in.start[3];
+        s.seg_a = d0->in.start[4];
+        s.seg_g = d0->in.start[5];
+        s.kv_heads = d0->rule.kv_heads;
+        s.taps = d0->rule.taps;
+    }
+    if (a0) {
+        s.latent_rows = a0->in.n_rows;
+        s.seg_kv = a0->in.start[1];
+        s.q_rank = a0->q_rank;
+        s.kv_rank = a0->kv_rank;
+        s.ld_q = a0->w_uq.ld;
+        s.ld_kv = a0->w_ukv.ld;
+        s.window = a0->attn.window;
+        s.capacity = a0->attn.capacity;
+        s.attn_scale = a0->attn.scale;
+    }
+    if (!rmi_walk_vogizen_fits(s)) return true;
+    std::vector<RmiWalkVgRun> table;
+    const float *before = nullptr;
+    for (const VogizenRun &r : runs) {
+        const VogizenLayer &l = layers[r.layer];
+        RmiWalkVgRun t{};
+        const uint64_t flags = (l.delta ? RmiWalkVgRun::kDelta : 0) | (r.loop_begins ? RmiWalkVgRun::kLoopBegins : 0);
+        t.stream = {l.w_in.data, l.w_ff.data, l.w_down.data, l.w_uq.data, l.w_ukv.data, l.norm1, l.norm2, l.down.s[0].gate, l.dq_norm, l.dkv_norm, before, flags};
+        t.chain = {l.w_out.data, l.w_gate.data, l.w_proj.data, l.gate.s[0].mul, l.out.s[0].gate, before, flags};
+        t.delta = {l.conv, l.rate, l.bias, l.head_norm, {r.hist[0], r.hist[1]}, {r.state[0], r.state[1]}};
+        t.latent = {r.k_cache, r.v_cache};
+        table.push_back(t);
+        before = l.side_norm;
+    }
+    walk_words = rmi_walk_vogizen_words(s);
+    RmiWalkVgRun *d = alloc<RmiWalkVgRun>(table.size());
+    uint64_t *words = alloc<uint64_t>(walk_words, true);
+    if (!d || !words) return false;
+    if (hipMemcpy(d, table.data(), table.size() * sizeof table[0], hipMemcpyHostToDevice) != hipSuccess ||
+        hipHostMalloc(reinterpret_cast<void **>(&walk.failed), 64, hipHostMallocMapped) != hipSuccess) {
+        walk.failed = nullptr;
+        rmi_set_error("the walk's tables could not be uploaded");
+        return false;
+    }
+    *walk.failed = 0;
+    walk.s = s;
+    walk.runs = d;
+    walk.w_loop = w_loop.data;
+    walk.words = words;
+    walk.spins = kWalkVgSpins;
+    return true;
 }
 
 // ------------------------------------------------------------------ loading
@@ -512,7 +641,7 @@ bool VogizenSession::load(const RmiModelFolder &folder) {
         for (uint32_t i = start; i < stop; i++) ok = ok && add_run(i, i == start);
     for (uint32_t i = stop; i < n_layer; i++) ok = ok && add_run(i, false);
     n_runs = uint32_t(runs.size());
-    return ok && rd.ok;
+    return ok && rd.ok && prepare_walk();
 }
 
 }  // namespace
