@@ -124,7 +124,7 @@ struct VogizenSession : rmi_hip_folder_session {
     int loop_in(uint32_t n, bool one, hipStream_t st);
     int mixer(const VogizenLayer &l, const VogizenRun &r, uint32_t step0, uint32_t n, bool one, hipStream_t st);
     int add(const RmiDense &w, const RmiColSegs &segs, uint32_t n, bool one, hipStream_t st) {
-        return one ? rmi_dense_gemv_residual(elem, w, act, segs, x, width, st) : rmi_dense_gemm_residual(elem, w, act, segs, x, width, n, st);
+        return one ? rmi_dense_gemv_residual(elem, w, act, segs, x, width, st) : rmi_dense_gemm_residual(elem, w, act, segs, x, width, n, work, st);
     }
     bool fits(uint32_t k) const { return rmi_dense_gemv_fits(elem, rmi_dense_pad(k, kDenseKAlign)); }
     bool load_latent(RmiFolderReader &rd, VogizenLayer &l, const std::string &p);
@@ -150,7 +150,7 @@ int VogizenSession::read(const RmiDense &w, RmiInput in, const RmiRowSegs &segs,
     if (in.y) in.x_out = x;
     pending = nullptr;
     const int rc = rmi_dense_input(elem, in, nullptr, h, n, w.k_pad, st);
-    return rc == RMI_HIP_OK ? rmi_dense_gemm(elem, w, h, segs, n, st) : rc;
+    return rc == RMI_HIP_OK ? rmi_dense_gemm(elem, w, h, segs, n, work, st) : rc;
 }
 
 int VogizenSession::loop_in(uint32_t n, bool one, hipStream_t st) {
@@ -172,7 +172,7 @@ int VogizenSession::loop_in(uint32_t n, bool one, hipStream_t st) {
         return rc;
     }
     const int rc = rmi_dense_input(elem, in, nullptr, h, n, w_loop.k_pad, st);
-    return rc == RMI_HIP_OK ? rmi_dense_gemm(elem, w_loop, h, s, n, st) : rc;
+    return rc == RMI_HIP_OK ? rmi_dense_gemm(elem, w_loop, h, s, n, work, st) : rc;
 }
 
 // the mixer's result in act, from what the product in front of it left
@@ -212,9 +212,9 @@ int VogizenSession::mixer(const VogizenLayer &l, const VogizenRun &r, uint32_t s
         rc = rmi_dense_gemv_pair(elem, l.w_uq, in_q, l.uq, l.w_ukv, in_kv, l.ukv, st);
     } else {
         rc = rmi_dense_input(elem, in_q, nullptr, h, n, l.w_uq.k_pad, st);
-        if (rc == RMI_HIP_OK) rc = rmi_dense_gemm(elem, l.w_uq, h, l.uq, n, st);
+        if (rc == RMI_HIP_OK) rc = rmi_dense_gemm(elem, l.w_uq, h, l.uq, n, work, st);
         if (rc == RMI_HIP_OK) rc = rmi_dense_input(elem, in_kv, nullptr, h, n, l.w_ukv.k_pad, st);
-        if (rc == RMI_HIP_OK) rc = rmi_dense_gemm(elem, l.w_ukv, h, l.ukv, n, st);
+        if (rc == RMI_HIP_OK) rc = rmi_dense_gemm(elem, l.w_ukv, h, l.ukv, n, work, st);
     }
     if (rc != RMI_HIP_OK) return rc;
     RmiAttnArgs a{};
@@ -278,7 +278,7 @@ int VogizenSession::enqueue_layers(uint32_t step0, uint32_t n, hipStream_t st, f
             in.n = g.s[0].n;
             rc = rmi_dense_gemv(elem, l.w_proj, in, l.proj, st);
         } else {
-            rc = rmi_dense_gemm(elem, l.w_proj, side, l.proj, n, st);
+            rc = rmi_dense_gemm(elem, l.w_proj, side, l.proj, n, work, st);
         }
         pending = l.side_norm;
         if (rc == RMI_HIP_OK && (host_layers || !in_prologue)) rc = settle(n, st);

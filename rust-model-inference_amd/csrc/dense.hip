@@ -33,6 +33,8 @@ __global__ __launch_bounds__(256) void embed_token_kernel(RmiEmbed e, uint32_t t
 // through LDS; a row of a buffer is eight 16-byte pieces, piece p at slot p ^ (row & 7), so that the sixteen rows of a
 // fragment spread over the banks.
 constexpr uint32_t kStepBytes = 128;
+constexpr uint32_t kSplitSteps = 4;  // of small tiles: steps of a round, the unit in which k is divided
+constexpr uint32_t kMaxSplit = 16;
 constexpr int kResidual = -1;  // the epilogue that adds to the residual stream; the others are RmiEpilogue's
 
 // A wave's results, NN x NT tiles of sixteen rows x sixteen tokens: a lane has rows 4 g .. 4 g + 3 of one token of each.
@@ -279,13 +281,115 @@ struct ResidualLines {
     }
 };
 
+// What a column segment adds to the residual stream, onto z, and the accumulators at zero again.
+template <int NN, int NT>
+__device__ __forceinline__ void gather_segment(f32x4 (&acc)[NN][NT], f32x4 (&z)[NN][NT], const RmiColSeg &s, uint32_t width, uint32_t n_tokens, uint32_t row0,
+                                               uint32_t tok0) {
+    const bool quads = (width & 3) == 0;
+#pragma unroll
+    for (int j = 0; j < NT; j++) {
+        const uint32_t tok = tok0 + j * 16;
+#pragma unroll
+        for (int i = 0; i < NN; i++) {
+            const uint32_t row = row0 + i * 16;
+            f32x4 gate = {1.f, 1.f, 1.f, 1.f};
+            if (s.gate && tok < n_tokens && row < width) {
+                const float *at = s.gate + size_t(tok) * s.gate_ld + row;
+                if (quads) {
+                    gate = *reinterpret_cast<const f32x4 *>(at);
+                } else {
+#pragma unroll
+                    for (int r = 0; r < 4; r++)
+                        if (row + r < width) gate[r] = at[r];
+                }
+            }
+            z[i][j] += acc[i][j] * s.scale * gate;
+            acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+        }
+    }
+}
+template <int NN, int NT>
+__device__ __forceinline__ void join_stream(const f32x4 (&z)[NN][NT], float *__restrict__ x, uint32_t width, uint32_t n_tokens, uint32_t row0, uint32_t tok0) {
+    const bool quads = (width & 3) == 0;
+#pragma unroll
+    for (int j = 0; j < NT; j++) {
+        const uint32_t tok = tok0 + j * 16;
+#pragma unroll
+        for (int i = 0; i < NN; i++) {
+            const uint32_t row = row0 + i * 16;
+            if (tok >= n_tokens || row >= width) continue;
+            const size_t at = size_t(tok) * width + row;
+            if (quads) {
+                *reinterpret_cast<f32x4 *>(x + at) += z[i][j];
+            } else {
+#pragma unroll
+                for (int r = 0; r < 4; r++)
+                    if (row + r < width) x[at + r] += z[i][j][r];
+            }
+        }
+    }
+}
+
+// A tile's k over `parts` workgroups.  Each leaves its sums (past the caches, as the parts' workgroups sit on any XCD); the one that
+// counts last adds all of them, in the parts' order, and goes on to the epilogue.  Nobody waits for another.
+struct DenseParts {
+    uint32_t parts, tiles;
+    uint32_t *counts;  // one a tile, zero before and after
+    float *sums;       // [tile][part][values of a thread, by twos][thread]
+};
+template <int NN, int NT>
+__device__ __forceinline__ bool parts_meet(f32x4 (&v)[NN][NT], const DenseParts &dp, uint32_t tile, uint32_t part, uint32_t *last) {
+    constexpr uint32_t kPairs = NN * NT * 2, kPart = kPairs * 256;
+    uint64_t *all = reinterpret_cast<uint64_t *>(dp.sums) + size_t(tile) * dp.parts * kPart + threadIdx.x, *mine = all + size_t(part) * kPart;
+#pragma unroll
+    for (uint32_t k = 0; k < kPairs; k++) {
+        const f32x4 &q = v[k / 2 / NT][k / 2 % NT];
+        const uint64_t pair = uint64_t(__float_as_uint(q[k % 2 * 2])) | uint64_t(__float_as_uint(q[k % 2 * 2 + 1])) << 32;
+        __hip_atomic_store(mine + k * 256, pair, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // (the stores are out before the count says so)
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        const uint32_t n = __hip_atomic_fetch_add(dp.counts + tile, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        *last = n == dp.parts - 1;
+        if (n == dp.parts - 1) __hip_atomic_store(dp.counts + tile, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // for the next launch
+    }
+    __syncthreads();
+    if (!*last) return false;
+#pragma unroll
+    for (int i = 0; i < NN; i++)
+#pragma unroll
+        for (int j = 0; j < NT; j++) v[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    auto add = [&](auto at_a_time, uint32_t p0) {  // parts whose loads are under way together
+        constexpr uint32_t N = at_a_time.value;
+        uint64_t pair[N][kPairs];
+#pragma unroll
+        for (uint32_t p = 0; p < N; p++)
+#pragma unroll
+            for (uint32_t k = 0; k < kPairs; k++)
+                pair[p][k] = __hip_atomic_load(all + size_t(p0 + p) * kPart + k * 256, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+        for (uint32_t p = 0; p < N; p++)
+#pragma unroll
+            for (uint32_t k = 0; k < kPairs; k++) {
+                f32x4 &q = v[k / 2 / NT][k / 2 % NT];
+                q[k % 2 * 2] += __uint_as_float(uint32_t(pair[p][k]));
+                q[k % 2 * 2 + 1] += __uint_as_float(uint32_t(pair[p][k] >> 32));
+            }
+    };
+    uint32_t p = 0;
+    for (; p + 4 <= dp.parts; p += 4) add(std::integral_constant<uint32_t, 4>(), p);
+    for (; p < dp.parts; p++) add(std::integral_constant<uint32_t, 1>(), p);
+    return true;
+}
+
 // Four waves; the pieces of the next PD steps are on their way to registers while one is multiplied.  Small tiles, for
 // products that would leave compute units idle otherwise, have two LDS buffers; 128 x 128 keeps one (NB = 1), so that three
 // workgroups share a compute unit: one round where wider tiles would start a second one for a few workgroups.
-template <typename T, int BN, int BT, int WN, int WT, int PD, int NB, int WPS, int EPI>
+template <typename T, int BN, int BT, int WN, int WT, int PD, int NB, int WPS, int EPI, bool SPLIT = false>
 __global__ __launch_bounds__(256, WPS) void dense_gemm_kernel(const T *__restrict__ w, const T *__restrict__ a, uint32_t n_rows,
                                                               uint32_t k_pad, uint32_t ld, uint32_t n_tokens, uint32_t grid_n, uint32_t grid_t, uint32_t xcd_split,
-                                                         RmiRowSegs rs, RmiColSegs cs, float *__restrict__ x, uint32_t width) {
+                                                         RmiRowSegs rs, RmiColSegs cs, float *__restrict__ x, uint32_t width, DenseParts dp) {
     constexpr bool RESIDUAL = EPI == kResidual;
     static_assert((BN / WN) * (BT / WT) == 4, "four waves");
     static_assert(kDenseKAlign * sizeof(T) % (kStepBytes * PD) == 0, "whole rounds of the register slots");
@@ -293,8 +397,9 @@ __global__ __launch_bounds__(256, WPS) void dense_gemm_kernel(const T *__restric
     constexpr int PW = BN * 8 / 256, PA = (BT * 8 + 255) / 256;  // pieces a thread loads per step
     __shared__ u32x4 lds[NB][(BN + BT) * 8];
     const uint32_t tid = threadIdx.x, lane = tid & 63, wave = uint32_t(__builtin_amdgcn_readfirstlane(int(tid >> 6)));
+    const uint32_t part = SPLIT ? blockIdx.x / dp.tiles : 0, tile = blockIdx.x - part * dp.tiles;
     uint32_t n_tile, t_tile;
-    rmi_gemm_tile_of(blockIdx.x, grid_n, grid_t, 1u, xcd_split, n_tile, t_tile);
+    rmi_gemm_tile_of(tile, grid_n, grid_t, 1u, xcd_split, n_tile, t_tile);
     const uint32_t row0 = n_tile * BN, tok0 = t_tile * BT;
     const uint32_t wn = (wave % (BN / WN)) * WN, wt = (wave / (BN / WN)) * WT;
     const size_t stride = size_t(ld) * sizeof(T);
@@ -321,12 +426,13 @@ __global__ __launch_bounds__(256, WPS) void dense_gemm_kernel(const T *__restric
 #pragma unroll
         for (int j = 0; j < NT; j++) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
     constexpr uint32_t kStepElems = kStepBytes / sizeof(T);
-    const uint32_t n_steps = k_pad / kStepElems;
+    const uint32_t n_steps = k_pad / kStepElems, rounds = n_steps / PD;
+    const uint32_t first = SPLIT ? part * rounds / dp.parts * PD : 0, end = SPLIT ? (part + 1) * rounds / dp.parts * PD : n_steps;
     u32x4 rw[PD][PW], ra[PD][PA];
     auto load = [&](int slot, uint32_t step) {
         // always issued (past the end the last step again): the waits count loads, and a skipped one would make every
         // wait a wait for all
-        step = step < n_steps ? step : n_steps - 1;
+        step = step < end ? step : end - 1;
 #pragma unroll
         for (int i = 0; i < PW; i++) rw[slot][i] = *reinterpret_cast<const u32x4 *>(wsrc[i] + size_t(step) * kStepBytes);
 #pragma unroll
@@ -341,17 +447,26 @@ __global__ __launch_bounds__(256, WPS) void dense_gemm_kernel(const T *__restric
     const uint32_t fr = lane & 15, g = lane >> 4;
 #pragma unroll
     for (int j = 0; j < PD; j++) {
-        load(j, j);
+        load(j, first + j);
         asm volatile("" ::: "memory");  // in this order, and here: the waits in the loop count on it
     }
     park(0, 0);
-    load(0, PD);
+    load(0, first + PD);
     asm volatile("" ::: "memory");
     __syncthreads();
-    uint32_t step = 0;
+    uint32_t step = first;
+    constexpr bool kGather = SPLIT && RESIDUAL;
+    f32x4 z[NN][NT];  // what a part's segments add
+    if constexpr (kGather) {
+#pragma unroll
+        for (int i = 0; i < NN; i++)
+#pragma unroll
+            for (int j = 0; j < NT; j++) z[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
     for (uint32_t seg = 0; seg < (RESIDUAL ? cs.n_segs : 1u); seg++) {
         // segments end at multiples of kDenseKAlign, whole rounds of the register slots
-        const uint32_t seg_end = RESIDUAL ? cs.s[seg].k_end / kStepElems : n_steps;
+        const uint32_t k_end = RESIDUAL ? cs.s[seg].k_end / kStepElems : n_steps, seg_end = SPLIT && end < k_end ? end : k_end;
+        if (SPLIT && seg_end <= step) continue;
         for (; step < seg_end; step += PD) {
 #pragma unroll
             for (int j = 0; j < PD; j++) {  // register slots by compile-time index
@@ -380,9 +495,22 @@ __global__ __launch_bounds__(256, WPS) void dense_gemm_kernel(const T *__restric
                 __syncthreads();
             }
         }
-        if constexpr (RESIDUAL) fold_segment<NN, NT>(acc, cs.s[seg], x, width, n_tokens, row0 + wn + g * 4, tok0 + wt + fr);
+        if constexpr (kGather)
+            gather_segment<NN, NT>(acc, z, cs.s[seg], width, n_tokens, row0 + wn + g * 4, tok0 + wt + fr);
+        else if constexpr (RESIDUAL)
+            fold_segment<NN, NT>(acc, cs.s[seg], x, width, n_tokens, row0 + wn + g * 4, tok0 + wt + fr);
     }
 
+    if constexpr (SPLIT) {
+        __shared__ uint32_t last;
+        bool here;
+        if constexpr (RESIDUAL)
+            here = parts_meet<NN, NT>(z, dp, tile, part, &last);
+        else
+            here = parts_meet<NN, NT>(acc, dp, tile, part, &last);
+        if (!here) return;
+    }
+    if constexpr (kGather) join_stream<NN, NT>(z, x, width, n_tokens, row0 + wn + g * 4, tok0 + wt + fr);
     if constexpr (!RESIDUAL) store_rows<T, EPI, NN, NT>(acc, rs, n_rows, n_tokens, row0 + wn, tok0 + wt + fr, g);
 }
 
@@ -555,7 +683,9 @@ struct TileCost {
     uint32_t rows, tokens, waves, fit;
     float fixed, round, first, more, whole, out, activated, residual;
 };
-constexpr TileCost kTile16 = {kTile64x16, 64, 16, 4, 4, 0, 0, 0, 0, 0, 0, 0, 0};
+// 64 x 16 is what up to sixteen tokens take; its estimates only say over how many workgroups k goes
+constexpr TileCost kTile16Bf16 = {kTile64x16, 64, 16, 4, 4, 4.0f, 0.66f, 0.165f, 0.07f, 0.1f, 0.2f, 0, 0};
+constexpr TileCost kTile16F32 = {kTile64x16, 64, 16, 4, 4, 4.2f, 0.72f, 0.25f, 0.05f, 0.12f, 0.3f, 0, 0};
 constexpr TileCost kCostsBf16[] = {
     {kTile64x32, 64, 32, 4, 4, 4.04f, 0.728f, 0.174f, 0.078f, 0.113f, 0.347f, 0, 0},
     {kTile64x64, 64, 64, 4, 4, 3.86f, 0.845f, 0.302f, 0.0412f, 0.154f, 1.08f, 1.81f, 0.973f},
@@ -570,62 +700,86 @@ constexpr TileCost kCostsF32[] = {
     {kTile64x128, 64, 128, 8, 2, 3.56f, 1.78f, 0.959f, 0, 0.845f, 2.04f, 2.0f, 6.56f},
     {kTile128x128, 128, 128, 8, 2, 6.12f, 3.54f, 1.81f, 0.04f, 1.67f, 2.36f, 5.63f, 16.2f}};
 
-const TileCost &dense_tile_of(bool bf16, int epilogue, uint32_t n_rows, uint32_t n_tokens, uint32_t n_steps) {
-    if (n_tokens <= kTile16.tokens) return kTile16;
+// k over several workgroups a tile (where the caller has memory for it): a workgroup takes its share of the steps, and the parts' sums cost a
+// hand-over and a way out and back.  bf16 stays within a workgroup a compute unit, beyond which L2 bounds it; f32 is divided also where the
+// tiles are a round and a bit, as the matrix cores bound it and the bit costs a whole one.  Three in a hundred at least are to be gained.
+// us by the tile without parts | so: bf16 residual 1024 x 6144, 9 tokens 19.4 | 9.1, 40 tokens 19.6 | 9.5, 128 tokens 21.5 | 10.8, 300 tokens
+// 20.2 | 18.2; 4096 x 12288, 64 tokens 45 | 29; f32 residual 2048 x 6144, 300 tokens 110 | 75, 1024 x 3072, 60 tokens 34 | 12; rows
+// 128 x 2048, 300 tokens in f32 23.5 | 9.5.  Not divided: bf16 2048 x 12288, 512 tokens, 54 whole, 57 by two; f32 6144 x 2048, 300 tokens, 68, 76.
+struct DenseChoice {
+    const TileCost *tile;
+    uint32_t parts;
+};
+DenseChoice dense_tile_of(bool bf16, int epilogue, uint32_t n_rows, uint32_t n_tokens, uint32_t n_steps, bool may_split) {
     const uint32_t cus = rmi_device_cus() > 0 ? uint32_t(rmi_device_cus()) : 1;
-    const TileCost *best = nullptr;
+    DenseChoice best{nullptr, 1};
     double least = 0;
     auto consider = [&](const TileCost &c) {
         if (epilogue == kResidual && c.tile == kTile256x256) return;  // (2 % the better at the widest at most, and registers spilled, by the older way out)
         const uint64_t tiles = uint64_t((n_rows + c.rows - 1) / c.rows) * ((n_tokens + c.tokens - 1) / c.tokens);
-        const uint64_t rounds = tiles / (c.fit * cus), left = tiles % (c.fit * cus);
-        double step = double(rounds) * c.round;
-        if (left) step += c.first + c.whole * double((left - 1) / cus) + (left > cus ? c.more * (double(left) / cus - 1.0) : 0.0);
-        const double end = c.out + (epilogue == kResidual ? c.residual : epilogue == kRowsActed || epilogue == kRowsTimesTable ? c.activated : 0.0f);
-        const double us = c.fixed + n_steps * step + double(tiles) / cus * end;
-        if (!best || us < least) least = us, best = &c;
+        const uint32_t rounds = n_steps / kSplitSteps;
+        for (uint32_t parts = 1; parts <= kMaxSplit; parts++) {
+            const uint64_t groups = tiles * parts, sums = groups * c.rows * c.tokens;
+            if (parts > 1 && (!may_split || c.tokens > 64 || parts > rounds || tiles > kDenseCounters || sums > kDenseSums || (bf16 && groups > cus))) break;
+            const uint64_t full = groups / (c.fit * cus), left = groups % (c.fit * cus);
+            double step = double(full) * c.round;
+            if (left) step += c.first + c.whole * double((left - 1) / cus) + (left > cus ? c.more * (double(left) / cus - 1.0) : 0.0);
+            const double end = c.out + (epilogue == kResidual ? c.residual : epilogue == kRowsActed || epilogue == kRowsTimesTable ? c.activated : 0.0f);
+            double us = c.fixed + (parts == 1 ? n_steps : (rounds + parts - 1) / parts * kSplitSteps) * step + double(tiles) / cus * end;
+            if (parts > 1) us = (us + 2.0 + double(sums) * 8 / 4.5e6) * 1.03;
+            if (!best.tile || us < least) least = us, best = DenseChoice{&c, parts};
+        }
     };
-    if (bf16)
+    if (n_tokens <= kTile16Bf16.tokens)
+        consider(bf16 ? kTile16Bf16 : kTile16F32);
+    else if (bf16)
         for (const TileCost &c : kCostsBf16) consider(c);
     else
         for (const TileCost &c : kCostsF32) consider(c);
-    return *best;
+    return best;
 }
 
 template <typename T, int EPI>
 int launch_gemm(const RmiDense &w, const void *a, const RmiRowSegs &rs, const RmiColSegs &cs, float *x, uint32_t width,
-                uint32_t n_tokens, hipStream_t st) {
+                uint32_t n_tokens, const RmiDenseWork *work, hipStream_t st) {
     const uint32_t n_rows = EPI == kResidual ? width : w.n_rows;
-    const TileCost &tile = dense_tile_of(sizeof(T) == 2, EPI, n_rows, n_tokens, uint32_t(w.k_pad * sizeof(T) / kStepBytes));
-    auto launch = [&](auto kernel, const RmiColSegs &c) {
-        const uint32_t gn = (n_rows + tile.rows - 1) / tile.rows, gt = (n_tokens + tile.tokens - 1) / tile.tokens;
-        const uint32_t split = rmi_gemm_xcd_split(gn, gt, double(n_rows) * w.k_pad, double(n_tokens) * w.k_pad);
-        hipLaunchKernelGGL(kernel, dim3(gn * gt), dim3(64 * tile.waves), 0, st, static_cast<const T *>(w.data), static_cast<const T *>(a), n_rows,
-                           w.k_pad, w.ld, n_tokens, gn, gt, split, rs, c, x, width);
+    const DenseChoice choice = dense_tile_of(sizeof(T) == 2, EPI, n_rows, n_tokens, uint32_t(w.k_pad * sizeof(T) / kStepBytes), work != nullptr);
+    const TileCost &tile = *choice.tile;
+    const uint32_t gn = (n_rows + tile.rows - 1) / tile.rows, gt = (n_tokens + tile.tokens - 1) / tile.tokens;
+    const uint32_t split = rmi_gemm_xcd_split(gn, gt, double(n_rows) * w.k_pad, double(n_tokens) * w.k_pad);
+    auto launch = [&](auto kernel, uint32_t blocks, const RmiColSegs &c, auto... more) {
+        hipLaunchKernelGGL(kernel, dim3(blocks), dim3(64 * tile.waves), 0, st, static_cast<const T *>(w.data), static_cast<const T *>(a), n_rows,
+                           w.k_pad, w.ld, n_tokens, gn, gt, split, rs, c, x, width, more...);
     };
-    auto go = [&](auto kernel) { launch(kernel, cs); };
+    auto go = [&](auto whole, auto in_parts) {
+        const DenseParts dp{choice.parts, gn * gt, work ? work->counts : nullptr, work ? work->sums : nullptr};
+        if (choice.parts > 1)
+            launch(in_parts, gn * gt * choice.parts, cs, dp);
+        else
+            launch(whole, gn * gt, cs, dp);
+    };
     auto go_wide = [&](auto kernel) {  // a launch for every column segment
         if constexpr (EPI != kResidual) {
-            launch(kernel, cs);
+            launch(kernel, gn * gt, cs);
         } else {
             for (uint32_t i = 0; i < cs.n_segs; i++) {
                 RmiColSegs one{};
                 one.s[0] = cs.s[i];
                 one.n_segs = 1;
                 one.k_begin = i ? cs.s[i - 1].k_end : 0;
-                launch(kernel, one);
+                launch(kernel, gn * gt, one);
             }
         }
     };
     switch (tile.tile) {
-    case kTile64x16: go(dense_gemm_kernel<T, 64, 16, 16, 16, 4, 2, 4, EPI>); break;
-    case kTile64x32: go(dense_gemm_kernel<T, 64, 32, 32, 16, 4, 2, 4, EPI>); break;
-    case kTile64x64: go(dense_gemm_kernel<T, 64, 64, 32, 32, 4, 2, 4, EPI>); break;
+    case kTile64x16: go(dense_gemm_kernel<T, 64, 16, 16, 16, kSplitSteps, 2, 4, EPI>, dense_gemm_kernel<T, 64, 16, 16, 16, kSplitSteps, 2, 4, EPI, true>); break;
+    case kTile64x32: go(dense_gemm_kernel<T, 64, 32, 32, 16, kSplitSteps, 2, 4, EPI>, dense_gemm_kernel<T, 64, 32, 32, 16, kSplitSteps, 2, 4, EPI, true>); break;
+    case kTile64x64: go(dense_gemm_kernel<T, 64, 64, 32, 32, kSplitSteps, 2, 4, EPI>, dense_gemm_kernel<T, 64, 64, 32, 32, kSplitSteps, 2, 4, EPI, true>); break;
     case kTile64x128: go_wide(dense_gemm_wide_kernel<T, 64, 128, 32, 32, 3, 2, EPI>); break;
     case kTile128x128: go_wide(dense_gemm_wide_kernel<T, 128, 128, 64, 32, 2, 4, EPI>); break;
     default:
         if constexpr (sizeof(T) == 2) {
-            if (tile.tile == kTile128x128w4) go(dense_gemm_kernel<T, 128, 128, 64, 64, 1, 1, 3, EPI>);
+            if (tile.tile == kTile128x128w4) launch(dense_gemm_kernel<T, 128, 128, 64, 64, 1, 1, 3, EPI>, gn * gt, cs, DenseParts{});
             if (tile.tile == kTile128x256) go_wide(dense_gemm_wide_kernel<T, 128, 256, 64, 64, 3, 2, EPI>);
             if constexpr (EPI != kResidual)
                 if (tile.tile == kTile256x256) go_wide(dense_gemm_wide_kernel<T, 256, 256, 128, 64, 2, 2, EPI>);
@@ -638,8 +792,13 @@ int launch_gemm(const RmiDense &w, const void *a, const RmiRowSegs &rs, const Rm
 }  // namespace
 
 uint32_t rmi_dense_tile(uint32_t elem_bytes, int epilogue, uint32_t n_rows, uint32_t k_pad, uint32_t n_tokens) {
-    const TileCost &t = dense_tile_of(elem_bytes == 2, epilogue, n_rows, n_tokens, k_pad * elem_bytes / kStepBytes);
+    const TileCost &t = *dense_tile_of(elem_bytes == 2, epilogue, n_rows, n_tokens, k_pad * elem_bytes / kStepBytes, false).tile;
     return t.rows << 16 | t.tokens << 4 | t.waves;
+}
+
+uint32_t rmi_dense_parts(uint32_t elem_bytes, int epilogue, uint32_t n_rows, uint32_t k_pad, uint32_t n_tokens) {
+    const DenseChoice c = dense_tile_of(elem_bytes == 2, epilogue, n_rows, n_tokens, k_pad * elem_bytes / kStepBytes, true);
+    return c.parts << 16 | c.tile->tokens << 4 | c.tile->waves;
 }
 
 int rmi_dense_input(uint32_t elem_bytes, const RmiInput &in, const uint32_t *rows, void *h, uint32_t n_tokens, uint32_t k_pad,
@@ -679,27 +838,36 @@ int rmi_dense_embed_token(uint32_t elem_bytes, const RmiEmbed &e, uint32_t token
     return RMI_HIP_OK;
 }
 
-int rmi_dense_gemm(uint32_t elem_bytes, const RmiDense &w, const void *a, const RmiRowSegs &segs, uint32_t n_tokens, hipStream_t st) {
+int rmi_dense_gemm(uint32_t elem_bytes, const RmiDense &w, const void *a, const RmiRowSegs &segs, uint32_t n_tokens, const RmiDenseWork &work, hipStream_t st) {
     if (n_tokens == 0 || w.n_rows == 0) return RMI_HIP_OK;
     const int rc = rmi_check_row_segs(elem_bytes, w, segs);
     if (rc != RMI_HIP_OK) return rc;
     auto go = [&](auto type) {
         using T = decltype(type);
         switch (rmi_epilogue_of(segs)) {
-            case kRowsActed: return launch_gemm<T, kRowsActed>(w, a, segs, RmiColSegs{}, nullptr, 0, n_tokens, st);
-            case kRowsPaired: return launch_gemm<T, kRowsPaired>(w, a, segs, RmiColSegs{}, nullptr, 0, n_tokens, st);
-            case kRowsTimesTable: return launch_gemm<T, kRowsTimesTable>(w, a, segs, RmiColSegs{}, nullptr, 0, n_tokens, st);
-            default: return launch_gemm<T, kRowsPlain>(w, a, segs, RmiColSegs{}, nullptr, 0, n_tokens, st);
+            case kRowsActed: return launch_gemm<T, kRowsActed>(w, a, segs, RmiColSegs{}, nullptr, 0, n_tokens, work.counts ? &work : nullptr, st);
+            case kRowsPaired: return launch_gemm<T, kRowsPaired>(w, a, segs, RmiColSegs{}, nullptr, 0, n_tokens, work.counts ? &work : nullptr, st);
+            case kRowsTimesTable: return launch_gemm<T, kRowsTimesTable>(w, a, segs, RmiColSegs{}, nullptr, 0, n_tokens, work.counts ? &work : nullptr, st);
+            default: return launch_gemm<T, kRowsPlain>(w, a, segs, RmiColSegs{}, nullptr, 0, n_tokens, work.counts ? &work : nullptr, st);
         }
     };
     return elem_bytes == 2 ? go(rmi_bf16()) : go(float());
 }
 
 int rmi_dense_gemm_residual(uint32_t elem_bytes, const RmiDense &w, const void *a, const RmiColSegs &segs, float *x, uint32_t width,
-                            uint32_t n_tokens, hipStream_t st) {
+                            uint32_t n_tokens, const RmiDenseWork &work, hipStream_t st) {
     if (n_tokens == 0) return RMI_HIP_OK;
     const int rc = rmi_check_col_segs(elem_bytes, w, segs, width);
     if (rc != RMI_HIP_OK) return rc;
-    return elem_bytes == 2 ? launch_gemm<rmi_bf16, kResidual>(w, a, RmiRowSegs{}, segs, x, width, n_tokens, st)
-                           : launch_gemm<float, kResidual>(w, a, RmiRowSegs{}, segs, x, width, n_tokens, st);
+    return elem_bytes == 2 ? launch_gemm<rmi_bf16, kResidual>(w, a, RmiRowSegs{}, segs, x, width, n_tokens, work.counts ? &work : nullptr, st)
+                           : launch_gemm<float, kResidual>(w, a, RmiRowSegs{}, segs, x, width, n_tokens, work.counts ? &work : nullptr, st);
+}
+
+int rmi_dense_gemm(uint32_t elem_bytes, const RmiDense &w, const void *a, const RmiRowSegs &segs, uint32_t n_tokens, hipStream_t st) {
+    return rmi_dense_gemm(elem_bytes, w, a, segs, n_tokens, RmiDenseWork{}, st);
+}
+
+int rmi_dense_gemm_residual(uint32_t elem_bytes, const RmiDense &w, const void *a, const RmiColSegs &segs, float *x, uint32_t width,
+                            uint32_t n_tokens, hipStream_t st) {
+    return rmi_dense_gemm_residual(elem_bytes, w, a, segs, x, width, n_tokens, RmiDenseWork{}, st);
 }

@@ -22,6 +22,7 @@ struct rmi_hip_folder_session : RmiSession {
     float *x = nullptr;    // the residual stream of a pass, [token][width]; a design may exchange it for another buffer
     float *x_embedded = nullptr;  // a copy of the embedding output, for designs that read it again
     void *h = nullptr;            // the operand of the product under way
+    RmiDenseWork work;            // of the products of several tokens
     float *logits = nullptr;
     uint32_t *want_rows = nullptr;
     uint32_t position = 0;    // tokens of the current sequence so far

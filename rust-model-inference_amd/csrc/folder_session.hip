@@ -49,7 +49,7 @@ int rmi_hip_folder_session::enqueue_logits(const uint32_t *rows, uint32_t n_rows
     const RmiInput in = head_input();
     if (n_rows == 1 && !rows && rmi_dense_gemv_fits(elem, k_in)) return rmi_dense_gemv(elem, head, in, s, st);
     const int rc = rmi_dense_input(elem, in, rows, h, n_rows, k_in, st);
-    return rc == RMI_HIP_OK ? rmi_dense_gemm(elem, head, h, s, n_rows, st) : rc;
+    return rc == RMI_HIP_OK ? rmi_dense_gemm(elem, head, h, s, n_rows, work, st) : rc;
 }
 
 // last: the place of the pass's last sampled position, whose token's embedding is left for the next step
@@ -200,7 +200,8 @@ bool rmi_hip_folder_session::load_common(RmiFolderReader &rd) {
 bool rmi_hip_folder_session::alloc_common(uint32_t max_k) {
     if (max_k < k_in) max_k = k_in;
     return alloc_sampling() && (x = alloc<float>(size_t(pass_rows) * width, true)) &&
-           (h = alloc_bytes(size_t(pass_rows) * (max_k + 128) * elem, true)) && (logits = alloc<float>(size_t(logit_rows) * vocab, true)) &&
+           (h = alloc_bytes(size_t(pass_rows) * (max_k + 128) * elem, true)) && (work.counts = alloc<uint32_t>(kDenseCounters, true)) &&
+           (work.sums = alloc<float>(kDenseSums, false)) && (logits = alloc<float>(size_t(logit_rows) * vocab, true)) &&
            (want_rows = alloc<uint32_t>(kLogitRows, true)) && (partial = alloc_bytes(size_t(logit_rows) * kArgmaxGroups * kTopBytes, false));
 }
 
