@@ -127,8 +127,7 @@ int RuvenexSession::enqueue_layers(uint32_t step0, uint32_t n, hipStream_t st, f
         } else {
             rc = rmi_dense_input(elem, normed(y.norm), nullptr, h, n, k_in, st);
             if (rc == RMI_HIP_OK) rc = rmi_dense_gemm(elem, y.w_in, h, y.in, n, work, st);
-            if (rc == RMI_HIP_OK) rc = rmi_attn_pass(elem, y.attn, a, st);
-            if (rc == RMI_HIP_OK) rc = rmi_recur_pass(elem, y.recur, r, st);
+            if (rc == RMI_HIP_OK) rc = rmi_mixers_pass(elem, y.attn, a, y.recur, r, st);
             if (rc == RMI_HIP_OK) rc = rmi_dense_gemm_residual(elem, y.w_out, act, y.out, x, width, n, work, st);
         }
         if (host_layers && rc == RMI_HIP_OK) rc = copy_layer(host_layers, l, n, st);

@@ -92,6 +92,8 @@ size_t rmi_delta_scratch_floats(const RmiDeltaShape &s, uint32_t max_tokens);
 // several tokens: the convolution's launch, the attention's; the recurrence's three; the delta rule's three
 int rmi_attn_pass(uint32_t elem_bytes, const RmiAttnShape &s, const RmiAttnArgs &a, hipStream_t st);
 int rmi_recur_pass(uint32_t elem_bytes, const RmiRecurShape &s, const RmiRecurArgs &a, hipStream_t st);
+// both mixers of the same tokens, side by side where their heads are of 128
+int rmi_mixers_pass(uint32_t elem_bytes, const RmiAttnShape &as, const RmiAttnArgs &aa, const RmiRecurShape &rs, const RmiRecurArgs &ra, hipStream_t st);
 // one token: either mixer may be left out (nullptr); both go into one launch
 int rmi_mixers_step(uint32_t elem_bytes, const RmiAttnShape *as, const RmiAttnArgs *aa, const RmiRecurShape *rs, const RmiRecurArgs *ra,
                     const RmiAhead &ahead, hipStream_t st);

@@ -132,13 +132,13 @@ __device__ __forceinline__ float2 pair_row(const RmiAttnShape &s, const RmiAttnA
 
 // A run of tokens: the taps and a sliding window of projected values stay in registers; every row is read once.
 template <typename T>
-__global__ __launch_bounds__(256) void conv_rotate_pairs_kernel(RmiAttnShape s, RmiAttnArgs a) {
-    const uint32_t lane = threadIdx.x & 63, head = blockIdx.x;
+__device__ __forceinline__ void conv_rotate_pairs(const RmiAttnShape &s, const RmiAttnArgs &a, uint32_t head, uint32_t run) {
+    const uint32_t lane = threadIdx.x & 63;
     const uint32_t channels = (s.heads + s.kv_heads) * s.dim + s.kv_heads * s.vdim;
     const ConvCtx x{a.u, a.hist_in, a.conv, channels, s.taps};
-    if (blockIdx.y == 0) conv_head_carry(x, s, a, head);
+    if (run == 0) conv_head_carry(x, s, a, head);
     // runs end at multiples of kConvRun positions: a value block takes four keys of a channel in one store
-    const uint32_t p_run = a.pos0 / kConvRun * kConvRun + (blockIdx.y * 4 + uint32_t(__builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6)))) * kConvRun;
+    const uint32_t p_run = a.pos0 / kConvRun * kConvRun + (run * 4 + uint32_t(__builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6)))) * kConvRun;
     if (p_run >= a.pos0 + a.n_tokens) return;
     const uint32_t skip = p_run < a.pos0 ? a.pos0 - p_run : 0;  // positions of the first run that came before
     const uint32_t t0 = p_run + skip - a.pos0;
@@ -228,6 +228,10 @@ __global__ __launch_bounds__(256) void conv_rotate_pairs_kernel(RmiAttnShape s, 
             }
         }
     }
+}
+template <typename T>
+__global__ __launch_bounds__(256) void conv_rotate_pairs_kernel(RmiAttnShape s, RmiAttnArgs a) {
+    conv_rotate_pairs<T>(s, a, blockIdx.x, blockIdx.y);
 }
 
 // p + bytes: a uniform pointer and 32 bits of a lane's own, which an access takes as they are
@@ -447,11 +451,10 @@ __device__ __forceinline__ void attn_store(const RmiAttnShape &s, const RmiAttnA
 
 // several tokens: a workgroup takes QT tiles, each of its four waves a quarter of the keys they see; merged in LDS
 template <typename T, int BUCKET, int QT, bool EVERY>
-__global__ __launch_bounds__(256) void attn_pass_kernel(RmiAttnShape s, RmiAttnArgs a) {
-    extern __shared__ __attribute__((aligned(16))) uint8_t lds_raw[];
+__device__ __forceinline__ void attn_pass_block(const RmiAttnShape &s, const RmiAttnArgs &a, uint32_t block, uint32_t n_blocks, uint8_t *lds_raw) {
     const uint32_t tid = threadIdx.x, lane = tid & 63, wave = uint32_t(__builtin_amdgcn_readfirstlane(int(tid >> 6))), fr = lane & 15, g4 = lane >> 4;
-    const uint32_t group = s.heads / s.kv_heads, kvh = blockIdx.x % s.kv_heads, n_cols = a.n_tokens * group;
-    const uint32_t tile = gridDim.x / s.kv_heads - 1 - blockIdx.x / s.kv_heads;  // the longest columns first
+    const uint32_t group = s.heads / s.kv_heads, kvh = block % s.kv_heads, n_cols = a.n_tokens * group;
+    const uint32_t tile = n_blocks / s.kv_heads - 1 - block / s.kv_heads;  // the longest columns first
     AttnWave<T, BUCKET, QT, EVERY> w;
     w.init();
     int last[QT];
@@ -506,6 +509,11 @@ __global__ __launch_bounds__(256) void attn_pass_kernel(RmiAttnShape s, RmiAttnA
         const uint32_t mc = first_col + c, t = mc / group, head = kvh * group + mc % group;
         attn_store<T>(s, a, t, head, d, o * ((a.gate ? a.gate[size_t(t) * s.heads + head] : 1.0f) / sum));
     }
+}
+template <typename T, int BUCKET, int QT, bool EVERY>
+__global__ __launch_bounds__(256) void attn_pass_kernel(RmiAttnShape s, RmiAttnArgs a) {
+    extern __shared__ __attribute__((aligned(16))) uint8_t lds_raw[];
+    attn_pass_block<T, BUCKET, QT, EVERY>(s, a, blockIdx.x, gridDim.x, lds_raw);
 }
 
 // Few columns: the keys are divided over `parts` workgroups and their four waves; each workgroup merges its waves in
@@ -1005,56 +1013,91 @@ __host__ __device__ inline RecurScratch recur_scratch_at(float *p, const RmiRecu
     return r;
 }
 
-// one chunk of one head
-__global__ __launch_bounds__(256) void recur_factors_kernel(RmiRecurShape s, RmiRecurArgs a, uint32_t n_chunks) {
-    extern __shared__ __attribute__((aligned(16))) uint8_t lds_raw[];
-    float *fl = reinterpret_cast<float *>(lds_raw);            // [16][d_pad + 4]
-    const uint32_t ld = s.d_pad + 4;
-    float *ql = fl + kChunk * ld;                              // [16][d_pad + 4]
-    float *red = ql + kChunk * ld;                             // [4][16][16]
-    const uint32_t tid = threadIdx.x, chunk = blockIdx.x, head = blockIdx.y, t0 = chunk * kChunk;
+// One chunk of one head, of up to BUCKET channels.  What bounds it: f and q come by loads that no branch stands in front of (a value past the
+// end is taken out behind them), so that all are under way together; with one behind a branch each, 64 workgroups took 14.6 us.  The two
+// products over a chunk's tokens are a wave's each, and A reads four channels at a time.
+template <uint32_t BUCKET>
+constexpr uint32_t kFactorsLds = 2 * kChunk * (BUCKET + 4) + 1024;  // floats
+template <uint32_t BUCKET>
+__device__ __forceinline__ void recur_factors(const RmiRecurShape &s, const RmiRecurArgs &a, uint32_t n_chunks, uint32_t chunk, uint32_t head, float *lds) {
+    constexpr uint32_t ld = BUCKET + 4, kQuads = BUCKET / 4, kSlots = kChunk * kQuads / 256;
+    float *fl = lds, *ql = fl + kChunk * ld, *red = ql + kChunk * ld;  // [16][ld] twice, [4][16][16]
+    const uint32_t tid = threadIdx.x, t0 = chunk * kChunk;
     const RecurScratch ws = recur_scratch_at(a.scratch, s, n_chunks);
     const size_t hc = size_t(head) * n_chunks + chunk;
-    for (uint32_t e = tid; e < kChunk * s.d_pad; e += 256) {
-        const uint32_t t = e / s.d_pad, d = e % s.d_pad;
-        const bool live = t0 + t < a.n_tokens && d < s.dim;
-        const size_t at = size_t(t0 + t) * s.heads * s.dim + size_t(head) * s.dim + d;
-        fl[t * ld + d] = live ? a.f[at] : 1.0f;  // a token past the end changes nothing
-        ql[t * ld + d] = live ? a.q[at] : 0.0f;
+    f32x4 fv[kSlots], qv[kSlots];
+    auto source = [&](uint32_t i, uint32_t e) {  // of channel e of the slot's quad
+        const uint32_t t = t0 + (tid + i * 256) / kQuads, d = (tid + i * 256) % kQuads * 4 + e;
+        return size_t(t < a.n_tokens ? t : a.n_tokens - 1) * s.heads * s.dim + size_t(head) * s.dim + (d < s.dim ? d : 0);
+    };
+    if (s.dim % 4 == 0) {
+#pragma unroll
+        for (uint32_t i = 0; i < kSlots; i++) {
+            fv[i] = *reinterpret_cast<const f32x4 *>(a.f + source(i, 0));
+            qv[i] = *reinterpret_cast<const f32x4 *>(a.q + source(i, 0));
+        }
+    } else {
+#pragma unroll
+        for (uint32_t i = 0; i < kSlots; i++)
+#pragma unroll
+            for (uint32_t e = 0; e < 4; e++) {
+                fv[i][e] = a.f[source(i, e)];
+                qv[i][e] = a.q[source(i, e)];
+            }
+    }
+#pragma unroll
+    for (uint32_t i = 0; i < kSlots; i++) {
+        const uint32_t t = (tid + i * 256) / kQuads, d = (tid + i * 256) % kQuads * 4;
+#pragma unroll
+        for (uint32_t e = 0; e < 4; e++) {
+            const bool live = t0 + t < a.n_tokens && d + e < s.dim;
+            fv[i][e] = live ? fv[i][e] : 1.0f;  // a token past the end changes nothing
+            qv[i][e] = live ? qv[i][e] : 0.0f;
+        }
+        *reinterpret_cast<f32x4 *>(fl + t * ld + d) = fv[i];
+        *reinterpret_cast<f32x4 *>(ql + t * ld + d) = qv[i];
     }
     __syncthreads();
-    for (uint32_t d = tid; d < s.d_pad; d += 256) {
+    for (uint32_t i = tid; i < 2 * BUCKET; i += 256) {
+        const uint32_t d = i % BUCKET;
+        if (d >= s.d_pad) continue;
         float p = 1.0f;
+        if (i < BUCKET) {
 #pragma unroll
-        for (uint32_t t = 0; t < kChunk; t++) {
-            p *= fl[t * ld + d];
-            ws.qp[(hc * kChunk + t) * s.d_pad + d] = ql[t * ld + d] * p;
+            for (uint32_t t = 0; t < kChunk; t++) {
+                p *= fl[t * ld + d];
+                ws.qp[(hc * kChunk + t) * s.d_pad + d] = ql[t * ld + d] * p;
+            }
+            ws.pc[hc * s.d_pad + d] = p;
+        } else {
+            float k[kChunk];
+#pragma unroll
+            for (int t = kChunk - 1; t >= 0; t--) {
+                const float f = fl[t * ld + d];
+                k[t] = (1.0f - f) * p;
+                p *= f;
+            }
+#pragma unroll
+            for (uint32_t j = 0; j < kChunk / 4; j++)
+                *reinterpret_cast<f32x4 *>(ws.kt + (hc * s.d_pad + d) * kChunk + 4 * j) = f32x4{k[4 * j], k[4 * j + 1], k[4 * j + 2], k[4 * j + 3]};
         }
-        ws.pc[hc * s.d_pad + d] = p;
-        float k[kChunk];
-        p = 1.0f;
-#pragma unroll
-        for (int t = kChunk - 1; t >= 0; t--) {
-            const float f = fl[t * ld + d];
-            k[t] = (1.0f - f) * p;
-            p *= f;
-        }
-#pragma unroll
-        for (uint32_t j = 0; j < kChunk / 4; j++)
-            *reinterpret_cast<f32x4 *>(ws.kt + (hc * s.d_pad + d) * kChunk + 4 * j) = f32x4{k[4 * j], k[4 * j + 1], k[4 * j + 2], k[4 * j + 3]};
     }
-    // A: thread (column s, slice of channels)
+    // A: thread (column s, every sixteenth quad of channels)
     const uint32_t col = tid & 15, slice = tid >> 4;
     float acc[kChunk];
 #pragma unroll
     for (uint32_t t = 0; t < kChunk; t++) acc[t] = 0.0f;
-    for (uint32_t d = slice; d < s.d_pad; d += 16) {
-        float w = 0.0f;
-        const float k = 1.0f - fl[col * ld + d];
+    for (uint32_t d = slice * 4; d < s.d_pad; d += 64) {
+        const f32x4 fc = *reinterpret_cast<const f32x4 *>(fl + col * ld + d);
+        f32x4 w = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (uint32_t t = 0; t < kChunk; t++) {
-            w = t == col ? k : w * fl[t * ld + d];
-            acc[t] = __builtin_fmaf(ql[t * ld + d], w, acc[t]);
+            const f32x4 f = *reinterpret_cast<const f32x4 *>(fl + t * ld + d), q = *reinterpret_cast<const f32x4 *>(ql + t * ld + d);
+#pragma unroll
+            for (uint32_t e = 0; e < 4; e++) {
+                w[e] = t == col ? 1.0f - fc[e] : w[e] * f[e];
+                acc[t] = __builtin_fmaf(q[e], w[e], acc[t]);
+            }
         }
     }
 #pragma unroll
@@ -1064,6 +1107,33 @@ __global__ __launch_bounds__(256) void recur_factors_kernel(RmiRecurShape s, Rmi
     }
     __syncthreads();
     ws.am[hc * 256 + tid] = (red[tid] + red[256 + tid]) + (red[512 + tid] + red[768 + tid]);
+}
+template <uint32_t BUCKET>
+__global__ __launch_bounds__(256) void recur_factors_kernel(RmiRecurShape s, RmiRecurArgs a, uint32_t n_chunks) {
+    __shared__ __attribute__((aligned(16))) float lds[kFactorsLds<BUCKET>];
+    recur_factors<BUCKET>(s, a, n_chunks, blockIdx.x, blockIdx.y, lds);
+}
+
+// The first launch of a pass with both mixers: neither kind of workgroup waits for the other, and of either alone a short prompt has less
+// than one a compute unit.  us, convolution and factors (with a load behind every branch) one after the other | so: 16 heads of attention,
+// 8 of recurrence, 128 tokens 6.8 + 14.6 | 7.0; 32 and 32, 2048 tokens 31 + 70 | 59.
+struct MixersPass {
+    RmiAttnShape s;
+    RmiAttnArgs a;
+    SplitPlan plan;
+    RmiRecurShape rs;
+    RmiRecurArgs ra;
+    uint32_t n_chunks, seg_chunks, recur_blocks, attn_blocks;
+};
+template <typename T>
+__global__ __launch_bounds__(256) void mixers_prepare_kernel(MixersPass p) {
+    __shared__ __attribute__((aligned(16))) float lds[kFactorsLds<128>];
+    if (blockIdx.x < p.recur_blocks) {
+        recur_factors<128>(p.rs, p.ra, p.n_chunks, blockIdx.x / p.rs.heads, blockIdx.x % p.rs.heads, lds);
+    } else {
+        const uint32_t n_heads = p.s.heads + 2 * p.s.kv_heads, b = blockIdx.x - p.recur_blocks;
+        conv_rotate_pairs<T>(p.s, p.a, b % n_heads, b / n_heads);
+    }
 }
 
 // One workgroup: sixteen value channels of one head over the chunks of one segment of the pass; wave w holds the
@@ -1077,12 +1147,14 @@ __global__ __launch_bounds__(256) void recur_factors_kernel(RmiRecurShape s, Rmi
 // side; a value past the end is taken out where it is used, not behind its load, and whole groups of chunks have no way out
 // (either made the compiler wait for every load in flight once a turn of the ring).  2048 tokens, the two launches: 47 and 118
 // us with a barrier and a branch a chunk and the value blocks of a head on eight XCDs, 45 and 104 with the head on one, 36 and 88.
+constexpr uint32_t kScanGroup = 4;  // chunks whose parts of o meet at one barrier
+typedef f32x4 ScanParts[kScanGroup][4][64];
 template <int TPW, bool STATE_ONLY, bool FULL>
-__global__ __launch_bounds__(256) void recur_scan_kernel(RmiRecurShape s, RmiRecurArgs a, uint32_t n_chunks, uint32_t seg_chunks) {
-    constexpr uint32_t kGroup = 4;  // chunks whose parts of o meet at one barrier
-    __shared__ f32x4 part[STATE_ONLY ? 1 : 2][kGroup][4][64];
+__device__ __forceinline__ void recur_scan(const RmiRecurShape &s, const RmiRecurArgs &a, uint32_t n_chunks, uint32_t seg_chunks, uint32_t head,
+                                           uint32_t v_block, uint32_t seg, ScanParts *part) {
+    constexpr uint32_t kGroup = kScanGroup;
     const uint32_t tid = threadIdx.x, lane = tid & 63, wave = uint32_t(__builtin_amdgcn_readfirstlane(int(tid >> 6))), fr = lane & 15, g = lane >> 4;
-    const uint32_t head = blockIdx.x, v0 = blockIdx.y * 16, seg = blockIdx.z, n_tiles = s.d_pad / 16;
+    const uint32_t v0 = v_block * 16, n_tiles = s.d_pad / 16;
     const uint32_t c_begin = seg * seg_chunks, c_end = c_begin + seg_chunks < n_chunks ? c_begin + seg_chunks : n_chunks;
     const RecurScratch ws = recur_scratch_at(a.scratch, s, n_chunks);
     f32x4 st[TPW], kept[TPW];
@@ -1184,6 +1256,28 @@ __global__ __launch_bounds__(256) void recur_scan_kernel(RmiRecurShape s, RmiRec
         for (int r = 0; r < 4; r++) out[size_t(tile * 16 + g * 4 + r) * s.v_pad] = st[i][r];
         if (STATE_ONLY && v0 == 0 && fr == 0)
             *reinterpret_cast<f32x4 *>(ws.seg_decay + (size_t(seg) * s.heads + head) * s.d_pad + tile * 16 + g * 4) = kept[i];
+    }
+}
+template <int TPW, bool STATE_ONLY, bool FULL>
+__global__ __launch_bounds__(256) void recur_scan_kernel(RmiRecurShape s, RmiRecurArgs a, uint32_t n_chunks, uint32_t seg_chunks) {
+    __shared__ ScanParts part[STATE_ONLY ? 1 : 2];
+    recur_scan<TPW, STATE_ONLY, FULL>(s, a, n_chunks, seg_chunks, blockIdx.x, blockIdx.y, blockIdx.z, part);
+}
+
+// The second launch of a pass with both mixers: the scans, whose chains are what takes longest, and beside them attention.  us, attention and
+// scan one after the other | so: as above, 128 tokens 9.0 + 9.2 | 10.6; 2048 tokens 124 + 40 + 94 | 216.
+template <typename T, bool SPLIT>
+__global__ __launch_bounds__(256) void mixers_pass_kernel(MixersPass p) {
+    extern __shared__ __attribute__((aligned(16))) uint8_t lds_raw[];
+    if (blockIdx.x < p.recur_blocks) {
+        const uint32_t rest = blockIdx.x / p.rs.heads, v_tiles = p.rs.v_pad / 16;
+        recur_scan<2, false, true>(p.rs, p.ra, p.n_chunks, p.seg_chunks, blockIdx.x % p.rs.heads, rest % v_tiles, rest / v_tiles,
+                                   reinterpret_cast<ScanParts *>(lds_raw));
+    } else if constexpr (SPLIT) {
+        __shared__ uint32_t flag;
+        attn_split<T, 128, false, true>(p.s, p.a, blockIdx.x - p.recur_blocks, p.plan, lds_raw, &flag);
+    } else {
+        attn_pass_block<T, 128, 2, true>(p.s, p.a, blockIdx.x - p.recur_blocks, p.attn_blocks, lds_raw);
     }
 }
 
@@ -1322,6 +1416,57 @@ int check_recur(const RmiRecurShape &s) {
     return RMI_HIP_OK;
 }
 
+// chunks of a segment: of eight or more, as many segments as still find `fill` places on a compute unit
+uint32_t segment_of(const RmiRecurShape &s, uint32_t n_chunks, uint32_t fill) {
+    const uint32_t columns = s.heads * (s.v_pad / 16);
+    uint32_t segs = (fill * uint32_t(rmi_device_cus()) + columns - 1) / columns;
+    if (segs > n_chunks / 8) segs = n_chunks / 8;
+    if (segs > kMaxSegs) segs = kMaxSegs;
+    if (segs < 1) segs = 1;
+    return (n_chunks + segs - 1) / segs;
+}
+
+template <typename T>
+void recur_norm(const RmiRecurShape &s, const RmiRecurArgs &a, uint32_t n_chunks, hipStream_t st) {
+    hipLaunchKernelGGL(recur_norm_kernel<T>, dim3((a.n_tokens + 3) / 4, s.heads), dim3(256), 0, st, s, a, n_chunks);
+}
+
+// Both mixers' several tokens, heads of 128: convolution and factors in one launch, attention and scan in one.  The scan's workgroups stay in
+// memory for the whole of theirs, so they take one place a compute unit and leave the other to attention.
+template <typename T>
+int mixers_pass(const RmiAttnShape &s, const RmiAttnArgs &a, const RmiRecurShape &rs, const RmiRecurArgs &ra, hipStream_t st) {
+    MixersPass p{s, a, {}, rs, ra};
+    const uint32_t group = s.heads / s.kv_heads, n_cols = a.n_tokens * group;
+    p.n_chunks = (ra.n_tokens + kChunk - 1) / kChunk;
+    p.recur_blocks = p.n_chunks * rs.heads;
+    const uint32_t conv_blocks = (s.heads + 2 * s.kv_heads) * ((a.pos0 % kConvRun + a.n_tokens + 4 * kConvRun - 1) / (4 * kConvRun));
+    hipLaunchKernelGGL(mixers_prepare_kernel<T>, dim3(p.recur_blocks + conv_blocks), dim3(256), 0, st, p);
+    p.seg_chunks = segment_of(rs, p.n_chunks, 1);
+    const uint32_t segs = (p.n_chunks + p.seg_chunks - 1) / p.seg_chunks, columns = rs.heads * (rs.v_pad / 16);
+    if (segs > 1)
+        hipLaunchKernelGGL((recur_scan_kernel<2, true, true>), dim3(rs.heads, rs.v_pad / 16, segs - 1), dim3(256), 0, st, rs, ra, p.n_chunks, p.seg_chunks);
+    p.recur_blocks = columns * segs;
+    const bool split = n_cols <= kSplitMaxCols;
+    size_t lds = size_t(4) * 32 * (128 + 6) * 4;
+    p.attn_blocks = (n_cols + 31) / 32 * s.kv_heads;
+    if (split) {
+        p.plan = attn_parts(s, a.n_tokens, a.pos0);
+        p.attn_blocks = s.kv_heads * p.plan.tiles.by * p.plan.parts.by;
+        lds = split_lds(sizeof(T), s, a.n_tokens);
+    }
+    if (lds < 2 * sizeof(ScanParts)) lds = 2 * sizeof(ScanParts);
+    auto go = [&](auto kernel) {
+        const int rc = rmi_allow_lds(kernel, lds);
+        if (rc == RMI_HIP_OK) hipLaunchKernelGGL(kernel, dim3(p.recur_blocks + p.attn_blocks), dim3(256), lds, st, p);
+        return rc;
+    };
+    const int rc = split ? go(mixers_pass_kernel<T, true>) : go(mixers_pass_kernel<T, false>);
+    if (rc != RMI_HIP_OK) return rc;
+    recur_norm<T>(rs, ra, p.n_chunks, st);
+    RMI_HIP_CHECK(hipGetLastError());
+    return RMI_HIP_OK;
+}
+
 template <typename T>
 int mixers_step(const RmiAttnShape *as, const RmiAttnArgs *aa, const RmiRecurShape *rs, const RmiRecurArgs *ra, const RmiAhead &ahead,
                 hipStream_t st) {
@@ -1388,16 +1533,9 @@ int rmi_recur_pass(uint32_t elem_bytes, const RmiRecurShape &s, const RmiRecurAr
     const int rc = check_recur(s);
     if (rc != RMI_HIP_OK) return rc;
     const uint32_t n_chunks = (a.n_tokens + kChunk - 1) / kChunk;
-    const size_t lds = (2 * size_t(kChunk) * (s.d_pad + 4) + 1024) * 4;
-    hipLaunchKernelGGL(recur_factors_kernel, dim3(n_chunks, s.heads), dim3(256), lds, st, s, a, n_chunks);
-    // segments of eight chunks or more, as many as still find an idle compute unit
-    const uint32_t columns = s.heads * (s.v_pad / 16);
-    uint32_t segs = (2 * uint32_t(rmi_device_cus()) + columns - 1) / columns;
-    if (segs > n_chunks / 8) segs = n_chunks / 8;
-    if (segs > kMaxSegs) segs = kMaxSegs;
-    if (segs < 1) segs = 1;
-    const uint32_t seg_chunks = (n_chunks + segs - 1) / segs;
-    segs = (n_chunks + seg_chunks - 1) / seg_chunks;
+    auto factors = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3(n_chunks, s.heads), dim3(256), 0, st, s, a, n_chunks); };
+    s.d_pad <= 64 ? factors(recur_factors_kernel<64>) : s.d_pad <= 128 ? factors(recur_factors_kernel<128>) : factors(recur_factors_kernel<256>);
+    const uint32_t seg_chunks = segment_of(s, n_chunks, 2), segs = (n_chunks + seg_chunks - 1) / seg_chunks;
     auto scan = [&](auto state_only, auto whole) {
         if (segs > 1) hipLaunchKernelGGL(state_only, dim3(s.heads, s.v_pad / 16, segs - 1), dim3(256), 0, st, s, a, n_chunks, seg_chunks);
         hipLaunchKernelGGL(whole, dim3(s.heads, s.v_pad / 16, segs), dim3(256), 0, st, s, a, n_chunks, seg_chunks);
@@ -1414,13 +1552,20 @@ int rmi_recur_pass(uint32_t elem_bytes, const RmiRecurShape &s, const RmiRecurAr
         scan(recur_scan_kernel<4, true, true>, recur_scan_kernel<4, false, true>);
     else
         scan(recur_scan_kernel<4, true, false>, recur_scan_kernel<4, false, false>);
-    const dim3 ngrid((a.n_tokens + 3) / 4, s.heads);
-    if (elem_bytes == 2)
-        hipLaunchKernelGGL(recur_norm_kernel<rmi_bf16>, ngrid, dim3(256), 0, st, s, a, n_chunks);
-    else
-        hipLaunchKernelGGL(recur_norm_kernel<float>, ngrid, dim3(256), 0, st, s, a, n_chunks);
+    elem_bytes == 2 ? recur_norm<rmi_bf16>(s, a, n_chunks, st) : recur_norm<float>(s, a, n_chunks, st);
     RMI_HIP_CHECK(hipGetLastError());
     return RMI_HIP_OK;
+}
+
+int rmi_mixers_pass(uint32_t elem_bytes, const RmiAttnShape &as, const RmiAttnArgs &aa, const RmiRecurShape &rs, const RmiRecurArgs &ra, hipStream_t st) {
+    if (aa.n_tokens == 0) return RMI_HIP_OK;
+    int rc = check_attn(as, aa);
+    if (rc == RMI_HIP_OK) rc = check_recur(rs);
+    if (rc != RMI_HIP_OK) return rc;
+    if (conv_pairs_fit(as) && as.dk_pad == 128 && as.dv_pad == 128 && rs.d_pad == 128)
+        return elem_bytes == 2 ? mixers_pass<rmi_bf16>(as, aa, rs, ra, st) : mixers_pass<float>(as, aa, rs, ra, st);
+    rc = rmi_attn_pass(elem_bytes, as, aa, st);
+    return rc == RMI_HIP_OK ? rmi_recur_pass(elem_bytes, rs, ra, st) : rc;
 }
 
 int rmi_mixers_step(uint32_t elem_bytes, const RmiAttnShape *as, const RmiAttnArgs *aa, const RmiRecurShape *rs, const RmiRecurArgs *ra,
