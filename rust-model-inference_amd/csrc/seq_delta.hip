@@ -187,8 +187,8 @@ __host__ __device__ inline size_t delta_scratch_at(float *p, const RmiDeltaShape
     const size_t wk = take(rows_k), q = take(rows_k), v = take(rows_v), o = take(rows_v);
     const size_t kt = take(size_t(s.kv_heads) * n_chunks * kChunk * s.d_pad), dk = take(hc * 2 * kChunk);
     if (w) {
-        w->w = p + wk;   // [head][chunk][16][d_pad]
-        w->q = p + q;    // [head][chunk][16][d_pad]
+        w->w = p + wk;   // [head][chunk][d_pad / 16][16 t][16 d]: what a wave reads at a time lies in one piece
+        w->q = p + q;    // the same
         w->v = p + v;    // [head][chunk][v_pad][16]: T v
         w->o = p + o;    // [head][chunk][16][v_pad]: M T v, then o
         w->kt = p + kt;  // [kv_head][chunk][d_pad][16]
@@ -347,7 +347,7 @@ __global__ __launch_bounds__(kFactorThreads) void delta_factors_kernel(RmiDeltaS
             const f32x4 gk = quad(kt + (i * 16 + fr) * kTl + q4 * 4) * gt;
             const f32x4 w = mma16_f32(tr, gk, zero), wt = mma16_f32(gk, tr, zero), mw = mma16_f32(w, mr, zero);
             const uint32_t c = i * 16 + q4 * 4;
-            const size_t to = (hc * kChunk + fr) * s.d_pad + c;
+            const size_t to = ((hc * k_tiles + i) * kChunk + fr) * 16 + q4 * 4;
             *reinterpret_cast<f32x4 *>(ws.w + to) = wt;
             *reinterpret_cast<f32x4 *>(ws.q + to) = quad(ql + fr * ld + c) * gl[fr] - mw;
         } else {
@@ -386,7 +386,7 @@ __global__ __launch_bounds__(256) void delta_scan_kernel(RmiDeltaShape s, RmiDel
     const float *pd = ws.dk + size_t(h) * n_pad * 2 * kChunk;
     float *po = ws.o + size_t(h) * n_pad * kChunk * s.v_pad;
     const size_t step_k = size_t(kChunk) * s.d_pad, step_v = size_t(kChunk) * s.v_pad;  // floats
-    uint32_t off_w[TPW], off_k[TPW];
+    uint32_t off_k[TPW];
     bool has[TPW];
     f32x4 st[TPW];
     const size_t at = size_t(h) * s.d_pad * s.v_pad + v0 + fr;
@@ -394,7 +394,6 @@ __global__ __launch_bounds__(256) void delta_scan_kernel(RmiDeltaShape s, RmiDel
     for (int i = 0; i < TPW; i++) {
         has[i] = FULL || wave + 4 * i < n_tiles;
         const uint32_t tile = has[i] ? wave + 4 * i : n_tiles - 1;
-        off_w[i] = (fr * s.d_pad + tile * 16 + g4 * 4) * 4;
         off_k[i] = ((tile * 16 + fr) * kChunk + g4 * 4) * 4;
         st[i] = f32x4{0.f, 0.f, 0.f, 0.f};
         if (a.pos0 == 0 || !has[i]) continue;
@@ -411,12 +410,12 @@ __global__ __launch_bounds__(256) void delta_scan_kernel(RmiDeltaShape s, RmiDel
         Operands x;
         const uint32_t c = chunk < n_pad ? chunk : n_pad - 1;
 #pragma unroll
-        for (int i = 0; i < TPW; i++) x.w[i] = quad_at(pw + c * step_k, off_w[i]);
+        for (int i = 0; i < TPW; i++) x.w[i] = quad_at(pw + c * step_k, off_k[i]);
         x.v = quad_at(pv + c * step_v, off_v);
         x.d = quad_at(pd + size_t(c) * 2 * kChunk, off_d);
         x.keep = pd[size_t(c) * 2 * kChunk + kChunk];
 #pragma unroll
-        for (int i = 0; i < TPW; i++) x.q[i] = quad_at(pq + c * step_k, off_w[i]);
+        for (int i = 0; i < TPW; i++) x.q[i] = quad_at(pq + c * step_k, off_k[i]);
 #pragma unroll
         for (int i = 0; i < TPW; i++) x.kt[i] = quad_at(pk + c * step_k, off_k[i]);
         return x;
