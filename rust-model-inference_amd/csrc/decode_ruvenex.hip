@@ -51,6 +51,9 @@ struct RuvenexSession : rmi_hip_folder_session {
     }
     bool prepare_walk();
     bool walk_gave_up() override;
+    bool walk_embeds(uint32_t step0, const float *host_layers) const override {
+        return walks && walk.words && !host_layers && step0 > 0 && step0 < kWalkRvMaxKeys;
+    }
     void back_one() override {
         position--;
         now ^= 1;
@@ -71,7 +74,7 @@ struct RuvenexSession : rmi_hip_folder_session {
 
 int RuvenexSession::enqueue_layers(uint32_t step0, uint32_t n, hipStream_t st, float *host_layers) {
     int rc = RMI_HIP_OK;
-    if (n == 1 && walks && walk.words && !host_layers && step0 > 0 && step0 < kWalkRvMaxKeys) {
+    if (n == 1 && walk_embeds(step0, host_layers)) {
         if (walk.tag0 > 0xffffffffu - n_runs - 1) {  // the words' tags start anew
             RMI_HIP_CHECK(hipMemsetAsync(walk.words, 0, walk_words * 8, st));
             walk.tag0 = 0;
@@ -80,6 +83,7 @@ int RuvenexSession::enqueue_layers(uint32_t step0, uint32_t n, hipStream_t st, f
         a.x = x;
         a.pos = step0;
         a.now = uint32_t(now);
+        give_token(&a, step0);
         if (walk_spins) a.spins = walk_spins;
         walk.tag0 += n_runs + 1;
         rc = rmi_launch_walk_ruvenex(a, st);

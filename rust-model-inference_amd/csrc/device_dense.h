@@ -165,6 +165,18 @@ __device__ __forceinline__ float2 sin_cos_turns(double r) {
     return make_float2(q & 2 ? -a : a, (q + 1) & 2 ? -b : b);
 }
 
+// what embed_row leaves in a column, the same bits
+template <typename T>
+__device__ __forceinline__ float embed_value(const RmiEmbed &e, uint32_t token, uint32_t p, uint32_t col) {
+    if (token >= e.vocab) token = e.vocab - 1;
+    float v = to_f32(static_cast<const T *>(e.table)[size_t(token) * e.ld + col]) * e.scale;
+    if (e.turns) {
+        const double r = double(p) * e.turns[col / 2];
+        const float2 sc = sin_cos_turns(r - rint(r));
+        v += col & 1 ? sc.y : sc.x;
+    }
+    return v;
+}
 // A workgroup of 256: row t of the stream, a token's embedding at position p.  A thread takes pairs of channels, eight at
 // a time, all their loads under way together.
 template <typename T>

@@ -27,6 +27,7 @@ struct rmi_hip_folder_session : RmiSession {
     uint32_t *want_rows = nullptr;
     uint32_t position = 0;    // tokens of the current sequence so far
     uint32_t embedded = ~0u;  // the position whose embedding the last sampling launch left in x
+    const uint32_t *lone = nullptr;  // a token by itself that the host knows and no launch has embedded yet
     bool walks = true;        // a token's layers may go through one launch, where the design has it
     uint32_t walk_spins = 0;  // how often a wait inside such a launch asks; 0: as often as the design has it
 
@@ -35,6 +36,8 @@ struct rmi_hip_folder_session : RmiSession {
     // The layers over positions step0 .. step0 + n - 1, whose embeddings are in x.  host_layers: the residual stream
     // behind every layer run, [run][n][width] (synchronises; for comparisons).
     virtual int enqueue_layers(uint32_t step0, uint32_t n, hipStream_t st, float *host_layers) = 0;
+    // Whether enqueue_layers of the token at `step0` takes it from `lone`.
+    virtual bool walk_embeds(uint32_t step0, const float *host_layers) const { return false; }
     // The sequence as it was before its last token, which was the last call's only one.
     virtual void back_one() { position--; }
     // What the head reads of the stream behind the last layer (x_out is not used).
@@ -56,11 +59,18 @@ struct rmi_hip_folder_session : RmiSession {
     bool load_common(struct RmiFolderReader &rd);
     bool alloc_common(uint32_t max_k);
     float *upload_vector(const RmiTensor *t);
+    RmiEmbed embed_to() const;
+    // a walk's arguments for the token, where it is a lone one
+    template <typename Args>
+    void give_token(Args *a, uint32_t step0) const {
+        a->embed = lone ? embed_to() : RmiEmbed{};
+        a->token = lone ? *lone : 0;
+        a->tok_out = tok + step0;
+    }
     int copy_layer(float *host_layers, uint32_t run, uint32_t n, hipStream_t st);
 
   private:
     int feed_passes(const uint32_t *tokens, uint32_t n, const uint32_t *want, uint32_t n_want, float *out, float *host_layers, hipStream_t st);
-    RmiEmbed embed_to() const;
     int embed_tokens(uint32_t step0, uint32_t n, hipStream_t st);
     int enqueue_logits(const uint32_t *rows, uint32_t n_rows, hipStream_t st);
     int enqueue_sample(uint32_t step0, const uint32_t *rows, uint32_t n_rows, uint32_t last, hipStream_t st);

@@ -137,8 +137,10 @@ int rmi_hip_folder_session::feed_passes(const uint32_t *tokens, uint32_t n, cons
     const uint32_t most = prompt_pass ? (prompt_pass < pass_rows ? prompt_pass : pass_rows) : 1;
     for (uint32_t at = 0; at < n;) {
         const uint32_t m = n - at < most ? n - at : most;
-        int rc = n == 1 ? rmi_dense_embed_token(elem, embed_to(), tokens[0], tok + step0, step0, st) : embed_tokens(step0 + at, m, st);
+        lone = n == 1 && walk_embeds(step0, host_layers) ? tokens : nullptr;
+        int rc = lone ? RMI_HIP_OK : n == 1 ? rmi_dense_embed_token(elem, embed_to(), tokens[0], tok + step0, step0, st) : embed_tokens(step0 + at, m, st);
         if (rc == RMI_HIP_OK) rc = enqueue_layers(step0 + at, m, st, host_layers);
+        lone = nullptr;
         if (rc != RMI_HIP_OK) return rc;
         std::vector<uint32_t> rows, slots;  // this pass's rows, and where their logits go
         for (uint32_t i = 0; i < n_want; i++)

@@ -39,6 +39,9 @@ struct RmiWalkRvArgs {
     uint64_t *words;   // zeros at first
     uint32_t *failed;  // set where a wait did not end; the host's memory
     uint32_t tag0, spins, pos, now;
+    RmiEmbed embed;    // with a table: the token is `token`, which the walk embeds itself and leaves in tok_out; else its embedding is in x
+    uint32_t token;
+    uint32_t *tok_out;
     uint32_t n_output;  // workgroups of everything that ends in x
 };
 

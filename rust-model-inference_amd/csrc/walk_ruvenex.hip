@@ -67,6 +67,11 @@ struct RvLds {  // (arrays that are read by pieces of 16 bytes lie at such: a pi
     alignas(16) float o[T / 32][kDim];
 };
 
+// the token's embedding: a launch of its own in front of a cooperative one is 14 us of a token of 411
+__device__ __forceinline__ float embedded(const RmiWalkRvArgs &a, uint32_t col) {
+    return a.embed.table ? embed_value<rmi_bf16>(a.embed, a.token, a.pos, col) : a.x[col];
+}
+
 struct RvCtx {
     const RmiWalkRvArgs &a;
     RvWords at;
@@ -379,7 +384,7 @@ __device__ __forceinline__ void walk_input(const RvCtx &c, uint32_t idx, RvLds &
         float x[kX], sq = 0.0f;
         if (l == 0) {
 #pragma unroll
-            for (uint32_t j = 0; j < kX; j++) x[j] = tid + j * T < s.width ? a.x[tid + j * T] : 0.0f;
+            for (uint32_t j = 0; j < kX; j++) x[j] = tid + j * T < s.width ? embedded(a, tid + j * T) : 0.0f;
         } else {
             gptr_word from[kX];
             uint32_t w[kX];
@@ -437,7 +442,7 @@ __device__ __forceinline__ void walk_output(const RvCtx &c, uint32_t idx, RvLds 
     const float part_scale = part_of == 0 ? s.left_scale : part_of == 1 ? s.right_scale : 1.0f;
     const bool has = tid < pieces;
     const uint32_t my_row = out0 + (lane & 15);  // of lanes whose lane & 15 is below kOutRows
-    float x_own = a.x[my_row < s.width ? my_row : s.width - 1];
+    float x_own = embedded(a, my_row < s.width ? my_row : s.width - 1);
     load(0);
     // words of act to LDS
     auto stage = [&](uint32_t first, uint32_t n, uint32_t tag) {
@@ -516,6 +521,7 @@ __global__ __launch_bounds__(T) void ruvenex_walk_kernel(RmiWalkRvArgs a) {
     gptr_word words = as_global<gptr_word>(a.words);
     const RvCtx c{a, at, words, words + die_half() * at.n, WalkBound{a.failed, a.spins}};
     if (threadIdx.x == 0) sm.bad = 0;
+    if (a.embed.table && blockIdx.x == 0 && threadIdx.x == 0) *a.tok_out = a.token;
     __syncthreads();
     const uint32_t b = blockIdx.x, n_mix = s.heads + s.recur_heads;
     if (b < n_mix) {

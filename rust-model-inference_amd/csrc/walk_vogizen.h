@@ -48,6 +48,9 @@ struct RmiWalkVgArgs {
     uint64_t *words;        // zeros at first
     uint32_t *failed;       // set where a wait did not end; the host's memory
     uint32_t tag0, spins, pos, now;
+    RmiEmbed embed;    // with a table: the token is `token`, which the walk embeds itself and leaves in tok_out; else its embedding is in x
+    uint32_t token;
+    uint32_t *tok_out;
 };
 
 constexpr uint32_t kWalkVgKeys = 1024;  // most that a position sees, itself included

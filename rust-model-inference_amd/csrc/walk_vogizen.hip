@@ -253,10 +253,15 @@ __device__ __forceinline__ void vg_stream(const VgCtx &c, uint32_t idx, VgLds<El
         };
         auto in_base = [&](uint32_t i) { return as_global<gptr_u4>(y.w_in) + size_t(row0 + i * kWaves) * (s.ld_w / kPieceE); };
         float x[KX], wn[KX], yw[KX];
+        auto embedded = [&](const float *from, float (&v)[KX]) {  // by a launch in front, or here: without that launch a token is 14 us faster
+            if (!a.embed.table) return vec(from, v);
+#pragma unroll
+            for (uint32_t j = 0; j < KX; j++) v[j] = embed_value<El>(a.embed, a.token, a.pos, tid + j * T);
+        };
         // ---- the stream behind the run before
         auto stream_in = [&] {
             if (run == 0) {
-                vec(a.x, x);
+                embedded(a.x, x);
                 return;
             }
             uint32_t v[2 * KX], yv[KX];
@@ -283,7 +288,7 @@ __device__ __forceinline__ void vg_stream(const VgCtx &c, uint32_t idx, VgLds<El
             };
             float e[KX];
             if (run) vec(y.side_before, yw);
-            vec(a.embedded, e);
+            embedded(a.embedded, e);
             first(Three{}, n, base);
             stream_in();
 #pragma unroll
@@ -733,7 +738,7 @@ __device__ __forceinline__ void vg_chain(const VgCtx &c, uint32_t b, VgLds<El, W
             for (uint32_t p = 0; p < K::NPO; p++)
                 wo[i][p] = __builtin_nontemporal_load(as_global<gptr_u4>(w) + size_t(row0 + i) * (s.ld_v / kPieceE) + p * 64 + (t & 63));
     };
-    const uint32_t id = a.tok[a.pos] < s.vocab ? a.tok[a.pos] : s.vocab - 1;
+    const uint32_t token = a.embed.table ? a.token : a.tok[a.pos], id = token < s.vocab ? token : s.vocab - 1;
     for (uint32_t run = 0; run < s.n_run; run++) {
         const RmiWalkVgRun::Chain y = table_entry(&a.runs[run].chain);
         uint32_t tid = threadIdx.x;
@@ -746,7 +751,7 @@ __device__ __forceinline__ void vg_chain(const VgCtx &c, uint32_t b, VgLds<El, W
         const float scale = as_global<gptr_f32>(y.ls1)[own0 + wave * K::kOwnUnits + (half < K::kOwnUnits ? half : 0)];
         // ---- own rows of the stream in front of the mixer
         if (run == 0 && !(flags & RmiWalkVgRun::kLoopBegins)) {
-            if (tid < K::kOwn) m.own[tid] = a.x[own0 + tid];
+            if (tid < K::kOwn) m.own[tid] = a.embed.table ? embed_value<El>(a.embed, a.token, a.pos, own0 + tid) : a.x[own0 + tid];
         } else if (flags & RmiWalkVgRun::kLoopBegins) {
             if (tid < 64) {
                 const gptr_word at[1] = {from + c.at.xl + own0 + (tid < K::kOwn ? tid : 0)};
@@ -887,6 +892,7 @@ __global__ __launch_bounds__(T) void vogizen_walk_kernel(RmiWalkVgArgs a) {
     gptr_word words = as_global<gptr_word>(a.words);
     const VgCtx c{a, at, words, words + die_half() * 2 * at.n, WalkBound{a.failed, a.spins}};
     if (threadIdx.x == 0) sm.bad = 0;
+    if (a.embed.table && blockIdx.x == 0 && threadIdx.x == 0) *a.tok_out = a.token;
     __syncthreads();
     if (blockIdx.x < kChain)
         vg_chain<El, W>(c, blockIdx.x, sm, staged);
