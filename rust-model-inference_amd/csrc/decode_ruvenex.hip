@@ -84,6 +84,11 @@ int RuvenexSession::enqueue_layers(uint32_t step0, uint32_t n, hipStream_t st, f
         a.pos = step0;
         a.now = uint32_t(now);
         give_token(&a, step0);
+        a.head = want_logits ? head.data : nullptr;
+        a.head_norm = final_norm;
+        a.logits = logits;
+        a.vocab = vocab;
+        logits_there = want_logits;
         if (walk_spins) a.spins = walk_spins;
         walk.tag0 += n_runs + 1;
         rc = rmi_launch_walk_ruvenex(a, st);

@@ -28,6 +28,8 @@ struct rmi_hip_folder_session : RmiSession {
     uint32_t position = 0;    // tokens of the current sequence so far
     uint32_t embedded = ~0u;  // the position whose embedding the last sampling launch left in x
     const uint32_t *lone = nullptr;  // a token by itself that the host knows and no launch has embedded yet
+    bool want_logits = false;  // of the one token that enqueue_layers is asked for; logits_there: they are behind it, by the same launch
+    bool logits_there = false;
     bool walks = true;        // a token's layers may go through one launch, where the design has it
     uint32_t walk_spins = 0;  // how often a wait inside such a launch asks; 0: as often as the design has it
 

@@ -46,6 +46,10 @@ int rmi_hip_folder_session::enqueue_logits(const uint32_t *rows, uint32_t n_rows
     s.s[0].n = s.s[0].ld = vocab;
     s.s[0].act = kActNone;
     rmi_row_segs_done(&s);
+    if (logits_there && n_rows == 1 && !rows) {
+        logits_there = false;
+        return RMI_HIP_OK;
+    }
     const RmiInput in = head_input();
     if (n_rows == 1 && !rows && rmi_dense_gemv_fits(elem, k_in)) return rmi_dense_gemv(elem, head, in, s, st);
     const int rc = rmi_dense_input(elem, in, rows, h, n_rows, k_in, st);
@@ -76,7 +80,10 @@ int rmi_hip_folder_session::set_rows(const uint32_t *want, uint32_t n_want, hipS
 
 int rmi_hip_folder_session::enqueue_step(uint32_t step, hipStream_t st) {
     int rc = embedded == step ? RMI_HIP_OK : embed_tokens(step, 1, st);
+    want_logits = true;
+    logits_there = false;
     if (rc == RMI_HIP_OK) rc = enqueue_layers(step, 1, st, nullptr);
+    want_logits = false;
     if (rc == RMI_HIP_OK) rc = enqueue_logits(nullptr, 1, st);
     if (rc == RMI_HIP_OK) rc = enqueue_sample(step, nullptr, 1, 0, st);
     embedded = step + 1;
@@ -139,8 +146,11 @@ int rmi_hip_folder_session::feed_passes(const uint32_t *tokens, uint32_t n, cons
         const uint32_t m = n - at < most ? n - at : most;
         lone = n == 1 && walk_embeds(step0, host_layers) ? tokens : nullptr;
         int rc = lone ? RMI_HIP_OK : n == 1 ? rmi_dense_embed_token(elem, embed_to(), tokens[0], tok + step0, step0, st) : embed_tokens(step0 + at, m, st);
+        want_logits = n == 1 && n_want > 0;
+        logits_there = false;
         if (rc == RMI_HIP_OK) rc = enqueue_layers(step0 + at, m, st, host_layers);
         lone = nullptr;
+        want_logits = false;
         if (rc != RMI_HIP_OK) return rc;
         std::vector<uint32_t> rows, slots;  // this pass's rows, and where their logits go
         for (uint32_t i = 0; i < n_want; i++)

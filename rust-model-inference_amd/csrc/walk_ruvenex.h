@@ -42,6 +42,10 @@ struct RmiWalkRvArgs {
     RmiEmbed embed;    // with a table: the token is `token`, which the walk embeds itself and leaves in tok_out; else its embedding is in x
     uint32_t token;
     uint32_t *tok_out;
+    const void *head;  // the vocabulary's rows, in_ld apart, or nullptr: no logits
+    const float *head_norm;
+    float *logits;
+    uint32_t vocab;
     uint32_t n_output;  // workgroups of everything that ends in x
 };
 

@@ -502,13 +502,75 @@ __device__ __forceinline__ void walk_output(const RvCtx &c, uint32_t idx, RvLds 
 #pragma unroll
             for (uint32_t w = 0; w < T / 64; w++) z += sm.part[w][(lane & 15) < kOutRows ? lane & 15 : 0];
             x_own += z;
-            if (lane < 32 && (lane & 15) < kOutRows && my_row < s.width && l + 1 < s.n_layer)
+            if (lane < 32 && (lane & 15) < kOutRows && my_row < s.width && (l + 1 < s.n_layer || a.head))
                 word_store(c.words + (lane >> 4) * c.at.n + (l & 1 ? c.at.x[0] : c.at.x[1]) + my_row, __float_as_uint(x_own), tag + 1);
         }
         __syncthreads();  // (x first, too)
         if (l + 1 < s.n_layer) load(l + 1);
     }
     if (tid < kOutRows && my_row < s.width) a.x[my_row] = x_own;
+}
+
+// ---- the vocabulary: every workgroup, eight rows a wave at a time.  A launch behind a cooperative one begins 11 us after it; here the first
+// rows are asked for in front of the last layer's vector, and a row's place in the registers takes the next one as soon as it is multiplied.
+template <uint32_t NQ>
+__device__ __forceinline__ void walk_head(const RvCtx &c, RvLds &sm, u32x4 *h) {
+    const RmiWalkRvArgs &a = c.a;
+    const RmiWalkRvShape &s = a.s;
+    constexpr uint32_t kRows = 8, kX = NQ * 512 / T;
+    const uint32_t tid = threadIdx.x, lane = tid & 63, wave = uint32_t(__builtin_amdgcn_readfirstlane(int(tid >> 6)));
+    const uint32_t units = (a.vocab + kRows - 1) / kRows, step = gridDim.x * (T / 64);
+    uint32_t unit = blockIdx.x * (T / 64) + wave;
+    const gptr_u4 rows = as_global<gptr_u4>(a.head) + lane;
+    u32x4 w[kRows][NQ];
+    auto load = [&](uint32_t u, uint32_t r) {  // (rows are padded to sixteen)
+        const gptr_u4 at = rows + size_t((u < units ? u : units - 1) * kRows + r) * (s.in_ld / 8);
+#pragma unroll
+        for (uint32_t q = 0; q < NQ; q++) w[r][q] = __builtin_nontemporal_load(at + q * 64);
+    };
+#pragma unroll
+    for (uint32_t r = 0; r < kRows; r++) load(unit, r);
+    float x[kX], wn[kX], sq = 0.0f;
+    gptr_word from[kX];
+    uint32_t v[kX];
+#pragma unroll
+    for (uint32_t j = 0; j < kX; j++) {
+        wn[j] = as_global<gptr_f32>(a.head_norm)[tid + j * T];
+        from[j] = c.mine + (s.n_layer & 1 ? c.at.x[1] : c.at.x[0]) + tid + j * T;
+    }
+    if (!words_wait<kX>(from, a.tag0 + 1 + s.n_layer, v, c.bound)) sm.bad = 1;
+#pragma unroll
+    for (uint32_t j = 0; j < kX; j++) {
+        x[j] = __uint_as_float(v[j]);
+        sq = __builtin_fmaf(x[j], x[j], sq);
+    }
+    sq = wave_sum_f32(sq);
+    if (lane == 0) sm.red[wave] = sq;
+    __syncthreads();
+    if (sm.bad) return;
+    float total = 0.0f;
+#pragma unroll
+    for (uint32_t i = 0; i < T / 64; i++) total += sm.red[i];
+    const float scale = 1.0f / sqrtf(total / float(s.width) + s.eps);
+#pragma unroll
+    for (uint32_t j = 0; j < kX; j++) reinterpret_cast<rmi_bf16 *>(h)[tid + j * T] = f32_to_bf16(x[j] * scale * wn[j]);
+    __syncthreads();
+    u32x4 hv[NQ];
+#pragma unroll
+    for (uint32_t q = 0; q < NQ; q++) hv[q] = h[q * 64 + lane];
+    for (; unit < units; unit += step) {
+        float acc[kRows];
+#pragma unroll
+        for (uint32_t r = 0; r < kRows; r++) {
+            acc[r] = 0.0f;
+#pragma unroll
+            for (uint32_t q = 0; q < NQ; q++) acc[r] = dot_piece<rmi_bf16>(w[r][q], hv[q], acc[r]);
+            load(unit + step, r);
+        }
+        const float sum = sums8(acc);
+        const uint32_t row = unit * kRows + eighth(lane);
+        if ((lane & 15) < 2 && row < a.vocab) a.logits[row] = sum;
+    }
 }
 
 // NQ pieces of a row of the width a lane
@@ -536,6 +598,12 @@ __global__ __launch_bounds__(T) void ruvenex_walk_kernel(RmiWalkRvArgs a) {
         walk_output(c, b - n_mix, sm, staged);
     } else {
         walk_input<NQ>(c, b - n_mix - a.n_output, sm, staged);
+    }
+    if (a.head) {
+        __syncthreads();
+        const bool bad = sm.bad != 0;
+        __syncthreads();  // (nobody gives up a wait before everybody has read it)
+        if (!bad) walk_head<NQ>(c, sm, staged);
     }
 }
 
