@@ -1211,6 +1211,7 @@ struct rmi_hip_qwen3 : RmiSession {
     RmiWalkShape walk_shape{};
     size_t walk_words = 0;
     bool walk_off = false;               // a wait of a walk was given up once
+    bool walked = false;                 // there was a walk since the last look at its waits, which is a copy of 20 us
 
     ~rmi_hip_qwen3() override;
     int enqueue_step(uint32_t step, hipStream_t st) override;
@@ -1461,11 +1462,14 @@ int rmi_hip_qwen3::enqueue_walk(uint32_t step, uint32_t n, uint32_t n_prompt, bo
     a.n_prompt = n_prompt;
     a.keep_logits = keep_logits;
     walk.tag0 += tags;
+    walked = true;
     return rmi_launch_walk_qwen3(walk_shape, a, st);
 }
 bool rmi_hip_qwen3::walk_gave_up() {
     uint32_t failed = 0;
-    if (!walk.words || walk_off || hipMemcpy(&failed, walk.failed, 4, hipMemcpyDeviceToHost) != hipSuccess) return false;
+    if (!walked) return false;
+    walked = false;
+    if (walk_off || hipMemcpy(&failed, walk.failed, 4, hipMemcpyDeviceToHost) != hipSuccess) return false;
     walk_off = failed != 0;
     return walk_off;
 }
