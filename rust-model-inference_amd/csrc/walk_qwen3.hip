@@ -80,7 +80,8 @@ struct WalkLds {  // of every role
     double red[8];
     float gu[64];
     Top top[64];
-    uint32_t bad, token;
+    Top all_top[8];  // by wave, of all workgroups: not in `top`, which wave 0 may still be reading when another wave has its words
+    uint32_t bad;
     alignas(16) uint16_t new16[3][128];  // (read by pieces of 16 bytes)
     uint64_t exp_tab[32];
     float max8[8];
@@ -630,12 +631,12 @@ __global__ __launch_bounds__(kWalkThreads) void qwen3_walk_kernel(RmiWalkArgs a)
                                 uint32_t(__shfl_xor(int(m.finite), s))};
                 m = top_merge(m, other);
             }
-            if (lane == 0) sm.top[wave] = m;
+            if (lane == 0) sm.all_top[wave] = m;
             __syncthreads();
             if (sm.bad) return;
-            m = sm.top[0];
+            m = sm.all_top[0];
 #pragma unroll
-            for (int s = 1; s < int(kWalkThreads / 64); s++) m = top_merge(m, sm.top[s]);
+            for (int s = 1; s < int(kWalkThreads / 64); s++) m = top_merge(m, sm.all_top[s]);
             uint32_t token = step + 1 >= a.n_prompt ? m.id : told;
             if (idx == 0 && tid == 0) {
                 a.step_argmax[step] = m.id;

@@ -76,6 +76,26 @@ def test_a_wait_that_is_given_up_leaves_the_single_launches(hip, tmp_path):
     s.close()
 
 
+def test_largest_logits_of_every_wave(hip, tmp_path):
+    """A tile of eight rows a wave (256 workgroups of eight), so the two largest logits lie in all roles' workgroups and in all of their waves.  A
+    workgroup that merges all workgroups' largest logits keeps them apart from its own waves': those may not have been read yet."""
+    meta, tensors = _model(hip, tmp_path, vocab=16384, n_layer=1)
+    s = hip.decode.Qwen3Session(meta, tensors, 900)
+    rng = np.random.default_rng(4)
+    rows = []
+    for n in (5, 300):
+        prompt = rng.integers(0, s.vocab, n, dtype=np.uint32)
+        s.set_prompt_passes(0)  # every position of the prompt by a walk, too: other tokens than the model's own
+        s.set_walks(1)
+        walked = s.generate(prompt, 300, [n + 298])
+        s.set_walks(0)
+        _equal(walked, s.generate(prompt, 300, [n + 298]), n)
+        rows.append(walked["argmax"])
+    wave = np.concatenate(rows) // 8
+    assert set(wave % 8) == set(range(8)) and ((wave // 8 >= 64) & (wave // 8 < 128)).any()
+    s.close()
+
+
 def test_two_sessions_walk_on_two_threads(hip, tmp_path):
     meta, tensors = _model(hip, tmp_path)
     prompts = [np.random.default_rng(k).integers(0, 3000, 30 + 200 * k, dtype=np.uint32) for k in range(2)]
