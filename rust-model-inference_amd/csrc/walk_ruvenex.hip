@@ -618,6 +618,9 @@ Roles roles_of(const RmiWalkRvShape &s) {
 }  // namespace
 
 bool rmi_walk_ruvenex_fits(const RmiWalkRvShape &s) {
+    // The embedding lies where the last layer's x goes.  With a layer between, whose x all of the last one depends on, everybody has read it by
+    // then; with one layer an input workgroup that makes other rows' gates only may not have.
+    if (s.n_layer < 2) return false;
     if (s.k_in != 1024 || s.width != s.k_in || s.k_pad / 8 > T || roles_of(s).all() > uint32_t(rmi_device_cus())) return false;
     if (s.k_attn != s.heads * kDim || s.k_recur - s.k_attn != s.recur_heads * kDim || s.taps > 4 || s.taps < 2 || s.heads % s.kv_heads) return false;
     if (s.seg[kSegs] - s.seg[kSegUp] != s.k_pad - s.k_recur) return false;

@@ -64,6 +64,22 @@ def test_shapes_the_walk_does_not_take(open_model):
         assert rel(got, P.forward(cfg, w, t)) < TOL[BF16], kw
 
 
+def test_one_layer_goes_by_single_launches(open_model):
+    """Its walk would write the stream where workgroups that have not started yet read the embedding."""
+    cfg = model(**SHAPES[0], n_layer=1)
+    s, w = open_model(cfg, None, BF16, 80)
+    t = G.tokens(cfg, 60)
+    assert rel(feed(s, t, [40, 1]), P.forward(cfg, w, t)) < TOL[BF16]
+    got = []
+    for on in (1, 0):
+        s.set_walks(on)
+        s.reset()
+        got.append((feed(s, t, [40, 1]), s.generate(t[:40], 30, [39, 50, 68])))
+    assert np.array_equal(got[0][0], got[1][0])
+    for k in ("tokens", "argmax", "dump"):
+        assert np.array_equal(got[0][1][k], got[1][1][k]), k
+
+
 def test_a_wait_that_is_given_up_leaves_the_single_launches(open_model):
     cfg = model(**SHAPES[0])
     s, _ = open_model(cfg, None, BF16, 120)
