@@ -155,7 +155,7 @@ bool RuvenexSession::walk_gave_up() {
 
 // The walk's tables, where every layer is of one shape that it takes; false + error text only if memory is missing.
 bool RuvenexSession::prepare_walk() {
-    if (elem != 2) return true;
+    if (elem != 2 || layers.empty()) return true;
     const RuvenexLayer &y0 = layers[0];
     const RmiAttnShape &a = y0.attn;
     const RmiRecurShape &r = y0.recur;

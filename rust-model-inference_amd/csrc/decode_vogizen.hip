@@ -302,7 +302,7 @@ bool VogizenSession::walk_gave_up() {
 
 // The walk's tables, where all layers of a kind are of one shape that it takes; false + error text only if memory is missing.
 bool VogizenSession::prepare_walk() {
-    if (!one_token_gemv || k_in != width) return true;
+    if (!one_token_gemv || k_in != width || runs.empty()) return true;
     const VogizenLayer *d0 = nullptr, *a0 = nullptr;
     constexpr uint32_t kDeltaSegs = 6, kDim = 128, kHeads = 16;
     for (const VogizenLayer &l : layers) {

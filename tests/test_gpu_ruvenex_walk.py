@@ -7,7 +7,7 @@ import numpy as np
 import pytest
 import ruvenex_gen as G
 import ruvenex_plain as P
-from folder_helpers import BF16, TOL, Opener, feed, rel
+from folder_helpers import BF16, F32, TOL, Opener, feed, rel
 
 pytestmark = pytest.mark.gpu
 
@@ -78,6 +78,14 @@ def test_one_layer_goes_by_single_launches(open_model):
     assert np.array_equal(got[0][0], got[1][0])
     for k in ("tokens", "argmax", "dump"):
         assert np.array_equal(got[0][1][k], got[1][1][k]), k
+
+
+def test_no_layers(open_model):
+    cfg = G.config([], 1024, 90)
+    for dtype in (BF16, F32):
+        s, w = open_model(cfg, None, dtype, 20)
+        t = G.tokens(cfg, 9)
+        assert rel(feed(s, t, [4, 1]), P.forward(cfg, w, t)) < TOL[dtype]
 
 
 def test_a_wait_that_is_given_up_leaves_the_single_launches(open_model):

@@ -78,6 +78,14 @@ def test_shapes_the_walk_does_not_take(open_model):
 
 
 @pytest.mark.parametrize("dtype", [F32, BF16])
+def test_no_layers(open_model, dtype):
+    cfg = G.config([], 1024, 90, loop=None)
+    s, w = open_model(cfg, None, dtype, 20)
+    t = G.tokens(cfg, 9)
+    assert rel(feed(s, t, [4, 1]), P.forward(cfg, w, t)) < TOL[dtype]
+
+
+@pytest.mark.parametrize("dtype", [F32, BF16])
 def test_a_wait_that_is_given_up_leaves_the_single_launches(open_model, dtype):
     cfg = model(1024, "da", loop=(0, 2, 2))
     s, _ = open_model(cfg, None, dtype, 120)
