@@ -1469,8 +1469,7 @@ bool rmi_hip_qwen3::walk_gave_up() {
     uint32_t failed = 0;
     if (!walked) return false;
     walked = false;
-    if (walk_off || hipMemcpy(&failed, walk.failed, 4, hipMemcpyDeviceToHost) != hipSuccess) return false;
-    walk_off = failed != 0;
+    walk_off = walk_off || hipMemcpy(&failed, walk.failed, 4, hipMemcpyDeviceToHost) != hipSuccess || failed != 0;  // (not known is not finished)
     return walk_off;
 }
 rmi_hip_qwen3::~rmi_hip_qwen3() {
@@ -1849,7 +1848,8 @@ int rmi_hip_qwen3_set_walks(rmi_hip_qwen3 *s, int enabled) {
     if (!s) return rmi_fail(RMI_HIP_E_INVALID, "null session");
     s->walk_off = enabled <= 0;
     s->walk.spins = enabled > 1 ? uint32_t(enabled) : kWalkSpins;
-    if (enabled > 0 && s->walk.words) RMI_HIP_CHECK(hipMemset(s->walk.failed, 0, 4));
+    const uint32_t none = 0;  // (a copy has arrived when it returns, a fill may still be on its way when the next walk has given up)
+    if (enabled > 0 && s->walk.words) RMI_HIP_CHECK(hipMemcpy(s->walk.failed, &none, 4, hipMemcpyHostToDevice));
     return RMI_HIP_OK;
 }
 
