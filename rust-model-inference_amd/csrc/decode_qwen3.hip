@@ -1221,6 +1221,7 @@ struct rmi_hip_qwen3 : RmiSession {
     uint32_t walk_steps(uint32_t step, uint32_t most) const override;
     int enqueue_walk(uint32_t step, uint32_t n, uint32_t n_prompt, bool keep_logits, hipStream_t st) override;
     bool walk_gave_up() override;
+    void walk_tags_from(uint32_t tag0) override { walk.tag0 = tag0; }
 };
 
 namespace {
@@ -1463,6 +1464,7 @@ int rmi_hip_qwen3::enqueue_walk(uint32_t step, uint32_t n, uint32_t n_prompt, bo
     a.keep_logits = keep_logits;
     walk.tag0 += tags;
     walked = true;
+    walks_enqueued++;
     return rmi_launch_walk_qwen3(walk_shape, a, st);
 }
 bool rmi_hip_qwen3::walk_gave_up() {
@@ -1470,6 +1472,7 @@ bool rmi_hip_qwen3::walk_gave_up() {
     if (!walked) return false;
     walked = false;
     walk_off = walk_off || hipMemcpy(&failed, walk.failed, 4, hipMemcpyDeviceToHost) != hipSuccess || failed != 0;  // (not known is not finished)
+    walks_given_up += walk_off;
     return walk_off;
 }
 rmi_hip_qwen3::~rmi_hip_qwen3() {

@@ -51,6 +51,7 @@ struct RuvenexSession : rmi_hip_folder_session {
     }
     bool prepare_walk();
     bool walk_gave_up() override;
+    void walk_tags_from(uint32_t tag0) override { walk.tag0 = tag0; }
     bool walk_embeds(uint32_t step0, const float *host_layers) const override {
         return walks && walk.words && !host_layers && step0 > 0 && step0 < kWalkRvMaxKeys;
     }
@@ -91,6 +92,7 @@ int RuvenexSession::enqueue_layers(uint32_t step0, uint32_t n, hipStream_t st, f
         logits_there = want_logits;
         if (walk_spins) a.spins = walk_spins;
         walk.tag0 += n_runs + 1;
+        walks_enqueued++;
         rc = rmi_launch_walk_ruvenex(a, st);
         now ^= 1;
         position = step0 + 1;
@@ -150,6 +152,7 @@ bool RuvenexSession::walk_gave_up() {
     if (!walk.failed || !*static_cast<volatile uint32_t *>(walk.failed)) return false;
     *walk.failed = 0;
     walks = false;
+    walks_given_up++;
     return true;
 }
 

@@ -75,6 +75,7 @@ struct VogizenSession : rmi_hip_folder_session {
     }
     bool prepare_walk();
     bool walk_gave_up() override;
+    void walk_tags_from(uint32_t tag0) override { walk.tag0 = tag0; }
     bool walk_embeds(uint32_t step0, const float *host_layers) const override {
         return walks && walk.words && !host_layers && step0 > 0 && (step0 < walk.s.window ? step0 + 1 : walk.s.window) <= kWalkVgKeys;
     }
@@ -253,6 +254,7 @@ int VogizenSession::enqueue_layers(uint32_t step0, uint32_t n, hipStream_t st, f
         give_token(&a, step0);
         if (walk_spins) a.spins = walk_spins;
         walk.tag0 += n_runs + 1;
+        walks_enqueued++;
         rc = rmi_launch_walk_vogizen(a, st);
         pending = layers[runs.back().layer].side_norm;
         now ^= 1;
@@ -297,6 +299,7 @@ bool VogizenSession::walk_gave_up() {
     if (!walk.failed || !*static_cast<volatile uint32_t *>(walk.failed)) return false;
     *walk.failed = 0;
     walks = false;
+    walks_given_up++;
     return true;
 }
 

@@ -67,7 +67,13 @@ struct RmiSession {
     }
     // Whether a walk enqueued before could not finish (asked behind a synchronisation); walk_steps gives 0 from then on.
     virtual bool walk_gave_up() { return false; }
+    // The tag behind which the next walk's words begin: 0, or more than any before it.
+    virtual void walk_tags_from(uint32_t tag0) { (void)tag0; }
+    uint64_t walks_enqueued = 0, walks_given_up = 0;  // launches, and how often walk_gave_up said so
 };
+// for tests: the two counts, and walk_tags_from
+void rmi_session_walk_counts(const RmiSession *s, uint64_t counts[2]);
+void rmi_session_walk_tags_from(RmiSession *s, uint32_t tag0);
 
 // rmi_hip_<model>_generate: see rmi_hip_qwen3_generate in the header
 int rmi_session_generate(RmiSession *s, const uint32_t *prompt, uint32_t n_prompt, uint32_t max_new, uint32_t *generated,

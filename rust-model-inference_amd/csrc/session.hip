@@ -45,6 +45,12 @@ int rmi_session_set_stop_ids(RmiSession *s, const uint32_t *ids, uint32_t n_ids)
     return RMI_HIP_OK;
 }
 
+void rmi_session_walk_counts(const RmiSession *s, uint64_t counts[2]) {
+    counts[0] = s->walks_enqueued;
+    counts[1] = s->walks_given_up;
+}
+void rmi_session_walk_tags_from(RmiSession *s, uint32_t tag0) { s->walk_tags_from(tag0); }
+
 static int session_generate_once(RmiSession *s, const uint32_t *prompt, uint32_t n_prompt, uint32_t max_new, uint32_t *generated,
                                  uint32_t *step_argmax, float *step_top2, const uint32_t *dump_steps, uint32_t n_dump,
                                  float *dump_logits, double *seconds, bool *again) {

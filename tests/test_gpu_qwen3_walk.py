@@ -6,6 +6,7 @@ import threading
 
 import numpy as np
 import pytest
+from folder_helpers import walk_tags_from, walks
 
 pytestmark = pytest.mark.gpu
 
@@ -37,10 +38,14 @@ def test_walk_is_the_single_launches_bit_for_bit(hip, tmp_path, kw, drop, roundi
         dumps = sorted({n - 1, n + new // 2 - 1, n + new - 2})
         s.set_prompt_passes(passes)
         s.set_walks(1)
+        before = walks(hip, s)
         walked = s.generate(prompt, new, dumps)
         again = s.generate(prompt, new, dumps)
+        after = walks(hip, s)
+        assert (after[0] > before[0]) == (new > 1 or not passes) and after[1] == 0
         s.set_walks(0)
         single = s.generate(prompt, new, dumps)
+        assert walks(hip, s) == after
         _equal(walked, single, (kw, n, new))
         _equal(again, single, (kw, n, new, "again"))
     s.close()
@@ -55,6 +60,7 @@ def test_walk_is_the_cpu_loop(hip, oracle, tmp_path, n, new):
     cpu = oracle.Qwen3Decoder(meta, tensors, pool).generate(prompt, new, dump_steps=dumps)
     s = hip.decode.Qwen3Session(meta, tensors, n + new)
     _equal(s.generate(prompt, new, dumps), cpu, n)
+    assert walks(hip, s)[0] > 0 and walks(hip, s)[1] == 0
     s.close()
     pool.close()
 
@@ -65,14 +71,33 @@ def test_a_wait_that_is_given_up_leaves_the_single_launches(hip, tmp_path):
     prompt = np.random.default_rng(8).integers(0, 3000, 100, dtype=np.uint32)
     good = s.generate(prompt, 40, [99, 120, 138])
     s.set_walks(2)  # no vector crosses the chip that fast
+    assert walks(hip, s)[1] == 0
     _equal(s.generate(prompt, 40, [99, 120, 138]), good, "given up")
+    given_up = walks(hip, s)
+    assert given_up[1] == 1
     _equal(s.generate(prompt, 40, [99, 120, 138]), good, "single launches from then on")
+    assert walks(hip, s) == given_up
     s.set_walks(1)
     _equal(s.generate(prompt, 40, [99, 120, 138]), good, "on again")
+    assert walks(hip, s)[0] > given_up[0] and walks(hip, s)[1] == 1
     stop = int(good["tokens"][21])
     first = int(np.flatnonzero(good["tokens"] == stop)[0])
     s.set_stop_ids([stop])
     assert np.array_equal(s.generate(prompt, 40)["tokens"], good["tokens"][:first])
+    s.close()
+
+
+def test_tags_begin_anew(hip, tmp_path):
+    """16 tokens a launch of two layers are 49 tags: launches across the last tag, with words of all tags before them."""
+    meta, tensors = _model(hip, tmp_path)
+    s = hip.decode.Qwen3Session(meta, tensors, 200)
+    prompt = np.random.default_rng(9).integers(0, 3000, 20, dtype=np.uint32)
+    want = s.generate(prompt, 70, [30, 60, 88])
+    for left in (48, 49, 60, 99):
+        walk_tags_from(hip, s, 2**32 - 1 - left)
+        before = walks(hip, s)
+        _equal(s.generate(prompt, 70, [30, 60, 88]), want, left)
+        assert walks(hip, s)[0] > before[0] and walks(hip, s)[1] == 0
     s.close()
 
 
@@ -87,7 +112,9 @@ def test_largest_logits_of_every_wave(hip, tmp_path):
         prompt = rng.integers(0, s.vocab, n, dtype=np.uint32)
         s.set_prompt_passes(0)  # every position of the prompt by a walk, too: other tokens than the model's own
         s.set_walks(1)
+        before = walks(hip, s)
         walked = s.generate(prompt, 300, [n + 298])
+        assert walks(hip, s)[0] > before[0] and walks(hip, s)[1] == 0
         s.set_walks(0)
         _equal(walked, s.generate(prompt, 300, [n + 298]), n)
         rows.append(walked["argmax"])
@@ -116,4 +143,5 @@ def test_two_sessions_walk_on_two_threads(hip, tmp_path):
         assert len(got[k]) == 6
         for g in got[k]:
             _equal(g, alone[k], k)
+        assert walks(hip, sessions[k])[0] > 0 and walks(hip, sessions[k])[1] == 0
         sessions[k].close()

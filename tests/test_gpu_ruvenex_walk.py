@@ -7,7 +7,7 @@ import numpy as np
 import pytest
 import ruvenex_gen as G
 import ruvenex_plain as P
-from folder_helpers import BF16, F32, TOL, Opener, feed, rel
+from folder_helpers import BF16, F32, TOL, Opener, feed, generated_as_stepped, rel, tags_begin_anew, walks
 
 pytestmark = pytest.mark.gpu
 
@@ -51,6 +51,19 @@ def test_walk_against_single_launches_and_plain(open_model, kw):
     assert differ  # (the walk adds in another order: it was taken, though most logits come from the same bf16 values)
 
 
+@pytest.mark.parametrize("kw,n", [(SHAPES[0], 5), (SHAPES[1], 120), (SHAPES[2], 250), (SHAPES[3], 40)])
+def test_generated_tokens(hip, open_model, kw, n):
+    cfg = model(**kw)
+    s, w = open_model(cfg, None, BF16, n + 20)
+    generated_as_stepped(hip, s, G.tokens(cfg, n), 16, lambda t: P.forward(cfg, w, t), TOL[BF16])
+
+
+def test_tags_begin_anew(hip, open_model):
+    cfg = model(**SHAPES[0], n_layer=3)
+    s, _ = open_model(cfg, None, BF16, 40)
+    tags_begin_anew(hip, s, G.tokens(cfg, 14), 4)
+
+
 def test_shapes_the_walk_does_not_take(open_model):
     for kw in (dict(ff=None), dict(heads=3, kv_heads=1), dict(taps=1), dict(taps=5), dict(ff=300), dict(vdim=64), dict(rheads=3),
                dict(heads=16, kv_heads=8, rheads=16, ff=3072)):  # (the last: more workgroups than compute units)
@@ -88,7 +101,7 @@ def test_no_layers(open_model):
         assert rel(feed(s, t, [4, 1]), P.forward(cfg, w, t)) < TOL[dtype]
 
 
-def test_a_wait_that_is_given_up_leaves_the_single_launches(open_model):
+def test_a_wait_that_is_given_up_leaves_the_single_launches(hip, open_model):
     cfg = model(**SHAPES[0])
     s, _ = open_model(cfg, None, BF16, 120)
     t = G.tokens(cfg, 60)
@@ -98,9 +111,12 @@ def test_a_wait_that_is_given_up_leaves_the_single_launches(open_model):
     s.reset()
     s.set_walks(2)  # no vector crosses the chip that fast
     assert np.array_equal(feed(s, t[:41], [40, 1]), single[:41])
+    assert walks(hip, s) == [1, 1]
     assert np.array_equal(feed(s, t[41:], [1]), single[41:])  # by single launches from then on
+    assert walks(hip, s) == [1, 1]
     s.set_walks(2)
     again = s.generate(t[:40], 30, [39, 50, 68])
+    assert walks(hip, s) == [30, 2]
     for k in ("tokens", "argmax", "dump"):
         assert np.array_equal(again[k], made[k]), k
     s.reset()

@@ -7,7 +7,7 @@ import numpy as np
 import pytest
 import vogizen_gen as G
 import vogizen_plain as P
-from folder_helpers import BF16, F32, TOL, Opener, feed, rel
+from folder_helpers import BF16, F32, TOL, Opener, feed, generated_as_stepped, rel, tags_begin_anew, walks
 
 pytestmark = pytest.mark.gpu
 
@@ -54,6 +54,21 @@ def test_walk_against_single_launches_and_plain(open_model, kw, dtype):
 
 
 @pytest.mark.parametrize("dtype", [F32, BF16])
+@pytest.mark.parametrize("kw,n", [(dict(width=1024, kinds="da", loop=(0, 2, 2)), 5), (dict(width=2048, kinds="da", loop=(1, 2, 2), side=128), 90),
+                                  (dict(width=1024, kinds="ad", window=40), 60), (dict(width=2048, kinds="d"), 130)])
+def test_generated_tokens(hip, open_model, kw, n, dtype):
+    cfg = model(**kw)
+    s, w = open_model(cfg, None, dtype, n + 20)
+    generated_as_stepped(hip, s, G.tokens(cfg, n), 16, lambda t: P.forward(cfg, w, t), TOL[dtype])
+
+
+def test_tags_begin_anew(hip, open_model):
+    cfg = model(1024, "da", loop=(0, 2, 2))
+    s, _ = open_model(cfg, None, BF16, 40)
+    tags_begin_anew(hip, s, G.tokens(cfg, 14), 5)
+
+
+@pytest.mark.parametrize("dtype", [F32, BF16])
 def test_last_keys_and_a_ring(open_model, dtype):
     for kw, capacity, starts in ((dict(window=1024), 1100, (1017, 1050)), (dict(window=1100), 1200, (1018, 1060)), (dict(window=40), 2300, (2075, 2107, 2140)),
                                  (dict(window=1024), 3200, (3065, 3100))):
@@ -86,7 +101,7 @@ def test_no_layers(open_model, dtype):
 
 
 @pytest.mark.parametrize("dtype", [F32, BF16])
-def test_a_wait_that_is_given_up_leaves_the_single_launches(open_model, dtype):
+def test_a_wait_that_is_given_up_leaves_the_single_launches(hip, open_model, dtype):
     cfg = model(1024, "da", loop=(0, 2, 2))
     s, _ = open_model(cfg, None, dtype, 120)
     t = G.tokens(cfg, 60)
@@ -96,9 +111,12 @@ def test_a_wait_that_is_given_up_leaves_the_single_launches(open_model, dtype):
     s.reset()
     s.set_walks(2)  # no vector crosses the chip that fast
     assert np.array_equal(feed(s, t[:41], [40, 1]), single[:41])
+    assert walks(hip, s) == [1, 1]
     assert np.array_equal(feed(s, t[41:], [1]), single[41:])  # by single launches from then on
+    assert walks(hip, s) == [1, 1]
     s.set_walks(2)
     again = s.generate(t[:40], 30, [39, 50, 68])
+    assert walks(hip, s) == [30, 2]
     for k in ("tokens", "argmax", "dump"):
         assert np.array_equal(again[k], made[k]), k
     s.reset()
