@@ -1446,8 +1446,12 @@ bool rmi_hip_qwen3::pass_possible(uint32_t step0, uint32_t n) const { return pro
 int rmi_hip_qwen3::enqueue_pass(uint32_t step0, uint32_t n, const uint32_t *want, uint32_t n_want, bool, hipStream_t st, const RmiLogitsOf &of) {
     return enqueue_prompt_pass(this, step0, n, want, n_want, st, of);
 }
+// A walk has the chip to itself, while sessions' single launches fill the gaps between one another's: a session walks while no other one is at
+// work.  (The bits are the same.)  us a token of all, sessions of 28 layers behind 60 keys, launches | walked | by this rule: one 587 | 428 | 419,
+// two 337 | 416 | 337, four 348 | 415 | 349.  (Where the runtime puts two sessions' streams on one hardware queue, launches fill no gaps.)  The
+// other designs always walk, as walks' results differ from launches' within rounding and what a call gives is not to depend on other threads.
 uint32_t rmi_hip_qwen3::walk_steps(uint32_t step, uint32_t most) const {
-    if (!walk.words || walk_off || step == 0 || step + 1 >= kWalkMaxKeys) return 0;
+    if (!walk.words || walk_off || step == 0 || step + 1 >= kWalkMaxKeys || rmi_sessions_busy() > 1) return 0;
     const uint32_t fit = kWalkMaxKeys - 1 - step, n = most < fit ? most : fit;
     return n < kWalkMaxSteps ? n : kWalkMaxSteps;
 }

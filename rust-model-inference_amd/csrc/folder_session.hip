@@ -121,6 +121,7 @@ int rmi_hip_folder_session::feed(const uint32_t *tokens, uint32_t n, const uint3
     RmiThreadCtx *ctx = rmi_thread_ctx();
     if (!ctx) return RMI_HIP_E_RUNTIME;
     hipStream_t st = ctx->stream;
+    const RmiSessionBusy busy;
     const uint32_t step0 = position;
     // A token by itself travels with its embedding's launch: a copy and the wait for it took 20 us in front of the first kernel.
     if (n > 1) {

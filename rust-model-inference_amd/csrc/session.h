@@ -71,6 +71,14 @@ struct RmiSession {
     virtual void walk_tags_from(uint32_t tag0) { (void)tag0; }
     uint64_t walks_enqueued = 0, walks_given_up = 0;  // launches, and how often walk_gave_up said so
 };
+// A session's call that keeps the GPU busy is one of these while it lasts; how many there are in the process.
+struct RmiSessionBusy {
+    RmiSessionBusy();
+    ~RmiSessionBusy();
+    RmiSessionBusy(const RmiSessionBusy &) = delete;
+    RmiSessionBusy &operator=(const RmiSessionBusy &) = delete;
+};
+uint32_t rmi_sessions_busy();
 // for tests: the two counts, and walk_tags_from
 void rmi_session_walk_counts(const RmiSession *s, uint64_t counts[2]);
 void rmi_session_walk_tags_from(RmiSession *s, uint32_t tag0);

@@ -2,7 +2,15 @@
 #include "session.h"
 
 #include <algorithm>
+#include <atomic>
 #include <chrono>
+
+namespace {
+std::atomic<uint32_t> sessions_busy{0};
+}
+RmiSessionBusy::RmiSessionBusy() { sessions_busy++; }
+RmiSessionBusy::~RmiSessionBusy() { sessions_busy--; }
+uint32_t rmi_sessions_busy() { return sessions_busy; }
 
 RmiSession::~RmiSession() {
     for (void *p : owned) (void)hipFree(p);
@@ -169,6 +177,7 @@ static int session_generate_once(RmiSession *s, const uint32_t *prompt, uint32_t
 int rmi_session_generate(RmiSession *s, const uint32_t *prompt, uint32_t n_prompt, uint32_t max_new, uint32_t *generated,
                          uint32_t *step_argmax, float *step_top2, const uint32_t *dump_steps, uint32_t n_dump,
                          float *dump_logits, double *seconds) {
+    const RmiSessionBusy busy;
     bool again = false;
     int rc = session_generate_once(s, prompt, n_prompt, max_new, generated, step_argmax, step_top2, dump_steps, n_dump, dump_logits, seconds, &again);
     if (again)  // a walk could not finish: the whole sequence once more, by single launches

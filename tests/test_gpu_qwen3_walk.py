@@ -2,6 +2,7 @@
 single launches and against the CPU loop: tokens, every step's argmax and two largest logits and the asked logits bit for bit,
 where its branches change: heads that share their keys' scores (from 352 keys on), slices of values longer than what is loaded
 ahead (from 769 keys on), the last position it takes (1279 keys), launches of up to 16 tokens."""
+import ctypes as C
 import threading
 
 import numpy as np
@@ -120,6 +121,23 @@ def test_largest_logits_of_every_wave(hip, tmp_path):
         rows.append(walked["argmax"])
     wave = np.concatenate(rows) // 8
     assert set(wave % 8) == set(range(8)) and ((wave // 8 >= 64) & (wave // 8 < 128)).any()
+    s.close()
+
+
+def test_a_session_walks_only_while_no_other_is_at_work(hip, tmp_path):
+    meta, tensors = _model(hip, tmp_path)
+    s = hip.decode.Qwen3Session(meta, tensors, 100)
+    prompt = np.random.default_rng(7).integers(0, 3000, 30, dtype=np.uint32)
+    alone, before = s.generate(prompt, 40, [60]), walks(hip, s)
+    other = (C.c_uint8 * 8)()
+    hip.hip.lib._ZN14RmiSessionBusyC1Ev(other)  # what another session's call holds
+    try:
+        _equal(s.generate(prompt, 40, [60]), alone, "beside another")
+        assert walks(hip, s) == before
+    finally:
+        hip.hip.lib._ZN14RmiSessionBusyD1Ev(other)
+    _equal(s.generate(prompt, 40, [60]), alone, "alone again")
+    assert walks(hip, s)[0] == 2 * before[0]
     s.close()
 
 
