@@ -462,8 +462,8 @@ int rmi_hip_qwen3_set_stop_ids(rmi_hip_qwen3 *s, const uint32_t *ids, uint32_t n
  * most 1024).  Measured on a 1999-token prompt of a Qwen3-0.6B model: 1.1 ms a position step by step beyond 1280 keys,
  * 0.0145 ms in passes. */
 int rmi_hip_qwen3_set_prompt_passes(rmi_hip_qwen3 *s, int enabled);
-/* Tokens of a model of Qwen3-0.6B's widths (head dimension 128, up to 1279 keys) are generated up to 16 to a cooperative launch
- * that walks all layers, the bits of the single launches.  enabled = 1 (the default): so; 0: single launches only; n > 1: so, and a
+/* Tokens of a model of width 512 or 1024 with 8 or 16 heads of 128, a feed-forward of one to four times 1024 and up to 1279 keys are
+ * generated up to 16 to a cooperative launch that walks all layers, the bits of the single launches.  enabled = 1 (the default): so; 0: single launches only; n > 1: so, and a
  * wait between workgroups is given up after it has asked n times (by default 131072, 65 ms or more: some other program's kernel held
  * compute units meanwhile), after which rmi_hip_qwen3_generate begins anew by single launches and the session keeps to them until the next
  * call of this.  Such a launch holds every compute unit for up to 8 ms; while other sessions of the process are at work, too, single

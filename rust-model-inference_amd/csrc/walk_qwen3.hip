@@ -741,12 +741,29 @@ WalkChoice walk_choice() {
     if (lds < kWalkAttnLds) lds = kWalkAttnLds;
     return WalkChoice{qwen3_walk_kernel<NE, NO, ND>, lds};
 }
+// The kernel for a width of NE octets: NO and ND follow from the o and the down product's rows, whose quarters are whole octets.
+// us a token of eight layers and a vocabulary of 32768 by launches | walked, behind 100 keys and behind 1240, width, heads, n_ff:
+//   512, 8, 1024 154 | 103, 247 | 171; 512, 16, 4096 180 | 119, 269 | 184; 1024, 8, 1024 170 | 112, 263 | 180;
+//   1024, 8, 3072 165 | 120, 256 | 186; 1024, 16, 3072 180 | 125, 272 | 190; 1024, 16, 4096 198 | 127, 287 | 189.
+// A workgroup of the norm role makes one block of 32 gate|up rows with weights that it has before the norm; all these sizes have as many
+// norm workgroups as blocks.  Width 2048 with 16 heads and n_ff = 6144, as <8, 2, 6>, leaves 64 for 192 blocks, three rounds of which two
+// wait for their weights: 294 | 305 behind 100 keys, 344 | 330 behind 700.  A product's rows that are no multiple of 1024 are not whole
+// octets a wave, and 768 values of x not whole ones a thread.
+template <int NE, int NO, int ND>
+WalkChoice walk_choose_sizes(uint32_t n_attn, uint32_t n_ff) {
+    if (n_attn == NO * 1024 && n_ff == ND * 1024) return walk_choice<NE, NO, ND>();
+    if constexpr (ND < 4)
+        return walk_choose_sizes<NE, NO, ND + 1>(n_attn, n_ff);
+    else if constexpr (NO < 2)
+        return walk_choose_sizes<NE, NO + 1, NO + 1>(n_attn, n_ff);
+    else
+        return WalkChoice{nullptr, 0};
+}
 WalkChoice walk_choose(const RmiWalkShape &s) {
     const uint32_t n_attn = s.n_head * 128;
-    // (Width 2048 with n_ff = 6144 as <8, 2, 6> has 64 norm workgroups for 192 blocks of gate|up, three rounds of which two wait for
-    // their weights: us a token of eight layers by launches | walked, behind 100 keys 294 | 305, 700: 344 | 330.)
-    if (s.n_embd == 1024 && n_attn == 2048 && s.n_ff == 3072) return walk_choice<4, 2, 3>();
-    return WalkChoice{nullptr, 0};
+    return s.n_embd == 512    ? walk_choose_sizes<2, 1, 1>(n_attn, s.n_ff)
+           : s.n_embd == 1024 ? walk_choose_sizes<4, 1, 1>(n_attn, s.n_ff)
+                              : WalkChoice{nullptr, 0};
 }
 
 }  // namespace

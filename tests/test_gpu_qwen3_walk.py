@@ -52,6 +52,31 @@ def test_walk_is_the_single_launches_bit_for_bit(hip, tmp_path, kw, drop, roundi
     s.close()
 
 
+@pytest.mark.parametrize("width,heads,kv,ff", [(512, 8, 8, 1024), (512, 8, 1, 3072), (512, 16, 2, 2048), (512, 16, 16, 4096), (1024, 8, 4, 1024), (1024, 8, 8, 4096),
+                                               (1024, 8, 2, 3072), (1024, 16, 4, 2048), (1024, 16, 8, 4096)])
+def test_sizes_of_the_walk(hip, tmp_path, width, heads, kv, ff):
+    meta, tensors = _model(hip, tmp_path, n_embd=width, n_head=heads, n_head_kv=kv, n_ff=ff, vocab=1500)
+    s = hip.decode.Qwen3Session(meta, tensors, 1300)
+    for n, new in ((1, 20), (345, 16), (764, 10), (1262, 24)):
+        prompt = np.random.default_rng(n).integers(0, s.vocab, n, dtype=np.uint32)
+        s.set_walks(1)
+        before = walks(hip, s)
+        walked = s.generate(prompt, new, [n - 1, n + new - 2])
+        assert walks(hip, s)[0] > before[0] and walks(hip, s)[1] == 0
+        s.set_walks(0)
+        _equal(walked, s.generate(prompt, new, [n - 1, n + new - 2]), n)
+    s.close()
+
+
+@pytest.mark.parametrize("width,heads,kv,ff", [(768, 8, 4, 3072), (1024, 16, 8, 2560), (1024, 12, 4, 3072), (1024, 16, 8, 5120), (2048, 16, 8, 6144)])
+def test_sizes_that_are_not_the_walks(hip, tmp_path, width, heads, kv, ff):
+    meta, tensors = _model(hip, tmp_path, n_embd=width, n_head=heads, n_head_kv=kv, n_ff=ff, vocab=500, n_layer=1)
+    s = hip.decode.Qwen3Session(meta, tensors, 60)
+    assert s.generate(np.arange(30, dtype=np.uint32), 20)["tokens"].size == 20
+    assert walks(hip, s) == [0, 0]
+    s.close()
+
+
 @pytest.mark.parametrize("n,new", [(1, 12), (348, 8), (766, 6)])
 def test_walk_is_the_cpu_loop(hip, oracle, tmp_path, n, new):
     meta, tensors = _model(hip, tmp_path)
