@@ -119,14 +119,10 @@ struct RmiEmbed {
 int rmi_dense_embed(uint32_t elem_bytes, const RmiEmbed &e, const uint32_t *tok, uint32_t pos0, uint32_t n_tokens, hipStream_t st);
 // one token that the host knows: it travels with the launch, which leaves it in *tok for those behind it
 int rmi_dense_embed_token(uint32_t elem_bytes, const RmiEmbed &e, uint32_t token, uint32_t *tok, uint32_t pos, hipStream_t st);
-// several tokens: matrix cores; a = [n_tokens] rows of k_pad elements, rmi_dense_ld apart
-int rmi_dense_gemm(uint32_t elem_bytes, const RmiDense &w, const void *a, const RmiRowSegs &segs, uint32_t n_tokens, hipStream_t st);
-int rmi_dense_gemm_residual(uint32_t elem_bytes, const RmiDense &w, const void *a, const RmiColSegs &segs, float *x, uint32_t width,
-                            uint32_t n_tokens, hipStream_t st);
-// The same with memory of the caller's (a stream's own): a product whose tiles would leave compute units idle may divide k over several
-// workgroups a tile, which leave their sums there.
+// Several tokens: matrix cores; a = [n_tokens] rows of k_pad elements, rmi_dense_ld apart.  With memory of the caller's (a stream's own) a
+// product whose tiles would leave compute units idle may divide k over several workgroups a tile, which leave their sums there.
 constexpr uint32_t kDenseCounters = 4096;     // zero before a product, and behind it
-constexpr uint32_t kDenseSums = 4096 * 1024;  // floats
+constexpr uint32_t kDenseSums = 4096 * 1024;  // floats: 16 MB of every session, whatever its model's size
 struct RmiDenseWork {
     uint32_t *counts = nullptr;
     float *sums = nullptr;
@@ -135,9 +131,9 @@ int rmi_dense_gemm(uint32_t elem_bytes, const RmiDense &w, const void *a, const 
                    hipStream_t st);
 int rmi_dense_gemm_residual(uint32_t elem_bytes, const RmiDense &w, const void *a, const RmiColSegs &segs, float *x, uint32_t width,
                             uint32_t n_tokens, const RmiDenseWork &work, hipStream_t st);
-// the workgroups a tile that these take, parts << 16 | tokens of a tile << 4 | waves (as below)
+// the workgroups a tile that these take with such memory, parts << 16 | tokens of a tile << 4 | waves (as below)
 uint32_t rmi_dense_parts(uint32_t elem_bytes, int epilogue, uint32_t n_rows, uint32_t k_pad, uint32_t n_tokens);
-// the tile that such a product takes, weight rows << 16 | tokens << 4 | waves (n_rows: of the weight, or a residual one's width;
+// the tile that a product takes without it, weight rows << 16 | tokens << 4 | waves (n_rows: of the weight, or a residual one's width;
 // epilogue: -1 residual, else RmiEpilogue's)
 uint32_t rmi_dense_tile(uint32_t elem_bytes, int epilogue, uint32_t n_rows, uint32_t k_pad, uint32_t n_tokens);
 // one token: the input in front of the product is part of the launch, for as many columns as a workgroup holds; the

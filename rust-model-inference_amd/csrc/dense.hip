@@ -862,12 +862,3 @@ int rmi_dense_gemm_residual(uint32_t elem_bytes, const RmiDense &w, const void *
     return elem_bytes == 2 ? launch_gemm<rmi_bf16, kResidual>(w, a, RmiRowSegs{}, segs, x, width, n_tokens, work.counts ? &work : nullptr, st)
                            : launch_gemm<float, kResidual>(w, a, RmiRowSegs{}, segs, x, width, n_tokens, work.counts ? &work : nullptr, st);
 }
-
-int rmi_dense_gemm(uint32_t elem_bytes, const RmiDense &w, const void *a, const RmiRowSegs &segs, uint32_t n_tokens, hipStream_t st) {
-    return rmi_dense_gemm(elem_bytes, w, a, segs, n_tokens, RmiDenseWork{}, st);
-}
-
-int rmi_dense_gemm_residual(uint32_t elem_bytes, const RmiDense &w, const void *a, const RmiColSegs &segs, float *x, uint32_t width,
-                            uint32_t n_tokens, hipStream_t st) {
-    return rmi_dense_gemm_residual(elem_bytes, w, a, segs, x, width, n_tokens, RmiDenseWork{}, st);
-}

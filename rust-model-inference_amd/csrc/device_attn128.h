@@ -18,13 +18,6 @@ __device__ __forceinline__ double quad_sum(double v) {  // (l0 + l1) + (l2 + l3)
     v += __hiloint2double(__builtin_amdgcn_mov_dpp(hi, 0x4E, 0xf, 0xf, true), __builtin_amdgcn_mov_dpp(lo, 0x4E, 0xf, 0xf, true));
     return v;
 }
-template <int XOR>
-__device__ __forceinline__ double swizzle_xor_f64(double v) {  // the value of lane ^ XOR (XOR < 32)
-    constexpr int kPattern = 0x1f | (XOR << 10);
-    return __hiloint2double(__builtin_amdgcn_ds_swizzle(__double2hiint(v), kPattern),
-                            __builtin_amdgcn_ds_swizzle(__double2loint(v), kPattern));
-}
-__device__ __forceinline__ double swizzle_xor16_f64(double v) { return swizzle_xor_f64<16>(v); }
 // Two registers exchange lanes in one vector instruction (v_permlane32_swap: lanes 32..63 of the first with lanes
 // 0..31 of the second; v_permlane16_swap: the odd rows of sixteen of the first with the even rows of the second).
 // a + b afterwards is, in the lower half (the even rows), a summed over both halves (both rows of a pair), and in the

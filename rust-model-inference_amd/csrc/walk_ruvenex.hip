@@ -22,6 +22,11 @@
 // words and its gates of the layer before; mixers' words are behind everything that norms.  x itself is kept twice, by odd and even
 // layers: a row of the next x does not depend on workgroups that make other rows' gates only, that of the one after next does.
 // What crosses tokens (caches, history, state) crosses launches.
+//
+// Width 1024 only: a thread has whole values of x and a lane whole pieces of a row, which 512 and 1536 do not give, and 2048 would want 205
+// output workgroups.  A wave's weights, six rows or a piece of ten, are what 128 registers hold beside the rest (of 48 bytes a lane that do
+// not fit, addresses of the history, a mixer's wave reads some back in front of its wait for words): with those, 28-layer sizes of width
+// 1024 and a feed-forward of 3072 are 256 workgroups, and more rows go by the single launches.
 #include "walk_ruvenex.h"
 
 #include "device_dense.h"
@@ -30,6 +35,7 @@
 namespace {
 
 constexpr uint32_t T = 1024;
+constexpr uint32_t kWidth = 1024, NQ = kWidth / 512;  // 16-byte pieces a lane of a row of the width
 constexpr uint32_t kInRows = 6;    // of a wave, everything that reads h
 constexpr uint32_t kOutRows = 10;  // of a workgroup, everything that ends in x
 constexpr uint32_t kDim = 128;    // of every head
@@ -344,7 +350,6 @@ __device__ __forceinline__ bool walk_recur(const RvCtx &c, uint32_t of_head, uin
 }
 
 // ---- everything that reads h: kInRows rows a wave
-template <uint32_t NQ>
 __device__ __forceinline__ void walk_input(const RvCtx &c, uint32_t idx, RvLds &sm, u32x4 *h) {
     const RmiWalkRvArgs &a = c.a;
     const RmiWalkRvShape &s = a.s;
@@ -513,7 +518,6 @@ __device__ __forceinline__ void walk_output(const RvCtx &c, uint32_t idx, RvLds 
 
 // ---- the vocabulary: every workgroup, eight rows a wave at a time.  A launch behind a cooperative one begins 11 us after it; here the first
 // rows are asked for in front of the last layer's vector, and a row's place in the registers takes the next one as soon as it is multiplied.
-template <uint32_t NQ>
 __device__ __forceinline__ void walk_head(const RvCtx &c, RvLds &sm, u32x4 *h) {
     const RmiWalkRvArgs &a = c.a;
     const RmiWalkRvShape &s = a.s;
@@ -573,8 +577,6 @@ __device__ __forceinline__ void walk_head(const RvCtx &c, RvLds &sm, u32x4 *h) {
     }
 }
 
-// NQ pieces of a row of the width a lane
-template <uint32_t NQ>
 __global__ __launch_bounds__(T) void ruvenex_walk_kernel(RmiWalkRvArgs a) {
     __shared__ RvLds sm;
     __shared__ u32x4 staged[T];  // the normed stream, or what the last product reads
@@ -597,13 +599,13 @@ __global__ __launch_bounds__(T) void ruvenex_walk_kernel(RmiWalkRvArgs a) {
     } else if (b < n_mix + a.n_output) {
         walk_output(c, b - n_mix, sm, staged);
     } else {
-        walk_input<NQ>(c, b - n_mix - a.n_output, sm, staged);
+        walk_input(c, b - n_mix - a.n_output, sm, staged);
     }
     if (a.head) {
         __syncthreads();
         const bool bad = sm.bad != 0;
         __syncthreads();  // (nobody gives up a wait before everybody has read it)
-        if (!bad) walk_head<NQ>(c, sm, staged);
+        if (!bad) walk_head(c, sm, staged);
     }
 }
 
@@ -621,12 +623,12 @@ bool rmi_walk_ruvenex_fits(const RmiWalkRvShape &s) {
     // The embedding lies where the last layer's x goes.  With a layer between, whose x all of the last one depends on, everybody has read it by
     // then; with one layer an input workgroup that makes other rows' gates only may not have.
     if (s.n_layer < 2) return false;
-    if (s.k_in != 1024 || s.width != s.k_in || s.k_pad / 8 > T || roles_of(s).all() > uint32_t(rmi_device_cus())) return false;
+    if (s.k_in != kWidth || s.width != s.k_in || s.k_pad / 8 > T || roles_of(s).all() > uint32_t(rmi_device_cus())) return false;
     if (s.k_attn != s.heads * kDim || s.k_recur - s.k_attn != s.recur_heads * kDim || s.taps > 4 || s.taps < 2 || s.heads % s.kv_heads) return false;
     if (s.seg[kSegs] - s.seg[kSegUp] != s.k_pad - s.k_recur) return false;
     int coop = 0, per_cu = 0;
     if (hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, rmi_device()) != hipSuccess || !coop ||
-        hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, ruvenex_walk_kernel<2>, int(T), 0) != hipSuccess) {
+        hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, ruvenex_walk_kernel, int(T), 0) != hipSuccess) {
         (void)hipGetLastError();
         return false;
     }
@@ -640,6 +642,6 @@ int rmi_launch_walk_ruvenex(RmiWalkRvArgs a, hipStream_t st) {
     const Roles r = roles_of(a.s);
     a.n_output = r.output;
     void *args[] = {&a};
-    RMI_HIP_CHECK(hipLaunchCooperativeKernel(reinterpret_cast<const void *>(ruvenex_walk_kernel<2>), dim3(r.all()), dim3(T), args, 0, st));
+    RMI_HIP_CHECK(hipLaunchCooperativeKernel(reinterpret_cast<const void *>(ruvenex_walk_kernel), dim3(r.all()), dim3(T), args, 0, st));
     return RMI_HIP_OK;
 }

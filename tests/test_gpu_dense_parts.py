@@ -7,22 +7,10 @@ import ctypes as C
 import numpy as np
 import pytest
 
-from test_gpu_dense_tiles import ColSeg, Dense, RowSeg, RowSegs, _check, _operand
+from test_gpu_dense_tiles import PARTS, RESIDUAL, ROWS, ColSeg, ColSegs, Dense, RowSeg, RowSegs, Work, _check, _operand
 
 pytestmark = pytest.mark.gpu
 
-
-class ColSegs(C.Structure):
-    _fields_ = [("s", ColSeg * 4), ("n_segs", C.c_uint32), ("k_begin", C.c_uint32)]
-
-
-class Work(C.Structure):
-    _fields_ = [("counts", C.c_void_p), ("sums", C.c_void_p)]
-
-
-ROWS = "_Z14rmi_dense_gemmjRK8RmiDensePKvRK10RmiRowSegsjRK12RmiDenseWorkP12ihipStream_t"
-RESIDUAL = "_Z23rmi_dense_gemm_residualjRK8RmiDensePKvRK10RmiColSegsPfjjRK12RmiDenseWorkP12ihipStream_t"
-PARTS = "_Z15rmi_dense_partsjijjj"
 COUNTERS, SUMS = 4096, 4096 * 1024
 
 

@@ -26,15 +26,21 @@ class ColSeg(C.Structure):
 
 
 class ColSegs(C.Structure):
-    _fields_ = [("s", ColSeg * 4), ("n_segs", C.c_uint32)]
+    _fields_ = [("s", ColSeg * 4), ("n_segs", C.c_uint32), ("k_begin", C.c_uint32)]
 
 
 class Dense(C.Structure):
     _fields_ = [("data", C.c_void_p), ("n_rows", C.c_uint32), ("k_pad", C.c_uint32), ("ld", C.c_uint32)]
 
 
-ROWS = "_Z14rmi_dense_gemmjRK8RmiDensePKvRK10RmiRowSegsjP12ihipStream_t"
-RESIDUAL = "_Z23rmi_dense_gemm_residualjRK8RmiDensePKvRK10RmiColSegsPfjjP12ihipStream_t"
+class Work(C.Structure):
+    _fields_ = [("counts", C.c_void_p), ("sums", C.c_void_p)]
+
+
+ROWS = "_Z14rmi_dense_gemmjRK8RmiDensePKvRK10RmiRowSegsjRK12RmiDenseWorkP12ihipStream_t"
+RESIDUAL = "_Z23rmi_dense_gemm_residualjRK8RmiDensePKvRK10RmiColSegsPfjjRK12RmiDenseWorkP12ihipStream_t"
+PARTS = "_Z15rmi_dense_partsjijjj"
+UNDIVIDED = C.byref(Work())  # no memory for the parts' sums: whole products (test_gpu_dense_parts has divided ones)
 K_RELU_GLU = 5
 
 
@@ -73,7 +79,7 @@ def test_rows(hip, elem, rows, k, tokens):
     segs.start[2:] = [rows] * 10
     segs.n_segs, segs.n_rows = 2, rows
     fn = getattr(H.lib, ROWS)
-    assert fn(C.c_uint32(elem), C.byref(Dense(d_w.ptr, rows, k, ld)), C.c_void_p(d_x.ptr), C.byref(segs), C.c_uint32(tokens), None) == 0
+    assert fn(C.c_uint32(elem), C.byref(Dense(d_w.ptr, rows, k, ld)), C.c_void_p(d_x.ptr), C.byref(segs), C.c_uint32(tokens), UNDIVIDED, None) == 0
     H.check(H.lib.rmi_hip_synchronize())
     _check(d_y.to_array(np.float32, (tokens, rows)), wv, xv)
 
@@ -95,7 +101,7 @@ def test_residual_column_segments(hip, elem, rows, k, tokens):
     segs.s[0], segs.s[1], segs.n_segs = ColSeg(bufs[3].ptr, rows, 0.5, half), ColSeg(bufs[4].ptr, 0, 2.0, k), 2
     fn = getattr(H.lib, RESIDUAL)
     assert fn(C.c_uint32(elem), C.byref(Dense(bufs[0].ptr, padded, k, ld)), C.c_void_p(bufs[1].ptr), C.byref(segs), C.c_void_p(bufs[2].ptr),
-              C.c_uint32(rows), C.c_uint32(tokens), None) == 0
+              C.c_uint32(rows), C.c_uint32(tokens), UNDIVIDED, None) == 0
     H.check(H.lib.rmi_hip_synchronize())
     got, wv = bufs[2].to_array(np.float32, (tokens, rows)), wv[:rows]
     want = x + 0.5 * gate * (av[:, :half] @ wv[:, :half].T) + 2.0 * one * (av[:, half:] @ wv[:, half:].T)
@@ -116,7 +122,7 @@ def test_relu_pairs(hip, elem, rows, k, tokens):
     segs.start[1:] = [rows] * 11
     segs.n_segs, segs.n_rows = 1, rows
     fn = getattr(H.lib, ROWS)
-    assert fn(C.c_uint32(elem), C.byref(Dense(d_w.ptr, rows, k, ld)), C.c_void_p(d_x.ptr), C.byref(segs), C.c_uint32(tokens), None) == 0
+    assert fn(C.c_uint32(elem), C.byref(Dense(d_w.ptr, rows, k, ld)), C.c_void_p(d_x.ptr), C.byref(segs), C.c_uint32(tokens), UNDIVIDED, None) == 0
     H.check(H.lib.rmi_hip_synchronize())
     if elem == 2:
         got = (d_y.to_array(np.uint16, (tokens, rows // 2)).astype(np.uint32) << 16).view(np.float32)
@@ -176,6 +182,14 @@ def _chosen(hip, elem, kind, rows, k, tokens):
     return t >> 16, t >> 4 & 0xfff, t & 15
 
 
+def _whole_in_sessions(hip, kind, rows, k, tokens):
+    """A session, which has memory for parts, takes such a bf16 product whole and by the same tile."""
+    fn = getattr(hip.hip.lib, PARTS)
+    fn.restype = C.c_uint32
+    t = fn(C.c_uint32(2), C.c_int(EPILOGUES[kind]), C.c_uint32(rows), C.c_uint32(k), C.c_uint32(tokens))
+    return (t >> 16, t >> 4 & 0xfff, t & 15) == (1, *_chosen(hip, 2, kind, rows, k, tokens)[1:])
+
+
 # us of bf16 products, each launch with a weight from HBM, by the tiles of 64 x 64, 64 x 128, 128 x 128 with four and with eight
 # waves, 128 x 256 and 256 x 256: as the estimates were fitted, when the wide tiles' results left from the registers, and as the
 # tiles are (SiLU, results in bf16; residual products have no 256 x 256)
@@ -195,6 +209,7 @@ def test_the_choice_follows_the_measurements(hip, kind, rows, k, tokens, us):
     if hip.hip.device_info()[1] != 256:
         pytest.skip("measured on 256 compute units")
     assert us[MEASURED_TILES.index(_chosen(hip, 2, kind, rows, k, tokens))] <= 1.03 * min(us)
+    assert _whole_in_sessions(hip, kind, rows, k, tokens)
 
 
 @pytest.mark.parametrize("kind,rows,k,tokens,us", MEASURED_SINCE)
@@ -204,6 +219,7 @@ def test_how_far_the_choice_is_from_todays_tiles(hip, kind, rows, k, tokens, us)
     if hip.hip.device_info()[1] != 256:
         pytest.skip("measured on 256 compute units")
     assert us[MEASURED_TILES.index(_chosen(hip, 2, kind, rows, k, tokens))] <= 1.4 * min(us)
+    assert _whole_in_sessions(hip, kind, rows, k, tokens)
 
 
 @pytest.mark.parametrize("tile,kind,size", CASES, ids=["%d-%dx%dx%d-%s" % (*t, k) for t, k, _ in CASES])
@@ -235,7 +251,7 @@ def test_every_tile(hip, tile, kind, size):
         segs = ColSegs()
         segs.s[0], segs.s[1], segs.n_segs = ColSeg(bufs[3].ptr, rows, 0.5, half), ColSeg(None, 0, 2.0, k), 2
         assert getattr(H.lib, RESIDUAL)(C.c_uint32(elem), C.byref(d_w), C.c_void_p(bufs[1].ptr), C.byref(segs), C.c_void_p(bufs[2].ptr),
-                                        C.c_uint32(rows), C.c_uint32(tokens), None) == 0
+                                        C.c_uint32(rows), C.c_uint32(tokens), UNDIVIDED, None) == 0
         H.check(H.lib.rmi_hip_synchronize())
         got = bufs[2].to_array(np.float32, (tokens, rows))
         want = acc + 0.5 * gate * (xv[:, :half] @ wv[:, :half].T) + 2.0 * (xv[:, half:] @ wv[:, half:].T)
@@ -259,7 +275,7 @@ def test_every_tile(hip, tile, kind, size):
         segs.start[i] = a
     segs.start[4:] = [rows] * 8
     segs.n_segs, segs.n_rows = 4, rows
-    assert getattr(H.lib, ROWS)(C.c_uint32(elem), C.byref(d_w), C.c_void_p(bufs[1].ptr), C.byref(segs), C.c_uint32(tokens), None) == 0
+    assert getattr(H.lib, ROWS)(C.c_uint32(elem), C.byref(d_w), C.c_void_p(bufs[1].ptr), C.byref(segs), C.c_uint32(tokens), UNDIVIDED, None) == 0
     H.check(H.lib.rmi_hip_synchronize())
     for i in range(4):
         at = slice(cuts[i], cuts[i + 1])
@@ -297,7 +313,7 @@ def test_residual_segments_of_one_gate(hip, elem, rows, tokens):
             first = ends[i]
         segs.n_segs = 4
         assert getattr(H.lib, RESIDUAL)(C.c_uint32(elem), C.byref(Dense(bufs[0].ptr, padded, ends[-1], ld)), C.c_void_p(bufs[1].ptr), C.byref(segs),
-                                        C.c_void_p(bufs[2].ptr), C.c_uint32(rows), C.c_uint32(tokens), None) == 0
+                                        C.c_void_p(bufs[2].ptr), C.c_uint32(rows), C.c_uint32(tokens), UNDIVIDED, None) == 0
         H.check(H.lib.rmi_hip_synchronize())
         got = bufs[2].to_array(np.float32, (tokens, rows))
         # sums of k products as above, and a few roundings of what they are part of
@@ -333,7 +349,7 @@ def test_segments_join_one_after_the_other(hip, elem, rows, tokens, size, scales
             segs.s[i] = ColSeg(gates[gate_of[j]].ptr, rows, scales[j], ends[j] - first)
         segs.n_segs = len(segments)
         assert getattr(H.lib, RESIDUAL)(C.c_uint32(elem), C.byref(Dense(d_w.ptr, padded, k, ld)), C.c_void_p(d_a.ptr), C.byref(segs),
-                                        C.c_void_p(d_x.ptr), C.c_uint32(rows), C.c_uint32(tokens), None) == 0
+                                        C.c_void_p(d_x.ptr), C.c_uint32(rows), C.c_uint32(tokens), UNDIVIDED, None) == 0
         H.check(H.lib.rmi_hip_synchronize())
 
     together, apart = H.DeviceBuffer.from_array(x), H.DeviceBuffer.from_array(x)
@@ -367,7 +383,7 @@ def test_narrow_segments_of_a_wide_tile(hip, elem, last, k, tokens, narrow):
         row += (n + 15) // 16 * 16
     segs.start[len(lengths):] = [rows] * (12 - len(lengths))
     segs.n_segs, segs.n_rows = len(lengths), rows
-    assert getattr(H.lib, ROWS)(C.c_uint32(elem), C.byref(Dense(bufs[0].ptr, rows, k, ld)), C.c_void_p(bufs[1].ptr), C.byref(segs), C.c_uint32(tokens), None) == 0
+    assert getattr(H.lib, ROWS)(C.c_uint32(elem), C.byref(Dense(bufs[0].ptr, rows, k, ld)), C.c_void_p(bufs[1].ptr), C.byref(segs), C.c_uint32(tokens), UNDIVIDED, None) == 0
     H.check(H.lib.rmi_hip_synchronize())
     for buf, (row0, n, stride, dtype) in zip(bufs[2:], outs):
         got = buf.to_array(dtype, (tokens, stride))
