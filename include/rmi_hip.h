@@ -566,11 +566,11 @@ int rmi_hip_folder_reset(rmi_hip_folder_session *s);               /* the sequen
 int rmi_hip_folder_set_stop_ids(rmi_hip_folder_session *s, const uint32_t *ids, uint32_t n_ids);
 int rmi_hip_folder_set_prompt_passes(rmi_hip_folder_session *s, int enabled);
 /* As rmi_hip_qwen3_set_walks.  A single token behind the first goes through one launch that walks all layers where they are of one
- * shape that has one: Ruvenex in bf16, width 1024, heads of 128, two to four taps, a feed-forward of whole 256s, positions up to 511;
- * Vogizen of width 1024 or 2048, 16 heads of 128, a feed-forward of three times the width, a token side of 64 or 128, ranks of whole 256s
- * up to 768 and 256 or 1024 and 512, positions that see up to 1024 keys.  It agrees with the single launches within
- * rounding; a token whose launch gave up (an rmi_hip_folder_generate: the sequence) is done again by them.  Walks of several sessions
- * take turns, for a token's length each.  us a token of all, bf16, single launches | walks: Ruvenex with 28 layers of width 1024, one
+ * shape that has one: Ruvenex in bf16, width 1024, heads of 128, two layers or more, two to four taps, a feed-forward that is whole 256s
+ * when padded to 16, positions up to 511; Vogizen of width 1024 or 2048, 16 heads of 128, a feed-forward of three times the width, a token
+ * side of 64 or 128, ranks of whole 256s up to 768 and 256 or 1024 and 512, positions that see up to 1024 keys.  It agrees with the single
+ * launches within rounding; a token whose launch gave up (an rmi_hip_folder_generate: the sequence) is done again by them.  Walks of several
+ * sessions take turns, for a token's length each.  us a token of all, bf16, single launches | walks: Ruvenex with 28 layers of width 1024, one
  * session 542 | 314, two 392 | 277, four 375 | 277; Vogizen with 8 runs of width 1024 462 | 317, 283 | 269, 262 | 278. */
 int rmi_hip_folder_set_walks(rmi_hip_folder_session *s, int enabled);
 int rmi_hip_folder_generate(rmi_hip_folder_session *s, const uint32_t *prompt, uint32_t n_prompt, uint32_t max_new,

@@ -30,7 +30,7 @@ struct RmiWalkArgs {
     uint32_t step0, n_steps, n_prompt;
     uint32_t tag0;                 // every word of this launch carries a tag above it
     uint32_t keep_logits;
-    uint32_t n_attn, n_res, n_norm;  // workgroups by role (rmi_walk_qwen3_roles)
+    uint32_t n_attn, n_res, n_norm;  // workgroups by role (walk_roles)
     uint32_t spins;                  // how often a wait asks before it is given up
     float eps;
     int rounding;

@@ -3,9 +3,9 @@
 //
 // A token by launches is 144 dependent ones.  Each takes 2.4 us before its first instruction has run and the last one's results
 // can be read, another 0.8 to read them, and its weights are asked for only then; 0.70 ms a token of width 1024 and 28 layers,
-// of which 0.1 is what HBM needs for the weights.  Here a boundary is one exchange (1.5 to 2 us from the first store to the
-// last word read, with 64 to 256 workgroups that read 256 to 1024 words), and the weights of a workgroup's next product are in
-// its registers before the vector arrives: they are loaded right behind the product before.
+// of which 0.1 is what HBM needs for the weights.  Here a boundary is one exchange (1.0 to 1.5 us from the last workgroup's words
+// stored to the last one's read, with 64 to 256 workgroups that read 256 to 1024 words), and the weights of a workgroup's next
+// product are in its registers before the vector arrives: they are loaded right behind the product before.
 //
 // Exchange: a word of 64 bits is 32 bits of a vector and the tag of (token, layer) that it belongs to, stored and loaded whole
 // by relaxed atomics of agent scope; a reader asks until all its words have the tag.  No fence and no counter is needed:
@@ -16,12 +16,13 @@
 //   qkv  norm -> attention    the next x depends on all of attention's words
 //   att  attention -> residual, xm residual -> norm, h norm -> residual, top all -> residual: likewise one stage on
 // Every wait is bounded: a wave that has asked `spins` times marks the launch as failed, which ends the others' waits too, and the
-// session generates again by single launches.  All workgroups run at once, since the launch is a cooperative one.
+// session generates again by single launches.  The launch is a cooperative one: every workgroup has a place, whoever starts first.
 //
 // us a token, 28 layers and a vocabulary of 151936, by launches | walked: behind 100 keys 590 | 425, 700: 761 | 520, 1250: 932 | 685.
-// What a layer takes: six exchanges of 0.9 to 1.4 us (a word alone takes 0.4 to one's own XCD, 0.6 to another, and the last of
-// 64 to 128 workgroups counts), the norms in front of two products 0.75 each, the products, and attention, of which the f32 sum
-// in key order is 1.8 at 544 keys.
+// What a layer takes, us behind 100 | 544 | 1200 keys: 13.8 | 16.9 | 21.9, of that five exchanges 6.0 | 6.1 | 6.0 (a word alone takes
+// 0.4 to one's own XCD, 0.6 to another, and the last of 64 to 128 workgroups counts), two norms and quantizers 1.0, the four
+// products and what follows them 3.7, attention 3.0 | 6.1 | 11.2: scores 0.8 | 1.8 | 2.9, their largest (from 352 keys on with a
+// sixth exchange) 0.6 | 1.0 | 1.2, exp and the f32 sum in key order 0.7 | 2.2 | 4.2, weighted values 0.9 | 1.1 | 3.0.
 //
 // A workgroup's words go out before any of its waves asks for the next weights (the barriers in front of those loads): stores
 // of a late wave queue behind the other waves' loads, and everybody waits for that wave's words.  Without the barriers, and with

@@ -13,9 +13,11 @@
 // that held both products' weights found the feed-forward's words 5.7 us after their own product, in the place of 1.2).
 //
 // us a token by launches | walked, 28 layers of width 1024, the vocabulary's product and its copy apart: behind 140 keys 500 | 295,
-// 420: 521 | 330; 4 layers behind 20: 88 | 77 (a cooperative launch costs some 15 more than another).  A layer is 9.3: the norm
-// and its product 2.1, the mixers 3, the last product 1.1 and three exchanges.  A head's keys and values have to be in its workgroup's
-// registers, so up to 511 keys; behind that, and for the first token, the single launches.
+// 420: 521 | 330; 4 layers behind 20: 88 | 77 (a cooperative launch costs some 15 more than another).  A layer, us behind 128 | 400 keys:
+// 9.2 | 10.4, of that three exchanges 5.4 | 5.9 (x, which the input weights hold up behind few keys, 3.0 | 1.4; what the mixers read, for
+// which keys and values have to be there, 1.1 | 3.5; their results 1.3 | 1.0), norm 0.5, the two products 0.8 to 1.1 each, mixers 1.6 | 2.2.
+// A head's keys and values have to be in its workgroup's registers, so up to 511 keys; behind that, and for the first token, the single
+// launches (a token of 28 layers and a vocabulary of 151936 then takes 560 us; walked it is 335 behind 110 keys, 384 behind 470).
 //
 // Words and tags as in walk_qwen3.hip.  A buffer is written again by a workgroup only behind words that depend on all its readers:
 // everything that norms is behind the whole x of its layer, of which each row's owner has read the mixers' and the feed-forward's

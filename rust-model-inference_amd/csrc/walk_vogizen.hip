@@ -12,8 +12,8 @@
 //
 // us a token by launches | walked, without the vocabulary's product: eight runs of width 2048 behind 300 keys, bf16 418 | 278, f32 562 |
 // 446; 28 of width 1024 behind 60, bf16 985 | 600 to 630, f32 1099 | 770 to 830.  A run with a delta rule then is 27 us in bf16 and 47 in
-// f32, where memory is busy most of the time (4.6 TB/s; a phase's loads start 2 us behind the words before them).  Of the 20 of width
-// 1024 in bf16 products are 4 and the mixer 3.3, norms 2.4, the rest is exchanges of 1.2 to 2.5, seven of them.
+// f32, where memory is busy most of the time (4.6 TB/s; a phase's loads start 2 us behind the words before them).  Of the 19.4 of width
+// 1024 in bf16 products are 3.9 and the mixer 2.9, norms 1.5, the rest is exchanges of 1.2 to 2.4, seven of them.
 //
 // Words and tags as in walk_qwen3.hip.  All of a run's vectors are kept twice, by odd and even runs: a workgroup writes one again only
 // after it has waited for words of the run between, which depend on every other workgroup's: the feed-forward's on all of the stream's,
