@@ -1048,7 +1048,7 @@ def run_decode(args, pkg, ev):
         "workload": "device-resident greedy decode of a synthetic Q8_0 GGUF (Qwen3-0.6B architecture, 28 layers, "
                     "vocab 151936), 512 prompt positions (one pass) + 127 generated tokens = 639 token-steps per "
                     "generation, logits computed at every position; one bench step = one generation",
-        "token_steps_per_generation": token_steps, "generated_tokens_per_launch": "up to 16 (one cooperative launch walks all layers)",
+        "token_steps_per_generation": token_steps, "generated_tokens_per_launch": "up to 4 (one cooperative launch walks all layers)",
         "device": dev_name.strip(), "compute_units": cus})
     result["ms_per_token_step"] = round(per_token * 1e3, 4)
     # the two phases apart: the prompt (positions known in advance: the session takes them up to 1024 to a pass, each

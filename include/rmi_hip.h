@@ -463,11 +463,12 @@ int rmi_hip_qwen3_set_stop_ids(rmi_hip_qwen3 *s, const uint32_t *ids, uint32_t n
  * 0.0145 ms in passes. */
 int rmi_hip_qwen3_set_prompt_passes(rmi_hip_qwen3 *s, int enabled);
 /* Tokens of a model of width 512 or 1024 with 8 or 16 heads of 128, a feed-forward of one to four times 1024 and up to 1279 keys are
- * generated up to 16 to a cooperative launch that walks all layers, the bits of the single launches.  enabled = 1 (the default): so; 0: single launches only; n > 1: so, and a
- * wait between workgroups is given up after it has asked n times (by default 131072, 65 ms or more: some other program's kernel held
- * compute units meanwhile), after which rmi_hip_qwen3_generate begins anew by single launches and the session keeps to them until the next
- * call of this.  Such a launch holds every compute unit for up to 8 ms; while other sessions of the process are at work, too, single
- * launches are taken, which fill one another's gaps. */
+ * generated up to four to a cooperative launch that walks all layers, the bits of the single launches.  enabled = 1 (the default): so;
+ * 0: single launches only; n > 1: so, and a wait between workgroups is given up after it has asked n times (by default 131072, 65 ms or
+ * more: some other program's kernel held compute units meanwhile), after which rmi_hip_qwen3_generate begins anew by single launches
+ * and the session keeps to them until the next call of this.  Such a launch holds every compute unit for up to 2.7 ms, and what other
+ * threads have enqueued starts behind it (a 13-token product on host slices takes 0.6 ms beside a session that generates, 0.05 beside
+ * single launches).  While other sessions of the process are at work, single launches are taken, which fill one another's gaps. */
 int rmi_hip_qwen3_set_walks(rmi_hip_qwen3 *s, int enabled);
 /* Runs up to n_prompt + max_new - 1 steps, one token per step, positions 0.. (the prompt is fed token by
  * token as generate_inner does), greedy sampling (temperature 0, sample_token's argmax branch).  With stop
@@ -570,7 +571,8 @@ int rmi_hip_folder_set_prompt_passes(rmi_hip_folder_session *s, int enabled);
  * when padded to 16, positions up to 511; Vogizen of width 1024 or 2048, 16 heads of 128, a feed-forward of three times the width, a token
  * side of 64 or 128, ranks of whole 256s up to 768 and 256 or 1024 and 512, positions that see up to 1024 keys.  It agrees with the single
  * launches within rounding; a token whose launch gave up (an rmi_hip_folder_generate: the sequence) is done again by them.  Walks of several
- * sessions take turns, for a token's length each.  us a token of all, bf16, single launches | walks: Ruvenex with 28 layers of width 1024, one
+ * sessions take turns, for a token's length each, 0.3 to 0.5 ms, and so does what other threads have enqueued: a session of single launches gets
+ * a third of its rate beside one that walks.  us a token of all, bf16, single launches | walks: Ruvenex with 28 layers of width 1024, one
  * session 542 | 314, two 392 | 277, four 375 | 277; Vogizen with 8 runs of width 1024 462 | 317, 283 | 269, 262 | 278. */
 int rmi_hip_folder_set_walks(rmi_hip_folder_session *s, int enabled);
 int rmi_hip_folder_generate(rmi_hip_folder_session *s, const uint32_t *prompt, uint32_t n_prompt, uint32_t max_new,

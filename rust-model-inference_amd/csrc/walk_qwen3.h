@@ -38,7 +38,9 @@ struct RmiWalkArgs {
 
 // From this position on a head's keys are more than the walk holds.
 constexpr uint32_t kWalkMaxKeys = 1280;
-constexpr uint32_t kWalkMaxSteps = 16;  // of a launch, which holds every compute unit meanwhile: 8 ms
+// Tokens of a launch, which holds every compute unit meanwhile.  us a token of 28 layers behind 100 keys with 1 | 2 | 4 | 8 | 16 of them 437 | 425 |
+// 419 | 415 | 413; a product on host slices beside it, on another thread, 257 | 645 | 622 | 2264 | 5546 us, beside single launches 48.
+constexpr uint32_t kWalkMaxSteps = 4;
 constexpr uint32_t kWalkSpins = 1u << 17;  // at more than half a microsecond each
 
 // Whether a session of this shape can be walked on this device.

@@ -1,7 +1,7 @@
 """Generated tokens of a Qwen3 session by the launch that walks all layers (csrc/walk_qwen3.hip), against the same session by
 single launches and against the CPU loop: tokens, every step's argmax and two largest logits and the asked logits bit for bit,
 where its branches change: heads that share their keys' scores (from 352 keys on), slices of values longer than what is loaded
-ahead (from 769 keys on), the last position it takes (1279 keys), launches of up to 16 tokens."""
+ahead (from 769 keys on), the last position it takes (1279 keys), launches of up to four tokens."""
 import ctypes as C
 import threading
 
@@ -114,12 +114,12 @@ def test_a_wait_that_is_given_up_leaves_the_single_launches(hip, tmp_path):
 
 
 def test_tags_begin_anew(hip, tmp_path):
-    """16 tokens a launch of two layers are 49 tags: launches across the last tag, with words of all tags before them."""
+    """Four tokens a launch of two layers are 13 tags: launches across the last tag, with words of all tags before them."""
     meta, tensors = _model(hip, tmp_path)
     s = hip.decode.Qwen3Session(meta, tensors, 200)
     prompt = np.random.default_rng(9).integers(0, 3000, 20, dtype=np.uint32)
     want = s.generate(prompt, 70, [30, 60, 88])
-    for left in (48, 49, 60, 99):
+    for left in (12, 13, 20, 40):
         walk_tags_from(hip, s, 2**32 - 1 - left)
         before = walks(hip, s)
         _equal(s.generate(prompt, 70, [30, 60, 88]), want, left)
@@ -154,6 +154,7 @@ def test_a_session_walks_only_while_no_other_is_at_work(hip, tmp_path):
     s = hip.decode.Qwen3Session(meta, tensors, 100)
     prompt = np.random.default_rng(7).integers(0, 3000, 30, dtype=np.uint32)
     alone, before = s.generate(prompt, 40, [60]), walks(hip, s)
+    assert before[0] == 10  # 39 tokens by fours, and one launch ends at the logits asked for: other threads' work starts between them
     other = (C.c_uint8 * 8)()
     hip.hip.lib._ZN14RmiSessionBusyC1Ev(other)  # what another session's call holds
     try:
