@@ -570,10 +570,11 @@ int rmi_hip_folder_set_prompt_passes(rmi_hip_folder_session *s, int enabled);
  * shape that has one: Ruvenex in bf16, width 1024, heads of 128, two layers or more, two to four taps, a feed-forward that is whole 256s
  * when padded to 16, positions up to 511; Vogizen of width 1024 or 2048, 16 heads of 128, a feed-forward of three times the width, a token
  * side of 64 or 128, ranks of whole 256s up to 768 and 256 or 1024 and 512, positions that see up to 1024 keys.  It agrees with the single
- * launches within rounding; a token whose launch gave up (an rmi_hip_folder_generate: the sequence) is done again by them.  Walks of several
- * sessions take turns, for a token's length each, 0.3 to 0.5 ms, and so does what other threads have enqueued: a session of single launches gets
- * a third of its rate beside one that walks.  us a token of all, bf16, single launches | walks: Ruvenex with 28 layers of width 1024, one
- * session 542 | 314, two 392 | 277, four 375 | 277; Vogizen with 8 runs of width 1024 462 | 317, 283 | 269, 262 | 278. */
+ * launches within rounding; a token whose launch gave up (an rmi_hip_folder_generate: the sequence) is done again by them.
+ * Other threads' work waits for the end of a walk, a token's 0.3 to 0.5 ms: walks of several sessions take turns, and a session of single
+ * launches gets a quarter to a third of its rate beside one that walks; where sessions of both kinds share a device, 0 for all of them
+ * shares it evenly.  us a token of all, bf16, single launches | walks: Ruvenex with 28 layers of width 1024, one session 542 | 314, two
+ * 392 | 277, four 375 | 277; Vogizen with 8 runs of width 1024 462 | 317, 283 | 269, 262 | 278. */
 int rmi_hip_folder_set_walks(rmi_hip_folder_session *s, int enabled);
 int rmi_hip_folder_generate(rmi_hip_folder_session *s, const uint32_t *prompt, uint32_t n_prompt, uint32_t max_new,
                             uint32_t *generated, uint32_t *step_argmax, float *step_top2, const uint32_t *dump_steps,
